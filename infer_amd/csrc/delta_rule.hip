@@ -10,6 +10,8 @@
 //   delta_scan_kernel    walks the chunks of a portion; a wavefront holds 16 columns of the state as float32 MFMA
 //                        accumulators
 //   delta_out_kernel     output norm and gate of the scanned tokens; the convolution's tail goes to its ring
+//   delta_scan_wide_kernel   scan, output norm and gate in one launch, for batches that fill the chip with one workgroup per
+//                        (portion, head); delta_ring_kernel then writes the rings
 //
 // Chunk form.  Let G_i be the sum of g over the chunk's tokens up to i, S the state before the chunk.
 //     u_i = beta_i (v_i - S^T (e^{G_i} k_i) - sum_{j<i} A_ij u_j),    A_ij = sum_d k_i[d] k_j[d] e^{G_i - G_j}[d]
@@ -17,12 +19,14 @@
 //     o_i = (e^{G_i} q_i)^T S + sum_{j<=i} B_ij u_j,                  B_ij = sum_d q_i[d] k_j[d] e^{G_i - G_j}[d]
 //     S'  = e^{G_last} S + sum_j (e^{G_last - G_j} k_j) u_j^T.
 // Every exponent is a difference that is <= 0, so nothing overflows however strong the decay is.  All of it is
-// float32, the products included (v_mfma_f32_16x16x4_f32).
+// float32, the products included (v_mfma_f32_16x16x4_f32; in the wide scan six bf16 products of the pieces of a float).
 //
 // The last `taps` inputs of the convolution live in a ring per sequence (entry position % taps).  A position below
 // zero counts as zero and a portion that starts at position 0 starts from a zero state, so a slot needs no clearing
 // when another sequence takes it over.
-#include "elem.h"
+#include "pieces.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -574,6 +578,264 @@ __global__ void __launch_bounds__(256) delta_scan_kernel(const PortionDesc* port
             for (int r = 0; r < 4; ++r) sp[(int64_t)(16 * t + 4 * q + r) * vdim_pad] = s[t][r];
 }
 
+// x summed over the 32 lanes of a half of the wavefront, in all of them
+__device__ __forceinline__ float half_sum(float x) {
+    auto ror = [](float v, auto C) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(C)::value, 0xf, 0xf, false)); };
+    x += ror(x, std::integral_constant<int, 0x128>{});          // rotations by 8, 4, 2 and 1 within rows of 16 lanes
+    x += ror(x, std::integral_constant<int, 0x124>{});
+    x += ror(x, std::integral_constant<int, 0x122>{});
+    x += ror(x, std::integral_constant<int, 0x121>{});
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned lo = r[0], hi = r[1];
+    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+
+// hi + mid + lo = x exactly, two floats at a time: a residual is one dot product with (-1, 0) or (0, -1) instead of a mask and a subtraction
+template <int N>
+__device__ __forceinline__ void split3(const float (&x)[N], uint32_t (&p)[3][N / 2]) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    uint32_t c0 = 0x0000bf80u, c1 = 0xbf800000u;       // (-1, 0) and (0, -1)
+    asm("" : "+s"(c0), "+s"(c1));                      // in registers: as an inline constant the compiler writes -1.0, which is another pair
+    const bf16x2_t first = __builtin_bit_cast(bf16x2_t, c0), second = __builtin_bit_cast(bf16x2_t, c1);
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        p[0][i] = pack(x[2 * i], x[2 * i + 1]);
+        const bf16x2_t hi = __builtin_bit_cast(bf16x2_t, p[0][i]);
+        const float a = __builtin_amdgcn_fdot2_f32_bf16(hi, first, x[2 * i], false), b = __builtin_amdgcn_fdot2_f32_bf16(hi, second, x[2 * i + 1], false);
+        p[1][i] = pack(a, b);
+        const bf16x2_t mid = __builtin_bit_cast(bf16x2_t, p[1][i]);
+        p[2][i] = pack(__builtin_amdgcn_fdot2_f32_bf16(mid, first, a, false), __builtin_amdgcn_fdot2_f32_bf16(mid, second, b, false));
+    }
+}
+
+// A record in LDS: sums of three bf16 numbers, hi + mid + lo = the float exactly, so that the products run on the bf16 matrix pipe.  Of
+// the nine products of two such sums the six down to 2^-16 of the first are added; what is left out lies below the last bit of a float
+// product.
+struct WideBuffer {
+    u32x4_t* p;
+    int ks;
+    __device__ __forceinline__ u32x4_t* wq(int which, int kk, int piece) const { return p + (((which * ks + kk) * 3 + piece) * 64); }
+    __device__ __forceinline__ u32x4_t* k(int t, int form) const { return p + (6 * ks + 2 * t + form) * 64; }          // 0: [hi | mid], 1: [hi | lo]
+    __device__ __forceinline__ u32x4_t* b(int form) const { return p + (10 * ks + form) * 64; }
+    __device__ __forceinline__ u32x4_t* e() const { return p + (10 * ks + 2) * 64; }
+};
+__host__ __device__ constexpr int wide_buffer_units(int dt) { return 64 * (5 * dt + 2) + 4 * dt; }
+
+// All columns of a head in one workgroup: eight wavefronts, of which `slabs` own 16 columns of the state each and all bring the next
+// record to LDS, cut into pieces.  A chunk's outputs go through LDS to rows of a wavefront's half, which the next step norms and gates,
+// so they do not pass through memory in between.
+// A batch takes as long as its longest portion's chunks one after the other; a step of eight wavefronts on a compute unit is 3200 clocks
+// of matrix pipe per wavefront with float products and 1200 with pieces, which cost about 180 vector instructions.  32 heads, 8 portions
+// of 590 to 2560 tokens: scan, output and ring 655 us with delta_scan_kernel, 435 us here.  What a step waits for is requested a step
+// before, by every thread and without branches: with requests in branches, or stores between a request and its use, the compiler waits
+// for everything in flight (830 us).  Tried as well: float products for W S (690 us); the two wavefronts of a vector unit in opposite
+// phases (550); four wavefronts that only serve eight that compute (460).
+template <class T, int DT>
+__global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a, const PortionDesc* portions, const ChunkDesc* chunks,
+                                                                 const float* records, int slabs) {
+    constexpr int dp = 16 * DT, KS = DT / 2, kShared = 49 * dp + 256, kPitch = 132;
+    extern __shared__ __attribute__((aligned(16))) u32x4_t lds[];     // [2] buffers, then outputs [2][16][kPitch]
+    float* outputs = reinterpret_cast<float*>(lds + 2 * wide_buffer_units(DT));
+    const int tid = threadIdx.x, lane = tid & 63, vt = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, m = lane & 15;
+    const int h = blockIdx.x;
+    const PortionDesc p = portions[blockIdx.y];
+    const bool live = vt < slabs;
+    const int vdim_pad = a.vdim_pad;
+    const int64_t rec_len = record_floats(dp, vdim_pad);
+    const f32x4_t* rec = reinterpret_cast<const f32x4_t*>(records + ((int64_t)p.chunk0 * a.heads + h) * rec_len);
+    const int64_t rec_step = (int64_t)a.heads * rec_len / 4;
+    float* sp = a.state + (((int64_t)p.slot * a.heads + h) * dp) * vdim_pad + 16 * vt + m;
+    f32x4_t s[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+        s[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (live && p.pos0 > 0)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[t][r] = sp[(int64_t)(16 * t + 4 * q + r) * vdim_pad];
+    }
+
+    // Every request is made by every thread, so that the compiler knows how many are in flight; what a thread has no use for is the
+    // record's start.
+    const int w_at = tid < 64 * DT ? (tid / (64 * KS)) * 4 * dp + ((tid >> 6) % KS) * 128 + lane : 0, k_at = tid < 64 * DT ? 8 * dp + tid : 0;
+    const int b_at = tid < 64 + dp / 4 ? 12 * dp + tid : 0, v_at = live ? kShared / 4 + vt * 64 + lane : 0;
+    f32x4_t w0, w1, kf, be, vn;
+    auto fetch = [&](int c) {
+        const f32x4_t* src = rec + (c < p.chunks ? c : p.chunks - 1) * rec_step;
+        w0 = src[w_at];
+        w1 = src[w_at + 64];
+        kf = src[k_at];
+        be = src[b_at];
+        vn = src[v_at];
+    };
+    auto put = [&](int half) {
+        const WideBuffer buf{lds + half * wide_buffer_units(DT), KS};
+        auto two_forms = [&](f32x4_t x, u32x4_t* d0, u32x4_t* d1) {
+            const float f[4] = {x[0], x[1], x[2], x[3]};
+            uint32_t pc[3][2];
+            split3<4>(f, pc);
+            d0[lane] = u32x4_t{pc[0][0], pc[0][1], pc[1][0], pc[1][1]};
+            d1[lane] = u32x4_t{pc[0][0], pc[0][1], pc[2][0], pc[2][1]};
+        };
+        if (DT == 8 || tid < 64 * DT) {
+            const float f[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
+            uint32_t pc[3][4];
+            split3<8>(f, pc);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) buf.wq(vt / KS, vt % KS, i)[lane] = u32x4_t{pc[i][0], pc[i][1], pc[i][2], pc[i][3]};
+            two_forms(kf, buf.k(vt, 0), buf.k(vt, 1));
+        }
+        if (vt == 0) two_forms(be, buf.b(0), buf.b(1));
+        else if (tid < 64 + dp / 4) buf.e()[tid - 64] = __builtin_bit_cast(u32x4_t, be);
+    };
+    auto mma = [](u32x4_t x, bf16x8_t y, f32x4_t acc) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x), y, acc, 0, 0, 0); };
+
+    // Rows 2 vt and 2 vt + 1 of a chunk's outputs, four columns per lane.  The gate is requested with the chunk, a step before it is used.
+    const int out_row = 2 * vt + (lane >> 5), out_col = 4 * (lane & 31);
+    const bool out_in = out_col < a.vdim;
+    typedef T t4_t __attribute__((ext_vector_type(4)));
+    t4_t gate;
+    float norm[4];
+    load_elems<4>(a.norm + (out_in ? out_col : 0), norm);
+    const T* gates = a.gate + (int64_t)h * a.vdim + (out_in ? out_col : 0);
+    T* outs = a.out + (int64_t)h * a.vdim + out_col;
+    int done_row = 0, done_count = 0;
+    const float inv_vdim = 1.f / (float)a.vdim;
+    auto finish = [&](int half) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(outputs + (half * 16 + out_row) * kPitch + out_col);
+        float ss = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
+        ss = half_sum(ss);
+        const float rs = rsqrtf(ss * inv_vdim + a.eps);
+        float y[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] = x[r] * (rs * norm[r] * sigmoid_f((float)gate[r]));
+        if (out_in && out_row < done_count) store_elems<4>(outs + (int64_t)(done_row + out_row) * a.out_stride, y);
+    };
+
+    // A step first brings the next record, requested a step ago, to LDS and requests the one behind it: what a step waits for has
+    // had a whole step to arrive.
+    int zero = 0;
+    asm volatile("" : "+v"(zero));                     // by the vector path: a scalar load in flight would be waited for with every LDS read
+    const int32_t* descs = &chunks[p.chunk0].row0 + zero;
+    constexpr int kDesc = sizeof(ChunkDesc) / sizeof(int32_t);
+    int next_row = descs[0], next_count = descs[1];
+    int row = __builtin_amdgcn_readfirstlane(next_row), count = __builtin_amdgcn_readfirstlane(next_count);
+    const int second = p.chunks > 1 ? kDesc : 0;
+    next_row = descs[second];
+    next_count = descs[second + 1];
+    for (int i = tid; i < 2 * 16 * kPitch; i += 512) outputs[i] = 0.f;           // columns behind the last slab stay so
+    fetch(0);
+    f32x4_t v = vn;
+    put(0);
+    fetch(1);
+    __syncthreads();
+    for (int c = 0; c < p.chunks; ++c) {
+        const WideBuffer buf{lds + (c & 1) * wide_buffer_units(DT), KS};
+        f32x4_t u = v;
+        if (c + 1 < p.chunks) {
+            v = vn;
+            put((c + 1) & 1);
+        }
+        if (c > 0) finish((c - 1) & 1);
+        fetch(c + 2);
+        gate = *reinterpret_cast<const t4_t*>(gates + (int64_t)(row + (out_row < count ? out_row : count - 1)) * a.gate_stride);
+        __builtin_amdgcn_sched_barrier(0);             // requests stay here, a step ahead of their use
+        if (live) {
+            // the vector unit cuts the next part of the state while the matrix pipe works on one
+            f32x4_t x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1, x3 = x1, o1 = x1, o2 = x1, o3 = x1;
+            uint32_t pc[KS][3][4];
+            u32x4_t w[KS][3], qv[KS][3];
+            auto part = [&](int kk) {
+                const float f[8] = {s[2 * kk][0], s[2 * kk][1], s[2 * kk][2], s[2 * kk][3], s[2 * kk + 1][0], s[2 * kk + 1][1], s[2 * kk + 1][2], s[2 * kk + 1][3]};
+#pragma unroll
+                for (int i = 0; i < 3; ++i) { w[kk][i] = buf.wq(0, kk, i)[lane]; qv[kk][i] = buf.wq(1, kk, i)[lane]; }
+                split3<8>(f, pc[kk]);
+            };
+            part(0);
+#pragma unroll
+            for (int kk = 0; kk < KS; ++kk) {
+                const bf16x8_t sh = frag(pc[kk][0]), sm = frag(pc[kk][1]), sl = frag(pc[kk][2]);
+                if (kk + 1 < KS) part(kk + 1);
+                x1 = mma(w[kk][0], sh, x1);
+                o1 = mma(qv[kk][0], sh, o1);
+                x2 = mma(w[kk][1], sh, x2);
+                o2 = mma(qv[kk][1], sh, o2);
+                x3 = mma(w[kk][2], sh, x3);
+                o3 = mma(qv[kk][2], sh, o3);
+                x2 = mma(w[kk][0], sm, x2);
+                o2 = mma(qv[kk][0], sm, o2);
+                x3 = mma(w[kk][1], sm, x3);
+                o3 = mma(qv[kk][1], sm, o3);
+                x3 = mma(w[kk][0], sl, x3);
+                o3 = mma(qv[kk][0], sl, o3);
+            }
+            u = u - (x1 + (x2 + x3));
+            uint32_t uc[3][2];
+            {
+                const float f[4] = {u[0], u[1], u[2], u[3]};
+                split3<4>(f, uc);
+            }
+            const bf16x8_t uhh = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[0][0], uc[0][1], uc[0][0], uc[0][1]});
+            const bf16x8_t umm = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[1][0], uc[1][1], uc[1][0], uc[1][1]});
+            const bf16x8_t ulh = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[2][0], uc[2][1], uc[0][0], uc[0][1]});
+            const u32x4_t b0 = buf.b(0)[lane], b1 = buf.b(1)[lane];
+            o3 = mma(b1, ulh, o3);
+            o2 = mma(b0, umm, o2);
+            o1 = mma(b0, uhh, o1);
+            const f32x4_t* e = reinterpret_cast<const f32x4_t*>(buf.e());
+            u32x4_t k0[DT], k1[DT];
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                k0[t] = buf.k(t, 0)[lane];
+                k1[t] = buf.k(t, 1)[lane];
+                s[t] *= e[4 * t + q];
+            }
+#pragma unroll
+            for (int t = 0; t < DT; ++t) s[t] = mma(k1[t], ulh, s[t]);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) s[t] = mma(k0[t], umm, s[t]);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) s[t] = mma(k0[t], uhh, s[t]);
+            const f32x4_t o = o1 + (o2 + o3);
+            float* to = outputs + ((c & 1) * 16 + 4 * q) * kPitch + 16 * vt + m;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) to[r * kPitch] = o[r];
+        }
+        done_row = row;
+        done_count = count;
+        row = __builtin_amdgcn_readfirstlane(next_row);
+        count = __builtin_amdgcn_readfirstlane(next_count);
+        const int after = c + 2 < p.chunks ? c + 2 : p.chunks - 1;
+        next_row = descs[after * kDesc];
+        next_count = descs[after * kDesc + 1];
+        __syncthreads();
+    }
+    finish((p.chunks - 1) & 1);
+    if (!live) return;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sp[(int64_t)(16 * t + 4 * q + r) * vdim_pad] = s[t][r];
+}
+
+// The inputs of the convolution that a portion's last tokens leave in its ring; a workgroup looks at 64 rows and copies VEC * 256 channels
+// of those it finds.
+template <class T, int VEC>
+__global__ void __launch_bounds__(256) delta_ring_kernel(DeltaArgs<T> a, int64_t row0, int64_t rows, const int32_t* ring_slot, const int64_t* positions) {
+    typedef T vec_t __attribute__((ext_vector_type(VEC)));
+    const int64_t first = row0 + 64 * (int64_t)blockIdx.x, mine = first + (threadIdx.x & 63);
+    const int c = (blockIdx.y * 256 + threadIdx.x) * VEC;
+    const int slot = mine < row0 + rows ? ring_slot[2 * mine] : -1;
+    const int follow = mine < row0 + rows ? ring_slot[2 * mine + 1] : a.taps;
+    uint64_t found = __ballot(slot >= 0 && slot < a.num_slots && follow < a.taps);
+    while (found) {
+        const int i = __builtin_ctzll(found);
+        found &= found - 1;
+        const int64_t row = first + i, to = (int64_t)__builtin_amdgcn_readlane(slot, i) * a.taps + positions[row] % a.taps;
+        if (c < a.channels) *reinterpret_cast<vec_t*>(a.ring + to * a.channels + c) = *reinterpret_cast<const vec_t*>(a.proj + row * a.proj_stride + c);
+    }
+}
+
 // One workgroup per token row behind `row0`.  LANES lanes share a head, four values each (vdim = 4 LANES);
 // LANES = 0: any vdim, one wavefront per head.
 template <class T, int LANES>
@@ -637,6 +899,19 @@ int launch_scan(const PortionDesc* p, int64_t portions, const ChunkDesc* c, cons
     return (int)hipGetLastError();
 }
 
+template <class T, int DT>
+int launch_scan_wide(const DeltaArgs<T>& a, const PortionDesc* p, int64_t portions, const ChunkDesc* c, const float* records, hipStream_t st) {
+    constexpr size_t lds = (size_t)2 * wide_buffer_units(DT) * 16 + 2 * 16 * 132 * sizeof(float);
+    if (lds > 60 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_scan_wide_kernel<T, DT>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL((delta_scan_wide_kernel<T, DT>), dim3((unsigned)a.heads, (unsigned)portions), dim3(512), lds, st, a, p, c, records,
+                       a.vdim_pad / 16);
+    return (int)hipGetLastError();
+}
+
 template <class T>
 int make_args(DeltaArgs<T>& a, const void* proj, int64_t proj_stride, int64_t beta_off, const void* decay, int64_t decay_stride,
               const void* gate, int64_t gate_stride, const float* conv, const float* a_log, const float* dt_bias, const float* norm,
@@ -694,11 +969,26 @@ int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t nu
     hipLaunchKernelGGL(prep, dim3((unsigned)num_chunks, (unsigned)a.heads), dim3(256), lds, st, a, chunks, records);
     int rc = (int)hipGetLastError();
     if (rc) return rc;
+    const bool out4 = rows4 && fours(a.gate, a.gate_stride) && fours(a.out, a.out_stride) && ptr_aligned(o, 16) && ptr_aligned(a.norm, 16);
+    // Up to 256 workgroups of four wavefronts, those of delta_scan_kernel have a vector unit each, and its shorter step wins: one portion
+    // of 2000 tokens, 16 heads 358 us against 387; of 9000, 32 heads 1702 against 1810.  Beyond, two share one: 32 heads, 16 portions
+    // of 800 tokens 872 us against 711; 60 portions of 110 539 against 444.
+    if (out4 && 2 * (int64_t)a.heads * num_portions > 256 && a.vdim_pad <= 128 && (a.dim_pad == 32 || a.dim_pad == 64 || a.dim_pad == 96 || a.dim_pad == 128)) {
+#define GO(N) case N: rc = launch_scan_wide<T, N>(a, portions, num_portions, chunks, records, st); break
+        switch (a.dim_pad / 16) { GO(2); GO(4); GO(6); GO(8); }
+#undef GO
+        if (rc) return rc;
+        const unsigned groups = (unsigned)((rows + 63) / 64);
+        if (rows4 && fours(a.proj, a.proj_stride) && fours(a.ring, a.channels))
+            hipLaunchKernelGGL((delta_ring_kernel<T, 4>), dim3(groups, (unsigned)((a.channels + 1023) / 1024)), dim3(256), 0, st, a, row0, rows, ring_slot, positions);
+        else
+            hipLaunchKernelGGL((delta_ring_kernel<T, 1>), dim3(groups, (unsigned)((a.channels + 255) / 256)), dim3(256), 0, st, a, row0, rows, ring_slot, positions);
+        return (int)hipGetLastError();
+    }
 #define GO(N) case N: rc = launch_scan<N>(portions, num_portions, chunks, records, a.state, o, a.heads, a.vdim_pad, st); break
     switch (a.dim_pad / 16) { GO(1); GO(2); GO(3); GO(4); GO(6); GO(8); GO(12); GO(16); default: return INFER_KV_EUNSUPPORTED; }
 #undef GO
     if (rc) return rc;
-    const bool out4 = rows4 && fours(a.gate, a.gate_stride) && fours(a.out, a.out_stride) && ptr_aligned(o, 16) && ptr_aligned(a.norm, 16);
 #define GO(N) hipLaunchKernelGGL((delta_out_kernel<T, N>), dim3((unsigned)rows), dim3(256), 0, st, a, (const float*)o, row0, ring_slot, positions)
     if (out4 && a.vdim == 32) GO(8);
     else if (out4 && a.vdim == 64) GO(16);

@@ -395,6 +395,46 @@ def test_delta_batches_slots_and_padding(gpu):
     again.check([2, 1, 17], slot=2)
 
 
+@BOTH
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,decay", [(36, 18, 32, 16, -2.0), (33, 11, 20, 40, -6.0), (34, 17, 64, 64, 40.0), (36, 9, 96, 72, -2.0),
+                                                           (40, 40, 128, 128, -4.0), (33, 33, 120, 124, 0.0)])
+def test_delta_batch_that_fills_the_chip(gpu, dtype, heads, kv_heads, dim, vdim, decay):
+    """More than 128 (portion, head) pairs, so that one workgroup holds all columns of a head: portions of one token more than a chunk,
+    of whole chunks and of two tokens, from a first position and continued from the state and the ring they left."""
+    n = [[17, 16, 2, 47], [5, 33, 16, 31]]
+    cases = [DeltaCase(heads, kv_heads, dim, vdim, 4, a + b, dtype, seed=30 + i, decay=decay, slots=5) for i, (a, b) in enumerate(zip(*n))]
+    c0, s = cases[0], cases[0].s
+    for c in cases[1:]:
+        c.conv, c.a_log, c.dt, c.norm = c0.conv, c0.a_log, c0.dt, c0.norm
+    slots, done, outs = [3, 0, 4, 1], [0] * 4, [[] for _ in range(4)]
+    for part in n:
+        cat = lambda name: dev(np.concatenate([getattr(c, name)[d:d + k] for c, d, k in zip(cases, done, part)]), dtype)
+        chunks, portions, ring, pos, row = [], [], [], [], 0
+        for slot, d, k in zip(slots, done, part):
+            portions.append((len(chunks), -(-k // 16), slot, d))
+            chunks += [(row + r, min(16, k - r), d + r, d, slot, 0) for r in range(0, k, 16)]
+            ring += [(slot, k - 1 - r) for r in range(k)]
+            pos += range(d, d + k)
+            row += k
+        out = torch.full((row, heads * vdim), float("nan"), dtype=dtype, device="cuda")
+        ho.delta_chunks(s, cat("proj"), c0.beta_off, cat("decay"), cat("gate"), *c0.weights, c0.ring, c0.state, dev(portions, torch.int32),
+                        dev(chunks, torch.int32), dev(ring, torch.int32), dev(pos, torch.int64), 0, out)
+        at = 0
+        for i, k in enumerate(part):
+            outs[i].append(host(out[at:at + k]))
+            at += k
+            done[i] += k
+    for i, c in enumerate(cases):
+        want, want_state = c.want()
+        # the bounds of the other delta tests: float32 sums of up to 128 terms over 64 tokens, bfloat16 outputs
+        assert np.abs(np.concatenate(outs[i]) - want).max() <= tol(dtype, 3e-5, 1e-2) * np.abs(want).max()
+        close(c0.state[slots[i]][:, :dim, :vdim], want_state, 3e-5)
+        rest = host(c0.state[slots[i]])
+        assert (rest[:, dim:] == 0).all() and (rest[:, :, vdim:] == 0).all()
+        assert torch.equal(c0.ring[slots[i]].float().cpu(), torch.tensor(np.stack([c.proj[[p for p in range(c.n) if p % 4 == j][-1], :s.channels] for j in range(4)])).float())
+    assert torch.isnan(c0.state[2]).all()
+
+
 def test_sizes_outside_are_refused_on_the_host(gpu):
     with pytest.raises(RuntimeError):
         ho.delta_layout(300, 16)
