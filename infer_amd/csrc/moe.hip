@@ -5,13 +5,15 @@
 //   moe_scatter_kernel    rows sorted by expert: place of every choice, token and expert of every place, row tiles
 //   moe_block_kernel      products of many rows per expert: 256 rows x 256 columns per workgroup, straight from memory to LDS
 //   moe_tile_kernel       products of large row tiles: 128 rows x 128 columns per workgroup, through registers to LDS
-//   moe_row_kernel        products of 16-row tiles (decode): the weights stream past the rows, k split over wavefronts
+//   moe_row_kernel        products of up to 32 rows (decode): the weights stream past the rows, k split over wavefronts
 //   moe_any_kernel        any size and element type
 //
 // The first product takes gate and up columns side by side and stores act = silu(gate) * up, the second stores one row per
 // place; the weighted sum of a token's rows is part of the next residual step (pre_norm.hip).  A choice beyond the experts is
 // the identity: place -1, no row.
-#include "elem.h"
+#include "weight_stream.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -30,6 +32,16 @@ struct RouteArgs {
     int n;
 };
 
+// the maximum over the wavefront's lanes, without a trip through LDS
+__device__ __forceinline__ float wave_max(float x) {
+    auto ror = [](float v, auto C) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(C)::value, 0xf, 0xf, false)); };
+    x = fmaxf(x, ror(x, std::integral_constant<int, 0x128>{}));           // rotations by 8, 4, 2 and 1 within rows of 16 lanes
+    x = fmaxf(x, ror(x, std::integral_constant<int, 0x124>{}));
+    x = fmaxf(x, ror(x, std::integral_constant<int, 0x122>{}));
+    x = fmaxf(x, ror(x, std::integral_constant<int, 0x121>{}));
+    return max_xor16_32(x);
+}
+
 // The choices of one token by one wavefront; `z` are its logits in LDS.  Ties go to the lower index.
 template <int NE, class T>
 __device__ __forceinline__ void choose(const RouteArgs<T>& a, const float* z, int64_t token, int* hist, int* rank_out) {
@@ -42,8 +54,7 @@ __device__ __forceinline__ void choose(const RouteArgs<T>& a, const float* z, in
         s[i] = e < a.all ? z[e] : -INFINITY;
         mx = fmaxf(mx, s[i]);
     }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+    mx = wave_max(mx);
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < NE; ++i) {
@@ -59,20 +70,21 @@ __device__ __forceinline__ void choose(const RouteArgs<T>& a, const float* z, in
         c[i] = e < a.all ? s[i] + (a.correction ? a.correction[e] : 0.f) : -INFINITY;
         if (e < a.all && a.keep >= a.groups) open |= 1u << i;
     }
-    // the largest of the entries whose bit in `of` is set; -1: none
+    // the largest of the entries whose bit in `of` is set, the first of equal ones (of numbers that do not compare: the first); -1: none
     auto best = [&](unsigned of) {
         float v = -INFINITY;
-        int at = 0x7fffffff;
 #pragma unroll
         for (int i = 0; i < NE; ++i)
-            if ((of >> i & 1u) && (at == 0x7fffffff || c[i] > v)) { v = c[i]; at = lane + 64 * i; }
+            if (of >> i & 1u) v = fmaxf(v, c[i]);
+        v = wave_max(v);
+        int at = -1, any = -1;
 #pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            const float ov = __shfl_xor(v, m, 64);
-            const int oat = __shfl_xor(at, m, 64);
-            if (oat != 0x7fffffff && (at == 0x7fffffff || ov > v || (ov == v && oat < at))) { v = ov; at = oat; }
+        for (int i = 0; i < NE; ++i) {
+            const uint64_t set = __ballot(of >> i & 1u), top = __ballot((of >> i & 1u) && c[i] == v);
+            if (at < 0 && top) at = __builtin_ctzll(top) + 64 * i;
+            if (any < 0 && set) any = __builtin_ctzll(set) + 64 * i;
         }
-        return at == 0x7fffffff ? -1 : at;
+        return at < 0 ? any : at;
     };
     if (a.keep < a.groups) {               // groups in the order of their largest entry
         unsigned valid = 0;
@@ -155,18 +167,33 @@ __global__ void __launch_bounds__(64 * W) moe_route_tile_kernel(RouteArgs<__bf16
             for (int u = 0; u < U; ++u) acc[u][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x[u], acc[u][i], 0, 0, 0);
         }
     }
-    for (int w = 0; w < W; ++w) {
-        if (wave == w)
+    if constexpr (ET == 1 && U <= 2) {                 // every wavefront's part side by side, added by a thread per logit
+        __shared__ float part[W][256 * U];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int i = 0; i < ET; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float* p = z + (16 * u + n) * kRow + 16 * i + 4 * g + e;
-                        *p = w == 0 ? acc[u][i][e] : *p + acc[u][i][e];
-                    }
+        for (int u = 0; u < U; ++u)
+            *reinterpret_cast<f32x4_t*>(&part[wave][256 * u + 16 * n + 4 * g]) = acc[u][0];
         __syncthreads();
+        for (int i = tid; i < 256 * U; i += 64 * W) {
+            float sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < W; ++w) sum += part[w][i];
+            z[(i >> 4) * kRow + (i & 15)] = sum;
+        }
+        __syncthreads();
+    } else {
+        for (int w = 0; w < W; ++w) {
+            if (wave == w)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int i = 0; i < ET; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            float* p = z + (16 * u + n) * kRow + 16 * i + 4 * g + e;
+                            *p = w == 0 ? acc[u][i][e] : *p + acc[u][i][e];
+                        }
+            __syncthreads();
+        }
     }
     const int tokens = token0 + 16 * U < a.n ? 16 * U : (int)(a.n - token0);
     for (int t = wave; t < tokens; t += W) choose<(ET + 3) / 4>(a, z + t * kRow, token0 + t, hist, ranks + t * a.top);
@@ -176,6 +203,7 @@ __global__ void __launch_bounds__(64 * W) moe_route_tile_kernel(RouteArgs<__bf16
 template <int ET>
 void launch_route(const RouteArgs<__bf16>& a, hipStream_t st) {
     if (a.n <= 2048) hipLaunchKernelGGL((moe_route_tile_kernel<ET, 1, 16>), dim3((unsigned)((a.n + 15) / 16)), dim3(1024), 0, st, a);
+    else if constexpr (ET == 1) hipLaunchKernelGGL((moe_route_tile_kernel<ET, 2, 16>), dim3((unsigned)((a.n + 31) / 32)), dim3(1024), 0, st, a);
     else hipLaunchKernelGGL((moe_route_tile_kernel<ET, 2, 4>), dim3((unsigned)((a.n + 31) / 32)), dim3(256), 0, st, a);
 }
 
@@ -507,65 +535,62 @@ __global__ void __launch_bounds__(kBlockThreads, 2) moe_block_kernel(GemmArgs<__
     }
 }
 
-// A workgroup: 16 rows of one expert x 32 rows of W (GATED: 16 gate and 16 up); wavefront w takes the k-steps w, w + 4, ...
-constexpr int kSmallRows = 16;
+// A workgroup: up to 32 rows of one expert x 16 rows of W (GATED: 8 gate and 8 up), which stream past them; the second half of the rows
+// costs only where there are that many.  64 rows, three of 16 experts of 3072 x 4096: 258 us with 32 rows of W past 16 rows through
+// operand registers, 181 us now (5.9 TB/s of weights).
+constexpr int kSmallRows = 32, kRowWaves = 4;
+constexpr int kRowRing = 3 * stream_stage_bytes(1, 1);           // of a wavefront: three steps with 16 rows, two with 32
+static_assert(2 * stream_stage_bytes(1, 2) <= kRowRing, "both rings fit");
+template <bool GATED, int MT>
+__device__ __forceinline__ void moe_row_product(const GemmArgs<__bf16>& a, int expert, int first, int rows, int c0, unsigned char* lds) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const __bf16* w[2];
+    const __bf16* x[2 * MT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        int col = c0 + stream_row() + (GATED ? 0 : 8 * i);
+        col = col < a.cols ? col : a.cols - 1;
+        w[i] = a.w + (int64_t)expert * a.w_expert + (int64_t)(GATED && i ? a.up_row + col : col) * a.w_stride;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+        const int r = stream_row() + 8 * i, xr = first + (r < rows ? r : rows - 1);
+        x[i] = a.x + (int64_t)(a.row_token ? a.row_token[xr] : xr) * a.x_stride;
+    }
+    f32x4_t acc[1][MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[0][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    stream_product<1, MT, kRowWaves, MT == 1 ? 3 : 2>(w, x, a.k, wave, lds + wave * kRowRing, acc);
+    stream_reduce<1, MT, kRowWaves>(acc, wave, lds, [&](int, int t, f32x4_t sum) {
+        const int r = 16 * t + n;
+        __bf16* o = a.out + (int64_t)(first + r) * a.out_stride;
+        if constexpr (GATED) {                         // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float up = __shfl_xor(sum[e], 32, 64);
+                sum[e] = silu_f(sum[e]) * up;
+            }
+            if (g >= 2) return;
+        }
+        if (r >= rows) return;
+        const int c = c0 + 4 * g;
+        bf16x4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (__bf16)(c + e < a.cols ? sum[e] : 0.f);
+        if (c + 4 <= a.out_cols) *reinterpret_cast<bf16x4_t*>(o + c) = v;       // out_cols is a multiple of eight
+    });
+}
 template <bool GATED>
-__global__ void __launch_bounds__(kThreads) moe_row_kernel(GemmArgs<__bf16> a) {
-    __shared__ float part[4][2][16][17];
+__global__ void __launch_bounds__(64 * kRowWaves) moe_row_kernel(GemmArgs<__bf16> a) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kRowWaves * kRowRing];
     clear_counts(a);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
     const int tile = blockIdx.x / a.col_blocks, cb = blockIdx.x % a.col_blocks;
     const int expert = a.tiles[2 * tile];
     if (expert < 0 || expert >= a.experts) return;
     const int first = a.offsets[expert] + a.tiles[2 * tile + 1], end = a.offsets[expert + 1];
-    const int rows = end - first < kSmallRows ? end - first : kSmallRows;
-    const int c0 = cb * (GATED ? 16 : 32), xr = first + (n < rows ? n : rows - 1);
-    const __bf16* x = a.x + (int64_t)(a.row_token ? a.row_token[xr] : xr) * a.x_stride;
-    const __bf16* w = a.w + (int64_t)expert * a.w_expert;
-    const __bf16* wr[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        int col = c0 + n + (GATED ? 0 : 16 * i);
-        col = col < a.cols ? col : a.cols - 1;
-        wr[i] = w + (int64_t)(GATED && i ? a.up_row + col : col) * a.w_stride;
-    }
-    f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    constexpr int kAhead = 4;
-    for (int k0 = 32 * wave; k0 < a.k; k0 += 128 * kAhead) {
-        bf16x8_t xf[kAhead], wf[kAhead][2];
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            const int k = k0 + 128 * j + 8 * g;
-            const int at = k < a.k ? k : 0;
-            xf[j] = *reinterpret_cast<const bf16x8_t*>(x + at);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) wf[j][i] = *reinterpret_cast<const bf16x8_t*>(wr[i] + at);
-        }
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            if (k0 + 128 * j + 8 * g >= a.k) xf[j] = bf16x8_t{};
-#pragma unroll
-            for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][i], xf[j], acc[i], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) part[wave][i][n][4 * g + e] = acc[i][e];
-    __syncthreads();
-    const int r = tid >> 4, c = tid & 15;
-    if (r >= rows) return;
-    float v[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) v[i] = part[0][i][r][c] + part[1][i][r][c] + part[2][i][r][c] + part[3][i][r][c];
-    __bf16* o = a.out + (int64_t)(first + r) * a.out_stride + c0 + c;
-    if constexpr (GATED) {
-        if (c0 + c < a.out_cols) o[0] = (__bf16)(c0 + c < a.cols ? silu_f(v[0]) * v[1] : 0.f);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            if (c0 + 16 * i + c < a.out_cols) o[16 * i] = (__bf16)(c0 + 16 * i + c < a.cols ? v[i] : 0.f);
-    }
+    const int rows = end - first < kSmallRows ? end - first : kSmallRows, c0 = cb * (GATED ? 8 : 16);
+    if (rows <= 16) moe_row_product<GATED, 1>(a, expert, first, rows, c0, lds);
+    else moe_row_product<GATED, 2>(a, expert, first, rows, c0, lds);
 }
 
 // one wavefront per (place, four columns)
@@ -610,7 +635,7 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t max_places, hipStrea
             return (int)hipGetLastError();
         }
         if (tile_rows == kBigRows || tile_rows == kSmallRows) {
-            const int per = tile_rows == kBigRows ? (gated ? 64 : 128) : (gated ? 16 : 32);
+            const int per = tile_rows == kBigRows ? (gated ? 64 : 128) : (gated ? 8 : 16);
             a.col_blocks = (a.out_cols + per - 1) / per;
             grid = (int64_t)a.max_tiles * a.col_blocks;
             if (grid > 0x7fffffff) return INFER_KV_EINVAL;

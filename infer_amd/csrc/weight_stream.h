@@ -1,0 +1,102 @@
+// Rows of weights streamed past a few rows of activations: y[16 MT][16 RT] = x w^T for one workgroup, the steps of k dealt out to its
+// wavefronts, each of which brings its own steps to a ring in LDS and multiplies them without ever waiting for another one.
+//
+// A step is 64 elements of every row, a whole 128-byte line.  One request of a wavefront fills 1 KiB of LDS with eight rows of a step,
+// straight from memory; 16-byte unit c of row r lies at place c ^ (r % 8), so that the reads of a matrix operand meet all banks.
+// Weights carry the streaming hint, activations stay in the second-level cache.  What this is worth, 16 rows past 24576 x 4096 weights:
+// requests of 64 bytes of 16 rows straight into operand registers 52.8 us (3.8 TB/s), this 35.3 us (5.7 TB/s); a read of the weights
+// alone in lines takes 31.5 us with the hint and 33.7 without, in halves of lines 37.7.
+#pragma once
+#include "elem.h"
+
+constexpr int kStreamK = 64;                       // elements of a step
+constexpr int stream_stage_bytes(int rt, int mt) { return 2048 * (rt + mt); }
+
+// Where a lane of a request starts in the row it reads: row lane / 8 of eight, its unit of the step
+__device__ __forceinline__ int stream_row() { return (threadIdx.x & 63) >> 3; }
+__device__ __forceinline__ int stream_col() { return 8 * ((threadIdx.x & 7) ^ ((threadIdx.x & 63) >> 3)); }
+
+// w[i], x[i]: this lane's row stream_row() + 8 i of the weights and of the activations, at the first element of k (16-byte aligned);
+// k: elements, a multiple of eight; ring: D * stream_stage_bytes(RT, MT) bytes of the wavefront's own.  Adds to acc[r][t] (lane (g, n):
+// row n of tile t of x, rows 4 g + e of tile r of w) what the steps `wave`, `wave` + NW, ... contribute.
+template <int RT, int MT, int NW, int D>
+__device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT], const __bf16* const (&x)[2 * MT], int k, int wave,
+                                               unsigned char* ring, f32x4_t (&acc)[RT][MT]) {
+    constexpr int kRequests = 2 * (RT + MT), kStage = stream_stage_bytes(RT, MT);
+    static_assert(D >= 2 && D <= 4 && (D - 1) * kRequests <= 63, "requests in flight are counted in six bits");
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, col = stream_col();
+    const int all = (k + kStreamK - 1) / kStreamK, steps = all > wave ? (all - wave + NW - 1) / NW : 0;
+    const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ring);
+    // Inline assembly, since the compiler would put a wait for all requests in front of every read of LDS.  Nothing else here uses M0.
+    auto request = [&](int s, int stage) {
+        const int at = (s * NW + wave) * kStreamK + col, from = at < k ? at : 0;       // behind the end: something, which meets zeros
+#pragma unroll
+        for (int i = 0; i < kRequests; ++i) {
+            const uint32_t to = base + stage * kStage + 1024 * i;
+            if (i < 2 * RT)
+                __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(w[i < 2 * RT ? i : 0] + from), "s"(to) : "memory", "m0");
+            else
+                __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(x[i < 2 * RT ? 0 : i - 2 * RT] + from), "s"(to) : "memory", "m0");
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < steps) request(d, d);
+    const int place = 128 * n + 16 * (g ^ (n & 7));
+    int stage = 0;
+    for (int s = 0; s < steps; ++s) {
+        const int behind = steps - 1 - s;              // steps that have been requested and are not waited for: as many, at most D - 1
+        if (behind >= D - 1) __asm__ volatile("s_waitcnt vmcnt(%0)" :: "n"((D - 1) * kRequests) : "memory");
+        else if (D > 3 && behind == 2) __asm__ volatile("s_waitcnt vmcnt(%0)" :: "n"(D > 3 ? 2 * kRequests : 0) : "memory");
+        else if (D > 2 && behind == 1) __asm__ volatile("s_waitcnt vmcnt(%0)" :: "n"(D > 2 ? kRequests : 0) : "memory");
+        else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        bf16x8_t a[RT][2], b[MT][2];
+        const unsigned char* p = ring + stage * kStage;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r) a[r][h] = *reinterpret_cast<const bf16x8_t*>(p + 2048 * r + (place ^ (64 * h)));
+#pragma unroll
+            for (int t = 0; t < MT; ++t) b[t][h] = *reinterpret_cast<const bf16x8_t*>(p + 2048 * (RT + t) + (place ^ (64 * h)));
+        }
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // read before the stage is filled again
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + D < steps) request(s + D, stage);
+        const int first = (s * NW + wave) * kStreamK;
+        if (first + kStreamK > k)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (first + 32 * h + 8 * g >= k)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) b[t][h] = bf16x8_t{};
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int r = 0; r < RT; ++r) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][h], b[t][h], acc[r][t], 0, 0, 0);
+        stage = stage + 1 == D ? 0 : stage + 1;
+    }
+}
+
+// The sum of the wavefronts' parts of every tile, tile q = r * MT + t by wavefront q % NW, which gets it as f(r, t, sum) in the layout of
+// acc.  `lds` holds NW * RT * MT KiB; everybody is past its own ring.
+template <int RT, int MT, int NW, class F>
+__device__ __forceinline__ void stream_reduce(const f32x4_t (&acc)[RT][MT], int wave, unsigned char* lds, F f) {
+    f32x4_t* part = reinterpret_cast<f32x4_t*>(lds);
+    const int lane = threadIdx.x & 63;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) part[(wave * RT * MT + r * MT + t) * 64 + lane] = acc[r][t];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RT * MT; ++q) {
+        if (q % NW != wave) continue;
+        f32x4_t sum = part[q * 64 + lane];
+#pragma unroll
+        for (int v = 1; v < NW; ++v) sum += part[(v * RT * MT + q) * 64 + lane];
+        f(q / MT, q % MT, sum);
+    }
+}

@@ -491,6 +491,21 @@ def test_moe_when_all_tokens_want_the_same_expert(gpu):
     close(x, y * (p[:, 4] / p.sum(-1))[:, None], 2e-2)
 
 
+@pytest.mark.parametrize("width,ff", [(8, 8), (72, 40), (64, 128), (256, 24), (520, 200), (1024, 72)])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 32, 33, 70])
+def test_moe_rows_around_the_tiles_that_weights_stream_past(gpu, width, ff, n):
+    """All rows at one of four experts: one to three tiles of 16 and 32 rows; k of one step, of many and of parts of steps."""
+    rng, bf = np.random.default_rng(n + width), torch.bfloat16
+    s = ho.MoeShape(width, ff, 4, 1, 0, 1, 1, 1.0)
+    w = [rounded(rng.standard_normal(shape) * shape[-1] ** -0.5, bf) for shape in ((4, width), (4, 2 * ff, width), (4, width, ff))]
+    h = rounded(rng.standard_normal((n, width)), bf)
+    r = ho.moe(s, dev(h, bf), dev(w[0], bf), dev(np.array([0.0, 0.0, 3.0, 0.0])), dev(w[1], bf), dev(w[2], bf), torch.zeros(4, dtype=torch.int32, device=gpu))
+    act = silu(h @ w[1][2][:ff].T) * (h @ w[1][2][ff:].T)
+    # two roundings to bfloat16, the first of which passes through a product of unit norm
+    assert np.abs(host(r.rows)[host(r.places)[:, 0].astype(int)] - act @ w[2][2].T).max() <= 1.5e-2 * np.abs(act @ w[2][2].T).max()
+    close(r.weights, (np.exp(h @ w[0].T) / np.exp(h @ w[0].T).sum(-1, keepdims=True))[:, 2:3], 1e-5)
+
+
 def test_bad_arguments_are_refused(gpu):
     z = torch.zeros(8, 64, device=gpu)
     counts = torch.zeros(4, dtype=torch.int32, device=gpu)
