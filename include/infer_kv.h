@@ -316,6 +316,12 @@ int infer_skinny_gemm_bf16(const void* x, int64_t x_stride0, const void* w, void
 int infer_skinny_gemm_partial_bf16(const void* x, int64_t x_stride0, const void* w, void* y, int64_t y_stride0,
                                    int64_t m, int64_t n, int64_t k, void* workspace, size_t workspace_bytes,
                                    int* splits_out, void* stream);
+
+/* The first product of a SwiGLU feed-forward and its gate in one launch (MLP.py:207-226; matmul followed by silu_and_mul): w [2 ff, k] holds
+ * gate rows, then up rows; y [m, ff] = silu(x gate^T) * (x up^T) with the roundings of the two operators.  m <= 64, ff % 8 == 0,
+ * k % 128 == 0. */
+int infer_skinny_gate_silu_bf16(const void* x, int64_t x_stride0, const void* w, void* y, int64_t y_stride0, int64_t m,
+                                int64_t ff, int64_t k, void* stream);
 /* infer_rms_norm_bf16 whose input is still in pieces: x[r] = bf16(sum over s of partial[s][r]) with
  * partial[s][r] at partial + s * split_stride + r * partial_stride0 (float32 elements), added in
  * split order and rounded once - bit-identical to reducing first - then the same normalisation.

@@ -20,6 +20,9 @@
 //   buffered, 272-byte rows: conflict-free for 16-byte reads of consecutive rows) and read as B
 //   operands; every fragment read feeds both row tiles of the wavefront, which halves the LDS
 //   traffic per weight byte (LDS delivers 128 B/clk and would otherwise bound the kernel).
+//
+// That is skinny_gemm_kernel, for 65 to 128 rows.  Up to 64, skinny_stream_kernel streams the weights through LDS (weight_stream.h); its
+// wavefronts split K among themselves, so that K is cut over workgroups only where there are few of them.
 // * SK == 1: the accumulators are rounded to bf16 and stored.  SK > 1: float32 partial sums
 //   [SK][M][N] go to the workspace and `skinny_gemm_reduce_kernel` adds them and rounds once.
 #include <hip/hip_runtime.h>
@@ -28,6 +31,7 @@
 #include <type_traits>
 
 #include "../../include/infer_kv.h"
+#include "weight_stream.h"
 
 namespace {
 
@@ -53,9 +57,8 @@ struct GemmArgs {
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
-// MT = number of 16-row tiles of the batch (M <= 16 MT)
-template <int MT>
 __global__ void __launch_bounds__(256) skinny_gemm_kernel(GemmArgs a) {
+    constexpr int MT = 8;            // 16-row tiles of the batch
     __shared__ __attribute__((aligned(16))) unsigned char xs[2][16 * MT * kXRow];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -182,6 +185,64 @@ __global__ void __launch_bounds__(256) skinny_gemm_kernel(GemmArgs a) {
     }
 }
 
+__device__ __forceinline__ float round_bf16(float x) { return (float)(__bf16)x; }
+
+// 16 RT rows of weights past up to 16 MT rows of the batch, NW wavefronts with D steps each in LDS.  GATED: the weights are gate rows and as
+// many up rows, a.n / 2 each; a tile is eight gate rows and the eight up rows of the same places, and y = silu(gate) * up with the
+// roundings of storing both and reading them again.
+template <int RT, int MT, int NW, int D, bool GATED>
+__global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
+    constexpr int kRing = D * stream_stage_bytes(RT, MT), kLds = NW * (kRing > 1024 * RT * MT ? kRing : 1024 * RT * MT);
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = a.n / 2, n0 = blockIdx.x * (GATED ? 8 : 16) * RT, split = blockIdx.y;
+    const int64_t k_lo = (int64_t)split * a.chunks * kKC;
+    const __bf16* w[2 * RT];
+    const __bf16* x[2 * MT];
+#pragma unroll
+    for (int i = 0; i < 2 * RT; ++i) {
+        int row = n0 + stream_row() + 8 * (GATED ? i / 2 : i);
+        const int rows = GATED ? half : a.n;
+        row = (row < rows ? row : rows - 1) + (GATED && (i & 1) ? half : 0);
+        w[i] = (const __bf16*)a.w + (int64_t)row * a.k + k_lo;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+        const int row = stream_row() + 8 * i;
+        x[i] = (const __bf16*)a.x + (int64_t)(row < a.m ? row : a.m - 1) * a.x_stride0 + k_lo;
+    }
+    f32x4_t acc[RT][MT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    stream_product<RT, MT, NW, D>(w, x, a.chunks * kKC, wave, lds + wave * kRing, acc);
+    stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) {
+        const int row = 16 * t + n;
+        if constexpr (GATED) {                         // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
+            bf16x4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float gate = round_bf16(sum[e]), up = __shfl_xor(gate, 32, 64);
+                v[e] = (__bf16)(round_bf16(gate / (1.0f + expf(-gate))) * up);
+            }
+            const int col = n0 + 8 * r + 4 * g;
+            if (g < 2 && col < half && row < a.m) *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
+            return;
+        }
+        const int col = n0 + 16 * r + 4 * g;
+        if (col >= a.n || row >= a.m) return;          // N is a multiple of 8: a quad is in or out as a whole
+        if (a.partial) {
+            *reinterpret_cast<f32x4_t*>(a.partial + ((int64_t)split * a.m + row) * a.n + col) = sum;
+        } else {
+            bf16x4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (__bf16)sum[e];
+            *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
+        }
+    });
+}
+
 struct ReduceArgs {
     const float* partial;
     uint16_t* y; int64_t y_stride0;
@@ -206,11 +267,26 @@ __global__ void __launch_bounds__(256) skinny_gemm_reduce_kernel(ReduceArgs a) {
     *reinterpret_cast<u32x4*>(a.y + (int64_t)row * a.y_stride0 + 8 * c) = r.u;
 }
 
+// Weight rows of a workgroup.  Many rows amortise the batch, which every workgroup reads whole; few fill the chip.  Measured on weights of
+// n x 4096, us (16 / 32 / 48 / 64 / 96 rows):
+//   32 of the batch   n = 6144: - / 14.8 / 15.2 / 17.3 / 21.9    n = 12288: - / 27.5 / 19.3 / 20.9 / 24.7    n = 24576: - / 49.0 / 34.6 / 43.3 / 37.4
+//   64 of the batch   n = 6144: - / 17.2 / 19.1 / 21.8 / 27.3    n = 12288: - / 33.8 / 22.5 / 25.0 / 30.0    n = 24576: - / 58.5 / 44.6 / 49.7 / 40.3
+// so 33 to 64 want one workgroup per compute unit.  Up to 16, 16 rows are as good as any (n = 24576: 33 to 37 us), except past a
+// vocabulary, where more than 8 of the batch take 61 us (k = 1024) with 16 rows and 52 with 32.
+int rows_per_workgroup(int64_t m, int64_t n) {
+    if (m <= 16) return m > 8 && n >= 65536 ? 32 : 16;
+    if (m <= 32) return n >= 8192 ? 48 : n > 5120 ? 32 : 16;
+    if (m > 64) return kBN;
+    if (n <= 5120) return 64;                    // cut over k (choose_splits)
+    return n <= 8192 ? 32 : n > 24576 ? 80 : 16 * (int)((n + 4095) / 4096);
+}
+
 // Split-K factor: a divisor of the chunk count that brings the grid to at least one workgroup per
 // compute unit (256 on MI355X) while leaving every split at least four chunks to stream.
-int choose_splits(int64_t n, int64_t k) {
-    const int64_t tiles = (n + kBN - 1) / kBN;
+int choose_splits(int64_t m, int64_t n, int64_t k) {
+    const int64_t rows = rows_per_workgroup(m, n), tiles = (n + rows - 1) / rows;
     const int64_t chunks = k / kKC;
+    if (m <= 64 && n > 5120) return 1;          // what 180 workgroups lack of the chip is less than the sums of a split cost
     int best = 1;
     for (int s = 1; s <= 32; ++s) {
         if (chunks % s != 0 || chunks / s < 4) continue;
@@ -220,11 +296,30 @@ int choose_splits(int64_t n, int64_t k) {
     return best;
 }
 
+template <bool GATED>
+void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
+    const int rows = rows_per_workgroup(a.m, a.n);
+    const dim3 grid((unsigned)((a.n + rows - 1) / rows), (unsigned)splits);
+#define GO(RT, MT, NW, D) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED>), grid, dim3(64 * NW), 0, st, a)
+    if (a.m <= 16 && rows == 16) GO(1, 1, 4, 4);
+    else if (a.m <= 16) GO(2, 1, 4, 3);
+    else if (a.m <= 32 && rows == 16) GO(1, 2, 4, 3);
+    else if (a.m <= 32 && rows == 32) GO(2, 2, 4, 2);
+    else if (a.m <= 32) GO(3, 2, 4, 2);
+    else if (a.m <= 64 && rows == 32) GO(2, 4, 4, 2);
+    else if (a.m <= 64 && rows == 48) GO(3, 4, 4, 2);
+    else if (a.m <= 64 && rows == 64) GO(4, 4, 4, 2);
+    else if (a.m <= 64 && rows == 80) GO(5, 4, 4, 2);
+    else if (a.m <= 64) GO(6, 4, 3, 2);
+    else if constexpr (!GATED) hipLaunchKernelGGL(skinny_gemm_kernel, grid, dim3(256), 0, st, a);
+#undef GO
+}
+
 }  // namespace
 
 extern "C" size_t infer_skinny_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || m > 128 || n <= 0 || k <= 0 || k % kKC != 0) return 0;
-    const int s = choose_splits(n, k);
+    const int s = choose_splits(m, n, k);
     return s > 1 ? (size_t)s * (size_t)m * (size_t)n * sizeof(float) : 0;
 }
 
@@ -241,24 +336,19 @@ int run_gemm(const void* x, int64_t x_stride0, const void* w, void* y, int64_t y
     if (x_stride0 < k || y_stride0 < n) return INFER_KV_EINVAL;
     if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) || (x_stride0 & 7) || (y_stride0 & 7)) return INFER_KV_EALIGN;
     if (n > (1 << 24) || k > (1 << 24)) return INFER_KV_EINVAL;
-    const int splits = choose_splits(n, k);
+    const int splits = choose_splits(m, n, k);
     const size_t need = splits > 1 ? (size_t)splits * (size_t)m * (size_t)n * sizeof(float) : 0;
     if (need && (!workspace || workspace_bytes < need)) return INFER_KV_EWORKSPACE;
     if (need && ((uintptr_t)workspace & 15)) return INFER_KV_EALIGN;
     GemmArgs a{(const uint16_t*)x, x_stride0, (const uint16_t*)w, (uint16_t*)y, y_stride0,
                splits > 1 ? (float*)workspace : nullptr, (int)m, (int)n, (int)k, (int)(k / kKC / splits)};
-    const dim3 grid((unsigned)((n + kBN - 1) / kBN), (unsigned)splits);
-    hipStream_t st = (hipStream_t)stream;
-    if (m <= 16) hipLaunchKernelGGL(skinny_gemm_kernel<1>, grid, dim3(256), 0, st, a);
-    else if (m <= 32) hipLaunchKernelGGL(skinny_gemm_kernel<2>, grid, dim3(256), 0, st, a);
-    else if (m <= 64) hipLaunchKernelGGL(skinny_gemm_kernel<4>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(skinny_gemm_kernel<8>, grid, dim3(256), 0, st, a);
+    launch_stream<false>(a, splits, (hipStream_t)stream);
     int rc = (int)hipGetLastError();
     if (splits_out) *splits_out = splits;
     if (rc != 0 || splits == 1 || !reduce) return rc;
     ReduceArgs r{(const float*)workspace, (uint16_t*)y, y_stride0, (int)m, (int)n, splits};
     const int64_t items = m * (n / 8);
-    hipLaunchKernelGGL(skinny_gemm_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, r);
+    hipLaunchKernelGGL(skinny_gemm_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, (hipStream_t)stream, r);
     return (int)hipGetLastError();
 }
 }  // namespace
@@ -274,4 +364,17 @@ extern "C" int infer_skinny_gemm_partial_bf16(const void* x, int64_t x_stride0, 
                                               size_t workspace_bytes, int* splits_out, void* stream) {
     if (!splits_out) return INFER_KV_EINVAL;
     return run_gemm(x, x_stride0, w, y, y_stride0, m, n, k, workspace, workspace_bytes, false, splits_out, stream);
+}
+
+extern "C" int infer_skinny_gate_silu_bf16(const void* x, int64_t x_stride0, const void* w, void* y, int64_t y_stride0, int64_t m, int64_t ff,
+                                           int64_t k, void* stream) {
+    if (m < 0 || ff <= 0 || k <= 0) return INFER_KV_EINVAL;
+    if (m == 0) return INFER_KV_OK;
+    if (!x || !w || !y) return INFER_KV_EINVAL;
+    if (m > 64 || k % kKC != 0 || ff % 8 != 0) return INFER_KV_EUNSUPPORTED;
+    if (x_stride0 < k || y_stride0 < ff || ff > (1 << 23) || k > (1 << 24)) return INFER_KV_EINVAL;
+    if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) || (x_stride0 & 7) || (y_stride0 & 7)) return INFER_KV_EALIGN;
+    const GemmArgs a{(const uint16_t*)x, x_stride0, (const uint16_t*)w, (uint16_t*)y, y_stride0, nullptr, (int)m, (int)(2 * ff), (int)k, (int)(k / kKC)};
+    launch_stream<true>(a, 1, (hipStream_t)stream);
+    return (int)hipGetLastError();
 }

@@ -374,34 +374,47 @@ def skinny_linear_supported(m: int, n: int, k: int) -> bool:
 
 
 def _gemm_workspace(device, need: int) -> torch.Tensor | None:
-    key = str(device)
-    ws = _gemm_workspaces.get(key)
-    if need and (ws is None or ws.numel() < need):
-        if ws is not None:
-            _retired_workspaces.append(ws)
-        ws = torch.empty(max(need, 64 << 20), dtype=torch.uint8, device=device)
-        _gemm_workspaces[key] = ws
-    return ws
+    """Where split products leave their partial sums: one workspace per stream, so that calls on different streams do not meet, and one
+    for everything that is captured into graphs, which is set aside with the first one (a captured call does not allocate)."""
+    if not need:
+        return None
+    device = torch.device(device)
+    if torch.cuda.is_current_stream_capturing():
+        keys = [(str(device), "captured")]
+    else:
+        keys = [(str(device), torch.cuda.current_stream(device).cuda_stream), (str(device), "captured")]
+    for key in keys:
+        ws = _gemm_workspaces.get(key)
+        if ws is None or ws.numel() < need:
+            if ws is not None:
+                _retired_workspaces.append(ws)
+            _gemm_workspaces[key] = torch.empty(max(need, 64 << 20), dtype=torch.uint8, device=device)
+    return _gemm_workspaces[keys[0]]
 
 
 class SplitKSum:
     """Result of a split-K GEMM that has not been reduced yet: ``partial`` ``[splits, M, N]`` float32
-    lives in the shared GEMM workspace, so it must be consumed (``rms_norm`` does, ``materialize``
-    does) before the next split-K GEMM on the device runs; ``generation`` guards that."""
-    _generation: dict = {}
+    lives at the start of the stream's GEMM workspace, so it must be consumed (``rms_norm`` does, ``materialize``
+    does) before the next split-K GEMM on the stream runs; ``generation`` guards that."""
+    _generation: dict = {}          # address of a workspace -> products that were left in it
+
+    @classmethod
+    def overwritten(cls, address: int) -> int:
+        """What was left in the workspace at ``address`` is gone."""
+        cls._generation[address] = cls._generation.get(address, 0) + 1
+        return cls._generation[address]
 
     def __init__(self, partial: torch.Tensor, dtype):
         self.partial = partial
         self.dtype = dtype
-        key = str(partial.device)
-        self.generation = SplitKSum._generation[key] = SplitKSum._generation.get(key, 0) + 1
+        self.generation = SplitKSum.overwritten(partial.data_ptr())
 
     @property
     def shape(self):
         return self.partial.shape[1:]
 
     def check_alive(self):
-        if SplitKSum._generation.get(str(self.partial.device)) != self.generation:
+        if SplitKSum._generation.get(self.partial.data_ptr()) != self.generation:
             raise RuntimeError("split-K partial sums were overwritten by a later GEMM before they were consumed")
 
     def materialize(self) -> torch.Tensor:
@@ -427,7 +440,7 @@ def skinny_linear_deferred(x: torch.Tensor, weight: torch.Tensor):
         return skinny_linear(x, weight, out)
     ws = _gemm_workspace(x.device, need)
     splits = ctypes.c_int(0)
-    rc = lib.infer_skinny_gemm_partial_bf16(x.data_ptr(), x.stride(0), weight.data_ptr(), out.data_ptr(),
+    rc = lib.infer_skinny_gemm_partial_bf16(x.data_ptr(), _row_stride(x), weight.data_ptr(), out.data_ptr(),
                                             out.stride(0), m, n, k, ws.data_ptr(), ws.numel(),
                                             ctypes.byref(splits), _stream_ptr(x))
     _lib.check(rc, "skinny_linear_deferred")
@@ -440,7 +453,7 @@ def skinny_linear_deferred(x: torch.Tensor, weight: torch.Tensor):
 def skinny_linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear(x, weight)`` for ``x`` ``[M, K]`` with ``M <= 128`` (``Linear.forward``,
     ``infer/ops/MLP.py:103-149``): the weight matrix ``[N, K]`` is streamed once by a hand-written
-    split-K kernel.  The float32 workspace is cached per device and only ever grows (a captured graph
+    split-K kernel.  The float32 workspace is cached per stream and only ever grows (a captured graph
     keeps pointing at the one it was captured with, so outgrown buffers are kept alive)."""
     m, k = x.shape
     n = weight.shape[0]
@@ -454,8 +467,8 @@ def skinny_linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | Non
     need = lib.infer_skinny_gemm_workspace_bytes(m, n, k)
     ws = _gemm_workspace(x.device, need)
     if need:      # any unconsumed SplitKSum in this workspace is gone after this launch
-        SplitKSum._generation[str(x.device)] = SplitKSum._generation.get(str(x.device), 0) + 1
-    rc = lib.infer_skinny_gemm_bf16(x.data_ptr(), x.stride(0), weight.data_ptr(), out.data_ptr(), out.stride(0),
+        SplitKSum.overwritten(ws.data_ptr())
+    rc = lib.infer_skinny_gemm_bf16(x.data_ptr(), _row_stride(x), weight.data_ptr(), out.data_ptr(), out.stride(0),
                                     m, n, k, ws.data_ptr() if need else None, ws.numel() if need else 0,
                                     _stream_ptr(x))
     _lib.check(rc, "skinny_linear")
@@ -466,13 +479,24 @@ _linear_choice: dict = {}
 _linear_timings: dict = {}      # (device, batch bucket, N, K) -> (vendor ms, own ms), for inspection
 _flush_buffers: dict = {}
 
-# Weight matrices with at most this many rows go to the split-K kernel at decode batch sizes: the vendor
+# Up to this many rows of the batch the streaming kernel is ahead of the vendor GEMM on every weight matrix measured (1024 to 151936
+# rows, K of 1024 to 12288; us, vendor / streaming): 1 row 8.0 / 2.9 on 1024 x 2048, 44 / 33 on 24576 x 4096, 244 / 188 on 151936 x 4096;
+# 16 rows 7.5 / 3.9 on 4096 x 1024, 44 / 37, 254 / 214; 64 rows 49 / 40, 262 / 257.
+STREAM_MAX_BATCH = 64
+# Beyond, weight matrices with at most this many rows go to the split-K kernel: the vendor
 # GEMM has too few output tiles to fill the chip there (o_proj, down_proj: 4096 rows = 32 tiles of 128 on
 # 256 compute units, 27 and 68 us against 22 and 38), and is ahead on every wider projection measured
 # (qkv 6144, gate_up 24576, lm_head 151936 rows) and on short reductions (K below 2048).  On the three
 # published Qwen3 shapes the rule picks what a cold-cache timing of both kernels picks, within 2.5 %
 # of a decode step on the smallest.
 SKINNY_MAX_ROWS = 5120
+
+
+def _own_kernel(m: int, n: int, k: int, defer: bool) -> bool:
+    if m > STREAM_MAX_BATCH:
+        return n <= SKINNY_MAX_ROWS and k >= 2048
+    # a split over k whose pieces nobody takes has a launch more: 1024 x 2048, 48 rows 8.0 us against 8.6 (5.7 unreduced)
+    return defer or m <= 32 or n >= 2048
 
 
 def _linear_mode() -> str:
@@ -506,22 +530,37 @@ def _time_cold(fn, device, reps: int = 6) -> float:
     return times[len(times) // 2]
 
 
+def _streamable(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the kernels of this package can take the product: types, sizes, strides and alignment, and nobody wants a gradient."""
+    if x.dim() != 2 or not x.is_cuda or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.dim() != 2:
+        return False
+    m, k = x.shape
+    if not skinny_linear_supported(m, weight.shape[0], k) or weight.shape[1] != k or not weight.is_contiguous() or x.stride(1) != 1:
+        return False
+    if m > 1 and (x.stride(0) < k or x.stride(0) % 8) or x.data_ptr() % 16 or weight.data_ptr() % 16:
+        return False
+    return not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+
+
+def _row_stride(x: torch.Tensor) -> int:
+    """Elements from one row to the next; a single row has whatever stride it was made with."""
+    return x.stride(0) if x.shape[0] > 1 else x.shape[1]
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, defer: bool = False):
-    """``F.linear(x, weight)`` that sends decode-sized batches over narrow weight matrices to the split-K
-    weight-streaming kernel and everything else to the vendor GEMM.  The choice is a fixed rule on the
+    """``F.linear(x, weight)`` that sends decode-sized batches to the weight-streaming kernels (more than 64 rows: over narrow
+    weight matrices only) and everything else to the vendor GEMM.  The choice is a fixed rule on the
     shape (see ``_linear_mode`` for the alternatives), so a shape runs the same kernel, with the same
     rounding, in every process and inside and outside a captured graph."""
-    if x.dim() != 2 or not x.is_cuda or x.dtype != torch.bfloat16:
+    if not _streamable(x, weight):
         return torch.nn.functional.linear(x, weight)
     m, k = x.shape
     n = weight.shape[0]
-    if not skinny_linear_supported(m, n, k) or not weight.is_contiguous() or x.stride(1) != 1:
-        return torch.nn.functional.linear(x, weight)
     mode = _linear_mode()
     if mode == "vendor":
         return torch.nn.functional.linear(x, weight)
     if mode == "static":
-        use = n <= SKINNY_MAX_ROWS and k >= 2048
+        use = _own_kernel(m, n, k, defer)
     else:
         bucket = 16 if m <= 16 else 32 if m <= 32 else 64 if m <= 64 else 128
         key = (str(x.device), bucket, n, k)
@@ -538,3 +577,21 @@ def linear(x: torch.Tensor, weight: torch.Tensor, defer: bool = False):
         return torch.nn.functional.linear(x, weight)
     # ``defer``: the caller hands the result straight to ``rms_norm``, which adds the partial sums itself
     return skinny_linear_deferred(x, weight) if defer else skinny_linear(x, weight)
+
+
+def gate_up_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``silu_and_mul`` of ``linear(x, weight)``: ``weight`` ``[2 ff, K]`` holds gate rows, then up rows.  One launch where the streaming
+    kernel takes the product whole (few rows, no split over K), with the bits of the two."""
+    ff = weight.shape[0] // 2
+    if _streamable(x, weight) and x.shape[0] <= STREAM_MAX_BATCH and weight.shape[0] == 2 * ff and ff % 8 == 0 and _linear_mode() == "static":
+        m, k = x.shape
+        lib = _lib.load()
+        if _own_kernel(m, 2 * ff, k, False) and lib.infer_skinny_gemm_workspace_bytes(m, 2 * ff, k) == 0:
+            out = torch.empty((m, ff), dtype=x.dtype, device=x.device)
+            rc = lib.infer_skinny_gate_silu_bf16(x.data_ptr(), _row_stride(x), weight.data_ptr(), out.data_ptr(), ff, m, ff, k, _stream_ptr(x))
+            _lib.check(rc, "gate_up_silu")
+            return out
+    y = linear(x, weight)
+    out = torch.empty(y.shape[:-1] + (ff,), dtype=y.dtype, device=y.device)
+    silu_and_mul(out, y)
+    return out

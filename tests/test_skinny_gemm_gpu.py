@@ -116,3 +116,64 @@ def test_partial_sums_cannot_be_used_after_a_later_split_gemm(gpu):
     ops.skinny_linear_deferred(x, w)
     with pytest.raises(RuntimeError, match="overwritten"):
         ops.rms_norm(first, torch.ones(1024, dtype=torch.bfloat16, device=gpu), 1e-6)
+
+
+@pytest.mark.parametrize("m", [1, 7, 8, 9, 16, 17, 32, 33, 48, 64])
+@pytest.mark.parametrize("n,k", [(8, 128), (136, 256), (1024, 2048), (4096, 640), (5120, 512), (5128, 128), (6152, 384), (8200, 256), (12296, 128), (16400, 128),
+                                 (20488, 128), (24584, 256), (65544, 128)])
+def test_streamed_weights_around_tiles_and_rules(gpu, m, n, k):
+    """Small integers, whose products and sums are exact: every number of rows per workgroup, the last rows of the weights and of the
+    batch, k of one step per wavefront and fewer; unreduced sums add up to the same."""
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = torch.randint(-1, 2, (m, k + 8), generator=g, device=gpu).to(torch.bfloat16)[:, 8:]
+    w = torch.randint(-1, 2, (n, k), generator=g, device=gpu).to(torch.bfloat16)
+    want = reference(x, w)
+    assert want.abs().max() <= 256                      # representable in bf16 without rounding
+    assert torch.equal(ops.skinny_linear(x, w).float(), want)
+    deferred = ops.linear(x, w, defer=True)
+    assert torch.equal((deferred.materialize() if isinstance(deferred, ops.SplitKSum) else deferred).float(), want)
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 40, 64, 65])
+@pytest.mark.parametrize("ff,k", [(8, 128), (2568, 256), (3072, 1024), (4104, 384), (6160, 256), (10248, 128), (12288, 512)])
+def test_gate_and_up_in_one_launch_have_the_bits_of_two(gpu, m, ff, k):
+    g = torch.Generator(device=gpu).manual_seed(m + ff)
+    x = torch.randn(m, k, generator=g, device=gpu).to(torch.bfloat16)
+    w = (torch.randn(2 * ff, k, generator=g, device=gpu) * 3 * k ** -0.5).to(torch.bfloat16)
+    want = torch.empty(m, ff, dtype=torch.bfloat16, device=gpu)
+    ops.silu_and_mul(want, ops.linear(x, w))
+    got = ops.gate_up_silu(x, w)
+    # the same sums in the same order wherever both products run on the streaming kernel; otherwise a gate may round the other way
+    if torch.equal(got, want):
+        return
+    assert (got.float() - want.float()).abs().max() <= 2.0 ** -7 * want.float().abs().max()
+
+
+def test_linear_takes_what_the_streaming_kernel_cannot(gpu):
+    """Odd strides and starts, rows on top of each other, a gradient: the vendor GEMM, as before."""
+    g = torch.Generator(device=gpu).manual_seed(3)
+    w = torch.randn(512, 256, generator=g, device=gpu).to(torch.bfloat16)
+    wide = torch.randn(9, 300, generator=g, device=gpu).to(torch.bfloat16)
+    for x in (wide[:, 3:259], wide[1:2, 8:264], wide[:1, :256].expand(5, 256), wide[:, :256]):
+        close(ops.linear(x, w), reference(x, w))
+    x = wide[:, :256].contiguous().requires_grad_()
+    ops.linear(x, w).float().sum().backward()
+    assert torch.isfinite(x.grad.float()).all()
+
+
+def test_split_products_on_two_streams_do_not_meet(gpu):
+    g = torch.Generator(device=gpu).manual_seed(4)
+    x = torch.randn(8, 4096, generator=g, device=gpu).to(torch.bfloat16)
+    w = (torch.randn(1024, 4096, generator=g, device=gpu) * 0.05).to(torch.bfloat16)
+    gamma = torch.ones(1024, dtype=torch.bfloat16, device=gpu)
+    first = ops.skinny_linear_deferred(x, w)
+    want = ops.rms_norm(first, gamma, 1e-6)
+    first = ops.skinny_linear_deferred(x, w)
+    torch.cuda.synchronize()
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(other):
+        second = ops.skinny_linear_deferred(-x, w)
+        assert second.partial.data_ptr() != first.partial.data_ptr()
+        minus = ops.rms_norm(second, gamma, 1e-6)
+    other.synchronize()
+    assert torch.equal(ops.rms_norm(first, gamma, 1e-6), want) and torch.equal(minus, -want)
