@@ -16,6 +16,8 @@
 #include "elem.h"
 #include "masks.h"
 
+#include <type_traits>
+
 namespace {
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -45,6 +47,51 @@ struct DensePrefillArgs {
     float out_scale;                          // of the output
     float lambda, eps;                        // two maps: rms(o1 - lambda o2) * out_scale
 };
+
+// Results of a wavefront's queries: denominators (and the sink's), the difference of two maps and its norm, the gate.
+template <int VT, int MAPS>
+__device__ __forceinline__ void finish(const DensePrefillArgs& a, f32x4_t (&acc)[2][VT], const f32x4_t (&lacc)[2], const float (&m_neg)[2], int q_beg, int q0,
+                                       int sq, int h, int g, int n) {
+    auto store = [&](int qi, auto value) {
+        __bf16* o = a.out + (int64_t)(q_beg + qi) * a.out_stride + (int64_t)h * a.vdim + 4 * g;
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+            if (16 * t + 4 * g < a.vdim) {
+                bf16x4_t v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = (__bf16)value(t, e);
+                *reinterpret_cast<bf16x4_t*>(o + 16 * t) = v;
+            }
+    };
+    auto gate_of = [&](int qi) { return a.gate ? sigmoid_f((float)a.gate[(int64_t)(q_beg + qi) * a.gate_stride + h]) : 1.f; };
+    if constexpr (MAPS == 2) {
+        const float f0 = lacc[0][0] > 0.f ? 1.f / lacc[0][0] : 0.f, f1 = lacc[1][0] > 0.f ? -a.lambda / lacc[1][0] : 0.f;
+        float ss = 0.f;
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc[0][t][e] = acc[0][t][e] * f0 + acc[1][t][e] * f1;
+                if (16 * t + 4 * g < a.vdim) ss += acc[0][t][e] * acc[0][t][e];
+            }
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        const int qi = q0 + n;
+        if (qi >= sq) return;
+        const float f = rsqrtf(ss / (float)a.vdim + a.eps) * a.out_scale * gate_of(qi);
+        store(qi, [&](int t, int e) { return acc[0][t][e] * f; });
+    } else {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int qi = q0 + 16 * u + n;
+            if (qi >= sq) continue;
+            float l = lacc[u][0];
+            if (a.sink && l > 0.f) l += __builtin_amdgcn_exp2f(a.sink[h] * kLog2e + m_neg[u]);
+            const float f = (l > 0.f ? a.out_scale / l : 0.f) * gate_of(qi);
+            store(qi, [&](int t, int e) { return acc[u][t][e] * f; });
+        }
+    }
+}
 
 template <int KS, int VT, int MAPS>
 __global__ void __launch_bounds__(64 * kWaves, 2) dense_prefill_kernel(DensePrefillArgs a) {
@@ -236,46 +283,238 @@ __global__ void __launch_bounds__(64 * kWaves, 2) dense_prefill_kernel(DensePref
         step(s, lds, lds + kBuf, st0, st1);
         if (s + 1 < nsteps) step(s + 1, lds + kBuf, lds, st1, st0);
     }
-    if (!live) return;
-    auto store = [&](int qi, auto value) {
-        __bf16* o = a.out + (int64_t)(q_beg + qi) * a.out_stride + (int64_t)h * a.vdim + 4 * g;
+    if (live) finish<VT, MAPS>(a, acc, lacc, m_neg, q_beg, q0, sq, h, g, n);
+}
+
+// The same for keys of at most 128 entries (two maps: 64 each) without a part that all heads share, and values of 65 to 128: tiles of keys
+// and values go from memory to LDS without passing through registers, in a ring of three (a step's tile is requested two steps ahead), so
+// that three wavefronts share a vector unit.
+//
+// A tile is 32 rows of 16 chunks of 16 bytes (of the key of map m: chunks 8 m ..).  Key k of the step is row 16 ((k >> 2) & 1) + 4 (k >> 3)
+// + (k & 3), so that what one matrix operand reads is consecutive rows; a request of a wavefront fills four rows, chunk c of row r at
+// (r / 4) * kGroupB + (c / 4) * 256 + (r % 4) * 64 + (c % 4) * 16, whose pad spreads the reads over the banks.  Chunks behind the real sizes
+// repeat chunk 0: they meet zeros of the query, or are results that nobody stores.
+//
+// A score is compared with the running maximum where it already is the exponent, lane by lane; the maximum of a row, across lanes, is only
+// searched when some exponent of the wavefront exceeds kLazy.  Per score two instructions less than a search in every step.
+// 8 x 2048, 32 heads of 8 keys, gather included (us, the kernel above / this one): two maps in chunks of 2048 786 / 490, a window of 1024
+// 407 / 288, chunks of 2048 with a bias, whose maxima grow from step to step, 570 / 481.
+constexpr int kGroupB = 1024 + 32, kTileB = 2 * (kStep / 4) * kGroupB, kRing = 3;      // bytes: four rows, keys and values of a step
+
+template <int MAPS, bool BIASED>
+__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(3, 3))) dense_prefill_ring_kernel(DensePrefillArgs a) {
+    constexpr int KS = 4 / MAPS, VT = 8;
+    constexpr int kTileQ = MAPS == 2 ? 0 : 16, kWaveQ = 32 / MAPS, kWgQ = kWaveQ * kWaves;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kRing * kTileB];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, n = lane & 15;
+    const unsigned total = gridDim.x, id = blockIdx.x, die = id & 7u, per_die = total >> 3, extra = total & 7u;
+    const unsigned wg = die * per_die + (die < extra ? die : extra) + (id >> 3);
+    const int qblk = a.qblocks - 1 - (int)(wg % a.qblocks);
+    const int b = (int)((wg / a.qblocks) % a.nseq), h = (int)(wg / ((unsigned)a.qblocks * a.nseq));
+    const int q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, k_beg = a.cu_k[b], sk = a.cu_k[b + 1] - k_beg;
+    const int wq0 = qblk * kWgQ;
+    if (wq0 >= sq) return;
+    const int q0 = wq0 + kWaveQ * wave;
+    const bool live = q0 < sq;
+    const int shift = sk - sq;
+    const int last_q = wq0 + kWgQ < sq ? wq0 + kWgQ - 1 : sq - 1, nsteps = (last_q + shift + 1 + kStep - 1) / kStep;
+    const int my_last = q0 + kWaveQ - 1 < sq ? q0 + kWaveQ - 1 : sq - 1;
+    const int first_step = a.mask.first(wq0 + shift) / kStep, my_first = a.mask.first(q0 + shift) / kStep;
+    const int my_steps = live ? (my_last + shift + 1 + kStep - 1) / kStep : 0;
+    const int qk = a.dim;
+    bf16x8_t qreg[2][KS], ones;
+    const float slope = BIASED ? distance_slope(h, a.heads) * kLog2e / a.scale_log2 : 0.f;
 #pragma unroll
-        for (int t = 0; t < VT; ++t)
-            if (16 * t + 4 * g < a.vdim) {
-                bf16x4_t v;
+    for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.f;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = (__bf16)value(t, e);
-                *reinterpret_cast<bf16x4_t*>(o + 16 * t) = v;
-            }
-    };
-    auto gate_of = [&](int qi) { return a.gate ? sigmoid_f((float)a.gate[(int64_t)(q_beg + qi) * a.gate_stride + h]) : 1.f; };
-    if constexpr (MAPS == 2) {
-        const float f0 = lacc[0][0] > 0.f ? 1.f / lacc[0][0] : 0.f, f1 = lacc[1][0] > 0.f ? -a.lambda / lacc[1][0] : 0.f;
-        float ss = 0.f;                                          // values behind the real size are zero
+    for (int u = 0; u < 2; ++u) {
+        const int qi = q0 + kTileQ * u + n;
+        const __bf16* qp = a.q + (int64_t)(q_beg + (qi < sq ? qi : sq - 1)) * a.q_stride + (int64_t)(MAPS == 2 ? 2 * h + u : h) * qk + 8 * g;
 #pragma unroll
-        for (int t = 0; t < VT; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                acc[0][t][e] = acc[0][t][e] * f0 + acc[1][t][e] * f1;
-                ss += acc[0][t][e] * acc[0][t][e];
-            }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
-        const int qi = q0 + n;
-        if (qi >= sq) return;
-        const float f = rsqrtf(ss / (float)a.vdim + a.eps) * a.out_scale * gate_of(qi);
-        store(qi, [&](int t, int e) { return acc[0][t][e] * f; });
-    } else {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int qi = q0 + 16 * u + n;
-            if (qi >= sq) continue;
-            float l = lacc[u][0];
-            if (a.sink && l > 0.f) l += __builtin_amdgcn_exp2f(a.sink[h] * kLog2e + m_neg[u]);
-            const float f = (l > 0.f ? a.out_scale / l : 0.f) * gate_of(qi);
-            store(qi, [&](int t, int e) { return acc[u][t][e] * f; });
+        for (int j = 0; j < KS; ++j) {
+            qreg[u][j] = bf16x8_t{};
+            if (32 * j + 8 * g < qk) qreg[u][j] = *reinterpret_cast<const bf16x8_t*>(qp + 32 * j);
         }
     }
+
+    // Requests w, w + 4 of a wavefront are keys, the other two values; request L fills rows 4 (L % 8) .. + 3.
+    const int hk = h / a.group;
+    const unsigned char* k_at = reinterpret_cast<const unsigned char*>(a.kp + (int64_t)hk * a.kp_head + (int64_t)(k_beg + first_step * kStep) * a.kp_stride);
+    const unsigned char* v_at = reinterpret_cast<const unsigned char*>(a.v + (int64_t)hk * a.v_head + (int64_t)(k_beg + first_step * kStep) * a.v_stride);
+    const int chunk = (lane & 3) + 4 * (lane >> 4), dc = qk / 8, k_chunk = MAPS == 2 ? ((chunk & 7) < dc ? chunk & 7 : 0) + (chunk >> 3) * dc : chunk < dc ? chunk : 0;
+    const int v_chunk = chunk < a.vdim / 8 ? chunk : 0;
+    const uint32_t k_row = 2u * (uint32_t)a.kp_stride, v_row = 2u * (uint32_t)a.v_stride;       // bytes; 32 rows below 2^31 (host)
+    uint32_t to[4];
+    auto key_of = [&](int i) {                                   // of this lane's row of request i
+        const int r = 4 * (wave + 4 * i) + ((lane >> 2) & 3);
+        return (((r >> 2) & 3) << 3) | ((r >> 4) << 2) | (r & 3);
+    };
+    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        to[i] = __builtin_amdgcn_readfirstlane(base + (uint32_t)((wave + 4 * i) * kGroupB));
+        to[2 + i] = to[i] + (kStep / 4) * kGroupB;
+    }
+    const uint32_t k_off[2] = {key_of(0) * k_row + 16u * k_chunk, key_of(1) * k_row + 16u * k_chunk};
+    const uint32_t v_off[2] = {key_of(0) * v_row + 16u * v_chunk, key_of(1) * v_row + 16u * v_chunk};
+    const int whole = sk / kStep;                                // tiles in front of this index are whole
+    // Inline assembly, since the compiler would put a wait for all requests in front of every read of LDS.  Nothing else here uses M0.
+    auto request = [&](uint32_t off, const unsigned char* from, uint32_t at) {
+        __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(from), "s"(at) : "memory", "m0");
+    };
+    auto fetch = [&](int s, int ring) {
+        if (s < whole) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                request(k_off[i], k_at, to[i] + (uint32_t)ring);
+                request(v_off[i], v_at, to[2 + i] + (uint32_t)ring);
+            }
+        } else {                                                 // keys behind the last one re-read it; their weights are zero
+            const int last = sk - 1 - s * kStep;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t back = key_of(i) > last ? key_of(i) - last : 0;
+                request(k_off[i] - back * k_row, k_at, to[i] + (uint32_t)ring);
+                request(v_off[i] - back * v_row, v_at, to[2 + i] + (uint32_t)ring);
+            }
+        }
+        k_at += (int64_t)kStep * k_row;
+        v_at += (int64_t)kStep * v_row;
+    };
+    auto landed_but_newest = [&] { __builtin_amdgcn_s_waitcnt(0x0F70 | 4); };
+    auto landed_all = [&] { __builtin_amdgcn_s_waitcnt(0x0F70); };
+
+    f32x4_t acc[2][VT], lacc[2];
+    float m_neg[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        m_neg[u] = kNoMax;
+        lacc[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < VT; ++t) acc[u][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    const int k_addr = (n >> 2) * kGroupB + (n & 3) * 64 + g * 16;
+    const int v_addr = (kStep / 4) * kGroupB + g * kGroupB + (n >> 2) * 64 + ((n & 3) >> 1) * 16 + (n & 1) * 8;
+    if (nsteps > first_step) fetch(first_step, 0);               // otherwise no query of the workgroup sees a key
+    if (nsteps > first_step + 1) fetch(first_step + 1, kTileB);
+    landed_all();                                                // the query, too: the compiler knows nothing of the requests
+    __syncthreads();
+
+    // inner: a step that requests another, and whose keys everybody's queries see
+    auto step = [&](int s, auto ring_tag, auto next_tag, auto inner_tag) {
+        constexpr int ring = decltype(ring_tag)::value, ring_next = decltype(next_tag)::value;
+        constexpr bool kInner = decltype(inner_tag)::value;
+        if (kInner || s + 2 < nsteps) fetch(s + 2, ring_next);
+        if (kInner || (s >= my_first && s < my_steps)) {
+            const unsigned char* buf = lds + ring;
+            const int tok0 = s * kStep;
+            f32x4_t sc[2][2];
+            float by = slope;
+            if (BIASED) asm volatile("" : "+v"(by));             // its multiples are not kept from step to step
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                // the accumulators start at the bias of the distance
+                const float from = BIASED ? by * (float)(tok0 + 8 * g - (q0 + kTileQ * u + n + shift)) : 0.f;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sc[u][t][e] = BIASED ? __builtin_fmaf(by, (float)(4 * t + e), from) : 0.f;
+            }
+#pragma unroll
+            for (int j = 0; j < KS; ++j)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(buf + k_addr + 4 * t * kGroupB + 256 * j);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        if (MAPS == 2 && u == 1) kf = *reinterpret_cast<const bf16x8_t*>(buf + k_addr + 4 * t * kGroupB + 256 * (KS + j));
+                        sc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qreg[u][j], sc[u][t], 0, 0, 0);
+                    }
+                }
+            bf16x8_t pb[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float sv[8], x[8];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sv[4 * t + e] = sc[u][t][e];
+                if (!kInner && tok0 + kStep - 1 > q0 + kTileQ * u + shift) {      // the earliest query of the tile does not see all of it
+                    const int rel = q0 + kTileQ * u + n + shift - tok0 - 8 * g;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (i > rel) sv[i] = -INFINITY;
+                }
+                if (!kInner && tok0 < a.mask.first(q0 + kTileQ * u + 15 + shift)) {   // nor the latest one
+                    const int rel = a.mask.first(q0 + kTileQ * u + n + shift) - tok0 - 8 * g;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (i < rel) sv[i] = -INFINITY;
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(sv[i], a.scale_log2, m_neg[u]);
+                const float top = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+                if (__any(top > kLazy)) {              // always with the first key that is seen
+                    float mx = sv[0];
+#pragma unroll
+                    for (int i = 1; i < 8; ++i) mx = fmaxf(mx, sv[i]);
+                    mx = max_xor16_32(mx) * a.scale_log2;
+                    const bool grow = mx + m_neg[u] > kLazy;
+                    const float alpha = grow ? __builtin_amdgcn_exp2f(-m_neg[u] - mx) : 1.f;
+                    m_neg[u] = grow ? -mx : m_neg[u];
+                    lacc[u] *= alpha;
+#pragma unroll
+                    for (int t = 0; t < VT; ++t) acc[u][t] *= alpha;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(sv[i], a.scale_log2, m_neg[u]);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) pb[u][i] = (__bf16)__builtin_amdgcn_exp2f(x[i]);
+                lacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[u], lacc[u], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < VT; ++t) {
+                const unsigned char* src = buf + v_addr + (t >> 1) * 256 + (t & 1) * 32;
+                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)src);
+                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 4 * kGroupB));
+                const bf16x8_t vt = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, pb[u], acc[u][t], 0, 0, 0);
+            }
+        }
+        // the next tile must be in LDS for everybody: own requests first, then the barrier
+        if (kInner || s + 2 < nsteps) landed_but_newest();
+        else landed_all();
+        __syncthreads();
+    };
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, kTileB>;
+    using B2 = std::integral_constant<int, 2 * kTileB>;
+    using Inner = std::true_type;
+    using Outer = std::false_type;
+    // Steps that all queries of the workgroup see whole: behind what its last query's mask hides, in front of its first query's diagonal.
+    const int seen_from = (a.mask.first(last_q + shift) + kStep - 1) / kStep, seen_to = (wq0 + shift + 1) / kStep;
+    const bool full = wq0 + kWgQ <= sq;                          // every wavefront has queries
+    const int inner_end = !full ? 0 : nsteps - 2 < seen_to ? nsteps - 2 : seen_to;
+    int s = first_step;
+    for (; s + 2 < nsteps && s < seen_from; s += 3) {
+        step(s, B0{}, B2{}, Outer{});
+        step(s + 1, B1{}, B0{}, Outer{});
+        step(s + 2, B2{}, B1{}, Outer{});
+    }
+    for (; s + 2 < inner_end; s += 3) {
+        step(s, B0{}, B2{}, Inner{});
+        step(s + 1, B1{}, B0{}, Inner{});
+        step(s + 2, B2{}, B1{}, Inner{});
+    }
+    for (; s + 2 < nsteps; s += 3) {
+        step(s, B0{}, B2{}, Outer{});
+        step(s + 1, B1{}, B0{}, Outer{});
+        step(s + 2, B2{}, B1{}, Outer{});
+    }
+    if (s < nsteps) step(s, B0{}, B2{}, Outer{});
+    if (s + 1 < nsteps) step(s + 1, B1{}, B0{}, Outer{});
+    if (live) finish<VT, MAPS>(a, acc, lacc, m_neg, q_beg, q0, sq, h, g, n);
 }
 
 // (k-steps, value tiles) the kernel is built for, smallest first
@@ -303,9 +542,15 @@ int run(DensePrefillArgs& a, int64_t num_seqs, int64_t max_seqlen_q, float scale
     a.scale_log2 = scale * kLog2e;
     hipStream_t st = (hipStream_t)stream;
     const unsigned grid = (unsigned)total;
+    // Smaller values leave half of a ring's tile empty, wider keys do not fit it, and parts that heads share come from two places.
+    if (a.rot == 0 && a.vdim > 64 && qk <= 128 / maps) {
+        if (maps == 2) hipLaunchKernelGGL((dense_prefill_ring_kernel<2, false>), dim3(grid), dim3(64 * kWaves), 0, st, a);
+        else if (a.biased) hipLaunchKernelGGL((dense_prefill_ring_kernel<1, true>), dim3(grid), dim3(64 * kWaves), 0, st, a);
+        else hipLaunchKernelGGL((dense_prefill_ring_kernel<1, false>), dim3(grid), dim3(64 * kWaves), 0, st, a);
+        return (int)hipGetLastError();
+    }
     if (maps == 2) {
         if (qk <= 64 && a.vdim <= 64) return go<2, 4, 2>(a, grid, st);
-        if (qk <= 64) return go<2, 8, 2>(a, grid, st);
         return go<4, 8, 2>(a, grid, st);
     }
     if (qk <= 64 && a.vdim <= 64) return go<2, 4>(a, grid, st);

@@ -272,6 +272,35 @@ def test_masked_prefill(gpu, heads, kv_heads, dim, vdim, maps, mask, size):
         close(out, want.reshape(total, -1), 2e-2)
 
 
+@pytest.mark.parametrize("dim,vdim,maps", [(128, 128, 1), (8, 72, 1), (72, 120, 1), (120, 128, 1), (64, 128, 2), (40, 72, 2), (8, 96, 2)])
+@pytest.mark.parametrize("mask,size", [(None, 1), ("window", 40), ("window", 64), ("window", 97), ("chunk", 32), ("chunk", 50), ("chunk", 160)])
+def test_masked_prefill_around_the_steps_of_the_ring(gpu, dim, vdim, maps, mask, size):
+    """Sequences of one to ten steps of 32 keys that end in, at and behind a step, new in whole or behind a prefix, so that a workgroup has
+    one, two, three and more steps, with and without steps that all its queries see.  Weights are rounded to bf16 in front of the product
+    with the values (2^-8 of the sum of |weight x value| at most), the result once more: 2e-2 as in the test above."""
+    rng, bf, heads, kv_heads = np.random.default_rng(dim + vdim + size), torch.bfloat16, 2, 1
+    s = ho.MaskedShape(heads, kv_heads, dim, vdim, 0.5 * dim ** -0.5, maps=maps, mask=mask, mask_size=size, distance_bias=maps == 1 and size != 97,
+                       out_scale=0.6, lam=0.7, eps=1e-3)
+    lens, new = [1, 31, 32, 33, 65, 96, 128, 129, 200, 300], [1, 31, 32, 33, 1, 96, 128, 129, 17, 170]
+    p = Pages(rng, lens, s, 64, bf)
+    seqs = list(range(len(lens)))
+    cu_q, cu_k = np.cumsum([0] + new), np.cumsum([0] + lens)
+    q = np.concatenate([np.stack([standing_out(rng, s, p, i, lens[i] - new[i] + t, bf, lens) if t % 3 else rounded(
+        rng.standard_normal((heads, maps, dim)), bf) for t in range(new[i])]) for i in seqs])
+    cu = dev(cu_q, torch.int32), dev(cu_k, torch.int32)
+    rows = ho.masked_gather(s, p.cache, p.tables, dev(seqs, torch.int32), *cu, int(cu_k[-1]), max(lens))
+    sink = rng.standard_normal(heads) * 3 if maps == 1 else None
+    out = torch.full((int(cu_q[-1]) + 1, heads * vdim), 9.0, dtype=bf, device=gpu)
+    ho.masked_prefill(s, dev(q.reshape(len(q), -1), bf), rows, out[:-1], *cu, max(new), None if sink is None else dev(sink), None)
+    want = np.zeros((len(q), heads, vdim))
+    for i in seqs:
+        for t in range(new[i]):
+            want[cu_q[i] + t] = one_query(s, q[cu_q[i] + t], p.k[i], p.v[i], lens[i] - new[i] + t,
+                                          np.full(heads, -np.inf) if sink is None else sink, np.full(heads, np.inf))
+    close(out[:-1], want.reshape(len(q), -1), 2e-2)
+    assert (out[-1] == 9.0).all()
+
+
 # ------------------------------------------------------------------ state space
 class Ssm:
     """Random weights of a layer, and sequences that are fed to it in portions."""
