@@ -301,6 +301,25 @@ def test_masked_prefill_around_the_steps_of_the_ring(gpu, dim, vdim, maps, mask,
     assert (out[-1] == 9.0).all()
 
 
+@pytest.mark.parametrize("maps,dim,vdim,mask,size", [(1, 64, 128, None, 1), (2, 64, 128, "chunk", 100), (1, 24, 16, "window", 500), (1, 64, 80, "window", 70)])
+def test_masked_prefill_of_more_workgroups_than_run_at_once(gpu, maps, dim, vdim, mask, size):
+    """More than 1024 workgroups: their blocks go by place over the sequences (a window that ends before the sequences: by sequence)."""
+    rng, bf, heads = np.random.default_rng(dim + vdim), torch.bfloat16, 32
+    s = ho.MaskedShape(heads, 4, dim, vdim, 0.5 * dim ** -0.5, maps=maps, mask=mask, mask_size=size, distance_bias=False, out_scale=0.6, lam=0.7, eps=1e-3)
+    lens = [5, 16, 1, 290, 40, 3, 130, 2, 9, 12, 4]
+    p = Pages(rng, lens, s, 64, bf)
+    cu_n = np.cumsum([0] + lens)
+    cu = dev(cu_n, torch.int32)
+    q = rounded(rng.standard_normal((int(cu_n[-1]), heads, maps, dim)), bf)
+    rows = ho.masked_gather(s, p.cache, p.tables, dev(list(range(len(lens))), torch.int32), cu, cu, int(cu_n[-1]), max(lens))
+    out = torch.empty((len(q), heads * vdim), dtype=bf, device=gpu)
+    assert len(lens) * heads * -(-max(lens) // (128 // maps)) > 1024
+    ho.masked_prefill(s, dev(q.reshape(len(q), -1), bf), rows, out, cu, cu, max(lens), None, None)
+    want = np.stack([one_query(s, q[cu_n[i] + t], p.k[i], p.v[i], t, np.full(heads, -np.inf), np.full(heads, np.inf))
+                     for i in range(len(lens)) for t in range(lens[i])])
+    close(out, want.reshape(len(q), -1), 2e-2)
+
+
 # ------------------------------------------------------------------ state space
 class Ssm:
     """Random weights of a layer, and sequences that are fed to it in portions."""
