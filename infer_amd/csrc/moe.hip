@@ -238,7 +238,7 @@ struct ScatterArgs {
     int32_t* places;                       // [choices]
     int32_t* row_token; int32_t* row_expert;           // [place]
     int32_t* offsets;                      // [experts + 1]
-    int32_t* tiles;                        // [max_tiles][2]: expert (-1: none), first row inside the expert
+    int32_t* tiles;                        // [max_tiles][2]: expert, first row inside the expert; behind the last: -1, number of tiles
 };
 
 // exclusive prefix sum over the workgroup
@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(kThreads) moe_scatter_kernel(ScatterArgs a) {
         int total = 0;
         for (int i = 0; i < 4; ++i) total += part[1][i];
         // part[1] holds every wavefront's number of tiles
-        for (int t = total + tid; t < a.max_tiles; t += kThreads) a.tiles[2 * t] = -1;
+        for (int t = total + tid; t < a.max_tiles; t += kThreads) a.tiles[2 * t] = -1, a.tiles[2 * t + 1] = total;
     }
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * kThreads + tid;
@@ -430,44 +430,59 @@ __global__ void __launch_bounds__(kThreads, 2) moe_tile_kernel(GemmArgs<__bf16> 
     }
 }
 
-// A workgroup of eight wavefronts: 256 rows of one expert x 256 rows of W (GATED: 128 gate rows and the same 128 up rows), k in steps
-// of 64 (a multiple of which k is) through two LDS buffers that are filled from memory without passing through registers: the
-// requests of the next step travel while this one is consumed.  Wavefront (wm, wn) has 128 rows x 64 rows of W as 8 x 4 tiles.
+// A workgroup of four wavefronts: 256 rows of one expert x 256 rows of W (GATED: 128 gate rows and the same 128 up rows), k in steps
+// of 64 (a multiple of which k is) through LDS buffers that are filled from memory without passing through registers.  Wavefront
+// (wm, wn) has 128 rows x 128 rows of W as 8 x 8 tiles: one wavefront on a vector unit, with all of its registers.
+//
+// A step is two phases of 64 products each.  While the operands of one phase are multiplied, those of the next are read from LDS, and the
+// reads and the requests are spread over the products, so that the matrix units wait for neither.  One barrier a step, between the
+// phases: in front of it a wavefront has read the last of the step's buffers and its requests of the next step have landed; behind it
+// the step's buffers are free for requests: rows two steps ahead go to them in the second phase, W two steps ahead went to the third of its
+// buffers in the first (W comes from farther away, and requests in one phase alone are as many as a compute unit can issue in it).
+//
+// 8000 rows, three of 14 experts of 3072 x 4096 and two that return their row: 1015 + 560 us with eight wavefronts of 128 x 64 that read 1.5
+// times as much of LDS and issued a step's requests and reads in front of its products, 870 + 490 us now (1.2 PFLOP/s; products alone, without
+// reads and requests, 0.92 of it).  16000 rows 3010 -> 2690 us in all.
+//
 // A row of a buffer is eight units of 16 bytes, unit c at place c ^ (row % 8), so that reads of a column meet all banks.
-constexpr int kBlockRows = 256, kBlockThreads = 512;
-// (tiles, column blocks) that one die works on at a time: as many as it has compute units, and as square as column blocks of 256 allow
-constexpr int kPatchTiles = 4, kPatchCols = 8, kPatch = kPatchTiles * kPatchCols;
+constexpr int kBlockRows = 256, kBlockThreads = 256;
+// Tiles of an expert that are worked on side by side: a die's compute units then share that many blocks of rows and 32 / kSideTiles of W.
+constexpr int kSideTiles = 8;
 template <bool GATED>
-__global__ void __launch_bounds__(kBlockThreads, 2) moe_block_kernel(GemmArgs<__bf16> a) {
-    constexpr int kMat = kBlockRows * 128, kBuf = 2 * kMat;      // bytes
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kBuf];
+__global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) moe_block_kernel(GemmArgs<__bf16> a) {
+    constexpr int kMat = kBlockRows * 128;                       // bytes
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[5 * kMat];   // three buffers of W, two of rows
     if (a.zero && blockIdx.x == 0)
         for (int i = threadIdx.x; i < a.num_zero; i += kBlockThreads) a.zero[i] = 0;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // workgroups go to the eight dies round-robin, and so do the patches
-    const unsigned seq = blockIdx.x >> 3, patch = seq / kPatch * 8u + (blockIdx.x & 7u), in_patch = seq % kPatch;
-    const unsigned across = (unsigned)(a.col_blocks + kPatchCols - 1) / kPatchCols;
-    const int tile = (int)(patch / across * kPatchTiles + in_patch % kPatchTiles);
-    const int cb = (int)(patch % across * kPatchCols + in_patch / kPatchTiles);
-    if (tile >= a.max_tiles || cb >= a.col_blocks) return;
-    const int expert = a.tiles[2 * tile];
+    // Workgroups go to the eight dies round-robin, and each die gets a contiguous run of (expert, group of tiles, columns, tile): those that
+    // run at the same time share rows and weights of one expert.  Behind the tiles there are, their number stands (scatter kernel).
+    const int none = a.tiles[2 * a.max_tiles - 2] < 0, total = none ? a.tiles[2 * a.max_tiles - 1] : a.max_tiles;
+    const unsigned columns = (unsigned)a.col_blocks, units = (unsigned)total * columns, die = blockIdx.x & 7u, extra = units & 7u;
+    if ((blockIdx.x >> 3) >= units / 8 + (die < extra ? 1 : 0)) return;
+    const unsigned unit = die * (units / 8) + (die < extra ? die : extra) + (blockIdx.x >> 3);
+    const int some = (int)(unit / columns);                      // a tile of the unit's expert
+    const int expert = a.tiles[2 * some];
     if (expert < 0 || expert >= a.experts) return;
-    const int first = a.offsets[expert] + a.tiles[2 * tile + 1], end = a.offsets[expert + 1];
+    const int row0 = a.offsets[expert], end = a.offsets[expert + 1], tile0 = some - a.tiles[2 * some + 1] / kBlockRows;
+    const unsigned tiles = (unsigned)(end - row0 + kBlockRows - 1) / kBlockRows, groups = (tiles + kSideTiles - 1) / kSideTiles;
+    const unsigned side = (tiles + groups - 1) / groups, of_expert = unit - (unsigned)tile0 * columns, group = of_expert / (side * columns);
+    const unsigned here = tiles - group * side < side ? tiles - group * side : side, rest = of_expert - group * side * columns;
+    const int cb = (int)(rest / here), first = row0 + kBlockRows * (int)(group * side + rest % here);
     const int rows = end - first < kBlockRows ? end - first : kBlockRows;
     const int c0 = cb * (GATED ? 128 : 256);
-    // load i of a wavefront fills rows 8 (4 wave + i) .. + 7: lane l place l % 8 of row l / 8
-    uint32_t x_off[4], w_off[4], to[4];                          // bytes (checked on the host to fit)
-    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+    // load i of a wavefront fills rows 8 (8 wave + i) .. + 7: lane l place l % 8 of row l / 8
+    uint32_t x_off[8], w_off[8];                                 // bytes (checked on the host to fit)
+    const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(8192 * wave));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = 8 * (4 * wave + i) + (lane >> 3), unit = (lane & 7) ^ (lane >> 3);
+    for (int i = 0; i < 8; ++i) {
+        const int r = 8 * (8 * wave + i) + (lane >> 3), unit = (lane & 7) ^ (lane >> 3);
         const int xr = first + (r < rows ? r : rows - 1);
         x_off[i] = 2u * ((uint32_t)(a.row_token ? a.row_token[xr] : xr) * (uint32_t)a.x_stride + 8u * unit);
         int col = GATED ? c0 + 32 * (r >> 6) + (r & 31) : c0 + r;
         col = col < a.cols ? col : a.cols - 1;
         w_off[i] = 2u * ((uint32_t)(GATED && (r & 32) ? a.up_row + col : col) * (uint32_t)a.w_stride + 8u * unit);
-        to[i] = __builtin_amdgcn_readfirstlane(base + (uint32_t)(1024 * (4 * wave + i)));
     }
     const __bf16* xs = a.x;
     const __bf16* ws = a.w + (int64_t)expert * a.w_expert;
@@ -475,45 +490,95 @@ __global__ void __launch_bounds__(kBlockThreads, 2) moe_block_kernel(GemmArgs<__
     auto request = [&](uint32_t off, const __bf16* from, uint32_t at) {
         __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(from), "s"(at) : "memory", "m0");
     };
-    auto fetch = [&](int s, uint32_t buf) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            request(x_off[i], xs + 64 * s, to[i] + buf);
-            request(w_off[i], ws + 64 * s, to[i] + buf + kMat);
-        }
-    };
+    auto fetch_x = [&](int i, int s) { request(x_off[i], xs + 64 * s, to + (uint32_t)(3 + (s & 1)) * kMat + 1024u * i); };
+    auto fetch_w = [&](int i, int s, uint32_t buf) { request(w_off[i], ws + 64 * s, to + buf + 1024u * i); };
     const int wm = wave & 1, wn = wave >> 1;
-    const bool live = 128 * wm < rows;
-    f32x4_t acc[4][8];                                           // [tile of W][tile of rows]
+    f32x4_t acc[8][8];                                           // [tile of W][tile of rows]
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const int steps = a.k / 64;
-    fetch(0, 0);
-    const int unit0 = n * 128 + 16 * (g ^ (n & 7));
-    for (int s = 0; s < steps; ++s) {
-        // this wavefront's requests have landed; behind the barrier everybody's have, and nobody reads the other buffer any more
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        if (s + 1 < steps) fetch(s + 1, (uint32_t)((s + 1) & 1) * kBuf);
-        if (!live) continue;
-        const unsigned char* xb = lds + (s & 1) * kBuf + 128 * 128 * wm;
-        const unsigned char* wb = lds + (s & 1) * kBuf + kMat + 64 * 128 * wn;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int at = unit0 ^ (64 * k);
-            bf16x8_t xf[8], wf[4];
+    for (int i = 0; i < 8; ++i) fetch_w(i, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) wf[i] = *reinterpret_cast<const bf16x8_t*>(wb + at + 2048 * i);
+    for (int i = 0; i < 8; ++i) fetch_x(i, 0);
+    if (steps > 1) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) xf[j] = *reinterpret_cast<const bf16x8_t*>(xb + at + 2048 * j);
+        for (int i = 0; i < 8; ++i) fetch_w(i, 1, kMat);
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
-        }
+        for (int i = 0; i < 8; ++i) fetch_x(i, 1);
     }
+    if (steps > 1) __builtin_amdgcn_s_waitcnt(0x4F70);           // step 0 has landed: 16 requests at most are under way
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    bf16x8_t xf[2][8], wf[2][8];
+    const unsigned char* xl = lds + 3 * kMat + 128 * 128 * wm + n * 128 + 16 * (g ^ (n & 7));
+    const unsigned char* wl = lds + 128 * 128 * wn + n * 128 + 16 * (g ^ (n & 7));
+    const int flip = 64 - 2 * (16 * (g ^ (n & 7)) & 64);         // from the unit of the first phase to that of the second
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        wf[0][i] = *reinterpret_cast<const bf16x8_t*>(wl + 2048 * i);
+        xf[0][i] = *reinterpret_cast<const bf16x8_t*>(xl + 2048 * i);
+    }
+    // In place by assembly: all accumulation registers are taken, and the compiler, which moves results around, has none to move them through.
+    auto product = [](f32x4_t& c, const bf16x8_t& w, const bf16x8_t& x) {
+        __asm__ volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
+    };
+    // 64 products, with `aux(i)`, i < 32, behind two each
+    auto phase = [&](const bf16x8_t (&w)[8], const bf16x8_t (&x)[8], auto aux) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                product(acc[i][j], w[i], x[j]);
+                product(acc[i][j + 1], w[i], x[j + 1]);
+                aux(4 * i + j / 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+    auto read = [&](bf16x8_t (&w)[8], bf16x8_t (&x)[8], const unsigned char* wb, const unsigned char* xb, int i) {
+        if (i < 8) x[i] = *reinterpret_cast<const bf16x8_t*>(xb + 2048 * i);
+        else if (i < 16) w[i - 8] = *reinterpret_cast<const bf16x8_t*>(wb + 2048 * (i - 8));
+    };
+    uint32_t at_w = 0, far_w = 2 * kMat;                         // buffers of W of this step and of the one after the next
+    auto step = [&](int s, auto inner_tag) {
+        constexpr bool kInner = decltype(inner_tag)::value;      // a step with two more behind it
+        const unsigned char* xb = xl + (s & 1) * kMat;
+        const unsigned char* wb = wl + at_w;
+        phase(wf[0], xf[0], [&](int i) {
+            if (kInner || s + 2 < steps)
+                if (i % 4 == 3) fetch_w(i / 4, s + 2, far_w);
+            read(wf[1], xf[1], wb + flip, xb + flip, i);
+        });
+        far_w = at_w;
+        at_w = at_w == 2 * kMat ? 0 : at_w + kMat;
+        const bool more = kInner || s + 1 < steps;
+        if (more) {
+            if (kInner || s + 2 < steps) __builtin_amdgcn_s_waitcnt(0x0070 | 8);
+            else __builtin_amdgcn_s_waitcnt(0x0070);
+            __syncthreads();
+        }
+        xb = xl + ((s + 1) & 1) * kMat;
+        wb = wl + at_w;
+        phase(wf[1], xf[1], [&](int i) {
+            if (kInner || s + 2 < steps)
+                if (i % 4 == 3) fetch_x(i / 4, s + 2);
+            if (more) read(wf[0], xf[0], wb, xb, i);
+        });
+    };
+    auto settle = [&] {                                          // of accumulators: what is in front of this and behind it stays there
+#pragma unroll
+        for (int i = 0; i < 64; ++i) __asm__ volatile("" : "+a"(acc[i >> 3][i & 7]));
+        __asm__ volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+        for (int i = 0; i < 64; ++i) __asm__ volatile("" : "+a"(acc[i >> 3][i & 7]));
+    };
+    settle();
+    int s = 0;
+    for (; s + 2 < steps; ++s) step(s, std::true_type{});
+    for (; s < steps; ++s) step(s, std::false_type{});
+    settle();
     // lane (g, n): row n of a row tile, columns 4 g + e
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -521,13 +586,14 @@ __global__ void __launch_bounds__(kBlockThreads, 2) moe_block_kernel(GemmArgs<__
         if (r >= rows) continue;
         __bf16* o = a.out + (int64_t)(first + r) * a.out_stride;
 #pragma unroll
-        for (int i = 0; i < (GATED ? 2 : 4); ++i) {
-            const int c = c0 + (GATED ? 32 : 64) * wn + 16 * i + 4 * g;
+        for (int i = 0; i < 8; ++i) {
+            if (GATED && (i & 2)) continue;
+            const int c = c0 + (GATED ? 64 * wn + 32 * (i >> 2) + 16 * (i & 1) : 128 * wn + 16 * i) + 4 * g;
             bf16x4_t v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float x = acc[i][j][e];
-                if constexpr (GATED) x = silu_f(x) * acc[i + 2][j][e];
+                if constexpr (GATED) x = silu_f(x) * acc[(i + 2) & 7][j][e];
                 v[e] = (__bf16)(c + e < a.cols ? x : 0.f);
             }
             if (c + 4 <= a.out_cols) *reinterpret_cast<bf16x4_t*>(o + c) = v;       // out_cols is a multiple of eight
@@ -627,8 +693,7 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t max_places, hipStrea
     if constexpr (sizeof(T) == 2) {
         if (tile_rows == kBlockRows) {
             a.col_blocks = (a.out_cols + (gated ? 127 : 255)) / (gated ? 128 : 256);
-            const int64_t patches = (int64_t)((a.max_tiles + kPatchTiles - 1) / kPatchTiles) * ((a.col_blocks + kPatchCols - 1) / kPatchCols);
-            grid = (patches + 7) / 8 * 8 * kPatch;
+            grid = ((int64_t)a.max_tiles * a.col_blocks + 7) / 8 * 8;
             if (grid > 0x7fffffff) return INFER_KV_EINVAL;
             if (gated) hipLaunchKernelGGL((moe_block_kernel<true>), dim3((unsigned)grid), dim3(kBlockThreads), 0, st, a);
             else hipLaunchKernelGGL((moe_block_kernel<false>), dim3((unsigned)grid), dim3(kBlockThreads), 0, st, a);
@@ -661,10 +726,13 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t max_places, hipStrea
 int rows_per_tile(int elem, int64_t n, int64_t width, int64_t ff_pad, int64_t experts, int64_t top) {
     if (elem != INFER_ELEM_BF16 || width % 8 || ff_pad % 8) return 0;
     if (n * top <= 24 * experts) return kSmallRows;
-    // large blocks pay when most of them are full; their offsets are 32 bits
+    // Large blocks pay where they are enough to fill most of the chip, and where an expert has more rows than its weights' way from memory
+    // takes anyway (of 14 experts, tiles of 128 rows / blocks, us: 3072 x 4096, 118 rows 284 / 302, 200 319 / 295, 800 471 / 322, 2100 879 / 510;
+    // 768 x 1024, 600 rows 57 / 66, 1200 67 / 71, 2300 104 / 81).  Their offsets are 32 bits.
     const int64_t far = 1ll << 31;
     const bool fits = width % 64 == 0 && ff_pad % 64 == 0 && n * width < far && n * top * ff_pad < far && 2 * ff_pad * width < far;
-    return fits && n * top >= 512 * experts ? kBlockRows : kBigRows;
+    const int64_t blocks = (n * top / kBlockRows + experts / 2) * ((ff_pad + 127) / 128);      // of the first product, about
+    return fits && (n * top >= 512 * experts || (n * top >= 32 * experts && blocks >= 160)) ? kBlockRows : kBigRows;
 }
 
 }  // namespace

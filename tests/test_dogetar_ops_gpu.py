@@ -539,6 +539,32 @@ def test_moe_when_all_tokens_want_the_same_expert(gpu):
     close(x, y * (p[:, 4] / p.sum(-1))[:, None], 2e-2)
 
 
+@pytest.mark.parametrize("width,ff,experts,n", [(256, 64, 5, 2600), (64, 5120, 8, 300), (448, 384, 1, 4700)])
+def test_moe_blocks_of_uneven_experts(gpu, width, ff, experts, n):
+    """Blocks of 256 rows: nearly all rows at one expert, in one and more groups of its tiles; few rows and many columns; one to seven steps.
+    Inner results are rounded to bf16, sums of up to 5120 products of theirs to bf16 once more: 2e-2 as for the other kernels."""
+    rng, bf = np.random.default_rng(ff), torch.bfloat16
+    s = ho.MoeShape(width, ff, experts, 1, 0, 1, 1, 1.0)
+    router, correction = rounded(rng.standard_normal((experts, width)) * 2 * width ** -0.5, bf), np.where(np.arange(experts) == experts // 2, 1.0, 0.0)
+    w = [rounded(rng.standard_normal(shape) * shape[-1] ** -0.5, bf) for shape in ((experts, 2 * ff, width), (experts, width, ff))]
+    h = rounded(rng.standard_normal((2 * n, width)), bf)
+    p = np.exp(h @ router.T)
+    p /= p.sum(-1, keepdims=True)
+    order = np.sort(p + correction, -1)
+    clear = np.ones(2 * n, bool) if experts == 1 else order[:, -1] - order[:, -2] > 2e-3
+    h, p = h[clear][:n], p[clear][:n]
+    assert len(h) == n
+    r = ho.moe(s, dev(h, bf), dev(router, bf), dev(correction), dev(w[0], bf), dev(w[1], bf), torch.zeros(experts, dtype=torch.int32, device=gpu))
+    x = torch.zeros((n, width), device=gpu)
+    ho.pre_norm(x, torch.ones(width, device=gpu), 1e-6, y=r)
+    chosen, want = (p + correction).argmax(-1), np.zeros((n, width))
+    for e in range(experts):
+        at = chosen == e
+        inner = silu(h[at] @ w[0][e][:ff].T) * (h[at] @ w[0][e][ff:].T)
+        want[at] = inner @ w[1][e].T * p[at, e][:, None]
+    close(x, want, 2e-2)
+
+
 @pytest.mark.parametrize("width,ff", [(8, 8), (72, 40), (64, 128), (256, 24), (520, 200), (1024, 72)])
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 32, 33, 70])
 def test_moe_rows_around_the_tiles_that_weights_stream_past(gpu, width, ff, n):
