@@ -22,7 +22,10 @@ _retired_workspaces: list = []      # outgrown workspaces stay alive: captured g
 
 
 def _stream_ptr(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The handle of the calling thread's current stream on the tensor's device.  Without the Stream object around it: 0.2 instead of
+    2 us, of the 21 that a decode call of a few short sequences took."""
+    device = t.get_device()
+    return torch._C._cuda_getCurrentRawStream(device) if device >= 0 else torch.cuda.current_stream(t.device).cuda_stream   # the latter raises
 
 
 def _require_gpu(*tensors):
@@ -127,7 +130,7 @@ def decode_workspace(device, max_batch: int, num_q_heads: int, num_kv_heads: int
     return ws[1]
 
 
-_workspace_streams: dict = {}      # data_ptr of a shared workspace -> the stream that used it last
+_workspace_streams: dict = {}      # data_ptr of a shared workspace -> the stream that used it last: (handle, Stream)
 
 
 def _claim_shared_workspace(workspace: torch.Tensor, device) -> None:
@@ -135,24 +138,28 @@ def _claim_shared_workspace(workspace: torch.Tensor, device) -> None:
     that use it must be ordered on one stream.  A call on another stream while the last one still has work
     pending is refused (a host-side check on a change of stream only; streams under capture are not
     queried): pass ``workspace=`` of its own to such a call."""
-    cur = torch.cuda.current_stream(device)
-    last = _workspace_streams.get(workspace.data_ptr())
-    if last is not None and last != cur and not torch.cuda.is_current_stream_capturing() and not last.query():
+    handle, key = _stream_ptr(workspace), workspace.data_ptr()
+    last = _workspace_streams.get(key)
+    if last is not None and last[0] == handle:
+        return
+    if last is not None and not torch.cuda.is_current_stream_capturing() and not last[1].query():
         raise RuntimeError("paged decode: the shared workspace is still in use on another stream; "
                            "order the calls on one stream or pass a workspace of their own")
-    _workspace_streams[workspace.data_ptr()] = cur
+    _workspace_streams[key] = (handle, torch.cuda.current_stream(device))
 
 
 def _decode_args(q3, k_cache, v_cache, cache_seqlens, block_table):
-    assert q3.dtype == torch.bfloat16 and k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16
+    bf16, i32 = torch.bfloat16, torch.int32
+    assert q3.dtype == bf16 and k_cache.dtype == bf16 and v_cache.dtype == bf16
     uniform = isinstance(cache_seqlens, int)      # one length for the whole batch, known on the host
-    assert block_table.dtype == torch.int32 and (uniform or cache_seqlens.dtype == torch.int32)
-    assert k_cache.dim() == 4 and k_cache.shape == v_cache.shape
-    assert k_cache.stride() == v_cache.stride()
+    assert block_table.dtype == i32 and (uniform or cache_seqlens.dtype == i32)
+    shape, strides, qs = k_cache.shape, k_cache.stride(), q3.stride()
+    assert len(shape) == 4 and shape == v_cache.shape
+    assert strides == v_cache.stride()
     b, hq, d = q3.shape
-    nblk, bs, hkv, dk = k_cache.shape
-    assert dk == d and q3.stride(2) == 1 and q3.stride(1) == d
-    assert k_cache.stride(3) == 1 and k_cache.stride(2) == d
+    nblk, bs, hkv, dk = shape
+    assert dk == d and qs[2] == 1 and qs[1] == d
+    assert strides[3] == 1 and strides[2] == d
     assert cache_seqlens >= 0 if uniform else (cache_seqlens.numel() == b and cache_seqlens.is_contiguous())
     assert block_table.dim() == 2 and block_table.shape[0] == b and block_table.shape[1] >= 1
     assert block_table.stride(1) == 1
@@ -224,8 +231,8 @@ def flash_attn_with_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     assert q.dim() == 4 and q.shape[1] == 1, "decode takes one query token per sequence"
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** -0.5
-    q3 = q[:, 0]
-    out = torch.empty((q.shape[0], q.shape[2], q.shape[3]), dtype=q.dtype, device=q.device)
+    q3 = q.select(1, 0)
+    out = q.new_empty(q3.shape)
     paged_attn_decode(q3, k_cache, v_cache, block_table, cache_seqlens, softmax_scale, out)
     return out.unsqueeze(1)
 
