@@ -39,7 +39,7 @@ struct TalkPrefillArgs {
     int key_pad, vdim_pad;
     const int32_t* bt; int64_t bt_stride; int table_cols, block_size, num_blocks;
     const int32_t* seqs; const int32_t* cu_q; const int32_t* cu_k;
-    int heads, kv_heads, dim, vdim, nseq, qblocks;
+    int heads, kv_heads, dim, vdim, nseq, qblocks, run;
     float scale_log2;
     const __bf16* talk;                   // [heads][heads]
     float out_scale;
@@ -79,13 +79,28 @@ struct PageWalk {
     }
 };
 
-// Workgroups go to the eight dies round-robin.  A die works on its own share of `pairs`, on the late query blocks, which see the most
-// keys, first.  False: no such pair.
-__device__ __forceinline__ bool place_of_block(unsigned id, int pairs, int qblocks, int& pair, int& qblk) {
-    const int die = (int)(id & 7u), i = (int)(id >> 3), per_die = (pairs + 7) / 8;
-    pair = die * per_die + i % per_die;
-    qblk = qblocks - 1 - i / per_die;
-    return pair < pairs;
+// How query blocks of pairs, late ones, which see the most keys, first, go to the dies; workgroups go to them round-robin.
+constexpr int kShares = 0;       // a die works on its own share of the pairs
+constexpr int kSpread = -1;      // all pairs of a row of blocks one behind the other
+// run > 0: `run` neighbouring blocks of a pair go to one die, the runs of all pairs in turn; the pairs turn from row to row.
+// False: no such block.
+__device__ __forceinline__ bool place_of_block(unsigned id, int pairs, int qblocks, int run, int& pair, int& qblk) {
+    const unsigned die = id & 7u, i = id >> 3, all = (unsigned)pairs;
+    if (run == kSpread) {
+        pair = (int)(id % all);
+        qblk = qblocks - 1 - (int)(id / all);
+    } else if (run == kShares) {
+        const unsigned per_die = (all + 7u) / 8u;
+        pair = (int)(die * per_die + i % per_die);
+        qblk = qblocks - 1 - (int)(i / per_die);
+    } else {
+        const unsigned unit = i / (unsigned)run * 8u + die, row = unit / all;
+        pair = (int)((unit + row) % all);
+        qblk = qblocks - 1 - (int)(row * (unsigned)run + i % (unsigned)run);
+    }
+    pair = __builtin_amdgcn_readfirstlane(pair);
+    qblk = __builtin_amdgcn_readfirstlane(qblk);
+    return pair < pairs && qblk >= 0;
 }
 
 // An operand at an address that all lanes share plus a byte offset of each
@@ -99,7 +114,7 @@ __global__ void __launch_bounds__(64 * kLseWaves, 2) talk_lse_kernel(TalkPrefill
     constexpr int kLseQ = 16 * U;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, n = lane & 15;
     int pair, qblk;
-    if (!place_of_block(blockIdx.x, a.nseq * a.heads, a.qblocks, pair, qblk)) return;
+    if (!place_of_block(blockIdx.x, a.nseq * a.heads, a.qblocks, a.run, pair, qblk)) return;
     const int b = pair / a.heads, h = pair - b * a.heads;
     const int q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, sk = a.cu_k[b + 1] - a.cu_k[b], shift = sk - sq;
     const int q0 = (qblk * kLseWaves + wave) * kLseQ;
@@ -225,12 +240,7 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, n = lane & 15;
     int b, qblk;
     const int split = blockIdx.y;
-    if (a.nseq % 8 == 0) {                                       // a sequence belongs to one die, whose second-level cache has its keys
-        if (!place_of_block(blockIdx.x, a.nseq, a.qblocks, b, qblk)) return;
-    } else {
-        b = (int)(blockIdx.x % (unsigned)a.nseq);
-        qblk = a.qblocks - 1 - (int)(blockIdx.x / (unsigned)a.nseq);
-    }
+    if (!place_of_block(blockIdx.x, a.nseq, a.qblocks, a.run, b, qblk)) return;
     const int q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, sk = a.cu_k[b + 1] - a.cu_k[b], shift = sk - sq;
     const int q0 = qblk * Q;
     if (q0 >= sq) return;
@@ -516,11 +526,33 @@ void plan(int64_t heads, int64_t num_seqs, int64_t max_seqlen_q, int64_t max_key
     if (splits < 1) splits = 1;
 }
 
+// Eight sequences, sixteen, ...: where each belongs to a die its keys are read once, but a die with the longest one works on when the others
+// are done.  Runs of blocks, unless the lengths are nearly equal or all blocks of the mixture run at once (mixture and sums of exponentials, us,
+// shares / runs: 8 sequences of 700 .. 2300 397 / 323, 16 of 100 .. 1500 324 / 227, 8 of 1500 252 / 260, single blocks there 318).  Other numbers
+// of sequences spread by themselves (6 of 1214 .. 2313: 360 / 407).
+bool uneven_dies(const TalkPrefillArgs& a, int64_t max_seqlen_q) {
+    return a.nseq % 8 == 0 && (max_seqlen_q + 31) / 32 * a.nseq > 256 && 10 * a.tokens < 9 * a.nseq * max_seqlen_q;
+}
+// a run, so that every die gets eight of them if there are as many
+int64_t run_of(int64_t pairs, int64_t qblocks, int64_t most) {
+    const int64_t run = pairs * qblocks / 64;
+    return run < 1 ? 1 : run < most ? run : most;
+}
+// workgroups, also of blocks that there are not
+int64_t run_grid(int64_t pairs, int64_t qblocks, int64_t run) {
+    if (run == kSpread) return pairs * qblocks;      // no more: with an odd number of them, splits of a block go to several dies
+    if (run == kShares) return (pairs + 7) / 8 * 8 * qblocks;
+    return (pairs * ((qblocks + run - 1) / run) + 7) / 8 * 8 * run;
+}
+
 template <int KS, int U>
 int launch_lse_of(TalkPrefillArgs a, int64_t max_seqlen_q, bool bounded, hipStream_t st) {
-    const int64_t per = 16 * U * kLseWaves, qblocks = (max_seqlen_q + per - 1) / per, total = ((int64_t)a.nseq * a.heads + 7) / 8 * 8 * qblocks;
+    const int64_t per = 16 * U * kLseWaves, qblocks = (max_seqlen_q + per - 1) / per, pairs = (int64_t)a.nseq * a.heads;
+    const int64_t run = uneven_dies(a, max_seqlen_q) ? run_of(pairs, qblocks, 2) : kShares;
+    const int64_t total = run_grid(pairs, qblocks, run);
     if (total > 0x7fffffff) return INFER_KV_EINVAL;
     a.qblocks = (int)qblocks;
+    a.run = (int)run;
     if (bounded) hipLaunchKernelGGL((talk_lse_kernel<KS, U, true>), dim3((unsigned)total), dim3(64 * kLseWaves), 0, st, a);
     else hipLaunchKernelGGL((talk_lse_kernel<KS, U, false>), dim3((unsigned)total), dim3(64 * kLseWaves), 0, st, a);
     return (int)hipGetLastError();
@@ -534,8 +566,11 @@ int launch_lse(const TalkPrefillArgs& a, int64_t max_seqlen_q, bool bounded, hip
 
 template <int KS, int VT, int UH, int QT, bool SHARE>
 int launch_mix(TalkPrefillArgs a, int64_t max_seqlen_q, hipStream_t st) {
-    const int64_t qblocks = (max_seqlen_q + 16 * QT - 1) / (16 * QT), total = qblocks * a.nseq;
+    const int64_t qblocks = (max_seqlen_q + 16 * QT - 1) / (16 * QT);
+    const int64_t run = uneven_dies(a, max_seqlen_q) ? run_of(a.nseq, qblocks, 8) : a.nseq % 8 == 0 ? kShares : kSpread;
+    const int64_t total = run_grid(a.nseq, qblocks, run);
     if (total > 0x7fffffff) return INFER_KV_EINVAL;
+    a.run = (int)run;
     a.qblocks = (int)qblocks;
     auto kernel = &talk_mix_kernel<KS, VT, UH, QT, SHARE>;
     constexpr size_t lds = (size_t)16 * QT * kStep * kMixWaves * UH * (4 + 2) + (UH == 4 ? 4 : 1) * 2048;
@@ -604,7 +639,7 @@ extern "C" int infer_talking_prefill(const void* q, int64_t q_stride, const void
     plan(heads, num_seqs, max_seqlen_q, max_keys, tiles, splits, split_steps);
     const TalkPrefillArgs a{(const __bf16*)q, q_stride, (const __bf16*)keys, (const __bf16*)values, (int)key_pad, (int)vdim_pad, block_table,
                             bt_stride, (int)table_cols, (int)block_size, (int)num_blocks, seqs, cu_q, cu_k, (int)heads, (int)kv_heads, (int)dim,
-                            (int)vdim, (int)num_seqs, 0, scale * kLog2e, (const __bf16*)talk, out_scale, (__bf16*)out, out_stride, workspace, tokens, splits,
+                            (int)vdim, (int)num_seqs, 0, 0, scale * kLog2e, (const __bf16*)talk, out_scale, (__bf16*)out, out_stride, workspace, tokens, splits,
                             split_steps, workspace + (heads * tokens + 3) / 4 * 4};
     hipStream_t st = (hipStream_t)stream;
     const bool bounded = max_score * kLog2e <= kBound;

@@ -361,6 +361,13 @@ def test_prefill_and_rows_agree(gpu, heads, lens):
     close(a, host(b), 1.5e-2)
 
 
+@pytest.mark.parametrize("heads,lens", [(12, [1100, 40, 7, 300, 64, 200, 33, 96]), (16, [30, 700, 5, 64, 100, 31, 32, 33] * 2), (8, [2, 80, 1] * 8 + [401] * 8)])
+def test_prefill_of_uneven_sequences_on_all_dies(gpu, heads, lens):
+    """Eight sequences or a multiple of it, of unequal lengths and more blocks than run at once: runs of blocks go to the dies in turn."""
+    assert len(lens) % 8 == 0 and -(-max(lens) // 32) * len(lens) > 256 and 10 * sum(lens) < 9 * len(lens) * max(lens)
+    test_prefill_and_rows_agree(gpu, heads, lens)
+
+
 def test_what_the_prompt_kernels_do_not_serve(gpu):
     for heads, dim, vdim in ((33, 64, 64), (8, 136, 64), (8, 64, 136), (8, 20, 64), (8, 64, 12)):
         assert not ho.talking_prefill_supported(ho.TalkShape(heads, heads, dim, vdim, 1.0, 0.0))
