@@ -271,20 +271,23 @@ __global__ void __launch_bounds__(256) skinny_gemm_reduce_kernel(ReduceArgs a) {
 // n x 4096, us (16 / 32 / 48 / 64 / 96 rows):
 //   32 of the batch   n = 6144: - / 14.8 / 15.2 / 17.3 / 21.9    n = 12288: - / 27.5 / 19.3 / 20.9 / 24.7    n = 24576: - / 49.0 / 34.6 / 43.3 / 37.4
 //   64 of the batch   n = 6144: - / 17.2 / 19.1 / 21.8 / 27.3    n = 12288: - / 33.8 / 22.5 / 25.0 / 30.0    n = 24576: - / 58.5 / 44.6 / 49.7 / 40.3
-// so 33 to 64 want one workgroup per compute unit.  Up to 16, 16 rows are as good as any (n = 24576: 33 to 37 us), except past a
-// vocabulary, where more than 8 of the batch take 61 us (k = 1024) with 16 rows and 52 with 32.
-int rows_per_workgroup(int64_t m, int64_t n) {
-    if (m <= 16) return m > 8 && n >= 65536 ? 32 : 16;
+// so 33 to 64 want one workgroup per compute unit.  Past a vocabulary (n = 151936) there are many workgroups, and what counts is how little
+// of one passes before and behind its stream: one wavefront that holds 160 rows by itself, two such workgroups to a compute unit, against four
+// that split k of 80 rows and add up: 64 of the batch 259 -> 243 us (k = 4096), 79 -> 67 (k = 1024).  Up to 16, 16 rows are as good as any
+// (n = 24576: 33 to 37 us), except past a vocabulary with a short k: 32 rows 48 us (k = 1024), 16 rows 54, but 215 and 190 with k = 4096.
+constexpr int64_t kVocabulary = 65536;
+int rows_per_workgroup(int64_t m, int64_t n, int64_t k) {
+    if (m <= 16) return n >= kVocabulary && k <= 2048 ? 32 : 16;
     if (m <= 32) return n >= 8192 ? 48 : n > 5120 ? 32 : 16;
     if (m > 64) return kBN;
     if (n <= 5120) return 64;                    // cut over k (choose_splits)
-    return n <= 8192 ? 32 : n > 24576 ? 80 : 16 * (int)((n + 4095) / 4096);
+    return n <= 8192 ? 32 : n >= kVocabulary ? 160 : n > 24576 ? 80 : 16 * (int)((n + 4095) / 4096);
 }
 
 // Split-K factor: a divisor of the chunk count that brings the grid to at least one workgroup per
 // compute unit (256 on MI355X) while leaving every split at least four chunks to stream.
 int choose_splits(int64_t m, int64_t n, int64_t k) {
-    const int64_t rows = rows_per_workgroup(m, n), tiles = (n + rows - 1) / rows;
+    const int64_t rows = rows_per_workgroup(m, n, k), tiles = (n + rows - 1) / rows;
     const int64_t chunks = k / kKC;
     if (m <= 64 && n > 5120) return 1;          // what 180 workgroups lack of the chip is less than the sums of a split cost
     int best = 1;
@@ -298,7 +301,7 @@ int choose_splits(int64_t m, int64_t n, int64_t k) {
 
 template <bool GATED>
 void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
-    const int rows = rows_per_workgroup(a.m, a.n);
+    const int rows = rows_per_workgroup(a.m, a.n, a.k);
     const dim3 grid((unsigned)((a.n + rows - 1) / rows), (unsigned)splits);
 #define GO(RT, MT, NW, D) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED>), grid, dim3(64 * NW), 0, st, a)
     if (a.m <= 16 && rows == 16) GO(1, 1, 4, 4);
@@ -309,7 +312,9 @@ void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
     else if (a.m <= 64 && rows == 32) GO(2, 4, 4, 2);
     else if (a.m <= 64 && rows == 48) GO(3, 4, 4, 2);
     else if (a.m <= 64 && rows == 64) GO(4, 4, 4, 2);
-    else if (a.m <= 64 && rows == 80) GO(5, 4, 4, 2);
+    else if (a.m <= 64 && rows == 80 && a.n <= 80 * 512) GO(5, 4, 2, 2);      // all at once, two to a compute unit: n = 32000 60 -> 56 us
+    else if (a.m <= 64 && rows == 80) GO(5, 4, 4, 2);                // n = 50000: 92 us, with two wavefronts 106
+    else if (a.m <= 64 && rows == 160) GO(10, 4, 1, 2);
     else if (a.m <= 64) GO(6, 4, 3, 2);
     else if constexpr (!GATED) hipLaunchKernelGGL(skinny_gemm_kernel, grid, dim3(256), 0, st, a);
 #undef GO

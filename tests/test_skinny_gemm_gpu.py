@@ -120,7 +120,7 @@ def test_partial_sums_cannot_be_used_after_a_later_split_gemm(gpu):
 
 @pytest.mark.parametrize("m", [1, 7, 8, 9, 16, 17, 32, 33, 48, 64])
 @pytest.mark.parametrize("n,k", [(8, 128), (136, 256), (1024, 2048), (4096, 640), (5120, 512), (5128, 128), (6152, 384), (8200, 256), (12296, 128), (16400, 128),
-                                 (20488, 128), (24584, 256), (65544, 128)])
+                                 (20488, 128), (24584, 256), (40968, 128), (65544, 128)])
 def test_streamed_weights_around_tiles_and_rules(gpu, m, n, k):
     """Small integers, whose products and sums are exact: every number of rows per workgroup, the last rows of the weights and of the
     batch, k of one step per wavefront and fewer; unreduced sums add up to the same."""
