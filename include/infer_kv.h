@@ -299,10 +299,9 @@ int infer_decode_metadata(const int32_t* seq_lens, const int32_t* block_table, i
                           int32_t* context_lens, void* stream);
 
 /* Replaces Linear.forward (infer/ops/MLP.py:103-149, F.linear; the op matmul(input, weight, output) of
- * src/bindings.cpp:7) at the batch sizes of a decode step, for weight matrices with few rows (o_proj,
- * down_proj): y[M, N] = x[M, K] . w[N, K]^T, bf16 in, float32 accumulate, bf16 out, M <= 128.  The
- * weights (row-major [N, K], contiguous) are streamed from HBM once; K is cut over workgroups and
- * float32 partial sums pass through `workspace` (infer_skinny_gemm_workspace_bytes says how much,
+ * src/bindings.cpp:7) at the batch sizes of a decode step: y[M, N] = x[M, K] . w[N, K]^T, bf16 in, float32 accumulate, bf16 out, M <= 128.  The
+ * weights (row-major [N, K], contiguous) are streamed from HBM once; where there are few weight rows, K is
+ * cut over workgroups and float32 partial sums pass through `workspace` (infer_skinny_gemm_workspace_bytes says how much,
  * 0 if the shape needs no split).  K must be a multiple of 128 and N a multiple of 8; other shapes
  * return INFER_KV_EUNSUPPORTED and belong to the vendor GEMM. */
 size_t infer_skinny_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);

@@ -592,6 +592,7 @@ __device__ __forceinline__ float half_sum(float x) {
 }
 
 // hi + mid + lo = x exactly, two floats at a time: a residual is one dot product with (-1, 0) or (0, -1) instead of a mask and a subtraction
+// (829 -> 797 us with 8 x 500 .. 2600 tokens of 32 heads).  A pair lies along the sum that both enter, so an infinity spoils no other sum.
 template <int N>
 __device__ __forceinline__ void split3(const float (&x)[N], uint32_t (&p)[3][N / 2]) {
     typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
