@@ -275,12 +275,17 @@ __global__ void __launch_bounds__(256) skinny_gemm_reduce_kernel(ReduceArgs a) {
 // of one passes before and behind its stream: one wavefront that holds 160 rows by itself, two such workgroups to a compute unit, against four
 // that split k of 80 rows and add up: 64 of the batch 259 -> 243 us (k = 4096), 79 -> 67 (k = 1024).  Up to 16, 16 rows are as good as any
 // (n = 24576: 33 to 37 us), except past a vocabulary with a short k: 32 rows 48 us (k = 1024), 16 rows 54, but 215 and 190 with k = 4096.
-constexpr int64_t kVocabulary = 65536;
+// Few weight rows and a long k: 16 rows give every compute unit a workgroup that reads the batch once per 16 rows; 64 rows, cut over k, read it a
+// quarter as often.  Unreduced sums, us, 16 / 64 rows: n = 4096, k = 12288 9 of the batch 18.5 / 17.1, 16 20.2 / 17.3, 32 25.9 / 19.0; n = 5120,
+// k = 25600 60 / 52, 69 / 54, 91 / 60; n = 2560, k = 9728 12.7 / 10.4, 14.5 / 10.7, 19.1 / 15.7.  With a shorter k the launch that adds the
+// sums up for those who want them costs more than that (n = 4096, k = 4096, 16: 8.4 / 10.4 reduced, 8.6 / 7.4 unreduced).
+constexpr int64_t kVocabulary = 65536, kLongK = 8192;
 int rows_per_workgroup(int64_t m, int64_t n, int64_t k) {
+    if (m > 8 && m <= 32 && n <= 5120 && k >= kLongK) return 64;
     if (m <= 16) return n >= kVocabulary && k <= 2048 ? 32 : 16;
     if (m <= 32) return n >= 8192 ? 48 : n > 5120 ? 32 : 16;
     if (m > 64) return kBN;
-    if (n <= 5120) return 64;                    // cut over k (choose_splits)
+    if (n <= 5120) return 64;
     return n <= 8192 ? 32 : n >= kVocabulary ? 160 : n > 24576 ? 80 : 16 * (int)((n + 4095) / 4096);
 }
 
@@ -304,7 +309,9 @@ void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
     const int rows = rows_per_workgroup(a.m, a.n, a.k);
     const dim3 grid((unsigned)((a.n + rows - 1) / rows), (unsigned)splits);
 #define GO(RT, MT, NW, D) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED>), grid, dim3(64 * NW), 0, st, a)
-    if (a.m <= 16 && rows == 16) GO(1, 1, 4, 4);
+    if (a.m <= 16 && rows == 64) GO(4, 1, 4, 2);
+    else if (a.m <= 32 && rows == 64) GO(4, 2, 4, 2);
+    else if (a.m <= 16 && rows == 16) GO(1, 1, 4, 4);
     else if (a.m <= 16) GO(2, 1, 4, 3);
     else if (a.m <= 32 && rows == 16) GO(1, 2, 4, 3);
     else if (a.m <= 32 && rows == 32) GO(2, 2, 4, 2);

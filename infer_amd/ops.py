@@ -502,8 +502,9 @@ SKINNY_MAX_ROWS = 5120
 def _own_kernel(m: int, n: int, k: int, defer: bool) -> bool:
     if m > STREAM_MAX_BATCH:
         return n <= SKINNY_MAX_ROWS and k >= 2048
-    # a split over k whose pieces nobody takes has a launch more: 1024 x 2048, 48 rows 8.0 us against 8.6 (5.7 unreduced)
-    return defer or m <= 32 or n >= 2048
+    # a split over k whose pieces nobody takes has a launch more: 1024 x 2048, 48 rows 8.6 us against 8.0 (5.7 unreduced); 1024 x 3072
+    # 9.5 against 10.5, 1024 x 4096 9.8 against 14.2
+    return defer or m <= 32 or n >= 2048 or k > 2048
 
 
 def _linear_mode() -> str:

@@ -134,6 +134,20 @@ def test_streamed_weights_around_tiles_and_rules(gpu, m, n, k):
     assert torch.equal((deferred.materialize() if isinstance(deferred, ops.SplitKSum) else deferred).float(), want)
 
 
+@pytest.mark.parametrize("m", [8, 9, 16, 17, 32, 33])
+@pytest.mark.parametrize("n,k", [(136, 8192), (4104, 8320), (5120, 8064), (5128, 8192)])
+def test_streamed_weights_of_a_long_k(gpu, m, n, k):
+    """As above around the line from which few weight rows are cut over k; one in four activations is not zero, so that sums stay below 256."""
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = (torch.randint(-1, 2, (m, k), generator=g, device=gpu) * (torch.rand((m, k), generator=g, device=gpu) < 0.25)).to(torch.bfloat16)
+    w = torch.randint(-1, 2, (n, k), generator=g, device=gpu).to(torch.bfloat16)
+    want = reference(x, w)
+    assert want.abs().max() <= 256                      # representable in bf16 without rounding
+    assert torch.equal(ops.skinny_linear(x, w).float(), want)
+    deferred = ops.linear(x, w, defer=True)
+    assert torch.equal((deferred.materialize() if isinstance(deferred, ops.SplitKSum) else deferred).float(), want)
+
+
 @pytest.mark.parametrize("m", [1, 16, 17, 40, 64, 65])
 @pytest.mark.parametrize("ff,k", [(8, 128), (2568, 256), (3072, 1024), (4104, 384), (6160, 256), (10248, 128), (12288, 512)])
 def test_gate_and_up_in_one_launch_have_the_bits_of_two(gpu, m, ff, k):
