@@ -725,14 +725,15 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t max_places, hipStrea
 // rows per tile: 0 where only the any-size kernels serve
 int rows_per_tile(int elem, int64_t n, int64_t width, int64_t ff_pad, int64_t experts, int64_t top) {
     if (elem != INFER_ELEM_BF16 || width % 8 || ff_pad % 8) return 0;
-    if (n * top <= 24 * experts) return kSmallRows;
-    // Large blocks pay where they are enough to fill most of the chip, and where an expert has more rows than its weights' way from memory
-    // takes anyway (of 14 experts, tiles of 128 rows / blocks, us: 3072 x 4096, 118 rows 284 / 302, 200 319 / 295, 800 471 / 322, 2100 879 / 510;
-    // 768 x 1024, 600 rows 57 / 66, 1200 67 / 71, 2300 104 / 81).  Their offsets are 32 bits.
+    // an expert with more than one tile of 32 rows reads its weights again (of 14 experts of 3072 x 4096, tiles of 32 rows / blocks, us: 118 rows
+    // 252 / 268, 140 284 / 304, 180 357 / 300)
+    if (n * top <= 32 * experts) return kSmallRows;
+    // Large blocks pay where they are enough to fill most of the chip (of 14 experts, tiles of 128 rows / blocks, us: 3072 x 4096, 200 rows
+    // 319 / 295, 800 471 / 322, 2100 879 / 510; 768 x 1024, 600 rows 57 / 66, 1200 67 / 71, 2300 104 / 81).  Their offsets are 32 bits.
     const int64_t far = 1ll << 31;
     const bool fits = width % 64 == 0 && ff_pad % 64 == 0 && n * width < far && n * top * ff_pad < far && 2 * ff_pad * width < far;
     const int64_t blocks = (n * top / kBlockRows + experts / 2) * ((ff_pad + 127) / 128);      // of the first product, about
-    return fits && (n * top >= 512 * experts || (n * top >= 32 * experts && blocks >= 160)) ? kBlockRows : kBigRows;
+    return fits && (n * top >= 512 * experts || (blocks >= 160)) ? kBlockRows : kBigRows;
 }
 
 }  // namespace
