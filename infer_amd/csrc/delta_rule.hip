@@ -591,7 +591,8 @@ __device__ __forceinline__ float half_sum(float x) {
     return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
 }
 
-// hi + mid + lo = x exactly, two floats at a time: a residual is one dot product with (-1, 0) or (0, -1) instead of a mask and a subtraction
+// hi + mid + lo = x exactly, two floats at a time, hi and mid rounded to nearest, so that residuals have both signs: |mid| <= 2^-8 and
+// |lo| <= 2^-17 of x's power of two (a float past the largest bf16, 3.39e38, is infinite).  A residual is one dot product with (-1, 0) or (0, -1) instead of a mask and a subtraction
 // (829 -> 797 us with 8 x 500 .. 2600 tokens of 32 heads).  A pair lies along the sum that both enter, so an infinity spoils no other sum.
 template <int N>
 __device__ __forceinline__ void split3(const float (&x)[N], uint32_t (&p)[3][N / 2]) {
@@ -601,18 +602,18 @@ __device__ __forceinline__ void split3(const float (&x)[N], uint32_t (&p)[3][N /
     const bf16x2_t first = __builtin_bit_cast(bf16x2_t, c0), second = __builtin_bit_cast(bf16x2_t, c1);
 #pragma unroll
     for (int i = 0; i < N / 2; ++i) {
-        p[0][i] = pack(x[2 * i], x[2 * i + 1]);
+        p[0][i] = round_pack(x[2 * i], x[2 * i + 1]);
         const bf16x2_t hi = __builtin_bit_cast(bf16x2_t, p[0][i]);
         const float a = __builtin_amdgcn_fdot2_f32_bf16(hi, first, x[2 * i], false), b = __builtin_amdgcn_fdot2_f32_bf16(hi, second, x[2 * i + 1], false);
-        p[1][i] = pack(a, b);
+        p[1][i] = round_pack(a, b);
         const bf16x2_t mid = __builtin_bit_cast(bf16x2_t, p[1][i]);
         p[2][i] = pack(__builtin_amdgcn_fdot2_f32_bf16(mid, first, a, false), __builtin_amdgcn_fdot2_f32_bf16(mid, second, b, false));
     }
 }
 
 // A record in LDS: sums of three bf16 numbers, hi + mid + lo = the float exactly, so that the products run on the bf16 matrix pipe.  Of
-// the nine products of two such sums the six down to 2^-16 of the first are added; what is left out lies below the last bit of a float
-// product.
+// the nine products of two such sums six are added; the others, mid lo, lo mid and lo lo, are 2^-24 of the product at most, as much as a
+// float product is rounded by, and of either sign.
 struct WideBuffer {
     u32x4_t* p;
     int ks;
@@ -628,10 +629,11 @@ __host__ __device__ constexpr int wide_buffer_units(int dt) { return 64 * (5 * d
 // so they do not pass through memory in between.
 // A batch takes as long as its longest portion's chunks one after the other; a step of eight wavefronts on a compute unit is 3200 clocks
 // of matrix pipe per wavefront with float products and 1200 with pieces, which cost about 180 vector instructions.  32 heads, 8 portions
-// of 590 to 2560 tokens: scan, output and ring 655 us with delta_scan_kernel, 435 us here.  What a step waits for is requested a step
-// before, by every thread and without branches: with requests in branches, or stores between a request and its use, the compiler waits
-// for everything in flight (830 us).  Tried as well: float products for W S (690 us); the two wavefronts of a vector unit in opposite
-// phases (550); four wavefronts that only serve eight that compute (460).
+// of 590 to 2560 tokens: scan, output and ring 662 us with delta_scan_kernel, 525 us here (kernels alone, under a profiler; the call 963 and
+// 816 us).  What a step waits for is requested a step before, by every thread and without branches: with requests in branches, or
+// stores between a request and its use, the compiler waits for everything in flight.  Tried as well, against 435 us of a first form: 830
+// with such requests; float products for W S 690; the two wavefronts of a vector unit in opposite phases 550; four wavefronts that only
+// serve eight that compute 460.
 template <class T, int DT>
 __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a, const PortionDesc* portions, const ChunkDesc* chunks,
                                                                  const float* records, int slabs) {
@@ -742,7 +744,10 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
         gate = *reinterpret_cast<const t4_t*>(gates + (int64_t)(row + (out_row < count ? out_row : count - 1)) * a.gate_stride);
         __builtin_amdgcn_sched_barrier(0);             // requests stay here, a step ahead of their use
         if (live) {
-            // the vector unit cuts the next part of the state while the matrix pipe works on one
+            // The vector unit cuts the next part of the state while the matrix pipe works on one.  The pipe rounds its sums towards one
+            // side, so nothing stays in its accumulators from chunk to chunk: the state takes a chunk's sum by the vector unit.  3200
+            // tokens without decay, all of one sign: error of the state 5.7e-7 of its norm, 6.6e-6 with the state in the pipe's
+            // accumulators and pieces cut off instead of rounded, 1.4e-6 in delta_scan_kernel; 800 -> 816 us for the call with the batch above.
             f32x4_t x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1, x3 = x1, o1 = x1, o2 = x1, o3 = x1;
             uint32_t pc[KS][3][4];
             u32x4_t w[KS][3], qv[KS][3];
@@ -785,18 +790,24 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
             o1 = mma(b0, uhh, o1);
             const f32x4_t* e = reinterpret_cast<const f32x4_t*>(buf.e());
             u32x4_t k0[DT], k1[DT];
+            f32x4_t ds[DT];
 #pragma unroll
             for (int t = 0; t < DT; ++t) {
                 k0[t] = buf.k(t, 0)[lane];
                 k1[t] = buf.k(t, 1)[lane];
-                s[t] *= e[4 * t + q];
             }
 #pragma unroll
-            for (int t = 0; t < DT; ++t) s[t] = mma(k1[t], ulh, s[t]);
+            for (int t = 0; t < DT; ++t) ds[t] = mma(k1[t], ulh, f32x4_t{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-            for (int t = 0; t < DT; ++t) s[t] = mma(k0[t], umm, s[t]);
+            for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], umm, ds[t]);
 #pragma unroll
-            for (int t = 0; t < DT; ++t) s[t] = mma(k0[t], uhh, s[t]);
+            for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], uhh, ds[t]);
+#pragma unroll
+            for (int t = 0; t < DT; ++t) {
+                const f32x4_t et = e[4 * t + q];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[t][r] = __builtin_fmaf(s[t][r], et[r], ds[t][r]);
+            }
             const f32x4_t o = o1 + (o2 + o3);
             float* to = outputs + ((c & 1) * 16 + 4 * q) * kPitch + 16 * vt + m;
 #pragma unroll

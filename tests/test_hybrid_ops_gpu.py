@@ -435,6 +435,31 @@ def test_delta_batch_that_fills_the_chip(gpu, dtype, heads, kv_heads, dim, vdim,
     assert torch.isnan(c0.state[2]).all()
 
 
+def test_delta_state_of_operands_of_one_sign_does_not_drift(gpu):
+    """3200 tokens without decay whose keys, values and inner results are all positive, beside seven short portions, so that one workgroup
+    holds all columns of a head.  Roundings to nearest of the 200 chunks' sums partly cancel: sqrt(200) of them are 14 x 2^-24, as many as
+    six of the operands' come on top, and ten of beta = sigmoid(-9), whose exponent is rounded at 9 log2(e) = 13 and so is off by 2^-21, with
+    the constant in it: 30 x 2^-24 = 1.8e-6 of the state's norm.  A rounding towards one side, or terms left out of one sign, in each of a
+    chunk's products adds up instead."""
+    heads, n = 33, 3200
+    c = DeltaCase(heads, 1, 32, 32, 4, n + 7 * 16, torch.float32, slots=8, decay=-20.0)
+    rng, f32 = np.random.default_rng(5), lambda x: rounded(x, torch.float32)
+    c.proj, c.conv, c.a_log = f32(0.5 + rng.random(c.proj.shape)), f32(0.2 + 0.2 * rng.random(c.conv.shape)), np.zeros(heads)
+    c.proj[:, c.beta_off:] = f32(-9 + 0.1 * rng.standard_normal(c.proj[:, c.beta_off:].shape))
+    chunks = [(r, 16, r, 0, 0, 0) for r in range(0, n, 16)] + [(n + 16 * i, 16, 0, 0, i + 1, 0) for i in range(7)]
+    portions = [(0, n // 16, 0, 0)] + [(n // 16 + i, 1, i + 1, 0) for i in range(7)]
+    ring = [(0, n - 1 - r) for r in range(n)] + [(i + 1, 15 - r) for i in range(7) for r in range(16)]
+    out = torch.empty((c.n, heads * 32), device="cuda")
+    ho.delta_chunks(c.s, dev(c.proj), c.beta_off, dev(c.decay), dev(c.gate), *c.weights, c.ring, c.state, dev(portions, torch.int32),
+                    dev(chunks, torch.int32), dev(ring, torch.int32), dev(list(range(n)) + 7 * list(range(16)), torch.int64), 0, out)
+    state = host(c.state[0])
+    c.n = n
+    c.proj, c.decay, c.gate = c.proj[:n], c.decay[:n], c.gate[:n]
+    want = c.want()[1]
+    assert want.min() > 0
+    assert np.linalg.norm(state - want) <= 30 * 2.0 ** -24 * np.linalg.norm(want)
+
+
 def test_sizes_outside_are_refused_on_the_host(gpu):
     with pytest.raises(RuntimeError):
         ho.delta_layout(300, 16)
