@@ -539,8 +539,11 @@ def _time_cold(fn, device, reps: int = 6) -> float:
 
 
 def _streamable(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether the kernels of this package can take the product: types, sizes, strides and alignment, and nobody wants a gradient."""
+    """Whether the kernels of this package can take the product: place, types, sizes, strides and alignment, and nobody wants a gradient."""
     if x.dim() != 2 or not x.is_cuda or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.dim() != 2:
+        return False
+    device = x.get_device()
+    if weight.get_device() != device or torch.cuda.current_device() != device:      # kernels are launched on the current device
         return False
     m, k = x.shape
     if not skinny_linear_supported(m, weight.shape[0], k) or weight.shape[1] != k or not weight.is_contiguous() or x.stride(1) != 1:
