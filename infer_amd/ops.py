@@ -14,6 +14,9 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -538,8 +541,32 @@ def _time_cold(fn, device, reps: int = 6) -> float:
     return times[len(times) // 2]
 
 
+def _plain(t: torch.Tensor) -> bool:
+    """Whether a tensor is its memory and nothing else: no subclass with operators of its own, no tangent, no batch or level of a transform."""
+    kind = type(t)
+    if kind is not torch.Tensor and (kind.__torch_function__ is not torch._C._disabled_torch_function_impl or
+                                     kind.__torch_dispatch__ is not torch._C._disabled_torch_dispatch_impl):
+        return False
+    if torch._C._functorch.is_functorch_wrapped_tensor(t):
+        return False
+    return forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None
+
+
+def _operators_are_watched() -> bool:
+    """Whether somebody follows the operators that are called, or changes their types: a compiler, a tracer, a mode (other than that of a
+    default device), autocast to another type.  They see F.linear and would not see a launch."""
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack():
+        return True
+    if torch._C._len_torch_function_stack() and not all(isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack()):
+        return True
+    return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16
+
+
 def _streamable(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether the kernels of this package can take the product: place, types, sizes, strides and alignment, and nobody wants a gradient."""
+    """Whether the kernels of this package can take the product: place, types, sizes, strides and alignment, and nobody wants a gradient, a
+    tangent or the operator itself."""
+    if _operators_are_watched() or not _plain(x) or not _plain(weight):
+        return False
     if x.dim() != 2 or not x.is_cuda or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.dim() != 2:
         return False
     device = x.get_device()
