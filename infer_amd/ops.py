@@ -12,6 +12,8 @@ current stream.  Tensors must live on the GPU; there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+import threading
+from collections import OrderedDict
 
 import torch
 from torch.autograd import forward_ad
@@ -375,7 +377,15 @@ def decode_metadata(seq_lens: torch.Tensor, block_table: torch.Tensor, block_siz
     _lib.check(rc, "decode_metadata")
 
 
-_gemm_workspaces: dict = {}
+class _Workspaces(threading.local):
+    """A thread's workspaces of split products by (device, stream), the one used last at the end."""
+    MOST = 4
+
+    def __init__(self):
+        self.of: OrderedDict = OrderedDict()
+
+
+_gemm_workspaces = _Workspaces()
 
 
 def skinny_linear_supported(m: int, n: int, k: int) -> bool:
@@ -384,28 +394,30 @@ def skinny_linear_supported(m: int, n: int, k: int) -> bool:
 
 
 def _gemm_workspace(device, need: int) -> torch.Tensor | None:
-    """Where split products leave their partial sums: one workspace per stream, so that calls on different streams do not meet, and one
-    for everything that is captured into graphs, which is set aside with the first one (a captured call does not allocate)."""
+    """Where a split product leaves its partial sums.  Streams and threads have one each, so that products that run side by side, or a product
+    and the sum of another one's pieces, do not meet; a thread keeps those of the four streams it used last (16 MiB each, or what the largest
+    product needed).  A captured product has memory of its own from the graph's pool: streams forked in a capture run side by side, and graphs
+    may be replayed on any stream."""
     if not need:
         return None
     device = torch.device(device)
+    index = torch.cuda.current_device() if device.index is None else device.index
     if torch.cuda.is_current_stream_capturing():
-        keys = [(str(device), "captured")]
-    else:
-        keys = [(str(device), torch.cuda.current_stream(device).cuda_stream), (str(device), "captured")]
-    for key in keys:
-        ws = _gemm_workspaces.get(key)
-        if ws is None or ws.numel() < need:
-            if ws is not None:
-                _retired_workspaces.append(ws)
-            _gemm_workspaces[key] = torch.empty(max(need, 64 << 20), dtype=torch.uint8, device=device)
-    return _gemm_workspaces[keys[0]]
+        return torch.empty(need, dtype=torch.uint8, device=device)
+    key, of = (index, torch._C._cuda_getCurrentRawStream(index)), _gemm_workspaces.of
+    ws = of.get(key)
+    if ws is None or ws.numel() < need:
+        ws = of[key] = torch.empty(max(need, 16 << 20), dtype=torch.uint8, device=device)
+        if len(of) > _Workspaces.MOST:
+            of.popitem(last=False)
+    of.move_to_end(key)
+    return ws
 
 
 class SplitKSum:
     """Result of a split-K GEMM that has not been reduced yet: ``partial`` ``[splits, M, N]`` float32
     lives at the start of the stream's GEMM workspace, so it must be consumed (``rms_norm`` does, ``materialize``
-    does) before the next split-K GEMM on the stream runs; ``generation`` guards that."""
+    does) before the next split-K GEMM of the thread on the stream runs; ``generation`` guards that."""
     _generation: dict = {}          # address of a workspace -> products that were left in it
 
     @classmethod
@@ -463,8 +475,7 @@ def skinny_linear_deferred(x: torch.Tensor, weight: torch.Tensor):
 def skinny_linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear(x, weight)`` for ``x`` ``[M, K]`` with ``M <= 128`` (``Linear.forward``,
     ``infer/ops/MLP.py:103-149``): the weight matrix ``[N, K]`` is streamed once by a hand-written
-    split-K kernel.  The float32 workspace is cached per stream and only ever grows (a captured graph
-    keeps pointing at the one it was captured with, so outgrown buffers are kept alive)."""
+    split-K kernel (``_gemm_workspace``: where its float32 sums lie)."""
     m, k = x.shape
     n = weight.shape[0]
     assert weight.shape == (n, k) and weight.is_contiguous()

@@ -158,7 +158,7 @@ class QwenForCausalLM(nn.Module):
         """Workspaces of a decode step: split-KV attention for the largest batch, split-K products."""
         c = self.config
         ops.decode_workspace(device, max_batch, c.num_attention_heads, c.num_key_value_heads, c.head_dim)
-        ops._gemm_workspace(device, 64 << 20)
+        ops._gemm_workspace(device, 16 << 20)
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         return self.model(input_ids, positions)
