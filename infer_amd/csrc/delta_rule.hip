@@ -658,6 +658,15 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
             for (int r = 0; r < 4; ++r) s[t][r] = sp[(int64_t)(16 * t + 4 * q + r) * vdim_pad];
     }
 
+    auto keep_state = [&] {
+        if (!live) return;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sp[(int64_t)(16 * t + 4 * q + r) * vdim_pad] = s[t][r];
+    };
+    if (p.chunks <= 0) return keep_state();            // an empty portion has no record to request
+
     // Every request is made by every thread, so that the compiler knows how many are in flight; what a thread has no use for is the
     // record's start.
     const int w_at = tid < 64 * DT ? (tid / (64 * KS)) * 4 * dp + ((tid >> 6) % KS) * 128 + lane : 0, k_at = tid < 64 * DT ? 8 * dp + tid : 0;
@@ -741,7 +750,8 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
         }
         if (c > 0) finish((c - 1) & 1);
         fetch(c + 2);
-        gate = *reinterpret_cast<const t4_t*>(gates + (int64_t)(row + (out_row < count ? out_row : count - 1)) * a.gate_stride);
+        // rows behind a chunk's last repeat it; an empty chunk has none, and row 0 exists
+        gate = *reinterpret_cast<const t4_t*>(gates + (int64_t)(count > 0 ? row + (out_row < count ? out_row : count - 1) : 0) * a.gate_stride);
         __builtin_amdgcn_sched_barrier(0);             // requests stay here, a step ahead of their use
         if (live) {
             // The vector unit cuts the next part of the state while the matrix pipe works on one.  The pipe rounds its sums towards one
@@ -823,11 +833,7 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
         __syncthreads();
     }
     finish((p.chunks - 1) & 1);
-    if (!live) return;
-#pragma unroll
-    for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sp[(int64_t)(16 * t + 4 * q + r) * vdim_pad] = s[t][r];
+    keep_state();
 }
 
 // The inputs of the convolution that a portion's last tokens leave in its ring; a workgroup looks at 64 rows and copies VEC * 256 channels

@@ -435,6 +435,25 @@ def test_delta_batch_that_fills_the_chip(gpu, dtype, heads, kv_heads, dim, vdim,
     assert torch.isnan(c0.state[2]).all()
 
 
+def test_delta_empty_portions_and_chunks(gpu):
+    """In front of the rows and behind them, in one workgroup per head: a portion without chunks keeps its slot's state, or clears it at the
+    first position; a chunk without tokens changes nothing."""
+    c = DeltaCase(33, 33, 32, 32, 4, 20, torch.float32, slots=12)
+    chunks = [(0, 0, 0, 0, 1, 0), (0, 16, 0, 0, 1, 0), (16, 4, 16, 0, 1, 0), (0, 0, 20, 0, 1, 0)]
+    portions = [(0, 0, 0, 5), (0, 4, 1, 0), (0, 0, 2, 0), (3, 0, 3, 7)] + [(0, 0, 4 + i, 3) for i in range(8)]
+    c.state[[0, 3]] = torch.randn(c.state[[0, 3]].shape, device="cuda")
+    before = c.state.clone()
+    chunks += [(0, 0, 0, 0, 1, 0)] * (len(portions) - len(chunks))
+    ring = [(1, 19 - r) for r in range(20)]
+    out = torch.full((20, 33 * 32), float("nan"), device="cuda")
+    ho.delta_chunks(c.s, dev(c.proj), c.beta_off, dev(c.decay), dev(c.gate), *c.weights, c.ring, c.state, dev(portions, torch.int32),
+                    dev(chunks, torch.int32), dev(ring, torch.int32), dev(np.arange(20), torch.int64), 0, out)
+    want, want_state = c.want()
+    close(out, want, 3e-5)
+    close(c.state[1], want_state, 3e-5)
+    assert torch.equal(c.state[0], before[0]) and torch.equal(c.state[3], before[3]) and (c.state[2] == 0).all()
+
+
 def test_delta_state_of_operands_of_one_sign_does_not_drift(gpu):
     """3200 tokens without decay whose keys, values and inner results are all positive, beside seven short portions, so that one workgroup
     holds all columns of a head.  Roundings to nearest of the 200 chunks' sums partly cancel: sqrt(200) of them are 14 x 2^-24, as many as
