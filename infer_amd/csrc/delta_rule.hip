@@ -630,7 +630,7 @@ __host__ __device__ constexpr int wide_buffer_units(int dt) { return 64 * (5 * d
 // A batch takes as long as its longest portion's chunks one after the other; a step of eight wavefronts on a compute unit is 3200 clocks
 // of matrix pipe per wavefront with float products and 1200 with pieces, which cost about 180 vector instructions.  32 heads, 8 portions
 // of 590 to 2560 tokens: scan, output and ring 662 us with delta_scan_kernel, 525 us here (kernels alone, under a profiler; the call 963 and
-// 816 us).  What a step waits for is requested a step before, by every thread and without branches: with requests in branches, or
+// 807 us).  What a step waits for is requested a step before, by every thread and without branches: with requests in branches, or
 // stores between a request and its use, the compiler waits for everything in flight.  Tried as well, against 435 us of a first form: 830
 // with such requests; float products for W S 690; the two wavefronts of a vector unit in opposite phases 550; four wavefronts that only
 // serve eight that compute 460.
@@ -757,7 +757,7 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
             // The vector unit cuts the next part of the state while the matrix pipe works on one.  The pipe rounds its sums towards one
             // side, so nothing stays in its accumulators from chunk to chunk: the state takes a chunk's sum by the vector unit.  3200
             // tokens without decay, all of one sign: error of the state 5.7e-7 of its norm, 6.6e-6 with the state in the pipe's
-            // accumulators and pieces cut off instead of rounded, 1.4e-6 in delta_scan_kernel; 800 -> 816 us for the call with the batch above.
+            // accumulators and pieces cut off instead of rounded, 1.4e-6 in delta_scan_kernel; 794 -> 807 us for the call with the batch above.
             f32x4_t x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1, x3 = x1, o1 = x1, o2 = x1, o3 = x1;
             uint32_t pc[KS][3][4];
             u32x4_t w[KS][3], qv[KS][3];
@@ -800,11 +800,12 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
             o1 = mma(b0, uhh, o1);
             const f32x4_t* e = reinterpret_cast<const f32x4_t*>(buf.e());
             u32x4_t k0[DT], k1[DT];
-            f32x4_t ds[DT];
+            f32x4_t ds[DT], et[DT];
 #pragma unroll
             for (int t = 0; t < DT; ++t) {
                 k0[t] = buf.k(t, 0)[lane];
                 k1[t] = buf.k(t, 1)[lane];
+                et[t] = e[4 * t + q];
             }
 #pragma unroll
             for (int t = 0; t < DT; ++t) ds[t] = mma(k1[t], ulh, f32x4_t{0.f, 0.f, 0.f, 0.f});
@@ -814,9 +815,8 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
             for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], uhh, ds[t]);
 #pragma unroll
             for (int t = 0; t < DT; ++t) {
-                const f32x4_t et = e[4 * t + q];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) s[t][r] = __builtin_fmaf(s[t][r], et[r], ds[t][r]);
+                for (int r = 0; r < 4; ++r) s[t][r] = __builtin_fmaf(s[t][r], et[t][r], ds[t][r]);
             }
             const f32x4_t o = o1 + (o2 + o3);
             float* to = outputs + ((c & 1) * 16 + 4 * q) * kPitch + 16 * vt + m;
