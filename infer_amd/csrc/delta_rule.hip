@@ -988,10 +988,16 @@ int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t nu
     int rc = (int)hipGetLastError();
     if (rc) return rc;
     const bool out4 = rows4 && fours(a.gate, a.gate_stride) && fours(a.out, a.out_stride) && ptr_aligned(o, 16) && ptr_aligned(a.norm, 16);
-    // Up to 256 workgroups of four wavefronts, those of delta_scan_kernel have a vector unit each, and its shorter step wins: one portion
-    // of 2000 tokens, 16 heads 358 us against 387; of 9000, 32 heads 1702 against 1810.  Beyond, two share one: 32 heads, 16 portions
-    // of 800 tokens 872 us against 711; 60 portions of 110 539 against 444.
-    if (out4 && 2 * (int64_t)a.heads * num_portions > 256 && a.vdim_pad <= 128 && (a.dim_pad == 32 || a.dim_pad == 64 || a.dim_pad == 96 || a.dim_pad == 128)) {
+    // A (portion, head) on half of the compute units or fewer leaves delta_scan_kernel alone on its vector units, and its shorter step wins:
+    // heads of 128 x 128, one portion of 2000 tokens, 16 heads 358 us against 387; of 9000, 32 heads 1702 against 1810.  Beyond, one
+    // workgroup for a head and its outputs wins: 32 heads, 16 portions of 800 tokens 853 us against 712, 60 of 110 512 against 428; heads
+    // of 64 x 64, 5 of 800 183 against 156; of 128 x 16, 5 of 800 465 against 181.  Small heads give most of its eight wavefronts no
+    // columns, which costs where there are more workgroups than compute units, unless delta_out_kernel has no form for the columns
+    // either: 60 portions of 110, heads of 32 x 32 153 us against 195, 32 x 64 201 against 213, 64 x 32 220 against 253, but 32 x 48 210
+    // against 197.
+    const int64_t pairs = (int64_t)a.heads * num_portions;
+    const bool small = a.dim_pad * a.vdim_pad <= 2048 && (a.vdim == 32 || a.vdim == 64);
+    if (out4 && 2 * pairs > 256 && !(small && pairs > 256) && a.vdim_pad <= 128 && (a.dim_pad == 32 || a.dim_pad == 64 || a.dim_pad == 96 || a.dim_pad == 128)) {
 #define GO(N) case N: rc = launch_scan_wide<T, N>(a, portions, num_portions, chunks, records, st); break
         switch (a.dim_pad / 16) { GO(2); GO(4); GO(6); GO(8); }
 #undef GO

@@ -397,9 +397,10 @@ def test_delta_batches_slots_and_padding(gpu):
 
 @BOTH
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,decay", [(36, 18, 32, 16, -2.0), (33, 11, 20, 40, -6.0), (34, 17, 64, 64, 40.0), (36, 9, 96, 72, -2.0),
-                                                           (40, 40, 128, 128, -4.0), (33, 33, 120, 124, 0.0)])
+                                                           (40, 40, 128, 128, -4.0), (33, 33, 120, 124, 0.0), (64, 16, 32, 32, -2.0),
+                                                           (65, 13, 32, 32, -2.0), (66, 11, 64, 32, -2.0), (66, 33, 32, 64, -2.0)])
 def test_delta_batch_that_fills_the_chip(gpu, dtype, heads, kv_heads, dim, vdim, decay):
-    """More than 128 (portion, head) pairs, so that one workgroup holds all columns of a head: portions of one token more than a chunk,
+    """More than 128 (portion, head) pairs, so that one workgroup holds all columns of a head (not of small heads, more than 256 of them): portions of one token more than a chunk,
     of whole chunks and of two tokens, from a first position and continued from the state and the ring they left."""
     n = [[17, 16, 2, 47], [5, 33, 16, 31]]
     cases = [DeltaCase(heads, kv_heads, dim, vdim, 4, a + b, dtype, seed=30 + i, decay=decay, slots=5) for i, (a, b) in enumerate(zip(*n))]
@@ -438,14 +439,14 @@ def test_delta_batch_that_fills_the_chip(gpu, dtype, heads, kv_heads, dim, vdim,
 def test_delta_empty_portions_and_chunks(gpu):
     """In front of the rows and behind them, in one workgroup per head: a portion without chunks keeps its slot's state, or clears it at the
     first position; a chunk without tokens changes nothing."""
-    c = DeltaCase(33, 33, 32, 32, 4, 20, torch.float32, slots=12)
+    c = DeltaCase(33, 33, 32, 16, 4, 20, torch.float32, slots=12)
     chunks = [(0, 0, 0, 0, 1, 0), (0, 16, 0, 0, 1, 0), (16, 4, 16, 0, 1, 0), (0, 0, 20, 0, 1, 0)]
     portions = [(0, 0, 0, 5), (0, 4, 1, 0), (0, 0, 2, 0), (3, 0, 3, 7)] + [(0, 0, 4 + i, 3) for i in range(8)]
     c.state[[0, 3]] = torch.randn(c.state[[0, 3]].shape, device="cuda")
     before = c.state.clone()
     chunks += [(0, 0, 0, 0, 1, 0)] * (len(portions) - len(chunks))
     ring = [(1, 19 - r) for r in range(20)]
-    out = torch.full((20, 33 * 32), float("nan"), device="cuda")
+    out = torch.full((20, 33 * 16), float("nan"), device="cuda")
     ho.delta_chunks(c.s, dev(c.proj), c.beta_off, dev(c.decay), dev(c.gate), *c.weights, c.ring, c.state, dev(portions, torch.int32),
                     dev(chunks, torch.int32), dev(ring, torch.int32), dev(np.arange(20), torch.int64), 0, out)
     want, want_state = c.want()
@@ -455,22 +456,22 @@ def test_delta_empty_portions_and_chunks(gpu):
 
 
 def test_delta_state_of_operands_of_one_sign_does_not_drift(gpu):
-    """3200 tokens without decay whose keys, values and inner results are all positive, beside seven short portions, so that one workgroup
+    """3200 tokens without decay whose keys, values and inner results are all positive, beside six short portions, so that one workgroup
     holds all columns of a head.  Roundings to nearest of the 200 chunks' sums partly cancel: sqrt(200) of them are 14 x 2^-24, as many as
     six of the operands' come on top, and ten of beta = sigmoid(-9), whose exponent is rounded at 9 log2(e) = 13 and so is off by 2^-21, with
     the constant in it: 30 x 2^-24 = 1.8e-6 of the state's norm.  A rounding towards one side, or terms left out of one sign, in each of a
     chunk's products adds up instead."""
     heads, n = 33, 3200
-    c = DeltaCase(heads, 1, 32, 32, 4, n + 7 * 16, torch.float32, slots=8, decay=-20.0)
+    c = DeltaCase(heads, 1, 32, 32, 4, n + 6 * 16, torch.float32, slots=7, decay=-20.0)
     rng, f32 = np.random.default_rng(5), lambda x: rounded(x, torch.float32)
     c.proj, c.conv, c.a_log = f32(0.5 + rng.random(c.proj.shape)), f32(0.2 + 0.2 * rng.random(c.conv.shape)), np.zeros(heads)
     c.proj[:, c.beta_off:] = f32(-9 + 0.1 * rng.standard_normal(c.proj[:, c.beta_off:].shape))
-    chunks = [(r, 16, r, 0, 0, 0) for r in range(0, n, 16)] + [(n + 16 * i, 16, 0, 0, i + 1, 0) for i in range(7)]
-    portions = [(0, n // 16, 0, 0)] + [(n // 16 + i, 1, i + 1, 0) for i in range(7)]
-    ring = [(0, n - 1 - r) for r in range(n)] + [(i + 1, 15 - r) for i in range(7) for r in range(16)]
+    chunks = [(r, 16, r, 0, 0, 0) for r in range(0, n, 16)] + [(n + 16 * i, 16, 0, 0, i + 1, 0) for i in range(6)]
+    portions = [(0, n // 16, 0, 0)] + [(n // 16 + i, 1, i + 1, 0) for i in range(6)]
+    ring = [(0, n - 1 - r) for r in range(n)] + [(i + 1, 15 - r) for i in range(6) for r in range(16)]
     out = torch.empty((c.n, heads * 32), device="cuda")
     ho.delta_chunks(c.s, dev(c.proj), c.beta_off, dev(c.decay), dev(c.gate), *c.weights, c.ring, c.state, dev(portions, torch.int32),
-                    dev(chunks, torch.int32), dev(ring, torch.int32), dev(list(range(n)) + 7 * list(range(16)), torch.int64), 0, out)
+                    dev(chunks, torch.int32), dev(ring, torch.int32), dev(list(range(n)) + 6 * list(range(16)), torch.int64), 0, out)
     state = host(c.state[0])
     c.n = n
     c.proj, c.decay, c.gate = c.proj[:n], c.decay[:n], c.gate[:n]
