@@ -523,7 +523,8 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
     }
     // In place by assembly: all accumulation registers are taken, and the compiler, which moves results around, has none to move them through.
     // It does not know these for matrix instructions and so keeps no distance between them and others: operands come from LDS reads alone, which
-    // it waits for, and nothing but products touches the accumulators between two calls of settle().
+    // it waits for, and nothing but products touches the accumulators between two calls of settle().  Every build is looked over for that
+    // (check_products.py).
     auto product = [](f32x4_t& c, const bf16x8_t& w, const bf16x8_t& x) {
         __asm__ volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
     };
