@@ -302,7 +302,7 @@ int infer_decode_metadata(const int32_t* seq_lens, const int32_t* block_table, i
  * src/bindings.cpp:7) at the batch sizes of a decode step: y[M, N] = x[M, K] . w[N, K]^T, bf16 in, float32 accumulate, bf16 out, M <= 128.  The
  * weights (row-major [N, K], contiguous) are streamed from HBM once; where there are few weight rows, K is
  * cut over workgroups and float32 partial sums pass through `workspace` (infer_skinny_gemm_workspace_bytes says how much,
- * 0 if the shape needs no split).  K must be a multiple of 128 and N a multiple of 8; other shapes
+ * for M rows or fewer; 0 if they need no split).  K must be a multiple of 128 and N a multiple of 8; other shapes
  * return INFER_KV_EUNSUPPORTED and belong to the vendor GEMM. */
 size_t infer_skinny_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int infer_skinny_gemm_bf16(const void* x, int64_t x_stride0, const void* w, void* y, int64_t y_stride0,

@@ -301,6 +301,15 @@ int choose_splits(int64_t m, int64_t n, int64_t k) {
         best = s;
         if (tiles * s >= 256) break;
     }
+    if (m <= 32 || m > 64) return best;
+    // One workgroup of four wavefronts past 64 of the batch fills a compute unit's LDS, so 320 of them take as long as 512: of the smaller
+    // factors, the first with the shortest chain of chunks, where a workgroup's start and end cost as much as four.  Where there are more than
+    // 256 all the same, they have two wavefronts, two to a compute unit.  Unreduced sums, 64 of the batch, us, the first factor with 256
+    // workgroups / this: 3072 x 4096 12.8 / 9.7, 2560 x 4096 12.3 / 9.3, 5120 x 3072 15.0 / 10.6, 2560 x 9728 20.0 / 17.2, 5120 x 12288
+    // 38.0 / 27.4.
+    auto chain = [&](int s) { return (tiles * s + 255) / 256 * (chunks / s + 4); };
+    for (int s = best - 1; s >= 1; --s)
+        if (chunks % s == 0 && chain(s) <= chain(best)) best = s;
     return best;
 }
 
@@ -318,6 +327,7 @@ void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
     else if (a.m <= 32) GO(3, 2, 4, 2);
     else if (a.m <= 64 && rows == 32) GO(2, 4, 4, 2);
     else if (a.m <= 64 && rows == 48) GO(3, 4, 4, 2);
+    else if (a.m <= 64 && rows == 64 && grid.x * grid.y > 256) GO(4, 4, 2, 2);
     else if (a.m <= 64 && rows == 64) GO(4, 4, 4, 2);
     else if (a.m <= 64 && rows == 80 && a.n <= 80 * 512) GO(5, 4, 2, 2);      // all at once, two to a compute unit: n = 32000 60 -> 56 us
     else if (a.m <= 64 && rows == 80) GO(5, 4, 4, 2);                // n = 50000: 92 us, with two wavefronts 106
@@ -331,8 +341,15 @@ void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
 
 extern "C" size_t infer_skinny_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || m > 128 || n <= 0 || k <= 0 || k % kKC != 0) return 0;
-    const int s = choose_splits(m, n, k);
-    return s > 1 ? (size_t)s * (size_t)m * (size_t)n * sizeof(float) : 0;
+    auto need = [&](int64_t rows) {
+        const int s = choose_splits(rows, n, k);
+        return s > 1 ? (size_t)s * (size_t)rows * (size_t)n * sizeof(float) : 0;
+    };
+    // enough for smaller batches as well: 33 rows may be cut less often than 32
+    size_t most = need(m);
+    for (int64_t rows : {8, 16, 32, 64})
+        if (rows < m && need(rows) > most) most = need(rows);
+    return most;
 }
 
 namespace {

@@ -148,6 +148,13 @@ def test_streamed_weights_of_a_long_k(gpu, m, n, k):
     assert torch.equal((deferred.materialize() if isinstance(deferred, ops.SplitKSum) else deferred).float(), want)
 
 
+@pytest.mark.parametrize("m", [33, 48, 64])
+@pytest.mark.parametrize("n,k", [(1536, 9728), (1000, 9728), (4616, 6656), (4608, 3072), (5120, 3200)])
+def test_streamed_weights_cut_into_more_workgroups_than_compute_units_and_fewer(gpu, m, n, k):
+    """As above: more than 256 workgroups of two wavefronts each, and factors that leave 146 and 216 of four."""
+    test_streamed_weights_of_a_long_k(gpu, m, n, k)
+
+
 @pytest.mark.parametrize("m", [1, 16, 17, 40, 64, 65])
 @pytest.mark.parametrize("ff,k", [(8, 128), (2568, 256), (3072, 1024), (4104, 384), (6160, 256), (10248, 128), (12288, 512)])
 def test_gate_and_up_in_one_launch_have_the_bits_of_two(gpu, m, ff, k):
