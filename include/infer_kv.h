@@ -305,6 +305,8 @@ int infer_decode_metadata(const int32_t* seq_lens, const int32_t* block_table, i
  * for M rows or fewer; 0 if they need no split).  K must be a multiple of 128 and N a multiple of 8; other shapes
  * return INFER_KV_EUNSUPPORTED and belong to the vendor GEMM. */
 size_t infer_skinny_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
+/* 1 if the kernels take the sizes and measure faster than the vendor's product; reduced: whether pieces are added up by a launch of their own. */
+int infer_skinny_gemm_pays(int64_t m, int64_t n, int64_t k, int reduced);
 int infer_skinny_gemm_bf16(const void* x, int64_t x_stride0, const void* w, void* y, int64_t y_stride0,
                            int64_t m, int64_t n, int64_t k, void* workspace, size_t workspace_bytes,
                            void* stream);

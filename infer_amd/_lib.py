@@ -44,6 +44,7 @@ SIGNATURES = {
     "infer_silu_and_mul_bf16": (_c.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp]),
     "infer_decode_metadata": (_c.c_int, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
     "infer_skinny_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "infer_skinny_gemm_pays": (_c.c_int, [_i64, _i64, _i64, _c.c_int]),
     "infer_skinny_gemm_bf16": (_c.c_int, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
     "infer_skinny_gate_silu_bf16": (_c.c_int, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "infer_skinny_gemm_partial_bf16": (_c.c_int, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _sz, _vp, _vp]),

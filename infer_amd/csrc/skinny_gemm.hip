@@ -274,15 +274,15 @@ __global__ void __launch_bounds__(256) skinny_gemm_reduce_kernel(ReduceArgs a) {
 // so 33 to 64 want one workgroup per compute unit.  Past a vocabulary (n = 151936) there are many workgroups, and what counts is how little
 // of one passes before and behind its stream: one wavefront that holds 160 rows by itself, two such workgroups to a compute unit, against four
 // that split k of 80 rows and add up: 64 of the batch 259 -> 243 us (k = 4096), 79 -> 67 (k = 1024).  Up to 16, 16 rows are as good as any
-// (n = 24576: 33 to 37 us), except past a vocabulary with a short k: 32 rows 48 us (k = 1024), 16 rows 54, but 215 and 190 with k = 4096.
+// (n = 24576: 33 to 37 us), except past many with a short k: n = 151936 32 rows 48 us (k = 1024), 16 rows 54, but 215 and 190 with k = 4096.
 // Few weight rows and a long k: 16 rows give every compute unit a workgroup that reads the batch once per 16 rows; 64 rows, cut over k, read it a
 // quarter as often.  Unreduced sums, us, 16 / 64 rows: n = 4096, k = 12288 9 of the batch 18.5 / 17.1, 16 20.2 / 17.3, 32 25.9 / 19.0; n = 5120,
 // k = 25600 60 / 52, 69 / 54, 91 / 60; n = 2560, k = 9728 12.7 / 10.4, 14.5 / 10.7, 19.1 / 15.7.  With a shorter k the launch that adds the
 // sums up for those who want them costs more than that (n = 4096, k = 4096, 16: 8.4 / 10.4 reduced, 8.6 / 7.4 unreduced).
-constexpr int64_t kVocabulary = 65536, kLongK = 8192;
+constexpr int64_t kMany = 40960, kVocabulary = 65536, kLongK = 8192;
 int rows_per_workgroup(int64_t m, int64_t n, int64_t k) {
     if (m > 8 && m <= 32 && n <= 5120 && k >= kLongK) return 64;
-    if (m <= 16) return n >= kVocabulary && k <= 2048 ? 32 : 16;
+    if (m <= 16) return n >= kMany && k <= 2048 ? 32 : 16;
     if (m <= 32) return n >= 8192 ? 48 : n > 5120 ? 32 : 16;
     if (m > 64) return kBN;
     if (n <= 5120) return 64;
@@ -337,7 +337,36 @@ void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
 #undef GO
 }
 
+// Whether the kernels are ahead of the vendor's product, from a sweep of 3000 sizes (n of 64 to 262144, k of 128 to 28672) with weights that no
+// cache holds, vendor / these, us.  Inside, 1.3 times as fast on average; outside, sizes of both signs:
+//   65 to 128 of the batch: few weight rows give the vendor too few tiles to fill the chip (o_proj, down_proj: 4096 rows 27 and 68 us against
+//     22 and 38); it is ahead on wider ones and on a short k.
+//   few weight rows: all, except that a split over k whose pieces nobody takes has a launch more (33 to 64 of the batch: 5120 x 1536 8.7 / 11.5,
+//     1024 x 2048 8.0 / 8.6, 1024 x 4096 14.2 / 9.8; 24: 256 x 1024 4.6 / 5.5), and that very few do not fill the chip without one (512 x 768,
+//     40 5.0 / 6.7).
+//   many: a short k (36864 x 128, 16 of the batch 5.7 / 8.4), a long one (5128 x 16384 35.7 / 46.8; 24584 x 28672, 64 275 / 348) and more rows than a
+//     vocabulary has (262144 x 5120, 16 0.86 times as fast) are the vendor's.  Where a workgroup takes long, the last round of them has to be
+//     nearly full: 33 to 64 of the batch 24584 rows 19.7 / 23.0 (k = 1536) and 48.1 / 50.3 (4096), 65528 rows 0.76 to 1.0 times as fast, but 36864
+//     rows 1.25 and 151936 1.1 times; 17 to 32 16384 rows 94.8 / 114.8 (k = 16384) and 0.85 times as fast with k = 5120.
+bool pays(int64_t m, int64_t n, int64_t k, bool reduced) {
+    if (m > 64) return n <= 5120 && k >= 2048;
+    if (n <= 5120) {
+        if (!reduced || k > 2048) return true;
+        if (m <= 32) return n >= 512 || k == 2048 || choose_splits(m, n, k) == 1;
+        return n >= 2048 && (k == 2048 || choose_splits(m, n, k) == 1);
+    }
+    if ((k < 512 && n > 20480) || k > 12288 || n > 163840) return false;
+    const int64_t rows = rows_per_workgroup(m, n, k), groups = (n + rows - 1) / rows, rounds = (groups + 255) / 256;
+    if (m <= 16) return true;
+    if (m <= 32) return k <= 2048 || 10 * groups >= 7 * 256 * rounds;
+    return n <= 24576 || 20 * groups >= 17 * 256 * rounds;
+}
+
 }  // namespace
+
+extern "C" int infer_skinny_gemm_pays(int64_t m, int64_t n, int64_t k, int reduced) {
+    return m > 0 && m <= 128 && n > 0 && k > 0 && k % kKC == 0 && n % 8 == 0 && pays(m, n, k, reduced != 0);
+}
 
 extern "C" size_t infer_skinny_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (m <= 0 || m > 128 || n <= 0 || k <= 0 || k % kKC != 0) return 0;

@@ -500,25 +500,13 @@ _linear_choice: dict = {}
 _linear_timings: dict = {}      # (device, batch bucket, N, K) -> (vendor ms, own ms), for inspection
 _flush_buffers: dict = {}
 
-# Up to this many rows of the batch the streaming kernel is ahead of the vendor GEMM on every weight matrix measured (1024 to 151936
-# rows, K of 1024 to 12288; us, vendor / streaming): 1 row 8.0 / 2.9 on 1024 x 2048, 44 / 33 on 24576 x 4096, 244 / 188 on 151936 x 4096;
-# 16 rows 7.5 / 3.9 on 4096 x 1024, 44 / 37, 254 / 214; 64 rows 49 / 40, 262 / 257.
+# Up to this many rows of the batch, the streaming kernels and the launch of gate, up and activation
 STREAM_MAX_BATCH = 64
-# Beyond, weight matrices with at most this many rows go to the split-K kernel: the vendor
-# GEMM has too few output tiles to fill the chip there (o_proj, down_proj: 4096 rows = 32 tiles of 128 on
-# 256 compute units, 27 and 68 us against 22 and 38), and is ahead on every wider projection measured
-# (qkv 6144, gate_up 24576, lm_head 151936 rows) and on short reductions (K below 2048).  On the three
-# published Qwen3 shapes the rule picks what a cold-cache timing of both kernels picks, within 2.5 %
-# of a decode step on the smallest.
-SKINNY_MAX_ROWS = 5120
 
 
 def _own_kernel(m: int, n: int, k: int, defer: bool) -> bool:
-    if m > STREAM_MAX_BATCH:
-        return n <= SKINNY_MAX_ROWS and k >= 2048
-    # a split over k whose pieces nobody takes has a launch more: 1024 x 2048, 48 rows 8.6 us against 8.0 (5.7 unreduced); 1024 x 3072
-    # 9.5 against 10.5, 1024 x 4096 9.8 against 14.2
-    return defer or m <= 32 or n >= 2048 or k > 2048
+    """Whether the kernels of this package measure faster than the vendor's product, by sizes alone."""
+    return bool(_lib.load().infer_skinny_gemm_pays(m, n, k, not defer))
 
 
 def _linear_mode() -> str:
@@ -597,8 +585,8 @@ def _row_stride(x: torch.Tensor) -> int:
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, defer: bool = False):
-    """``F.linear(x, weight)`` that sends decode-sized batches to the weight-streaming kernels (more than 64 rows: over narrow
-    weight matrices only) and everything else to the vendor GEMM.  The choice is a fixed rule on the
+    """``F.linear(x, weight)`` that sends decode-sized batches to the weight-streaming kernels where they are ahead (``_own_kernel``)
+    and everything else to the vendor GEMM.  The choice is a fixed rule on the
     shape (see ``_linear_mode`` for the alternatives), so a shape runs the same kernel, with the same
     rounding, in every process and inside and outside a captured graph."""
     if not _streamable(x, weight):
