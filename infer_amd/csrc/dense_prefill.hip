@@ -95,9 +95,10 @@ __device__ __forceinline__ void finish(const DensePrefillArgs& a, f32x4_t (&acc)
 
 // Sequence, block of queries and head of the workgroup with index `wg`, the longest work first.  Late blocks see the most keys, so a head's
 // blocks go by their place in the sequence, over all sequences: the chip runs dry together (6 ragged sequences of 32 heads 341 -> 332 us, 8 x
-// 2048 in chunks 480 -> 432).  A die hands its workgroups to its four shader engines in turn; the rotation keeps an engine from getting the same
-// sequences every time.  Where that gains nothing the blocks of a sequence stay together, whose keys are then read once: nearly all workgroups
-// run at once (480 of them: 50 us against 51), or a window ends before the sequences do, so that most blocks see as many keys (287 us against 283).
+// 2048 in chunks 480 -> 432).  A die hands its workgroups to its four shader engines in turn; the rotation (two sequences: in every second row)
+// keeps an engine from getting the same sequences every time.  Where that gains nothing the blocks of a sequence stay together, whose keys
+// are then read once: nearly all workgroups run at once (480 of them: 50 us against 51), or a window ends before the sequences do, so that
+// most blocks see as many keys (287 us against 283).
 struct Place { int b, qblk, h; };
 __device__ __forceinline__ Place place_of(const DensePrefillArgs& a, unsigned wg, unsigned total, int queries) {
     const unsigned blocks = (unsigned)a.qblocks, seqs = (unsigned)a.nseq;
@@ -105,7 +106,7 @@ __device__ __forceinline__ Place place_of(const DensePrefillArgs& a, unsigned wg
     if (total <= 1024 || (a.mask.kind == 2 && a.mask.size < (int64_t)blocks * queries))
         return {(int)(wg / blocks % seqs), (int)(blocks - 1 - wg % blocks), h};
     const unsigned row = wg / seqs;
-    return {(int)((wg + row) % seqs), (int)(blocks - 1 - row % blocks), h};
+    return {(int)((wg + (seqs == 2 ? row / 2 : row)) % seqs), (int)(blocks - 1 - row % blocks), h};
 }
 
 template <int KS, int VT, int MAPS>

@@ -143,9 +143,12 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     const unsigned wg_id = __builtin_amdgcn_readfirstlane(die * per_die + (die < extra ? die : extra) + (wg_linear >> 3));
     // Query blocks of all sequences by their place in the sequence, the late ones, which see the most keys, first: the die
     // runs dry together (16 sequences of 64 .. 2048 272 -> 265 us, 8 of 800 69 -> 62).  A die hands its workgroups to its four
-    // shader engines in turn: without the rotation an engine gets the same sequences every time (306 us against 298).
-    const int b = (int)((wg_id + wg_id / gridDim.y) % gridDim.y);
-    const int block_x = (int)((wg_id / gridDim.y) % gridDim.x);
+    // shader engines in turn: without the rotation an engine gets the same sequences every time (306 us against 298).  Two
+    // sequences one behind the other: in rows of two, two engines get one of them each (2588 and 5177 tokens, 16 heads 207 us
+    // against 159; turned in every second row 174).
+    const bool by_place = gridDim.y > 2;
+    const int b = (int)((by_place ? wg_id + wg_id / gridDim.y : wg_id / gridDim.x) % gridDim.y);
+    const int block_x = (int)((by_place ? wg_id / gridDim.y : wg_id) % gridDim.x);
     const int block_z = (int)(wg_id / (gridDim.x * gridDim.y));
     const int parts = a.group / kHeads;                    // workgroups that share one KV head
     const int kvh = block_z / parts;

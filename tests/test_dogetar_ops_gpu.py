@@ -301,12 +301,15 @@ def test_masked_prefill_around_the_steps_of_the_ring(gpu, dim, vdim, maps, mask,
     assert (out[-1] == 9.0).all()
 
 
+@pytest.mark.parametrize("lens", [[5, 16, 1, 290, 40, 3, 130, 2, 9, 12, 4], [1100, 150]])
 @pytest.mark.parametrize("maps,dim,vdim,mask,size", [(1, 64, 128, None, 1), (2, 64, 128, "chunk", 100), (1, 24, 16, "window", 500), (1, 64, 80, "window", 70)])
-def test_masked_prefill_of_more_workgroups_than_run_at_once(gpu, maps, dim, vdim, mask, size):
-    """More than 1024 workgroups: their blocks go by place over the sequences (a window that ends before the sequences: by sequence)."""
+def test_masked_prefill_of_more_workgroups_than_run_at_once(gpu, maps, dim, vdim, mask, size, lens):
+    """More than 1024 workgroups: their blocks go by place over the sequences (a window that ends before the sequences: by sequence; two
+    sequences change places in every second row)."""
+    if len(lens) == 2 and maps == 1:
+        lens = [2 * lens[0], lens[1]]
     rng, bf, heads = np.random.default_rng(dim + vdim), torch.bfloat16, 32
     s = ho.MaskedShape(heads, 4, dim, vdim, 0.5 * dim ** -0.5, maps=maps, mask=mask, mask_size=size, distance_bias=False, out_scale=0.6, lam=0.7, eps=1e-3)
-    lens = [5, 16, 1, 290, 40, 3, 130, 2, 9, 12, 4]
     p = Pages(rng, lens, s, 64, bf)
     cu_n = np.cumsum([0] + lens)
     cu = dev(cu_n, torch.int32)

@@ -137,6 +137,15 @@ def test_random_ragged_batches(gpu, seed):
     assert err <= ATTN_ATOL, (hq, hkv, bs, lens, cached, float(err))
 
 
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (3, 1), (10, 2)])
+@pytest.mark.parametrize("lens,cached", [([1, 700], [0, 0]), ([417, 290], [0, 256]), ([1300, 40], [256, 0]), ([64, 64], [0, 0])])
+def test_two_sequences(gpu, hq, hkv, lens, cached):
+    """Their blocks are handed out one sequence behind the other, those of more in rows of one of each."""
+    wl = workloads.make_prefill_workload("two", lens, cached, hq, hkv, seed=sum(lens) + hq).to(gpu)
+    out, kc, vc = run_paged(wl)
+    assert np.abs(f32(out) - oracle_paged(wl, kc, vc)).max() <= ATTN_ATOL
+
+
 def test_packed_keys_without_block_table_equals_causal_sdpa(gpu):
     """No prefix cached: K and V are the packed new rows and sq == sk, which reduces to
     scaled_dot_product_attention(is_causal=True), the convention of the reference's own attention
