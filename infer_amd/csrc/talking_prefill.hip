@@ -526,12 +526,15 @@ void plan(int64_t heads, int64_t num_seqs, int64_t max_seqlen_q, int64_t max_key
     if (splits < 1) splits = 1;
 }
 
-// Eight sequences, sixteen, ...: where each belongs to a die its keys are read once, but a die with the longest one works on when the others
+// Eight sequences, or sixteen: where each belongs to a die its keys are read once, but a die with the longest one works on when the others
 // are done.  Runs of blocks, unless the lengths are nearly equal or all blocks of the mixture run at once (mixture and sums of exponentials, us,
-// shares / runs: 8 sequences of 700 .. 2300 397 / 323, 16 of 100 .. 1500 324 / 227, 8 of 1500 252 / 260, single blocks there 318).  Other numbers
-// of sequences spread by themselves (6 of 1214 .. 2313: 360 / 407).
+// shares / runs: 8 sequences of 700 .. 2300 397 / 323, 16 of 100 .. 1500 324 / 227, 8 of 1500 252 / 260, single blocks there 318).  Two sequences
+// of a die even out between them, so that sixteen have to differ more (of 56 .. 922 165 / 122, of 990 .. 1292 272 / 289), and more of them do
+// without runs (24 of 151 .. 441 76 / 91, 48 of 61 .. 179 45 / 65, 64 of 161 .. 245 85 / 108).  Other numbers of sequences spread by themselves
+// (6 of 1214 .. 2313: 360 / 407).
 bool uneven_dies(const TalkPrefillArgs& a, int64_t max_seqlen_q) {
-    return a.nseq % 8 == 0 && (max_seqlen_q + 31) / 32 * a.nseq > 256 && 10 * a.tokens < 9 * a.nseq * max_seqlen_q;
+    const int64_t longest = a.nseq * max_seqlen_q;     // tokens if all were as long
+    return (max_seqlen_q + 31) / 32 * a.nseq > 256 && ((a.nseq == 8 && 10 * a.tokens < 9 * longest) || (a.nseq == 16 && 4 * a.tokens < 3 * longest));
 }
 // a run, so that every die gets eight of them if there are as many
 int64_t run_of(int64_t pairs, int64_t qblocks, int64_t most) {

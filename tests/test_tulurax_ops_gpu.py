@@ -363,7 +363,8 @@ def test_prefill_and_rows_agree(gpu, heads, lens):
 
 @pytest.mark.parametrize("heads,lens", [(12, [1100, 40, 7, 300, 64, 200, 33, 96]), (16, [30, 700, 5, 64, 100, 31, 32, 33] * 2), (8, [2, 80, 1] * 8 + [401] * 8)])
 def test_prefill_of_uneven_sequences_on_all_dies(gpu, heads, lens):
-    """Eight sequences or a multiple of it, of unequal lengths and more blocks than run at once: runs of blocks go to the dies in turn."""
+    """A multiple of eight sequences of unequal lengths and more blocks than run at once: of eight and sixteen, runs of blocks go to the dies
+    in turn; of more, a die has its own sequences."""
     assert len(lens) % 8 == 0 and -(-max(lens) // 32) * len(lens) > 256 and 10 * sum(lens) < 9 * len(lens) * max(lens)
     test_prefill_and_rows_agree(gpu, heads, lens)
 
