@@ -728,15 +728,21 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t max_places, hipStrea
 // rows per tile: 0 where only the any-size kernels serve
 int rows_per_tile(int elem, int64_t n, int64_t width, int64_t ff_pad, int64_t experts, int64_t top) {
     if (elem != INFER_ELEM_BF16 || width % 8 || ff_pad % 8) return 0;
-    // an expert with more than one tile of 32 rows reads its weights again (of 14 experts of 3072 x 4096, tiles of 32 rows / blocks, us: 118 rows
-    // 252 / 268, 140 284 / 304, 180 357 / 300)
-    if (n * top <= 32 * experts) return kSmallRows;
+    // An expert with more than one tile of 32 rows reads its weights again, and around 32 choices per expert half of them have more.  That costs
+    // little where the weights are few, more where there are many of them or many experts; us, tiles of 32 rows / the others: 8 experts of
+    // 1536 x 4096, 32 choices each 105 / 136; 8 of 2048 x 8192, 28 234 / 275; 14 of 4096 x 3072, 25 261 / 282, 32 330 / 280; 8 of 4096 x 14336, 26
+    // 685 / 642; 32 of 2880 x 2880, 25 405 / 380, 32 507 / 375; 128 of 2048 x 768, 26 351 / 305, 32 419 / 312.
+    const double weights = 6.0 * experts * width * ff_pad;       // bytes
+    if (n * top <= (weights <= 3.2e8 ? 32 : experts <= 16 && weights <= 2e9 ? 28 : 24) * experts) return kSmallRows;
     // Large blocks pay where they are enough to fill most of the chip (of 14 experts, tiles of 128 rows / blocks, us: 3072 x 4096, 200 rows
-    // 319 / 295, 800 471 / 322, 2100 879 / 510; 768 x 1024, 600 rows 57 / 66, 1200 67 / 71, 2300 104 / 81).  Their offsets are 32 bits.
+    // 319 / 295, 800 471 / 322, 2100 879 / 510; 768 x 1024, 600 rows 57 / 66, 1200 67 / 71, 2300 104 / 81).  More than a round of them, of few rows
+    // and a short k, does not: with 33 choices each 14 experts of 1024 x 3072 109 / 133, 24 of 2048 x 3072 233 / 257, 8 of 2048 x 8192 274 / 293.
+    // Their offsets are 32 bits.
     const int64_t far = 1ll << 31;
     const bool fits = width % 64 == 0 && ff_pad % 64 == 0 && n * width < far && n * top * ff_pad < far && 2 * ff_pad * width < far;
-    const int64_t blocks = (n * top / kBlockRows + experts / 2) * ((ff_pad + 127) / 128);      // of the first product, about
-    return fits && (n * top >= 512 * experts || (blocks >= 160)) ? kBlockRows : kBigRows;
+    const int64_t columns = (ff_pad + 127) / 128, blocks = (n * top / kBlockRows + experts / 2) * columns, work = n * top * width;   // first product, about
+    const bool worth = width >= 2880 || experts * columns <= 256 || work >= 150000 * experts || work >= 2200000;
+    return fits && (n * top >= 512 * experts || (blocks >= 160 && worth)) ? kBlockRows : kBigRows;
 }
 
 }  // namespace
