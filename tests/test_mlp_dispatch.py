@@ -1,5 +1,7 @@
-"""`MLP.forward` takes its first projection and the gate in one launch only where nobody could tell: on the host, with stand-ins for the
-kernels."""
+"""`MLP.forward` takes its first projection and the gate in one launch, and `Linear.forward` leaves sums in pieces, only where nobody could
+tell: on the host, with stand-ins for the kernels."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -111,3 +113,18 @@ def test_backward_hooks_are_called(mlp):
     mlp.gate_up_proj.register_full_backward_hook(lambda module, inputs, outputs: seen.append(module))
     mlp(rows().clone().requires_grad_()).sum().backward()
     assert seen == [mlp.gate_up_proj] and mlp.fused == 0
+
+
+@pytest.mark.parametrize("register", [nn.Module.register_forward_hook, nn.Module.register_full_backward_hook,
+                                      lambda layer, hook: modules.register_module_forward_hook(hook),
+                                      lambda layer, hook: modules.register_module_full_backward_hook(hook)])
+def test_hooks_see_a_tensor_and_not_sums_in_pieces(monkeypatch, register):
+    monkeypatch.setattr(ops, "linear", lambda x, weight, defer=False: "pieces" if defer else "tensor")
+    layer, x = layers.Linear(256, 64), SimpleNamespace(shape=torch.Size((4, 256)), is_cuda=True, dim=lambda: 2)
+    assert layer.forward(x, defer=True) == "pieces" and layer.forward(x) == "tensor"
+    handle = register(layer, lambda module, args, result: None)
+    try:
+        assert layer.forward(x, defer=True) == "tensor"
+    finally:
+        handle.remove()
+    assert layer.forward(x, defer=True) == "pieces"
