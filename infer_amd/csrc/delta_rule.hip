@@ -629,7 +629,7 @@ __host__ __device__ constexpr int wide_buffer_units(int dt) { return 64 * (5 * d
 // so they do not pass through memory in between.
 // A batch takes as long as its longest portion's chunks one after the other; a step of eight wavefronts on a compute unit is 3200 clocks
 // of matrix pipe per wavefront with float products and 1200 with pieces, which cost about 180 vector instructions.  32 heads, 8 portions
-// of 590 to 2560 tokens: scan, output and ring 662 us with delta_scan_kernel, 525 us here (kernels alone, under a profiler; the call 963 and
+// of 590 to 2560 tokens: scan, output and ring 662 us with delta_scan_kernel, 515 us here (kernels alone, under a profiler; the call 963 and
 // 807 us).  What a step waits for is requested a step before, by every thread and without branches: with requests in branches, or
 // stores between a request and its use, the compiler waits for everything in flight.  Tried as well, against 435 us of a first form: 830
 // with such requests; float products for W S 690; the two wavefronts of a vector unit in opposite phases 550; four wavefronts that only
