@@ -60,6 +60,9 @@ const char* infer_kv_strerror(int code);
  * calls this once per device beforehand.  Thread safe; later calls return at once. */
 int infer_kv_init(void);
 
+/* The identity of the capture that `stream` is part of, the same for all streams of one capture and for no other capture; 0: none. */
+uint64_t infer_stream_capture_id(void* stream);
+
 /* ------------------------------------------------------------------ 1. KV append
  * Replaces store_kvcache / store_kvcache_kernel (infer/ops/attention.py:16-45), called from
  * Attention.forward_offical_fa_impl (infer/ops/attention.py:108-109).

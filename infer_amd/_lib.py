@@ -140,6 +140,7 @@ SIGNATURES = {
     "infer_pool_can_append": (_c.c_int, [_vp, _i64]),
     "infer_pool_may_append": (_i64, [_vp, _vp, _i64, _vp, _i64, _i64]),
     "infer_pool_may_append_block": (_i64, [_vp, _vp, _i64, _vp, _i64, _i64]),
+    "infer_stream_capture_id": (_c.c_uint64, [_vp]),
     "infer_pool_hash": (_c.c_uint64, [_vp, _i64, _c.c_int, _c.c_uint64]),
     "infer_xxh64": (_c.c_uint64, [_vp, _sz, _c.c_uint64]),
     "infer_pool_ref_count": (_i32, [_vp, _i32]),

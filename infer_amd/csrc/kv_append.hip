@@ -199,6 +199,12 @@ int infer_kv_append_bf16(const void* key, int64_t key_stride0, const void* value
 
 const char* infer_kv_version(void) { return "0.3"; }
 
+uint64_t infer_stream_capture_id(void* stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    return hipStreamGetCaptureInfo((hipStream_t)stream, &status, &id) == hipSuccess && status == hipStreamCaptureStatusActive ? id : 0;
+}
+
 const char* infer_kv_strerror(int code) {
     switch (code) {
         case INFER_KV_OK: return "ok";

