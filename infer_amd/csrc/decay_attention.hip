@@ -138,7 +138,7 @@ struct ChunkArgs {
     DecayOutArgs<__bf16> b;
     bool finish;                                 // norm (per head) and gate here; a.o is not written
     const Span* spans;
-    int seg_len, max_seg, slabs;                 // tokens per segment (a multiple of kC), segments of the longest span
+    int seg_len, max_seg, slabs;                 // most tokens of a segment (a multiple of kC), segments of the longest span
     float* ws;                                   // [span][max_seg][heads][dim_pad][vdim_pad], if max_seg > 1
 };
 
@@ -160,6 +160,13 @@ __device__ __forceinline__ u32x4_t silu8(u32x4_t x) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) r[i] = (__bf16)silu_f(y[i]);
     return __builtin_bit_cast(u32x4_t, r);
+}
+
+// Tokens of a segment of a portion of `count`: as many segments as `most` tokens each would make, all of one length but for the last one's
+// rest, so that a portion a little longer than `most` does not leave a workgroup with almost nothing.
+__device__ __forceinline__ int own_segment(int count, int most) {
+    const int segs = (count + most - 1) / most;
+    return segs > 1 ? ((count + segs - 1) / segs + kC - 1) / kC * kC : most;
 }
 
 // A workgroup of four wavefronts serves one head and 64 VT columns of its state over the chunks of one segment.
@@ -186,11 +193,11 @@ __global__ void __launch_bounds__(256, 2) decay_chunk_kernel(ChunkArgs args) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
     const Span span = args.spans[blockIdx.z];
-    const int first = seg * args.seg_len;
+    const int seg_len = own_segment(span.count, args.seg_len), first = seg * seg_len;
     if (span.slot < 0 || span.slot >= a.num_slots || first >= span.count) return;
-    const bool last_seg = first + args.seg_len >= span.count;
+    const bool last_seg = first + seg_len >= span.count;
     if (!OUT && last_seg) return;                                // nobody needs its final state yet
-    const int count = last_seg ? span.count - first : args.seg_len;
+    const int count = last_seg ? span.count - first : seg_len;
     const int row0 = span.row0 + first, pos0 = span.pos0 + first, chunks = (count + kC - 1) / kC;
     const int v0 = slab * kSlab + wave * 16 * VT;                // this wavefront's first column
     const bool live = v0 < a.vdim_pad;
@@ -553,13 +560,14 @@ __global__ void __launch_bounds__(kThreads) decay_join_kernel(ChunkArgs args) {
     const Span span = args.spans[blockIdx.z];
     const int64_t state_len = (int64_t)a.dim_pad * a.vdim_pad, i = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 4;
     if (span.slot < 0 || span.slot >= a.num_slots || i >= state_len) return;
-    const float seg_decay = exp2f((float)args.seg_len * a.decay[2 * a.heads + h]);
+    const int seg_len = own_segment(span.count, args.seg_len);
+    const float seg_decay = exp2f((float)seg_len * a.decay[2 * a.heads + h]);
     f32x4_t s = {0.f, 0.f, 0.f, 0.f};
     if (span.pos0 > 0) s = *reinterpret_cast<const f32x4_t*>(a.state + ((int64_t)span.slot * a.heads + h) * state_len + i);
-    for (int seg = 0; seg * args.seg_len < span.count; ++seg) {
+    for (int seg = 0; seg * seg_len < span.count; ++seg) {
         f32x4_t* p = reinterpret_cast<f32x4_t*>(args.ws + (((int64_t)blockIdx.z * args.max_seg + seg) * a.heads + h) * state_len + i);
         f32x4_t add = {0.f, 0.f, 0.f, 0.f};
-        if ((seg + 1) * args.seg_len < span.count) add = *p;
+        if ((seg + 1) * seg_len < span.count) add = *p;
         *p = s;
         s = s * seg_decay + add;
     }
@@ -774,10 +782,14 @@ int slabs_of(int64_t dim_pad, int64_t vdim_pad) {
     const int cols = 64 * column_tiles(dim_pad, vdim_pad);
     return (int)((vdim_pad + cols - 1) / cols);
 }
-// tokens per segment: enough segments for two workgroups per compute unit, none shorter than four chunks
+// Most tokens of a segment: enough segments for two workgroups per compute unit, none shorter than four chunks; portions that fill the chip
+// with one workgroup per compute unit stay whole, since cut ones are walked twice.  Heads of 128 x 128, the call in us, cut / whole: 32 heads, 8
+// portions of 1500 tokens 252 / 212, 10 of 800 to 1800 297 / 273, 12 of 100 to 1500 284 / 241; 16 heads, 16 of 100 to 1500 209 / 179; but 32
+// heads, 6 of 900 to 3700 320 / 390; 16 heads, 10 of 800 to 1800 190 / 209.  Segments of one length per portion instead of one for the batch:
+// 6 portions of 900 to 3700 of 32 heads 338 -> 320, 5 of them 347 -> 298.
 int64_t segment_len(int64_t heads, int64_t slabs, int64_t num_spans, int64_t max_span) {
     const int64_t groups = heads * slabs * num_spans;
-    int64_t n = (512 + groups - 1) / groups;
+    int64_t n = groups >= 256 ? 1 : (512 + groups - 1) / groups;
     const int64_t most = max_span / (4 * kC);
     if (n > most) n = most;
     if (n <= 1) return (max_span + kC - 1) / kC * kC;

@@ -268,10 +268,17 @@ __global__ void __launch_bounds__(kThreads) ssm_scan_any_kernel(SsmArgs<T> a, co
 struct ChunkArgs {
     SsmArgs<__bf16> a;
     const Span* spans;
-    int seg_len, max_seg, slabs;                 // tokens per segment (a multiple of kC), segments of the longest span
+    int seg_len, max_seg, slabs;                 // most tokens of a segment (a multiple of kC), segments of the longest span
     float* ws;                                   // [span][max_seg][heads][state][vdim], then [span][max_seg][heads]: log2 of the decay
     float* ws_decay;
 };
+
+// Tokens of a segment of a portion of `count`: as many segments as `most` tokens each would make, all of one length but for the last one's
+// rest, so that a portion a little longer than `most` does not leave a workgroup with almost nothing.
+__device__ __forceinline__ int own_segment(int count, int most) {
+    const int segs = (count + most - 1) / most;
+    return segs > 1 ? ((count + segs - 1) / segs + kC - 1) / kC * kC : most;
+}
 
 // A workgroup of four wavefronts serves one head and 64 columns of its state over the chunks of one segment; wavefront w owns 16
 // columns as accumulators: lane (g, n) holds state rows 16 t + 4 g + e of column n.  That is an operand of the product with C as it
@@ -289,11 +296,11 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
     const Span span = args.spans[blockIdx.z];
-    const int first = seg * args.seg_len;
+    const int seg_len = own_segment(span.count, args.seg_len), first = seg * seg_len;
     if (span.slot < 0 || span.slot >= a.num_slots || first >= span.count) return;
-    const bool last_seg = first + args.seg_len >= span.count;
+    const bool last_seg = first + seg_len >= span.count;
     if (!OUT && last_seg) return;                                // nobody needs its final state yet
-    const int count = last_seg ? span.count - first : args.seg_len;
+    const int count = last_seg ? span.count - first : seg_len;
     const int row0 = span.row0 + first, chunks = (count + kC - 1) / kC;
     const int N = a.state_n, inner = a.heads * a.vdim, grp = h / (a.heads / a.groups);
     const int v0 = slab * kSlab + wave * 16;                     // this wavefront's first column
@@ -496,7 +503,7 @@ __global__ void __launch_bounds__(kThreads) ssm_join_kernel(ChunkArgs args) {
     const int64_t state_len = (int64_t)a.state_n * a.vdim, i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= state_len || span.slot < 0 || span.slot >= a.num_slots) return;
     float cur = span.pos0 > 0 ? a.state[((int64_t)span.slot * a.heads + h) * state_len + i] : 0.f;
-    const int segs = (span.count + args.seg_len - 1) / args.seg_len;
+    const int seg_len = own_segment(span.count, args.seg_len), segs = (span.count + seg_len - 1) / seg_len;
     for (int k = 0; k < segs; ++k) {
         const int64_t rec = ((int64_t)blockIdx.z * args.max_seg + k) * a.heads + h;
         float* w = args.ws + rec * state_len + i;
@@ -580,10 +587,14 @@ __global__ void __launch_bounds__(kThreads) ssm_norm_kernel(NormArgs<T> b) {
 // ------------------------------------------------------------------ launches
 bool chunked(int elem, int64_t vdim, int64_t state_n) { return elem == INFER_ELEM_BF16 && vdim % 8 == 0 && state_n % 8 == 0 && state_n <= 256; }
 
-// segments that portions are cut into, so that enough workgroups run: tokens per segment and their largest number
+// Segments that portions are cut into, so that enough workgroups run: most tokens of a segment and their largest number.  Cut portions are
+// walked twice, which pays below one and a half workgroups per compute unit.  Heads of 128 x 64, the call in us, cut for three workgroups per
+// compute unit / whole: 12 portions of 100 to 1500 tokens of 32 heads 181 / 172, 6 of 900 to 3700 of 64 heads 337 / 325, 7 of them
+// 385 / 348; but 5 of them 268 / 297, 4 of 500 to 3000 207 / 239.  Segments of one length per portion instead of one for the batch: 6 portions
+// of 32 heads 228 -> 220, 2 of 2000 to 5000 of 64 heads 181 -> 174.
 void segments(int64_t heads, int64_t slabs, int64_t num_spans, int64_t max_span, int64_t& seg_len, int64_t& max_seg) {
     const int64_t units = heads * slabs * num_spans, chunks = (max_span + kC - 1) / kC;
-    int64_t want = units > 0 && units < 512 ? (768 + units - 1) / units : 1;       // three workgroups per compute unit
+    int64_t want = units > 0 && units < 384 ? (768 + units - 1) / units : 1;       // three workgroups per compute unit
     if (want > chunks / 4) want = chunks / 4;              // no segment shorter than four chunks
     if (want < 1) want = 1;
     const int64_t per = (chunks + want - 1) / want;

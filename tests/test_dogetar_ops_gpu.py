@@ -417,6 +417,22 @@ def test_state_space_segments_of_a_long_portion(gpu, shape):
     close(m.state[2], states, 1e-2)
 
 
+@pytest.mark.parametrize("lens", [(1333, 127, 128, 129, 161), (640, 641, 33), (700, 1, 2, 257)])
+def test_state_space_portions_are_cut_by_their_own_lengths(gpu, lens):
+    """Portions of one call around the lengths at which another segment begins: segments of equal length per portion, joined by their own decay."""
+    m = Ssm(np.random.default_rng(len(lens)), SSM[2], torch.bfloat16, a_log=(-9.0, -5.0))
+    x = [m.inputs(n) for n in lens]
+    want = [m.want(a) for a in x]
+    order = sorted(range(len(lens)), key=lambda i: lens[i] > 1)              # decoded tokens come first
+    first = {i: a[:20] for i, a in enumerate(x) if len(a) > 40}
+    if first:
+        m.run([(i, 0, a) for i, a in first.items()])
+    got = m.run([(i, len(first.get(i, ())), x[i][len(first.get(i, ())):]) for i in order])
+    for i, y in zip(order, got):
+        close(torch.tensor(y), want[i][0][len(first.get(i, ())):], 2e-2)
+        close(m.state[i], want[i][1], 1e-2)
+
+
 @BOTH
 @pytest.mark.parametrize("a_log,dt", [((4.0, 9.0), 3.0), ((-20.0, -12.0), 1.0), ((-1.0, 0.0), 12.0)])
 def test_state_space_extreme_decays(gpu, dtype, a_log, dt):

@@ -403,6 +403,26 @@ def test_decay_segments(gpu, kind, n):
 
 
 @BYKIND
+@pytest.mark.parametrize("lens", [(1333, 127, 128, 129, 161), (640, 641, 33), (700, 257, 300)])
+def test_decay_portions_are_cut_by_their_own_lengths(gpu, kind, lens):
+    """Portions of one call around the lengths at which another segment begins: segments of equal length per portion, joined by their own decay."""
+    bf = torch.bfloat16
+    d = Decay(kind, (0.99951171875, 0.9, 1.0), 64, 64, 64, bf, seed=sum(lens))
+    x = rounded(d.inputs(sum(lens)) * 0.05, bf)
+    state, spans, row = d.state(len(lens)), [], 0
+    starts = [d.rng.standard_normal((3, 64, 64)) if i % 2 else np.zeros((3, 64, 64)) for i in range(len(lens))]
+    for i, n in enumerate(lens):
+        d.fill(state, i, starts[i])
+        spans.append((row, n, i, 7 * (i % 2)))
+        row += n
+    out = d.run(x, state, None, None, 0, spans)
+    for row, n, i, pos0 in spans:
+        want, end = d.want(x[row:row + n], pos0, starts[i], round_silu=True)
+        close(out[row:row + n], want, 2e-2)
+        d.check_state(state, i, end, 6e-3 if kind == "lightning" else 3e-6)
+
+
+@BYKIND
 def test_decay_state_does_not_drift_over_many_steps(gpu, kind):
     """4000 decoded tokens of zeros: what is left of the state is decay^4000 of it to float precision."""
     d = Decay(kind, (1.0 - 1.1e-4, 0.9998), 32, 32, 32, torch.float32)
