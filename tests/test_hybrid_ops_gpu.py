@@ -224,6 +224,28 @@ def test_latent_gather(gpu):
     assert np.array_equal(host(out), np.concatenate([keys[2], keys[0]]))
 
 
+@pytest.mark.parametrize("block", [1, 31, 32, 48, 64, 256])
+@pytest.mark.parametrize("heads,row", [(1, 8), (1, 576), (3, 40), (8, 256)])
+def test_gather_of_pages_of_any_size(gpu, heads, row, block):
+    """Rows of every token of every head, bit for bit: pages that end within a workgroup's tokens, rows that no power of two divides."""
+    lens = [0, 1, 31, 32, 33, 65, 300, 2 * block]
+    gen = torch.Generator().manual_seed(row + block)
+    per = [-(-n // block) for n in lens]
+    cache = torch.randn(sum(per) + 2, heads, block, row, generator=gen).to(torch.bfloat16)
+    order, at = torch.randperm(sum(per) + 2, generator=gen).tolist(), 0
+    tables = torch.full((len(lens), max(per)), -1, dtype=torch.int32)
+    for i, n in enumerate(per):
+        tables[i, :n] = torch.tensor(order[at:at + n], dtype=torch.int32)
+        at += n
+    seqs, want = [5, 2, 0, 7, 6, 1, 3, 4], []
+    for s in seqs:
+        t = torch.arange(lens[s])
+        want.append(cache[tables[s][t // block].long(), :, t % block])
+    cu = torch.tensor([0] + [lens[s] for s in seqs]).cumsum(0).to(torch.int32)
+    out = ho.grouped_gather(cache.cuda(), tables.cuda(), torch.tensor(seqs, dtype=torch.int32).cuda(), cu.cuda(), int(cu[-1]), max(lens))
+    assert torch.equal(out.cpu(), torch.cat(want))
+
+
 @pytest.mark.parametrize("heads,dim,rot,vdim", [(3, 16, 8, 24), (5, 48, 16, 40), (2, 96, 32, 64), (2, 64, 32, 128), (3, 128, 64, 128), (1, 192, 64, 104), (2, 24, 40, 8)])
 def test_latent_prefill(gpu, heads, dim, rot, vdim):
     """Portions with and without a prefix, lengths around the tiles; one query-key pair stands out."""
