@@ -336,6 +336,15 @@ int infer_rms_norm_splitk_bf16(const float* partial, int64_t splits, int64_t spl
                                const void* weight, void* out, int64_t out_stride0,
                                int64_t n_rows, int64_t hidden, float eps, void* stream);
 
+/* infer_rms_norm_bf16 (or, with `partial`, infer_rms_norm_splitk_bf16) and the product of its result in one launch, for few rows: the bits of
+ * the two.  sum [m, k] = x + residual goes to a place of its own (residual may be null, then there is no sum).  gated: y [m, n / 2] as
+ * infer_skinny_gate_silu_bf16 gives it.  infer_norm_product_supported: 1 if the sizes are served and the product alone is not the vendor's. */
+int infer_norm_product_supported(int64_t m, int64_t n, int64_t k, int gated);
+int infer_norm_product_bf16(const void* x, int64_t x_stride0, const float* partial, int64_t splits, int64_t split_stride,
+                            int64_t partial_stride0, const void* residual, int64_t residual_stride0, void* sum, int64_t sum_stride0,
+                            const void* gain, float eps, const void* w, void* y, int64_t y_stride0, int64_t m, int64_t n, int64_t k,
+                            int gated, void* stream);
+
 /* ------------------------------------------------------------------ operators of the hybrid models
  * Models that mix latent attention (one compressed cache row per token) with recurrent layers (one
  * fixed-size state per sequence) and keep the residual stream in float32.  No counterpart in the

@@ -57,6 +57,9 @@ SIGNATURES = {
                                    _vp, _i64, _vp, _vp, _i64, _i64, _i64, _f32, _vp]),
     "infer_silu_and_mul": (_c.c_int, [_c.c_int, _vp, _i64, _vp, _i64, _i64, _i64, _vp]),
     "infer_clamped_gate_and_mul": (_c.c_int, [_c.c_int, _vp, _i64, _vp, _i64, _i64, _i64, _f32, _vp]),
+    "infer_norm_product_supported": (_c.c_int, [_i64, _i64, _i64, _c.c_int]),
+    "infer_norm_product_bf16": (_c.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _f32, _vp, _vp, _i64, _i64, _i64, _i64,
+                                           _c.c_int, _vp]),
     "infer_latent_front": (_c.c_int, [_c.c_int, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _f32, _vp,
                                       _i64, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp]),
     "infer_head_matmul": (_c.c_int, [_c.c_int, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64,

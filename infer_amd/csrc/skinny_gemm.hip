@@ -187,6 +187,32 @@ __global__ void __launch_bounds__(256) skinny_gemm_kernel(GemmArgs a) {
 
 __device__ __forceinline__ float round_bf16(float x) { return (float)(__bf16)x; }
 
+// Four sums of row `row` at the places 16 r + 4 g of a workgroup whose weights begin at row n0 (GATED: as described below)
+template <bool GATED>
+__device__ __forceinline__ void finish_tile(const GemmArgs& a, int split, int n0, int r, int row, int g, f32x4_t sum) {
+    if constexpr (GATED) {                         // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
+        bf16x4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float gate = round_bf16(sum[e]), up = __shfl_xor(gate, 32, 64);
+            v[e] = (__bf16)(round_bf16(gate / (1.0f + expf(-gate))) * up);
+        }
+        const int col = n0 + 8 * r + 4 * g;
+        if (g < 2 && col < a.n / 2 && row < a.m) *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
+    } else {
+        const int col = n0 + 16 * r + 4 * g;
+        if (col >= a.n || row >= a.m) return;          // N is a multiple of 8: a quad is in or out as a whole
+        if (a.partial) {
+            *reinterpret_cast<f32x4_t*>(a.partial + ((int64_t)split * a.m + row) * a.n + col) = sum;
+        } else {
+            bf16x4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (__bf16)sum[e];
+            *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
+        }
+    }
+}
+
 // 16 RT rows of weights past up to 16 MT rows of the batch, NW wavefronts with D steps each in LDS.  GATED: the weights are gate rows and as
 // many up rows, a.n / 2 each; a tile is eight gate rows and the eight up rows of the same places, and y = silu(gate) * up with the
 // roundings of storing both and reading them again.
@@ -217,30 +243,132 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     stream_product<RT, MT, NW, D>(w, x, a.chunks * kKC, wave, lds + wave * kRing, acc);
-    stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) {
-        const int row = 16 * t + n;
-        if constexpr (GATED) {                         // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
-            bf16x4_t v;
+    stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, split, n0, r, 16 * t + n, g, sum); });
+}
+
+// What stands in front of a product of few rows: y = norm(x + residual) w^T, where x may still be the pieces of a split product.
+struct NormSource {
+    const float* partial; int splits; int64_t split_stride, partial_stride0;      // if partial: x[r] = bf16(sum over splits of partial[s][r])
+    const uint16_t* x; int64_t x_stride0;
+    const uint16_t* residual; int64_t residual_stride0;                            // or null
+    uint16_t* sum; int64_t sum_stride0;                                            // x + residual
+    const uint16_t* gain;
+    float inv_k, eps;
+};
+constexpr int kFewRows = 2, kFewPieces = 8, kNormGroup = 512;       // rows of the batch; pieces of a row of kNormGroup elements in all
+constexpr int kFewMany = 16384;                                     // from so many weight rows on a workgroup takes 32
+constexpr int kFewPad = 64;                                         // bytes behind a row in LDS: rows meet other banks
+
+// A product of few rows with the norm of its input in front of it.  Every workgroup norms the rows for itself, out of the second-level cache
+// and while its weights are on their way, since a launch in between costs more: a step of a 0.6B model, one sequence, 1063 -> 949 us with
+// 56 of its 252 launches less.  The first workgroup leaves x + residual, in another place than the residual, which others still read.
+// NP: pieces of 64 x 8 elements per wavefront.  Sums, order and roundings are those of rms_norm_kernel and of skinny_stream_kernel: the
+// same bits.
+// What bounds it is what all workgroups read in front, rows times their bytes.  Norm and product, us, two launches / one, for 1, 2, 4 rows:
+// 4096 x 1024 behind four pieces 6.2 / 4.2, 6.4 / 4.3, 6.4 / 6.8; 6144 x 1024 gated 7.6 / 5.7, 7.6 / 6.0, 7.7 / 8.0; 6144 x 4096 14.1 / 12.6,
+// 13.5 / 13.3, 13.7 / 22.4; 24576 x 4096 gated 35.5 / 33.7, 33.8 / 42.4.  So one row up to 4096 elements, two of half as many.
+template <int RT, int NP, bool GATED>
+__global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSource f) {
+    constexpr int NW = 4, D = 4, kRing = D * stream_stage_bytes(RT, 0);
+    static_assert(NW * kRing >= NW * RT * 1024, "sums of the wavefronts");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];      // rings, then rows of x, then sums of squares
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * (GATED ? 8 : 16) * RT, half = a.n / 2;
+    const int row_bytes = 2 * a.k + kFewPad;
+    unsigned char* xs = few_lds + NW * kRing;
+    float* squares = reinterpret_cast<float*>(xs + a.m * row_bytes);               // [kFewRows][8]
+    const __bf16* w[2 * RT];
+#pragma unroll
+    for (int i = 0; i < 2 * RT; ++i) {
+        int row = n0 + stream_row() + 8 * (GATED ? i / 2 : i);
+        const int rows = GATED ? half : a.n;
+        row = (row < rows ? row : rows - 1) + (GATED && (i & 1) ? half : 0);
+        w[i] = (const __bf16*)a.w + (int64_t)row * a.k;
+    }
+    const int groups = (a.k + kNormGroup - 1) / kNormGroup, pieces = a.m * groups;
+    int row[NP], c[NP];
+    bool in[NP];
+    u32x4 gain[NP], res[NP], raw[NP];
+    f32x4 lo[NP], hi[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int p = wave + NW * i;
+        row[i] = p / groups;
+        c[i] = 64 * (p - row[i] * groups) + lane;
+        in[i] = p < pieces && 8 * c[i] < a.k;
+        if (!in[i]) row[i] = c[i] = 0;
+        gain[i] = load16(f.gain + 8 * c[i]);
+        if (f.residual) res[i] = load16(f.residual + row[i] * f.residual_stride0 + 8 * c[i]);
+        if (!f.partial) raw[i] = load16(f.x + row[i] * f.x_stride0 + 8 * c[i]);
+        lo[i] = hi[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (f.partial) {
+        constexpr int kBatch = 4;                        // splits requested at once
+        for (int s0 = 0; s0 < f.splits; s0 += kBatch) {
+            f32x4 l[kBatch][NP], h[kBatch][NP];
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b)
+#pragma unroll
+                for (int i = 0; i < NP; ++i) {
+                    const float* p = f.partial + (s0 + b < f.splits ? s0 + b : s0) * f.split_stride + row[i] * f.partial_stride0 + 8 * c[i];
+                    l[b][i] = *reinterpret_cast<const f32x4*>(p);
+                    h[b][i] = *reinterpret_cast<const f32x4*>(p + 4);
+                }
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b)
+                if (s0 + b < f.splits)
+#pragma unroll
+                    for (int i = 0; i < NP; ++i) { lo[i] += l[b][i]; hi[i] += h[b][i]; }
+        }
+    }
+    auto norm = [&] {
+        float v[NP][8];
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float gate = round_bf16(sum[e]), up = __shfl_xor(gate, 32, 64);
-                v[e] = (__bf16)(round_bf16(gate / (1.0f + expf(-gate))) * up);
+                v[i][e] = f.partial ? round_bf16(lo[i][e]) : __builtin_bit_cast(float, e & 1 ? raw[i][e / 2] & 0xffff0000u : raw[i][e / 2] << 16);
+                v[i][4 + e] = f.partial ? round_bf16(hi[i][e]) : __builtin_bit_cast(float, e & 1 ? raw[i][2 + e / 2] & 0xffff0000u : raw[i][2 + e / 2] << 16);
             }
-            const int col = n0 + 8 * r + 4 * g;
-            if (g < 2 && col < half && row < a.m) *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
-            return;
-        }
-        const int col = n0 + 16 * r + 4 * g;
-        if (col >= a.n || row >= a.m) return;          // N is a multiple of 8: a quad is in or out as a whole
-        if (a.partial) {
-            *reinterpret_cast<f32x4_t*>(a.partial + ((int64_t)split * a.m + row) * a.n + col) = sum;
-        } else {
-            bf16x4_t v;
+            if (f.residual) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (__bf16)sum[e];
-            *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
+                for (int e = 0; e < 8; ++e) v[i][e] += __builtin_bit_cast(float, e & 1 ? res[i][e / 2] & 0xffff0000u : res[i][e / 2] << 16);
+                if (blockIdx.x == 0 && in[i]) {
+                    bf16x8 o;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[e] = (__bf16)v[i][e];
+                    *reinterpret_cast<bf16x8*>(f.sum + row[i] * f.sum_stride0 + 8 * c[i]) = o;
+                }
+            }
+            float ss = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
+            if (!in[i]) ss = 0.f;
+#pragma unroll
+            for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+            const int p = wave + NW * i;
+            if (lane == 0 && p < pieces) squares[8 * (p / groups) + p % groups] = ss;
         }
-    });
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            if (!in[i]) continue;
+            float ss = 0.f;
+            for (int j = 0; j < groups; ++j) ss += squares[8 * row[i] + j];
+            const float rs = rsqrtf(ss * f.inv_k + f.eps);
+            bf16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                o[e] = (__bf16)(round_bf16(v[i][e] * rs) * __builtin_bit_cast(float, e & 1 ? gain[i][e / 2] & 0xffff0000u : gain[i][e / 2] << 16));
+            *reinterpret_cast<bf16x8*>(xs + row[i] * row_bytes + 16 * c[i]) = o;
+        }
+        __syncthreads();
+    };
+    f32x4_t acc[RT][1];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    stream_product_held<RT, NW, D>(w, xs + (n < a.m ? n : a.m - 1) * row_bytes + 16 * g, a.k, wave, few_lds + wave * kRing, norm, acc);
+    stream_reduce<RT, 1, NW>(acc, wave, few_lds, [&](int r, int, f32x4_t sum) { finish_tile<GATED>(a, 0, n0, r, n, g, sum); });
 }
 
 struct ReduceArgs {
@@ -435,4 +563,56 @@ extern "C" int infer_skinny_gate_silu_bf16(const void* x, int64_t x_stride0, con
     const GemmArgs a{(const uint16_t*)x, x_stride0, (const uint16_t*)w, (uint16_t*)y, y_stride0, nullptr, (int)m, (int)(2 * ff), (int)k, (int)(k / kKC)};
     launch_stream<true>(a, 1, (hipStream_t)stream);
     return (int)hipGetLastError();
+}
+
+namespace {
+template <bool GATED>
+int launch_norm_product(const GemmArgs& a, const NormSource& f, hipStream_t st) {
+    const int pieces = a.m * ((a.k + kNormGroup - 1) / kNormGroup), rows = a.n >= kFewMany ? 32 : 16;
+    const size_t lds = 4 * 4 * stream_stage_bytes(rows / 16, 0) + (size_t)a.m * (2 * a.k + kFewPad) + kFewRows * 8 * sizeof(float);
+    const dim3 grid((unsigned)((a.n + rows - 1) / rows));
+#define GO(RT, NP) do { \
+        if (lds > 60 * 1024) { \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&norm_product_kernel<RT, NP, GATED>), \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+            if (e != hipSuccess) return (int)e; \
+        } \
+        hipLaunchKernelGGL((norm_product_kernel<RT, NP, GATED>), grid, dim3(256), lds, st, a, f); \
+    } while (0)
+    if (rows == 16) {
+        if (pieces <= 4) GO(1, 1);
+        else GO(1, 2);
+    } else {
+        if (pieces <= 4) GO(2, 1);
+        else GO(2, 2);
+    }
+#undef GO
+    return (int)hipGetLastError();
+}
+}  // namespace
+
+extern "C" int infer_norm_product_supported(int64_t m, int64_t n, int64_t k, int gated) {
+    if (m < 1 || m > kFewRows || n < 1 || k < 1 || k % kKC || n % (gated ? 16 : 8) || n > (1 << 24) || k > kFewPieces * kNormGroup) return 0;
+    if (m * ((k + kNormGroup - 1) / kNormGroup) > kFewPieces || !pays(m, n, k, true)) return 0;
+    return choose_splits(m, n, k) == 1;
+}
+
+extern "C" int infer_norm_product_bf16(const void* x, int64_t x_stride0, const float* partial, int64_t splits, int64_t split_stride,
+                                       int64_t partial_stride0, const void* residual, int64_t residual_stride0, void* sum, int64_t sum_stride0,
+                                       const void* gain, float eps, const void* w, void* y, int64_t y_stride0, int64_t m, int64_t n, int64_t k,
+                                       int gated, void* stream) {
+    if (!infer_norm_product_supported(m, n, k, gated)) return INFER_KV_EUNSUPPORTED;
+    if (!(x || partial) || !gain || !w || !y || (residual && !sum)) return INFER_KV_EINVAL;
+    if (partial ? splits < 1 || splits > 64 || partial_stride0 < k || (splits > 1 && split_stride < m * partial_stride0) : x_stride0 < k) return INFER_KV_EINVAL;
+    if (residual && (residual_stride0 < k || sum_stride0 < k || sum == residual)) return INFER_KV_EINVAL;
+    if (y_stride0 < (gated ? n / 2 : n)) return INFER_KV_EINVAL;
+    uintptr_t all = (uintptr_t)gain | (uintptr_t)w | (uintptr_t)y | (uintptr_t)(partial ? (const void*)partial : x);
+    if (residual) all |= (uintptr_t)residual | (uintptr_t)sum;
+    if ((all & 15) || (y_stride0 & 7) || (partial ? (partial_stride0 | split_stride) & 3 : x_stride0 & 7) ||
+        (residual && ((residual_stride0 | sum_stride0) & 7)))
+        return INFER_KV_EALIGN;
+    const GemmArgs a{nullptr, 0, (const uint16_t*)w, (uint16_t*)y, y_stride0, nullptr, (int)m, (int)n, (int)k, (int)(k / kKC)};
+    const NormSource f{partial, (int)splits, split_stride, partial_stride0, (const uint16_t*)x, x_stride0, (const uint16_t*)residual, residual_stride0,
+                       (uint16_t*)sum, sum_stride0, (const uint16_t*)gain, 1.0f / (float)k, eps};
+    return gated ? launch_norm_product<true>(a, f, (hipStream_t)stream) : launch_norm_product<false>(a, f, (hipStream_t)stream);
 }

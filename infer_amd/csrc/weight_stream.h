@@ -79,6 +79,56 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
     }
 }
 
+// The same past activations that lie in LDS as a whole: only the weights are requested, and `before` runs behind the first requests, while
+// they are on their way; it puts the activations where x points (this lane's row, at element 8 g of the first step) and ends with a barrier.
+// k: a multiple of kStreamK; ring: D * stream_stage_bytes(RT, 0) bytes.
+template <int RT, int NW, int D, class Before>
+__device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 * RT], const unsigned char* x, int k, int wave, unsigned char* ring,
+                                                    Before before, f32x4_t (&acc)[RT][1]) {
+    constexpr int kRequests = 2 * RT, kStage = stream_stage_bytes(RT, 0);
+    static_assert(D >= 2 && D <= 4, "the waits below");
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, col = stream_col();
+    const int all = k / kStreamK, steps = all > wave ? (all - wave + NW - 1) / NW : 0;
+    const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ring);
+    auto request = [&](int s, int stage) {
+        const int from = (s * NW + wave) * kStreamK + col;
+#pragma unroll
+        for (int i = 0; i < kRequests; ++i)
+            __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(w[i] + from), "s"(base + stage * kStage + 1024 * i) : "memory", "m0");
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < steps) request(d, d);
+    before();
+    const int place = 128 * n + 16 * (g ^ (n & 7));
+    int stage = 0;
+    for (int s = 0; s < steps; ++s) {
+        // requests of later steps are the only ones behind this step's, or there are stores in between, with which this waits longer
+        const int behind = steps - 1 - s;
+        if (behind >= D - 1) __asm__ volatile("s_waitcnt vmcnt(%0)" :: "n"((D - 1) * kRequests) : "memory");
+        else if (D > 3 && behind == 2) __asm__ volatile("s_waitcnt vmcnt(%0)" :: "n"(D > 3 ? 2 * kRequests : 0) : "memory");
+        else if (D > 2 && behind == 1) __asm__ volatile("s_waitcnt vmcnt(%0)" :: "n"(D > 2 ? kRequests : 0) : "memory");
+        else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        bf16x8_t a[RT][2], b[2];
+        const unsigned char* p = ring + stage * kStage;
+        const unsigned char* from = x + 2 * kStreamK * (s * NW + wave);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r) a[r][h] = *reinterpret_cast<const bf16x8_t*>(p + 2048 * r + (place ^ (64 * h)));
+            b[h] = *reinterpret_cast<const bf16x8_t*>(from + 64 * h);
+        }
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // read before the stage is filled again
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + D < steps) request(s + D, stage);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][h], b[h], acc[r][0], 0, 0, 0);
+        stage = stage + 1 == D ? 0 : stage + 1;
+    }
+}
+
 // The sum of the wavefronts' parts of every tile, tile q = r * MT + t by wavefront q % NW, which gets it as f(r, t, sum) in the layout of
 // acc.  `lds` holds NW * RT * MT KiB; everybody is past its own ring.
 template <int RT, int MT, int NW, class F>

@@ -344,6 +344,42 @@ def _rms_norm_splitk(x: "SplitKSum", weight, eps, residual, out):
     return out if residual is None else (out, residual)
 
 
+def norm_linear(x, norm_weight: torch.Tensor, eps: float, residual: torch.Tensor | None, weight: torch.Tensor, gated: bool = False):
+    """``linear(rms_norm(x, norm_weight, eps, residual), weight)``, or ``gate_up_silu`` of it, in one launch: ``(result, x + residual)``, the
+    bits of the two launches (without ``residual``, ``x`` itself stands in the second place).  ``None`` where the kernel does not take the
+    call: few rows only, and nobody follows the operators.  The sum has memory of its own; ``residual`` stays as it is."""
+    pieces = isinstance(x, SplitKSum)
+    rows = residual if pieces else x
+    if rows is None or rows.dim() != 2 or not _streamable(rows, weight) or _linear_mode() != "static":
+        return None
+    m, k = rows.shape
+    n = weight.shape[0]
+    lib = _lib.load()
+    if tuple(x.shape) != (m, k) or not lib.infer_norm_product_supported(m, n, k, int(gated)):
+        return None
+    others = [norm_weight] if residual is None or pieces else [norm_weight, residual]
+    if not all(_plain(t) and t.dtype == torch.bfloat16 and t.get_device() == rows.get_device() and t.data_ptr() % 16 == 0 and
+               not (torch.is_grad_enabled() and t.requires_grad) for t in others):
+        return None
+    if norm_weight.shape != (k,) or not norm_weight.is_contiguous():
+        return None
+    if residual is not None and (residual.shape != (m, k) or residual.stride(1) != 1 or (m > 1 and (residual.stride(0) < k or residual.stride(0) % 8))):
+        return None
+    out = torch.empty((m, n // 2 if gated else n), dtype=weight.dtype, device=weight.device)
+    total = torch.empty((m, k), dtype=weight.dtype, device=weight.device) if residual is not None else x
+    if pieces:
+        x.check_alive()
+        part = x.partial
+        source = None, 0, part.data_ptr(), part.shape[0], part.stride(0), part.stride(1)
+    else:
+        source = x.data_ptr(), _row_stride(x), None, 0, 0, 0
+    res = (None, 0, None, 0) if residual is None else (residual.data_ptr(), _row_stride(residual), total.data_ptr(), k)
+    rc = lib.infer_norm_product_bf16(*source, *res, norm_weight.data_ptr(), float(eps), weight.data_ptr(), out.data_ptr(), out.shape[1], m, n, k,
+                                     int(gated), _stream_ptr(weight))
+    _lib.check(rc, "norm_linear")
+    return out, total
+
+
 def silu_and_mul(out: torch.Tensor, x: torch.Tensor) -> None:
     """``silu_and_mul(result, input)`` of ``src/bindings.cpp:22``: ``out = silu(x[..., :d]) * x[..., d:]``."""
     d = x.shape[-1] // 2
@@ -503,6 +539,8 @@ _flush_buffers: dict = {}
 
 # Up to this many rows of the batch, the streaming kernels and the launch of gate, up and activation
 STREAM_MAX_BATCH = 64
+# Up to this many, a norm in the product behind it
+FEW_ROWS = 2
 
 
 def _own_kernel(m: int, n: int, k: int, defer: bool) -> bool:

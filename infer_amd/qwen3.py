@@ -13,7 +13,7 @@ from . import kv_runner, ops
 from .attention import Attention
 from .cache import PagedKVLayout
 from .context import get_context
-from .layers import MLP, Embedding, Linear, LMHead, QKVLinear, RMSNorm, cos_sin_table
+from .layers import MLP, Embedding, Linear, LMHead, QKVLinear, RMSNorm, _is_bare, cos_sin_table, is_bare_mlp, norm_and_project
 
 
 class QwenAttention(nn.Module):
@@ -47,8 +47,10 @@ class QwenAttention(nn.Module):
             self._no_cache = torch.zeros(1, 256, self.num_kv_heads, self.head_dim, dtype=torch.bfloat16, device=device)
         return self._no_cache, self._no_cache, False
 
-    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor) -> torch.Tensor:
-        qkv = self.qkv_proj(hidden_states)
+    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor, qkv: torch.Tensor | None = None) -> torch.Tensor:
+        """``qkv``: the projections where the caller has them; then there are no hidden states."""
+        if qkv is None:
+            qkv = self.qkv_proj(hidden_states)
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
         q = q.view(-1, self.num_heads, self.head_dim)
         k = k.view(-1, self.num_kv_heads, self.head_dim)
@@ -71,6 +73,9 @@ class QwenAttention(nn.Module):
         return self.o_proj(o, defer=True)           # consumed by post_attention_layernorm
 
 
+_attention_forward = QwenAttention.forward
+
+
 class QwenDecoderLayer(nn.Module):
 
     def __init__(self, config, layer_idx: int):
@@ -91,15 +96,25 @@ class QwenDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor, residual: torch.Tensor | None):
-        if residual is None:
+        # a step of few rows has its norms inside the products behind them
+        attn, mlp, fused = self.self_attn, self.mlp, None
+        if type(attn.qkv_proj) is QKVLinear and _is_bare(attn, QwenAttention, _attention_forward):
+            fused = norm_and_project(self.input_layernorm, attn.qkv_proj, hidden_states, residual)
+        if fused is not None:
+            qkv, residual = fused
+            hidden_states = attn(positions, None, qkv=qkv)
+        elif residual is None:
             residual = hidden_states
-            hidden_states = self.input_layernorm(hidden_states)
+            hidden_states = attn(positions, self.input_layernorm(hidden_states))
         else:
             hidden_states, residual = self.input_layernorm(hidden_states, residual)
-        hidden_states = self.self_attn(positions, hidden_states)
+            hidden_states = attn(positions, hidden_states)
+        fused = norm_and_project(self.post_attention_layernorm, mlp.gate_up_proj, hidden_states, residual, gated=True) if is_bare_mlp(mlp) else None
+        if fused is not None:
+            act, residual = fused
+            return mlp(None, gated=act), residual
         hidden_states, residual = self.post_attention_layernorm(hidden_states, residual)
-        hidden_states = self.mlp(hidden_states)
-        return hidden_states, residual
+        return mlp(hidden_states), residual
 
 
 class QwenModel(nn.Module):

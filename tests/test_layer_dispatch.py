@@ -1,0 +1,89 @@
+"""A decoder layer takes its norms into the products behind them only where nobody could tell: on the host, with stand-ins for the kernels."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from infer_amd import ops, qwen3
+
+
+def _norm(x, weight, eps, residual=None, out=None):
+    x = x if residual is None else residual.add_(x)
+    y = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + eps) * weight
+    return y if residual is None else (y, residual)
+
+
+class Mixed(torch.nn.Module):
+    k_cache = v_cache = torch.zeros(0)
+
+    def forward(self, q, k, v, kv_stored):
+        return q.reshape(q.shape[0], -1) * 2 + k.reshape(k.shape[0], -1).repeat(1, 2)
+
+
+@pytest.fixture
+def layer(monkeypatch):
+    torch.manual_seed(0)
+    config = SimpleNamespace(hidden_size=16, num_attention_heads=2, num_key_value_heads=1, max_position_embeddings=8, rms_norm_eps=1e-6, head_dim=8,
+                             intermediate_size=24)
+    it = qwen3.QwenDecoderLayer(config, 0).float()
+    for p in it.parameters():
+        torch.nn.init.normal_(p)
+    it.fused = 0
+
+    def fused(x, gain, eps, residual, weight, gated=False):
+        it.fused += 1
+        total = x if residual is None else x + residual
+        y = F.linear(_norm(total, gain, eps), weight)
+        return (F.silu(y[:, :24]) * y[:, 24:] if gated else y), total
+
+    monkeypatch.setattr(ops, "norm_linear", fused)
+    monkeypatch.setattr(ops, "rms_norm", _norm)
+    monkeypatch.setattr(ops, "silu_and_mul", lambda out, y: out.copy_(F.silu(y[..., :24]) * y[..., 24:]))
+    monkeypatch.setattr(ops, "gate_up_silu", lambda x, w: F.silu(F.linear(x, w)[:, :24]) * F.linear(x, w)[:, 24:])
+    monkeypatch.setattr(ops, "qk_norm_rope_store_kvcache", lambda *a, **k: None)
+    monkeypatch.setattr(qwen3, "cos_sin_table", lambda *a: None)
+    monkeypatch.setattr(qwen3, "get_context", lambda: SimpleNamespace(slot_mapping=torch.zeros(0), is_prefill=False, block_tables=None))
+    it.self_attn.attn = Mixed()
+    return it
+
+
+def _plain(it, x, residual):
+    """The layer in plain calls."""
+    s = x if residual is None else x + residual
+    a = it.self_attn
+    qkv = a.qkv_proj(_norm(s, it.input_layernorm.weight, 1e-6))
+    o = a.o_proj(qkv[:, :16] * 2 + qkv[:, 16:24].repeat(1, 2))
+    s = s + o
+    y = it.mlp.gate_up_proj(_norm(s, it.post_attention_layernorm.weight, 1e-6))
+    return it.mlp.down_proj(F.silu(y[:, :24]) * y[:, 24:]), s
+
+
+@pytest.mark.parametrize("rows,fused", [(1, 2), (ops.FEW_ROWS, 2), (ops.FEW_ROWS + 1, 0)])
+@pytest.mark.parametrize("first", [False, True])
+def test_layers_of_few_rows(layer, rows, fused, first):
+    x, residual = torch.randn(rows, 16), None if first else torch.randn(rows, 16)
+    want = _plain(layer, x, residual)
+    got = layer(None, x, None if first else residual.clone())
+    assert layer.fused == fused
+    torch.testing.assert_close(got, want, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("where,left", [("input_layernorm", 1), ("self_attn", 1), ("self_attn.qkv_proj", 1), ("post_attention_layernorm", 1), ("mlp", 1),
+                                        ("mlp.gate_up_proj", 1), ("mlp.down_proj", 2), ("self_attn.o_proj", 2)])
+def test_somebody_who_looks_sees_the_call(layer, where, left):
+    seen = []
+    layer.get_submodule(where).register_forward_hook(lambda m, args, out: seen.append((args, out)))
+    x, residual = torch.randn(2, 16), torch.randn(2, 16)
+    want = _plain(layer, x, residual)
+    seen.clear()
+    torch.testing.assert_close(layer(None, x, residual.clone()), want, atol=1e-4, rtol=1e-4)
+    assert layer.fused == left and len(seen) == 1
+    assert all(isinstance(a, torch.Tensor) or a is None for a in seen[0][0])
+
+
+def test_a_forward_of_its_own_is_called(layer):
+    inner = layer.input_layernorm.forward
+    layer.input_layernorm.forward = lambda x, residual=None: tuple(2 * t for t in inner(x, residual))
+    layer(None, torch.randn(2, 16), torch.randn(2, 16))
+    assert layer.fused == 1
