@@ -1,0 +1,249 @@
+// Paged decode attention of a few sequences for gfx950 (MI355X): one query token per sequence, bf16 in, float32 sums.
+//
+// With little to read, what counts is the chain of waits from the launch to the result.  paged_decode.hip lays all steps of a batch end to
+// end and cuts them into equal spans, for which it first reads all lengths, adds them up and gathers block ids, and it gives a compute
+// unit eight wavefronts of one span each: right for a full chip, but a few sequences wait for the plan, and for a compute unit that brings 40
+// KB/us.  Here workgroup (p, h, b) takes the steps p, p + P, p + 2 P, ... of 32 tokens of sequence b, a wavefront every fourth of
+// them: the length, the block id and the query are requested at once, keys and values behind them, and neighbouring steps lie on different compute
+// units.  A second launch adds the pieces of a head up.
+//
+// Layouts of the two products are those of paged_decode.hip: S^T = K Q^T with keys as they lie in memory, O^T += V^T P^T with values
+// through a tile of the wavefront's own in LDS.
+#include "decode_few.h"
+
+#include "../../include/infer_kv.h"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef short i16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+
+constexpr int kD = 128, kStep = 32, kWaves = 4;
+constexpr int kRow = 288;                          // bytes of a value row in LDS: four rows meet different banks
+constexpr int kTile = kStep * kRow;                // of a wavefront; later its partial result
+static_assert(kTile >= 16 * 130 * 4, "a partial result of 16 heads");
+
+__device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
+__device__ __forceinline__ u32x4 load16_stream(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
+__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 x) { return __builtin_bit_cast(bf16x8, x); }
+__device__ __forceinline__ void lds_order() { __asm__ volatile("" ::: "memory"); }
+
+__global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds_all[kWaves * kTile];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, n = lane & 15;
+    const int p = blockIdx.x, h = blockIdx.y, b = blockIdx.z, G = a.group, P = a.pieces;
+    unsigned char* lds = lds_all + wave * kTile;
+    const int32_t* bt = a.bt + (int64_t)b * a.bt_stride0;
+    const int last_col = a.max_ctx / a.block_size - 1;
+    const unsigned per_block = (unsigned)a.block_size / kStep;
+    auto block_of = [&](int step) {                // read whether or not the sequence has the step
+        const int col = (int)((unsigned)step / per_block);
+        return bt[col < last_col ? col : last_col];
+    };
+    const int first = p + P * wave, stride = P * kWaves;
+    int blk = block_of(first), next_blk = block_of(first + stride);
+    int len = a.ctx[b];
+    u32x4 q[4];
+    {
+        const uint16_t* qp = a.q + (int64_t)b * a.q_stride0 + (int64_t)(h * G + (n < G ? n : 0)) * kD + 8 * g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[j] = load16(qp + 32 * j);
+    }
+    len = len < a.max_ctx ? len : a.max_ctx;
+    const int steps = len > 0 ? (len + kStep - 1) / kStep : 0;
+    if (p >= steps) return;                        // the whole workgroup
+    const int waves = (steps - p + P - 1) / P < kWaves ? (steps - p + P - 1) / P : kWaves;
+    if (n >= G)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[j] = u32x4{0u, 0u, 0u, 0u};
+
+    f32x4 acc[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+
+    // Row r of key tile t is token 8 (r / 4) + 4 t + r % 4 of the step, so that lane group g ends up with tokens 8 g .. 8 g + 7.
+    const int64_t k_lane = (8 * (n >> 2) + (n & 3)) * a.tok_stride + 8 * g, v_lane = g * a.tok_stride + 8 * n;
+    u32x4 k[2][4], v[8];
+    auto request = [&](int step, int id) {
+        id = id < 0 ? 0 : id >= a.num_blocks ? a.num_blocks - 1 : id;
+        const int in = (int)((unsigned)step % per_block) * kStep;
+        const int64_t at = (int64_t)id * a.blk_stride + in * a.tok_stride + (int64_t)h * kD;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) k[t][j] = load16(a.k + at + k_lane + 4 * t * a.tok_stride + 32 * j);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = load16_stream(a.v + at + v_lane + 4 * i * a.tok_stride);
+    };
+    if (first < steps) request(first, blk);
+    for (int step = first; step < steps; step += stride) {
+        f32x4 s[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k[t][j]), as_bf16x8(q[j]), s[t], 0, 0, 0);
+        }
+        const int tok0 = step * kStep;
+        const bool tail = tok0 + kStep > len;
+        if (tail) {                                // rows behind the end: their weights are 0, and 0 * NaN must not leak
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (tok0 + 4 * i + g >= len) v[i] = u32x4{0u, 0u, 0u, 0u};
+        }
+        lds_order();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4*>(lds + (4 * i + g) * kRow + n * 16) = v[i];
+        lds_order();
+        if (step + stride < steps) {
+            blk = next_blk;
+            next_blk = block_of(step + 2 * stride);
+            request(step + stride, blk);
+        }
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = s[i >> 2][i & 3] * a.scale_log2;
+        if (tail) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (tok0 + 8 * g + i >= len) x[i] = -INFINITY;
+        }
+        float top = x[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) top = fmaxf(top, x[i]);
+        top = fmaxf(top, __shfl_xor(top, 16));
+        top = fmaxf(top, __shfl_xor(top, 32));
+        top = fmaxf(top, m);
+        const float keep = __builtin_amdgcn_exp2f(m - top);
+        m = top;
+        float sum = 0.f;
+        bf16x8 w;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float e = __builtin_amdgcn_exp2f(x[i] - top);
+            sum += e;
+            w[i] = (__bf16)e;
+        }
+        l = l * keep + sum;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            acc[t] *= keep;
+            // in each group of 16 lanes, lane i points at four elements of row i / 4 and lane c receives column c of those rows
+            const unsigned char* src = lds + (8 * g + (n >> 2)) * kRow + (16 * t + 4 * (n & 3)) * 2;
+            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
+            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 4 * kRow));
+            const i16x8 vt = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vt), w, acc[t], 0, 0, 0);
+        }
+        lds_order();
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+
+    // lane (g, n) holds columns 16 t + 4 g .. + 3 of head n
+    auto leave = [&](float* to) {
+        if (n >= G) return;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) *reinterpret_cast<f32x4*>(to + n * kD + 16 * t + 4 * g) = acc[t];
+        if (g == 0) *reinterpret_cast<float2*>(to + G * kD + 2 * n) = make_float2(m, l);
+    };
+    if (waves > 1) {
+        lds_order();
+        if (wave > 0 && wave < waves) leave(reinterpret_cast<float*>(lds));
+        __syncthreads();
+        if (wave > 0) return;
+        for (int w = 1; w < waves; ++w) {
+            const float* from = reinterpret_cast<const float*>(lds_all + w * kTile);
+            const int nn = n < G ? n : 0;
+            const float2 o = *reinterpret_cast<const float2*>(from + G * kD + 2 * nn);
+            const float top = fmaxf(m, o.x), f1 = __builtin_amdgcn_exp2f(m - top), f2 = __builtin_amdgcn_exp2f(o.x - top);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) acc[t] = acc[t] * f1 + *reinterpret_cast<const f32x4*>(from + nn * kD + 16 * t + 4 * g) * f2;
+            l = l * f1 + o.y * f2;
+            m = top;
+        }
+    } else if (wave > 0) {
+        return;
+    }
+    leave(a.rec + (((int64_t)b * a.num_kv_heads + h) * P + p) * few_record_floats(G));
+}
+
+constexpr int kMostPieces = 64;
+
+// Up to 8 N pieces.  Grid (query heads, batch): 32 lanes hold the columns of the head, the eight halves of wavefronts every eighth piece.  Pieces are requested before it
+// is known how many there are; what lies behind the last is not looked at.
+template <int N>
+__global__ void __launch_bounds__(256) few_decode_sum_kernel(FewDecode a) {
+    __shared__ f32x4 sums[7][32];
+    __shared__ float2 mls[7];
+    const int head = blockIdx.x, b = blockIdx.y, G = a.group, h = head / G, n = head - h * G, c = threadIdx.x & 31, part = threadIdx.x >> 5;
+    const int floats = few_record_floats(G);
+    const float* rec = a.rec + ((int64_t)b * a.num_kv_heads + h) * a.pieces * floats;
+    f32x4 v[N];
+    float2 ml[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int p = part + 8 * i;
+        const float* from = rec + (int64_t)(p < a.pieces ? p : 0) * floats;
+        v[i] = *reinterpret_cast<const f32x4*>(from + n * kD + 4 * c);
+        ml[i] = *reinterpret_cast<const float2*>(from + G * kD + 2 * n);
+    }
+    int len = a.ctx[b];
+    len = len < a.max_ctx ? len : a.max_ctx;
+    const int steps = len > 0 ? (len + kStep - 1) / kStep : 0, pieces = steps < a.pieces ? steps : a.pieces;
+    f32x4 num = {0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, den = 0.f;
+    auto add = [&](f32x4 x, float2 o) {
+        const float top = fmaxf(m, o.x), f1 = m == top ? 1.f : __builtin_amdgcn_exp2f(m - top), f2 = o.x == top ? 1.f : __builtin_amdgcn_exp2f(o.x - top);
+        num = num * f1 + x * f2;
+        den = den * f1 + o.y * f2;
+        m = top;
+    };
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (part + 8 * i < pieces) add(v[i], ml[i]);
+    if (part > 0) {
+        sums[part - 1][c] = num;
+        if (c == 0) mls[part - 1] = make_float2(m, den);
+    }
+    __syncthreads();
+    if (part > 0) return;
+    for (int w = 1; w < 8 && w < pieces; ++w) add(sums[w - 1][c], mls[w - 1]);
+    const float inv = den > 0.f ? 1.f / den : 0.f;
+    bf16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (__bf16)(num[e] * inv);
+    *reinterpret_cast<bf16x4*>(a.out + (int64_t)b * a.out_stride0 + (int64_t)head * kD + 4 * c) = o;
+}
+
+}  // namespace
+
+// Pairs of a sequence and a KV head, against paged_decode.hip, us, both launches (32 heads on 8, tokens of each sequence or of the shortest and
+// longest): 1 x 700 12.4 / 7.2, 1 x 4000 18.5 / 11.1, 1 x 30000 40 / 30, 4 x 700 13.6 / 9.3, 4 x 16000 53.6 / 53.1, 4 x 100 .. 16000 33 / 23,
+// 6 x 2541 .. 7125 32.5 / 31.6, 8 x 700 14.7 / 12.7, 8 x 4000 32.1 / 31.4, 8 x 100 .. 16000 29.8 / 26.9, but 8 x 1420 .. 7184 35.8 / 36.7 and 8 x
+// 16000 92 / 98; 16 x 372 .. 7560 54 / 63.  So 48 pairs, and up to 64 where the table holds no more than 4096 tokens.  As many pieces as make 1024
+// workgroups, but no more than there is use for: 256 of them leave a compute unit's memory requests short (8 x 100 .. 16000 55), and more
+// records cost their sum (8 x 700 11.8 with 256).  Up to seven pairs 64 pieces, so that a long sequence meets the whole chip (1 x 120000, 8 heads on
+// 2, 51 / 37, with 32 pieces 55).
+int few_decode_pieces(int64_t batch, int64_t num_kv_heads, int64_t max_tokens) {
+    if (batch < 1 || num_kv_heads < 1 || batch > 64 || num_kv_heads > 64) return 0;
+    const int64_t pairs = batch * num_kv_heads, p = 1024 / pairs, most = pairs < 8 ? kMostPieces : kMostPieces / 2;
+    if (pairs > 64 || (pairs > 48 && max_tokens > 4096)) return 0;
+    return (int)(p > most ? most : p);
+}
+
+int launch_few_decode(const FewDecode& a, hipStream_t stream) {
+    hipLaunchKernelGGL(few_decode_kernel, dim3((unsigned)a.pieces, (unsigned)a.num_kv_heads, (unsigned)a.batch), dim3(64 * kWaves), 0, stream, a);
+    const int rc = (int)hipGetLastError();
+    if (rc) return rc;
+    const dim3 grid((unsigned)(a.group * a.num_kv_heads), (unsigned)a.batch), block(256);
+    if (a.pieces <= 32) hipLaunchKernelGGL(few_decode_sum_kernel<4>, grid, block, 0, stream, a);
+    else hipLaunchKernelGGL(few_decode_sum_kernel<8>, grid, block, 0, stream, a);
+    return (int)hipGetLastError();
+}

@@ -33,6 +33,7 @@
 
 #include <type_traits>
 
+#include "decode_few.h"
 #include "decode_layout.h"
 
 namespace {
@@ -1086,6 +1087,20 @@ int launch_merge(void* out, int64_t out_stride0, const int32_t* context_lens, in
     return (int)hipGetLastError();
 }
 
+// A few sequences, if their pieces fit the memory laid out as `ws`: true and the launches' return code.
+bool run_few(const DecodeCall& c, const DecodeWorkspace& ws, void* base, void* out, int64_t out_stride0, hipStream_t stream, int* rc) {
+    const int64_t max_ctx = c.table_cols * c.block_size;
+    const int pieces = few_decode_pieces(c.batch, c.num_kv_heads, max_ctx), group = (int)(c.num_q_heads / c.num_kv_heads);
+    const size_t need = (size_t)c.batch * c.num_kv_heads * pieces * few_record_floats(group) * sizeof(float);
+    if (pieces == 0 || need > ws.total_bytes - ws.rec_first_off) return false;
+    const FewDecode a{(const uint16_t*)c.q, c.q_stride0, (const uint16_t*)c.k_cache, (const uint16_t*)c.v_cache, c.cache_block_stride,
+                      c.cache_token_stride, c.block_table, c.bt_stride0, c.context_lens, max_ctx > 0x7fffffffLL ? 0x7fffffff : (int)max_ctx,
+                      (int)c.batch, group, (int)c.num_kv_heads, (int)c.block_size, (int)c.num_blocks, c.scale * 1.4426950408889634f, pieces,
+                      (float*)((char*)base + ws.rec_first_off), (uint16_t*)out, out_stride0};
+    *rc = launch_few_decode(a, stream);
+    return true;
+}
+
 // The decode op on memory laid out as `ws`: the streaming kernel and the merge kernel behind it.
 int run_decode(const DecodeCall& c, const Launch& L, const DecodeWorkspace& ws, void* base, void* out,
                int64_t out_stride0, hipStream_t stream) {
@@ -1170,6 +1185,7 @@ int infer_paged_decode_bf16(const void* q, int64_t q_stride0, const void* k_cach
     DeviceState* dev = nullptr;
     rc = init_device((hipStream_t)stream, true, &dev);
     if (rc) return rc;
+    if (split_workgroups == 0 && run_few(c, ws, workspace, out, out_stride0, (hipStream_t)stream, &rc)) return rc;
     Launch L;
     rc = plan_launch(num_kv_heads, split_workgroups, dev->cus, INFER_KV_DECODE_PARTS, &L);
     if (rc) return rc;
@@ -1250,6 +1266,7 @@ int infer_paged_decode_noalloc_bf16(const void* q, int64_t q_stride0, const void
     // laid out for the span positions this call launches, not for the largest count a workspace allows
     const DecodeWorkspace ws = decode_workspace_layout(batch, num_q_heads / num_kv_heads, num_kv_heads, L.S);
     if (ws.total_bytes > kNoAllocScratchBytes) return INFER_KV_EWORKSPACE;
+    if (run_few(c, ws, scratch, out, out_stride0, (hipStream_t)stream, &rc)) return rc;
     return run_decode(c, L, ws, scratch, out, out_stride0, (hipStream_t)stream);
 }
 

@@ -1,0 +1,107 @@
+"""Decode attention of a few sequences: steps dealt out to workgroups and wavefronts, against float64 and around every edge of the plan.
+
+Bar: weights of the values are rounded to bfloat16 (2^-9 each, of either sign) and the result once more (2^-9)."""
+import pytest
+import torch
+
+from infer_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def _inputs(gen, lens, hq, hkv, block, columns=None):
+    per = columns or max(1, -(-max(lens) // block))
+    blocks = len(lens) * per + 2
+    k, v = (torch.randn(blocks, block, hkv, 128, generator=gen).to(BF16).cuda() for _ in range(2))
+    table = torch.full((len(lens), per), -1, dtype=torch.int32)
+    order = torch.randperm(blocks, generator=gen).to(torch.int32)
+    for i, n in enumerate(lens):
+        used = -(-n // block)
+        table[i, :used] = order[i * per:i * per + used]
+    return torch.randn(len(lens), hq, 128, generator=gen).to(BF16).cuda(), k, v, table.cuda(), torch.tensor(lens, dtype=torch.int32).cuda()
+
+
+def _reference(q, k, v, table, lens, scale):
+    out, group = torch.zeros(q.shape, dtype=torch.float64), q.shape[1] // k.shape[2]
+    for i, n in enumerate(lens):
+        if n == 0:
+            continue
+        pages = table[i].clamp(min=0).long()
+        kk, vv = (t[pages].flatten(0, 1)[:n].double().cpu().repeat_interleave(group, 1) for t in (k, v))
+        w = torch.softmax(torch.einsum("hd,nhd->hn", q[i].double().cpu(), kk) * scale, -1)
+        out[i] = torch.einsum("hn,nhd->hd", w, vv)
+    return out
+
+
+def _check(q, k, v, table, ctx, lens, scale=128 ** -0.5):
+    out = torch.full_like(q, float("nan"))
+    ops.paged_attn_decode(q, k, v, table, ctx, scale, out)
+    want = _reference(q, k, v, table, lens, scale)
+    for i in range(len(lens)):
+        err = (out[i].double().cpu() - want[i]).norm() / max(want[i].norm().item(), 1e-9)
+        assert err <= 2.0 ** -8, (i, lens[i], float(err))
+    return out
+
+
+@pytest.mark.parametrize("lens,hq,hkv,block", [
+    ([1], 16, 8, 256), ([31, 32, 33, 0], 16, 8, 256), ([1023, 1024, 1025, 1057], 32, 8, 256), ([4095, 4097, 4128], 16, 8, 256),
+    ([0, 2081, 37, 2048, 640, 5, 991, 4096], 32, 8, 256), ([300, 1, 64, 500, 97, 33, 1300], 8, 8, 32), ([129] * 6, 48, 8, 96),
+    ([9000], 16, 1, 64), ([2049, 8193], 6, 2, 128), ([777] * 64, 4, 1, 512), ([1, 70, 3000], 5, 5, 256),
+])
+def test_against_float64(gpu, lens, hq, hkv, block):
+    gen = torch.Generator().manual_seed(sum(lens) + hq)
+    _check(*_inputs(gen, lens, hq, hkv, block), lens)
+
+
+def test_batches_on_either_side_of_the_rule_agree(gpu):
+    """Rows of a batch that takes the general kernel, and the same rows by themselves."""
+    gen = torch.Generator().manual_seed(5)
+    lens = [1500, 20, 700, 333, 1, 900, 64, 1200, 256, 31, 2000, 511]
+    q, k, v, table, ctx = _inputs(gen, lens, 16, 8, 256)
+    whole = _check(q, k, v, table, ctx, lens)
+    for i in range(0, 12, 3):
+        part = _check(q[i:i + 3], k, v, table[i:i + 3], ctx[i:i + 3], lens[i:i + 3])
+        assert (part.float() - whole[i:i + 3].float()).norm() <= 2.0 ** -8 * whole[i:i + 3].float().norm()
+    # eight sequences of a table for more than 4096 tokens are the general kernel's
+    wide = _inputs(gen, lens[:8], 16, 8, 256, columns=17)
+    _check(*wide, lens[:8])
+
+
+def test_what_lies_behind_the_end_is_not_looked_at(gpu):
+    """Stale NaN in keys and values behind a length, ids out of range behind the last block, a length beyond the table."""
+    gen = torch.Generator().manual_seed(6)
+    lens = [40, 300, 512]
+    q, k, v, table, ctx = _inputs(gen, lens, 16, 8, 256)
+    want = _check(q, k, v, table, ctx, lens)
+    for i, n in enumerate(lens):
+        if n % 256:
+            for t in (k, v):
+                t[table[i, n // 256], n % 256:] = float("nan")
+    table[0, 1] = 1 << 30
+    ctx[2] = 5000
+    got = torch.empty_like(q)
+    ops.paged_attn_decode(q, k, v, table, ctx, 128 ** -0.5, got)
+    assert torch.equal(got, want)
+
+
+def test_captured_and_replayed_with_other_lengths(gpu):
+    gen = torch.Generator().manual_seed(7)
+    lens = [900, 10, 2000, 450]
+    q, k, v, table, ctx = _inputs(gen, lens, 16, 8, 256)
+    table = table.clamp(min=0)
+    out, ws = torch.empty_like(q), ops.decode_workspace(q.device, 64, 16, 8, 128).clone()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        ops.paged_attn_decode(q, k, v, table, ctx, 128 ** -0.5, out, workspace=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.paged_attn_decode(q, k, v, table, ctx, 128 ** -0.5, out, workspace=ws)
+    for now in ([900, 10, 2000, 450], [1, 0, 33, 2048], [1024, 700, 64, 0]):
+        ctx.copy_(torch.tensor(now, dtype=torch.int32))
+        out.fill_(float("nan"))
+        graph.replay()
+        want = _reference(q, k, v, table, now, 128 ** -0.5)
+        assert (out.double().cpu() - want).norm() <= 2.0 ** -8 * want.norm()
