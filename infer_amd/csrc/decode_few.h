@@ -18,9 +18,22 @@ struct FewDecode {
     uint16_t* out; int64_t out_stride0;
 };
 
+// What stands in front of the attention of new tokens: norms of their query and key heads, rotary positions, the append (as in
+// qk_norm_rope_append.hip).
+struct FewFront {
+    const uint16_t* k; int64_t k_stride0;      // the new tokens' rows
+    const uint16_t* v; int64_t v_stride0;
+    const int64_t* positions;
+    const uint16_t* q_weight; const uint16_t* k_weight;
+    const uint16_t* cos_sin; int64_t max_position;
+    uint16_t* k_cache; uint16_t* v_cache;      // those of FewDecode
+    const int32_t* slots; int64_t num_slots;
+    float eps;
+};
+
 // What a piece leaves: [group][128] unnormalised sums, then [group] (running maximum in the log2 domain, sum).
 __host__ __device__ inline int few_record_floats(int group) { return 130 * group + (group & 1 ? 2 : 0); }
 
 // Pieces per (sequence, KV head), or 0 where the batch is not small.
 int few_decode_pieces(int64_t batch, int64_t num_kv_heads, int64_t max_tokens);
-int launch_few_decode(const FewDecode& a, hipStream_t stream);      // records, then their sum in `out`
+int launch_few_decode(const FewDecode& a, hipStream_t stream, const FewFront* front = nullptr);      // records, then their sum in `out`

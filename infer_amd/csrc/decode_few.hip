@@ -11,6 +11,8 @@
 // through a tile of the wavefront's own in LDS.
 #include "decode_few.h"
 
+#include <type_traits>
+
 #include "../../include/infer_kv.h"
 
 namespace {
@@ -26,14 +28,50 @@ typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 constexpr int kD = 128, kStep = 32, kWaves = 4;
 constexpr int kRow = 288;                          // bytes of a value row in LDS: four rows meet different banks
 constexpr int kTile = kStep * kRow;                // of a wavefront; later its partial result
-static_assert(kTile >= 16 * 130 * 4, "a partial result of 16 heads");
+static_assert(kTile >= 16 * 130 * 4 && kTile >= 17 * 272, "a partial result of 16 heads; 16 queries and a key");
 
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 __device__ __forceinline__ u32x4 load16_stream(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 x) { return __builtin_bit_cast(bf16x8, x); }
 __device__ __forceinline__ void lds_order() { __asm__ volatile("" ::: "memory"); }
 
-__global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a) {
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float lo16(uint32_t x) { return __builtin_bit_cast(float, x << 16); }
+__device__ __forceinline__ float hi16(uint32_t x) { return __builtin_bit_cast(float, x & 0xffff0000u); }
+__device__ __forceinline__ uint32_t pack(float lo, float hi) { return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi}); }
+
+// Norm and rotation of a head: 16 lanes hold eight elements each.  w: weights, c, s: cosines and sines of lanes 0 .. 7 and again of 8 .. 15, the
+// sines of the lower half with the other sign.  Sums, order and roundings are those of qk_norm_rope_append.hip.
+__device__ __forceinline__ u32x4 norm_and_rotate(u32x4 x, u32x4 w, u32x4 c, u32x4 s, float eps) {
+    auto dot2 = [](uint32_t a, uint32_t b, float z) { return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), z, false); };
+    auto ror = [](uint32_t v, auto C) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + decltype(C)::value, 0xf, 0xf, false); };
+    auto plus = [&](float v, auto C) { return v + __builtin_bit_cast(float, ror(__builtin_bit_cast(uint32_t, v), C)); };
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss = dot2(x[i], x[i], ss);
+    ss = plus(ss, std::integral_constant<int, 8>{});
+    ss = plus(ss, std::integral_constant<int, 4>{});
+    ss = plus(ss, std::integral_constant<int, 2>{});
+    ss = plus(ss, std::integral_constant<int, 1>{});
+    const float r = __builtin_amdgcn_rsqf(__builtin_fmaf(ss, 1.0f / kD, eps));
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t y = pack(lo16(x[i]) * r, hi16(x[i]) * r), z = pack(lo16(y) * lo16(w[i]), hi16(y) * hi16(w[i])), one = 0x3f803f80u;
+        const uint32_t other = ror(z, std::integral_constant<int, 8>{});
+        o[i] = pack(dot2(pack(lo16(z) * lo16(c[i]), lo16(other) * lo16(s[i])), one, 0.f), dot2(pack(hi16(z) * hi16(c[i]), hi16(other) * hi16(s[i])), one, 0.f));
+    }
+    return o;
+}
+
+// FRONT: queries and new keys are as projected, and nothing of the new tokens is in the caches yet.  Every wavefront with a step norms and
+// rotates the queries that it uses, four heads at once, while its keys and values are on their way; the one with a sequence's last step does
+// so with the new key, takes key and value from its registers, since what it has requested is older, and puts them into the caches at its
+// end, where nothing waits for the stores.  us, 16 heads on 8, front and attention in launches of their own / this: 1 x 700 tokens 9.7 / 8.1,
+// 4 x 700 12.4 / 11.2, 8 x 700 16.2 / 15.4; 32 heads 10.2 / 8.2, 12.8 / 11.9, 16.9 / 16.5; a step of a 0.6B model with one sequence 820 -> 778.
+// (With the stores in front of the products, with front loads of wavefronts without a step, or with heads spread as operands are, it gained nothing.)
+template <bool FRONT>
+__global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a, FewFront f) {
     __shared__ __attribute__((aligned(16))) unsigned char lds_all[kWaves * kTile];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, n = lane & 15;
     const int p = blockIdx.x, h = blockIdx.y, b = blockIdx.z, G = a.group, P = a.pieces;
@@ -49,18 +87,68 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a) {
     int blk = block_of(first), next_blk = block_of(first + stride);
     int len = a.ctx[b];
     u32x4 q[4];
-    {
+    if constexpr (!FRONT) {
         const uint16_t* qp = a.q + (int64_t)b * a.q_stride0 + (int64_t)(h * G + (n < G ? n : 0)) * kD + 8 * g;
 #pragma unroll
         for (int j = 0; j < 4; ++j) q[j] = load16(qp + 32 * j);
     }
+    int64_t slot = -1, pos = 0;
+    if constexpr (FRONT) {
+        slot = f.slots[b];
+        pos = f.positions[b];
+        pos = pos < 0 ? 0 : pos >= f.max_position ? f.max_position - 1 : pos;
+    }
+    // Heads 4 i .. 4 i + 3 of the group's queries with the new key behind them, 16 lanes each
+    u32x4 x[2], w[2], cs, sn, kn[4], vn;
+    auto load_heads = [&](int i, u32x4& xi, u32x4& wi) {
+        const int head = 4 * i + g;
+        const bool query = head < G;
+        xi = load16(query ? a.q + (int64_t)b * a.q_stride0 + (int64_t)(h * G + head) * kD + 8 * n : f.k + (int64_t)b * f.k_stride0 + h * kD + 8 * n);
+        wi = load16((query ? f.q_weight : f.k_weight) + 8 * n);
+    };
+    auto load_front = [&](bool two) {
+        cs = load16(f.cos_sin + pos * kD + 8 * (n & 7));
+        sn = load16(f.cos_sin + pos * kD + 64 + 8 * (n & 7));
+        vn = load16(f.v + (int64_t)b * f.v_stride0 + h * kD + 8 * n);
+        load_heads(0, x[0], w[0]);
+        if (two) load_heads(1, x[1], w[1]);
+    };
+    constexpr int kHead = 272;                     // bytes of a head in LDS, where they change to the layout of operands
+    auto finish_front = [&](int heads) {
+        if (n < 8) sn ^= u32x4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+        for (int i = 0; 4 * i < heads; ++i) {
+            u32x4 xi = x[0], wi = w[0];
+            if (i == 1) { xi = x[1]; wi = w[1]; }
+            if (i > 1) load_heads(i, xi, wi);
+            xi = norm_and_rotate(xi, wi, cs, sn, f.eps);
+            if (4 * i + g <= G) *reinterpret_cast<u32x4*>(lds + (4 * i + g) * kHead + 16 * n) = xi;
+        }
+        lds_order();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            q[j] = *reinterpret_cast<const u32x4*>(lds + (n < G ? n : 0) * kHead + 64 * j + 16 * g);
+            kn[j] = *reinterpret_cast<const u32x4*>(lds + G * kHead + 64 * j + 16 * g);      // of the wavefront that needs it
+        }
+        lds_order();
+    };
+    auto append = [&] {
+        if (slot < 0 || slot >= f.num_slots) return;
+        const int64_t at = (slot * a.num_kv_heads + h) * kD;
+        if (n == 0)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(f.k_cache + at + 32 * j + 8 * g) = kn[j];
+        if (g == 0) *reinterpret_cast<u32x4*>(f.v_cache + at + 8 * n) = vn;
+    };
     len = len < a.max_ctx ? len : a.max_ctx;
     const int steps = len > 0 ? (len + kStep - 1) / kStep : 0;
+    if constexpr (FRONT)
+        if (steps == 0 && p == 0 && wave == 0) {
+            load_front(G >= 4);
+            finish_front(G + 1);
+            append();
+        }
     if (p >= steps) return;                        // the whole workgroup
     const int waves = (steps - p + P - 1) / P < kWaves ? (steps - p + P - 1) / P : kWaves;
-    if (n >= G)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) q[j] = u32x4{0u, 0u, 0u, 0u};
 
     f32x4 acc[8];
 #pragma unroll
@@ -68,21 +156,55 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a) {
     float m = -INFINITY, l = 0.f;
 
     // Row r of key tile t is token 8 (r / 4) + 4 t + r % 4 of the step, so that lane group g ends up with tokens 8 g .. 8 g + 7.
-    const int64_t k_lane = (8 * (n >> 2) + (n & 3)) * a.tok_stride + 8 * g, v_lane = g * a.tok_stride + 8 * n;
+    const uint32_t tok = (uint32_t)a.tok_stride, k_lane = (8 * (n >> 2) + (n & 3)) * tok + 8 * g, v_lane = g * tok + 8 * n;
     u32x4 k[2][4], v[8];
+    int64_t row0 = 0;                              // slot of the requested step's first token
     auto request = [&](int step, int id) {
-        id = id < 0 ? 0 : id >= a.num_blocks ? a.num_blocks - 1 : id;
+        id = __builtin_amdgcn_readfirstlane(id < 0 ? 0 : id >= a.num_blocks ? a.num_blocks - 1 : id);
         const int in = (int)((unsigned)step % per_block) * kStep;
         const int64_t at = (int64_t)id * a.blk_stride + in * a.tok_stride + (int64_t)h * kD;
+        const uint16_t *kb = a.k + at, *vb = a.v + at;       // one for the wavefront; lanes differ in 32 bits
+        row0 = (int64_t)id * a.block_size + in;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) k[t][j] = load16(a.k + at + k_lane + 4 * t * a.tok_stride + 32 * j);
+            for (int j = 0; j < 4; ++j) k[t][j] = load16(kb + 4 * t * a.tok_stride + k_lane + 32 * j);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = load16_stream(a.v + at + v_lane + 4 * i * a.tok_stride);
+        for (int i = 0; i < 8; ++i) v[i] = load16_stream(vb + 4 * i * a.tok_stride + v_lane);
     };
-    if (first < steps) request(first, blk);
+    bool newest = false;                           // this wavefront has the sequence's last step
+    if (first < steps) {
+        if constexpr (FRONT) {
+            newest = (steps - 1 - first) % stride == 0;
+            const int heads = G + newest;
+            load_front(heads > 4);
+            __builtin_amdgcn_sched_barrier(0);
+            request(first, blk);
+            __builtin_amdgcn_sched_barrier(0);     // the rest while keys and values are on their way
+            finish_front(heads);
+        } else {
+            request(first, blk);
+        }
+    }
+    if (n >= G)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[j] = u32x4{0u, 0u, 0u, 0u};
     for (int step = first; step < steps; step += stride) {
+        if constexpr (FRONT) {
+            if (step == steps - 1) {
+                const int i = len - 1 - step * kStep;      // the new token's place in the step, if the cache has it there
+                if (row0 + i == slot) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        if (8 * (n >> 2) + (n & 3) + 4 * t == i)
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) k[t][j] = kn[j];
+#pragma unroll
+                    for (int t = 0; t < 8; ++t)
+                        if (4 * t + g == i) v[t] = vn;
+                }
+            }
+        }
         f32x4 s[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -157,6 +279,8 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a) {
         lds_order();
         if (wave > 0 && wave < waves) leave(reinterpret_cast<float*>(lds));
         __syncthreads();
+        if constexpr (FRONT)
+            if (newest) append();                  // nothing waits for the stores any more
         if (wave > 0) return;
         for (int w = 1; w < waves; ++w) {
             const float* from = reinterpret_cast<const float*>(lds_all + w * kTile);
@@ -168,8 +292,10 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a) {
             l = l * f1 + o.y * f2;
             m = top;
         }
-    } else if (wave > 0) {
-        return;
+    } else {
+        if (wave > 0) return;
+        if constexpr (FRONT)
+            if (newest) append();
     }
     leave(a.rec + (((int64_t)b * a.num_kv_heads + h) * P + p) * few_record_floats(G));
 }
@@ -238,8 +364,10 @@ int few_decode_pieces(int64_t batch, int64_t num_kv_heads, int64_t max_tokens) {
     return (int)(p > most ? most : p);
 }
 
-int launch_few_decode(const FewDecode& a, hipStream_t stream) {
-    hipLaunchKernelGGL(few_decode_kernel, dim3((unsigned)a.pieces, (unsigned)a.num_kv_heads, (unsigned)a.batch), dim3(64 * kWaves), 0, stream, a);
+int launch_few_decode(const FewDecode& a, hipStream_t stream, const FewFront* front) {
+    const dim3 pieces((unsigned)a.pieces, (unsigned)a.num_kv_heads, (unsigned)a.batch);
+    if (front) hipLaunchKernelGGL(few_decode_kernel<true>, pieces, dim3(64 * kWaves), 0, stream, a, *front);
+    else hipLaunchKernelGGL(few_decode_kernel<false>, pieces, dim3(64 * kWaves), 0, stream, a, FewFront{});
     const int rc = (int)hipGetLastError();
     if (rc) return rc;
     const dim3 grid((unsigned)(a.group * a.num_kv_heads), (unsigned)a.batch), block(256);

@@ -1087,16 +1087,21 @@ int launch_merge(void* out, int64_t out_stride0, const int32_t* context_lens, in
     return (int)hipGetLastError();
 }
 
+// The arguments of the kernels for a few sequences; false where the batch is not small.
+bool few_args(const DecodeCall& c, void* records, void* out, int64_t out_stride0, FewDecode* a) {
+    const int64_t max_ctx = c.table_cols * c.block_size;
+    *a = FewDecode{(const uint16_t*)c.q, c.q_stride0, (const uint16_t*)c.k_cache, (const uint16_t*)c.v_cache, c.cache_block_stride,
+                   c.cache_token_stride, c.block_table, c.bt_stride0, c.context_lens, max_ctx > 0x7fffffffLL ? 0x7fffffff : (int)max_ctx,
+                   (int)c.batch, (int)(c.num_q_heads / c.num_kv_heads), (int)c.num_kv_heads, (int)c.block_size, (int)c.num_blocks,
+                   c.scale * 1.4426950408889634f, few_decode_pieces(c.batch, c.num_kv_heads, max_ctx), (float*)records, (uint16_t*)out, out_stride0};
+    return a->pieces > 0;
+}
+size_t few_bytes(const FewDecode& a) { return (size_t)a.batch * a.num_kv_heads * a.pieces * few_record_floats(a.group) * sizeof(float); }
+
 // A few sequences, if their pieces fit the memory laid out as `ws`: true and the launches' return code.
 bool run_few(const DecodeCall& c, const DecodeWorkspace& ws, void* base, void* out, int64_t out_stride0, hipStream_t stream, int* rc) {
-    const int64_t max_ctx = c.table_cols * c.block_size;
-    const int pieces = few_decode_pieces(c.batch, c.num_kv_heads, max_ctx), group = (int)(c.num_q_heads / c.num_kv_heads);
-    const size_t need = (size_t)c.batch * c.num_kv_heads * pieces * few_record_floats(group) * sizeof(float);
-    if (pieces == 0 || need > ws.total_bytes - ws.rec_first_off) return false;
-    const FewDecode a{(const uint16_t*)c.q, c.q_stride0, (const uint16_t*)c.k_cache, (const uint16_t*)c.v_cache, c.cache_block_stride,
-                      c.cache_token_stride, c.block_table, c.bt_stride0, c.context_lens, max_ctx > 0x7fffffffLL ? 0x7fffffff : (int)max_ctx,
-                      (int)c.batch, group, (int)c.num_kv_heads, (int)c.block_size, (int)c.num_blocks, c.scale * 1.4426950408889634f, pieces,
-                      (float*)((char*)base + ws.rec_first_off), (uint16_t*)out, out_stride0};
+    FewDecode a;
+    if (!few_args(c, (char*)base + ws.rec_first_off, out, out_stride0, &a) || few_bytes(a) > ws.total_bytes - ws.rec_first_off) return false;
     *rc = launch_few_decode(a, stream);
     return true;
 }
@@ -1268,6 +1273,38 @@ int infer_paged_decode_noalloc_bf16(const void* q, int64_t q_stride0, const void
     if (ws.total_bytes > kNoAllocScratchBytes) return INFER_KV_EWORKSPACE;
     if (run_few(c, ws, scratch, out, out_stride0, (hipStream_t)stream, &rc)) return rc;
     return run_decode(c, L, ws, scratch, out, out_stride0, (hipStream_t)stream);
+}
+
+size_t infer_few_decode_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_tokens) {
+    if (num_kv_heads < 1 || num_q_heads < 1 || num_q_heads % num_kv_heads || num_q_heads / num_kv_heads > 16 || head_dim != kD) return 0;
+    const int pieces = few_decode_pieces(batch, num_kv_heads, max_tokens);
+    return (size_t)batch * num_kv_heads * pieces * few_record_floats((int)(num_q_heads / num_kv_heads)) * sizeof(float);
+}
+
+int infer_few_decode_front_bf16(const void* q, int64_t q_stride0, const void* k, int64_t k_stride0, const void* v, int64_t v_stride0,
+                                const int64_t* positions, const void* q_norm_weight, const void* k_norm_weight, float eps,
+                                const void* cos_sin_cache, int64_t max_position, void* k_cache, void* v_cache, const int32_t* slot_mapping,
+                                void* out, int64_t out_stride0, const int32_t* block_table, int64_t bt_stride0, int64_t table_cols,
+                                const int32_t* context_lens, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
+                                int64_t block_size, int64_t num_blocks, float scale, void* workspace, size_t workspace_bytes, void* stream) {
+    const int64_t token = num_kv_heads * head_dim;
+    const DecodeCall c{q, q_stride0, k_cache, v_cache, block_size * token, token, block_table, bt_stride0, table_cols, context_lens, batch,
+                       num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, scale};
+    if (!context_lens || !k || !v || !positions || !q_norm_weight || !k_norm_weight || !cos_sin_cache || !slot_mapping || max_position <= 0) return INFER_KV_EINVAL;
+    int rc = check_split(c, 0, workspace);
+    if (rc) return rc;
+    rc = check_out(out, out_stride0, num_q_heads);
+    if (rc) return rc;
+    if (k_stride0 < token || v_stride0 < token || q_stride0 < num_q_heads * head_dim) return INFER_KV_EINVAL;
+    if ((((uintptr_t)k | (uintptr_t)v | (uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight | (uintptr_t)cos_sin_cache) & 15) || ((k_stride0 | v_stride0) & 7))
+        return INFER_KV_EALIGN;
+    FewDecode a;
+    if (!few_args(c, workspace, out, out_stride0, &a)) return INFER_KV_EUNSUPPORTED;
+    if (few_bytes(a) > workspace_bytes) return INFER_KV_EWORKSPACE;
+    const FewFront f{(const uint16_t*)k, k_stride0, (const uint16_t*)v, v_stride0, positions, (const uint16_t*)q_norm_weight,
+                     (const uint16_t*)k_norm_weight, (const uint16_t*)cos_sin_cache, max_position, (uint16_t*)k_cache, (uint16_t*)v_cache,
+                     slot_mapping, num_blocks * block_size, eps};
+    return launch_few_decode(a, (hipStream_t)stream, &f);
 }
 
 }  // extern "C"

@@ -115,6 +115,44 @@ def qk_norm_rope_store_kvcache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     _lib.check(rc, "qk_norm_rope_store_kvcache")
 
 
+def few_decode_with_front(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, positions: torch.Tensor, q_norm_weight: torch.Tensor,
+                          k_norm_weight: torch.Tensor, eps: float, cos_sin_cache: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                          slot_mapping: torch.Tensor, block_table: torch.Tensor, context_lens: torch.Tensor, scale: float) -> torch.Tensor | None:
+    """``qk_norm_rope_store_kvcache`` and decode attention behind it, of one new token of each of a few sequences, or ``None`` where the
+    batch is not small.  The rows stay as they are; the caches get what they would get.  A sequence's last position is its row's slot, and
+    no row's slot lies in the context of another row."""
+    n, hq, d = q.shape
+    nblk, bs, hkv, _ = k_cache.shape
+    if context_lens is None or block_table is None or n == 0 or block_table.shape[0] != n or block_table.shape[1] < 1 or bs % 32:
+        return None
+    nbytes = _lib.load().infer_few_decode_workspace_bytes(n, hq, hkv, d, block_table.shape[1] * bs)
+    if not nbytes:
+        return None
+    assert k.shape == (n, hkv, d) and v.shape == (n, hkv, d)
+    for t in (q, k, v, q_norm_weight, k_norm_weight, cos_sin_cache, k_cache, v_cache):
+        assert t.dtype == torch.bfloat16
+    for t in (q, k, v):
+        assert t.stride(2) == 1 and t.stride(1) == d
+    assert q_norm_weight.shape == (d,) and k_norm_weight.shape == (d,)
+    assert q_norm_weight.is_contiguous() and k_norm_weight.is_contiguous()
+    assert cos_sin_cache.dim() == 2 and cos_sin_cache.shape[1] == d and cos_sin_cache.is_contiguous()
+    assert positions.dtype == torch.int64 and positions.numel() == n and positions.is_contiguous()
+    for t in (slot_mapping, context_lens):
+        assert t.dtype == torch.int32 and t.numel() == n and t.is_contiguous()
+    assert block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1
+    assert k_cache.shape == v_cache.shape and k_cache.is_contiguous() and v_cache.is_contiguous()
+    _require_gpu(q, k, v, positions, q_norm_weight, k_norm_weight, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, context_lens)
+    pieces = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+    out = torch.empty((n, hq, d), dtype=q.dtype, device=q.device)
+    rc = _lib.load().infer_few_decode_front_bf16(
+        q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), positions.data_ptr(), q_norm_weight.data_ptr(),
+        k_norm_weight.data_ptr(), float(eps), cos_sin_cache.data_ptr(), cos_sin_cache.shape[0], k_cache.data_ptr(), v_cache.data_ptr(),
+        slot_mapping.data_ptr(), out.data_ptr(), out.stride(0), block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
+        context_lens.data_ptr(), n, hq, hkv, d, bs, nblk, float(scale), pieces.data_ptr(), nbytes, _stream_ptr(q))
+    _lib.check(rc, "few_decode_with_front")
+    return out
+
+
 def decode_workspace(device, max_batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int) -> torch.Tensor:
     """Workspace for the split-KV partial results, cached per (device, shape): allocated once so that
     steady-state decode steps (and HIP graph replays) never allocate."""

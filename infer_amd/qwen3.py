@@ -13,7 +13,8 @@ from . import kv_runner, ops
 from .attention import Attention
 from .cache import PagedKVLayout
 from .context import get_context
-from .layers import MLP, Embedding, Linear, LMHead, QKVLinear, RMSNorm, _is_bare, cos_sin_table, is_bare_mlp, norm_and_project
+from .layers import (MLP, Embedding, Linear, LMHead, QKVLinear, RMSNorm, _is_bare, cos_sin_table, is_bare_attention, is_bare_mlp, is_bare_norm,
+                     norm_and_project)
 
 
 class QwenAttention(nn.Module):
@@ -67,6 +68,12 @@ class QwenAttention(nn.Module):
         # keys are read back from the packed rows only by a prefill without a cached prefix
         keys_from_rows = context.is_prefill and context.block_tables is None
         table = cos_sin_table(self.head_dim, self.max_position, self.rope_theta, q.device)
+        if bound and not context.is_prefill and is_bare_norm(self.q_norm) and is_bare_norm(self.k_norm) and is_bare_attention(self.attn):
+            # a few sequences: norms, rotary positions and append in the launch of the attention
+            o = ops.few_decode_with_front(q, k, v, positions, self.q_norm.weight, self.k_norm.weight, self.q_norm.eps, table, k_cache, v_cache, slots,
+                                          context.block_tables, context.context_lens, self.attn.scale)
+            if o is not None:
+                return self.o_proj(o.view(-1, self.q_size), defer=True)
         ops.qk_norm_rope_store_kvcache(q, k, v, positions, self.q_norm.weight, self.k_norm.weight,
                                        self.q_norm.eps, table, k_cache, v_cache, slots, write_key=keys_from_rows)
         o = self.attn(q, k, v, kv_stored=True)

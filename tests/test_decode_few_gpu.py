@@ -105,3 +105,52 @@ def test_captured_and_replayed_with_other_lengths(gpu):
         graph.replay()
         want = _reference(q, k, v, table, now, 128 ** -0.5)
         assert (out.double().cpu() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("lens,hq,hkv,block", [
+    ([1], 16, 8, 256), ([31, 32, 33, 0], 16, 8, 256), ([1024, 1025, 2049], 32, 8, 256), ([700, 64, 257, 4096, 1, 96, 128, 3000], 32, 8, 256),
+    ([9000], 16, 1, 64), ([129] * 6, 48, 8, 96), ([33, 65], 5, 5, 32), ([65, 70], 4, 1, 64),
+])
+def test_with_the_front_as_in_two_launches(gpu, lens, hq, hkv, block):
+    """Norms, rotary positions and the append inside: the bits of the launches one after the other, in the caches and in the result.  Stale
+    NaN lies where the new rows belong; one row's slot is elsewhere, one has none, one has a slot and no tokens."""
+    gen = torch.Generator().manual_seed(sum(lens) + hkv)
+    _, k, v, table, ctx = _inputs(gen, lens, hq, hkv, block)
+    n, spare = len(lens), (k.shape[0] - 1) * block
+    slots = [int(table[i, (m - 1) // block]) * block + (m - 1) % block if m else -1 for i, m in enumerate(lens)]
+    free = sorted(set(range(k.shape[0])) - set(table.flatten().tolist()))
+    for i, s in enumerate(slots):
+        if s >= 0:
+            for t in (k, v):
+                t.view(-1, hkv, 128)[s] = float("nan")
+    if n > 2:
+        slots[1] = free[0] * block + 3                    # elsewhere: what the cache has there is attended
+        k.view(-1, hkv, 128)[int(table[1, (lens[1] - 1) // block]) * block + (lens[1] - 1) % block] = 1.0
+        v.view(-1, hkv, 128)[int(table[1, (lens[1] - 1) // block]) * block + (lens[1] - 1) % block] = 1.0
+        if lens[-1] == 0:
+            slots[-1] = free[0] * block + 5
+    slots = torch.tensor(slots, dtype=torch.int32).cuda()
+    qkv = (3 * torch.randn(n, (hq + 2 * hkv) * 128 + 64, generator=gen)).to(BF16).cuda()[:, 64:]
+    q, kn, vn = (t.view(n, -1, 128) for t in qkv.split([hq * 128, hkv * 128, hkv * 128], -1))
+    wq, wk = ((1 + 0.3 * torch.randn(128, generator=gen)).to(BF16).cuda() for _ in range(2))
+    cs = torch.randn(max(lens) + 9, 128, generator=gen).to(BF16).cuda()
+    positions = torch.tensor([max(m - 1, 0) + 5 * (i % 2) for i, m in enumerate(lens)]).cuda()
+    k2, v2, kept = k.clone(), v.clone(), qkv.clone()
+    out = ops.few_decode_with_front(q, kn, vn, positions, wq, wk, 1e-6, cs, k2, v2, slots, table, ctx, 0.09)
+    assert torch.equal(qkv, kept)
+    ops.qk_norm_rope_store_kvcache(q, kn, vn, positions, wq, wk, 1e-6, cs, k, v, slots, write_key=False)
+    want = torch.empty_like(out)
+    ops.paged_attn_decode(q, k, v, table, ctx, 0.09, want)
+    same = lambda a, b: torch.equal(a.view(torch.int16), b.view(torch.int16))
+    assert same(k, k2) and same(v, v2)
+    assert torch.isfinite(out.float()).all() and torch.equal(out, want)
+
+
+def test_batches_that_are_not_small_are_left_alone(gpu):
+    gen = torch.Generator().manual_seed(9)
+    q, k, v, table, ctx = _inputs(gen, [64] * 9, 16, 8, 256)
+    rows, w = torch.zeros(9, 8, 128, dtype=BF16, device="cuda"), torch.ones(128, dtype=BF16, device="cuda")
+    cs, at = torch.ones(64, 128, dtype=BF16, device="cuda"), torch.zeros(9, dtype=torch.int64, device="cuda")
+    kept = k.clone()
+    assert ops.few_decode_with_front(q, rows, rows, at, w, w, 1e-6, cs, k, v, at.int(), table, ctx, 0.1) is None
+    assert torch.equal(k, kept)
