@@ -12,6 +12,9 @@ current stream.  Tensors must live on the GPU; there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
+import os
 import threading
 from collections import OrderedDict
 
@@ -176,7 +179,19 @@ def decode_workspace(device, max_batch: int, num_q_heads: int, num_kv_heads: int
 _workspace_streams: dict = {}      # data_ptr of a shared workspace -> the stream that used it last: (handle, Stream)
 
 
-def _claim_shared_workspace(workspace: torch.Tensor, device) -> None:
+def _load_decode_call():
+    """The native form of ``flash_attn_with_kvcache``.  It stands on the library next to it, so it is left out where another one is asked for."""
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_decode_call.so")
+    if "INFER_KV_LIB" in os.environ or not os.path.exists(path):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("_decode_call", path)
+    return importlib.util.module_from_spec(importlib.machinery.ModuleSpec("_decode_call", loader, origin=path))
+
+
+_decode_call = _load_decode_call()
+
+
+def _claim_shared_workspace(workspace: torch.Tensor, device, heads=None) -> None:
     """The shared workspace holds the partial results of a call until its merge kernel has run, so calls
     that use it must be ordered on one stream.  A call on another stream while the last one still has work
     pending is refused (a host-side check on a change of stream only; streams under capture are not
@@ -189,6 +204,8 @@ def _claim_shared_workspace(workspace: torch.Tensor, device) -> None:
         raise RuntimeError("paged decode: the shared workspace is still in use on another stream; "
                            "order the calls on one stream or pass a workspace of their own")
     _workspace_streams[key] = (handle, torch.cuda.current_stream(device))
+    if _decode_call is not None and heads is not None:
+        _decode_call.claim(workspace.get_device(), *heads, key, workspace.numel(), handle)
 
 
 def _decode_args(q3, k_cache, v_cache, cache_seqlens, block_table):
@@ -226,7 +243,7 @@ def paged_attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     assert out.shape == q.shape and out.dtype == torch.bfloat16 and out.stride(2) == 1 and out.stride(1) == d
     if workspace is None:
         workspace = decode_workspace(q.device, b, hq, hkv, d)
-        _claim_shared_workspace(workspace, q.device)
+        _claim_shared_workspace(workspace, q.device, (hq, hkv))
     lib = _lib.load()
     if isinstance(context_lens, int):
         rc = lib.infer_paged_decode_uniform_bf16(
@@ -271,6 +288,10 @@ def flash_attn_with_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     """``q`` is ``[B, 1, Hq, D]``; returns ``[B, 1, Hq, D]``.  With a single query token the causal
     mask hides nothing, so ``causal`` only has to be accepted.  ``cache_seqlens`` is an int32 tensor
     ``[B]`` or one int for the whole batch, as in flash-attn."""
+    if _decode_call is not None:
+        done = _decode_call.decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale)
+        if done is not None:
+            return done
     assert q.dim() == 4 and q.shape[1] == 1, "decode takes one query token per sequence"
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** -0.5
@@ -590,7 +611,6 @@ def _linear_mode() -> str:
     """``INFER_AMD_LINEAR``: ``static`` (default: the fixed rule above, the same kernel for a shape in every
     process), ``vendor`` (never the split-K kernel), ``measure`` (time both once per shape with cold caches and
     keep the faster: a tuning aid, not reproducible from run to run)."""
-    import os
     mode = os.environ.get("INFER_AMD_LINEAR", "static")
     if mode not in ("static", "vendor", "measure"):
         raise RuntimeError(f"INFER_AMD_LINEAR must be static, vendor or measure, not {mode!r}")
