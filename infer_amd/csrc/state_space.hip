@@ -31,7 +31,6 @@ typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 constexpr int kThreads = 256;
 constexpr int kC = 32;          // tokens per chunk
 constexpr int kSlab = 64;       // state columns per workgroup of the chunk kernel
-constexpr int kAhead = kThreads / 64;   // chunks whose step sizes are computed together, one per wavefront
 
 struct Span { int32_t row0, count, slot, pos0; };       // consecutive tokens of one sequence
 
@@ -280,20 +279,34 @@ __device__ __forceinline__ int own_segment(int count, int most) {
     return segs > 1 ? ((count + segs - 1) / segs + kC - 1) / kC * kC : most;
 }
 
-// A workgroup of four wavefronts serves one head and 64 columns of its state over the chunks of one segment; wavefront w owns 16
-// columns as accumulators: lane (g, n) holds state rows 16 t + 4 g + e of column n.  That is an operand of the product with C as it
-// lies, when the state rows of a k-step of 32 are taken in the order 16 tau + 4 g + e.  The 32 x 32 products C_i B_j are shared
-// out over the wavefronts, weighted, and exchanged through LDS.  OUT = false: only the final state, from zero.
-template <int NS, bool OUT>
-__global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) {
+// A workgroup serves one head and 64 columns of its state over the chunks of one segment.  Wavefront w owns 16 columns as accumulators, of
+// eight wavefronts half the state rows each: lane (g, n) holds state rows 16 t + 4 g + e of column n.  That is an operand of the product with C
+// as it lies, when the state rows of a k-step of 32 are taken in the order 16 tau + 4 g + e.  The 32 x 32 products C_i B_j are shared
+// out over the wavefronts of the first half, weighted, and exchanged through LDS; those of the second add up and write the results.
+// OUT = false: only the final state, from zero.
+// A portion takes as long as its chunks one after the other, and a chunk as long as one wavefront's instructions and reads of LDS (four
+// wavefronts: 445 and 30 reads, 3900 clocks with three barriers).  Eight halve what follows one another, and where two chunks lie in LDS one
+// barrier is left, behind which a chunk's results are finished under the next one's products.  6 portions of 900 to 3700 tokens of 64 heads,
+// the call: 324 us, 310 with the barriers alone, 286 with eight wavefronts.
+template <int NS, int WAVES, bool OUT>
+__global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm_chunk_kernel(ChunkArgs args) {
     constexpr int kRow = NS * 64 + 16, kXRow = 2 * kSlab + 16, kMRow = 2 * kC + 16;      // bytes
-    constexpr int NU = NS > 2 ? NS / 2 : 1;                      // 16-byte units of B (and of C) per thread
-    __shared__ __attribute__((aligned(16))) unsigned char bbuf[kC * kRow], cbuf[OUT ? kC * kRow : 16], xbuf[kC * kXRow];
-    __shared__ __attribute__((aligned(16))) unsigned char mbuf[OUT ? 2 * kC * kMRow : 16];
-    __shared__ __attribute__((aligned(16))) float sums[kAhead][kC], steps[kAhead][kC], weights[kAhead][kC];
+    constexpr int kThr = 64 * WAVES, kParts = WAVES / 4, NT = 2 * NS / kParts;      // tiles of 16 state rows per wavefront
+    constexpr int kAhead = WAVES;                                // chunks whose step sizes are computed together, one per wavefront
+    constexpr int NU = (NS * 2 * kC * 2 + kThr - 1) / kThr;      // 16-byte units of B (and of C) per thread
+    constexpr int kBufs = NS > 4 || WAVES == 4 ? 1 : 2;                        // chunks of B, C and x in LDS
+    extern __shared__ __attribute__((aligned(16))) unsigned char chunk_lds[];
+    auto &bbufs = *reinterpret_cast<unsigned char(*)[kBufs][kC * kRow]>(chunk_lds), &cbufs = *reinterpret_cast<unsigned char(*)[kBufs][kC * kRow]>(chunk_lds + sizeof(bbufs));
+    auto& xbufs = *reinterpret_cast<unsigned char(*)[kBufs][kC * kXRow]>(chunk_lds + (OUT ? 2 : 1) * sizeof(bbufs));
+    unsigned char* behind = chunk_lds + (OUT ? 2 : 1) * sizeof(bbufs) + sizeof(xbufs);
+    auto& sums = *reinterpret_cast<float(*)[2][kAhead][kC]>(behind);
+    auto& steps = *reinterpret_cast<float(*)[2][kAhead][kC]>(behind + sizeof(sums));
+    auto& weights = *reinterpret_cast<float(*)[2][kAhead][kC]>(behind + 2 * sizeof(sums));
+    auto& mbufs = *reinterpret_cast<unsigned char(*)[2][2 * kC * kMRow]>(behind + 3 * sizeof(sums));               // OUT
+    auto& ybufs = *reinterpret_cast<f32x4_t(*)[2][4][2][64]>(behind + 3 * sizeof(sums) + sizeof(mbufs));           // OUT
     const SsmArgs<__bf16>& a = args.a;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2, cw = wave & 3;
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
     const Span span = args.spans[blockIdx.z];
     const int seg_len = own_segment(span.count, args.seg_len), first = seg * seg_len;
@@ -303,7 +316,7 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
     const int count = last_seg ? span.count - first : seg_len;
     const int row0 = span.row0 + first, chunks = (count + kC - 1) / kC;
     const int N = a.state_n, inner = a.heads * a.vdim, grp = h / (a.heads / a.groups);
-    const int v0 = slab * kSlab + wave * 16;                     // this wavefront's first column
+    const int v0 = slab * kSlab + cw * 16, r0 = half * 16 * NT;  // this wavefront's first column and state row
     const int64_t state_len = (int64_t)N * a.vdim;
     float* from = a.state + ((int64_t)span.slot * a.heads + h) * state_len;
     float* to = from;
@@ -314,30 +327,28 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
     }
     const bool load = OUT && (args.max_seg > 1 || span.pos0 > 0), col_live = v0 + n < a.vdim;
 
-    f32x4_t s[2 * NS];
+    f32x4_t s[NT];
 #pragma unroll
-    for (int t = 0; t < 2 * NS; ++t) {
+    for (int t = 0; t < NT; ++t) {
         s[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         if (load && col_live)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (16 * t + 4 * g + e < N) s[t][e] = from[(int64_t)(16 * t + 4 * g + e) * a.vdim + v0 + n];
+                if (r0 + 16 * t + 4 * g + e < N) s[t][e] = from[(int64_t)(r0 + 16 * t + 4 * g + e) * a.vdim + v0 + n];
     }
     // entries behind the real sizes stay zero
-    for (int i = tid; i < (int)sizeof(bbuf) / 16; i += kThreads) reinterpret_cast<u32x4_t*>(bbuf)[i] = u32x4_t{0u, 0u, 0u, 0u};
-    for (int i = tid; i < (int)sizeof(cbuf) / 16; i += kThreads) reinterpret_cast<u32x4_t*>(cbuf)[i] = u32x4_t{0u, 0u, 0u, 0u};
-    for (int i = tid; i < (int)sizeof(xbuf) / 16; i += kThreads) reinterpret_cast<u32x4_t*>(xbuf)[i] = u32x4_t{0u, 0u, 0u, 0u};
+    for (int i = tid; i < (int)((OUT ? 2 : 1) * sizeof(bbufs) + sizeof(xbufs)) / 16; i += kThr) reinterpret_cast<u32x4_t*>(chunk_lds)[i] = u32x4_t{0u, 0u, 0u, 0u};
 
     const int units = N / 8;
     int u_tok[NU], u_col[NU];                                    // token -1: no such unit; its load repeats another one
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-        const int u = tid + kThreads * i;
+        const int u = tid + kThr * i;
         u_tok[i] = u < kC * units ? u / units : -1;
         u_col[i] = 8 * (u % units);
     }
-    const int x_tok = tid >> 3, x_col = 8 * (tid & 7);
-    const bool x_in = slab * kSlab + x_col < a.vdim;
+    const int x_tok = tid >> 3 & (kC - 1), x_col = 8 * (tid & 7);
+    const bool x_in = tid < 8 * kC && slab * kSlab + x_col < a.vdim;
     const __bf16* rows = a.xbc + (row0 - a.xbc_row0) * a.xbc_stride;
     const __bf16* b_src = rows + inner + grp * N;
     const __bf16* c_src = b_src + a.groups * N;
@@ -362,74 +373,108 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
     };
     const float a2 = -expf(a.a_log[h]) * kLog2e, bias = a.dt_bias[h], dh = a.d[h];
     float total = 0.f;                                           // log2 of the segment's decay
-    fetch(0);
-    fetch_dt(wave);
-    for (int c = 0; c < chunks; ++c) {
-        __syncthreads();
-        if (c % kAhead == 0) {                                   // this wavefront's chunk is c + wave
-            const float dt = (c + wave) * kC + (lane & 31) < count ? softplus_f((float)dtreg + bias) : 0.f;
-            float G = fmaxf(a2 * dt, -160.f);                    // nothing is left beyond, and sums stay precise
+    // step sizes of chunks c .. c + 3, this wavefront's being c + wave
+    auto put_steps = [&](int c) {
+        const int group = (c / kAhead) & 1;
+        const float dt = (c + wave) * kC + (lane & 31) < count ? softplus_f((float)dtreg + bias) : 0.f;
+        float G = fmaxf(a2 * dt, -160.f);                        // nothing is left beyond, and sums stay precise
 #pragma unroll
-            for (int m = 1; m < kC; m <<= 1) {
-                const float up = __shfl_up(G, m, 32);
-                G += (lane & 31) >= m ? up : 0.f;
-            }
-            const float end = __shfl(G, kC - 1, 64);
-            if (lane < kC) {
-                sums[wave][lane] = G;
-                steps[wave][lane] = dt;
-                weights[wave][lane] = __builtin_amdgcn_exp2f(end - G) * dt;
-            }
-            fetch_dt(c + kAhead + wave);
+        for (int m = 1; m < kC; m <<= 1) {
+            const float up = __shfl_up(G, m, 32);
+            G += (lane & 31) >= m ? up : 0.f;
         }
+        const float end = __shfl(G, kC - 1, 64);
+        if (lane < kC) {
+            sums[group][wave][lane] = G;
+            steps[group][wave][lane] = dt;
+            weights[group][wave][lane] = __builtin_amdgcn_exp2f(end - G) * dt;
+        }
+        fetch_dt(c + kAhead + wave);
+    };
+    auto put = [&](int c) {
 #pragma unroll
         for (int i = 0; i < NU; ++i)
             if (u_tok[i] >= 0) {
-                *reinterpret_cast<u32x4_t*>(bbuf + u_tok[i] * kRow + 2 * u_col[i]) = breg[i];
-                if constexpr (OUT) *reinterpret_cast<u32x4_t*>(cbuf + u_tok[i] * kRow + 2 * u_col[i]) = creg[i];
+                *reinterpret_cast<u32x4_t*>(bbufs[c % kBufs] + u_tok[i] * kRow + 2 * u_col[i]) = breg[i];
+                if constexpr (OUT) *reinterpret_cast<u32x4_t*>(cbufs[c % kBufs] + u_tok[i] * kRow + 2 * u_col[i]) = creg[i];
             }
-        if (x_in) *reinterpret_cast<u32x4_t*>(xbuf + x_tok * kXRow + 2 * x_col) = xreg;
-        if (c + 1 < chunks) fetch(c + 1);
+        if (x_in) *reinterpret_cast<u32x4_t*>(xbufs[c % kBufs] + x_tok * kXRow + 2 * x_col) = xreg;
+    };
+    f32x4_t y[2];
+    bf16x8_t xf;
+    // what the chunk's own tokens add to the results, and their way out
+    auto finish = [&](int c) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if constexpr (kParts > 1) y[t] += ybufs[c & 1][cw][t][lane];
+#pragma unroll
+            for (int k = 1; k >= 0; --k) {
+                const bf16x8_t mf = *reinterpret_cast<const bf16x8_t*>(mbufs[c & 1] + k * kC * kMRow + (16 * t + n) * kMRow + 16 * g);
+                y[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, mf, y[t], 0, 0, 0);
+            }
+            const int tok = c * kC + 16 * t + n;
+            if (tok < count && v0 + 4 * g < a.vdim) {
+                bf16x4_t o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = (__bf16)y[t][e];
+                *reinterpret_cast<bf16x4_t*>(a.y + (row0 + tok) * a.y_stride + h * a.vdim + v0 + 4 * g) = o;
+            }
+        }
+    };
+    fetch(0);
+    fetch_dt(wave);
+    __syncthreads();                                             // the zero fill
+    put_steps(0);
+    put(0);
+    if (chunks > 1) fetch(1);
+    // Behind the barrier the chunk lies in LDS, and the products of the last chunk's tokens, whose results are finished while
+    // this chunk's products run.  Everything that is written between two barriers was read last in front of the first.
+#pragma unroll 1                                                 // unrolled it spills
+    for (int c = 0; c < chunks; ++c) {
         __syncthreads();
-        const float* sum = sums[c % kAhead];
-        const float* step = steps[c % kAhead];
-        const float* weight = weights[c % kAhead];
+        if constexpr (OUT)
+            if (half == kParts - 1 && c > 0) finish(c - 1);
+        unsigned char *bbuf = bbufs[c % kBufs], *cbuf = cbufs[c % kBufs], *xbuf = xbufs[c % kBufs], *mbuf = mbufs[c & 1];
+        const float* sum = sums[(c / kAhead) & 1][c % kAhead];
+        const float* step = steps[(c / kAhead) & 1][c % kAhead];
+        const float* weight = weights[(c / kAhead) & 1][c % kAhead];
         const float G_end = sum[kC - 1];
         // x of this wavefront's columns: lane (g, n) has tokens 8 g .. 8 g + 7 of column n
-        const unsigned char* xr = xbuf + (8 * g + (n >> 2)) * kXRow + (n & 3) * 8 + 32 * wave;
+        const unsigned char* xr = xbuf + (8 * g + (n >> 2)) * kXRow + (n & 3) * 8 + 32 * cw;
         const i16x4 xlo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)xr);
         const i16x4 xhi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(xr + 4 * kXRow));
-        const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(xlo, xhi, 0, 1, 2, 3, 4, 5, 6, 7));
-        f32x4_t y[2];
+        xf = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(xlo, xhi, 0, 1, 2, 3, 4, 5, 6, 7));
         if constexpr (OUT) {
-            // products C_i B_j of one 16 x 16 tile: lane (g, n) gets tokens j = 4 g + e and i = n of it
-            const int sj = wave >> 1, ti = wave & 1;
-            f32x4_t m = {0.f, 0.f, 0.f, 0.f};
-            if (sj <= ti) {
+            if (half == 0) {
+                // products C_i B_j of one 16 x 16 tile: lane (g, n) gets tokens j = 4 g + e and i = n of it
+                const int sj = cw >> 1, ti = cw & 1;
+                f32x4_t m = {0.f, 0.f, 0.f, 0.f};
+                if (sj <= ti) {
 #pragma unroll
-                for (int k = 0; k < NS; ++k) {
-                    const bf16x8_t bf = *reinterpret_cast<const bf16x8_t*>(bbuf + (16 * sj + n) * kRow + 64 * k + 16 * g);
-                    const bf16x8_t cf = *reinterpret_cast<const bf16x8_t*>(cbuf + (16 * ti + n) * kRow + 64 * k + 16 * g);
-                    m = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf, cf, m, 0, 0, 0);
+                    for (int k = 0; k < NS; ++k) {
+                        const bf16x8_t bf = *reinterpret_cast<const bf16x8_t*>(bbuf + (16 * sj + n) * kRow + 64 * k + 16 * g);
+                        const bf16x8_t cf = *reinterpret_cast<const bf16x8_t*>(cbuf + (16 * ti + n) * kRow + 64 * k + 16 * g);
+                        m = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf, cf, m, 0, 0, 0);
+                    }
                 }
-            }
-            const int i = 16 * ti + n, j0 = 16 * sj + 4 * g;
-            float v[4];
+                const int i = 16 * ti + n, j0 = 16 * sj + 4 * g;
+                float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int j = j0 + e;
-                v[e] = j <= i ? m[e] * __builtin_amdgcn_exp2f(sum[i] - sum[j]) * step[j] : 0.f;
-                if (j == i) v[e] += dh;
-            }
-            uint32_t p[2][2];
-            split<2, 4>(v, p);
+                for (int e = 0; e < 4; ++e) {
+                    const int j = j0 + e;
+                    v[e] = j <= i ? m[e] * __builtin_amdgcn_exp2f(sum[i] - sum[j]) * step[j] : 0.f;
+                    if (j == i) v[e] += dh;
+                }
+                uint32_t p[2][2];
+                split<2, 4>(v, p);
 #pragma unroll
-            for (int k = 0; k < 2; ++k)
-                *reinterpret_cast<uint2*>(mbuf + k * kC * kMRow + i * kMRow + 2 * j0) = uint2{p[k][0], p[k][1]};
+                for (int k = 0; k < 2; ++k)
+                    *reinterpret_cast<uint2*>(mbuf + k * kC * kMRow + i * kMRow + 2 * j0) = uint2{p[k][0], p[k][1]};
+            }
             // products of the state: lane (g, n) gets columns 4 g + e for token n
             y[0] = y[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int k = 0; k < NS; ++k) {
+            for (int k = 0; k < NT / 2; ++k) {
                 float sv[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) sv[e] = s[2 * k + e / 4][e % 4];
@@ -437,7 +482,7 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
                 split_frags<2>(sv, sp);
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    const unsigned char* cr = cbuf + (16 * t + n) * kRow + 64 * k + 8 * g;
+                    const unsigned char* cr = cbuf + (16 * t + n) * kRow + 64 * (half * (NT / 2) + k) + 8 * g;
                     const uint2 lo = *reinterpret_cast<const uint2*>(cr), hi = *reinterpret_cast<const uint2*>(cr + 32);
                     const bf16x8_t cf = __builtin_bit_cast(bf16x8_t, u32x4_t{lo.x, lo.y, hi.x, hi.y});
                     y[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sp[1], cf, y[t], 0, 0, 0);
@@ -445,7 +490,10 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
                 }
             }
 #pragma unroll
-            for (int t = 0; t < 2; ++t) y[t] *= __builtin_amdgcn_exp2f(sum[16 * t + n]);
+            for (int t = 0; t < 2; ++t) {
+                y[t] *= __builtin_amdgcn_exp2f(sum[16 * t + n]);
+                if (kParts > 1 && half == 0) ybufs[c & 1][cw][t][lane] = y[t];
+            }
         }
         // the state
         float wx[8], xv[8];
@@ -457,8 +505,8 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
         const float carry = __builtin_amdgcn_exp2f(G_end);
         total += G_end;
 #pragma unroll
-        for (int t = 0; t < 2 * NS; ++t) {
-            const unsigned char* br = bbuf + (8 * g + (n >> 2)) * kRow + (n & 3) * 8 + 32 * t;
+        for (int t = 0; t < NT; ++t) {
+            const unsigned char* br = bbuf + (8 * g + (n >> 2)) * kRow + (n & 3) * 8 + 2 * r0 + 32 * t;
             const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)br);
             const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(br + 4 * kRow));
             const bf16x8_t bf = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -466,33 +514,25 @@ __global__ void __launch_bounds__(kThreads, 2) ssm_chunk_kernel(ChunkArgs args) 
 #pragma unroll
             for (int k = 2; k >= 0; --k) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf, xp[k], s[t], 0, 0, 0);
         }
-        if constexpr (OUT) {
-            __syncthreads();
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-#pragma unroll
-                for (int k = 1; k >= 0; --k) {
-                    const bf16x8_t mf = *reinterpret_cast<const bf16x8_t*>(mbuf + k * kC * kMRow + (16 * t + n) * kMRow + 16 * g);
-                    y[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, mf, y[t], 0, 0, 0);
-                }
-                const int tok = c * kC + 16 * t + n;
-                if (tok < count && v0 + 4 * g < a.vdim) {
-                    bf16x4_t o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = (__bf16)y[t][e];
-                    *reinterpret_cast<bf16x4_t*>(a.y + (row0 + tok) * a.y_stride + h * a.vdim + v0 + 4 * g) = o;
-                }
-            }
+        if (c + 1 < chunks) {
+            if constexpr (kBufs == 1) __syncthreads();
+            if ((c + 1) % kAhead == 0) put_steps(c + 1);
+            put(c + 1);
+            if (c + 2 < chunks) fetch(c + 2);
         }
+    }
+    if constexpr (OUT) {
+        __syncthreads();
+        if (half == kParts - 1) finish(chunks - 1);
     }
     if (!OUT && slab == 0 && tid == 0) args.ws_decay[rec] = total;
     if (OUT && !last_seg) return;
     if (col_live)
 #pragma unroll
-        for (int t = 0; t < 2 * NS; ++t)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (16 * t + 4 * g + e < N) to[(int64_t)(16 * t + 4 * g + e) * a.vdim + v0 + n] = s[t][e];
+                if (r0 + 16 * t + 4 * g + e < N) to[(int64_t)(r0 + 16 * t + 4 * g + e) * a.vdim + v0 + n] = s[t][e];
 }
 
 // final states of segments from zero -> the states in front of the segments
@@ -587,32 +627,49 @@ __global__ void __launch_bounds__(kThreads) ssm_norm_kernel(NormArgs<T> b) {
 // ------------------------------------------------------------------ launches
 bool chunked(int elem, int64_t vdim, int64_t state_n) { return elem == INFER_ELEM_BF16 && vdim % 8 == 0 && state_n % 8 == 0 && state_n <= 256; }
 
-// Segments that portions are cut into, so that enough workgroups run: most tokens of a segment and their largest number.  Cut portions are
-// walked twice, which pays below one and a half workgroups per compute unit.  Heads of 128 x 64, the call in us, cut for three workgroups per
-// compute unit / whole: 12 portions of 100 to 1500 tokens of 32 heads 181 / 172, 6 of 900 to 3700 of 64 heads 337 / 325, 7 of them
-// 385 / 348; but 5 of them 268 / 297, 4 of 500 to 3000 207 / 239.  Segments of one length per portion instead of one for the batch: 6 portions
-// of 32 heads 228 -> 220, 2 of 2000 to 5000 of 64 heads 181 -> 174.
-void segments(int64_t heads, int64_t slabs, int64_t num_spans, int64_t max_span, int64_t& seg_len, int64_t& max_seg) {
-    const int64_t units = heads * slabs * num_spans, chunks = (max_span + kC - 1) / kC;
-    int64_t want = units > 0 && units < 384 ? (768 + units - 1) / units : 1;       // three workgroups per compute unit
+// How portions are walked: wavefronts of a workgroup, and the segments that they are cut into so that enough workgroups run (most tokens of a
+// segment and their largest number).  Cut portions are walked twice, which pays below one workgroup of eight wavefronts or one and a half
+// of four per compute unit.  Heads of 128 x 64, the call in us, four wavefronts cut for three workgroups per compute unit / eight cut for
+// two: 6 portions of 900 to 3700 tokens of 64 heads 325 / 286, 5 of 1000 to 3000 248 / 211, 8 of 1000 174 / 158, 4 of 500 to 4000 252 / 245, 11 of
+// 500 to 1500 of 32 heads 185 / 158, 1 of 300 40 / 36.  Two workgroups of eight fit a compute unit; where there are more, four are ahead
+// (10 of 800 to 1800 of 64 heads 250 / 256), and with a long portion by itself, cut into equal segments (9000 of 64 heads 217 / 222).
+// Segments of one length per portion instead of one for the batch: 6 portions of 32 heads 228 -> 220.
+struct Walk { int waves, seg_len, max_seg; };
+Walk walk_of(int64_t heads, int64_t vdim, int64_t state_n, int64_t num_spans, int64_t max_span) {
+    const int64_t units = heads * ((vdim + kSlab - 1) / kSlab) * num_spans, chunks = (max_span + kC - 1) / kC;
+    const bool wide = units <= 512 && state_n <= 128 && !(num_spans == 1 && max_span >= 4096);
+    const int64_t full = wide ? 256 : 384;
+    int64_t want = units > 0 && units < full ? (2 * full + units - 1) / units : 1;
     if (want > chunks / 4) want = chunks / 4;              // no segment shorter than four chunks
     if (want < 1) want = 1;
-    const int64_t per = (chunks + want - 1) / want;
-    seg_len = (per > 0 ? per : 1) * kC;
-    max_seg = max_span > 0 ? (max_span + seg_len - 1) / seg_len : 1;
+    const int64_t per = (chunks + want - 1) / want, seg_len = (per > 0 ? per : 1) * kC;
+    return Walk{wide ? 8 : 4, (int)seg_len, (int)(max_span > 0 ? (max_span + seg_len - 1) / seg_len : 1)};
 }
 
-template <int NS>
+template <int NS, int WAVES, bool OUT>
+int launch_chunk(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
+    constexpr size_t bufs = NS > 4 || WAVES == 4 ? 1 : 2;
+    constexpr size_t lds = kC * (bufs * ((OUT ? 2 : 1) * (NS * 64 + 16) + 2 * kSlab + 16) + (OUT ? 2 * 2 * (2 * kC + 16) : 0)) +
+                           3 * 2 * WAVES * kC * sizeof(float) + (OUT && WAVES == 8 ? 2 * 4 * 2 * 64 * sizeof(f32x4_t) : 0);
+    auto kernel = &ssm_chunk_kernel<NS, WAVES, OUT>;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(c.slabs * c.max_seg), (unsigned)c.a.heads, (unsigned)num_spans), dim3(64 * WAVES), lds, st, c);
+    return (int)hipGetLastError();
+}
+
+template <int NS, int WAVES>
 int launch_chunks(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
-    const dim3 grid((unsigned)(c.slabs * c.max_seg), (unsigned)c.a.heads, (unsigned)num_spans), block(kThreads);
     if (c.max_seg > 1) {
-        hipLaunchKernelGGL((ssm_chunk_kernel<NS, false>), grid, block, 0, st, c);
+        const int rc = launch_chunk<NS, WAVES, false>(c, num_spans, st);
+        if (rc) return rc;
         const int64_t state_len = (int64_t)c.a.state_n * c.a.vdim;
         hipLaunchKernelGGL(ssm_join_kernel, dim3((unsigned)((state_len + kThreads - 1) / kThreads), (unsigned)c.a.heads, (unsigned)num_spans),
-                           block, 0, st, c);
+                           dim3(kThreads), 0, st, c);
     }
-    hipLaunchKernelGGL((ssm_chunk_kernel<NS, true>), grid, block, 0, st, c);
-    return (int)hipGetLastError();
+    return launch_chunk<NS, WAVES, true>(c, num_spans, st);
 }
 
 template <class T>
@@ -633,20 +690,17 @@ int portions(SsmArgs<T>& a, const Span* spans, int64_t num_spans, int64_t max_sp
     else hipLaunchKernelGGL((ssm_conv_kernel<T, 1, 0>), grid, block, 0, st, a, spans, xbc);
     if constexpr (sizeof(T) == 2) {
         if (chunked(INFER_ELEM_BF16, a.vdim, a.state_n) && vec && a.y_stride % 4 == 0 && ptr_aligned(a.y, 8)) {
-            ChunkArgs c{a, spans, 0, 0, (a.vdim + kSlab - 1) / kSlab, nullptr, nullptr};
-            int64_t seg_len, max_seg;
-            segments(a.heads, c.slabs, num_spans, max_span, seg_len, max_seg);
-            c.seg_len = (int)seg_len;
-            c.max_seg = (int)max_seg;
-            if (max_seg > 1) {
-                const int64_t records = num_spans * max_seg * a.heads, len = (int64_t)a.state_n * a.vdim;
+            const Walk walk = walk_of(a.heads, a.vdim, a.state_n, num_spans, max_span);
+            ChunkArgs c{a, spans, walk.seg_len, walk.max_seg, (a.vdim + kSlab - 1) / kSlab, nullptr, nullptr};
+            if (c.max_seg > 1) {
+                const int64_t records = num_spans * c.max_seg * a.heads, len = (int64_t)a.state_n * a.vdim;
                 if (!ws || ws_floats < records * (len + 1)) return INFER_KV_EWORKSPACE;
                 c.ws = ws;
                 c.ws_decay = ws + records * len;
             }
-            if (a.state_n <= 64) return launch_chunks<2>(c, num_spans, st);
-            if (a.state_n <= 128) return launch_chunks<4>(c, num_spans, st);
-            return launch_chunks<8>(c, num_spans, st);
+            if (a.state_n > 128) return launch_chunks<8, 4>(c, num_spans, st);
+            if (walk.waves == 8) return a.state_n <= 64 ? launch_chunks<2, 8>(c, num_spans, st) : launch_chunks<4, 8>(c, num_spans, st);
+            return a.state_n <= 64 ? launch_chunks<2, 4>(c, num_spans, st) : launch_chunks<4, 4>(c, num_spans, st);
         }
     }
     const dim3 sgrid((unsigned)((a.vdim + 15) / 16), (unsigned)a.heads, (unsigned)num_spans);
@@ -664,8 +718,7 @@ bool size_in(int64_t v, int64_t lo, int64_t hi) { return v >= lo && v <= hi; }
 extern "C" int64_t infer_state_space_workspace_floats(int elem, int64_t heads, int64_t vdim, int64_t state_n, int64_t num_spans,
                                                       int64_t max_span) {
     if (!chunked(elem, vdim, state_n) || heads < 1 || num_spans < 1 || max_span < 1) return 0;
-    int64_t seg_len, max_seg;
-    segments(heads, (vdim + kSlab - 1) / kSlab, num_spans, max_span, seg_len, max_seg);
+    const int64_t max_seg = walk_of(heads, vdim, state_n, num_spans, max_span).max_seg;
     return max_seg > 1 ? num_spans * max_seg * heads * (state_n * vdim + 1) : 0;
 }
 

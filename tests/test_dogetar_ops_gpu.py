@@ -433,6 +433,24 @@ def test_state_space_portions_are_cut_by_their_own_lengths(gpu, lens):
         close(m.state[i], want[i][1], 1e-2)
 
 
+@pytest.mark.parametrize("shape", [SSM[2], (4, 72, 48, 2, 4, 2)])
+def test_state_space_of_many_portions_and_of_a_long_one(gpu, shape):
+    """More workgroups than two per compute unit, and one portion of more than 4096 tokens, are walked by four wavefronts each instead of eight."""
+    many = 520 // (shape[0] * -(-shape[1] // 64)) + 1
+    m = Ssm(np.random.default_rng(many), shape, torch.bfloat16, slots=many, a_log=(-9.0, -5.0))
+    lens = [2 + (7 * i) % 70 for i in range(many)]
+    x = [m.inputs(n) for n in lens]
+    got = m.run([(i, 0, a) for i, a in enumerate(x)])
+    for i in range(many):
+        want, states = m.want(x[i])
+        close(torch.tensor(got[i]), want, 2e-2)
+        close(m.state[i], states, 1e-2)
+    x = m.inputs(4133)
+    want, states = m.want(x)
+    close(torch.tensor(np.concatenate(m.run([(3, 0, x)]))), want, 2e-2)
+    close(m.state[3], states, 1e-2)
+
+
 @BOTH
 @pytest.mark.parametrize("a_log,dt", [((4.0, 9.0), 3.0), ((-20.0, -12.0), 1.0), ((-1.0, 0.0), 12.0)])
 def test_state_space_extreme_decays(gpu, dtype, a_log, dt):
