@@ -22,6 +22,7 @@
 // pieces (2^-17).  Projections, with silu behind them or not, are bf16 already: one piece.
 // A portion with few heads is cut into segments that run side by side: first every segment from a zero state, keeping
 // only its final state, then the states are joined in order, then every segment with its outputs.
+#include <algorithm>
 #include <type_traits>
 
 #include "elem.h"
@@ -169,26 +170,33 @@ __device__ __forceinline__ int own_segment(int count, int most) {
     return segs > 1 ? ((count + segs - 1) / segs + kC - 1) / kC * kC : most;
 }
 
-// A workgroup of four wavefronts serves one head and 64 VT columns of its state over the chunks of one segment.
+// A workgroup of four or eight wavefronts serves one head and 16 VT columns of its state per wavefront over the chunks of one segment.
 // Wavefront w owns the columns 16 VT w .. and their part of the state, DT tiles of 32 rows, as accumulators: lane (g, n)
 // holds rows 16 t + 4 g + e of column n.  That is an operand of the next product as it lies, when the rows of a
-// k-step of 32 are taken in the order 16 tau + 4 g + e.  The 32 x 32 products q_i k_j are shared out over the
+// k-step of 32 are taken in the order 16 tau + 4 g + e.  The 32 x 32 products q_i k_j are shared out over four
 // wavefronts, weighted, and exchanged through LDS while the products with the state run.
-// PC: pieces of k (3 behind a rotation, otherwise 1; q then has 2).  OUT = false: only the final state, from zero.
-template <int DT, int VT, int PC, bool OUT>
-__global__ void __launch_bounds__(256, 2) decay_chunk_kernel(ChunkArgs args) {
+// PC: pieces of k (3 behind a rotation, otherwise 1; q then has 2).  OUT = false: only the final state, from zero.  FINISH: norm over the head and
+// gate, too.
+// A portion takes as long as its chunks one after the other, and a chunk as long as one wavefront's instructions.  Eight wavefronts have half as many
+// each, and with two chunks in LDS one barrier a chunk instead of three.
+__host__ __device__ constexpr int chunk_bufs(int waves) { return waves == 8 ? 2 : 1; }      // chunks in LDS
+
+template <int DT, int VT, int WAVES, int PC, bool OUT, bool FINISH>
+__global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs args) {
     constexpr int kRow = DT * 64 + 16, kMat = kC * kRow;         // bytes: a token of q or k, one piece of a chunk
-    constexpr int kSlab = 64 * VT;
+    constexpr int kThr = 64 * WAVES, kSlab = 16 * VT * WAVES;
+    constexpr int kBufs = chunk_bufs(WAVES);
     constexpr int PQ = PC == 3 ? 2 : 1;                          // pieces of q
     constexpr int kVRow = 2 * kSlab + 16, kPRow = 2 * kC + 16, kPMat = kC * kPRow;
-    constexpr int NU = DT > 4 ? DT / 4 : 1;                      // units of 16 columns of q and k per thread
+    constexpr int NU = (64 * DT + kThr - 1) / kThr;              // units of 16 columns of q and k per thread
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const DecayArgs<__bf16>& a = args.a;
+    constexpr int kBuf = (PC + (OUT ? PQ : 0)) * kMat + kC * kVRow;                      // of a chunk: k, v, q
     unsigned char* kbuf = lds;                                   // [PC][kMat]
     unsigned char* vbuf = kbuf + PC * kMat;                      // [kC][kVRow]
     unsigned char* qbuf = vbuf + kC * kVRow;                     // [PQ][kMat]
-    unsigned char* pbuf = qbuf + PQ * kMat;                      // [2][kPMat]
-    float* squares = reinterpret_cast<float*>(pbuf + 2 * kPMat); // [4][kC]
+    unsigned char* pbufs = lds + kBufs * kBuf;                   // [kBufs][2][kPMat], OUT
+    float* squares = reinterpret_cast<float*>(pbufs + kBufs * 2 * kPMat);                // [kBufs][WAVES][kC], OUT
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
@@ -226,7 +234,7 @@ __global__ void __launch_bounds__(256, 2) decay_chunk_kernel(ChunkArgs args) {
         }
 
     // entries behind the real sizes stay zero
-    for (int i = tid; i < ((PC + (OUT ? PQ : 0)) * kMat + kC * kVRow) / 16; i += 256) reinterpret_cast<u32x4_t*>(lds)[i] = u32x4_t{0u, 0u, 0u, 0u};
+    for (int i = tid; i < kBufs * kBuf / 16; i += kThr) reinterpret_cast<u32x4_t*>(lds)[i] = u32x4_t{0u, 0u, 0u, 0u};
 
     // unit i of this thread: token, and two blocks of 8 columns, which turn together if they are rotated
     // (token -1: there is no such unit; its loads repeat another one and are not stored)
@@ -236,7 +244,7 @@ __global__ void __launch_bounds__(256, 2) decay_chunk_kernel(ChunkArgs args) {
     const float* u_cs[NU];
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-        const int u = tid + 256 * i, w = u % units, rotated = half / 8;
+        const int u = tid + kThr * i, w = u % units, rotated = half / 8;
         u_tok[i] = u < kC * units ? u / units : -1;
         u_pair[i] = PC == 3 && w < rotated ? 8 * w : -1;
         u_b0[i] = w < rotated ? 8 * w : 2 * half + 16 * (w - rotated);
@@ -248,7 +256,7 @@ __global__ void __launch_bounds__(256, 2) decay_chunk_kernel(ChunkArgs args) {
     const __bf16* v_src[VT];
 #pragma unroll
     for (int i = 0; i < VT; ++i) {
-        const int x = tid + 256 * i;
+        const int x = tid + kThr * i;
         v_tok[i] = x / (kSlab / 8);
         v_col[i] = slab * kSlab + 8 * (x % (kSlab / 8));
         v_src[i] = a.proj + (int64_t)(row0 + v_tok[i]) * a.proj_stride + a.v_off + h * a.vdim + (v_col[i] < a.vdim ? v_col[i] : 0);
@@ -318,19 +326,19 @@ __global__ void __launch_bounds__(256, 2) decay_chunk_kernel(ChunkArgs args) {
         }
     };
     auto put = [&](int c) {
-        const int left = count - c * kC;
+        const int left = count - c * kC, at = c % kBufs * kBuf;
 #pragma unroll
         for (int i = 0; i < NU; ++i) {
             if (u_tok[i] < 0) continue;
-            put_unit(std::integral_constant<int, PC>{}, kbuf + u_tok[i] * kRow, i, kreg[i], u_tok[i] < left);
-            if constexpr (OUT) put_unit(std::integral_constant<int, PQ>{}, qbuf + u_tok[i] * kRow, i, qreg[i], u_tok[i] < left);
+            put_unit(std::integral_constant<int, PC>{}, kbuf + at + u_tok[i] * kRow, i, kreg[i], u_tok[i] < left);
+            if constexpr (OUT) put_unit(std::integral_constant<int, PQ>{}, qbuf + at + u_tok[i] * kRow, i, qreg[i], u_tok[i] < left);
         }
 #pragma unroll
         for (int i = 0; i < VT; ++i) {
             if (v_col[i] >= a.vdim) continue;
             u32x4_t y = a.silu ? silu8(vreg[i]) : vreg[i];
             if (v_tok[i] >= left) y = u32x4_t{0u, 0u, 0u, 0u};
-            *reinterpret_cast<u32x4_t*>(vbuf + v_tok[i] * kVRow + 2 * (v_col[i] - slab * kSlab)) = y;
+            *reinterpret_cast<u32x4_t*>(vbuf + at + v_tok[i] * kVRow + 2 * (v_col[i] - slab * kSlab)) = y;
         }
     };
 
@@ -363,181 +371,239 @@ __global__ void __launch_bounds__(256, 2) decay_chunk_kernel(ChunkArgs args) {
                 asm volatile("" : "+v"(x));
                 s[t][v][e] = x;
             }
-    fetch(0);
-    __syncthreads();                                             // the zero fill
-    for (int c = 0; c < chunks; ++c) {
-        put(c);
-        __syncthreads();
+    f32x4_t acc[VT][2], done[VT][2];                             // rows are columns of the state, columns queries
+    u32x2_t gate[VT][2];                                         // of results, requested a chunk before they are there
+    bf16x8_t vf[VT];                                             // values of tokens 8 g .. + 7, column n
+    // what the chunk's own tokens add to its results, and their squares
+    auto own_tokens = [&](int c) {
+        const unsigned char* pr = pbufs + c % kBufs * 2 * kPMat;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            bf16x8_t pf[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) pf[k] = *reinterpret_cast<const bf16x8_t*>(pr + k * kPMat + (16 * t + n) * kPRow + 16 * g);
+            float ss = 0.f;
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+#pragma unroll
+                for (int k = 1; k >= 0; --k) acc[v][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[v], pf[k], acc[v][t], 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ss += acc[v][t][e] * acc[v][t][e];       // columns that pad the size are zero
+                done[v][t] = acc[v][t];
+            }
+            if constexpr (FINISH) {
+                ss += __shfl_xor(ss, 16, 64);
+                ss += __shfl_xor(ss, 32, 64);
+                if (g == 0) squares[(c % kBufs * WAVES + wave) * kC + 16 * t + n] = ss;
+            }
+        }
+    };
+    auto request_gates = [&](int c) {
+#pragma unroll
+        for (int v = 0; v < VT; ++v)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int left = count - c * kC, tok = 16 * t + n < left ? 16 * t + n : left - 1, col = v0 + 16 * v + 4 * g;
+                gate[v][t] = *reinterpret_cast<const u32x2_t*>(args.b.gate + (int64_t)(row0 + c * kC + tok) * args.b.gate_stride +
+                                                               (int64_t)h * a.vdim + (col < a.vdim ? col : 0));
+            }
+    };
+    // results, with the norm over the head and the gate if nobody else does them
+    auto results = [&](int c) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if (16 * t + n >= count - c * kC) continue;
+            const int64_t row = row0 + c * kC + 16 * t + n;
+            float rs = 1.f;
+            if constexpr (FINISH) {
+                float ss = 0.f;
+#pragma unroll
+                for (int w = 0; w < WAVES; ++w) ss += squares[(c % kBufs * WAVES + w) * kC + 16 * t + n];
+                rs = rsqrtf(ss / (float)a.vdim + args.b.eps);
+            }
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+                const int col = v0 + 16 * v + 4 * g;
+                if (col >= a.vdim) continue;
+                float x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = done[v][t][e];
+                __bf16* o = a.o + row * a.o_stride + (int64_t)h * a.vdim + col;
+                if constexpr (FINISH) {
+                    const bf16x4_t z = __builtin_bit_cast(bf16x4_t, gate[v][t]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] *= rs * gate_of(args.b, (float)z[e]);
+                    if (args.b.norm)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[e] *= args.b.norm[h * a.vdim + col + e];
+                    o = args.b.out + row * args.b.out_stride + (int64_t)h * a.vdim + col;
+                }
+                store_elems<4>(o, x);
+            }
+        }
+    };
+    // products of the chunk's queries with its keys and with the state
+    auto queries = [&](int c) {
+        const unsigned char *kc = kbuf + c % kBufs * kBuf, *qc = qbuf + c % kBufs * kBuf;
+        // ---- d^(i-j) q_i k_j: rows are keys, columns queries; the tile above the diagonal is all zeros
+        if (wave < 4) {
+            f32x4_t p = {0.f, 0.f, 0.f, 0.f};
+            if (wave != 1) {
+                const unsigned char* kr = kc + (16 * (wave & 1) + n) * kRow + 16 * g;
+                const unsigned char* qr = qc + (16 * (wave >> 1) + n) * kRow + 16 * g;
+#pragma unroll
+                for (int j = 0; j < DT; ++j) {
+                    bf16x8_t kf[PQ], qf[PQ];
+#pragma unroll
+                    for (int k = 0; k < PQ; ++k) {
+                        kf[k] = *reinterpret_cast<const bf16x8_t*>(kr + k * kMat + 64 * j);
+                        qf[k] = *reinterpret_cast<const bf16x8_t*>(qr + k * kMat + 64 * j);
+                    }
+                    p = mfma_pieces<2>(kf, qf, p);
+                }
+            }
+            float x[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = p[e] * pw[e];
+            uint32_t pp[2][2];
+            split<2, 4>(x, pp);
+            unsigned char* pr = pbufs + c % kBufs * 2 * kPMat + (16 * (wave >> 1) + n) * kPRow + 2 * (16 * (wave & 1) + 4 * g);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) *reinterpret_cast<u32x2_t*>(pr + k * kPMat) = u32x2_t{pp[k][0], pp[k][1]};
+        }
+        // ---- q_i^T S
+#pragma unroll
+        for (int v = 0; v < VT; ++v)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) acc[v][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (live)
+#pragma unroll
+            for (int j = 0; j < DT; ++j) {
+                bf16x8_t qf[2][PQ];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int k = 0; k < PQ; ++k) {
+                        const unsigned char* qr = qc + k * kMat + (16 * t + n) * kRow + 64 * j + 8 * g;
+                        const u32x2_t x = *reinterpret_cast<const u32x2_t*>(qr), y = *reinterpret_cast<const u32x2_t*>(qr + 32);
+                        qf[t][k] = __builtin_bit_cast(bf16x8_t, u32x4_t{x[0], x[1], y[0], y[1]});
+                    }
+#pragma unroll
+                for (int v = 0; v < VT; ++v) {
+                    float x[8];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) { x[e] = s[2 * j][v][e]; x[4 + e] = s[2 * j + 1][v][e]; }
+                    bf16x8_t sf[2];
+                    split_frags<2>(x, sf);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) acc[v][t] = mfma_pieces<2>(sf, qf[t], acc[v][t]);
+                }
+            }
+        if (live)
+#pragma unroll
+            for (int v = 0; v < VT; ++v)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) acc[v][t] *= qw[t];
+    };
+    auto take_values = [&](int c) {
+        const unsigned char* vr = vbuf + c % kBufs * kBuf + (8 * g + (n >> 2)) * kVRow + (n & 3) * 8 + 32 * VT * wave;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vr + 32 * v));
+            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vr + 32 * v + 4 * kVRow));
+            vf[v] = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    };
+    auto update = [&](int c) {
+        const unsigned char* kc = kbuf + c % kBufs * kBuf;
         const int left = count - c * kC;
-        fetch(c + 1);
         if (left < kC) {
             value_weights(left);
             chunk_decay = exp2f(left * log2d);
         }
-        u32x2_t gate[VT][2];                                     // of this chunk's results, for when they are there
-        f32x4_t acc[VT][2];                                      // rows are columns of the state, columns queries
-        if constexpr (OUT) {
-            // ---- d^(i-j) q_i k_j: rows are keys, columns queries; the tile above the diagonal is all zeros
-            {
-                f32x4_t p = {0.f, 0.f, 0.f, 0.f};
-                if (wave != 1) {
-                    const unsigned char* kr = kbuf + (16 * (wave & 1) + n) * kRow + 16 * g;
-                    const unsigned char* qr = qbuf + (16 * (wave >> 1) + n) * kRow + 16 * g;
+        // ---- S <- d^n S + sum_j k_j (d^(n-1-j) v_j)^T
+        bf16x8_t wf[VT][3];
 #pragma unroll
-                    for (int j = 0; j < DT; ++j) {
-                        bf16x8_t kf[PQ], qf[PQ];
+        for (int v = 0; v < VT; ++v) {
+            float x[8];
+            widen(__builtin_bit_cast(u32x4_t, vf[v]), x);
 #pragma unroll
-                        for (int k = 0; k < PQ; ++k) {
-                            kf[k] = *reinterpret_cast<const bf16x8_t*>(kr + k * kMat + 64 * j);
-                            qf[k] = *reinterpret_cast<const bf16x8_t*>(qr + k * kMat + 64 * j);
-                        }
-                        p = mfma_pieces<2>(kf, qf, p);
-                    }
-                }
-                float x[4];
+            for (int i = 0; i < 8; ++i) x[i] *= vw[i];
+            split_frags<3>(x, wf[v]);
+        }
+        const unsigned char* kr = kc + (8 * g + (n >> 2)) * kRow + (n & 3) * 8;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = p[e] * pw[e];
-                uint32_t pp[2][2];
-                split<2, 4>(x, pp);
-                unsigned char* pr = pbuf + (16 * (wave >> 1) + n) * kPRow + 2 * (16 * (wave & 1) + 4 * g);
+        for (int t = 0; t < 2 * DT; ++t) {
+            bf16x8_t kf[PC];
 #pragma unroll
-                for (int k = 0; k < 2; ++k) *reinterpret_cast<u32x2_t*>(pr + k * kPMat) = u32x2_t{pp[k][0], pp[k][1]};
+            for (int k = 0; k < PC; ++k) {
+                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(kr + k * kMat + 32 * t));
+                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(kr + k * kMat + 32 * t + 4 * kRow));
+                kf[k] = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             }
-            // ---- q_i^T S
 #pragma unroll
-            for (int v = 0; v < VT; ++v)
-#pragma unroll
-                for (int t = 0; t < 2; ++t) acc[v][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            if (live)
-#pragma unroll
-                for (int j = 0; j < DT; ++j) {
-                    bf16x8_t qf[2][PQ];
-#pragma unroll
-                    for (int t = 0; t < 2; ++t)
-#pragma unroll
-                        for (int k = 0; k < PQ; ++k) {
-                            const unsigned char* qr = qbuf + k * kMat + (16 * t + n) * kRow + 64 * j + 8 * g;
-                            const u32x2_t x = *reinterpret_cast<const u32x2_t*>(qr), y = *reinterpret_cast<const u32x2_t*>(qr + 32);
-                            qf[t][k] = __builtin_bit_cast(bf16x8_t, u32x4_t{x[0], x[1], y[0], y[1]});
-                        }
-#pragma unroll
-                    for (int v = 0; v < VT; ++v) {
-                        float x[8];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) { x[e] = s[2 * j][v][e]; x[4 + e] = s[2 * j + 1][v][e]; }
-                        bf16x8_t sf[2];
-                        split_frags<2>(x, sf);
-#pragma unroll
-                        for (int t = 0; t < 2; ++t) acc[v][t] = mfma_pieces<2>(sf, qf[t], acc[v][t]);
-                    }
-                }
-            if (args.finish)
-#pragma unroll
-                for (int v = 0; v < VT; ++v)
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        const int tok = 16 * t + n < left ? 16 * t + n : left - 1, col = v0 + 16 * v + 4 * g;
-                        gate[v][t] = *reinterpret_cast<const u32x2_t*>(args.b.gate + (int64_t)(row0 + c * kC + tok) * args.b.gate_stride +
-                                                                       (int64_t)h * a.vdim + (col < a.vdim ? col : 0));
-                    }
+            for (int v = 0; v < VT; ++v) {
+                s[t][v] *= chunk_decay;
+                s[t][v] = mfma_pieces<3>(kf, wf[v], s[t][v]);
+            }
+        }
+    };
+    if (OUT && FINISH && !live && lane < kC)
+        for (int i = 0; i < kBufs; ++i) squares[(i * WAVES + wave) * kC + lane] = 0.f;
+    fetch(0);
+    __syncthreads();                                             // the zero fill
+    if constexpr (kBufs == 1) {
+        for (int c = 0; c < chunks; ++c) {
+            put(c);
             __syncthreads();
-        }
-        if (live) {
-            bf16x8_t vf[VT];                                     // values of tokens 8 g .. + 7, column n
-            const unsigned char* vr = vbuf + (8 * g + (n >> 2)) * kVRow + (n & 3) * 8 + 32 * VT * wave;
-#pragma unroll
-            for (int v = 0; v < VT; ++v) {
-                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vr + 32 * v));
-                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vr + 32 * v + 4 * kVRow));
-                vf[v] = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            }
+            fetch(c + 1);
             if constexpr (OUT) {
-                // ---- the chunk's own tokens
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    bf16x8_t pf[2];
-#pragma unroll
-                    for (int k = 0; k < 2; ++k) pf[k] = *reinterpret_cast<const bf16x8_t*>(pbuf + k * kPMat + (16 * t + n) * kPRow + 16 * g);
-                    float ss = 0.f;
-#pragma unroll
-                    for (int v = 0; v < VT; ++v) {
-                        acc[v][t] *= qw[t];
-#pragma unroll
-                        for (int k = 1; k >= 0; --k) acc[v][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[v], pf[k], acc[v][t], 0, 0, 0);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) ss += acc[v][t][e] * acc[v][t][e];       // columns that pad the size are zero
-                    }
-                    if (args.finish) {
-                        ss += __shfl_xor(ss, 16, 64);
-                        ss += __shfl_xor(ss, 32, 64);
-                        if (g == 0) squares[wave * kC + 16 * t + n] = ss;
-                    }
-                }
+                queries(c);
+                if constexpr (FINISH)
+                    if (live) request_gates(c);
+                __syncthreads();
             }
-            // ---- S <- d^n S + sum_j k_j (d^(n-1-j) v_j)^T
-            bf16x8_t wf[VT][3];
-#pragma unroll
-            for (int v = 0; v < VT; ++v) {
-                float x[8];
-                widen(__builtin_bit_cast(u32x4_t, vf[v]), x);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] *= vw[i];
-                split_frags<3>(x, wf[v]);
+            if (live) {
+                take_values(c);
+                if constexpr (OUT) own_tokens(c);
+                update(c);
             }
-            const unsigned char* kr = kbuf + (8 * g + (n >> 2)) * kRow + (n & 3) * 8;
-#pragma unroll
-            for (int t = 0; t < 2 * DT; ++t) {
-                bf16x8_t kf[PC];
-#pragma unroll
-                for (int k = 0; k < PC; ++k) {
-                    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(kr + k * kMat + 32 * t));
-                    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(kr + k * kMat + 32 * t + 4 * kRow));
-                    kf[k] = __builtin_bit_cast(bf16x8_t, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                }
-#pragma unroll
-                for (int v = 0; v < VT; ++v) {
-                    s[t][v] *= chunk_decay;
-                    s[t][v] = mfma_pieces<3>(kf, wf[v], s[t][v]);
-                }
-            }
-        } else if (OUT && args.finish && lane < kC) {
-            squares[wave * kC + lane] = 0.f;
+            __syncthreads();
+            if constexpr (OUT)
+                if (live) results(c);
         }
-        __syncthreads();
+    } else {
+        // Behind the barrier of chunk c: its q, k and v, the products of chunk c - 1's own tokens, which are used while this chunk's products
+        // run, and, where results wait for the other wavefronts' squares, those of chunk c - 2.  Everything that is written between two barriers
+        // was read last in front of the first.
+        auto behind = [&](int c) {
+            if (!OUT || !live) return;
+            if (FINISH && c > 1) results(c - 2);
+            if (c > 0) own_tokens(c - 1);
+            if (FINISH && c > 0) request_gates(c - 1);
+            if (!FINISH && c > 0) results(c - 1);
+        };
+        put(0);
+        fetch(1);
+#pragma unroll 1
+        for (int c = 0; c < chunks; ++c) {
+            __syncthreads();
+            behind(c);
+            if constexpr (OUT) queries(c);
+            if (live) {
+                take_values(c);
+                update(c);
+            }
+            if (c + 1 < chunks) {
+                put(c + 1);
+                fetch(c + 2);
+            }
+        }
         if constexpr (OUT) {
-            // ---- results, with the norm over the head and the gate if nobody else does them
-            if (live)
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    if (16 * t + n >= left) continue;
-                    const int64_t row = row0 + c * kC + 16 * t + n;
-                    float rs = 1.f;
-                    if (args.finish) {
-                        float ss = 0.f;
-#pragma unroll
-                        for (int w = 0; w < 4; ++w) ss += squares[w * kC + 16 * t + n];
-                        rs = rsqrtf(ss / (float)a.vdim + args.b.eps);
-                    }
-#pragma unroll
-                    for (int v = 0; v < VT; ++v) {
-                        const int col = v0 + 16 * v + 4 * g;
-                        if (col >= a.vdim) continue;
-                        float x[4];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) x[e] = acc[v][t][e];
-                        __bf16* o = a.o + row * a.o_stride + (int64_t)h * a.vdim + col;
-                        if (args.finish) {
-                            const bf16x4_t z = __builtin_bit_cast(bf16x4_t, gate[v][t]);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) x[e] *= rs * gate_of(args.b, (float)z[e]);
-                            if (args.b.norm)
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) x[e] *= args.b.norm[h * a.vdim + col + e];
-                            o = args.b.out + row * args.b.out_stride + (int64_t)h * a.vdim + col;
-                        }
-                        store_elems<4>(o, x);
-                    }
-                }
+            __syncthreads();
+            behind(chunks);
+            __syncthreads();
+            if (FINISH && live) results(chunks - 1);
         }
     }
     if (OUT && !last_seg) return;
@@ -782,54 +848,78 @@ int slabs_of(int64_t dim_pad, int64_t vdim_pad) {
     const int cols = 64 * column_tiles(dim_pad, vdim_pad);
     return (int)((vdim_pad + cols - 1) / cols);
 }
-// Most tokens of a segment: enough segments for two workgroups per compute unit, none shorter than four chunks; portions that fill the chip
-// with one workgroup per compute unit stay whole, since cut ones are walked twice.  Heads of 128 x 128, the call in us, cut / whole: 32 heads, 8
-// portions of 1500 tokens 252 / 212, 10 of 800 to 1800 297 / 273, 12 of 100 to 1500 284 / 241; 16 heads, 16 of 100 to 1500 209 / 179; but 32
-// heads, 6 of 900 to 3700 320 / 390; 16 heads, 10 of 800 to 1800 190 / 209.  Segments of one length per portion instead of one for the batch:
-// 6 portions of 900 to 3700 of 32 heads 338 -> 320, 5 of them 347 -> 298.
-int64_t segment_len(int64_t heads, int64_t slabs, int64_t num_spans, int64_t max_span) {
-    const int64_t groups = heads * slabs * num_spans;
-    int64_t n = groups >= 256 ? 1 : (512 + groups - 1) / groups;
-    const int64_t most = max_span / (4 * kC);
+// How portions are walked: wavefronts of a workgroup (eight_waves), and the most tokens of a segment.  Portions are cut where they do not fill the chip, into
+// no less than four chunks, since cut ones are walked twice.  Four wavefronts: below one workgroup per compute unit, into two of them; 32 heads of
+// 128 x 128, the call in us, cut / whole: 8 portions of 1500 tokens 252 / 212, 12 of 100 to 1500 284 / 241, but 6 of 900 to 3700 320 / 390.
+// Segments of one length per portion instead of one for the batch: 6 portions of 900 to 3700 of 32 heads 338 -> 320, 5 of them 347 -> 298.
+// Eight wavefronts with 16 columns each, two chunks in LDS, one workgroup per compute unit; four with 32 / eight, us: 32 heads, 10 portions of 800
+// to 1800 271 / 241, 8 of 1500 210 / 190, 6 of 900 to 3700 331 / 316, 20 of 300 to 900 222 / 205, 1 of 9000 207 / 196; 16 heads, 16 of 200 to 1000 120 / 98, 11
+// of 500 to 1500 160 / 137, 8 of 100 to 600 70 / 58, 1 of 300 43 / 35.  Where whole portions leave much of the chip idle and cut ones are long, four
+// are ahead (16 heads, 8 of 1000 to 3000 220 / 257; 32 heads, 4 of 1000 to 2500 185 / 210), and where there are many workgroups or they are little
+// but their start (32 heads, 64 of 100 to 300 227 / 243, 30 of 200 to 500 189 / 192, 16 of 50 to 250 59 / 61).  Behind a rotation, where a key
+// is three pieces, there is no room for two chunks, and eight are behind (32 heads, 6 of 900 to 3700 371 / 506).
+// Whole portions take as long as the longest of them: between half a workgroup and one per compute unit eight pay if there are tokens for some 110
+// workgroups of that length (6 of 200 to 4000, 100 of them, 315 / 319; 5 of 800 to 5000 350 / 395), or if it is short.
+bool eight_waves(int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t rot_dims, int64_t num_spans, int64_t max_span, int64_t tokens) {
+    const int64_t per_token = heads * slabs_of(dim_pad, vdim_pad), groups = per_token * num_spans;
+    if (column_tiles(dim_pad, vdim_pad) != 2 || rot_dims > 0 || groups > 640 || (groups > 384 && max_span <= 256)) return false;
+    if (groups <= 32 || groups >= 256) return true;
+    return groups < 160 ? max_span <= 640 : max_span <= 2048 || per_token * tokens >= 110 * max_span;
+}
+int64_t segment_len(bool wide, int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t num_spans, int64_t max_span) {
+    const int64_t groups = heads * slabs_of(dim_pad, vdim_pad) * num_spans, full = wide ? 128 : 256, most = max_span / (4 * kC);
+    int64_t n = groups >= full ? 1 : (2 * full + groups - 1) / groups;
     if (n > most) n = most;
-    if (n <= 1) return (max_span + kC - 1) / kC * kC;
+    if (n < 1) n = 1;
     return ((max_span + n - 1) / n + kC - 1) / kC * kC;
 }
 
-template <int DT, int VT, int PC, bool OUT>
+template <int DT, int VT, int WAVES, int PC, bool OUT, bool FINISH = false>
 int launch_chunk(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
-    const size_t lds = (size_t)kC * ((OUT ? PC == 3 ? 5 : 2 : PC) * (DT * 64 + 16) + 128 * VT + 16) + (OUT ? kC * (2 * (2 * kC + 16) + 16) : 0);
-    auto kernel = &decay_chunk_kernel<DT, VT, PC, OUT>;
+    const size_t lds = (size_t)kC * chunk_bufs(WAVES) * ((OUT ? PC == 3 ? 5 : 2 : PC) * (DT * 64 + 16) + 32 * VT * WAVES + 16 +
+                                     (OUT ? 2 * (2 * kC + 16) + WAVES * sizeof(float) : 0));
+    auto kernel = &decay_chunk_kernel<DT, VT, WAVES, PC, OUT, FINISH>;
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
     }
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(c.slabs * c.max_seg), (unsigned)c.a.heads, (unsigned)num_spans), dim3(256), lds, st, c);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(c.slabs * c.max_seg), (unsigned)c.a.heads, (unsigned)num_spans), dim3(64 * WAVES), lds, st, c);
     return (int)hipGetLastError();
 }
 
-template <int DT, int VT>
-int launch_chunks(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
-    const bool rot = c.a.rot_pairs > 0;
-    int rc;
+template <int DT, int VT, int WAVES, int PC>
+int launch_pieces(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
     if (c.max_seg > 1) {
-        rc = rot ? launch_chunk<DT, VT, 3, false>(c, num_spans, st) : launch_chunk<DT, VT, 1, false>(c, num_spans, st);
+        int rc = launch_chunk<DT, VT, WAVES, PC, false>(c, num_spans, st);
         if (rc) return rc;
         const unsigned blocks = (unsigned)(((int64_t)c.a.dim_pad * c.a.vdim_pad / 4 + kThreads - 1) / kThreads);
         hipLaunchKernelGGL(decay_join_kernel, dim3(blocks, (unsigned)c.a.heads, (unsigned)num_spans), dim3(kThreads), 0, st, c);
         rc = (int)hipGetLastError();
         if (rc) return rc;
     }
-    return rot ? launch_chunk<DT, VT, 3, true>(c, num_spans, st) : launch_chunk<DT, VT, 1, true>(c, num_spans, st);
+    return c.finish ? launch_chunk<DT, VT, WAVES, PC, true, true>(c, num_spans, st) : launch_chunk<DT, VT, WAVES, PC, true>(c, num_spans, st);
 }
 
-int run_chunks(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
-    const int vt = column_tiles(c.a.dim_pad, c.a.vdim_pad);
+template <int DT, int VT, int WAVES>
+int launch_chunks(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
+    if constexpr (WAVES == 4)
+        if (c.a.rot_pairs > 0) return launch_pieces<DT, VT, 4, 3>(c, num_spans, st);
+    return launch_pieces<DT, VT, WAVES, 1>(c, num_spans, st);
+}
+
+// Columns of a workgroup are those of slabs_of(): 64, or 128 as four wavefronts with 32 or eight with 16.
+template <int DT>
+int run_tiles(const ChunkArgs& c, int waves, int64_t num_spans, hipStream_t st) {
+    if (column_tiles(c.a.dim_pad, c.a.vdim_pad) == 1) return launch_chunks<DT, 1, 4>(c, num_spans, st);
+    return waves == 8 ? launch_chunks<DT, 1, 8>(c, num_spans, st) : launch_chunks<DT, 2, 4>(c, num_spans, st);
+}
+
+int run_chunks(const ChunkArgs& c, int waves, int64_t num_spans, hipStream_t st) {
     switch (tiles_of(c.a.dim_pad)) {
-        case 1: return vt == 1 ? launch_chunks<1, 1>(c, num_spans, st) : launch_chunks<1, 2>(c, num_spans, st);
-        case 2: return vt == 1 ? launch_chunks<2, 1>(c, num_spans, st) : launch_chunks<2, 2>(c, num_spans, st);
-        case 4: return vt == 1 ? launch_chunks<4, 1>(c, num_spans, st) : launch_chunks<4, 2>(c, num_spans, st);
-        default: return launch_chunks<8, 1>(c, num_spans, st);
+        case 1: return run_tiles<1>(c, waves, num_spans, st);
+        case 2: return run_tiles<2>(c, waves, num_spans, st);
+        case 4: return run_tiles<4>(c, waves, num_spans, st);
+        default: return launch_chunks<8, 1, 4>(c, num_spans, st);
     }
 }
 
@@ -866,7 +956,11 @@ extern "C" int64_t infer_decay_workspace_floats(int elem, int64_t heads, int64_t
                                                 int64_t max_span) {
     int64_t pad[2];
     if (infer_decay_layout(dim, vdim, pad) || heads < 1 || num_spans < 1 || max_span < 1 || !chunks_fit(elem, dim, vdim, rot_dims)) return 0;
-    const int64_t len = segment_len(heads, slabs_of(pad[0], pad[1]), num_spans, max_span), n = (max_span + len - 1) / len;
+    int64_t n = 1;                                             // for both ways to walk: how many tokens there are is not known here
+    for (const bool wide : {false, true}) {
+        const int64_t len = segment_len(wide, heads, pad[0], pad[1], num_spans, max_span);
+        n = std::max(n, (max_span + len - 1) / len);
+    }
     return n > 1 ? num_spans * n * heads * pad[0] * pad[1] : 0;
 }
 
@@ -918,12 +1012,13 @@ extern "C" int infer_decay_attention(int elem, const void* proj, int64_t proj_st
                           out_stride % 4 == 0 && ptr_aligned(out, 8) && ptr_aligned(table, 16);
                 if (chunked) {
                     const int slabs = slabs_of(pad[0], pad[1]);
-                    const int64_t len = segment_len(heads, slabs, num_spans, max_span), n = (max_span + len - 1) / len;
+                    const bool wide = eight_waves(heads, pad[0], pad[1], rot_dims, num_spans, max_span, rows - decode_rows);
+                    const int64_t len = segment_len(wide, heads, pad[0], pad[1], num_spans, max_span), n = (max_span + len - 1) / len;
                     if (n > 1 && (!workspace || !ptr_aligned(workspace, 16) || workspace_floats < num_spans * n * heads * pad[0] * pad[1]))
                         return (int)INFER_KV_EWORKSPACE;
                     // a workgroup that has the whole head norms it, too
                     const bool finish = norm_per_head && slabs == 1 && finished == decode_rows && ptr_aligned(proj, 8) && g_off % 4 == 0;
-                    rc = run_chunks(ChunkArgs{a, b, finish, (const Span*)spans, (int)len, (int)n, slabs, workspace}, num_spans, st);
+                    rc = run_chunks(ChunkArgs{a, b, finish, (const Span*)spans, (int)len, (int)n, slabs, workspace}, wide ? 8 : 4, num_spans, st);
                     if (finish) finished = rows;
                 }
             }

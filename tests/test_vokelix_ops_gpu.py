@@ -434,3 +434,25 @@ def test_decay_state_does_not_drift_over_many_steps(gpu, kind):
     for _ in range(4000):
         ho.decay_attention(d.shape, *args)
     d.check_state(state, 0, start * (np.array(d.decay) ** 4000)[:, None, None], 2e-5)
+
+
+@pytest.mark.parametrize("kind", ["lightning", "plain", "retention"])
+@pytest.mark.parametrize("vdim", [72, 128])
+@pytest.mark.parametrize("heads,lens", [(2, (1, 65, 1300, 31)), (12, (700, 33, 96)), (12, (600, 64, 257)), (20, (2, 32, 70, 33, 200, 9, 64, 63)),
+                                        (40, (1, 2, 31, 32, 33, 97, 64, 150, 5, 40, 66))])
+def test_decay_workgroups_of_four_and_of_eight_wavefronts(gpu, kind, vdim, heads, lens):
+    """Few workgroups, some, enough for the chip and many short ones, cut and whole, with columns that only some wavefronts have."""
+    bf = torch.bfloat16
+    d = Decay(kind, tuple(1.0 - 2.0 ** -(2 + i % 9) for i in range(heads)), 32, vdim, 32, bf, seed=heads + vdim)
+    x = rounded(d.inputs(sum(lens)), bf)
+    state, spans, row = d.state(len(lens)), [], 0
+    starts = [d.rng.standard_normal((heads, 32, vdim)) if i % 2 else np.zeros((heads, 32, vdim)) for i in range(len(lens))]
+    for i, n in enumerate(lens):
+        d.fill(state, i, starts[i])
+        spans.append((row, n, i, 7 * (i % 2)))
+        row += n
+    out = d.run(x, state, None, None, 0, spans)
+    for row, n, i, pos0 in spans:
+        want, end = d.want(x[row:row + n], pos0, starts[i], round_silu=True)
+        close(out[row:row + n], want, tol(bf, 1e-5))
+        d.check_state(state, i, end, state_tol(d, bf))
