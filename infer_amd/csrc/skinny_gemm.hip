@@ -189,7 +189,7 @@ __device__ __forceinline__ float round_bf16(float x) { return (float)(__bf16)x; 
 
 // Four sums of row `row` at the places 16 r + 4 g of a workgroup whose weights begin at row n0 (GATED: as described below)
 template <bool GATED>
-__device__ __forceinline__ void finish_tile(const GemmArgs& a, int split, int n0, int r, int row, int g, f32x4_t sum) {
+__device__ __forceinline__ void finish_tile(const GemmArgs& a, int half, int split, int n0, int r, int row, int g, f32x4_t sum) {
     if constexpr (GATED) {                         // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
         bf16x4_t v;
 #pragma unroll
@@ -198,7 +198,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& a, int split, int n0
             v[e] = (__bf16)(round_bf16(gate / (1.0f + expf(-gate))) * up);
         }
         const int col = n0 + 8 * r + 4 * g;
-        if (g < 2 && col < a.n / 2 && row < a.m) *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
+        if (g < 2 && col < half && row < a.m) *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
     } else {
         const int col = n0 + 16 * r + 4 * g;
         if (col >= a.n || row >= a.m) return;          // N is a multiple of 8: a quad is in or out as a whole
@@ -243,7 +243,7 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     stream_product<RT, MT, NW, D>(w, x, a.chunks * kKC, wave, lds + wave * kRing, acc);
-    stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, split, n0, r, 16 * t + n, g, sum); });
+    stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, half, split, n0, r, 16 * t + n, g, sum); });
 }
 
 // What stands in front of a product of few rows: y = norm(x + residual) w^T, where x may still be the pieces of a split product.
@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSourc
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     stream_product_held<RT, NW, D>(w, xs + (n < a.m ? n : a.m - 1) * row_bytes + 16 * g, a.k, wave, few_lds + wave * kRing, norm, acc);
-    stream_reduce<RT, 1, NW>(acc, wave, few_lds, [&](int r, int, f32x4_t sum) { finish_tile<GATED>(a, 0, n0, r, n, g, sum); });
+    stream_reduce<RT, 1, NW>(acc, wave, few_lds, [&](int r, int, f32x4_t sum) { finish_tile<GATED>(a, half, 0, n0, r, n, g, sum); });
 }
 
 struct ReduceArgs {
