@@ -339,14 +339,18 @@ int infer_rms_norm_splitk_bf16(const float* partial, int64_t splits, int64_t spl
 /* infer_kv_qk_norm_rope_append_bf16 and infer_paged_decode_bf16 behind it for a few new tokens, one of every sequence: q, k, v are rows as
  * projected and stay as they are; keys and values land in the (dense) caches at slot_mapping, and a sequence's last position, if that is its
  * slot, is taken from the new row.  No slot of a row may lie in the context of another.  infer_few_decode_workspace_bytes: 0 where the batch is not
- * served (max_tokens: what a row of the block table holds). */
+ * served (max_tokens: what a row of the block table holds).  product [hidden, num_q_heads * head_dim] (or null): `out` is null, and `sums` gets the
+ * unreduced product of what it would have held, as infer_skinny_gemm_partial_bf16 leaves it; infer_few_product_bytes: its bytes, 0 where this is
+ * not served. */
 size_t infer_few_decode_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_tokens);
+size_t infer_few_product_bytes(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t max_tokens, int64_t hidden);
 int infer_few_decode_front_bf16(const void* q, int64_t q_stride0, const void* k, int64_t k_stride0, const void* v, int64_t v_stride0,
                                 const int64_t* positions, const void* q_norm_weight, const void* k_norm_weight, float eps,
                                 const void* cos_sin_cache, int64_t max_position, void* k_cache, void* v_cache, const int32_t* slot_mapping,
                                 void* out, int64_t out_stride0, const int32_t* block_table, int64_t bt_stride0, int64_t table_cols,
                                 const int32_t* context_lens, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
-                                int64_t block_size, int64_t num_blocks, float scale, void* workspace, size_t workspace_bytes, void* stream);
+                                int64_t block_size, int64_t num_blocks, float scale, void* workspace, size_t workspace_bytes,
+                                const void* product, int64_t hidden, float* sums, size_t sums_bytes, void* stream);
 
 /* infer_rms_norm_bf16 (or, with `partial`, infer_rms_norm_splitk_bf16) and the product of its result in one launch, for few rows: the bits of
  * the two.  sum [m, k] = x + residual goes to a place of its own (residual may be null, then there is no sum).  gated: y [m, n / 2] as

@@ -59,7 +59,8 @@ SIGNATURES = {
     "infer_clamped_gate_and_mul": (_c.c_int, [_c.c_int, _vp, _i64, _vp, _i64, _i64, _i64, _f32, _vp]),
     "infer_few_decode_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "infer_few_decode_front_bf16": (_c.c_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _f32, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _i64,
-                                               _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _vp, _sz, _vp]),
+                                               _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _vp, _sz, _vp, _i64, _vp, _sz, _vp]),
+    "infer_few_product_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "infer_norm_product_supported": (_c.c_int, [_i64, _i64, _i64, _c.c_int]),
     "infer_norm_product_bf16": (_c.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _f32, _vp, _vp, _i64, _i64, _i64, _i64,
                                            _c.c_int, _vp]),

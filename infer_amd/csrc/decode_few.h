@@ -34,6 +34,25 @@ struct FewFront {
 // What a piece leaves: [group][128] unnormalised sums, then [group] (running maximum in the log2 domain, sum).
 __host__ __device__ inline int few_record_floats(int group) { return 130 * group + (group & 1 ? 2 : 0); }
 
+// Of the steps of 32 tokens that a sequence has, no more than `pieces` are somebody's first.
+__device__ __forceinline__ int few_pieces_of(const FewDecode& a, int len) {
+    len = len < a.max_ctx ? len : a.max_ctx;
+    const int steps = len > 0 ? (len + 31) / 32 : 0;
+    return steps < a.pieces ? steps : a.pieces;
+}
+typedef float few_f32x4 __attribute__((ext_vector_type(4)));
+// Adds sums `x` with (maximum, sum of weights) `o` to `num` with `s`.  The products are fused as written, so that all callers get the same bits.
+__device__ __forceinline__ void few_add(few_f32x4& num, float2& s, few_f32x4 x, float2 o) {
+    const float top = fmaxf(s.x, o.x), f1 = s.x == top ? 1.f : __builtin_amdgcn_exp2f(s.x - top), f2 = o.x == top ? 1.f : __builtin_amdgcn_exp2f(o.x - top);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) num[e] = __builtin_fmaf(num[e], f1, x[e] * f2);
+    s = make_float2(top, __builtin_fmaf(s.y, f1, o.y * f2));
+}
+
 // Pieces per (sequence, KV head), or 0 where the batch is not small.
 int few_decode_pieces(int64_t batch, int64_t num_kv_heads, int64_t max_tokens);
-int launch_few_decode(const FewDecode& a, hipStream_t stream, const FewFront* front = nullptr);      // records, then their sum in `out`
+int launch_few_decode(const FewDecode& a, hipStream_t stream, const FewFront* front = nullptr);      // records, then their sum in `out`, if there is one
+
+// A product behind the pieces (skinny_gemm.hip): `hidden` rows of weights, float32 sums [splits][hidden].
+int few_product_splits(int64_t batch, int64_t num_q_heads, int64_t pieces, int64_t hidden);
+int launch_few_product(const FewDecode& f, const void* w, int64_t hidden, float* sums, int splits, hipStream_t stream);

@@ -320,28 +320,20 @@ __global__ void __launch_bounds__(256) few_decode_sum_kernel(FewDecode a) {
         v[i] = *reinterpret_cast<const f32x4*>(from + n * kD + 4 * c);
         ml[i] = *reinterpret_cast<const float2*>(from + G * kD + 2 * n);
     }
-    int len = a.ctx[b];
-    len = len < a.max_ctx ? len : a.max_ctx;
-    const int steps = len > 0 ? (len + kStep - 1) / kStep : 0, pieces = steps < a.pieces ? steps : a.pieces;
+    const int pieces = few_pieces_of(a, a.ctx[b]);
     f32x4 num = {0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, den = 0.f;
-    auto add = [&](f32x4 x, float2 o) {
-        const float top = fmaxf(m, o.x), f1 = m == top ? 1.f : __builtin_amdgcn_exp2f(m - top), f2 = o.x == top ? 1.f : __builtin_amdgcn_exp2f(o.x - top);
-        num = num * f1 + x * f2;
-        den = den * f1 + o.y * f2;
-        m = top;
-    };
+    float2 s = make_float2(-INFINITY, 0.f);
 #pragma unroll
     for (int i = 0; i < N; ++i)
-        if (part + 8 * i < pieces) add(v[i], ml[i]);
+        if (part + 8 * i < pieces) few_add(num, s, v[i], ml[i]);
     if (part > 0) {
         sums[part - 1][c] = num;
-        if (c == 0) mls[part - 1] = make_float2(m, den);
+        if (c == 0) mls[part - 1] = s;
     }
     __syncthreads();
     if (part > 0) return;
-    for (int w = 1; w < 8 && w < pieces; ++w) add(sums[w - 1][c], mls[w - 1]);
-    const float inv = den > 0.f ? 1.f / den : 0.f;
+    for (int w = 1; w < 8 && w < pieces; ++w) few_add(num, s, sums[w - 1][c], mls[w - 1]);
+    const float inv = s.y > 0.f ? 1.f / s.y : 0.f;
     bf16x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = (__bf16)(num[e] * inv);
@@ -369,7 +361,7 @@ int launch_few_decode(const FewDecode& a, hipStream_t stream, const FewFront* fr
     if (front) hipLaunchKernelGGL(few_decode_kernel<true>, pieces, dim3(64 * kWaves), 0, stream, a, *front);
     else hipLaunchKernelGGL(few_decode_kernel<false>, pieces, dim3(64 * kWaves), 0, stream, a, FewFront{});
     const int rc = (int)hipGetLastError();
-    if (rc) return rc;
+    if (rc || !a.out) return rc;
     const dim3 grid((unsigned)(a.group * a.num_kv_heads), (unsigned)a.batch), block(256);
     if (a.pieces <= 32) hipLaunchKernelGGL(few_decode_sum_kernel<4>, grid, block, 0, stream, a);
     else hipLaunchKernelGGL(few_decode_sum_kernel<8>, grid, block, 0, stream, a);

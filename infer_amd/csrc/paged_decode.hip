@@ -1281,30 +1281,40 @@ size_t infer_few_decode_workspace_bytes(int64_t batch, int64_t num_q_heads, int6
     return (size_t)batch * num_kv_heads * pieces * few_record_floats((int)(num_q_heads / num_kv_heads)) * sizeof(float);
 }
 
+size_t infer_few_product_bytes(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t max_tokens, int64_t hidden) {
+    return sizeof(float) * (size_t)(hidden > 0 ? hidden : 0) * few_product_splits(batch, num_q_heads, few_decode_pieces(batch, num_kv_heads, max_tokens), hidden);
+}
+
 int infer_few_decode_front_bf16(const void* q, int64_t q_stride0, const void* k, int64_t k_stride0, const void* v, int64_t v_stride0,
                                 const int64_t* positions, const void* q_norm_weight, const void* k_norm_weight, float eps,
                                 const void* cos_sin_cache, int64_t max_position, void* k_cache, void* v_cache, const int32_t* slot_mapping,
                                 void* out, int64_t out_stride0, const int32_t* block_table, int64_t bt_stride0, int64_t table_cols,
                                 const int32_t* context_lens, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
-                                int64_t block_size, int64_t num_blocks, float scale, void* workspace, size_t workspace_bytes, void* stream) {
+                                int64_t block_size, int64_t num_blocks, float scale, void* workspace, size_t workspace_bytes,
+                                const void* product, int64_t hidden, float* sums, size_t sums_bytes, void* stream) {
     const int64_t token = num_kv_heads * head_dim;
     const DecodeCall c{q, q_stride0, k_cache, v_cache, block_size * token, token, block_table, bt_stride0, table_cols, context_lens, batch,
                        num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, scale};
     if (!context_lens || !k || !v || !positions || !q_norm_weight || !k_norm_weight || !cos_sin_cache || !slot_mapping || max_position <= 0) return INFER_KV_EINVAL;
     int rc = check_split(c, 0, workspace);
     if (rc) return rc;
-    rc = check_out(out, out_stride0, num_q_heads);
+    if (!product) rc = check_out(out, out_stride0, num_q_heads);
+    else if (out || !sums) rc = INFER_KV_EINVAL;
+    else if (((uintptr_t)product | (uintptr_t)sums) & 15) rc = INFER_KV_EALIGN;
     if (rc) return rc;
     if (k_stride0 < token || v_stride0 < token || q_stride0 < num_q_heads * head_dim) return INFER_KV_EINVAL;
     if ((((uintptr_t)k | (uintptr_t)v | (uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight | (uintptr_t)cos_sin_cache) & 15) || ((k_stride0 | v_stride0) & 7))
         return INFER_KV_EALIGN;
     FewDecode a;
     if (!few_args(c, workspace, out, out_stride0, &a)) return INFER_KV_EUNSUPPORTED;
-    if (few_bytes(a) > workspace_bytes) return INFER_KV_EWORKSPACE;
+    const int splits = product ? few_product_splits(batch, num_q_heads, a.pieces, hidden) : 0;
+    if (product && !splits) return INFER_KV_EUNSUPPORTED;
+    if (few_bytes(a) > workspace_bytes || sizeof(float) * (size_t)hidden * splits > sums_bytes) return INFER_KV_EWORKSPACE;
     const FewFront f{(const uint16_t*)k, k_stride0, (const uint16_t*)v, v_stride0, positions, (const uint16_t*)q_norm_weight,
                      (const uint16_t*)k_norm_weight, (const uint16_t*)cos_sin_cache, max_position, (uint16_t*)k_cache, (uint16_t*)v_cache,
                      slot_mapping, num_blocks * block_size, eps};
-    return launch_few_decode(a, (hipStream_t)stream, &f);
+    rc = launch_few_decode(a, (hipStream_t)stream, &f);
+    return rc || !product ? rc : launch_few_product(a, product, hidden, sums, splits, (hipStream_t)stream);
 }
 
 }  // extern "C"

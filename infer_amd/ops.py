@@ -120,10 +120,12 @@ def qk_norm_rope_store_kvcache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
 
 def few_decode_with_front(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, positions: torch.Tensor, q_norm_weight: torch.Tensor,
                           k_norm_weight: torch.Tensor, eps: float, cos_sin_cache: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
-                          slot_mapping: torch.Tensor, block_table: torch.Tensor, context_lens: torch.Tensor, scale: float) -> torch.Tensor | None:
+                          slot_mapping: torch.Tensor, block_table: torch.Tensor, context_lens: torch.Tensor, scale: float,
+                          product: torch.Tensor | None = None):
     """``qk_norm_rope_store_kvcache`` and decode attention behind it, of one new token of each of a few sequences, or ``None`` where the
     batch is not small.  The rows stay as they are; the caches get what they would get.  A sequence's last position is its row's slot, and
-    no row's slot lies in the context of another row."""
+    no row's slot lies in the context of another row.  ``product``: the weight of the bare projection behind it.  Where the kernels take that in, too,
+    the result is its sums in pieces (``SplitKSum``, the bits of ``linear(result, product, defer=True)``)."""
     n, hq, d = q.shape
     nblk, bs, hkv, _ = k_cache.shape
     if context_lens is None or block_table is None or n == 0 or block_table.shape[0] != n or block_table.shape[1] < 1 or bs % 32:
@@ -146,14 +148,23 @@ def few_decode_with_front(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos
     assert k_cache.shape == v_cache.shape and k_cache.is_contiguous() and v_cache.is_contiguous()
     _require_gpu(q, k, v, positions, q_norm_weight, k_norm_weight, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, context_lens)
     pieces = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-    out = torch.empty((n, hq, d), dtype=q.dtype, device=q.device)
+    behind, out, sums = (None, 0, None, 0), None, None
+    if product is not None and _linear_mode() == "static" and product.shape[1] == hq * d and _streamable(q.view(n, hq * d) if n == 1 else q, product):
+        hidden = product.shape[0]
+        need = _lib.load().infer_few_product_bytes(n, hq, hkv, block_table.shape[1] * bs, hidden)
+        if need and _own_kernel(n, hidden, hq * d, True):
+            ws = _gemm_workspace(q.device, need)
+            behind, sums = (product.data_ptr(), hidden, ws.data_ptr(), need), ws[:need].view(torch.float32).view(-1, n, hidden)
+    if sums is None:
+        out = torch.empty((n, hq, d), dtype=q.dtype, device=q.device)
+    to = (None, 0) if out is None else (out.data_ptr(), out.stride(0))
     rc = _lib.load().infer_few_decode_front_bf16(
         q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), positions.data_ptr(), q_norm_weight.data_ptr(),
         k_norm_weight.data_ptr(), float(eps), cos_sin_cache.data_ptr(), cos_sin_cache.shape[0], k_cache.data_ptr(), v_cache.data_ptr(),
-        slot_mapping.data_ptr(), out.data_ptr(), out.stride(0), block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
-        context_lens.data_ptr(), n, hq, hkv, d, bs, nblk, float(scale), pieces.data_ptr(), nbytes, _stream_ptr(q))
+        slot_mapping.data_ptr(), *to, block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
+        context_lens.data_ptr(), n, hq, hkv, d, bs, nblk, float(scale), pieces.data_ptr(), nbytes, *behind, _stream_ptr(q))
     _lib.check(rc, "few_decode_with_front")
-    return out
+    return out if sums is None else SplitKSum(sums, q.dtype)
 
 
 def decode_workspace(device, max_batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int) -> torch.Tensor:

@@ -71,7 +71,10 @@ class QwenAttention(nn.Module):
         if bound and not context.is_prefill and is_bare_norm(self.q_norm) and is_bare_norm(self.k_norm) and is_bare_attention(self.attn):
             # a few sequences: norms, rotary positions and append in the launch of the attention
             o = ops.few_decode_with_front(q, k, v, positions, self.q_norm.weight, self.k_norm.weight, self.q_norm.eps, table, k_cache, v_cache, slots,
-                                          context.block_tables, context.context_lens, self.attn.scale)
+                                          context.block_tables, context.context_lens, self.attn.scale,
+                                          self.o_proj.weight if type(self.o_proj) is Linear and _is_bare(self.o_proj, Linear) else None)
+            if isinstance(o, ops.SplitKSum):
+                return o
             if o is not None:
                 return self.o_proj(o.view(-1, self.q_size), defer=True)
         ops.qk_norm_rope_store_kvcache(q, k, v, positions, self.q_norm.weight, self.k_norm.weight,

@@ -146,6 +146,45 @@ def test_with_the_front_as_in_two_launches(gpu, lens, hq, hkv, block):
     assert torch.isfinite(out.float()).all() and torch.equal(out, want)
 
 
+@pytest.mark.parametrize("length,hq,hkv,hidden", [(0, 16, 8, 1024), (1, 16, 8, 1024), (33, 16, 8, 1024), (260, 16, 8, 1000), (4097, 16, 8, 520),
+                                                  (700, 32, 8, 512), (9000, 32, 16, 248), (300, 24, 8, 768), (300, 12, 12, 744), (64, 16, 8, 4096), (64, 4, 1, 512),
+                                                  (700, 16, 8, 1024), (1024, 16, 8, 1024), (230, 16, 8, 1024)])
+def test_with_the_product_behind_it(gpu, length, hq, hkv, hidden):
+    """The pieces of a sequence's attention added up by the product's workgroups: the bits of attention and split product, again in replays of
+    a graph; not where a workgroup would have more than four heads, there are more workgroups than compute units, or pieces are many."""
+    gen = torch.Generator().manual_seed(length + hidden)
+    _, k, v, table, ctx = _inputs(gen, [length], hq, hkv, 256)
+    slots = torch.tensor([int(table[0, (length - 1) // 256]) * 256 + (length - 1) % 256 if length else -1], dtype=torch.int32).cuda()
+    qkv = (3 * torch.randn(1, (hq + 2 * hkv) * 128, generator=gen)).to(BF16).cuda()
+    q, kn, vn = (t.view(1, -1, 128) for t in qkv.split([hq * 128, hkv * 128, hkv * 128], -1))
+    wq, wk = ((1 + 0.3 * torch.randn(128, generator=gen)).to(BF16).cuda() for _ in range(2))
+    cs, positions = torch.randn(length + 9, 128, generator=gen).to(BF16).cuda(), torch.tensor([max(length - 1, 0)]).cuda()
+    weight = (0.02 * torch.randn(hidden, hq * 128, generator=gen)).to(BF16).cuda()
+    args = q, kn, vn, positions, wq, wk, 1e-6, cs, k, v, slots, table, ctx, 0.09
+    out = ops.few_decode_with_front(*args)
+    want = ops.linear(out.view(1, -1), weight, defer=True)
+    if isinstance(want, ops.SplitKSum):
+        splits, want = want.partial.shape[0], want.materialize()
+    else:
+        splits = 1
+    got = ops.few_decode_with_front(*args, weight)
+    if splits == 1 or hq // splits > 4 or hkv < 8 or -(-hidden // 16) * splits > 256:
+        assert torch.equal(got, out)
+        return
+    assert isinstance(got, ops.SplitKSum) and got.partial.shape == (splits, 1, hidden)
+    assert torch.equal(got.materialize(), want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.few_decode_with_front(*args, weight).materialize()
+    for _ in range(3):
+        got.fill_(float("nan"))
+        graph.replay()
+        ops.few_decode_with_front(*args, weight)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
 def test_batches_that_are_not_small_are_left_alone(gpu):
     gen = torch.Generator().manual_seed(9)
     q, k, v, table, ctx = _inputs(gen, [64] * 9, 16, 8, 256)
