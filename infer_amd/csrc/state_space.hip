@@ -632,12 +632,14 @@ bool chunked(int elem, int64_t vdim, int64_t state_n) { return elem == INFER_ELE
 // of four per compute unit.  Heads of 128 x 64, the call in us, four wavefronts cut for three workgroups per compute unit / eight cut for
 // two: 6 portions of 900 to 3700 tokens of 64 heads 325 / 286, 5 of 1000 to 3000 248 / 211, 8 of 1000 174 / 158, 4 of 500 to 4000 252 / 245, 11 of
 // 500 to 1500 of 32 heads 185 / 158, 1 of 300 40 / 36.  Two workgroups of eight fit a compute unit; where there are more, four are ahead
-// (10 of 800 to 1800 of 64 heads 250 / 256), and with a long portion by itself, cut into equal segments (9000 of 64 heads 217 / 222).
+// (10 of 800 to 1800 of 64 heads 250 / 256), and with a long portion by itself, cut into equal segments: what the chip has to do in all
+// counts there, not the longest chain.  1 of 3500 / 4319 / 6000 / 9000 / 13900, four / eight: 64 heads 105 / 101, 122.2 / 119.6, 154.4 / 157.1,
+// 216 / 221, 311 / 322; 32 heads 75.2 / 71.0, 87.8 / 82.8, 100.1 / 97.1, 131.4 / 131.4, 203 / 202.
 // Segments of one length per portion instead of one for the batch: 6 portions of 32 heads 228 -> 220.
 struct Walk { int waves, seg_len, max_seg; };
 Walk walk_of(int64_t heads, int64_t vdim, int64_t state_n, int64_t num_spans, int64_t max_span) {
     const int64_t units = heads * ((vdim + kSlab - 1) / kSlab) * num_spans, chunks = (max_span + kC - 1) / kC;
-    const bool wide = units <= 512 && state_n <= 128 && !(num_spans == 1 && max_span >= 4096);
+    const bool wide = units <= 512 && state_n <= 128 && !(num_spans == 1 && units * max_span > 64 * 5000);
     const int64_t full = wide ? 256 : 384;
     int64_t want = units > 0 && units < full ? (2 * full + units - 1) / units : 1;
     if (want > chunks / 4) want = chunks / 4;              // no segment shorter than four chunks
