@@ -336,12 +336,12 @@ int infer_rms_norm_splitk_bf16(const float* partial, int64_t splits, int64_t spl
                                const void* weight, void* out, int64_t out_stride0,
                                int64_t n_rows, int64_t hidden, float eps, void* stream);
 
-/* infer_kv_qk_norm_rope_append_bf16 and infer_paged_decode_bf16 behind it for a few new tokens, one of every sequence: q, k, v are rows as
- * projected and stay as they are; keys and values land in the (dense) caches at slot_mapping, and a sequence's last position, if that is its
- * slot, is taken from the new row.  No slot of a row may lie in the context of another.  infer_few_decode_workspace_bytes: 0 where the batch is not
- * served (max_tokens: what a row of the block table holds).  product [hidden, num_q_heads * head_dim] (or null): `out` is null, and `sums` gets the
- * unreduced product of what it would have held, as infer_skinny_gemm_partial_bf16 leaves it; infer_few_product_bytes: its bytes, 0 where this is
- * not served. */
+/* infer_kv_qk_norm_rope_append_bf16 and infer_paged_decode_bf16 behind it for a few new tokens, one of every row: q, k, v are rows as projected
+ * and stay as they are; keys and values land in the (dense) caches at slot_mapping, and every row whose context holds the slot of a new token, of
+ * whichever row, attends to that token, as behind an append in a launch of its own (two rows with one slot: to either).
+ * infer_few_decode_workspace_bytes: 0 where the batch is not served (max_tokens: what a row of the block table holds).  product [hidden,
+ * num_q_heads * head_dim] (or null): `out` is null, and `sums` gets the unreduced product of what it would have held, as
+ * infer_skinny_gemm_partial_bf16 leaves it; infer_few_product_bytes: its bytes, 0 where this is not served. */
 size_t infer_few_decode_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_tokens);
 size_t infer_few_product_bytes(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t max_tokens, int64_t hidden);
 int infer_few_decode_front_bf16(const void* q, int64_t q_stride0, const void* k, int64_t k_stride0, const void* v, int64_t v_stride0,

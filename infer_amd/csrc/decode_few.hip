@@ -67,7 +67,9 @@ __device__ __forceinline__ u32x4 norm_and_rotate(u32x4 x, u32x4 w, u32x4 c, u32x
 // FRONT: queries and new keys are as projected, and nothing of the new tokens is in the caches yet.  Every wavefront with a step norms and
 // rotates the queries that it uses, four heads at once, while its keys and values are on their way; the one with a sequence's last step does
 // so with the new key, takes key and value from its registers, since what it has requested is older, and puts them into the caches at its
-// end, where nothing waits for the stores.  us, 16 heads on 8, front and attention in launches of their own / this: 1 x 700 tokens 9.7 / 8.1,
+// end, where nothing waits for the stores.  Nobody waits for those stores either: a step that holds the slot of another new token (two rows of
+// one sequence, say), or its own in the middle, takes that row's key and value from the row, normed and rotated on the spot, whatever the caches
+// hold there by then.  us, 16 heads on 8, front and attention in launches of their own / this: 1 x 700 tokens 9.7 / 8.1,
 // 4 x 700 12.4 / 11.2, 8 x 700 16.2 / 15.4; 32 heads 10.2 / 8.2, 12.8 / 11.9, 16.9 / 16.5; a step of a 0.6B model with one sequence 820 -> 778.
 // (With the stores in front of the products, with front loads of wavefronts without a step, or with heads spread as operands are, it gained nothing.)
 template <bool FRONT>
@@ -93,10 +95,14 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a, Fe
         for (int j = 0; j < 4; ++j) q[j] = load16(qp + 32 * j);
     }
     int64_t slot = -1, pos = 0;
+    int row_slot = -1;                             // lane r: that of row r (a batch has no more than 64)
+    auto position_of = [&](int row) {
+        const int64_t at = f.positions[row];
+        return at < 0 ? 0 : at >= f.max_position ? f.max_position - 1 : at;
+    };
     if constexpr (FRONT) {
         slot = f.slots[b];
-        pos = f.positions[b];
-        pos = pos < 0 ? 0 : pos >= f.max_position ? f.max_position - 1 : pos;
+        pos = position_of(b);
     }
     // Heads 4 i .. 4 i + 3 of the group's queries with the new key behind them, 16 lanes each
     u32x4 x[2], w[2], cs, sn, kn[4], vn;
@@ -107,6 +113,7 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a, Fe
         wi = load16((query ? f.q_weight : f.k_weight) + 8 * n);
     };
     auto load_front = [&](bool two) {
+        row_slot = f.slots[lane < a.batch ? lane : b];
         cs = load16(f.cos_sin + pos * kD + 8 * (n & 7));
         sn = load16(f.cos_sin + pos * kD + 64 + 8 * (n & 7));
         vn = load16(f.v + (int64_t)b * f.v_stride0 + h * kD + 8 * n);
@@ -129,6 +136,19 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a, Fe
             q[j] = *reinterpret_cast<const u32x4*>(lds + (n < G ? n : 0) * kHead + 64 * j + 16 * g);
             kn[j] = *reinterpret_cast<const u32x4*>(lds + G * kHead + 64 * j + 16 * g);      // of the wavefront that needs it
         }
+        lds_order();
+    };
+    // Key and value of row r as its own wavefront appends them
+    auto new_row = [&](int r, u32x4 (&kr)[4], u32x4& vr) {
+        const uint16_t* turn = f.cos_sin + position_of(r) * kD + 8 * (n & 7);
+        u32x4 s = load16(turn + 64);
+        if (n < 8) s ^= u32x4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+        const u32x4 xr = norm_and_rotate(load16(f.k + (int64_t)r * f.k_stride0 + h * kD + 8 * n), load16(f.k_weight + 8 * n), load16(turn), s, f.eps);
+        vr = load16(f.v + (int64_t)r * f.v_stride0 + h * kD + 8 * n);
+        if (g == 0) *reinterpret_cast<u32x4*>(lds + 16 * n) = xr;
+        lds_order();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) kr[j] = *reinterpret_cast<const u32x4*>(lds + 64 * j + 16 * g);
         lds_order();
     };
     auto append = [&] {
@@ -191,18 +211,25 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a, Fe
         for (int j = 0; j < 4; ++j) q[j] = u32x4{0u, 0u, 0u, 0u};
     for (int step = first; step < steps; step += stride) {
         if constexpr (FRONT) {
-            if (step == steps - 1) {
-                const int i = len - 1 - step * kStep;      // the new token's place in the step, if the cache has it there
-                if (row0 + i == slot) {
+            auto put_row = [&](int i, const u32x4 (&kr)[4], u32x4 vr) {      // as token i of the step
 #pragma unroll
-                    for (int t = 0; t < 2; ++t)
-                        if (8 * (n >> 2) + (n & 3) + 4 * t == i)
+                for (int t = 0; t < 2; ++t)
+                    if (8 * (n >> 2) + (n & 3) + 4 * t == i)
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) k[t][j] = kn[j];
+                        for (int j = 0; j < 4; ++j) k[t][j] = kr[j];
 #pragma unroll
-                    for (int t = 0; t < 8; ++t)
-                        if (4 * t + g == i) v[t] = vn;
-                }
+                for (int t = 0; t < 8; ++t)
+                    if (4 * t + g == i) v[t] = vr;
+            };
+            const bool own = newest && (uint64_t)(slot - row0) < kStep;
+            if (own) put_row((int)(slot - row0), kn, vn);
+            uint64_t others = __ballot(lane < a.batch && (uint64_t)(row_slot - row0) < kStep && !(own && lane == b));
+            while (__builtin_expect(others != 0, 0)) {
+                const int r = __builtin_ctzll(others);
+                others &= others - 1;
+                u32x4 kr[4], vr;
+                new_row(r, kr, vr);
+                put_row((int)(__builtin_amdgcn_readlane(row_slot, r) - row0), kr, vr);
             }
         }
         f32x4 s[2];

@@ -123,9 +123,9 @@ def few_decode_with_front(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos
                           slot_mapping: torch.Tensor, block_table: torch.Tensor, context_lens: torch.Tensor, scale: float,
                           product: torch.Tensor | None = None):
     """``qk_norm_rope_store_kvcache`` and decode attention behind it, of one new token of each of a few sequences, or ``None`` where the
-    batch is not small.  The rows stay as they are; the caches get what they would get.  A sequence's last position is its row's slot, and
-    no row's slot lies in the context of another row.  ``product``: the weight of the bare projection behind it.  Where the kernels take that in, too,
-    the result is its sums in pieces (``SplitKSum``, the bits of ``linear(result, product, defer=True)``)."""
+    batch is not small.  The rows stay as they are; the caches get what they would get, and rows may see each other's tokens (two rows of one
+    sequence).  ``product``: the weight of the bare projection behind it.  Where the kernels take that in, too, the result is its sums in
+    pieces (``SplitKSum``, the bits of ``linear(result, product, defer=True)``)."""
     n, hq, d = q.shape
     nblk, bs, hkv, _ = k_cache.shape
     if context_lens is None or block_table is None or n == 0 or block_table.shape[0] != n or block_table.shape[1] < 1 or bs % 32:

@@ -146,6 +146,41 @@ def test_with_the_front_as_in_two_launches(gpu, lens, hq, hkv, block):
     assert torch.isfinite(out.float()).all() and torch.equal(out, want)
 
 
+@pytest.mark.parametrize("rows,hq,hkv,block", [
+    ([(0, 33), (0, 34)], 16, 8, 256), ([(0, 32), (0, 33)], 16, 8, 256), ([(0, 1), (0, 2), (0, 3)], 5, 5, 32), ([(0, 700 + i) for i in range(6)], 32, 8, 64),
+    ([(0, 66), (1, 40), (0, 65), (1, 41), (0, 64)], 48, 8, 32), ([(0, 4096), (0, 4097)], 16, 1, 256), ([(i % 2, 1 + 9 * i) for i in range(64)], 4, 1, 64),
+])
+@pytest.mark.parametrize("moved", [False, True])
+def test_rows_that_see_each_other(gpu, rows, hq, hkv, block, moved):
+    """Rows (sequence, length) of the same sequences: each attends to the new tokens of those in front of it, as behind an append of all.  Stale NaN
+    lies where the new rows belong.  ``moved``: the first row's slot lies in the middle of its own context, and a row without tokens has its slot in it, too."""
+    gen = torch.Generator().manual_seed(sum(m for _, m in rows) + hkv)
+    longest = [max([m for s, m in rows if s == i] or [1]) for i in range(2)]
+    _, k, v, table, _ = _inputs(gen, longest, hq, hkv, block)
+    lens, place = [m for _, m in rows], lambda s, m: int(table[s, (m - 1) // block]) * block + (m - 1) % block
+    slots, table = [place(s, m) for s, m in rows], table[[s for s, _ in rows]].contiguous()
+    if moved:
+        slots[0] = place(rows[0][0], (lens[0] + 1) // 2)
+        slots[-1], lens[-1] = place(rows[0][0], 1), 0
+        if slots[0] == slots[-1]:
+            slots[0] = -1
+    n = len(rows)
+    for t in (k, v):
+        t.view(-1, hkv, 128)[[s for s in slots if s >= 0]] = float("nan")
+    slots, ctx = (torch.tensor(x, dtype=torch.int32).cuda() for x in (slots, lens))
+    q, kn, vn = (3 * torch.randn(n, h, 128, generator=gen).to(BF16).cuda() for h in (hq, hkv, hkv))
+    wq, wk = ((1 + 0.3 * torch.randn(128, generator=gen)).to(BF16).cuda() for _ in range(2))
+    cs, positions = torch.randn(max(lens) + 9, 128, generator=gen).to(BF16).cuda(), torch.tensor([max(m - 1, 0) + 3 * (i % 2) for i, m in enumerate(lens)]).cuda()
+    k2, v2 = k.clone(), v.clone()
+    out = ops.few_decode_with_front(q, kn, vn, positions, wq, wk, 1e-6, cs, k2, v2, slots, table, ctx, 0.09)
+    ops.qk_norm_rope_store_kvcache(q, kn, vn, positions, wq, wk, 1e-6, cs, k, v, slots, write_key=False)
+    want = torch.empty_like(out)
+    ops.paged_attn_decode(q, k, v, table, ctx, 0.09, want)
+    same = lambda a, b: torch.equal(a.view(torch.int16), b.view(torch.int16))
+    assert same(k, k2) and same(v, v2)
+    assert torch.isfinite(want.float()).all() and same(out, want)
+
+
 @pytest.mark.parametrize("length,hq,hkv,hidden", [(0, 16, 8, 1024), (1, 16, 8, 1024), (33, 16, 8, 1024), (260, 16, 8, 1000), (4097, 16, 8, 520),
                                                   (700, 32, 8, 512), (9000, 32, 16, 248), (300, 24, 8, 768), (300, 12, 12, 744), (64, 16, 8, 4096), (64, 4, 1, 512),
                                                   (700, 16, 8, 1024), (1024, 16, 8, 1024), (230, 16, 8, 1024)])
