@@ -118,6 +118,33 @@ def qk_norm_rope_store_kvcache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     _lib.check(rc, "qk_norm_rope_store_kvcache")
 
 
+def _few_decode_bytes(q, k, v, positions, q_norm_weight, k_norm_weight, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, context_lens) -> int:
+    """Bytes of the records of ``few_decode_with_front``, 0 where it does not take the call: one length for the whole batch, no lengths or table, a
+    batch that is not small, or something that the launches in its place take another way or refuse."""
+    if not isinstance(context_lens, torch.Tensor) or not isinstance(block_table, torch.Tensor) or block_table.dim() != 2 or q.dim() != 3 or k_cache.dim() != 4:
+        return 0
+    (n, hq, d), (_, bs, hkv, dk), (rows, columns) = q.shape, k_cache.shape, block_table.shape
+    if n == 0 or rows != n or columns < 1 or dk != d or bs % 32:
+        return 0
+    nbytes = _lib.load().infer_few_decode_workspace_bytes(n, hq, hkv, d, columns * bs)
+    if not nbytes:
+        return 0
+    if k.shape != (n, hkv, d) or v.shape != k.shape or v_cache.shape != k_cache.shape or block_table.stride(1) != 1:
+        return 0
+    if q_norm_weight.shape != (d,) or k_norm_weight.shape != (d,) or cos_sin_cache.dim() != 2 or cos_sin_cache.shape[1] != d:
+        return 0
+    for t in (q, k, v):
+        if t.dtype != torch.bfloat16 or not t.is_cuda or t.stride(2) != 1 or t.stride(1) != d:
+            return 0
+    for t in (k_cache, v_cache, q_norm_weight, k_norm_weight, cos_sin_cache):
+        if t.dtype != torch.bfloat16 or not t.is_cuda or not t.is_contiguous():
+            return 0
+    for t, dtype in ((slot_mapping, torch.int32), (context_lens, torch.int32), (positions, torch.int64)):
+        if t.dtype != dtype or not t.is_cuda or t.numel() != n or not t.is_contiguous():
+            return 0
+    return nbytes if block_table.dtype == torch.int32 and block_table.is_cuda else 0
+
+
 def few_decode_with_front(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, positions: torch.Tensor, q_norm_weight: torch.Tensor,
                           k_norm_weight: torch.Tensor, eps: float, cos_sin_cache: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                           slot_mapping: torch.Tensor, block_table: torch.Tensor, context_lens: torch.Tensor, scale: float,
@@ -126,27 +153,11 @@ def few_decode_with_front(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos
     batch is not small.  The rows stay as they are; the caches get what they would get, and rows may see each other's tokens (two rows of one
     sequence).  ``product``: the weight of the bare projection behind it.  Where the kernels take that in, too, the result is its sums in
     pieces (``SplitKSum``, the bits of ``linear(result, product, defer=True)``)."""
-    n, hq, d = q.shape
-    nblk, bs, hkv, _ = k_cache.shape
-    if context_lens is None or block_table is None or n == 0 or block_table.shape[0] != n or block_table.shape[1] < 1 or bs % 32:
-        return None
-    nbytes = _lib.load().infer_few_decode_workspace_bytes(n, hq, hkv, d, block_table.shape[1] * bs)
+    nbytes = _few_decode_bytes(q, k, v, positions, q_norm_weight, k_norm_weight, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, context_lens)
     if not nbytes:
         return None
-    assert k.shape == (n, hkv, d) and v.shape == (n, hkv, d)
-    for t in (q, k, v, q_norm_weight, k_norm_weight, cos_sin_cache, k_cache, v_cache):
-        assert t.dtype == torch.bfloat16
-    for t in (q, k, v):
-        assert t.stride(2) == 1 and t.stride(1) == d
-    assert q_norm_weight.shape == (d,) and k_norm_weight.shape == (d,)
-    assert q_norm_weight.is_contiguous() and k_norm_weight.is_contiguous()
-    assert cos_sin_cache.dim() == 2 and cos_sin_cache.shape[1] == d and cos_sin_cache.is_contiguous()
-    assert positions.dtype == torch.int64 and positions.numel() == n and positions.is_contiguous()
-    for t in (slot_mapping, context_lens):
-        assert t.dtype == torch.int32 and t.numel() == n and t.is_contiguous()
-    assert block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.stride(1) == 1
-    assert k_cache.shape == v_cache.shape and k_cache.is_contiguous() and v_cache.is_contiguous()
-    _require_gpu(q, k, v, positions, q_norm_weight, k_norm_weight, cos_sin_cache, k_cache, v_cache, slot_mapping, block_table, context_lens)
+    n, hq, d = q.shape
+    nblk, bs, hkv, _ = k_cache.shape
     pieces = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
     behind, out, sums = (None, 0, None, 0), None, None
     if product is not None and _linear_mode() == "static" and product.shape[1] == hq * d and _streamable(q.view(n, hq * d) if n == 1 else q, product):

@@ -4,7 +4,8 @@ Bar: weights of the values are rounded to bfloat16 (2^-9 each, of either sign) a
 import pytest
 import torch
 
-from infer_amd import ops
+from infer_amd import ops, qwen3
+from infer_amd.context import reset_context, set_context
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -228,3 +229,22 @@ def test_batches_that_are_not_small_are_left_alone(gpu):
     kept = k.clone()
     assert ops.few_decode_with_front(q, rows, rows, at, w, w, 1e-6, cs, k, v, at.int(), table, ctx, 0.1) is None
     assert torch.equal(k, kept)
+
+
+def test_one_length_for_the_whole_batch(gpu):
+    """A decode step's context may hold one number instead of the lengths, as decode attention takes it."""
+    gen = torch.Generator().manual_seed(10)
+    _, k, v, table, ctx = _inputs(gen, [300, 300], 16, 8, 256)
+    slots, positions = (table[:, 1] * 256 + 299 % 256).to(torch.int32), torch.tensor([299, 299]).cuda()
+    layer = qwen3.QwenAttention(256, 16, 8, max_position=512).to(device="cuda", dtype=BF16)
+    for p in (layer.qkv_proj.weight, layer.o_proj.weight):
+        p.data.copy_(0.05 * torch.randn(p.shape, generator=gen))
+    x, out = torch.randn(2, 256, generator=gen).to(BF16).cuda(), []
+    for lens in (ctx, 300):
+        layer.attn.k_cache, layer.attn.v_cache = k.clone(), v.clone()
+        set_context(False, slot_mapping=slots, context_lens=lens, block_tables=table)
+        y = layer(positions, x)
+        out.append((y.materialize() if isinstance(y, ops.SplitKSum) else y, layer.attn.k_cache, layer.attn.v_cache))
+    reset_context()
+    assert torch.equal(out[0][1], out[1][1]) and torch.equal(out[0][2], out[1][2])
+    assert (out[0][0].float() - out[1][0].float()).norm() <= 2.0 ** -7 * out[1][0].float().norm()

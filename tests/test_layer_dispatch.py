@@ -87,3 +87,16 @@ def test_a_forward_of_its_own_is_called(layer):
     layer.input_layernorm.forward = lambda x, residual=None: tuple(2 * t for t in inner(x, residual))
     layer(None, torch.randn(2, 16), torch.randn(2, 16))
     assert layer.fused == 1
+
+
+def test_calls_that_the_launch_with_the_front_leaves_to_two():
+    """One length for the whole batch, which decode attention takes, no lengths, other types: not this launch's, and nothing is raised here."""
+    rows, w, cache = torch.zeros(2, 8, 128, dtype=torch.bfloat16), torch.ones(128, dtype=torch.bfloat16), torch.zeros(4, 256, 8, 128, dtype=torch.bfloat16)
+    table, lens, at = torch.zeros(2, 2, dtype=torch.int32), torch.ones(2, dtype=torch.int32), torch.zeros(2, dtype=torch.int64)
+
+    def call(lens=lens, table=table, rows=rows, slots=lens):
+        return ops.few_decode_with_front(rows, rows, rows, at, w, w, 1e-6, w.expand(9, 128).contiguous(), cache, cache, slots, table, lens, 0.1)
+    assert ops._lib.load().infer_few_decode_workspace_bytes(2, 8, 8, 128, 512) > 0
+    for change in ({"lens": 64}, {"lens": None}, {"lens": lens.long()}, {"table": None}, {"table": table[0]}, {"table": table.long()}, {"rows": rows.float()},
+                   {"rows": rows[:, :, :64]}, {"slots": lens.long()}, {}):
+        assert call(**change) is None
