@@ -108,7 +108,7 @@ class QwenDecoderLayer(nn.Module):
     def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor, residual: torch.Tensor | None):
         # a step of few rows has its norms inside the products behind them
         attn, mlp, fused = self.self_attn, self.mlp, None
-        if type(attn.qkv_proj) is QKVLinear and _is_bare(attn, QwenAttention, _attention_forward):
+        if _is_bare(attn, QwenAttention, _attention_forward) and type(attn.qkv_proj) is QKVLinear:
             fused = norm_and_project(self.input_layernorm, attn.qkv_proj, hidden_states, residual)
         if fused is not None:
             qkv, residual = fused

@@ -89,6 +89,19 @@ def test_a_forward_of_its_own_is_called(layer):
     assert layer.fused == 1
 
 
+class Echo(torch.nn.Module):
+    def forward(self, *args):
+        return args[-1] * 2
+
+
+@pytest.mark.parametrize("where,fused", [("self_attn", 1), ("mlp", 1)])
+def test_a_module_of_its_own_needs_none_of_the_parts(layer, where, fused):
+    """A block put in the place of the attention or the MLP is called, whatever it is made of."""
+    setattr(layer, where, Echo())
+    layer(None, torch.randn(2, 16), torch.randn(2, 16))
+    assert layer.fused == fused
+
+
 def test_calls_that_the_launch_with_the_front_leaves_to_two():
     """One length for the whole batch, which decode attention takes, no lengths, other types: not this launch's, and nothing is raised here."""
     rows, w, cache = torch.zeros(2, 8, 128, dtype=torch.bfloat16), torch.ones(128, dtype=torch.bfloat16), torch.zeros(4, 256, 8, 128, dtype=torch.bfloat16)
