@@ -16,6 +16,7 @@ import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 from collections import OrderedDict
 
 import torch
@@ -202,12 +203,17 @@ _workspace_streams: dict = {}      # data_ptr of a shared workspace -> the strea
 
 
 def _load_decode_call():
-    """The native form of ``flash_attn_with_kvcache``.  It stands on the library next to it, so it is left out where another one is asked for."""
+    """The native form of ``flash_attn_with_kvcache``.  It stands on the library next to it, so it is left out where another one is asked for, and it
+    only saves time: where it cannot be loaded (built for another torch, its library missing) the calls are made from here."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_decode_call.so")
     if "INFER_KV_LIB" in os.environ or not os.path.exists(path):
         return None
     loader = importlib.machinery.ExtensionFileLoader("_decode_call", path)
-    return importlib.util.module_from_spec(importlib.machinery.ModuleSpec("_decode_call", loader, origin=path))
+    try:
+        return importlib.util.module_from_spec(importlib.machinery.ModuleSpec("_decode_call", loader, origin=path))
+    except ImportError as error:
+        warnings.warn(f"{path} cannot be loaded, decode calls take longer without it ({error}); run `make -C infer_amd/csrc`", RuntimeWarning)
+        return None
 
 
 _decode_call = _load_decode_call()

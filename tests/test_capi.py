@@ -5,7 +5,7 @@ import re
 
 import pytest
 
-from infer_amd import _lib
+from infer_amd import _lib, ops
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -33,6 +33,16 @@ def test_library_exports_every_declared_symbol_and_binding_covers_it():
         assert name in _lib.SIGNATURES, f"{name} has no ctypes signature"
     for name in _lib.SIGNATURES:
         assert name in declared_functions(), f"{name} bound but not declared in include/"
+
+
+def test_a_decode_call_that_cannot_be_loaded_is_left_out(monkeypatch, tmp_path):
+    """The module only saves host time: one that does not fit this process is named in a warning, and the package is there without it."""
+    monkeypatch.delenv("INFER_KV_LIB", raising=False)
+    monkeypatch.setattr(ops, "__file__", str(tmp_path / "ops.py"))
+    assert ops._load_decode_call() is None
+    (tmp_path / "_decode_call.so").write_bytes(b"no library")
+    with pytest.warns(RuntimeWarning, match="cannot be loaded"):
+        assert ops._load_decode_call() is None
 
 
 def test_host_only_entry_points():
