@@ -49,7 +49,7 @@ const at::Tensor* plain(PyObject* o) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(o);
     const auto keys = t.key_set();
-    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.is_neg() || t.is_conj() || keys.has(c10::DispatchKey::Python) ||
+    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.is_nested() || t.is_neg() || t.is_conj() || keys.has(c10::DispatchKey::Python) ||
         keys.has(c10::DispatchKey::FuncTorchBatched) || keys.has(c10::DispatchKey::FuncTorchGradWrapper) || keys.has(c10::DispatchKey::Functionalize) ||
         !t.has_storage())
         return nullptr;
@@ -57,7 +57,7 @@ const at::Tensor* plain(PyObject* o) {
 }
 
 // decode(q [B, 1, Hq, D], k_cache, v_cache [blocks, block, Hkv, D], lengths [B], block_table [B, columns], scale) -> [B, 1, Hq, D] or None
-PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
+PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) try {
     if (n != 6) return PyErr_Format(PyExc_TypeError, "decode takes 6 arguments");
     const at::Tensor *q = plain(args[0]), *k = plain(args[1]), *v = plain(args[2]), *lens = plain(args[3]), *table = plain(args[4]);
     if (!q || !k || !v || !lens || !table || !(PyFloat_CheckExact(args[5]) || args[5] == Py_None)) Py_RETURN_NONE;
@@ -73,21 +73,19 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (k->get_device() != device || v->get_device() != device || lens->get_device() != device || table->get_device() != device) Py_RETURN_NONE;
     const auto found = claims().find({device, hq, hkv});
     if (found == claims().end()) Py_RETURN_NONE;
-    try {
-        if (c10::hip::current_device() != device) Py_RETURN_NONE;
-        void* stream = c10::hip::getCurrentHIPStream(device).stream();
-        if (stream != found->second.stream) Py_RETURN_NONE;
-        const double scale = args[5] == Py_None ? 1.0 / std::sqrt((double)d) : PyFloat_AS_DOUBLE(args[5]);
-        at::Tensor out = at::empty({b, 1, hq, d}, q->options().requires_grad(false));
-        if (!out.is_cuda() || out.scalar_type() != at::kBFloat16) Py_RETURN_NONE;
-        const int rc = infer_paged_decode_bf16(q->data_ptr(), q->stride(0), k->data_ptr(), v->data_ptr(), k->stride(0), k->stride(1), out.data_ptr(), hq * d,
-                                               (const int32_t*)table->data_ptr(), table->stride(0), table->size(1), (const int32_t*)lens->data_ptr(), b, hq,
-                                               hkv, d, k->size(1), k->size(0), (float)scale, 0, found->second.workspace, found->second.bytes, stream);
-        if (rc != 0) Py_RETURN_NONE;
-        return THPVariable_Wrap(out);
-    } catch (...) {
-        Py_RETURN_NONE;      // the general way meets the same and says it
-    }
+    if (c10::hip::current_device() != device) Py_RETURN_NONE;
+    void* stream = c10::hip::getCurrentHIPStream(device).stream();
+    if (stream != found->second.stream) Py_RETURN_NONE;
+    const double scale = args[5] == Py_None ? 1.0 / std::sqrt((double)d) : PyFloat_AS_DOUBLE(args[5]);
+    at::Tensor out = at::empty({b, 1, hq, d}, q->options().requires_grad(false));
+    if (!out.is_cuda() || out.scalar_type() != at::kBFloat16) Py_RETURN_NONE;
+    const int rc = infer_paged_decode_bf16(q->data_ptr(), q->stride(0), k->data_ptr(), v->data_ptr(), k->stride(0), k->stride(1), out.data_ptr(), hq * d,
+                                           (const int32_t*)table->data_ptr(), table->stride(0), table->size(1), (const int32_t*)lens->data_ptr(), b, hq,
+                                           hkv, d, k->size(1), k->size(0), (float)scale, 0, found->second.workspace, found->second.bytes, stream);
+    if (rc != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(out);
+} catch (...) {
+    Py_RETURN_NONE;      // the general way meets the same and says it
 }
 
 PyMethodDef methods[] = {

@@ -97,3 +97,14 @@ def test_what_was_refused_is_refused(call, wrong):
     with pytest.raises((AssertionError, RuntimeError)):
         ops.flash_attn_with_kvcache(**{**args, "k_cache": args["k_cache"].cpu(), "v_cache": args["v_cache"].cpu()})
     assert taken == [False, False]
+
+
+@pytest.mark.parametrize("name,parts", [("q", [(1, 8, 128), (2, 8, 128), (1, 8, 128)]), ("k_cache", [(64, 2, 128), (32, 2, 128)]), ("v_cache", [(64, 2, 128), (32, 2, 128)]),
+                                        ("block_table", [(3,), (2,), (3,)])])
+def test_nested_tensors_are_refused(call, name, parts):
+    """Tensors without sizes: an error of the general way, not one that leaves native code."""
+    args, taken, _ = call
+    nested = torch.nested.nested_tensor([torch.zeros(s) for s in parts], dtype=torch.int32 if name == "block_table" else BF16, device="cuda")
+    with pytest.raises((AssertionError, RuntimeError)):
+        ops.flash_attn_with_kvcache(**{**args, name: nested})
+    assert taken == [False]
