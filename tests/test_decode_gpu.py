@@ -11,6 +11,22 @@ from tests.helpers import ATTN_ATOL, assert_seeded_inputs, bits, f32, oracle_dec
 pytestmark = pytest.mark.gpu
 
 
+# A few sequences have kernels of their own; the same rows over and over are a batch of the general ones.
+FORMS = pytest.mark.parametrize("form", ["few", "general"])
+
+
+def sized(wl, form):
+    """The workload, or its rows as often as makes them the general kernels'; and that the library sees it so."""
+    if form == "general":
+        times = 64 // (len(wl.lengths) * wl.num_kv_heads) + 1
+        wl = workloads.DecodeWorkload(**{**wl.__dict__, "lengths": list(wl.lengths) * times, "q": wl.q.repeat(times, 1, 1), "k_new": wl.k_new.repeat(times, 1, 1),
+                                         "v_new": wl.v_new.repeat(times, 1, 1), "slot_mapping": wl.slot_mapping.repeat(times),
+                                         "block_table": wl.block_table.repeat(times, 1), "context_lens": wl.context_lens.repeat(times)})
+    few = ops._lib.load().infer_few_decode_workspace_bytes(len(wl.lengths), wl.num_q_heads, wl.num_kv_heads, 128, wl.block_table.shape[1] * wl.block_size)
+    assert (few > 0) == (form == "few")
+    return wl
+
+
 def gpu_decode(wl, splits=None):
     if splits is None:
         out = ops.flash_attn_with_kvcache(wl.q.unsqueeze(1), wl.k_cache, wl.v_cache,
@@ -69,30 +85,34 @@ def test_split_count_invariance(gpu, splits):
     check(wl, splits=splits)
 
 
+@FORMS
 @pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 8), (32, 8), (64, 8), (4, 1), (8, 2), (32, 4), (32, 16), (16, 1)])
-def test_group_sizes_and_head_counts(gpu, hq, hkv):
-    wl = workloads.make_decode_workload(f"g{hq}-{hkv}", [1, 31, 32, 33, 255, 256, 257, 600], hq, hkv,
-                                        seed=hq * 7 + hkv).to(gpu)
-    check(wl)
+def test_group_sizes_and_head_counts(gpu, hq, hkv, form):
+    lens = [1, 31, 32, 33, 255, 256, 257, 600]
+    wl = workloads.make_decode_workload(f"g{hq}-{hkv}", lens if form == "general" or hkv <= 8 else lens[::3], hq, hkv, seed=hq * 7 + hkv).to(gpu)
+    check(sized(wl, form))
 
 
+@FORMS
 @pytest.mark.parametrize("bs", [32, 64, 128, 256, 512])
-def test_block_sizes(gpu, bs):
+def test_block_sizes(gpu, bs, form):
     wl = workloads.make_decode_workload(f"bs{bs}", [5, 97, 511, 512, 513, 1300], 32, 8, bs=bs, seed=bs).to(gpu)
-    check(wl)
+    check(sized(wl, form))
 
 
-def test_single_token_returns_v(gpu):
+@FORMS
+def test_single_token_returns_v(gpu, form):
     """L = 1: softmax over one key is 1, so O = V[0] exactly (bf16 round trip)."""
-    wl = workloads.make_decode_workload("one", [1, 1, 1], 32, 8, seed=5).to(gpu)
+    wl = sized(workloads.make_decode_workload("one", [1, 1, 1], 32, 8, seed=5).to(gpu), form)
     got = gpu_decode(wl)
-    for i in range(3):
+    for i in range(len(wl.lengths)):
         v0 = wl.v_cache[int(wl.block_table[i, 0]), 0]                    # [Hkv, D]
         assert torch.equal(got[i], v0.repeat_interleave(4, dim=0))
 
 
-def test_equal_keys_give_mean_of_values(gpu):
-    wl = workloads.make_decode_workload("mean", [300, 64], 16, 8, seed=6).to(gpu)
+@FORMS
+def test_equal_keys_give_mean_of_values(gpu, form):
+    wl = sized(workloads.make_decode_workload("mean", [300, 64], 16, 8, seed=6).to(gpu), form)
     wl.k_cache[:] = wl.k_cache[0, 0]          # every key identical -> uniform softmax
     got = f32(gpu_decode(wl))
     for i, n in enumerate(wl.lengths):
@@ -101,12 +121,14 @@ def test_equal_keys_give_mean_of_values(gpu):
         assert np.abs(got[i] - np.repeat(mean, 2, axis=0)).max() <= 1e-2
 
 
-def test_row_maximum_covers_every_key_of_a_step(gpu):
+@pytest.mark.parametrize("form,hq,hkv", [("general", 16, 8), ("few", 4, 2)])
+def test_row_maximum_covers_every_key_of_a_step(gpu, form, hq, hkv):
     """One key whose score lies some 350 log2 units above all others, once at each of the 32 positions of
     a step: the softmax gives it weight 1 wherever it sits.  A running maximum taken over part of a step
     only (say, the keys one row of lanes holds) leaves the exponential of that key to overflow."""
     lens = [96] * 32
-    wl = workloads.make_decode_workload("spike", lens, 16, 8, seed=11).to(gpu)
+    wl = workloads.make_decode_workload("spike", lens, hq, hkv, seed=11).to(gpu)
+    assert form == "general" or sized(wl, form) is wl
     g = wl.num_q_heads // wl.num_kv_heads
     for i in range(32):
         pos = 32 + i                                                     # the second of three steps
@@ -124,8 +146,9 @@ def test_row_maximum_covers_every_key_of_a_step(gpu):
         assert np.array_equal(got[i, ::g], f32(wl.v_cache[blk, pos % wl.block_size]))
 
 
+@FORMS
 @pytest.mark.parametrize("direction", [1, -1])
-def test_scores_that_rise_or_fall_along_the_sequence(gpu, direction):
+def test_scores_that_rise_or_fall_along_the_sequence(gpu, direction, form):
     """Keys that are multiples of the query, the factor rising (or falling) by a fixed amount per token: the
     running maximum grows at every step (the accumulators are rescaled every time), or is set by the very
     first key and never again, with all later keys hundreds of log2 units below it."""
@@ -139,15 +162,17 @@ def test_scores_that_rise_or_fall_along_the_sequence(gpu, direction):
             f = 0.5 * (pos if direction > 0 else -pos)                   # 16 log2-ish units per 32-token step
             blk = int(wl.block_table[i, pos // wl.block_size])
             wl.k_cache[blk, pos % wl.block_size] = (f * unit).to(torch.bfloat16)
+    wl = sized(wl, form)
     got = f32(gpu_decode(wl))
     want = oracle_decode(wl)
     assert np.isfinite(got).all()
     assert np.abs(got - want).max() <= ATTN_ATOL
 
 
-def test_block_permutation_invariance(gpu):
+@FORMS
+def test_block_permutation_invariance(gpu, form):
     """Same logical tokens under a different physical placement give bit-identical output."""
-    wl = workloads.make_decode_workload("perm", [700, 1023, 40], 32, 8, nblk=32, seed=7).to(gpu)
+    wl = sized(workloads.make_decode_workload("perm", [700, 1023, 40], 32, 8, nblk=32, seed=7).to(gpu), form)
     a = gpu_decode(wl)
     perm = torch.randperm(32, generator=torch.Generator().manual_seed(1)).to(gpu)
     inv = torch.empty_like(perm)
@@ -159,23 +184,24 @@ def test_block_permutation_invariance(gpu):
     assert torch.equal(a, out)
 
 
-def test_zero_length_rows_and_graph_padding(gpu):
+@FORMS
+def test_zero_length_rows_and_graph_padding(gpu, form):
     """Rows with context_len 0 (the reference zero-fills its graph buffers:
     infer/engine/model_runner.py:144-146) give zeros and do not disturb their neighbours; unused
     table entries may hold -1 or garbage."""
-    wl = workloads.make_decode_workload("pad", [300, 1, 513, 77], 32, 8, seed=8).to(gpu)
+    wl = sized(workloads.make_decode_workload("pad", [300, 1, 513, 77], 32, 8, seed=8).to(gpu), form)
     ctx = wl.context_lens.clone()
-    ctx[1] = 0
+    ctx[1::4] = 0
     bt = wl.block_table.clone()
     bt[bt < 0] = 10_000_000           # must never be dereferenced
-    bt[1] = -1
+    bt[1::4] = -1
     out = ops.flash_attn_with_kvcache(wl.q.unsqueeze(1), wl.k_cache, wl.v_cache, cache_seqlens=ctx,
                                       block_table=bt, softmax_scale=wl.scale)[:, 0]
     torch.cuda.synchronize()
     want = oracle_decode(wl)
     got = f32(out)
-    assert not got[1].any()
-    for i in (0, 2, 3):
+    assert not got[1::4].any()
+    for i in (i for i in range(len(got)) if i % 4 != 1):
         assert np.abs(got[i] - want[i]).max() <= ATTN_ATOL
     ctx[:] = 0
     out = ops.flash_attn_with_kvcache(wl.q.unsqueeze(1), wl.k_cache, wl.v_cache, cache_seqlens=ctx,
@@ -183,10 +209,11 @@ def test_zero_length_rows_and_graph_padding(gpu):
     assert not out.any()
 
 
-def test_stale_nan_beyond_length_is_ignored(gpu):
+@FORMS
+def test_stale_nan_beyond_length_is_ignored(gpu, form):
     """Cache rows past a sequence's length may hold anything (a freed sequence's data, NaN bit
     patterns of never-written memory): they must not reach the output."""
-    wl = workloads.make_decode_workload("nan", [37, 289, 1000], 32, 8, seed=9).to(gpu)
+    wl = sized(workloads.make_decode_workload("nan", [37, 289, 1000], 32, 8, seed=9).to(gpu), form)
     want = oracle_decode(wl)
     for i, n in enumerate(wl.lengths):
         blk = int(wl.block_table[i, (n - 1) // 256])
@@ -298,10 +325,11 @@ def test_cfg4_long_context(gpu):
     print("cfg4 max abs err", err)
 
 
-def test_layer_view_of_fused_cache(gpu):
+@FORMS
+def test_layer_view_of_fused_cache(gpu, form):
     """Caches as per-layer views of one [2, layers, nblk, bs, Hkv, D] tensor
     (infer/engine/model_runner.py:58-64)."""
-    wl = workloads.make_decode_workload("layers", [400, 90], 32, 8, nblk=6, seed=12).to(gpu)
+    wl = sized(workloads.make_decode_workload("layers", [400, 90], 32, 8, nblk=6, seed=12).to(gpu), form)
     big = torch.zeros((2, 3, 6, 256, 8, 128), dtype=torch.bfloat16, device=gpu)
     big[0, 1], big[1, 1] = wl.k_cache, wl.v_cache
     out = ops.flash_attn_with_kvcache(wl.q.unsqueeze(1), big[0, 1], big[1, 1], cache_seqlens=wl.context_lens,
@@ -388,13 +416,14 @@ def test_split_then_merge_need_not_agree_on_a_setting(gpu):
         assert float(np.abs(f32(out) - want).max()) <= ATTN_ATOL
 
 
-def test_length_beyond_the_table_is_cut_to_the_table(gpu):
+@FORMS
+def test_length_beyond_the_table_is_cut_to_the_table(gpu, form):
     """A context length larger than table_cols * block_size (a corrupt length) must not make the kernel
     read block ids past its table row: the row is attended as if it were table_cols blocks long."""
-    wl = workloads.make_decode_workload("clamp", [512, 700, 256], 16, 8, seed=14).to(gpu)
-    cols = wl.block_table.shape[1]                      # 3 blocks
-    full = [cols * 256] * 3
-    bad = torch.tensor([10 ** 6, 2 ** 31 - 1, cols * 256 + 1], dtype=torch.int32, device=gpu)
+    wl = sized(workloads.make_decode_workload("clamp", [512, 700, 256], 16, 8, seed=14).to(gpu), form)
+    cols, rows = wl.block_table.shape[1], len(wl.lengths)      # 3 blocks
+    full = [cols * 256] * rows
+    bad = torch.tensor([10 ** 6, 2 ** 31 - 1, cols * 256 + 1] * (rows // 3), dtype=torch.int32, device=gpu)
     bt = wl.block_table.clamp(min=0).contiguous()       # every entry of the row is a real block
     out_bad = torch.empty_like(wl.q)
     out_full = torch.empty_like(wl.q)
@@ -405,18 +434,20 @@ def test_length_beyond_the_table_is_cut_to_the_table(gpu):
     assert np.array_equal(bits(out_bad), bits(out_full))
 
 
+@FORMS
 @pytest.mark.parametrize("scale", [0.02, 0.3])
-def test_softmax_scale_is_honoured(gpu, scale):
+def test_softmax_scale_is_honoured(gpu, scale, form):
     """A scale other than head_dim ** -0.5 (the reference passes its own, infer/models/Qwen3.py:76)."""
     wl = workloads.make_decode_workload("scale", [37, 300, 1025, 700], 32, 8, nblk=16, seed=31).to(gpu)
     wl.scale = scale
-    check(wl)
+    check(sized(wl, form))
 
 
-def test_query_and_output_rows_as_strided_views(gpu):
+@FORMS
+def test_query_and_output_rows_as_strided_views(gpu, form):
     """Q as a column slice of the fused qkv matrix (infer/models/Qwen3.py:110-111) and the output as a
     slice of a wider buffer: same bits as with contiguous tensors."""
-    wl = workloads.make_decode_workload("views", [37, 300, 1025, 700], 32, 8, nblk=16, seed=32).to(gpu)
+    wl = sized(workloads.make_decode_workload("views", [37, 300, 1025, 700], 32, 8, nblk=16, seed=32).to(gpu), form)
     want = gpu_decode(wl, splits=0)
     b, hq, d = wl.q.shape
     qkv = torch.randn((b, (hq + 16) * d), device=gpu).to(torch.bfloat16)

@@ -12,8 +12,11 @@ from tests.helpers import ATTN_ATOL, f32, oracle_decode
 pytestmark = pytest.mark.gpu
 
 
-def test_decode_step_graph_replays_match_eager(gpu):
-    hq, hkv, d, bs, max_bs, max_blocks, nblk = 32, 8, 128, 256, 8, 6, 64
+@pytest.mark.parametrize("max_bs,few", [(8, True), (12, False)])
+def test_decode_step_graph_replays_match_eager(gpu, max_bs, few):
+    """``few``: the batch of the kernels for a few sequences; with more rows it is the general ones'."""
+    hq, hkv, d, bs, max_blocks, nblk = 32, 8, 128, 256, 6, 64
+    assert (ops._lib.load().infer_few_decode_workspace_bytes(max_bs, hq, hkv, d, max_blocks * bs) > 0) == few
     g = torch.Generator().manual_seed(0)
     k_cache = torch.randn((nblk, bs, hkv, d), generator=g).to(torch.bfloat16).to(gpu)
     v_cache = torch.randn((nblk, bs, hkv, d), generator=g).to(torch.bfloat16).to(gpu)
