@@ -435,7 +435,7 @@ def test_state_space_portions_are_cut_by_their_own_lengths(gpu, lens):
 
 @pytest.mark.parametrize("shape", [SSM[2], (4, 72, 48, 2, 4, 2)])
 def test_state_space_of_many_portions_and_of_a_long_one(gpu, shape):
-    """More workgroups than two per compute unit, and one portion of more than 4096 tokens, are walked by four wavefronts each instead of eight."""
+    """More workgroups than two per compute unit, walked by four wavefronts each instead of eight, and one portion of many segments."""
     many = 520 // (shape[0] * -(-shape[1] // 64)) + 1
     m = Ssm(np.random.default_rng(many), shape, torch.bfloat16, slots=many, a_log=(-9.0, -5.0))
     lens = [2 + (7 * i) % 70 for i in range(many)]
@@ -449,6 +449,23 @@ def test_state_space_of_many_portions_and_of_a_long_one(gpu, shape):
     want, states = m.want(x)
     close(torch.tensor(np.concatenate(m.run([(3, 0, x)]))), want, 2e-2)
     close(m.state[3], states, 1e-2)
+
+
+@pytest.mark.parametrize("shape,n,segments", [((20, 200, 24, 2, 4, 2), 4010, 10), ((20, 200, 128, 2, 4, 2), 4010, 10), ((2, 136, 256, 2, 2, 4), 700, 5)])
+def test_state_space_segments_walked_by_four_wavefronts(gpu, shape, n, segments):
+    """One long portion (heads x slabs of 64 columns x tokens above 320000, which eight wavefronts would cut into 7 segments), and states of more than
+    128 rows, in segments that four wavefronts walk each.  The reference stores in bfloat16 what the layer does, behind the convolution and in front of
+    the norm: among 16 million results these roundings alone make 0.0245 of the largest (both in float64, first shape); what is left is the last rounding
+    (2^-9) and values near a tie that are stored as the neighbour (2^-8)."""
+    m = Ssm(np.random.default_rng(n), shape, torch.bfloat16, a_log=(-9.0, -5.0))
+    s = m.s
+    floats = ops._lib.load().infer_state_space_workspace_floats(ho.ELEM[torch.bfloat16], s.heads, s.vdim, s.state, 1, n)
+    assert floats == segments * s.heads * (s.state * s.vdim + 1)
+    x = m.inputs(30 + n)
+    want, states = m.want(x, lambda a: rounded(a, torch.bfloat16))
+    got = m.run([(2, 0, x[:30])]) + m.run([(2, 30, x[30:])])
+    close(torch.tensor(np.concatenate(got)), want, 2e-2)
+    close(m.state[2], states, 1e-2)
 
 
 @BOTH
