@@ -456,3 +456,24 @@ def test_decay_workgroups_of_four_and_of_eight_wavefronts(gpu, kind, vdim, heads
         want, end = d.want(x[row:row + n], pos0, starts[i], round_silu=True)
         close(out[row:row + n], want, tol(bf, 1e-5))
         d.check_state(state, i, end, state_tol(d, bf))
+
+
+@pytest.mark.parametrize("kind", ["lightning", "plain"])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("heads,lens", [(12, (700, 33, 96)), (44, (20, 3, 40, 33, 5, 32, 2, 64, 65, 31))])
+def test_decay_workgroups_of_four_wavefronts_and_wide_heads(gpu, kind, dim, heads, lens):
+    """Cut portions of some workgroups, and whole ones of many short ones, which four wavefronts walk, with 64 and 128 state rows."""
+    bf = torch.bfloat16
+    d = Decay(kind, tuple(1.0 - 2.0 ** -(2 + i % 9) for i in range(heads)), dim, 128, 32, bf, seed=heads + dim)
+    x = rounded(d.inputs(sum(lens)), bf)
+    state, spans, row = d.state(len(lens)), [], 0
+    starts = [d.rng.standard_normal((heads, dim, 128)) if i % 2 else np.zeros((heads, dim, 128)) for i in range(len(lens))]
+    for i, n in enumerate(lens):
+        d.fill(state, i, starts[i])
+        spans.append((row, n, i, 7 * (i % 2)))
+        row += n
+    out = d.run(x, state, None, None, 0, spans)
+    for row, n, i, pos0 in spans:
+        want, end = d.want(x[row:row + n], pos0, starts[i], round_silu=True)
+        close(out[row:row + n], want, tol(bf, 1e-5))
+        d.check_state(state, i, end, state_tol(d, bf))
