@@ -5,7 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from infer_amd import ops, qwen3
+from infer_amd import attention as attention_module, ops, qwen3
 
 
 def _norm(x, weight, eps, residual=None, out=None):
@@ -113,3 +113,88 @@ def test_calls_that_the_launch_with_the_front_leaves_to_two():
     for change in ({"lens": 64}, {"lens": None}, {"lens": lens.long()}, {"table": None}, {"table": table[0]}, {"table": table.long()}, {"rows": rows.float()},
                    {"rows": rows[:, :, :64]}, {"slots": lens.long()}, {}):
         assert call(**change) is None
+
+
+@pytest.fixture
+def attention(monkeypatch):
+    """An attention with its cache, in a decode step; ``given``: what the launch with the front was given as the product behind it, call by call."""
+    torch.manual_seed(1)
+    it = qwen3.QwenAttention(16, 2, 1, max_position=8, head_dim=8).float()
+    for p in it.parameters():
+        torch.nn.init.normal_(p)
+    it.attn.k_cache = it.attn.v_cache = torch.zeros(1, 4, 1, 8)
+    it.given = []
+    context = SimpleNamespace(slot_mapping=torch.zeros(2, dtype=torch.int32), is_prefill=False, block_tables=torch.zeros(2, 1), context_lens=torch.ones(2))
+
+    def few(q, *rest):
+        it.given.append(rest[-1])
+        return q * 2
+    monkeypatch.setattr(ops, "few_decode_with_front", few)
+    monkeypatch.setattr(ops, "flash_attn_with_kvcache", lambda q, *a, **k: q * 2)
+    monkeypatch.setattr(ops, "qk_norm_rope_store_kvcache", lambda *a, **k: None)
+    monkeypatch.setattr(qwen3, "cos_sin_table", lambda *a: None)
+    for module in (qwen3, attention_module):
+        monkeypatch.setattr(module, "get_context", lambda: context)
+    return it
+
+
+def _attend(it):
+    x = torch.randn(2, 16, generator=torch.Generator().manual_seed(2))
+    torch.testing.assert_close(it(None, x), F.linear(2 * it.qkv_proj(x)[:, :16], it.o_proj.weight, it.o_proj.bias))
+
+
+def test_attention_of_a_few_rows_takes_the_front_and_the_product(attention):
+    _attend(attention)
+    assert len(attention.given) == 1 and attention.given[0] is attention.o_proj.weight
+
+
+def test_sums_of_the_product_are_passed_on(attention, monkeypatch):
+    sums = ops.SplitKSum(torch.zeros(2, 2, 16), torch.float32)
+    monkeypatch.setattr(ops, "few_decode_with_front", lambda *a: sums)
+    attention.o_proj.forward = None
+    assert attention(None, torch.randn(2, 16)) is sums
+
+
+@pytest.mark.parametrize("how", ["hook", "pre-hook", "forward"])
+@pytest.mark.parametrize("where", ["q_norm", "k_norm", "attn"])
+def test_no_front_where_somebody_looks_at_its_parts(attention, where, how):
+    part = getattr(attention, where)
+    if how == "hook":
+        part.register_forward_hook(lambda *a: None)
+    elif how == "pre-hook":
+        part.register_forward_pre_hook(lambda *a: None)
+    else:
+        inner = part.forward
+        part.forward = lambda *a, **k: inner(*a, **k)
+    _attend(attention)
+    assert attention.given == []
+
+
+def test_no_front_where_decode_is_somebody_elses(attention):
+    seen, inner = [], attention.attn._decode
+    attention.attn._decode = lambda *a: seen.append(1) or inner(*a)
+    _attend(attention)
+    assert attention.given == [] and seen == [1]
+
+
+@pytest.mark.parametrize("how", ["hook", "pre-hook", "forward", "bias", "class"])
+def test_no_product_where_the_projection_is_more_than_its_weight(attention, how):
+    seen, proj = [], attention.o_proj
+    if how == "hook":
+        proj.register_forward_hook(lambda *a: seen.append(1))
+    elif how == "pre-hook":
+        proj.register_forward_pre_hook(lambda *a: seen.append(1))
+    elif how == "forward":
+        inner = proj.forward
+        proj.forward = lambda *a, **k: seen.append(1) or inner(*a, **k)
+    elif how == "bias":
+        proj.register_parameter("bias", torch.nn.Parameter(torch.randn(16)))
+        seen.append(1)
+    else:
+        class Other(type(proj)):
+            def forward(self, *a, **k):
+                seen.append(1)
+                return super().forward(*a, **k)
+        proj.__class__ = Other
+    _attend(attention)
+    assert attention.given == [None] and seen == [1]
