@@ -27,6 +27,7 @@
 
 #include "elem.h"
 #include "pieces.h"
+#include "segments.h"
 
 namespace {
 
@@ -163,13 +164,6 @@ __device__ __forceinline__ u32x4_t silu8(u32x4_t x) {
     return __builtin_bit_cast(u32x4_t, r);
 }
 
-// Tokens of a segment of a portion of `count`: as many segments as `most` tokens each would make, all of one length but for the last one's
-// rest, so that a portion a little longer than `most` does not leave a workgroup with almost nothing.
-__device__ __forceinline__ int own_segment(int count, int most) {
-    const int segs = (count + most - 1) / most;
-    return segs > 1 ? ((count + segs - 1) / segs + kC - 1) / kC * kC : most;
-}
-
 // A workgroup of four or eight wavefronts serves one head and 16 VT columns of its state per wavefront over the chunks of one segment.
 // Wavefront w owns the columns 16 VT w .. and their part of the state, DT tiles of 32 rows, as accumulators: lane (g, n)
 // holds rows 16 t + 4 g + e of column n.  That is an operand of the next product as it lies, when the rows of a
@@ -201,7 +195,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
     const Span span = args.spans[blockIdx.z];
-    const int seg_len = own_segment(span.count, args.seg_len), first = seg * seg_len;
+    const int seg_len = own_segment(span.count, args.seg_len, kC), first = seg * seg_len;
     if (span.slot < 0 || span.slot >= a.num_slots || first >= span.count) return;
     const bool last_seg = first + seg_len >= span.count;
     if (!OUT && last_seg) return;                                // nobody needs its final state yet
@@ -626,7 +620,7 @@ __global__ void __launch_bounds__(kThreads) decay_join_kernel(ChunkArgs args) {
     const Span span = args.spans[blockIdx.z];
     const int64_t state_len = (int64_t)a.dim_pad * a.vdim_pad, i = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 4;
     if (span.slot < 0 || span.slot >= a.num_slots || i >= state_len) return;
-    const int seg_len = own_segment(span.count, args.seg_len);
+    const int seg_len = own_segment(span.count, args.seg_len, kC);
     const float seg_decay = exp2f((float)seg_len * a.decay[2 * a.heads + h]);
     f32x4_t s = {0.f, 0.f, 0.f, 0.f};
     if (span.pos0 > 0) s = *reinterpret_cast<const f32x4_t*>(a.state + ((int64_t)span.slot * a.heads + h) * state_len + i);

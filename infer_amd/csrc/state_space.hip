@@ -21,6 +21,7 @@
 // float precision), the products of the output, which is rounded to bf16 next, take two (2^-17).
 #include "elem.h"
 #include "pieces.h"
+#include "segments.h"
 
 namespace {
 
@@ -272,13 +273,6 @@ struct ChunkArgs {
     float* ws_decay;
 };
 
-// Tokens of a segment of a portion of `count`: as many segments as `most` tokens each would make, all of one length but for the last one's
-// rest, so that a portion a little longer than `most` does not leave a workgroup with almost nothing.
-__device__ __forceinline__ int own_segment(int count, int most) {
-    const int segs = (count + most - 1) / most;
-    return segs > 1 ? ((count + segs - 1) / segs + kC - 1) / kC * kC : most;
-}
-
 // A workgroup serves one head and 64 columns of its state over the chunks of one segment.  Wavefront w owns 16 columns as accumulators, of
 // eight wavefronts half the state rows each: lane (g, n) holds state rows 16 t + 4 g + e of column n.  That is an operand of the product with C
 // as it lies, when the state rows of a k-step of 32 are taken in the order 16 tau + 4 g + e.  The 32 x 32 products C_i B_j are shared
@@ -309,7 +303,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2, cw = wave & 3;
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
     const Span span = args.spans[blockIdx.z];
-    const int seg_len = own_segment(span.count, args.seg_len), first = seg * seg_len;
+    const int seg_len = own_segment(span.count, args.seg_len, kC), first = seg * seg_len;
     if (span.slot < 0 || span.slot >= a.num_slots || first >= span.count) return;
     const bool last_seg = first + seg_len >= span.count;
     if (!OUT && last_seg) return;                                // nobody needs its final state yet
@@ -373,7 +367,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
     };
     const float a2 = -expf(a.a_log[h]) * kLog2e, bias = a.dt_bias[h], dh = a.d[h];
     float total = 0.f;                                           // log2 of the segment's decay
-    // step sizes of chunks c .. c + 3, this wavefront's being c + wave
+    // step sizes of chunks c .. c + kAhead - 1, this wavefront's being c + wave
     auto put_steps = [&](int c) {
         const int group = (c / kAhead) & 1;
         const float dt = (c + wave) * kC + (lane & 31) < count ? softplus_f((float)dtreg + bias) : 0.f;
@@ -543,7 +537,7 @@ __global__ void __launch_bounds__(kThreads) ssm_join_kernel(ChunkArgs args) {
     const int64_t state_len = (int64_t)a.state_n * a.vdim, i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= state_len || span.slot < 0 || span.slot >= a.num_slots) return;
     float cur = span.pos0 > 0 ? a.state[((int64_t)span.slot * a.heads + h) * state_len + i] : 0.f;
-    const int seg_len = own_segment(span.count, args.seg_len), segs = (span.count + seg_len - 1) / seg_len;
+    const int seg_len = own_segment(span.count, args.seg_len, kC), segs = (span.count + seg_len - 1) / seg_len;
     for (int k = 0; k < segs; ++k) {
         const int64_t rec = ((int64_t)blockIdx.z * args.max_seg + k) * a.heads + h;
         float* w = args.ws + rec * state_len + i;
