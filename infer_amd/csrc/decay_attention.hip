@@ -846,14 +846,18 @@ int slabs_of(int64_t dim_pad, int64_t vdim_pad) {
 // no less than four chunks, since cut ones are walked twice.  Four wavefronts: below one workgroup per compute unit, into two of them; 32 heads of
 // 128 x 128, the call in us, cut / whole: 8 portions of 1500 tokens 252 / 212, 12 of 100 to 1500 284 / 241, but 6 of 900 to 3700 320 / 390.
 // Segments of one length per portion instead of one for the batch: 6 portions of 900 to 3700 of 32 heads 338 -> 320, 5 of them 347 -> 298.
-// Eight wavefronts with 16 columns each, two chunks in LDS, one workgroup per compute unit; four with 32 / eight, us: 32 heads, 10 portions of 800
-// to 1800 271 / 241, 8 of 1500 210 / 190, 6 of 900 to 3700 331 / 316, 20 of 300 to 900 222 / 205, 1 of 9000 207 / 196; 16 heads, 16 of 200 to 1000 120 / 98, 11
-// of 500 to 1500 160 / 137, 8 of 100 to 600 70 / 58, 1 of 300 43 / 35.  Where whole portions leave much of the chip idle and cut ones are long, four
-// are ahead (16 heads, 8 of 1000 to 3000 220 / 257; 32 heads, 4 of 1000 to 2500 185 / 210), and where there are many workgroups or they are little
-// but their start (32 heads, 64 of 100 to 300 227 / 243, 30 of 200 to 500 189 / 192, 16 of 50 to 250 59 / 61).  Behind a rotation, where a key
-// is three pieces, there is no room for two chunks, and eight are behind (32 heads, 6 of 900 to 3700 371 / 506).
-// Whole portions take as long as the longest of them: between half a workgroup and one per compute unit eight pay if there are tokens for some 110
-// workgroups of that length (6 of 200 to 4000, 100 of them, 315 / 319; 5 of 800 to 5000 350 / 395), or if it is short.
+// Eight wavefronts with 16 columns each, two chunks in LDS, one workgroup per compute unit, portions whole from 128 workgroups on.  Behind a rotation, where a
+// key is three pieces, there is no room for two chunks, and eight are behind (32 heads, 6 of 900 to 3700 371 / 506).  Else by the number of workgroups; four
+// wavefronts with 32 columns / eight, us, heads x portions:
+// up to 32: both cut into what fills the chip.  32 x 1 of 9000 207 / 196, 16 x 1 of 300 43 / 35.
+// to 159: four cut, eight walk whole or nearly so, which leaves the chip idle; it pays where portions are short.  16 x 8 of 100 to 600 70 / 58, but of 1000 to 3000
+// 220 / 257, and 32 x 4 of 1000 to 2500 185 / 210: up to 640 tokens.
+// to 255: whole portions take as long as the longest, cut ones as long as all tokens together, twice.  16 x 11 of 500 to 1500 160 / 137; of longer ones what
+// counts is how many workgroups as long as the longest all tokens would make: 32 x 6 of 900 to 3700, 134 of them, 331 / 316, of 200 to 4000, 100, 315 / 319,
+// 32 x 5 of 800 to 5000, 93, 350 / 395: from 110.
+// from 256: 32 x 8 of 1500 210 / 190, 32 x 10 of 800 to 1800 271 / 241, 16 x 16 of 200 to 1000 120 / 98, 32 x 20 of 300 to 900 222 / 205; but two workgroups of
+// four share a unit, and where there are more than two and a half rounds (32 x 30 of 200 to 500 189 / 192, 32 x 64 of 100 to 300 227 / 243), or workgroups are
+// little but their start (32 x 16 of 50 to 250 59 / 61), they are ahead.
 bool eight_waves(int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t rot_dims, int64_t num_spans, int64_t max_span, int64_t tokens) {
     const int64_t per_token = heads * slabs_of(dim_pad, vdim_pad), groups = per_token * num_spans;
     if (column_tiles(dim_pad, vdim_pad) != 2 || rot_dims > 0 || groups > 640 || (groups > 384 && max_span <= 256)) return false;

@@ -106,6 +106,8 @@ class QwenDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor, residual: torch.Tensor | None):
+        """Returns the layer's output and the residual in front of the next norm.  That is the tensor to go on with: it may or may not lie where the
+        one given does, whose memory may be overwritten."""
         # a step of few rows has its norms inside the products behind them
         attn, mlp, fused = self.self_attn, self.mlp, None
         if _is_bare(attn, QwenAttention, _attention_forward) and type(attn.qkv_proj) is QKVLinear:
