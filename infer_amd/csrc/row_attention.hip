@@ -444,6 +444,7 @@ struct RowGatherArgs {
     uint16_t* out;             // [total][kv_heads][row]
     const int32_t* cu_q;       // [sequences + 1] or nullptr: rows that no query of these portions sees are left out
     KeyMask mask;
+    int group0;                // the launch's first kGather tokens of every sequence
 };
 
 // A workgroup copies kGather tokens of one head, kGatherBatch requests of a thread at a time: what a page holds of a head is consecutive, so unit
@@ -453,7 +454,7 @@ struct RowGatherArgs {
 constexpr int kGather = 32, kGatherBatch = 4;
 template <bool WHOLE>
 __global__ void __launch_bounds__(256) row_gather_kernel(RowGatherArgs a) {
-    const int s = blockIdx.y, h = blockIdx.x % a.kv_heads, first = blockIdx.x / a.kv_heads * kGather;
+    const int s = blockIdx.y, h = blockIdx.x % a.kv_heads, first = (a.group0 + blockIdx.x / a.kv_heads) * kGather;
     const int k0 = a.cu_k[s];
     int len = a.cu_k[s + 1] - k0;
     const int cap = a.table_cols * a.block_size;
@@ -595,13 +596,16 @@ int row_gather(const void* cache, int64_t row, int64_t kv_heads, int64_t block_s
         return INFER_KV_EINVAL;
     if (row % 8 || !ptr_aligned(cache, 16) || !ptr_aligned(out, 16)) return INFER_KV_EALIGN;
     RowGatherArgs a{(const uint16_t*)cache, (int)row, (int)kv_heads, (int)block_size, (int)num_blocks, (int)table_cols, block_table,
-                    bt_stride, seqs, cu_k, (uint16_t*)out, cu_q, mask};
+                    bt_stride, seqs, cu_k, (uint16_t*)out, cu_q, mask, 0};
     const int64_t most = table_cols * block_size < max_keys ? table_cols * block_size : max_keys;      // what a row of the table holds
-    const int64_t groups = (most + kGather - 1) / kGather * kv_heads;
-    if (groups > 0x7fffffff) return INFER_KV_EINVAL;
-    const dim3 grid((unsigned)groups, (unsigned)num_seqs), block(256);
-    if (block_size % kGather == 0) hipLaunchKernelGGL((row_gather_kernel<true>), grid, block, 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL((row_gather_kernel<false>), grid, block, 0, (hipStream_t)stream, a);
+    // a launch has less than 2^32 threads along x
+    const int64_t groups = (most + kGather - 1) / kGather, launch = ((1 << 24) - 1) / kv_heads;
+    for (int64_t at = 0; at < groups; at += launch) {
+        a.group0 = (int)at;
+        const dim3 grid((unsigned)((groups - at < launch ? groups - at : launch) * kv_heads), (unsigned)num_seqs), block(256);
+        if (block_size % kGather == 0) hipLaunchKernelGGL((row_gather_kernel<true>), grid, block, 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL((row_gather_kernel<false>), grid, block, 0, (hipStream_t)stream, a);
+    }
     return (int)hipGetLastError();
 }
 

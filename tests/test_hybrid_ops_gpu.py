@@ -246,6 +246,18 @@ def test_gather_of_pages_of_any_size(gpu, heads, row, block):
     assert torch.equal(out.cpu(), torch.cat(want))
 
 
+def test_gather_with_tables_for_more_workgroups_than_a_launch_has(gpu):
+    """Wide tables, many heads and a bound on the keys as loose as the table: 2^33 threads in all, of which a few have something to do."""
+    gen, lens = torch.Generator().manual_seed(2), [40, 1, 33]
+    cache = torch.randn(5, 4096, 32, 8, generator=gen).to(torch.bfloat16)
+    tables = torch.full((3, 8192), -1, dtype=torch.int32)
+    tables[0, :2], tables[1, :1], tables[2, :2] = torch.tensor([4, 1]), torch.tensor([2]), torch.tensor([0, 3])
+    want = [cache[tables[s][torch.arange(n) // 32].long(), :, torch.arange(n) % 32] for s, n in enumerate(lens)]
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    out = ho.grouped_gather(cache.cuda(), tables.cuda(), torch.arange(3, dtype=torch.int32).cuda(), cu.cuda(), sum(lens), 8192 * 32)
+    assert torch.equal(out.cpu(), torch.cat(want))
+
+
 @pytest.mark.parametrize("heads,dim,rot,vdim", [(3, 16, 8, 24), (5, 48, 16, 40), (2, 96, 32, 64), (2, 64, 32, 128), (3, 128, 64, 128), (1, 192, 64, 104), (2, 24, 40, 8)])
 def test_latent_prefill(gpu, heads, dim, rot, vdim):
     """Portions with and without a prefix, lengths around the tiles; one query-key pair stands out."""
