@@ -48,6 +48,33 @@ __device__ __forceinline__ void few_add(few_f32x4& num, float2& s, few_f32x4 x, 
     for (int e = 0; e < 4; ++e) num[e] = __builtin_fmaf(num[e], f1, x[e] * f2);
     s = make_float2(top, __builtin_fmaf(s.y, f1, o.y * f2));
 }
+// The same, the other product rounded by itself.
+__device__ __forceinline__ void few_append(few_f32x4& num, float2& s, few_f32x4 x, float2 o) {
+    const float top = fmaxf(s.x, o.x), f1 = s.x == top ? 1.f : __builtin_amdgcn_exp2f(s.x - top), f2 = o.x == top ? 1.f : __builtin_amdgcn_exp2f(o.x - top);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) num[e] = __builtin_fmaf(x[e], f2, num[e] * f1);
+    s = make_float2(top, __builtin_fmaf(o.y, f2, s.y * f1));
+}
+// Pieces meet in pairs, and every fourth pair in one of four parts: piece e of pair i of a part, and the sum of a part's N pairs, if there are any.
+__device__ __forceinline__ int few_piece(int part, int i, int e) { return 2 * (part + 4 * i) + e; }
+template <int N>
+__device__ __forceinline__ void few_part(few_f32x4& num, float2& s, int part, int pieces, const few_f32x4 (&v)[N][2], const float2 (&ml)[N][2]) {
+    num = few_f32x4{0.f, 0.f, 0.f, 0.f};
+    s = make_float2(-INFINITY, 0.f);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        few_f32x4 x = v[i][0];
+        float2 o = ml[i][0];
+        if (few_piece(part, i, 1) < pieces) few_add(x, o, v[i][1], ml[i][1]);
+        if (few_piece(part, i, 0) >= pieces) continue;
+        if (i > 0) {
+            few_append(num, s, x, o);
+        } else {
+            num = x;
+            s = o;
+        }
+    }
+}
 
 // Pieces per (sequence, KV head), or 0 where the batch is not small.
 int few_decode_pieces(int64_t batch, int64_t num_kv_heads, int64_t max_tokens);

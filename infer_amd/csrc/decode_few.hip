@@ -69,8 +69,8 @@ __device__ __forceinline__ u32x4 norm_and_rotate(u32x4 x, u32x4 w, u32x4 c, u32x
 // so with the new key, takes key and value from its registers, since what it has requested is older, and puts them into the caches at its
 // end, where nothing waits for the stores.  Nobody waits for those stores either: a step that holds the slot of another new token (two rows of
 // one sequence, say), or its own in the middle, takes that row's key and value from the row, normed and rotated on the spot, whatever the caches
-// hold there by then.  us, 16 heads on 8, front and attention in launches of their own / this: 1 x 700 tokens 9.7 / 8.1,
-// 4 x 700 12.4 / 11.2, 8 x 700 16.2 / 15.4; 32 heads 10.2 / 8.2, 12.8 / 11.9, 16.9 / 16.5; a step of a 0.6B model with one sequence 820 -> 778.
+// hold there by then.  us, 16 heads on 8, front and attention in launches of their own / this: 1 x 700 tokens 9.6 / 8.0,
+// 4 x 700 11.4 / 10.2, 8 x 700 16.3 / 15.4; 32 heads 9.9 / 8.2, 12.0 / 11.0, 16.8 / 16.3; a step of a 0.6B model with one sequence 820 -> 778.
 // (With the stores in front of the products, with front loads of wavefronts without a step, or with heads spread as operands are, it gained nothing.)
 template <bool FRONT>
 __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a, FewFront f) {
@@ -329,37 +329,39 @@ __global__ void __launch_bounds__(64 * kWaves) few_decode_kernel(FewDecode a, Fe
 
 constexpr int kMostPieces = 64;
 
-// Up to 8 N pieces.  Grid (query heads, batch): 32 lanes hold the columns of the head, the eight halves of wavefronts every eighth piece.  Pieces are requested before it
-// is known how many there are; what lies behind the last is not looked at.
+// Up to 8 N pieces.  Grid (query heads, batch): 32 lanes hold the columns of the head, the four halves of wavefronts every fourth pair of pieces.  Pieces are requested
+// before it is known how many there are; what lies behind the last is not looked at.  The order and the roundings are those of the general kernels where every
+// step has a wavefront of its own: there, too, two steps meet first (in LDS), then every fourth record.  So a single sequence with no more steps than pieces has the
+// bits of those kernels (KV heads in fours, up to two query heads each: as the compiler fuses their products).
 template <int N>
-__global__ void __launch_bounds__(256) few_decode_sum_kernel(FewDecode a) {
-    __shared__ f32x4 sums[7][32];
-    __shared__ float2 mls[7];
+__global__ void __launch_bounds__(128) few_decode_sum_kernel(FewDecode a) {
+    __shared__ f32x4 sums[3][32];
+    __shared__ float2 mls[3];
     const int head = blockIdx.x, b = blockIdx.y, G = a.group, h = head / G, n = head - h * G, c = threadIdx.x & 31, part = threadIdx.x >> 5;
     const int floats = few_record_floats(G);
     const float* rec = a.rec + ((int64_t)b * a.num_kv_heads + h) * a.pieces * floats;
-    f32x4 v[N];
-    float2 ml[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const int p = part + 8 * i;
-        const float* from = rec + (int64_t)(p < a.pieces ? p : 0) * floats;
-        v[i] = *reinterpret_cast<const f32x4*>(from + n * kD + 4 * c);
-        ml[i] = *reinterpret_cast<const float2*>(from + G * kD + 2 * n);
-    }
-    const int pieces = few_pieces_of(a, a.ctx[b]);
-    f32x4 num = {0.f, 0.f, 0.f, 0.f};
-    float2 s = make_float2(-INFINITY, 0.f);
+    f32x4 v[N][2];
+    float2 ml[N][2];
 #pragma unroll
     for (int i = 0; i < N; ++i)
-        if (part + 8 * i < pieces) few_add(num, s, v[i], ml[i]);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int p = few_piece(part, i, e);
+            const float* from = rec + (int64_t)(p < a.pieces ? p : 0) * floats;
+            v[i][e] = *reinterpret_cast<const f32x4*>(from + n * kD + 4 * c);
+            ml[i][e] = *reinterpret_cast<const float2*>(from + G * kD + 2 * n);
+        }
+    const int pieces = few_pieces_of(a, a.ctx[b]);
+    f32x4 num;
+    float2 s;
+    few_part<N>(num, s, part, pieces, v, ml);
     if (part > 0) {
         sums[part - 1][c] = num;
         if (c == 0) mls[part - 1] = s;
     }
     __syncthreads();
     if (part > 0) return;
-    for (int w = 1; w < 8 && w < pieces; ++w) few_add(num, s, sums[w - 1][c], mls[w - 1]);
+    for (int w = 1; w < 4 && 2 * w < pieces; ++w) few_add(num, s, sums[w - 1][c], mls[w - 1]);
     const float inv = s.y > 0.f ? 1.f / s.y : 0.f;
     bf16x4 o;
 #pragma unroll
@@ -370,12 +372,12 @@ __global__ void __launch_bounds__(256) few_decode_sum_kernel(FewDecode a) {
 }  // namespace
 
 // Pairs of a sequence and a KV head, against paged_decode.hip, us, both launches (32 heads on 8, tokens of each sequence or of the shortest and
-// longest): 1 x 700 12.4 / 7.2, 1 x 4000 18.5 / 11.1, 1 x 30000 40 / 30, 4 x 700 13.6 / 9.3, 4 x 16000 53.6 / 53.1, 4 x 100 .. 16000 33 / 23,
-// 6 x 2541 .. 7125 32.5 / 31.6, 8 x 700 14.7 / 12.7, 8 x 4000 32.1 / 31.4, 8 x 100 .. 16000 29.8 / 26.9, but 8 x 1420 .. 7184 35.8 / 36.7 and 8 x
+// longest): 1 x 700 12.5 / 7.0, 1 x 4000 18.1 / 10.3, 1 x 30000 39 / 28, 4 x 700 13.1 / 9.0, 4 x 16000 54.6 / 52.3, 4 x 100 .. 16000 33 / 23,
+// 6 x 2541 .. 7125 32.5 / 31.6, 8 x 700 13.7 / 12.9, 8 x 4000 31.2 / 30.2, 8 x 100 .. 16000 29.8 / 26.9, but 8 x 1420 .. 7184 35.8 / 36.7 and 8 x
 // 16000 92 / 98; 16 x 372 .. 7560 54 / 63.  So 48 pairs, and up to 64 where the table holds no more than 4096 tokens.  As many pieces as make 1024
 // workgroups, but no more than there is use for: 256 of them leave a compute unit's memory requests short (8 x 100 .. 16000 55), and more
 // records cost their sum (8 x 700 11.8 with 256).  Up to seven pairs 64 pieces, so that a long sequence meets the whole chip (1 x 120000, 8 heads on
-// 2, 51 / 37, with 32 pieces 55).
+// 2, 50 / 32, against 55 with 32 pieces).
 int few_decode_pieces(int64_t batch, int64_t num_kv_heads, int64_t max_tokens) {
     if (batch < 1 || num_kv_heads < 1 || batch > 64 || num_kv_heads > 64) return 0;
     const int64_t pairs = batch * num_kv_heads, p = 1024 / pairs, most = pairs < 8 ? kMostPieces : kMostPieces / 2;
@@ -389,7 +391,7 @@ int launch_few_decode(const FewDecode& a, hipStream_t stream, const FewFront* fr
     else hipLaunchKernelGGL(few_decode_kernel<false>, pieces, dim3(64 * kWaves), 0, stream, a, FewFront{});
     const int rc = (int)hipGetLastError();
     if (rc || !a.out) return rc;
-    const dim3 grid((unsigned)(a.group * a.num_kv_heads), (unsigned)a.batch), block(256);
+    const dim3 grid((unsigned)(a.group * a.num_kv_heads), (unsigned)a.batch), block(128);
     if (a.pieces <= 32) hipLaunchKernelGGL(few_decode_sum_kernel<4>, grid, block, 0, stream, a);
     else hipLaunchKernelGGL(few_decode_sum_kernel<8>, grid, block, 0, stream, a);
     return (int)hipGetLastError();

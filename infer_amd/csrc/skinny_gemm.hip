@@ -374,14 +374,14 @@ __global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSourc
 
 // A product, split over k, of one sequence's attention that still lies in pieces (decode_few.h): a workgroup has up to kPieceHeads heads of k, whose pieces
 // it adds up while its weights are on their way: a launch less in every layer, and what the pieces cost is a read of the second-level cache.  A step
-// of 28 layers of a 0.6B model, 700 tokens, 779 -> 751 us.  Sums, order and roundings are those of few_decode_sum_kernel and of skinny_stream_kernel:
+// of 28 layers of a 0.6B model, 700 tokens, 779 -> 731 us (751 with the pieces added up eight by eight, a chain of eleven sums instead of seven).  Sums, order and roundings are those of few_decode_sum_kernel and of skinny_stream_kernel:
 // the same bits.
-constexpr int kPieceHeads = 4, kPieceSets = 4;                      // heads of a workgroup; sets of eight pieces of a head
+constexpr int kPieceHeads = 4, kPieceSets = 4;                      // heads of a workgroup; sets of four pairs of pieces of a head
 __global__ void __launch_bounds__(256) piece_product_kernel(GemmArgs a, FewDecode f) {
     constexpr int NW = 4, D = 4, kRing = D * stream_stage_bytes(1, 0);
     __shared__ __attribute__((aligned(1024))) unsigned char lds[NW * kRing];
-    __shared__ f32x4 sums[4][kPieceHeads][32];
-    __shared__ float2 mls[4][kPieceHeads];
+    __shared__ f32x4 sums[2][kPieceHeads][32];
+    __shared__ float2 mls[2][kPieceHeads];
     __shared__ __attribute__((aligned(16))) __bf16 xs[kPieceHeads * kKC];
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n0 = blockIdx.x * 16, split = blockIdx.y;
@@ -391,32 +391,30 @@ __global__ void __launch_bounds__(256) piece_product_kernel(GemmArgs a, FewDecod
         const int row = n0 + stream_row() + 8 * i;
         w[i] = (const __bf16*)a.w + (int64_t)(row < a.n ? row : a.n - 1) * a.k + (int64_t)split * a.chunks * kKC;
     }
-    // 32 lanes hold the columns of a head, the workgroup's halves the pieces p with p % 8 below 4 and the others
+    // 32 lanes hold the columns of a head, the workgroup's halves two of the four parts of the pieces each
     const int c = threadIdx.x & 31, in = (threadIdx.x >> 5) & 3, half = threadIdx.x >> 7;
     const int head = split * a.chunks + (in < a.chunks ? in : 0), kv = head / f.group, q = head - kv * f.group, floats = few_record_floats(f.group);
     const float* rec = f.rec + (int64_t)kv * f.pieces * floats;
-    f32x4 v[4][kPieceSets];
-    float2 ml[4][kPieceSets];
+    f32x4 v[2][kPieceSets][2];
+    float2 ml[2][kPieceSets][2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < kPieceSets; ++i) {
-            const int p = 4 * half + j + 8 * i;
-            const float* from = rec + (int64_t)(p < f.pieces ? p : 0) * floats;
-            v[j][i] = *reinterpret_cast<const f32x4*>(from + q * kKC + 4 * c);
-            ml[j][i] = *reinterpret_cast<const float2*>(from + f.group * kKC + 2 * q);
-        }
+        for (int i = 0; i < kPieceSets; ++i)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int p = few_piece(2 * half + j, i, e);
+                const float* from = rec + (int64_t)(p < f.pieces ? p : 0) * floats;
+                v[j][i][e] = *reinterpret_cast<const f32x4*>(from + q * kKC + 4 * c);
+                ml[j][i][e] = *reinterpret_cast<const float2*>(from + f.group * kKC + 2 * q);
+            }
     const int pieces = few_pieces_of(f, f.ctx[0]);
     auto add = [&] {
-        f32x4 num[4];
-        float2 s[4];
+        f32x4 num[2];
+        float2 s[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            num[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            s[j] = make_float2(-INFINITY, 0.f);
-#pragma unroll
-            for (int i = 0; i < kPieceSets; ++i)
-                if (4 * half + j + 8 * i < pieces) few_add(num[j], s[j], v[j][i], ml[j][i]);
+        for (int j = 0; j < 2; ++j) {
+            few_part<kPieceSets>(num[j], s[j], 2 * half + j, pieces, v[j], ml[j]);
             if (half) {
                 sums[j][in][c] = num[j];
                 if (c == 0) mls[j][in] = s[j];
@@ -424,9 +422,10 @@ __global__ void __launch_bounds__(256) piece_product_kernel(GemmArgs a, FewDecod
         }
         __syncthreads();
         if (!half) {
+            if (2 < pieces) few_add(num[0], s[0], num[1], s[1]);
 #pragma unroll
-            for (int j = 1; j < 8; ++j)
-                if (j < pieces) few_add(num[0], s[0], j < 4 ? num[j < 4 ? j : 0] : sums[j & 3][in][c], j < 4 ? s[j < 4 ? j : 0] : mls[j & 3][in]);
+            for (int j = 2; j < 4; ++j)
+                if (2 * j < pieces) few_add(num[0], s[0], sums[j - 2][in][c], mls[j - 2][in]);
             const float inv = s[0].y > 0.f ? 1.f / s[0].y : 0.f;
             bf16x4_t o;
 #pragma unroll
@@ -688,8 +687,9 @@ extern "C" int infer_norm_product_bf16(const void* x, int64_t x_stride0, const f
 
 // The split over k of a product of `hidden` rows past one sequence's attention in pieces, or 0 where the pieces are added up first.  A workgroup
 // reads the pieces of its heads, 65 KB of four, which has to cost less than a launch, and none may wait for another's compute unit.  Attention with its
-// front and the product, us, three launches / two, for 20, 700, 4000 and 20000 tokens: 16 heads on 8, 1024 rows 9.3 / 8.6, 10.7 / 9.6, 12.7 / 12.2, 24.2 / 23.5;
-// 32 on 16, 512 rows 9.9 / 9.1, 10.9 / 10.1, 17.0 / 16.3, 36.7 / 35.9; but 24 on 8, 768 rows, 288 workgroups 9.7 / 9.9, 10.9 / 11.4, 13.5 / 14.0.
+// front and the product, us, three launches / two, for 20, 700, 4000 and 20000 tokens: 16 heads on 8, 1024 rows 9.4 / 8.8, 11.1 / 9.5, 14.4 / 13.0, 26.2 / 24.7;
+// 32 on 16, 512 rows 10.2 / 9.2, 11.9 / 10.4, 17.7 / 16.3, 39.4 / 38.2; but 24 on 8, 768 rows, 288 workgroups, with a sum some 0.8 longer, 9.7 / 9.9, 10.9 / 11.4,
+// 13.5 / 14.0.
 int few_product_splits(int64_t batch, int64_t num_q_heads, int64_t pieces, int64_t hidden) {
     const int64_t k = num_q_heads * kKC;
     if (batch != 1 || pieces < 1 || pieces > 8 * kPieceSets || hidden < 8 || hidden % 8 || hidden > 5120 || rows_per_workgroup(1, hidden, k) != 16) return 0;

@@ -69,6 +69,19 @@ def test_batches_on_either_side_of_the_rule_agree(gpu):
     _check(*wide, lens[:8])
 
 
+@pytest.mark.parametrize("hq,hkv,most", [(16, 8, 1024), (8, 8, 1024), (8, 4, 2048), (24, 12, 1024), (32, 16, 1024)])
+def test_one_sequence_has_the_bits_of_the_general_kernels(gpu, hq, hkv, most):
+    """Up to a wavefront per step of 32 tokens both leave the same partial results, and add them up in one order with the same roundings."""
+    gen = torch.Generator().manual_seed(hq + hkv)
+    for length in (1, 32, 33, 64, 65, 127, 129, 250, 257, 700, most - 31, most):
+        q, k, v, table, ctx = _inputs(gen, [length], hq, hkv, 256)
+        got, want, ws = torch.empty_like(q), torch.empty_like(q), ops.decode_workspace(q.device, 1, hq, hkv, 128)
+        ops.paged_attn_decode(q, k, v, table, ctx, 0.09, got)
+        ops.paged_attn_decode_split(q, k, v, table, ctx, 0.09, ws)
+        ops.paged_attn_decode_merge(want, ctx, hkv, ws)
+        assert torch.equal(got, want), length
+
+
 def test_what_lies_behind_the_end_is_not_looked_at(gpu):
     """Stale NaN in keys and values behind a length, ids out of range behind the last block, a length beyond the table."""
     gen = torch.Generator().manual_seed(6)
