@@ -142,6 +142,7 @@ struct ChunkArgs {
     const Span* spans;
     int seg_len, max_seg, slabs;                 // most tokens of a segment (a multiple of kC), segments of the longest span
     float* ws;                                   // [span][max_seg][heads][dim_pad][vdim_pad], if max_seg > 1
+    Turns turns;
 };
 
 // sum of the products of pieces i of x and j of y with i + j < MOST, the small ones first
@@ -194,7 +195,8 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
-    const Span span = args.spans[blockIdx.z];
+    const int portion = portion_of_turn(&args.spans->row0, args.turns, blockIdx.z);
+    const Span span = args.spans[portion];
     const int seg_len = own_segment(span.count, args.seg_len, kC), first = seg * seg_len;
     if (span.slot < 0 || span.slot >= a.num_slots || first >= span.count) return;
     const bool last_seg = first + seg_len >= span.count;
@@ -208,7 +210,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     float* from = a.state + ((int64_t)span.slot * a.heads + h) * state_len;
     float* to = from;
     if (args.max_seg > 1) {
-        float* ws = args.ws + (((int64_t)blockIdx.z * args.max_seg + seg) * a.heads + h) * state_len;
+        float* ws = args.ws + (((int64_t)portion * args.max_seg + seg) * a.heads + h) * state_len;
         if (OUT) from = ws;
         else to = ws;
     }
@@ -1016,7 +1018,7 @@ extern "C" int infer_decay_attention(int elem, const void* proj, int64_t proj_st
                         return (int)INFER_KV_EWORKSPACE;
                     // a workgroup that has the whole head norms it, too
                     const bool finish = norm_per_head && slabs == 1 && finished == decode_rows && ptr_aligned(proj, 8) && g_off % 4 == 0;
-                    rc = run_chunks(ChunkArgs{a, b, finish, (const Span*)spans, (int)len, (int)n, slabs, workspace}, wide ? 8 : 4, num_spans, st);
+                    rc = run_chunks(ChunkArgs{a, b, finish, (const Span*)spans, (int)len, (int)n, slabs, workspace, n > 1 ? Turns{} : turns_of(num_spans, heads * slabs, rows - decode_rows)}, wide ? 8 : 4, num_spans, st);
                     if (finish) finished = rows;
                 }
             }

@@ -25,6 +25,7 @@
 // zero counts as zero and a portion that starts at position 0 starts from a zero state, so a slot needs no clearing
 // when another sequence takes it over.
 #include "pieces.h"
+#include "segments.h"
 
 #include <type_traits>
 
@@ -488,14 +489,14 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaArgs<T> a, const C
 // first operand the records hold in fragment order.
 template <int DT>
 __global__ void __launch_bounds__(256) delta_scan_kernel(const PortionDesc* portions, const ChunkDesc* chunks, const float* records,
-                                                         float* state, float* o, int heads, int vdim_pad) {
+                                                         float* state, float* o, int heads, int vdim_pad, Turns turns) {
     constexpr int dp = 16 * DT;
     constexpr int kShared = 48 * dp + 256 + dp;                  // floats of a record all wavefronts read
     extern __shared__ __attribute__((aligned(16))) float sh[];   // [2][kShared]
     const int tid = threadIdx.x, threads = blockDim.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane >> 4, m = lane & 15;
     const int h = blockIdx.y;
-    const PortionDesc p = portions[blockIdx.z];
+    const PortionDesc p = portions[portion_of_turn(&portions->chunk0, turns, blockIdx.z)];
     const int vt = blockIdx.x * (threads >> 6) + wave;
     const bool live = vt < vdim_pad / 16;
     const int64_t rec_len = record_floats(dp, vdim_pad);
@@ -636,13 +637,13 @@ __host__ __device__ constexpr int wide_buffer_units(int dt) { return 64 * (5 * d
 // serve eight that compute 460.
 template <class T, int DT>
 __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a, const PortionDesc* portions, const ChunkDesc* chunks,
-                                                                 const float* records, int slabs) {
+                                                                 const float* records, int slabs, Turns turns) {
     constexpr int dp = 16 * DT, KS = DT / 2, kShared = 49 * dp + 256, kPitch = 132;
     extern __shared__ __attribute__((aligned(16))) u32x4_t lds[];     // [2] buffers, then outputs [2][16][kPitch]
     float* outputs = reinterpret_cast<float*>(lds + 2 * wide_buffer_units(DT));
     const int tid = threadIdx.x, lane = tid & 63, vt = __builtin_amdgcn_readfirstlane(tid >> 6), q = lane >> 4, m = lane & 15;
     const int h = blockIdx.x;
-    const PortionDesc p = portions[blockIdx.y];
+    const PortionDesc p = portions[portion_of_turn(&portions->chunk0, turns, blockIdx.y)];
     const bool live = vt < slabs;
     const int vdim_pad = a.vdim_pad;
     const int64_t rec_len = record_floats(dp, vdim_pad);
@@ -903,7 +904,7 @@ int tiles_of(int dim) {        // row tiles of the state, rounded up to what the
 }
 
 template <int DT>
-int launch_scan(const PortionDesc* p, int64_t portions, const ChunkDesc* c, const float* records, float* state, float* o,
+int launch_scan(const PortionDesc* p, int64_t portions, int64_t tokens, const ChunkDesc* c, const float* records, float* state, float* o,
                 int heads, int vdim_pad, hipStream_t st) {
     const int slabs = vdim_pad / 16, waves = slabs < 4 ? slabs : 4;
     constexpr size_t lds = (size_t)2 * (49 * 16 * DT + 256) * sizeof(float);
@@ -913,12 +914,12 @@ int launch_scan(const PortionDesc* p, int64_t portions, const ChunkDesc* c, cons
         if (e != hipSuccess) return (int)e;
     }
     hipLaunchKernelGGL((delta_scan_kernel<DT>), dim3((unsigned)((slabs + waves - 1) / waves), (unsigned)heads, (unsigned)portions),
-                       dim3(64 * waves), lds, st, p, c, records, state, o, heads, vdim_pad);
+                       dim3(64 * waves), lds, st, p, c, records, state, o, heads, vdim_pad, turns_of(portions, (int64_t)heads * ((slabs + waves - 1) / waves), tokens));
     return (int)hipGetLastError();
 }
 
 template <class T, int DT>
-int launch_scan_wide(const DeltaArgs<T>& a, const PortionDesc* p, int64_t portions, const ChunkDesc* c, const float* records, hipStream_t st) {
+int launch_scan_wide(const DeltaArgs<T>& a, const PortionDesc* p, int64_t portions, int64_t tokens, const ChunkDesc* c, const float* records, hipStream_t st) {
     constexpr size_t lds = (size_t)2 * wide_buffer_units(DT) * 16 + 2 * 16 * 132 * sizeof(float);
     if (lds > 60 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_scan_wide_kernel<T, DT>),
@@ -926,7 +927,7 @@ int launch_scan_wide(const DeltaArgs<T>& a, const PortionDesc* p, int64_t portio
         if (e != hipSuccess) return (int)e;
     }
     hipLaunchKernelGGL((delta_scan_wide_kernel<T, DT>), dim3((unsigned)a.heads, (unsigned)portions), dim3(512), lds, st, a, p, c, records,
-                       a.vdim_pad / 16);
+                       a.vdim_pad / 16, turns_of(portions, a.heads, tokens));
     return (int)hipGetLastError();
 }
 
@@ -998,7 +999,7 @@ int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t nu
     const int64_t pairs = (int64_t)a.heads * num_portions;
     const bool small = a.dim_pad * a.vdim_pad <= 2048 && (a.vdim == 32 || a.vdim == 64);
     if (out4 && 2 * pairs > 256 && !(small && pairs > 256) && a.vdim_pad <= 128 && (a.dim_pad == 32 || a.dim_pad == 64 || a.dim_pad == 96 || a.dim_pad == 128)) {
-#define GO(N) case N: rc = launch_scan_wide<T, N>(a, portions, num_portions, chunks, records, st); break
+#define GO(N) case N: rc = launch_scan_wide<T, N>(a, portions, num_portions, rows, chunks, records, st); break
         switch (a.dim_pad / 16) { GO(2); GO(4); GO(6); GO(8); }
 #undef GO
         if (rc) return rc;
@@ -1009,7 +1010,7 @@ int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t nu
             hipLaunchKernelGGL((delta_ring_kernel<T, 1>), dim3(groups, (unsigned)((a.channels + 255) / 256)), dim3(256), 0, st, a, row0, rows, ring_slot, positions);
         return (int)hipGetLastError();
     }
-#define GO(N) case N: rc = launch_scan<N>(portions, num_portions, chunks, records, a.state, o, a.heads, a.vdim_pad, st); break
+#define GO(N) case N: rc = launch_scan<N>(portions, num_portions, rows, chunks, records, a.state, o, a.heads, a.vdim_pad, st); break
     switch (a.dim_pad / 16) { GO(1); GO(2); GO(3); GO(4); GO(6); GO(8); GO(12); GO(16); default: return INFER_KV_EUNSUPPORTED; }
 #undef GO
     if (rc) return rc;

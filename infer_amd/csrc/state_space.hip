@@ -271,6 +271,7 @@ struct ChunkArgs {
     int seg_len, max_seg, slabs;                 // most tokens of a segment (a multiple of kC), segments of the longest span
     float* ws;                                   // [span][max_seg][heads][state][vdim], then [span][max_seg][heads]: log2 of the decay
     float* ws_decay;
+    Turns turns;
 };
 
 // A workgroup serves one head and 64 columns of its state over the chunks of one segment.  Wavefront w owns 16 columns as accumulators, of
@@ -302,7 +303,8 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2, cw = wave & 3;
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
-    const Span span = args.spans[blockIdx.z];
+    const int portion = portion_of_turn(&args.spans->row0, args.turns, blockIdx.z);
+    const Span span = args.spans[portion];
     const int seg_len = own_segment(span.count, args.seg_len, kC), first = seg * seg_len;
     if (span.slot < 0 || span.slot >= a.num_slots || first >= span.count) return;
     const bool last_seg = first + seg_len >= span.count;
@@ -314,7 +316,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
     const int64_t state_len = (int64_t)N * a.vdim;
     float* from = a.state + ((int64_t)span.slot * a.heads + h) * state_len;
     float* to = from;
-    const int64_t rec = ((int64_t)blockIdx.z * args.max_seg + seg) * a.heads + h;
+    const int64_t rec = ((int64_t)portion * args.max_seg + seg) * a.heads + h;
     if (args.max_seg > 1) {
         if (OUT) from = args.ws + rec * state_len;
         else to = args.ws + rec * state_len;
@@ -687,7 +689,8 @@ int portions(SsmArgs<T>& a, const Span* spans, int64_t num_spans, int64_t max_sp
     if constexpr (sizeof(T) == 2) {
         if (chunked(INFER_ELEM_BF16, a.vdim, a.state_n) && vec && a.y_stride % 4 == 0 && ptr_aligned(a.y, 8)) {
             const Walk walk = walk_of(a.heads, a.vdim, a.state_n, num_spans, max_span);
-            ChunkArgs c{a, spans, walk.seg_len, walk.max_seg, (a.vdim + kSlab - 1) / kSlab, nullptr, nullptr};
+            const int slabs = (a.vdim + kSlab - 1) / kSlab;
+            ChunkArgs c{a, spans, walk.seg_len, walk.max_seg, slabs, nullptr, nullptr, walk.max_seg > 1 ? Turns{} : turns_of(num_spans, (int64_t)a.heads * slabs, rows)};
             if (c.max_seg > 1) {
                 const int64_t records = num_spans * c.max_seg * a.heads, len = (int64_t)a.state_n * a.vdim;
                 if (!ws || ws_floats < records * (len + 1)) return INFER_KV_EWORKSPACE;

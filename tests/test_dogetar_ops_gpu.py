@@ -433,6 +433,18 @@ def test_state_space_portions_are_cut_by_their_own_lengths(gpu, lens):
         close(m.state[i], want[i][1], 1e-2)
 
 
+@pytest.mark.parametrize("heads,lens", [(90, (40, 70, 40)), (65, (33, 60, 9, 33, 70)), (260, (30, 41))])
+def test_state_space_portions_that_take_turns(gpu, heads, lens):
+    """More workgroups than compute units: the longest portions go first, equal ones in their order, several to the first round or not even one."""
+    m = Ssm(np.random.default_rng(heads), (heads, 8, 16, 5 if heads < 90 else 2, 4, 1), torch.bfloat16)
+    x = [m.inputs(n) for n in lens]
+    got = m.run([(len(lens) - 1 - i, 0, a) for i, a in enumerate(x)])
+    for i, a in enumerate(x):
+        want, states = m.want(a)
+        close(torch.tensor(got[i]), want, 2e-2)
+        close(m.state[len(lens) - 1 - i], states, 1e-2)
+
+
 @pytest.mark.parametrize("shape", [SSM[2], (4, 72, 48, 2, 4, 2)])
 def test_state_space_of_many_portions_and_of_a_long_one(gpu, shape):
     """More workgroups than two per compute unit, walked by four wavefronts each instead of eight, and one portion of many segments."""

@@ -470,6 +470,35 @@ def test_delta_batch_that_fills_the_chip(gpu, dtype, heads, kv_heads, dim, vdim,
     assert torch.isnan(c0.state[2]).all()
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(90, 64, 64), (90, 24, 20), (260, 32, 80)])
+def test_delta_portions_that_take_turns(gpu, heads, dim, vdim):
+    """More workgroups than compute units: the longest portions go first, equal and empty ones in their order, several to the first round or not even one."""
+    lens = (37, 97, 37, 0, 40)
+    c = DeltaCase(heads, heads, dim, vdim, 4, sum(lens), torch.float32, slots=len(lens))
+    c.dt -= 2.0
+    chunks, portions, ring, pos, row = [], [], [], [], 0
+    for slot, k in enumerate(lens):
+        portions.append((len(chunks), -(-k // 16), slot, 0))
+        chunks += [(row + r, min(16, k - r), r, 0, slot, 0) for r in range(0, k, 16)]
+        ring += [(slot, k - 1 - r) for r in range(k)]
+        pos += range(k)
+        row += k
+    assert len(lens) * heads > 256 and row >= 8 * len(lens) ** 2
+    out = torch.full((row, heads * vdim), float("nan"), device="cuda")
+    ho.delta_chunks(c.s, dev(c.proj), c.beta_off, dev(c.decay), dev(c.gate), *c.weights, c.ring, c.state, dev(portions, torch.int32),
+                    dev(chunks, torch.int32), dev(ring, torch.int32), dev(pos, torch.int64), 0, out)
+    row, proj, decay, gate = 0, c.proj, c.decay, c.gate
+    for slot, k in enumerate(lens):
+        if k:
+            c.n, c.proj, c.decay, c.gate = k, proj[row:row + k], decay[row:row + k], gate[row:row + k]
+            want, want_state = c.want()
+            close(out[row:row + k], want, 3e-5)
+            close(c.state[slot][:, :dim, :vdim], want_state, 3e-5)
+        else:
+            assert (c.state[slot] == 0).all()
+        row += k
+
+
 def test_delta_empty_portions_and_chunks(gpu):
     """In front of the rows and behind them, in one workgroup per head: a portion without chunks keeps its slot's state, or clears it at the
     first position; a chunk without tokens changes nothing."""

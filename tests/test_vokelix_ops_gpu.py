@@ -423,6 +423,24 @@ def test_decay_portions_are_cut_by_their_own_lengths(gpu, kind, lens):
 
 
 @BYKIND
+@pytest.mark.parametrize("heads,lens", [(90, (40, 70, 40)), (65, (33, 64, 1, 33, 73)), (260, (30, 41))])
+def test_decay_portions_that_take_turns(gpu, kind, heads, lens):
+    """More workgroups than compute units: the longest portions go first, equal ones in their order, several to the first round or not even one."""
+    bf = torch.bfloat16
+    d = Decay(kind, tuple(1.0 - 2.0 ** -(2 + i % 9) for i in range(heads)), 16, 16, 16, bf, seed=heads)
+    x = rounded(d.inputs(sum(lens)), bf)
+    state, spans, row = d.state(len(lens)), [], 0
+    for i, n in enumerate(lens):
+        spans.append((row, n, len(lens) - 1 - i, 0))
+        row += n
+    out = d.run(x, state, None, None, 0, spans)
+    for row, n, slot, _ in spans:
+        want, end = d.want(x[row:row + n], 0, np.zeros((heads, 16, 16)), round_silu=True)
+        close(out[row:row + n], want, tol(bf, 1e-5))
+        d.check_state(state, slot, end, state_tol(d, bf))
+
+
+@BYKIND
 def test_decay_state_does_not_drift_over_many_steps(gpu, kind):
     """4000 decoded tokens of zeros: what is left of the state is decay^4000 of it to float precision."""
     d = Decay(kind, (1.0 - 1.1e-4, 0.9998), 32, 32, 32, torch.float32)
