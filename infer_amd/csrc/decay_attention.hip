@@ -164,6 +164,17 @@ __device__ __forceinline__ u32x4_t silu8(u32x4_t x) {
     for (int i = 0; i < 8; ++i) r[i] = (__bf16)silu_f(y[i]);
     return __builtin_bit_cast(u32x4_t, r);
 }
+__device__ __forceinline__ u32x2_t silu8(u32x2_t x) {            // of half as many
+    bf16x4_t r = __builtin_bit_cast(bf16x4_t, x);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (__bf16)silu_f((float)r[i]);
+    return __builtin_bit_cast(u32x2_t, r);
+}
+// A value that the compiler takes for a new one: what is computed from it is not kept in registers over the whole loop.
+__device__ __forceinline__ int renewed(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
 
 // A workgroup of four or eight wavefronts serves one head and 16 VT columns of its state per wavefront over the chunks of one segment.
 // Wavefront w owns the columns 16 VT w .. and their part of the state, DT tiles of 32 rows, as accumulators: lane (g, n)
@@ -174,12 +185,17 @@ __device__ __forceinline__ u32x4_t silu8(u32x4_t x) {
 // gate, too.
 // A portion takes as long as its chunks one after the other, and a chunk as long as one wavefront's instructions.  Eight wavefronts have half as many
 // each, and with two chunks in LDS one barrier a chunk instead of three.
+// PARTS = 2: 64 columns, and a wavefront has half of the state rows of its 16.  The second half adds up and writes the results.  That is twice as many
+// workgroups, two to a compute unit, so that lengths even out, and shorter chunks (1.9 us by itself, 2.4 with all rows), though q and k are brought
+// twice: 3 portions of 3292 tokens of 32 heads 295 -> 243 us, 6 of 900 to 3700 313 -> 269.  128 registers are all there are: with addresses kept over the loop
+// it spilt eight, whose reads wait for the next chunk's requests as well (325).
 __host__ __device__ constexpr int chunk_bufs(int waves) { return waves == 8 ? 2 : 1; }      // chunks in LDS
 
-template <int DT, int VT, int WAVES, int PC, bool OUT, bool FINISH>
-__global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs args) {
+template <int DT, int VT, int WAVES, int PARTS, int PC, bool OUT, bool FINISH>
+__global__ void __launch_bounds__(64 * WAVES, PARTS == 2 ? 4 : 2) decay_chunk_kernel(ChunkArgs args) {
+    static_assert(PARTS == 1 || (WAVES == 8 && VT == 1 && !FINISH), "who adds up and writes the results");
     constexpr int kRow = DT * 64 + 16, kMat = kC * kRow;         // bytes: a token of q or k, one piece of a chunk
-    constexpr int kThr = 64 * WAVES, kSlab = 16 * VT * WAVES;
+    constexpr int kThr = 64 * WAVES, kSlab = 16 * VT * WAVES / PARTS, NT = 2 * DT / PARTS;     // NT: tiles of 16 state rows per wavefront
     constexpr int kBufs = chunk_bufs(WAVES);
     constexpr int PQ = PC == 3 ? 2 : 1;                          // pieces of q
     constexpr int kVRow = 2 * kSlab + 16, kPRow = 2 * kC + 16, kPMat = kC * kPRow;
@@ -192,8 +208,11 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     unsigned char* qbuf = vbuf + kC * kVRow;                     // [PQ][kMat]
     unsigned char* pbufs = lds + kBufs * kBuf;                   // [kBufs][2][kPMat], OUT
     float* squares = reinterpret_cast<float*>(pbufs + kBufs * 2 * kPMat);                // [kBufs][WAVES][kC], OUT
+    f32x4_t* ybufs = reinterpret_cast<f32x4_t*>(pbufs + kBufs * 2 * kPMat);              // [kBufs][4][2][64], OUT in two parts
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cw = PARTS == 2 ? wave & 3 : wave, part = PARTS == 2 ? wave >> 2 : 0;
+    const bool adds = part == PARTS - 1;                         // up what the parts have and writes the results
+    const int r0 = part * 16 * NT;                               // this wavefront's first state row
     const int h = blockIdx.y, slab = blockIdx.x % args.slabs, seg = blockIdx.x / args.slabs;
     const int portion = portion_of_turn(&args.spans->row0, args.turns, blockIdx.z);
     const Span span = args.spans[portion];
@@ -203,7 +222,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     if (!OUT && last_seg) return;                                // nobody needs its final state yet
     const int count = last_seg ? span.count - first : seg_len;
     const int row0 = span.row0 + first, pos0 = span.pos0 + first, chunks = (count + kC - 1) / kC;
-    const int v0 = slab * kSlab + wave * 16 * VT;                // this wavefront's first column
+    const int v0 = slab * kSlab + cw * 16 * VT;                // this wavefront's first column
     const bool live = v0 < a.vdim_pad;
     const float log2d = a.decay[2 * a.heads + h];
     const int64_t state_len = (int64_t)a.dim_pad * a.vdim_pad;
@@ -216,9 +235,9 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     }
     const bool load = OUT && (args.max_seg > 1 || span.pos0 > 0);
 
-    f32x4_t s[2 * DT][VT];
+    f32x4_t s[NT][VT];
 #pragma unroll
-    for (int t = 0; t < 2 * DT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
             s[t][v] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -226,7 +245,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
             if (load && col < a.vdim_pad)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (16 * t + 4 * g + e < a.dim_pad) s[t][v][e] = from[(int64_t)(16 * t + 4 * g + e) * a.vdim_pad + col];
+                    if (r0 + 16 * t + 4 * g + e < a.dim_pad) s[t][v][e] = from[(int64_t)(r0 + 16 * t + 4 * g + e) * a.vdim_pad + col];
         }
 
     // entries behind the real sizes stay zero
@@ -248,17 +267,20 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
         u_src[i] = a.proj + (int64_t)(row0 + (u_tok[i] > 0 ? u_tok[i] : 0)) * a.proj_stride + h * a.dim;
         u_cs[i] = a.table + 2 * (u_pair[i] > 0 ? u_pair[i] : 0);
     }
+    constexpr int kVCols = PARTS == 2 ? 4 : 8;                   // columns of v that a thread brings, VT times
+    typedef typename std::conditional<PARTS == 2, u32x2_t, u32x4_t>::type vvec_t;
     int v_tok[VT], v_col[VT];
     const __bf16* v_src[VT];
 #pragma unroll
     for (int i = 0; i < VT; ++i) {
         const int x = tid + kThr * i;
-        v_tok[i] = x / (kSlab / 8);
-        v_col[i] = slab * kSlab + 8 * (x % (kSlab / 8));
+        v_tok[i] = x / (kSlab / kVCols);
+        v_col[i] = slab * kSlab + kVCols * (x % (kSlab / kVCols));
         v_src[i] = a.proj + (int64_t)(row0 + v_tok[i]) * a.proj_stride + a.v_off + h * a.vdim + (v_col[i] < a.vdim ? v_col[i] : 0);
     }
     const int64_t step = kC * a.proj_stride;
-    u32x4_t kreg[NU][2], qreg[NU][2], vreg[VT];
+    u32x4_t kreg[NU][2], qreg[NU][2];
+    vvec_t vreg[VT];
     f32x4_t creg[PC == 3 ? NU : 1][4];
     // requests chunk c, the one behind the last request; no branches, so that nothing waits for a request before its use
     auto fetch = [&](int c) {
@@ -285,7 +307,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
 #pragma unroll
         for (int i = 0; i < VT; ++i) {
             const int over = v_tok[i] > last ? v_tok[i] - last : 0;
-            vreg[i] = *reinterpret_cast<const u32x4_t*>(v_src[i] - over * a.proj_stride);
+            vreg[i] = *reinterpret_cast<const vvec_t*>(v_src[i] - over * a.proj_stride);
             v_src[i] += step;
         }
     };
@@ -332,9 +354,9 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
 #pragma unroll
         for (int i = 0; i < VT; ++i) {
             if (v_col[i] >= a.vdim) continue;
-            u32x4_t y = a.silu ? silu8(vreg[i]) : vreg[i];
-            if (v_tok[i] >= left) y = u32x4_t{0u, 0u, 0u, 0u};
-            *reinterpret_cast<u32x4_t*>(vbuf + at + v_tok[i] * kVRow + 2 * (v_col[i] - slab * kSlab)) = y;
+            vvec_t y = a.silu ? silu8(vreg[i]) : vreg[i];
+            if (v_tok[i] >= left) y = vvec_t{};
+            *reinterpret_cast<vvec_t*>(vbuf + at + v_tok[i] * kVRow + 2 * (v_col[i] - slab * kSlab)) = y;
         }
     };
 
@@ -358,7 +380,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     float chunk_decay = exp2f(kC * log2d);
 
 #pragma unroll
-    for (int t = 0; t < 2 * DT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int v = 0; v < VT; ++v)
 #pragma unroll
@@ -371,7 +393,10 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     u32x2_t gate[VT][2];                                         // of results, requested a chunk before they are there
     bf16x8_t vf[VT];                                             // values of tokens 8 g .. + 7, column n
     // what the chunk's own tokens add to its results, and their squares
+    // two workgroups of eight wavefronts share a compute unit if a lane has 128 registers: no address stays in one from chunk to chunk
+    auto place = [](int x) { return PARTS == 2 ? renewed(x) : x; };
     auto own_tokens = [&](int c) {
+        const int lane = place(tid & 63), g = lane >> 4, n = lane & 15;
         const unsigned char* pr = pbufs + c % kBufs * 2 * kPMat;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -381,6 +406,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
             float ss = 0.f;
 #pragma unroll
             for (int v = 0; v < VT; ++v) {
+                if constexpr (PARTS == 2) acc[v][t] += ybufs[((c % kBufs * 4 + cw) * 2 + t) * 64 + lane];
 #pragma unroll
                 for (int k = 1; k >= 0; --k) acc[v][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[v], pf[k], acc[v][t], 0, 0, 0);
 #pragma unroll
@@ -406,6 +432,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     };
     // results, with the norm over the head and the gate if nobody else does them
     auto results = [&](int c) {
+        const int g = place(lane) >> 4, n = place(lane) & 15;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             if (16 * t + n >= count - c * kC) continue;
@@ -440,6 +467,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     };
     // products of the chunk's queries with its keys and with the state
     auto queries = [&](int c) {
+        const int g = place(lane) >> 4, n = place(lane) & 15;
         const unsigned char *kc = kbuf + c % kBufs * kBuf, *qc = qbuf + c % kBufs * kBuf;
         // ---- d^(i-j) q_i k_j: rows are keys, columns queries; the tile above the diagonal is all zeros
         if (wave < 4) {
@@ -474,13 +502,13 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
             for (int t = 0; t < 2; ++t) acc[v][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         if (live)
 #pragma unroll
-            for (int j = 0; j < DT; ++j) {
+            for (int j = 0; j < NT / 2; ++j) {
                 bf16x8_t qf[2][PQ];
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int k = 0; k < PQ; ++k) {
-                        const unsigned char* qr = qc + k * kMat + (16 * t + n) * kRow + 64 * j + 8 * g;
+                        const unsigned char* qr = qc + k * kMat + (16 * t + n) * kRow + 2 * r0 + 64 * j + 8 * g;
                         const u32x2_t x = *reinterpret_cast<const u32x2_t*>(qr), y = *reinterpret_cast<const u32x2_t*>(qr + 32);
                         qf[t][k] = __builtin_bit_cast(bf16x8_t, u32x4_t{x[0], x[1], y[0], y[1]});
                     }
@@ -499,10 +527,14 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
 #pragma unroll
             for (int v = 0; v < VT; ++v)
 #pragma unroll
-                for (int t = 0; t < 2; ++t) acc[v][t] *= qw[t];
+                for (int t = 0; t < 2; ++t) {
+                    acc[v][t] *= qw[t];
+                    if (!adds) ybufs[((c % kBufs * 4 + cw) * 2 + t) * 64 + lane] = acc[v][t];
+                }
     };
     auto take_values = [&](int c) {
-        const unsigned char* vr = vbuf + c % kBufs * kBuf + (8 * g + (n >> 2)) * kVRow + (n & 3) * 8 + 32 * VT * wave;
+        const int g = place(lane) >> 4, n = place(lane) & 15;
+        const unsigned char* vr = vbuf + c % kBufs * kBuf + (8 * g + (n >> 2)) * kVRow + (n & 3) * 8 + 32 * VT * cw;
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
             const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(vr + 32 * v));
@@ -511,6 +543,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
         }
     };
     auto update = [&](int c) {
+        const int g = place(lane) >> 4, n = place(lane) & 15;
         const unsigned char* kc = kbuf + c % kBufs * kBuf;
         const int left = count - c * kC;
         if (left < kC) {
@@ -527,9 +560,9 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
             for (int i = 0; i < 8; ++i) x[i] *= vw[i];
             split_frags<3>(x, wf[v]);
         }
-        const unsigned char* kr = kc + (8 * g + (n >> 2)) * kRow + (n & 3) * 8;
+        const unsigned char* kr = kc + (8 * g + (n >> 2)) * kRow + (n & 3) * 8 + 2 * r0;
 #pragma unroll
-        for (int t = 0; t < 2 * DT; ++t) {
+        for (int t = 0; t < NT; ++t) {
             bf16x8_t kf[PC];
 #pragma unroll
             for (int k = 0; k < PC; ++k) {
@@ -573,7 +606,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
         // run, and, where results wait for the other wavefronts' squares, those of chunk c - 2.  Everything that is written between two barriers
         // was read last in front of the first.
         auto behind = [&](int c) {
-            if (!OUT || !live) return;
+            if (!OUT || !live || !adds) return;
             if (FINISH && c > 1) results(c - 2);
             if (c > 0) own_tokens(c - 1);
             if (FINISH && c > 0) request_gates(c - 1);
@@ -604,14 +637,14 @@ __global__ void __launch_bounds__(64 * WAVES, 2) decay_chunk_kernel(ChunkArgs ar
     }
     if (OUT && !last_seg) return;
 #pragma unroll
-    for (int t = 0; t < 2 * DT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
             const int col = v0 + 16 * v + n;
             if (col < a.vdim_pad)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (16 * t + 4 * g + e < a.dim_pad) to[(int64_t)(16 * t + 4 * g + e) * a.vdim_pad + col] = s[t][v][e];
+                    if (r0 + 16 * t + 4 * g + e < a.dim_pad) to[(int64_t)(r0 + 16 * t + 4 * g + e) * a.vdim_pad + col] = s[t][v][e];
         }
 }
 
@@ -840,8 +873,9 @@ bool chunks_fit(int elem, int64_t dim, int64_t vdim, int64_t rot_dims) {
 }
 int tiles_of(int64_t dim_pad) { return dim_pad <= 32 ? 1 : dim_pad <= 64 ? 2 : dim_pad <= 128 ? 4 : 8; }
 int column_tiles(int64_t dim_pad, int64_t vdim_pad) { return vdim_pad <= 64 || dim_pad > 128 ? 1 : 2; }    // per wavefront
-int slabs_of(int64_t dim_pad, int64_t vdim_pad) {
-    const int cols = 64 * column_tiles(dim_pad, vdim_pad);
+enum Walk { kFour, kEight, kHalves };       // wavefronts of a workgroup; eight with all state rows each, or with half of them
+int slabs_of(Walk walk, int64_t dim_pad, int64_t vdim_pad) {
+    const int cols = walk == kHalves ? 64 : 64 * column_tiles(dim_pad, vdim_pad);
     return (int)((vdim_pad + cols - 1) / cols);
 }
 // How portions are walked: wavefronts of a workgroup (eight_waves), and the most tokens of a segment.  Portions are cut where they do not fill the chip, into
@@ -854,31 +888,48 @@ int slabs_of(int64_t dim_pad, int64_t vdim_pad) {
 // up to 32: both cut into what fills the chip.  32 x 1 of 9000 207 / 196, 16 x 1 of 300 43 / 35.
 // to 159: four cut, eight walk whole or nearly so, which leaves the chip idle; it pays where portions are short.  16 x 8 of 100 to 600 70 / 58, but of 1000 to 3000
 // 220 / 257, and 32 x 4 of 1000 to 2500 185 / 210: up to 640 tokens.
-// to 255: whole portions take as long as the longest, cut ones as long as all tokens together, twice.  16 x 11 of 500 to 1500 160 / 137; of longer ones what
+// to 255: whole portions take as long as the longest, cut ones as long as all tokens together, twice (where halves() does not take them).  16 x 11 of 500 to 1500 160 / 137; of longer ones what
 // counts is how many workgroups as long as the longest all tokens would make: 32 x 6 of 900 to 3700, 134 of them, 331 / 316, of 200 to 4000, 100, 315 / 319,
 // 32 x 5 of 800 to 5000, 93, 350 / 395: from 110.
-// from 256: 32 x 8 of 1500 210 / 190, 32 x 10 of 800 to 1800 271 / 241, 16 x 16 of 200 to 1000 120 / 98, 32 x 20 of 300 to 900 222 / 205; but two workgroups of
-// four share a unit, and where there are more than two and a half rounds (32 x 30 of 200 to 500 189 / 192, 32 x 64 of 100 to 300 227 / 243), or workgroups are
-// little but their start (32 x 16 of 50 to 250 59 / 61), they are ahead.
+// from 256, in turns: 32 x 8 of 1500 205 / 186, 32 x 10 of 800 to 1800 233 / 227, 16 x 24 of 300 to 900 128 / 129, 32 x 12 of 100 to 1500 188 / 165; but two
+// workgroups of four share a unit, and from two rounds on they are ahead: 32 x 16 of 500 to 1000 182 / 190, of 50 to 250 47 / 52, 32 x 20 of 300 to 900 191 / 205,
+// 32 x 30 of 200 to 500 174 / 189, 32 x 64 of 100 to 300 228 / 244.
 bool eight_waves(int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t rot_dims, int64_t num_spans, int64_t max_span, int64_t tokens) {
-    const int64_t per_token = heads * slabs_of(dim_pad, vdim_pad), groups = per_token * num_spans;
-    if (column_tiles(dim_pad, vdim_pad) != 2 || rot_dims > 0 || groups > 640 || (groups > 384 && max_span <= 256)) return false;
+    const int64_t per_token = heads * slabs_of(kEight, dim_pad, vdim_pad), groups = per_token * num_spans;
+    if (column_tiles(dim_pad, vdim_pad) != 2 || rot_dims > 0 || groups > 384) return false;
     if (groups <= 32 || groups >= 256) return true;
     return groups < 160 ? max_span <= 640 : max_span <= 2048 || per_token * tokens >= 110 * max_span;
 }
-int64_t segment_len(bool wide, int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t num_spans, int64_t max_span) {
-    const int64_t groups = heads * slabs_of(dim_pad, vdim_pad) * num_spans, full = wide ? 128 : 256, most = max_span / (4 * kC);
+// Halves of the state rows, for twice as many workgroups (not behind a rotation, as above, and not where a workgroup norms the head it has).  Two of them on a
+// compute unit take 1.6 times as long as one that does both, so they pay as long as the chip's share of all tokens stays below the longest portion's: up to
+// 158 workgroups as long as the longest.  Best of the others / halves, us, heads x portions (workgroups as long as the longest): 32 x 7 of 1000 (224) 120 / 144,
+// 32 x 8 of 1500 (256) 186 / 227, 32 x 10 of 800 to 1800 (231) 227 / 259, but 32 x 8 of 500 to 2500 (154) 244 / 239, of 100 to 1500 (137) 147 / 135, 32 x 7 of 500 to
+// 2500 (134) 221 / 196, 16 x 15 of 300 to 2000 (138) 189 / 163, 24 x 6 of 200 to 700 64 / 54, 32 x 4 of 1000 to 2500 183 / 174, 16 x 8 of 100 to 600 57 / 48, 24 x 5 of
+// 800 to 2000 148 / 133, 16 x 7 of 300 to 1200 85 / 80.  Fewer workgroups than that cut long portions into segments that fill the chip anyway (32 x 3 of 500 to 3000
+// 160 / 179 whole or cut, 16 x 3 of 300 to 900 49 / 59, 32 x 1 of 2000 59 / 69), but up to 640 tokens halves are ahead there, too: 32 x 3 of 100 to 400 45 / 35,
+// 32 x 2 of 300 to 600 45 / 41, 32 x 1 of 600 41 / 36, 16 x 1 of 300 36 / 30.
+bool halves(int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t rot_dims, bool norm_per_head, int64_t num_spans, int64_t max_span, int64_t tokens) {
+    if (column_tiles(dim_pad, vdim_pad) != 2 || rot_dims > 0 || norm_per_head || dim_pad <= 32) return false;
+    const int64_t per_token = heads * slabs_of(kEight, dim_pad, vdim_pad);
+    return per_token * tokens <= 158 * max_span && (per_token * num_spans >= 112 || max_span <= 640);
+}
+Walk walk_of(int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t rot_dims, bool norm_per_head, int64_t num_spans, int64_t max_span, int64_t tokens) {
+    if (halves(heads, dim_pad, vdim_pad, rot_dims, norm_per_head, num_spans, max_span, tokens)) return kHalves;
+    return eight_waves(heads, dim_pad, vdim_pad, rot_dims, num_spans, max_span, tokens) ? kEight : kFour;
+}
+int64_t segment_len(Walk walk, int64_t heads, int64_t dim_pad, int64_t vdim_pad, int64_t num_spans, int64_t max_span) {
+    const int64_t groups = heads * slabs_of(walk, dim_pad, vdim_pad) * num_spans, full = walk == kFour ? 256 : 128, most = max_span / (4 * kC);
     int64_t n = groups >= full ? 1 : (2 * full + groups - 1) / groups;
     if (n > most) n = most;
     if (n < 1) n = 1;
     return ((max_span + n - 1) / n + kC - 1) / kC * kC;
 }
 
-template <int DT, int VT, int WAVES, int PC, bool OUT, bool FINISH = false>
+template <int DT, int VT, int WAVES, int PARTS, int PC, bool OUT, bool FINISH = false>
 int launch_chunk(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
-    const size_t lds = (size_t)kC * chunk_bufs(WAVES) * ((OUT ? PC == 3 ? 5 : 2 : PC) * (DT * 64 + 16) + 32 * VT * WAVES + 16 +
-                                     (OUT ? 2 * (2 * kC + 16) + WAVES * sizeof(float) : 0));
-    auto kernel = &decay_chunk_kernel<DT, VT, WAVES, PC, OUT, FINISH>;
+    const size_t lds = (size_t)kC * chunk_bufs(WAVES) * ((OUT ? PC == 3 ? 5 : 2 : PC) * (DT * 64 + 16) + 32 * VT * WAVES / PARTS + 16 +
+                                     (OUT ? 2 * (2 * kC + 16) + (PARTS == 2 ? 256 : WAVES * sizeof(float)) : 0));
+    auto kernel = &decay_chunk_kernel<DT, VT, WAVES, PARTS, PC, OUT, FINISH>;
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
@@ -887,38 +938,42 @@ int launch_chunk(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-template <int DT, int VT, int WAVES, int PC>
+template <int DT, int VT, int WAVES, int PARTS, int PC>
 int launch_pieces(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
     if (c.max_seg > 1) {
-        int rc = launch_chunk<DT, VT, WAVES, PC, false>(c, num_spans, st);
+        int rc = launch_chunk<DT, VT, WAVES, PARTS, PC, false>(c, num_spans, st);
         if (rc) return rc;
         const unsigned blocks = (unsigned)(((int64_t)c.a.dim_pad * c.a.vdim_pad / 4 + kThreads - 1) / kThreads);
         hipLaunchKernelGGL(decay_join_kernel, dim3(blocks, (unsigned)c.a.heads, (unsigned)num_spans), dim3(kThreads), 0, st, c);
         rc = (int)hipGetLastError();
         if (rc) return rc;
     }
-    return c.finish ? launch_chunk<DT, VT, WAVES, PC, true, true>(c, num_spans, st) : launch_chunk<DT, VT, WAVES, PC, true>(c, num_spans, st);
+    if constexpr (PARTS == 1)
+        if (c.finish) return launch_chunk<DT, VT, WAVES, 1, PC, true, true>(c, num_spans, st);
+    return launch_chunk<DT, VT, WAVES, PARTS, PC, true>(c, num_spans, st);
 }
 
-template <int DT, int VT, int WAVES>
+template <int DT, int VT, int WAVES, int PARTS = 1>
 int launch_chunks(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
     if constexpr (WAVES == 4)
-        if (c.a.rot_pairs > 0) return launch_pieces<DT, VT, 4, 3>(c, num_spans, st);
-    return launch_pieces<DT, VT, WAVES, 1>(c, num_spans, st);
+        if (c.a.rot_pairs > 0) return launch_pieces<DT, VT, 4, 1, 3>(c, num_spans, st);
+    return launch_pieces<DT, VT, WAVES, PARTS, 1>(c, num_spans, st);
 }
 
-// Columns of a workgroup are those of slabs_of(): 64, or 128 as four wavefronts with 32 or eight with 16.
+// Columns of a workgroup are those of slabs_of(): 64, or 128 as four wavefronts with 32 or eight with 16; in halves always 64.
 template <int DT>
-int run_tiles(const ChunkArgs& c, int waves, int64_t num_spans, hipStream_t st) {
+int run_tiles(const ChunkArgs& c, Walk walk, int64_t num_spans, hipStream_t st) {
     if (column_tiles(c.a.dim_pad, c.a.vdim_pad) == 1) return launch_chunks<DT, 1, 4>(c, num_spans, st);
-    return waves == 8 ? launch_chunks<DT, 1, 8>(c, num_spans, st) : launch_chunks<DT, 2, 4>(c, num_spans, st);
+    if constexpr (DT > 1)
+        if (walk == kHalves) return launch_chunks<DT, 1, 8, 2>(c, num_spans, st);
+    return walk == kEight ? launch_chunks<DT, 1, 8>(c, num_spans, st) : launch_chunks<DT, 2, 4>(c, num_spans, st);
 }
 
-int run_chunks(const ChunkArgs& c, int waves, int64_t num_spans, hipStream_t st) {
+int run_chunks(const ChunkArgs& c, Walk walk, int64_t num_spans, hipStream_t st) {
     switch (tiles_of(c.a.dim_pad)) {
-        case 1: return run_tiles<1>(c, waves, num_spans, st);
-        case 2: return run_tiles<2>(c, waves, num_spans, st);
-        case 4: return run_tiles<4>(c, waves, num_spans, st);
+        case 1: return run_tiles<1>(c, walk, num_spans, st);
+        case 2: return run_tiles<2>(c, walk, num_spans, st);
+        case 4: return run_tiles<4>(c, walk, num_spans, st);
         default: return launch_chunks<8, 1, 4>(c, num_spans, st);
     }
 }
@@ -957,8 +1012,8 @@ extern "C" int64_t infer_decay_workspace_floats(int elem, int64_t heads, int64_t
     int64_t pad[2];
     if (infer_decay_layout(dim, vdim, pad) || heads < 1 || num_spans < 1 || max_span < 1 || !chunks_fit(elem, dim, vdim, rot_dims)) return 0;
     int64_t n = 1;                                             // for both ways to walk: how many tokens there are is not known here
-    for (const bool wide : {false, true}) {
-        const int64_t len = segment_len(wide, heads, pad[0], pad[1], num_spans, max_span);
+    for (const Walk walk : {kFour, kEight, kHalves}) {
+        const int64_t len = segment_len(walk, heads, pad[0], pad[1], num_spans, max_span);
         n = std::max(n, (max_span + len - 1) / len);
     }
     return n > 1 ? num_spans * n * heads * pad[0] * pad[1] : 0;
@@ -1011,14 +1066,14 @@ extern "C" int infer_decay_attention(int elem, const void* proj, int64_t proj_st
                 chunked = chunks_fit(elem, dim, vdim, rot_dims) && (q_off | k_off | v_off | proj_stride) % 8 == 0 && ptr_aligned(proj, 16) &&
                           out_stride % 4 == 0 && ptr_aligned(out, 8) && ptr_aligned(table, 16);
                 if (chunked) {
-                    const int slabs = slabs_of(pad[0], pad[1]);
-                    const bool wide = eight_waves(heads, pad[0], pad[1], rot_dims, num_spans, max_span, rows - decode_rows);
-                    const int64_t len = segment_len(wide, heads, pad[0], pad[1], num_spans, max_span), n = (max_span + len - 1) / len;
+                    const Walk walk = walk_of(heads, pad[0], pad[1], rot_dims, norm_per_head != 0, num_spans, max_span, rows - decode_rows);
+                    const int slabs = slabs_of(walk, pad[0], pad[1]);
+                    const int64_t len = segment_len(walk, heads, pad[0], pad[1], num_spans, max_span), n = (max_span + len - 1) / len;
                     if (n > 1 && (!workspace || !ptr_aligned(workspace, 16) || workspace_floats < num_spans * n * heads * pad[0] * pad[1]))
                         return (int)INFER_KV_EWORKSPACE;
                     // a workgroup that has the whole head norms it, too
                     const bool finish = norm_per_head && slabs == 1 && finished == decode_rows && ptr_aligned(proj, 8) && g_off % 4 == 0;
-                    rc = run_chunks(ChunkArgs{a, b, finish, (const Span*)spans, (int)len, (int)n, slabs, workspace, n > 1 ? Turns{} : turns_of(num_spans, heads * slabs, rows - decode_rows)}, wide ? 8 : 4, num_spans, st);
+                    rc = run_chunks(ChunkArgs{a, b, finish, (const Span*)spans, (int)len, (int)n, slabs, workspace, n > 1 ? Turns{} : turns_of(num_spans, heads * slabs, rows - decode_rows)}, walk, num_spans, st);
                     if (finish) finished = rows;
                 }
             }

@@ -476,6 +476,26 @@ def test_decay_workgroups_of_four_and_of_eight_wavefronts(gpu, kind, vdim, heads
         d.check_state(state, i, end, state_tol(d, bf))
 
 
+@pytest.mark.parametrize("dim,vdim", [(64, 72), (96, 128), (128, 200), (48, 128)])
+@pytest.mark.parametrize("heads,lens", [(3, (257,)), (12, (600, 33, 96)), (40, (100, 1, 31, 32)), (60, (160, 33, 64, 1, 40))])
+def test_decay_halves_of_the_state_rows(gpu, dim, vdim, heads, lens):
+    """Workgroups of 64 columns whose wavefronts have half of the state rows: cut and whole portions, in turns, columns that only some wavefronts have."""
+    bf = torch.bfloat16
+    d = Decay("lightning", tuple(1.0 - 2.0 ** -(2 + i % 9) for i in range(heads)), dim, vdim, 0, bf, seed=heads + dim)
+    x = rounded(d.inputs(sum(lens)), bf)
+    state, spans, row = d.state(len(lens)), [], 0
+    starts = [d.rng.standard_normal((heads, dim, vdim)) if i % 2 else np.zeros((heads, dim, vdim)) for i in range(len(lens))]
+    for i, n in enumerate(lens):
+        d.fill(state, i, starts[i])
+        spans.append((row, n, i, 7 * (i % 2)))
+        row += n
+    out = d.run(x, state, None, None, 0, spans)
+    for row, n, i, pos0 in spans:
+        want, end = d.want(x[row:row + n], pos0, starts[i], round_silu=True)
+        close(out[row:row + n], want, tol(bf, 1e-5))
+        d.check_state(state, i, end, state_tol(d, bf))
+
+
 @pytest.mark.parametrize("kind", ["lightning", "plain"])
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("heads,lens", [(12, (700, 33, 96)), (44, (20, 3, 40, 33, 5, 32, 2, 64, 65, 31))])
