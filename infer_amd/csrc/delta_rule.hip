@@ -273,6 +273,27 @@ __device__ __forceinline__ float softplus_log2(float z) {
 // Decay of a whole chunk, in log2 units, up to which e^{G_i - G_j} may be split into two factors.
 constexpr float kSplitRange = 48.f;
 
+// x summed over the rows of 16 lanes of a wavefront, and over the 32 lanes of its halves, in all of them
+__device__ __forceinline__ float row_sum(float x) {
+    auto ror = [](float v, auto C) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(C)::value, 0xf, 0xf, false)); };
+    x += ror(x, std::integral_constant<int, 0x128>{});          // rotations by 8, 4, 2 and 1
+    x += ror(x, std::integral_constant<int, 0x124>{});
+    x += ror(x, std::integral_constant<int, 0x122>{});
+    x += ror(x, std::integral_constant<int, 0x121>{});
+    return x;
+}
+__device__ __forceinline__ float half_sum(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, row_sum(x));
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned lo = r[0], hi = r[1];
+    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float x) {
+    static_assert(LANES == 16 || LANES == 32, "lanes");
+    return LANES == 16 ? row_sum(x) : half_sum(x);
+}
+
 // VEC: four channels at a time, four taps; otherwise any size, one element at a time.
 template <class T, bool VEC>
 __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaArgs<T> a, const ChunkDesc* chunks, float* records) {
@@ -484,6 +505,235 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaArgs<T> a, const C
     }
 }
 
+// The same for bf16 heads of dim = vdim = 16 DT and four taps.  A record of 34 KB and 8 KB of inputs for a chunk and head of 128 pass through memory, which
+// bounds it (4.6 TB/s; without the records' way to memory the call takes 66 us less).  The general form is bound by how long a chunk takes, of which four
+// fit a compute unit: here three wavefronts convolve while the fourth does the gates and adds them up token by token in registers, the lengths of k and q
+// come out of the pass that scales them, and sizes are constants.  8 portions of 500 to 2600 tokens, 32 heads of 128: the call 807 -> 735 us.  (Two, four
+// or eight chunks one after the other in a workgroup, the next one's inputs requested ahead: 744, 752, 769.)
+template <int DT>
+__global__ void __launch_bounds__(256, 4) delta_prep_square_kernel(DeltaArgs<__bf16> a, const ChunkDesc* chunks, float* records) {
+    constexpr int D = 16 * DT, P = D + 4, ND = D / 4, kConv = 6 * ND, CD = D / 64;      // CD: channels of a lane of the fourth wavefront
+    static_assert(DT == 4 || DT == 8, "lanes of the gates, items of the convolution, halves of a wavefront per token");
+    extern __shared__ __attribute__((aligned(16))) float sh[];
+    float* qs = sh;                    // [16][P] q, then e^G q / |q|
+    float* ks = qs + kC * P;           // [16][P] k, then e^G k / |k|
+    float* gs = ks + kC * P;           // [16][P] running log2 decay G, then e^{G_last - G} k / |k|
+    float* vs = gs + kC * P;           // [16][P]
+    float* pp = vs + kC * P;           // [2][2][256] products of the token pairs (k k, q k), in two parts each
+    float* lt = pp + 1024;             // [16][20] column s: beta * A of the tokens behind s
+    float* tb = lt;                    // [16][20] T * beta, when those have been used
+    float* gl = lt + kC * 20;          // [D] G_last
+    float* gi = gl + D;                // [D] e^{-G_last}
+    float* inv = gi + D;               // [2][16] 1 / length of k and q
+    float* bs = inv + 32;              // [16] beta
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.y;
+    const int lq = lane >> 4, lm = lane & 15, i = tid >> 4, j = tid & 15;
+    const ChunkDesc c = chunks[blockIdx.x];
+    const int row0 = c.count > 0 ? c.row0 : 0;                   // what an empty chunk reads is not used, and row 0 exists
+    float* rec = records + ((int64_t)blockIdx.x * a.heads + h) * record_floats(D, D);
+    const int group = a.heads / a.kv_heads, kvh = h / group;
+    const float rate = expf(a.a_log[h]);
+    const bool gates = wave == 3;
+    // item of the convolution: matrix, four channels, half of the tokens
+    const int item = tid < kConv ? tid : 0, t0 = 8 * (item / (3 * ND)), matrix = item / ND % 3, col = 4 * (item % ND);
+    const int channel = col + (matrix == 0 ? kvh * D : matrix == 1 ? (a.kv_heads + kvh) * D : 2 * a.kv_heads * D + h * D);
+    float* const conv_to = (matrix == 0 ? qs : matrix == 1 ? ks : vs) + t0 * P + col;
+    const int d0 = CD * lane;
+    float w[4][4], dt[CD];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) load_elems<4>(a.conv + 4 * (channel + e), w[e]);
+#pragma unroll
+    for (int e = 0; e < CD; ++e) dt[e] = a.dt_bias[h * D + d0 + e];
+
+    // Inputs: of the convolution tokens t0 - 3 .. t0 + 7, of the gates 16 tokens and a logit of the write strength
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 raw[11];
+    if (gates) {
+        const __bf16* src = a.decay + (int64_t)row0 * a.decay_stride + h * D + d0;
+        const int last = c.count > 0 ? c.count - 1 : 0;      // tokens behind the last one re-read it
+#pragma unroll
+        for (int t = 0; t < kC; ++t) {
+            const __bf16* p = src + (t < last ? t : last) * a.decay_stride;
+            raw[t / 2][t & 1] = CD == 2 ? *reinterpret_cast<const uint32_t*>(p) : *reinterpret_cast<const uint16_t*>(p);
+        }
+        raw[8][0] = *reinterpret_cast<const uint16_t*>(a.proj + (int64_t)(row0 + ((lane & 15) < last ? lane & 15 : last)) * a.proj_stride + a.beta_off + h);
+    } else if (c.count == kC && c.pos0 - 3 >= c.first_pos) {
+        const __bf16* src = a.proj + (int64_t)(row0 + t0 - 3) * a.proj_stride + channel;
+#pragma unroll
+        for (int x = 0; x < 11; ++x, src += a.proj_stride) raw[x] = *reinterpret_cast<const u32x2*>(src);
+    } else {
+#pragma unroll
+        for (int x = 0; x < 11; ++x) {
+            const int t = t0 + x - 3, p = c.pos0 + t;
+            // positions before the portion are in the ring; those before the sequence or behind the chunk's tokens are zero
+            const bool in = p >= 0 && t < c.count;
+            raw[x] = *reinterpret_cast<const u32x2*>(p >= c.first_pos || !in ? a.proj + (int64_t)(row0 + (in ? t : 0)) * a.proj_stride + channel
+                                                                             : a.ring + ((int64_t)c.slot * 4 + (p & 3)) * a.channels + channel);
+            if (!in) raw[x] = u32x2{0u, 0u};
+        }
+    }
+    int strong = 0;
+    if (gates) {
+        float sum[CD];
+#pragma unroll
+        for (int e = 0; e < CD; ++e) sum[e] = 0.f;
+#pragma unroll
+        for (int t = 0; t < kC; ++t)
+#pragma unroll
+            for (int e = 0; e < CD; ++e) {
+                const uint32_t bits = raw[t / 2][t & 1];
+                const float z = __builtin_bit_cast(float, e == 1 ? bits & 0xffff0000u : bits << 16) + dt[e], g = -rate * softplus_log2(z);
+                sum[e] += t < c.count ? g : 0.f;
+                gs[t * P + d0 + e] = sum[e];
+            }
+#pragma unroll
+        for (int e = 0; e < CD; ++e) {
+            gl[d0 + e] = sum[e];
+            gi[d0 + e] = __builtin_amdgcn_exp2f(-sum[e]);
+            strong |= sum[e] < -kSplitRange;
+        }
+        if (lane < kC) bs[lane] = lane < c.count ? sigmoid_f(__builtin_bit_cast(float, raw[8][0] << 16)) : 0.f;
+    } else if (tid < kConv) {
+        float x[4][4];                             // rows of the window, each in its place for four tokens
+        auto widen_row = [&](int r) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[r & 3][e] = __builtin_bit_cast(float, e & 1 ? raw[r][e / 2] & 0xffff0000u : raw[r][e / 2] << 16);
+        };
+#pragma unroll
+        for (int r = 0; r < 3; ++r) widen_row(r);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            widen_row(t + 3);
+            f32x4_t y;
+            const bool in = t0 + t < c.count;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float s = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) s += w[e][k] * x[(t + k) & 3][e];
+                y[e] = in ? silu_f(s) : 0.f;
+            }
+            *reinterpret_cast<f32x4_t*>(conv_to + t * P) = y;
+            if (t & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    strong = __syncthreads_or(strong);
+    float akk = 0.f, aqk = 0.f;                    // products of token pair (i, j)
+    if (strong) {
+        if (j <= i) {
+            // some channel decays so much over the chunk that only differences of G can be exponentiated
+            const float *ki = ks + i * P, *qi = qs + i * P, *gi_ = gs + i * P, *kj = ks + j * P, *gj = gs + j * P;
+            for (int d = 0; d < D; d += 4) {
+                const f32x4_t k1 = *reinterpret_cast<const f32x4_t*>(ki + d), q1 = *reinterpret_cast<const f32x4_t*>(qi + d);
+                const f32x4_t g1 = *reinterpret_cast<const f32x4_t*>(gi_ + d), k2 = *reinterpret_cast<const f32x4_t*>(kj + d);
+                const f32x4_t g2 = *reinterpret_cast<const f32x4_t*>(gj + d);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v = k2[e] * __builtin_amdgcn_exp2f(g1[e] - g2[e]);
+                    akk += k1[e] * v;
+                    aqk += q1[e] * v;
+                }
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int x = 0; x < kC * ND / 256; ++x) {      // ND lanes side by side hold a token
+        const int t = (tid + 256 * x) / ND, d = 4 * (tid % ND);
+        f32x4_t* gp = reinterpret_cast<f32x4_t*>(gs + t * P + d);
+        f32x4_t* kp = reinterpret_cast<f32x4_t*>(ks + t * P + d);
+        f32x4_t* qp = reinterpret_cast<f32x4_t*>(qs + t * P + d);
+        const f32x4_t last = *reinterpret_cast<const f32x4_t*>(gl + d);
+        f32x4_t g = *gp, k = *kp, q = *qp;
+        float sk = (k[0] * k[0] + k[1] * k[1]) + (k[2] * k[2] + k[3] * k[3]), sq = (q[0] * q[0] + q[1] * q[1]) + (q[2] * q[2] + q[3] * q[3]);
+        sk = lanes_sum<ND>(sk);
+        sq = lanes_sum<ND>(sq);
+        const float ik = rsqrtf(sk + 1e-6f), iq = rsqrtf(sq + 1e-6f) * a.q_scale;
+        if (tid % ND == 0) { inv[t] = ik; inv[16 + t] = iq; }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float up = __builtin_amdgcn_exp2f(g[e]), kn = k[e] * ik;
+            g[e] = kn * __builtin_amdgcn_exp2f(last[e] - g[e]);
+            k[e] = kn * up;
+            q[e] *= up * iq;
+        }
+        *gp = g; *kp = k; *qp = q;
+    }
+    __syncthreads();
+    if (!strong) {
+        // A_ij = sum_d (k_i e^{G_i - G_last}) (k_j e^{G_last - G_j}) on the matrix pipe: wavefronts 0 and 1 take half of the
+        // channels each, 2 and 3 do the same for q
+        f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+        const float* left = (wave < 2 ? ks : qs) + lm * P;
+#pragma unroll
+        for (int x = 0; x < DT / 2; ++x) {
+            const int d = 16 * (2 * x + (wave & 1)) + 4 * lq;
+            const f32x4_t x1 = *reinterpret_cast<const f32x4_t*>(left + d) * *reinterpret_cast<const f32x4_t*>(gi + d);
+            const f32x4_t k2 = *reinterpret_cast<const f32x4_t*>(gs + lm * P + d);
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1[e], k2[e], acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1[e + 1], k2[e + 1], acc1, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pp[wave * 256 + (4 * lq + e) * 16 + lm] = acc0[e] + acc1[e];    // row: token i, column: token j
+        __syncthreads();
+        akk = pp[tid] + pp[256 + tid];
+        aqk = pp[512 + tid] + pp[768 + tid];
+    } else {
+        akk *= inv[i] * inv[j];
+        aqk *= inv[16 + i] * inv[j];
+    }
+    lt[j * 20 + i] = j < i ? bs[i] * akk : 0.f;
+    rec[48 * D + ((j >> 2) * 16 + i) * 4 + (j & 3)] = j <= i ? aqk : 0.f;
+    __syncthreads();
+    if (wave == 0) {
+        // T = (I + L)^-1 column by column: lane m holds column m, row s is final when it is used
+        float t[kC];
+#pragma unroll
+        for (int r = 0; r < kC; ++r) t[r] = r == lm ? 1.f : 0.f;
+#pragma unroll
+        for (int s = 0; s < kC - 1; ++s)
+#pragma unroll
+            for (int r4 = 0; r4 < kC; r4 += 4)
+                if (r4 + 3 > s) {
+                    const f32x4_t l = *reinterpret_cast<const f32x4_t*>(lt + s * 20 + r4);      // zero for rows up to s
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (r4 + e > s) t[r4 + e] -= l[e] * t[s];
+                }
+        if (lane < kC) {
+            const float b = bs[lm];
+#pragma unroll
+            for (int r = 0; r < kC; ++r) tb[r * 20 + lm] = t[r] * b;
+        }
+    } else {
+        for (int t = wave - 1; t < DT; t += 3) {
+            f32x4_t k;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) k[e] = gs[(4 * lq + e) * P + 16 * t + lm];
+            *reinterpret_cast<f32x4_t*>(rec + 16 * D + 256 * t + 4 * lane) = *reinterpret_cast<const f32x4_t*>(qs + lm * P + 16 * t + 4 * lq);
+            *reinterpret_cast<f32x4_t*>(rec + 32 * D + 256 * t + 4 * lane) = k;
+        }
+        if (tid - 64 < D) rec[48 * D + 256 + tid - 64] = __builtin_amdgcn_exp2f(gl[tid - 64]);
+    }
+    __syncthreads();
+    const f32x4_t tv = *reinterpret_cast<const f32x4_t*>(tb + lm * 20 + 4 * lq);       // T beta, row lm
+#pragma unroll
+    for (int x = 0; x < DT / 4; ++x) {             // W^T = (e^G K)^T (T beta)^T: row d, column i; T beta V
+        const int t = 4 * x + wave;
+        f32x4_t wt = {0.f, 0.f, 0.f, 0.f}, vt = wt;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            wt = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[(4 * lq + e) * P + 16 * t + lm], tv[e], wt, 0, 0, 0);
+            vt = __builtin_amdgcn_mfma_f32_16x16x4f32(tv[e], vs[(4 * lq + e) * P + 16 * t + lm], vt, 0, 0, 0);
+        }
+        *reinterpret_cast<f32x4_t*>(rec + 256 * t + 4 * lane) = wt;
+        *reinterpret_cast<f32x4_t*>(rec + 49 * D + 256 + 256 * t + 4 * lane) = vt;
+    }
+}
+
 // Wavefront w of workgroup x owns state columns 16 (x * waves + w) .. + 15: DT accumulator tiles of 16 rows, lane (q, m)
 // holding rows 16 t + 4 q + r of column m.  That is also the layout of the second operand of the next product, whose
 // first operand the records hold in fragment order.
@@ -577,19 +827,6 @@ __global__ void __launch_bounds__(256) delta_scan_kernel(const PortionDesc* port
         for (int t = 0; t < DT; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) sp[(int64_t)(16 * t + 4 * q + r) * vdim_pad] = s[t][r];
-}
-
-// x summed over the 32 lanes of a half of the wavefront, in all of them
-__device__ __forceinline__ float half_sum(float x) {
-    auto ror = [](float v, auto C) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(C)::value, 0xf, 0xf, false)); };
-    x += ror(x, std::integral_constant<int, 0x128>{});          // rotations by 8, 4, 2 and 1 within rows of 16 lanes
-    x += ror(x, std::integral_constant<int, 0x124>{});
-    x += ror(x, std::integral_constant<int, 0x122>{});
-    x += ror(x, std::integral_constant<int, 0x121>{});
-    const unsigned u = __builtin_bit_cast(unsigned, x);
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    const unsigned lo = r[0], hi = r[1];
-    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
 }
 
 // hi + mid + lo = x exactly, two floats at a time, hi and mid rounded to nearest, so that residuals have both signs: |mid| <= 2^-8 and
@@ -970,6 +1207,15 @@ int launch_step(const DeltaArgs<T>& a, const int32_t* slots, const int64_t* posi
     return (int)hipGetLastError();
 }
 
+template <int DT>
+int launch_prep_square(const DeltaArgs<__bf16>& a, const ChunkDesc* chunks, int64_t num_chunks, float* records, hipStream_t st) {
+    constexpr int D = 16 * DT;
+    constexpr size_t lds = (size_t)(4 * kC * (D + 4) + 1024 + kC * 20 + 2 * D + 48) * sizeof(float);
+    static_assert(lds <= 40 * 1024, "four workgroups a compute unit");
+    hipLaunchKernelGGL((delta_prep_square_kernel<DT>), dim3((unsigned)num_chunks, (unsigned)a.heads), dim3(256), lds, st, a, chunks, records);
+    return (int)hipGetLastError();
+}
+
 template <class T>
 int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t num_portions, const ChunkDesc* chunks, int64_t num_chunks,
                   float* records, float* o, int64_t row0, int64_t rows, const int32_t* ring_slot, const int64_t* positions,
@@ -985,8 +1231,17 @@ int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t nu
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prep), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
     }
-    hipLaunchKernelGGL(prep, dim3((unsigned)num_chunks, (unsigned)a.heads), dim3(256), lds, st, a, chunks, records);
-    int rc = (int)hipGetLastError();
+    int rc = INFER_KV_OK;
+    bool prepared = false;
+    if constexpr (sizeof(T) == 2)
+        if (vec && a.dim == a.vdim && (a.dim == 64 || a.dim == 128) && a.decay_stride % 2 == 0) {
+            rc = a.dim == 64 ? launch_prep_square<4>(a, chunks, num_chunks, records, st) : launch_prep_square<8>(a, chunks, num_chunks, records, st);
+            prepared = true;
+        }
+    if (!prepared) {
+        hipLaunchKernelGGL(prep, dim3((unsigned)num_chunks, (unsigned)a.heads), dim3(256), lds, st, a, chunks, records);
+        rc = (int)hipGetLastError();
+    }
     if (rc) return rc;
     const bool out4 = rows4 && fours(a.gate, a.gate_stride) && fours(a.out, a.out_stride) && ptr_aligned(o, 16) && ptr_aligned(a.norm, 16);
     // A (portion, head) on half of the compute units or fewer leaves delta_scan_kernel alone on its vector units, and its shorter step wins:

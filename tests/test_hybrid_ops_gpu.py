@@ -376,6 +376,14 @@ def test_delta_decay_strengths(gpu, decay):
     DeltaCase(2, 1, 48, 64, 4, 70, torch.float32, seed=2, decay=decay).check([64, 1, 5])
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("decay", [-6.0, 0.0, 40.0])
+@pytest.mark.parametrize("cuts", [[50], [16, 2, 17, 15], [3, 33, 1, 2, 11]])
+def test_delta_square_heads(gpu, dim, decay, cuts):
+    """The chunk kernel of heads as wide as they are high: whole and ragged chunks, windows that begin in the ring, decays past what two factors hold."""
+    DeltaCase(3, 1, dim, dim, 4, 50, torch.bfloat16, seed=4, decay=decay).check(cuts)
+
+
 def test_delta_first_token_is_still_read_far_later(gpu):
     """Token 0 alone writes; almost no decay; the last query asks for what it wrote."""
     c = DeltaCase(1, 1, 32, 32, 1, 300, torch.float32, seed=3, decay=-16.0)
