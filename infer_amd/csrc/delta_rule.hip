@@ -9,6 +9,7 @@
 //                        gates and everything of a chunk that does not need the state
 //   delta_scan_kernel    walks the chunks of a portion; a wavefront holds 16 columns of the state as float32 MFMA
 //                        accumulators
+//   delta_scan_slab_kernel   the same for few portions and heads: a workgroup per head and 16 to 64 columns, the rows shared out over its wavefronts
 //   delta_out_kernel     output norm and gate of the scanned tokens; the convolution's tail goes to its ring
 //   delta_scan_wide_kernel   scan, output norm and gate in one launch, for batches that fill the chip with one workgroup per
 //                        (portion, head); delta_ring_kernel then writes the rings
@@ -19,7 +20,7 @@
 //     o_i = (e^{G_i} q_i)^T S + sum_{j<=i} B_ij u_j,                  B_ij = sum_d q_i[d] k_j[d] e^{G_i - G_j}[d]
 //     S'  = e^{G_last} S + sum_j (e^{G_last - G_j} k_j) u_j^T.
 // Every exponent is a difference that is <= 0, so nothing overflows however strong the decay is.  All of it is
-// float32, the products included (v_mfma_f32_16x16x4_f32; in the wide scan six bf16 products of the pieces of a float).
+// float32, the products included (v_mfma_f32_16x16x4_f32; in the wide and the slab scan six bf16 products of the pieces of a float).
 //
 // The last `taps` inputs of the convolution live in a ring per sequence (entry position % taps).  A position below
 // zero counts as zero and a portion that starts at position 0 starts from a zero state, so a slot needs no clearing
@@ -849,6 +850,238 @@ __device__ __forceinline__ void split3(const float (&x)[N], uint32_t (&p)[3][N /
     }
 }
 
+// Operands of products over 16 (tokens, or rows of the state) as pieces, two along the sum: six products of pieces are three instructions.
+struct LeftPieces {
+    bf16x8_t hm, hl;
+    LeftPieces() = default;
+    __device__ __forceinline__ explicit LeftPieces(f32x4_t x) {
+        const float f[4] = {x[0], x[1], x[2], x[3]};
+        uint32_t p[3][2];
+        split3<4>(f, p);
+        hm = __builtin_bit_cast(bf16x8_t, u32x4_t{p[0][0], p[0][1], p[1][0], p[1][1]});
+        hl = __builtin_bit_cast(bf16x8_t, u32x4_t{p[0][0], p[0][1], p[2][0], p[2][1]});
+    }
+};
+struct RightPieces {
+    bf16x8_t hh, mm, lh;
+    RightPieces() = default;
+    __device__ __forceinline__ explicit RightPieces(f32x4_t x) {
+        const float f[4] = {x[0], x[1], x[2], x[3]};
+        uint32_t p[3][2];
+        split3<4>(f, p);
+        hh = __builtin_bit_cast(bf16x8_t, u32x4_t{p[0][0], p[0][1], p[0][0], p[0][1]});
+        mm = __builtin_bit_cast(bf16x8_t, u32x4_t{p[1][0], p[1][1], p[1][0], p[1][1]});
+        lh = __builtin_bit_cast(bf16x8_t, u32x4_t{p[2][0], p[2][1], p[0][0], p[0][1]});
+    }
+};
+struct PieceSums {
+    f32x4_t large = {0.f, 0.f, 0.f, 0.f}, middle = large, small = large;
+    __device__ __forceinline__ void add(const LeftPieces& a, const RightPieces& b) {
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hl, b.lh, small, 0, 0, 0);
+        middle = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hm, b.mm, middle, 0, 0, 0);
+        large = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hm, b.hh, large, 0, 0, 0);
+    }
+    __device__ __forceinline__ f32x4_t sum() const { return large + (middle + small); }
+};
+
+// Few (portion, head) pairs: what counts is how long a chunk takes, and there are compute units enough for every 16 CT columns of a head to have one.
+// Wavefront w of NW owns RT tiles of 16 rows of the state (w RT + r) and brings their parts of the records straight into registers, PD chunks ahead; what
+// the products with all rows need, S^T K and S^T Q of a chunk, is added up through LDS, one barrier a chunk.  Two more wavefronts, each for every other
+// chunk, bring V and B and finish the outputs, so that nobody else stores anything.  Workgroups of a pair lie on one die and walk its records side by side, so
+// that these come from memory once.  Products as in delta_scan_wide_kernel, the state's sums by the vector unit.
+// A chunk takes 1.0 us with one tile, 1.3 with two and 2.1 with four (delta_scan_kernel: 2.5 and more), of which the loads are nothing (the same record again and
+// again: 3 % less), the products of S^T Q 13 % although they run while U is under way.  One portion of 2000 tokens, 32 heads of 128 x 128: the scan 262 -> 131 us under
+// a profiler, the call 382 -> 184.  With float products 186 (one tile), 408 instead of 323 (four); one wavefront for the outputs 200; eight wavefronts of one
+// row tile each 187.
+template <int DT, int CT>
+struct SlabSizes {
+    static constexpr int RT = DT >= 8 ? 2 : 1, NW = DT / RT, PD = CT == 4 ? 2 : 3, threads = 64 * (NW + 2);
+    static constexpr int lds = 2 * (2 * NW + 1) * CT * 1024;
+};
+template <int DT, int CT>
+__global__ void __launch_bounds__((SlabSizes<DT, CT>::threads)) delta_scan_slab_kernel(const PortionDesc* portions, const ChunkDesc* chunks, const float* records,
+                                                                                          float* state, float* o, int heads, int vdim_pad, int pairs, int slabs) {
+    using Z = SlabSizes<DT, CT>;
+    constexpr int dp = 16 * DT, RT = Z::RT, NW = Z::NW, PD = Z::PD;
+    extern __shared__ __attribute__((aligned(16))) f32x4_t slab_lds[];
+    f32x4_t* parts = slab_lds;                                  // [2][NW + 1][CT][64]: of S^T K, the last one -V
+    f32x4_t* outs = slab_lds + 2 * (NW + 1) * CT * 64;          // [2][NW][CT][64]: of S^T Q
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane >> 4, m = lane & 15;
+    const int die = blockIdx.x & 7, turn = blockIdx.x >> 3, pair = turn / slabs * 8 + die, slab = turn % slabs;
+    if (pair >= pairs) return;
+    const PortionDesc p = portions[pair / heads];
+    const int h = pair % heads, vt0 = slab * CT, tiles = vdim_pad / 16;
+    const int64_t rec_len = record_floats(dp, vdim_pad), rec_step = (int64_t)heads * rec_len;
+    const float* rec = records + ((int64_t)p.chunk0 * heads + h) * rec_len;
+    auto record = [&](int c) { return rec + (c < p.chunks ? c : p.chunks - 1) * rec_step; };
+    auto part = [&](int c, int w, int t) -> f32x4_t& { return parts[(((c & 1) * (NW + 1) + w) * CT + t) * 64 + lane]; };
+    auto out = [&](int c, int w, int t) -> f32x4_t& { return outs[(((c & 1) * NW + w) * CT + t) * 64 + lane]; };
+    auto update = [&](int c, int t) {                           // U: V - S^T K
+        f32x4_t u = part(c, NW, t);
+#pragma unroll
+        for (int w = 0; w < NW; ++w) u += part(c, w, t);
+        return -u;
+    };
+    if (wave < NW) {
+        f32x4_t s[RT][CT];
+        auto state_at = [&](int r, int t, int e) {
+            return state + (((int64_t)p.slot * heads + h) * dp + 16 * (wave * RT + r) + 4 * q + e) * vdim_pad + 16 * (vt0 + t) + m;
+        };
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int t = 0; t < CT; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[r][t][e] = p.pos0 > 0 && vt0 + t < tiles ? *state_at(r, t, e) : 0.f;
+        if (p.chunks > 0) {
+            struct Rows { f32x4_t w[RT], q[RT], k[RT], e[RT]; } ring[PD];
+            auto request = [&](Rows& f, int c) {
+                const float* src = record(c) + 256 * RT * wave + 4 * lane;
+#pragma unroll
+                for (int r = 0; r < RT; ++r) {
+                    f.w[r] = *reinterpret_cast<const f32x4_t*>(src + 256 * r);
+                    f.q[r] = *reinterpret_cast<const f32x4_t*>(src + 16 * dp + 256 * r);
+                    f.k[r] = *reinterpret_cast<const f32x4_t*>(src + 32 * dp + 256 * r);
+                    f.e[r] = *reinterpret_cast<const f32x4_t*>(record(c) + 48 * dp + 256 + 16 * (RT * wave + r) + 4 * q);
+                }
+            };
+#pragma unroll
+            for (int i = 0; i < PD; ++i) request(ring[i], i);
+            LeftPieces w[RT], qv[RT], k[RT];
+#pragma unroll
+            for (int r = 0; r < RT; ++r) w[r] = LeftPieces(ring[0].w[r]);
+            for (int c0 = 0; c0 < p.chunks; c0 += PD) {
+#pragma unroll
+                for (int i = 0; i < PD; ++i) {
+                    const int c = c0 + i;
+                    if (c >= p.chunks) break;
+                    const Rows& f = ring[i];
+                    RightPieces sp[RT][CT];
+#pragma unroll
+                    for (int t = 0; t < CT; ++t) {
+#pragma unroll
+                        for (int r = 0; r < RT; ++r) sp[r][t] = RightPieces(s[r][t]);
+                        PieceSums x;
+#pragma unroll
+                        for (int r = 0; r < RT; ++r) x.add(w[r], sp[r][t]);
+                        part(c, wave, t) = x.sum();
+                    }
+#pragma unroll
+                    for (int r = 0; r < RT; ++r) {
+                        qv[r] = LeftPieces(f.q[r]);
+                        k[r] = LeftPieces(f.k[r]);
+                    }
+                    __syncthreads();
+                    f32x4_t us[CT];
+#pragma unroll
+                    for (int t = 0; t < CT; ++t) us[t] = update(c, t);
+#pragma unroll
+                    for (int t = 0; t < CT; ++t) {
+                        PieceSums y;
+#pragma unroll
+                        for (int r = 0; r < RT; ++r) y.add(qv[r], sp[r][t]);
+                        out(c, wave, t) = y.sum();
+                    }
+#pragma unroll
+                    for (int t = 0; t < CT; ++t) {
+                        const RightPieces u(us[t]);
+#pragma unroll
+                        for (int r = 0; r < RT; ++r) {
+                            PieceSums d;
+                            d.add(k[r], u);
+                            const f32x4_t ds = d.sum();
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) s[r][t][e] = __builtin_fmaf(s[r][t][e], f.e[r][e], ds[e]);
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < RT; ++r) w[r] = LeftPieces(ring[(i + 1) % PD].w[r]);
+                    request(ring[i], c + PD);
+                }
+            }
+            __syncthreads();                                   // the last chunk's outputs
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int t = 0; t < CT; ++t)
+                if (vt0 + t < tiles)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) *state_at(r, t, e) = s[r][t][e];
+    } else if (p.chunks > 0) {
+        int zero = 0;
+        asm volatile("" : "+v"(zero));                         // by the vector path: a scalar load in flight would be waited for with every read of LDS
+        const int32_t* descs = &chunks[p.chunk0].row0 + zero;
+        constexpr int kDesc = sizeof(ChunkDesc) / sizeof(int32_t), kRing = 2;
+        struct Chunk { f32x4_t v[CT], b; int row0, count; } ring[kRing];
+        auto request = [&](Chunk& f, int c) {
+            const float* src = record(c);
+#pragma unroll
+            for (int t = 0; t < CT; ++t) f.v[t] = *reinterpret_cast<const f32x4_t*>(src + 49 * dp + 256 + 256 * (vt0 + t < tiles ? vt0 + t : 0) + 4 * lane);
+            f.b = *reinterpret_cast<const f32x4_t*>(src + 48 * dp + 4 * lane);
+            const int at = (c < p.chunks ? c : p.chunks - 1) * kDesc;
+            f.row0 = descs[at];
+            f.count = descs[at + 1];
+        };
+        const int64_t row_step = (int64_t)heads * vdim_pad;
+        float* const column = o + (int64_t)h * vdim_pad + 16 * vt0 + m + 4 * q * row_step;
+        f32x4_t y[CT];
+        auto store = [&](const Chunk& f, int c) {
+#pragma unroll
+            for (int t = 0; t < CT; ++t)
+#pragma unroll
+                for (int w = 0; w < NW; ++w) y[t] += out(c, w, t);
+            const int count = f.count - 4 * q;
+            float* to = column + __builtin_amdgcn_readfirstlane(f.row0) * row_step;
+#pragma unroll
+            for (int e = 0; e < 4; ++e, to += row_step)
+                if (e < count)
+#pragma unroll
+                    for (int t = 0; t < CT; ++t)
+                        if (vt0 + t < tiles) to[16 * t] = y[t][e];
+        };
+        // Chunks of one parity: in front of its barrier -V, behind it the outputs, behind the next one their way out
+        auto walk = [&](auto parity) {
+            constexpr int kOdd = decltype(parity)::value;
+#pragma unroll
+            for (int i = 0; i < kRing; ++i) request(ring[i], 2 * i + kOdd);
+            for (int c0 = 0; c0 < p.chunks; c0 += 2 * kRing)
+#pragma unroll
+                for (int i = 0; i < 2 * kRing; ++i) {
+                    const int c = c0 + i;
+                    if (c >= p.chunks) break;
+                    if ((i & 1) == kOdd) {
+#pragma unroll
+                        for (int t = 0; t < CT; ++t) part(c, NW, t) = -ring[i / 2].v[t];
+                    }
+                    __syncthreads();
+                    if ((i & 1) == kOdd) {
+                        const LeftPieces b(ring[i / 2].b);
+#pragma unroll
+                        for (int t = 0; t < CT; ++t) {
+                            PieceSums x;
+                            x.add(b, RightPieces(update(c, t)));
+                            y[t] = x.sum();
+                        }
+                    } else if (c > 0) {
+                        Chunk& last = ring[(i + 2 * kRing - 1) / 2 % kRing];
+                        store(last, c - 1);
+                        request(last, c - 1 + 2 * kRing);
+                    }
+                }
+            const int c = p.chunks - 1;
+            __syncthreads();
+            if ((c & 1) == kOdd) {
+#pragma unroll
+                for (int i = 0; i < kRing; ++i)
+                    if (c / 2 % kRing == i) store(ring[i], c);
+            }
+        };
+        if (wave == NW) walk(std::integral_constant<int, 0>{});
+        else walk(std::integral_constant<int, 1>{});
+    }
+}
+
 // A record in LDS: sums of three bf16 numbers, hi + mid + lo = the float exactly, so that the products run on the bf16 matrix pipe.  Of
 // the nine products of two such sums six are added; the others, mid lo, lo mid and lo lo, are 2^-24 of the product at most, as much as a
 // float product is rounded by, and of either sign.
@@ -1155,6 +1388,45 @@ int launch_scan(const PortionDesc* p, int64_t portions, int64_t tokens, const Ch
     return (int)hipGetLastError();
 }
 
+template <int DT, int CT>
+int launch_scan_slab(const PortionDesc* p, int64_t portions, const ChunkDesc* c, const float* records, float* state, float* o,
+                     int heads, int vdim_pad, hipStream_t st) {
+    using Z = SlabSizes<DT, CT>;
+    const int64_t pairs = portions * heads;
+    const int slabs = (vdim_pad / 16 + CT - 1) / CT;
+    auto kernel = &delta_scan_slab_kernel<DT, CT>;
+    if (Z::lds > 60 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, Z::lds);
+        if (e != hipSuccess) return (int)e;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((pairs + 7) / 8 * 8 * slabs)), dim3(Z::threads), Z::lds, st, p, c, records, state, o, heads, vdim_pad, (int)pairs, slabs);
+    return (int)hipGetLastError();
+}
+// Tiles of 16 columns per workgroup of delta_scan_slab_kernel, or 0 where the others are ahead.  Heads of 128 rows need a compute unit for a workgroup: one
+// tile as long as there are enough of them, otherwise two or four.  Others share it, and one tile is ahead up to two and a half workgroups per unit.  The call,
+// us, delta_scan_kernel (* delta_scan_wide_kernel) / 1 / 2 / 4 tiles, heads x portions of tokens: 128 x 128 16 x 1 of 2000 352 / 150 / 194 / 290, 32 x 1 of 12000 2197 / 1087 /
+// 1277 / 1823, 16 x 4 of 500 to 3000 528 / 358 / 333 / 446, 32 x 2 of 1000 233 / 187 / 156 / 204, 32 x 3 267 / 295 / 270 / 240, 32 x 4 297 / 392 / 310 / 277, but 32 x 5 302* / 486 /
+// 412 / 419; 64 x 64 32 x 4 of 1000 177 / 136 / 132 / 165, 32 x 5 176* / 196 / 212 / 195; 96 x 96 30 x 4 of 800 230 / 226 / 243 / 252; 256 x 128 16 x 5 of 600 355 / 303 /
+// 429; 192 x 192 16 x 3 of 300 to 1200 364 / 274; 48 x 48 30 x 7 of 600 189 / 144; 32 x 32 32 x 5 of 300 to 900 117* / 93; 16 x 16 30 x 20 of 700 290 / 276.
+int few_tiles(int dim_pad, int vdim_pad, int64_t pairs) {
+    const int tiles = vdim_pad / 16;
+    if (dim_pad != 128) return pairs * tiles <= 640 ? 1 : 0;
+    for (int n : {1, 2, 4})
+        if (pairs * ((tiles + n - 1) / n) <= 256) return n;
+    return 0;
+}
+template <int DT>
+int launch_few(const PortionDesc* p, int64_t portions, int64_t tokens, const ChunkDesc* c, const float* records, float* state, float* o,
+               int heads, int vdim_pad, hipStream_t st) {
+    const int tiles = few_tiles(16 * DT, vdim_pad, portions * heads);
+    if (tiles == 1) return launch_scan_slab<DT, 1>(p, portions, c, records, state, o, heads, vdim_pad, st);
+    if constexpr (DT == 8) {
+        if (tiles == 2) return launch_scan_slab<DT, 2>(p, portions, c, records, state, o, heads, vdim_pad, st);
+        if (tiles == 4) return launch_scan_slab<DT, 4>(p, portions, c, records, state, o, heads, vdim_pad, st);
+    }
+    return launch_scan<DT>(p, portions, tokens, c, records, state, o, heads, vdim_pad, st);
+}
+
 template <class T, int DT>
 int launch_scan_wide(const DeltaArgs<T>& a, const PortionDesc* p, int64_t portions, int64_t tokens, const ChunkDesc* c, const float* records, hipStream_t st) {
     constexpr size_t lds = (size_t)2 * wide_buffer_units(DT) * 16 + 2 * 16 * 132 * sizeof(float);
@@ -1244,16 +1516,16 @@ int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t nu
     }
     if (rc) return rc;
     const bool out4 = rows4 && fours(a.gate, a.gate_stride) && fours(a.out, a.out_stride) && ptr_aligned(o, 16) && ptr_aligned(a.norm, 16);
-    // A (portion, head) on half of the compute units or fewer leaves delta_scan_kernel alone on its vector units, and its shorter step wins:
-    // heads of 128 x 128, one portion of 2000 tokens, 16 heads 358 us against 387; of 9000, 32 heads 1702 against 1810.  Beyond, one
-    // workgroup for a head and its outputs wins: 32 heads, 16 portions of 800 tokens 853 us against 712, 60 of 110 512 against 428; heads
+    // Up to 128 pairs of a portion and a head, and some more of small heads (few_tiles), the columns of a head go to several workgroups.  Beyond, one
+    // workgroup for a head and its outputs wins, here against delta_scan_kernel: 32 heads, 16 portions of 800 tokens 853 us against 712, 60 of 110 512 against 428; heads
     // of 64 x 64, 5 of 800 183 against 156; of 128 x 16, 5 of 800 465 against 181.  Small heads give most of its eight wavefronts no
     // columns, which costs where there are more workgroups than compute units, unless delta_out_kernel has no form for the columns
     // either: 60 portions of 110, heads of 32 x 32 153 us against 195, 32 x 64 201 against 213, 64 x 32 220 against 253, but 32 x 48 210
     // against 197.
     const int64_t pairs = (int64_t)a.heads * num_portions;
     const bool small = a.dim_pad * a.vdim_pad <= 2048 && (a.vdim == 32 || a.vdim == 64);
-    if (out4 && 2 * pairs > 256 && !(small && pairs > 256) && a.vdim_pad <= 128 && (a.dim_pad == 32 || a.dim_pad == 64 || a.dim_pad == 96 || a.dim_pad == 128)) {
+    const bool slabs = pairs <= 128 || (few_tiles(a.dim_pad, a.vdim_pad, pairs) == 1 && pairs * (a.vdim_pad / 16) <= 320);
+    if (out4 && !slabs && !(small && pairs > 256) && a.vdim_pad <= 128 && (a.dim_pad == 32 || a.dim_pad == 64 || a.dim_pad == 96 || a.dim_pad == 128)) {
 #define GO(N) case N: rc = launch_scan_wide<T, N>(a, portions, num_portions, rows, chunks, records, st); break
         switch (a.dim_pad / 16) { GO(2); GO(4); GO(6); GO(8); }
 #undef GO
@@ -1265,7 +1537,7 @@ int launch_chunks(const DeltaArgs<T>& a, const PortionDesc* portions, int64_t nu
             hipLaunchKernelGGL((delta_ring_kernel<T, 1>), dim3(groups, (unsigned)((a.channels + 255) / 256)), dim3(256), 0, st, a, row0, rows, ring_slot, positions);
         return (int)hipGetLastError();
     }
-#define GO(N) case N: rc = launch_scan<N>(portions, num_portions, rows, chunks, records, a.state, o, a.heads, a.vdim_pad, st); break
+#define GO(N) case N: rc = launch_few<N>(portions, num_portions, rows, chunks, records, a.state, o, a.heads, a.vdim_pad, st); break
     switch (a.dim_pad / 16) { GO(1); GO(2); GO(3); GO(4); GO(6); GO(8); GO(12); GO(16); default: return INFER_KV_EUNSUPPORTED; }
 #undef GO
     if (rc) return rc;

@@ -478,6 +478,46 @@ def test_delta_batch_that_fills_the_chip(gpu, dtype, heads, kv_heads, dim, vdim,
     assert torch.isnan(c0.state[2]).all()
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(3, 128, 112), (12, 128, 112), (20, 128, 112), (20, 64, 104), (2, 16, 20), (3, 32, 24), (8, 48, 300), (9, 90, 40), (4, 192, 112),
+                                            (3, 256, 200)])
+def test_delta_slabs_of_few_portions(gpu, heads, dim, vdim):
+    """One, two and four column tiles per workgroup, not all of them there, one and two row tiles per wavefront: portions of one chunk, of two and of as many as
+    the rings hold and one more, empty chunks and portions among them, from zero and continued."""
+    lens = [(17, 48, 0, 97), (3, 33, 16, 16)]
+    c = DeltaCase(heads, heads, dim, vdim, 4, sum(lens[0]) + sum(lens[1]), torch.float32, slots=4, decay=-3.0)
+    done, outs = [0] * 4, [[] for _ in range(4)]
+    first = np.cumsum([0] + [a + b for a, b in zip(*lens)])
+    for part in lens:
+        rows, chunks, portions, ring, pos, row = [], [], [], [], [], 0
+        for slot, k in enumerate(part):
+            own = [(row + r, min(16, k - r), done[slot] + r, done[slot], slot, 0) for r in range(0, k, 16)]
+            if slot == 1:
+                own.insert(1, (0, 0, done[slot], done[slot], slot, 0))
+            portions.append((len(chunks), len(own), slot, done[slot]))
+            chunks += own
+            ring += [(slot, k - 1 - r) for r in range(k)]
+            pos += range(done[slot], done[slot] + k)
+            rows += range(first[slot] + done[slot], first[slot] + done[slot] + k)
+            row += k
+            done[slot] += k
+        out = torch.full((row, heads * vdim), float("nan"), device="cuda")
+        ho.delta_chunks(c.s, dev(c.proj[rows]), c.beta_off, dev(c.decay[rows]), dev(c.gate[rows]), *c.weights, c.ring, c.state, dev(portions, torch.int32),
+                        dev(chunks, torch.int32), dev(ring, torch.int32), dev(pos, torch.int64), 0, out)
+        at = 0
+        for slot, k in enumerate(part):
+            outs[slot].append(host(out[at:at + k]))
+            at += k
+    proj, decay, gate = c.proj, c.decay, c.gate
+    for slot in range(4):
+        rows = slice(first[slot], first[slot + 1])
+        c.n, c.proj, c.decay, c.gate = first[slot + 1] - first[slot], proj[rows], decay[rows], gate[rows]
+        want, want_state = c.want()
+        assert np.abs(np.concatenate(outs[slot]) - want).max() <= 3e-5 * np.abs(want).max()
+        close(c.state[slot][:, :dim, :vdim], want_state, 3e-5)
+        rest = host(c.state[slot])
+        assert (rest[:, dim:] == 0).all() and (rest[:, :, vdim:] == 0).all()
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(90, 64, 64), (90, 24, 20), (260, 32, 80)])
 def test_delta_portions_that_take_turns(gpu, heads, dim, vdim):
     """More workgroups than compute units: the longest portions go first, equal and empty ones in their order, several to the first round or not even one."""
