@@ -629,7 +629,7 @@ __device__ __forceinline__ void moe_row_product(const GemmArgs<__bf16>& a, int e
     f32x4_t acc[1][MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[0][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream_product<1, MT, kRowWaves, MT == 1 ? 3 : 2>(w, x, a.k, wave, lds + wave * kRowRing, acc);
+    stream_product<1, MT, kRowWaves, MT == 1 ? 3 : 2, 0>(w, x, a.k, wave, lds + wave * kRowRing, acc);
     stream_reduce<1, MT, kRowWaves>(acc, wave, lds, [&](int, int t, f32x4_t sum) {
         const int r = 16 * t + n;
         __bf16* o = a.out + (int64_t)(first + r) * a.out_stride;

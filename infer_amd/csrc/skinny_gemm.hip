@@ -21,8 +21,9 @@
 //   operands; every fragment read feeds both row tiles of the wavefront, which halves the LDS
 //   traffic per weight byte (LDS delivers 128 B/clk and would otherwise bound the kernel).
 //
-// That is skinny_gemm_kernel, for 65 to 128 rows.  Up to 64, skinny_stream_kernel streams the weights through LDS (weight_stream.h); its
-// wavefronts split K among themselves, so that K is cut over workgroups only where there are few of them.
+// That is skinny_gemm_kernel, for 65 to 128 rows.  Up to 64, the weights stream through LDS (weight_stream.h): skinny_stream_kernel, whose
+// wavefronts split K among themselves, so that K is cut over workgroups only where there are few of them, and skinny_shared_kernel, whose wavefronts
+// share every step of K and with it the batch.
 // * SK == 1: the accumulators are rounded to bf16 and stored.  SK > 1: float32 partial sums
 //   [SK][M][N] go to the workspace and `skinny_gemm_reduce_kernel` adds them and rounds once.
 #include <hip/hip_runtime.h>
@@ -217,7 +218,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& a, int half, int spl
 // 16 RT rows of weights past up to 16 MT rows of the batch, NW wavefronts with D steps each in LDS.  GATED: the weights are gate rows and as
 // many up rows, a.n / 2 each; a tile is eight gate rows and the eight up rows of the same places, and y = silu(gate) * up with the
 // roundings of storing both and reading them again.
-template <int RT, int MT, int NW, int D, bool GATED>
+template <int RT, int MT, int NW, int D, bool GATED, int TURN>
 __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
     constexpr int kRing = D * stream_stage_bytes(RT, MT), kLds = NW * (kRing > 1024 * RT * MT ? kRing : 1024 * RT * MT);
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
@@ -243,8 +244,46 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream_product<RT, MT, NW, D>(w, x, a.chunks * kKC, wave, lds + wave * kRing, acc);
+    stream_product<RT, MT, NW, D, TURN>(w, x, a.chunks * kKC, wave, lds + wave * kRing, acc);
     stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, half, split, n0, r, 16 * t + n, g, sum); });
+}
+
+// The same, the steps of k shared by the wavefronts (SharedStream)
+template <int RT, int MT, bool GATED>
+__global__ void __launch_bounds__(256) skinny_shared_kernel(GemmArgs a) {
+    using Stream = SharedStream<RT, MT>;
+    constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR, kRing = Stream::D * Stream::kStage;
+    static_assert(WK == 1 || 4096 * TW * MT <= kRing, "the sums fit the ring");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing];
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = a.n / 2, n0 = blockIdx.x * (GATED ? 8 : 16) * RT, split = blockIdx.y, wr = wave % WR;
+    const int64_t k_lo = (int64_t)split * a.chunks * kKC;
+    Stream stream(a.chunks * kKC, wave, lds,
+        [&](int i) {
+            int row = n0 + stream_row() + 8 * (GATED ? i / 2 : i);
+            const int rows = GATED ? half : a.n;
+            row = (row < rows ? row : rows - 1) + (GATED && (i & 1) ? half : 0);
+            return (const __bf16*)a.w + (int64_t)row * a.k + k_lo;
+        },
+        [&](int i) {
+            const int row = stream_row() + 8 * i;
+            return (const __bf16*)a.x + (int64_t)(row < a.m ? row : a.m - 1) * a.x_stride0 + k_lo;
+        });
+    f32x4_t acc[TW][MT];
+#pragma unroll
+    for (int r = 0; r < TW; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    stream.product(wave, lds, acc);
+    auto finish = [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, half, split, n0, wr * TW + r, 16 * t + n, g, sum); };
+    if constexpr (WK == 1) {
+#pragma unroll
+        for (int r = 0; r < TW; ++r)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) finish(r, t, acc[r][t]);
+    } else {
+        stream_reduce<TW, MT, WK>(acc, wave / WR, lds + wr * (1024 * WK * TW * MT), finish);
+    }
 }
 
 // What stands in front of a product of few rows: y = norm(x + residual) w^T, where x may still be the pieces of a split product.
@@ -268,7 +307,7 @@ constexpr int kFewPad = 64;                                         // bytes beh
 // What bounds it is what all workgroups read in front, rows times their bytes.  Norm and product, us, two launches / one, for 1, 2, 4 rows:
 // 4096 x 1024 behind four pieces 6.2 / 4.2, 6.4 / 4.3, 6.4 / 6.8; 6144 x 1024 gated 7.6 / 5.7, 7.6 / 6.0, 7.7 / 8.0; 6144 x 4096 14.1 / 12.6,
 // 13.5 / 13.3, 13.7 / 22.4; 24576 x 4096 gated 35.5 / 33.7, 33.8 / 42.4.  So one row up to 4096 elements, two of half as many.
-template <int RT, int NP, bool GATED>
+template <int RT, int NP, bool GATED, int TURN>
 __global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSource f) {
     constexpr int NW = 4, D = 4, kRing = D * stream_stage_bytes(RT, 0);
     static_assert(NW * kRing >= NW * RT * 1024, "sums of the wavefronts");
@@ -368,7 +407,7 @@ __global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSourc
     f32x4_t acc[RT][1];
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream_product_held<RT, NW, D>(w, xs + (n < a.m ? n : a.m - 1) * row_bytes + 16 * g, a.k, wave, few_lds + wave * kRing, norm, acc);
+    stream_product_held<RT, NW, D, TURN>(w, xs + (n < a.m ? n : a.m - 1) * row_bytes + 16 * g, a.k, wave, few_lds + wave * kRing, norm, acc);
     stream_reduce<RT, 1, NW>(acc, wave, few_lds, [&](int r, int, f32x4_t sum) { finish_tile<GATED>(a, half, 0, n0, r, n, g, sum); });
 }
 
@@ -435,7 +474,7 @@ __global__ void __launch_bounds__(256) piece_product_kernel(GemmArgs a, FewDecod
         __syncthreads();
     };
     f32x4_t acc[1][1] = {{f32x4_t{0.f, 0.f, 0.f, 0.f}}};
-    stream_product_held<1, NW, D>(w, reinterpret_cast<const unsigned char*>(xs) + 16 * g, a.chunks * kKC, wave, lds + wave * kRing, add, acc);
+    stream_product_held<1, NW, D, 0>(w, reinterpret_cast<const unsigned char*>(xs) + 16 * g, a.chunks * kKC, wave, lds + wave * kRing, add, acc);
     stream_reduce<1, 1, NW>(acc, wave, lds, [&](int r, int, f32x4_t sum) { finish_tile<false>(a, 0, split, n0, r, n, g, sum); });
 }
 
@@ -463,26 +502,39 @@ __global__ void __launch_bounds__(256) skinny_gemm_reduce_kernel(ReduceArgs a) {
     *reinterpret_cast<u32x4*>(a.y + (int64_t)row * a.y_stride0 + 8 * c) = r.u;
 }
 
-// Weight rows of a workgroup.  Many rows amortise the batch, which every workgroup reads whole; few fill the chip.  Measured on weights of
-// n x 4096, us (16 / 32 / 48 / 64 / 96 rows):
-//   32 of the batch   n = 6144: - / 14.8 / 15.2 / 17.3 / 21.9    n = 12288: - / 27.5 / 19.3 / 20.9 / 24.7    n = 24576: - / 49.0 / 34.6 / 43.3 / 37.4
-//   64 of the batch   n = 6144: - / 17.2 / 19.1 / 21.8 / 27.3    n = 12288: - / 33.8 / 22.5 / 25.0 / 30.0    n = 24576: - / 58.5 / 44.6 / 49.7 / 40.3
-// so 33 to 64 want one workgroup per compute unit.  Past a vocabulary (n = 151936) there are many workgroups, and what counts is how little
-// of one passes before and behind its stream: one wavefront that holds 160 rows by itself, two such workgroups to a compute unit, against four
-// that split k of 80 rows and add up: 64 of the batch 259 -> 243 us (k = 4096), 79 -> 67 (k = 1024).  Up to 16, 16 rows are as good as any
-// (n = 24576: 33 to 37 us), except past many with a short k: n = 151936 32 rows 48 us (k = 1024), 16 rows 54, but 215 and 190 with k = 4096.
-// Few weight rows and a long k: 16 rows give every compute unit a workgroup that reads the batch once per 16 rows; 64 rows, cut over k, read it a
-// quarter as often.  Unreduced sums, us, 16 / 64 rows: n = 4096, k = 12288 9 of the batch 18.5 / 17.1, 16 20.2 / 17.3, 32 25.9 / 19.0; n = 5120,
-// k = 25600 60 / 52, 69 / 54, 91 / 60; n = 2560, k = 9728 12.7 / 10.4, 14.5 / 10.7, 19.1 / 15.7.  With a shorter k the launch that adds the
-// sums up for those who want them costs more than that (n = 4096, k = 4096, 16: 8.4 / 10.4 reduced, 8.6 / 7.4 unreduced).
-constexpr int64_t kMany = 40960, kVocabulary = 65536, kLongK = 8192;
+// Weight rows of a workgroup.  At most 8 of the batch, and up to 16 past few rows: 16, wavefronts that split k (skinny_stream_kernel), which are as good
+// as any (32 past many with a short k: n = 151936 48 us with k = 1024, 54 with 16 rows).  More of the batch: the activations, which every workgroup reads
+// whole, want many rows, and the chip wants a workgroup for every compute unit: wavefronts that share the steps of k (skinny_shared_kernel), 16 times
+// shared_tiles rows.  Us, wavefronts that split k (before they began in different places) / this:
+//   64 of the batch   24576 x 4096 gate and up 42.8 / 33.7   151936 x 4096 240 / 202   151936 x 1024 66 / 59   32000 x 4096 56 / 41   49152 x 2048 50 / 33
+//   32                24576 x 4096 34 / 31   151936 x 4096 213 / 192   16384 x 2048 17 / 12   8192 x 4096 16.1 / 12.8
+//   16                24576 x 4096 34 / 31   151936 x 4096 209 / 184   16384 x 2048 17 / 11.5   4: 30.8 / 30.7, 187 / 181 (these now 175), 14.9 / 11.9 (12.6)
+// Three tiles of rows are none of its shapes: 12288 x 4096 with 64 of the batch 21.2 / 22.6.  Few weight rows and a long k: 16 rows give every compute unit
+// a workgroup that reads the batch once per 16 rows; 64 rows, cut over k, read it a quarter as often.  Unreduced sums, 16 / 64 rows (split k): n = 4096,
+// k = 12288 9 of the batch 18.5 / 17.1, 16 20.2 / 17.3, 32 25.9 / 19.0 (now 17.3); with a shorter k the launch that adds the sums up for those who want
+// them costs more than that (n = 4096, k = 4096, 16: 8.4 / 10.4 reduced).
+constexpr int64_t kMany = 40960, kLongK = 8192, kUnits = 256;
+// 16-row tiles of a workgroup of skinny_shared_kernel: those with which the compute units are through first, counting what a tile takes as three and what every
+// 16 of the batch take beside them as one (151936 x 4096, us per round of 2 / 4 / 8 / 12 / 16 / 20 tiles: 64 of the batch 15 / 24 / 43 / 58 / 74 / 101, 16
+// 11 / 19 / 38 / 53 / 67 / 92).
+int shared_tiles(int64_t m, int64_t n) {
+    int best = 0;
+    int64_t least = 0;
+    for (int t : {2, 4, 6, 8, 10, 12, 14, 16, 20}) {
+        const int64_t groups = (n + 16 * t - 1) / (16 * t), takes = (groups + kUnits - 1) / kUnits * (3 * t + (m <= 16 ? 1 : m <= 32 ? 2 : 4));
+        if (best == 0 || takes <= least) {
+            best = t;
+            least = takes;
+        }
+    }
+    return best;
+}
 int rows_per_workgroup(int64_t m, int64_t n, int64_t k) {
-    if (m > 8 && m <= 32 && n <= 5120 && k >= kLongK) return 64;
-    if (m <= 16) return n >= kMany && k <= 2048 ? 32 : 16;
-    if (m <= 32) return n >= 8192 ? 48 : n > 5120 ? 32 : 16;
     if (m > 64) return kBN;
-    if (n <= 5120) return 64;
-    return n <= 8192 ? 32 : n >= kVocabulary ? 160 : n > 24576 ? 80 : 16 * (int)((n + 4095) / 4096);
+    if (n <= 5120) return m > 32 || (m > 8 && k >= kLongK) ? 64 : 16;
+    if (m <= 16 && n >= kMany && k <= 2048) return 32;
+    if (m <= 8) return 16;
+    return m > 16 && n > 8192 && n <= 12288 ? 48 : 16 * shared_tiles(m, n);
 }
 
 // Split-K factor: a divisor of the chunk count that brings the grid to at least one workgroup per
@@ -498,38 +550,49 @@ int choose_splits(int64_t m, int64_t n, int64_t k) {
         if (tiles * s >= 256) break;
     }
     if (m <= 32 || m > 64) return best;
-    // One workgroup of four wavefronts past 64 of the batch fills a compute unit's LDS, so 320 of them take as long as 512: of the smaller
-    // factors, the first with the shortest chain of chunks, where a workgroup's start and end cost as much as four.  Where there are more than
-    // 256 all the same, they have two wavefronts, two to a compute unit.  Unreduced sums, 64 of the batch, us, the first factor with 256
-    // workgroups / this: 3072 x 4096 12.8 / 9.7, 2560 x 4096 12.3 / 9.3, 5120 x 3072 15.0 / 10.6, 2560 x 9728 20.0 / 17.2, 5120 x 12288
-    // 38.0 / 27.4.
+    // A workgroup's start and end cost as much as four chunks, and two of 64 rows fit a compute unit's LDS, but what the unit takes from memory they share:
+    // of the smaller factors, the first with the shortest chain of chunks.  Unreduced sums, 64 of the batch, us, the first factor with 256 workgroups / this
+    // (wavefronts that split k): 3072 x 4096 12.8 / 9.7, 2560 x 4096 12.3 / 9.3, 5120 x 3072 15.0 / 10.6, 2560 x 9728 20.0 / 17.2, 5120 x 12288 38.0 / 27.4.
     auto chain = [&](int s) { return (tiles * s + 255) / 256 * (chunks / s + 4); };
     for (int s = best - 1; s >= 1; --s)
         if (chunks % s == 0 && chain(s) <= chain(best)) best = s;
     return best;
 }
 
+// Whether wavefronts that split k begin at different places of it (stream_start).  With few workgroups or a short k, finding out where costs what it gives (a
+// step of 28 layers of a 0.6B model 729 / 733 us).  Products that norm their input have the bits of those that do not: the rule is one for both.
+bool begins_anywhere(int64_t n, int64_t k) { return k > 2048 && n > 8 * kUnits; }
+
+template <bool GATED, int MT>
+void launch_shared(const GemmArgs& a, int tiles, int splits, hipStream_t st) {
+    const dim3 grid((unsigned)((a.n + 16 * tiles - 1) / (16 * tiles)), (unsigned)splits);
+#define GO(RT) case RT: hipLaunchKernelGGL((skinny_shared_kernel<RT, MT, GATED>), grid, dim3(256), 0, st, a); return
+    switch (tiles) { GO(2); GO(4); GO(6); GO(8); GO(10); GO(12); GO(14); GO(16); GO(20); }
+#undef GO
+}
+
 template <bool GATED>
 void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
     const int rows = rows_per_workgroup(a.m, a.n, a.k);
     const dim3 grid((unsigned)((a.n + rows - 1) / rows), (unsigned)splits);
-#define GO(RT, MT, NW, D) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED>), grid, dim3(64 * NW), 0, st, a)
-    if (a.m <= 16 && rows == 64) GO(4, 1, 4, 2);
-    else if (a.m <= 32 && rows == 64) GO(4, 2, 4, 2);
+    const bool turned = begins_anywhere(a.n, a.chunks * kKC);
+#define TURNED(RT, MT, NW, D, TURN) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED, TURN>), grid, dim3(64 * NW), 0, st, a)
+#define GO(RT, MT, NW, D) do { if (turned) TURNED(RT, MT, NW, D, 3); else TURNED(RT, MT, NW, D, 0); } while (0)
+    if (turned && a.m <= kFewRows && rows == 16 && a.n >= kFewMany && a.n < kMany) TURNED(1, 1, 4, 4, 4);      // in twos, as 32 rows with a norm in front
     else if (a.m <= 16 && rows == 16) GO(1, 1, 4, 4);
-    else if (a.m <= 16) GO(2, 1, 4, 3);
+    else if (a.m <= 16 && a.n >= kMany && a.k <= 2048) GO(2, 1, 4, 3);
     else if (a.m <= 32 && rows == 16) GO(1, 2, 4, 3);
-    else if (a.m <= 32 && rows == 32) GO(2, 2, 4, 2);
-    else if (a.m <= 32) GO(3, 2, 4, 2);
-    else if (a.m <= 64 && rows == 32) GO(2, 4, 4, 2);
+    else if (a.m <= 32 && rows == 48) GO(3, 2, 4, 2);
     else if (a.m <= 64 && rows == 48) GO(3, 4, 4, 2);
-    else if (a.m <= 64 && rows == 64 && grid.x * grid.y > 256) GO(4, 4, 2, 2);
-    else if (a.m <= 64 && rows == 64) GO(4, 4, 4, 2);
-    else if (a.m <= 64 && rows == 80 && a.n <= 80 * 512) GO(5, 4, 2, 2);      // all at once, two to a compute unit: n = 32000 60 -> 56 us
-    else if (a.m <= 64 && rows == 80) GO(5, 4, 4, 2);                // n = 50000: 92 us, with two wavefronts 106
-    else if (a.m <= 64 && rows == 160) GO(10, 4, 1, 2);
-    else if (a.m <= 64) GO(6, 4, 3, 2);
+    else if (a.m <= 64) {
+        // half as many rows where 64 leave every second compute unit idle: 64 of the batch 4096 x 1024 5.5 / 4.6 us, 1024 x 3072 5.6 / 4.6
+        const int tiles = a.n <= 5120 && grid.x * grid.y <= kUnits / 2 ? 2 : rows / 16;
+        if (a.m <= 16) launch_shared<GATED, 1>(a, tiles, splits, st);
+        else if (a.m <= 32) launch_shared<GATED, 2>(a, tiles, splits, st);
+        else launch_shared<GATED, 4>(a, tiles, splits, st);
+    }
     else if constexpr (!GATED) hipLaunchKernelGGL(skinny_gemm_kernel, grid, dim3(256), 0, st, a);
+#undef TURNED
 #undef GO
 }
 
@@ -541,9 +604,9 @@ void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
 //     1024 x 2048 8.0 / 8.6, 1024 x 4096 14.2 / 9.8; 24: 256 x 1024 4.6 / 5.5), and that very few do not fill the chip without one (512 x 768,
 //     40 5.0 / 6.7).
 //   many: a short k (36864 x 128, 16 of the batch 5.7 / 8.4), a long one (5128 x 16384 35.7 / 46.8; 24584 x 28672, 64 275 / 348) and more rows than a
-//     vocabulary has (262144 x 5120, 16 0.86 times as fast) are the vendor's.  Where a workgroup takes long, the last round of them has to be
-//     nearly full: 33 to 64 of the batch 24584 rows 19.7 / 23.0 (k = 1536) and 48.1 / 50.3 (4096), 65528 rows 0.76 to 1.0 times as fast, but 36864
-//     rows 1.25 and 151936 1.1 times; 17 to 32 16384 rows 94.8 / 114.8 (k = 16384) and 0.85 times as fast with k = 5120.
+//     vocabulary has (262144 x 5120, 16 0.86 times as fast) are the vendor's.  From 17 of the batch the line is where workgroups of 32 to 160 rows that
+//     stream by themselves fill their last round (33 to 64 of the batch 36864 rows 1.25 times as fast as the vendor, 65528 0.76 to 1.0 times).  Those that
+//     share their steps are ahead behind it, too (64 of the batch 27648 x 4096 50 / 37, 64512 x 4096 121 / 80): widening it is open.
 bool pays(int64_t m, int64_t n, int64_t k, bool reduced) {
     if (m > 64) return n <= 5120 && k >= 2048;
     if (n <= 5120) {
@@ -552,10 +615,11 @@ bool pays(int64_t m, int64_t n, int64_t k, bool reduced) {
         return n >= 2048 && (k == 2048 || choose_splits(m, n, k) == 1);
     }
     if ((k < 512 && n > 20480) || k > 12288 || n > 163840) return false;
-    const int64_t rows = rows_per_workgroup(m, n, k), groups = (n + rows - 1) / rows, rounds = (groups + 255) / 256;
     if (m <= 16) return true;
-    if (m <= 32) return k <= 2048 || 10 * groups >= 7 * 256 * rounds;
-    return n <= 24576 || 20 * groups >= 17 * 256 * rounds;
+    const int64_t rows = m <= 32 ? (n >= 8192 ? 48 : 32) : n <= 8192 ? 32 : n >= 65536 ? 160 : n > 24576 ? 80 : 16 * ((n + 4095) / 4096);
+    const int64_t groups = (n + rows - 1) / rows, rounds = (groups + kUnits - 1) / kUnits;
+    if (m <= 32) return k <= 2048 || 10 * groups >= 7 * kUnits * rounds;
+    return n <= 24576 || 20 * groups >= 17 * kUnits * rounds;
 }
 
 }  // namespace
@@ -639,20 +703,25 @@ int launch_norm_product(const GemmArgs& a, const NormSource& f, hipStream_t st) 
     const int pieces = a.m * ((a.k + kNormGroup - 1) / kNormGroup), rows = a.n >= kFewMany ? 32 : 16;
     const size_t lds = 4 * 4 * stream_stage_bytes(rows / 16, 0) + (size_t)a.m * (2 * a.k + kFewPad) + kFewRows * 8 * sizeof(float);
     const dim3 grid((unsigned)((a.n + rows - 1) / rows));
-#define GO(RT, NP) do { \
+    const bool turned = begins_anywhere(a.n, a.k);
+#define GO(RT, NP, TURN) do { \
         if (lds > 60 * 1024) { \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&norm_product_kernel<RT, NP, GATED>), \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&norm_product_kernel<RT, NP, GATED, TURN>), \
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
             if (e != hipSuccess) return (int)e; \
         } \
-        hipLaunchKernelGGL((norm_product_kernel<RT, NP, GATED>), grid, dim3(256), lds, st, a, f); \
+        hipLaunchKernelGGL((norm_product_kernel<RT, NP, GATED, TURN>), grid, dim3(256), lds, st, a, f); \
     } while (0)
+    // four pieces: one row of at most 2048, or two of 1024
     if (rows == 16) {
-        if (pieces <= 4) GO(1, 1);
-        else GO(1, 2);
+        if (pieces <= 4) GO(1, 1, 0);
+        else if (turned) GO(1, 2, 3);
+        else GO(1, 2, 0);
     } else {
-        if (pieces <= 4) GO(2, 1);
-        else GO(2, 2);
+        if (pieces <= 4) GO(2, 1, 0);
+        else if (turned && a.n < kMany) GO(2, 2, 3);
+        else if (turned) GO(2, 2, 2);          // as 16 rows without a norm, which a vocabulary meets: 151936 x 4096 174 us, in twos 180
+        else GO(2, 2, 0);
     }
 #undef GO
     return (int)hipGetLastError();

@@ -7,6 +7,8 @@
 // requests of 64 bytes of 16 rows straight into operand registers 52.8 us (3.8 TB/s), this 35.3 us (5.7 TB/s); a read of the weights
 // alone in lines takes 31.5 us with the hint and 33.7 without, in halves of lines 37.7.
 #pragma once
+#include <type_traits>
+
 #include "elem.h"
 
 constexpr int kStreamK = 64;                       // elements of a step
@@ -16,10 +18,16 @@ constexpr int stream_stage_bytes(int rt, int mt) { return 2048 * (rt + mt); }
 __device__ __forceinline__ int stream_row() { return (threadIdx.x & 63) >> 3; }
 __device__ __forceinline__ int stream_col() { return 8 * ((threadIdx.x & 7) ^ ((threadIdx.x & 63) >> 3)); }
 
+// Where a workgroup begins its walk over k, of `steps`; behind the end it goes on at the front.  Rows of weights lie a power of two or a small multiple of
+// one apart, so workgroups that all begin at the front read the same few channels of memory at any one time, and the same lines of the activations.
+// Every eighth workgroup goes to the same die, whose 32 compute units begin evenly spread: `turn` counts eights of workgroups.  Everybody at the front / this, 64 of the
+// batch, us: gate and up of 24576 x 4096 42.8 / 37.2, 65536 x 4096 108 / 90, 8192 x 4096 20.8 / 16.6; four: 16384 x 2048 14.9 / 12.6.
+__device__ __forceinline__ int stream_start(int turn, int steps) { return (int)((turn & 31) * (unsigned)steps >> 5); }
+
 // w[i], x[i]: this lane's row stream_row() + 8 i of the weights and of the activations, at the first element of k (16-byte aligned);
-// k: elements, a multiple of eight; ring: D * stream_stage_bytes(RT, MT) bytes of the wavefront's own.  Adds to acc[r][t] (lane (g, n):
+// TURN: 0, or 2^TURN workgroups begin at one place (stream_start); k: elements, a multiple of eight; ring: D * stream_stage_bytes(RT, MT) bytes of the wavefront's own.  Adds to acc[r][t] (lane (g, n):
 // row n of tile t of x, rows 4 g + e of tile r of w) what the steps `wave`, `wave` + NW, ... contribute.
-template <int RT, int MT, int NW, int D>
+template <int RT, int MT, int NW, int D, int TURN>
 __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT], const __bf16* const (&x)[2 * MT], int k, int wave,
                                                unsigned char* ring, f32x4_t (&acc)[RT][MT]) {
     constexpr int kRequests = 2 * (RT + MT), kStage = stream_stage_bytes(RT, MT);
@@ -28,8 +36,10 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
     const int all = (k + kStreamK - 1) / kStreamK, steps = all > wave ? (all - wave + NW - 1) / NW : 0;
     const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ring);
     // Inline assembly, since the compiler would put a wait for all requests in front of every read of LDS.  Nothing else here uses M0.
-    auto request = [&](int s, int stage) {
-        const int at = (s * NW + wave) * kStreamK + col, from = at < k ? at : 0;       // behind the end: something, which meets zeros
+    int ahead = TURN ? stream_start((int)blockIdx.x >> TURN, steps) : 0, now = ahead;      // the steps to be requested and to be multiplied next
+    auto request = [&](int stage) {
+        const int at = (ahead * NW + wave) * kStreamK + col, from = at < k ? at : 0;   // behind the end: something, which meets zeros
+        ahead = TURN && ahead + 1 == steps ? 0 : ahead + 1;
 #pragma unroll
         for (int i = 0; i < kRequests; ++i) {
             const uint32_t to = base + stage * kStage + 1024 * i;
@@ -41,7 +51,7 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
     };
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        if (d < steps) request(d, d);
+        if (d < steps) request(d);
     const int place = 128 * n + 16 * (g ^ (n & 7));
     int stage = 0;
     for (int s = 0; s < steps; ++s) {
@@ -61,8 +71,9 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
         }
         __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // read before the stage is filled again
         __builtin_amdgcn_sched_barrier(0);
-        if (s + D < steps) request(s + D, stage);
-        const int first = (s * NW + wave) * kStreamK;
+        if (s + D < steps) request(stage);
+        const int first = (now * NW + wave) * kStreamK;
+        now = TURN && now + 1 == steps ? 0 : now + 1;
         if (first + kStreamK > k)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
@@ -82,7 +93,7 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
 // The same past activations that lie in LDS as a whole: only the weights are requested, and `before` runs behind the first requests, while
 // they are on their way; it puts the activations where x points (this lane's row, at element 8 g of the first step) and ends with a barrier.
 // k: a multiple of kStreamK; ring: D * stream_stage_bytes(RT, 0) bytes.
-template <int RT, int NW, int D, class Before>
+template <int RT, int NW, int D, int TURN, class Before>
 __device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 * RT], const unsigned char* x, int k, int wave, unsigned char* ring,
                                                     Before before, f32x4_t (&acc)[RT][1]) {
     constexpr int kRequests = 2 * RT, kStage = stream_stage_bytes(RT, 0);
@@ -90,15 +101,17 @@ __device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 *
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, col = stream_col();
     const int all = k / kStreamK, steps = all > wave ? (all - wave + NW - 1) / NW : 0;
     const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ring);
-    auto request = [&](int s, int stage) {
-        const int from = (s * NW + wave) * kStreamK + col;
+    int ahead = TURN ? stream_start((int)blockIdx.x >> TURN, steps) : 0, now = ahead;
+    auto request = [&](int stage) {
+        const int from = (ahead * NW + wave) * kStreamK + col;
+        ahead = TURN && ahead + 1 == steps ? 0 : ahead + 1;
 #pragma unroll
         for (int i = 0; i < kRequests; ++i)
             __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(w[i] + from), "s"(base + stage * kStage + 1024 * i) : "memory", "m0");
     };
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        if (d < steps) request(d, d);
+        if (d < steps) request(d);
     before();
     const int place = 128 * n + 16 * (g ^ (n & 7));
     int stage = 0;
@@ -111,7 +124,8 @@ __device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 *
         else __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         bf16x8_t a[RT][2], b[2];
         const unsigned char* p = ring + stage * kStage;
-        const unsigned char* from = x + 2 * kStreamK * (s * NW + wave);
+        const unsigned char* from = x + 2 * kStreamK * (now * NW + wave);
+        now = TURN && now + 1 == steps ? 0 : now + 1;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
@@ -120,7 +134,7 @@ __device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 *
         }
         __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // read before the stage is filled again
         __builtin_amdgcn_sched_barrier(0);
-        if (s + D < steps) request(s + D, stage);
+        if (s + D < steps) request(stage);
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -150,3 +164,91 @@ __device__ __forceinline__ void stream_reduce(const f32x4_t (&acc)[RT][MT], int 
         f(q / MT, q % MT, sum);
     }
 }
+
+// Rows of weights past activations that the four wavefronts of a workgroup share: they go through one ring of D steps, of which every wavefront brings
+// a quarter, and a wavefront multiplies RT / WR tiles of weight rows by all MT tiles of the batch: with all of a step's elements (WR = 4), or with one half
+// of them (WR = 2; the sums of the two halves remain to be added).  One barrier a step: behind it the step has arrived for everybody, and the place
+// of the one before is free.
+//
+// A wavefront that streams by itself (above) brings the batch for its own rows alone, and two steps of that are all that LDS holds; here the batch
+// takes 8 KB of a step of up to 48.  And in eight times as many smaller steps what is under way hardly falls while one is multiplied.
+template <int RT, int MT>
+struct SharedStream {
+    // Up to 96 rows leave room for a second workgroup on the compute unit, which begins while the other one ends
+    static constexpr int kWaves = 4, WR = RT <= 6 || RT % 4 ? 2 : 4, kTiles = RT / WR, KH = WR == 4 ? 2 : 1;
+    static constexpr int kStage = stream_stage_bytes(RT, MT), kFit = (RT <= 6 ? 80 : 160) * 1024 / kStage, D = kFit < 12 ? kFit : 12;
+    static constexpr int kOfWeights = 2 * RT / kWaves, kRequests = kOfWeights + (2 * MT + kWaves - 1) / kWaves;
+    static_assert(RT % WR == 0 && 2 * RT % kWaves == 0 && D >= 3 && (D - 2) * kRequests <= 63, "requests in flight are counted in six bits");
+    const __bf16* from[kRequests];
+    uint32_t to[kRequests];
+    int ahead, steps;
+
+    // weights(i), batch(i): this lane's row stream_row() + 8 i of either, at the first element of k (a multiple of kStreamK)
+    template <class Weights, class Batch>
+    __device__ __forceinline__ SharedStream(int k, int wave, const unsigned char* ring, Weights weights, Batch batch) {
+        const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)ring;
+#pragma unroll
+        for (int j = 0; j < kRequests; ++j) {
+            const int i = wave + kWaves * j, of_batch = (i - 2 * RT) & (2 * MT - 1);       // one too many repeats another
+            from[j] = (j < kOfWeights ? weights(i) : batch(of_batch)) + stream_col();
+            to[j] = __builtin_amdgcn_readfirstlane(base + 1024 * (j < kOfWeights ? i : 2 * RT + of_batch));
+        }
+        steps = k / kStreamK;
+        ahead = k < 2048 ? 0 : stream_start((int)blockIdx.x >> 3, steps);
+    }
+    __device__ __forceinline__ void request(int stage) {
+#pragma unroll
+        for (int j = 0; j < kRequests; ++j) {
+            const uint32_t at = to[j] + stage * kStage;
+            if (j < kOfWeights)
+                __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(from[j] + ahead * kStreamK), "s"(at) : "memory", "m0");
+            else
+                __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(from[j] + ahead * kStreamK), "s"(at) : "memory", "m0");
+        }
+        ahead = ahead + 1 == steps ? 0 : ahead + 1;
+    }
+    // Adds to acc[r][t]: tile kTiles (wave % WR) + r of the weights, tile t of the batch; layout as of stream_product
+    __device__ __forceinline__ void product(int wave, const unsigned char* ring, f32x4_t (&acc)[kTiles][MT]) {
+        const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, first = wave % WR * kTiles;
+        const int place = 128 * n + 16 * (g ^ (n & 7)) ^ (KH == 1 ? 64 * (wave / WR) : 0);
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (d < steps) request(d);
+        int stage = 0, free = D - 1;                   // where step s lies, and where the one D - 1 behind it will
+        auto step = [&](int s, auto behind) __attribute__((always_inline)) {       // behind: steps that have been requested and are not waited for
+            __asm__ volatile("s_waitcnt vmcnt(%0)" :: "n"(decltype(behind)::value * kRequests) : "memory");
+            __builtin_amdgcn_s_barrier();
+            __asm__ volatile("" ::: "memory");
+            bf16x8_t a[kTiles][KH], b[MT][KH];
+            const unsigned char* p = ring + stage * kStage;
+#pragma unroll
+            for (int h = 0; h < KH; ++h) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) b[t][h] = *reinterpret_cast<const bf16x8_t*>(p + 2048 * (RT + t) + (place ^ (64 * h)));
+#pragma unroll
+                for (int r = 0; r < kTiles; ++r) a[r][h] = *reinterpret_cast<const bf16x8_t*>(p + 2048 * (first + r) + (place ^ (64 * h)));
+            }
+            if (s + D - 1 < steps) request(free);
+            __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // read before the next barrier
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int h = 0; h < KH; ++h)
+#pragma unroll
+                for (int r = 0; r < kTiles; ++r)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][h], b[t][h], acc[r][t], 0, 0, 0);
+            stage = stage + 1 == D ? 0 : stage + 1;
+            free = free + 1 == D ? 0 : free + 1;
+        };
+        int s = 0;
+        for (; s + D - 2 < steps; ++s) step(s, std::integral_constant<int, D - 2>{});
+        last_steps<D - 3>(s, step);
+    }
+    template <int B, class Step>
+    __device__ __forceinline__ void last_steps(int s, Step& step) {
+        if constexpr (B >= 0) {
+            if (s + B == steps - 1) step(s++, std::integral_constant<int, B>{});
+            last_steps<B - 1>(s, step);
+        }
+    }
+};

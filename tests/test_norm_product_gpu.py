@@ -62,3 +62,14 @@ def test_stale_pieces_are_refused(gpu):
     ops.SplitKSum(part, BF16)
     with pytest.raises(RuntimeError, match="overwritten"):
         ops.norm_linear(old, _rand(gen, 1024), 1e-6, _rand(gen, 2, 1024), _rand(gen, 4096, 1024))
+
+
+@pytest.mark.parametrize("n,k", [(4112, 4096), (16400, 2176), (40976, 4096)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_bits_of_the_two_launches_wherever_a_row_begins(gpu, n, k, gated):
+    """As above with a long k, whose sums begin at different places of it: workgroups of 16 and of 32 rows of weights begin alike for the same row."""
+    gen = torch.Generator().manual_seed(n + k)
+    w, gain, x = _rand(gen, n, k, std=0.05), _rand(gen, k), _rand(gen, 1, k)
+    got, _ = ops.norm_linear(x, gain, 1e-6, None, w, gated)
+    normed = ops.rms_norm(x, gain, 1e-6)
+    assert torch.equal(got, ops.gate_up_silu(normed, w) if gated else ops.linear(normed, w))

@@ -203,3 +203,22 @@ def test_split_products_on_two_streams_do_not_meet(gpu):
         minus = ops.rms_norm(second, gamma, 1e-6)
     other.synchronize()
     assert torch.equal(ops.rms_norm(first, gamma, 1e-6), want) and torch.equal(minus, -want)
+
+
+@pytest.mark.parametrize("m", [9, 24, 64])
+@pytest.mark.parametrize("n", [8176, 16368, 24560, 32752, 40944, 49136, 57328, 65520, 81904])
+@pytest.mark.parametrize("k", [2176, 256])
+def test_steps_that_wavefronts_share(gpu, m, n, k):
+    """Exact sums for 2 to 20 tiles of weight rows per workgroup, the last one ragged: fewer steps of k than are under way at a time, and a walk over k that
+    begins somewhere else in every workgroup and goes on at the front.  Gate and up in one launch round where the two do."""
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = torch.randint(-1, 2, (m, k + 8), generator=g, device=gpu).to(torch.bfloat16)[:, 8:]
+    w = torch.randint(-1, 2, (n, k), generator=g, device=gpu, dtype=torch.int8).to(torch.bfloat16)
+    want = reference(x, w)
+    assert want.abs().max() <= 256                      # representable in bf16 without rounding
+    assert torch.equal(ops.skinny_linear(x, w[:-8]).float(), want[:, :-8])
+    both, fused = (torch.empty(m, n // 2, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    ops.silu_and_mul(both, want.to(torch.bfloat16))
+    rc = ops._lib.load().infer_skinny_gate_silu_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), fused.data_ptr(), n // 2, m, n // 2, k,
+                                                     torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(fused, both)
