@@ -5,7 +5,7 @@
 //   moe_scatter_kernel    rows sorted by expert: place of every choice, token and expert of every place, row tiles
 //   moe_block_kernel      products of many rows per expert: 256 rows x 256 columns per workgroup, straight from memory to LDS
 //   moe_tile_kernel       products of large row tiles: 128 rows x 128 columns per workgroup, through registers to LDS
-//   moe_row_kernel        products of up to 32 rows (decode): the weights stream past the rows, k split over wavefronts
+//   moe_row_kernel        products of up to 32 rows (decode): the weights stream past the rows; wavefronts split k or share its steps
 //   moe_any_kernel        any size and element type
 //
 // The first product takes gate and up columns side by side and stores act = silu(gate) * up, the second stores one row per
@@ -604,62 +604,93 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
     }
 }
 
-// A workgroup: up to 32 rows of one expert x 16 rows of W (GATED: 8 gate and 8 up), which stream past them; the second half of the rows
+// A workgroup: up to 32 rows of one expert x some rows of W (a tile: 16, GATED: 8 gate and 8 up), which stream past them; the second half of the rows
 // costs only where there are that many.  64 rows, three of 16 experts of 3072 x 4096: 258 us with 32 rows of W past 16 rows through
-// operand registers, 181 us now (5.9 TB/s of weights).
-constexpr int kSmallRows = 32, kRowWaves = 4;
+// operand registers, 181 us with one tile and wavefronts that split k (5.9 TB/s of weights).  Two tiles and wavefronts that share the steps of k read the
+// rows half as often, and every step is on its way for all of the workgroup: experts of a step of 64 rows (14 of 4096 x 3072, three each) 205 / 188 us, 100
+// rows 242 / 205, 130 rows 277 / 234; 14 of 1024 x 768, 16 rows the second product 6.9 / 5.8, 120 rows 9.1 / 6.6.  Four to eight tiles leave compute units
+// waiting at the end (64 rows 195 to 198), and so do two where few experts have rows: one token 62.8 / 67.1, 2 91.6 / 93.3, 9 160.3 / 160.5.
+constexpr int kSmallRows = 32, kRowWaves = 4, kSharedTiles = 2;
 constexpr int kRowRing = 3 * stream_stage_bytes(1, 1);           // of a wavefront: three steps with 16 rows, two with 32
 static_assert(2 * stream_stage_bytes(1, 2) <= kRowRing, "both rings fit");
+
+// Start of row 8 i + stream_row() of the rows of W that lie at column c0 and on
+template <bool GATED>
+__device__ __forceinline__ const __bf16* moe_weight_row(const GemmArgs<__bf16>& a, int expert, int c0, int i) {
+    int col = c0 + stream_row() + 8 * (GATED ? i / 2 : i);
+    col = col < a.cols ? col : a.cols - 1;
+    return a.w + (int64_t)expert * a.w_expert + (int64_t)(GATED && (i & 1) ? a.up_row + col : col) * a.w_stride;
+}
+// Of the rows that are multiplied
+__device__ __forceinline__ const __bf16* moe_input_row(const GemmArgs<__bf16>& a, int first, int rows, int i) {
+    const int r = stream_row() + 8 * i, xr = first + (r < rows ? r : rows - 1);
+    return a.x + (int64_t)(a.row_token ? a.row_token[xr] : xr) * a.x_stride;
+}
+// Four sums of row r at column c + 4 g
+template <bool GATED>
+__device__ __forceinline__ void moe_finish(const GemmArgs<__bf16>& a, int first, int rows, int r, int c, f32x4_t sum) {
+    const int g = (threadIdx.x & 63) >> 4;
+    if constexpr (GATED) {                             // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float up = __shfl_xor(sum[e], 32, 64);
+            sum[e] = silu_f(sum[e]) * up;
+        }
+        if (g >= 2) return;
+    }
+    if (r >= rows) return;
+    c += 4 * g;
+    bf16x4_t v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (__bf16)(c + e < a.cols ? sum[e] : 0.f);
+    if (c + 4 <= a.out_cols) *reinterpret_cast<bf16x4_t*>(a.out + (int64_t)(first + r) * a.out_stride + c) = v;       // out_cols is a multiple of eight
+}
 template <bool GATED, int MT>
 __device__ __forceinline__ void moe_row_product(const GemmArgs<__bf16>& a, int expert, int first, int rows, int c0, unsigned char* lds) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = threadIdx.x & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const __bf16* w[2];
     const __bf16* x[2 * MT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        int col = c0 + stream_row() + (GATED ? 0 : 8 * i);
-        col = col < a.cols ? col : a.cols - 1;
-        w[i] = a.w + (int64_t)expert * a.w_expert + (int64_t)(GATED && i ? a.up_row + col : col) * a.w_stride;
-    }
+    for (int i = 0; i < 2; ++i) w[i] = moe_weight_row<GATED>(a, expert, c0, i);
 #pragma unroll
-    for (int i = 0; i < 2 * MT; ++i) {
-        const int r = stream_row() + 8 * i, xr = first + (r < rows ? r : rows - 1);
-        x[i] = a.x + (int64_t)(a.row_token ? a.row_token[xr] : xr) * a.x_stride;
-    }
+    for (int i = 0; i < 2 * MT; ++i) x[i] = moe_input_row(a, first, rows, i);
     f32x4_t acc[1][MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[0][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     stream_product<1, MT, kRowWaves, MT == 1 ? 3 : 2, 0>(w, x, a.k, wave, lds + wave * kRowRing, acc);
-    stream_reduce<1, MT, kRowWaves>(acc, wave, lds, [&](int, int t, f32x4_t sum) {
-        const int r = 16 * t + n;
-        __bf16* o = a.out + (int64_t)(first + r) * a.out_stride;
-        if constexpr (GATED) {                         // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float up = __shfl_xor(sum[e], 32, 64);
-                sum[e] = silu_f(sum[e]) * up;
-            }
-            if (g >= 2) return;
-        }
-        if (r >= rows) return;
-        const int c = c0 + 4 * g;
-        bf16x4_t v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (__bf16)(c + e < a.cols ? sum[e] : 0.f);
-        if (c + 4 <= a.out_cols) *reinterpret_cast<bf16x4_t*>(o + c) = v;       // out_cols is a multiple of eight
-    });
+    stream_reduce<1, MT, kRowWaves>(acc, wave, lds, [&](int, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0, sum); });
 }
-template <bool GATED>
+// The same, two tiles of W and shared steps; k: a multiple of 64
+template <bool GATED, int MT>
+__device__ __forceinline__ void moe_shared_product(const GemmArgs<__bf16>& a, int expert, int first, int rows, int c0, unsigned char* lds) {
+    using Stream = SharedStream<kSharedTiles, MT>;
+    static_assert(Stream::WR == 2 && Stream::kTiles == 1, "a wavefront has one tile of W and half of every step");
+    const int n = threadIdx.x & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tile = wave % 2;
+    Stream stream(a.k, wave, lds, [&](int i) { return moe_weight_row<GATED>(a, expert, c0, i); }, [&](int i) { return moe_input_row(a, first, rows, i); });
+    f32x4_t acc[1][MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[0][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    stream.product(wave, lds, acc);
+    stream_reduce<1, MT, 2>(acc, wave / 2, lds + tile * (2048 * MT),
+                            [&](int, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0 + (GATED ? 8 : 16) * tile, sum); });
+}
+template <bool GATED, bool SHARED>
 __global__ void __launch_bounds__(64 * kRowWaves) moe_row_kernel(GemmArgs<__bf16> a) {
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[kRowWaves * kRowRing];
+    constexpr int kShared1 = SharedStream<kSharedTiles, 1>::kRing, kShared2 = SharedStream<kSharedTiles, 2>::kRing;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[!SHARED ? kRowWaves * kRowRing : kShared1 > kShared2 ? kShared1 : kShared2];
     clear_counts(a);
     const int tile = blockIdx.x / a.col_blocks, cb = blockIdx.x % a.col_blocks;
     const int expert = a.tiles[2 * tile];
     if (expert < 0 || expert >= a.experts) return;
     const int first = a.offsets[expert] + a.tiles[2 * tile + 1], end = a.offsets[expert + 1];
-    const int rows = end - first < kSmallRows ? end - first : kSmallRows, c0 = cb * (GATED ? 8 : 16);
-    if (rows <= 16) moe_row_product<GATED, 1>(a, expert, first, rows, c0, lds);
-    else moe_row_product<GATED, 2>(a, expert, first, rows, c0, lds);
+    const int rows = end - first < kSmallRows ? end - first : kSmallRows, c0 = cb * (GATED ? 8 : 16) * (SHARED ? kSharedTiles : 1);
+    if constexpr (SHARED) {
+        if (rows <= 16) moe_shared_product<GATED, 1>(a, expert, first, rows, c0, lds);
+        else moe_shared_product<GATED, 2>(a, expert, first, rows, c0, lds);
+    } else {
+        if (rows <= 16) moe_row_product<GATED, 1>(a, expert, first, rows, c0, lds);
+        else moe_row_product<GATED, 2>(a, expert, first, rows, c0, lds);
+    }
 }
 
 // one wavefront per (place, four columns)
@@ -690,7 +721,7 @@ __global__ void __launch_bounds__(kThreads) moe_any_kernel(GemmArgs<T> a) {
 bool size_in(int64_t v, int64_t lo, int64_t hi) { return v >= lo && v <= hi; }
 
 template <class T>
-int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t max_places, hipStream_t st) {
+int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t choices, int64_t max_places, hipStream_t st) {
     const dim3 block(kThreads);
     int64_t grid;
     if constexpr (sizeof(T) == 2) {
@@ -703,16 +734,20 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t max_places, hipStrea
             return (int)hipGetLastError();
         }
         if (tile_rows == kBigRows || tile_rows == kSmallRows) {
-            const int per = tile_rows == kBigRows ? (gated ? 64 : 128) : (gated ? 8 : 16);
+            const bool shared = tile_rows == kSmallRows && a.k % kStreamK == 0 && choices >= 2 * a.experts;
+            const int per = tile_rows == kBigRows ? (gated ? 64 : 128) : (gated ? 8 : 16) * (shared ? kSharedTiles : 1);
             a.col_blocks = (a.out_cols + per - 1) / per;
             grid = (int64_t)a.max_tiles * a.col_blocks;
             if (grid > 0x7fffffff) return INFER_KV_EINVAL;
             if (tile_rows == kBigRows) {
                 if (gated) hipLaunchKernelGGL((moe_tile_kernel<true>), dim3((unsigned)grid), block, 0, st, a);
                 else hipLaunchKernelGGL((moe_tile_kernel<false>), dim3((unsigned)grid), block, 0, st, a);
+            } else if (shared) {
+                if (gated) hipLaunchKernelGGL((moe_row_kernel<true, true>), dim3((unsigned)grid), block, 0, st, a);
+                else hipLaunchKernelGGL((moe_row_kernel<false, true>), dim3((unsigned)grid), block, 0, st, a);
             } else {
-                if (gated) hipLaunchKernelGGL((moe_row_kernel<true>), dim3((unsigned)grid), block, 0, st, a);
-                else hipLaunchKernelGGL((moe_row_kernel<false>), dim3((unsigned)grid), block, 0, st, a);
+                if (gated) hipLaunchKernelGGL((moe_row_kernel<true, false>), dim3((unsigned)grid), block, 0, st, a);
+                else hipLaunchKernelGGL((moe_row_kernel<false, false>), dim3((unsigned)grid), block, 0, st, a);
             }
             return (int)hipGetLastError();
         }
@@ -799,11 +834,11 @@ extern "C" int infer_moe(int elem, const void* h, int64_t h_stride, const void* 
         hipLaunchKernelGGL(moe_scatter_kernel, dim3((unsigned)((choices + kThreads - 1) / kThreads)), dim3(kThreads), 0, st, s);
         GemmArgs<T> up{(const T*)h, h_stride, row_token, row_expert, offsets, tiles, (const T*)gate_up, 2 * ff * width, width, (int)width, (int)ff,
                        (int)ff, (T*)act, ff_pad, (int)ff_pad, counts, (int)experts, (int)experts, (int)max_tiles, 0};
-        int rc = gemm(up, true, tile_rows, max_places, st);
+        int rc = gemm(up, true, tile_rows, choices, max_places, st);
         if (rc) return rc;
         GemmArgs<T> dn{(const T*)act, ff_pad, nullptr, row_expert, offsets, tiles, (const T*)down, width * ff_pad, ff_pad, (int)ff_pad, (int)width,
                        0, (T*)out, width, (int)width, nullptr, 0, (int)experts, (int)max_tiles, 0};
-        return gemm(dn, false, tile_rows, max_places, st);
+        return gemm(dn, false, tile_rows, choices, max_places, st);
     };
     if (elem == INFER_ELEM_BF16) return go(__bf16(0.f));
     if (elem == INFER_ELEM_F32) return go(0.f);

@@ -252,9 +252,9 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
 template <int RT, int MT, bool GATED>
 __global__ void __launch_bounds__(256) skinny_shared_kernel(GemmArgs a) {
     using Stream = SharedStream<RT, MT>;
-    constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR, kRing = Stream::D * Stream::kStage;
-    static_assert(WK == 1 || 4096 * TW * MT <= kRing, "the sums fit the ring");
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing];
+    constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR;
+    static_assert(WK == 1 || 4096 * TW * MT <= Stream::kRing, "the sums fit the ring");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[Stream::kRing];
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int half = a.n / 2, n0 = blockIdx.x * (GATED ? 8 : 16) * RT, split = blockIdx.y, wr = wave % WR;
     const int64_t k_lo = (int64_t)split * a.chunks * kKC;

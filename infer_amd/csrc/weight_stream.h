@@ -176,7 +176,7 @@ template <int RT, int MT>
 struct SharedStream {
     // Up to 96 rows leave room for a second workgroup on the compute unit, which begins while the other one ends
     static constexpr int kWaves = 4, WR = RT <= 6 || RT % 4 ? 2 : 4, kTiles = RT / WR, KH = WR == 4 ? 2 : 1;
-    static constexpr int kStage = stream_stage_bytes(RT, MT), kFit = (RT <= 6 ? 80 : 160) * 1024 / kStage, D = kFit < 12 ? kFit : 12;
+    static constexpr int kStage = stream_stage_bytes(RT, MT), kFit = (RT <= 6 ? 80 : 160) * 1024 / kStage, D = kFit < 12 ? kFit : 12, kRing = D * kStage;
     static constexpr int kOfWeights = 2 * RT / kWaves, kRequests = kOfWeights + (2 * MT + kWaves - 1) / kWaves;
     static_assert(RT % WR == 0 && 2 * RT % kWaves == 0 && D >= 3 && (D - 2) * kRequests <= 63, "requests in flight are counted in six bits");
     const __bf16* from[kRequests];

@@ -646,6 +646,13 @@ def test_moe_rows_around_the_tiles_that_weights_stream_past(gpu, width, ff, n):
     close(r.weights, (np.exp(h @ w[0].T) / np.exp(h @ w[0].T).sum(-1, keepdims=True))[:, 2:3], 1e-5)
 
 
+@pytest.mark.parametrize("width,ff", [(2304, 136), (128, 2176)])
+@pytest.mark.parametrize("n", [7, 8, 17, 40])
+def test_moe_rows_of_a_long_k(gpu, width, ff, n):
+    """The same around the line from which wavefronts share the steps of k, with more steps than are under way at a time and walks that begin inside."""
+    test_moe_rows_around_the_tiles_that_weights_stream_past(gpu, width, ff, n)
+
+
 def test_bad_arguments_are_refused(gpu):
     z = torch.zeros(8, 64, device=gpu)
     counts = torch.zeros(4, dtype=torch.int32, device=gpu)
