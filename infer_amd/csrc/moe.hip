@@ -5,6 +5,7 @@
 //   moe_scatter_kernel    rows sorted by expert: place of every choice, token and expert of every place, row tiles
 //   moe_block_kernel      products of many rows per expert: 256 rows x 256 columns per workgroup, straight from memory to LDS
 //   moe_tile_kernel       products of large row tiles: 128 rows x 128 columns per workgroup, through registers to LDS
+//   moe_span_kernel       products of up to 128 rows at a time: the weights pass the rows once
 //   moe_row_kernel        products of up to 32 rows (decode): the weights stream past the rows; wavefronts split k or share its steps
 //   moe_any_kernel        any size and element type
 //
@@ -660,19 +661,29 @@ __device__ __forceinline__ void moe_row_product(const GemmArgs<__bf16>& a, int e
     stream_product<1, MT, kRowWaves, MT == 1 ? 3 : 2, 0>(w, x, a.k, wave, lds + wave * kRowRing, acc);
     stream_reduce<1, MT, kRowWaves>(acc, wave, lds, [&](int, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0, sum); });
 }
-// The same, two tiles of W and shared steps; k: a multiple of 64
-template <bool GATED, int MT>
+// The same, RT tiles of W and up to 16 MT rows, steps shared; k: a multiple of 64
+template <bool GATED, int RT, int MT>
 __device__ __forceinline__ void moe_shared_product(const GemmArgs<__bf16>& a, int expert, int first, int rows, int c0, unsigned char* lds) {
-    using Stream = SharedStream<kSharedTiles, MT>;
-    static_assert(Stream::WR == 2 && Stream::kTiles == 1, "a wavefront has one tile of W and half of every step");
-    const int n = threadIdx.x & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tile = wave % 2;
+    using Stream = SharedStream<RT, MT>;
+    constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR;
+    static_assert(WK == 1 || 4096 * TW * MT <= Stream::kRing, "the sums fit the ring");
+    const int n = threadIdx.x & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave % WR;
     Stream stream(a.k, wave, lds, [&](int i) { return moe_weight_row<GATED>(a, expert, c0, i); }, [&](int i) { return moe_input_row(a, first, rows, i); });
-    f32x4_t acc[1][MT];
+    f32x4_t acc[TW][MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[0][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < TW; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     stream.product(wave, lds, acc);
-    stream_reduce<1, MT, 2>(acc, wave / 2, lds + tile * (2048 * MT),
-                            [&](int, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0 + (GATED ? 8 : 16) * tile, sum); });
+    auto finish = [&](int r, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0 + (GATED ? 8 : 16) * (wr * TW + r), sum); };
+    if constexpr (WK == 1) {
+#pragma unroll
+        for (int r = 0; r < TW; ++r)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) finish(r, t, acc[r][t]);
+    } else {
+        stream_reduce<TW, MT, WK>(acc, wave / WR, lds + wr * (1024 * WK * TW * MT), finish);
+    }
 }
 template <bool GATED, bool SHARED>
 __global__ void __launch_bounds__(64 * kRowWaves) moe_row_kernel(GemmArgs<__bf16> a) {
@@ -685,11 +696,40 @@ __global__ void __launch_bounds__(64 * kRowWaves) moe_row_kernel(GemmArgs<__bf16
     const int first = a.offsets[expert] + a.tiles[2 * tile + 1], end = a.offsets[expert + 1];
     const int rows = end - first < kSmallRows ? end - first : kSmallRows, c0 = cb * (GATED ? 8 : 16) * (SHARED ? kSharedTiles : 1);
     if constexpr (SHARED) {
-        if (rows <= 16) moe_shared_product<GATED, 1>(a, expert, first, rows, c0, lds);
-        else moe_shared_product<GATED, 2>(a, expert, first, rows, c0, lds);
+        if (rows <= 16) moe_shared_product<GATED, kSharedTiles, 1>(a, expert, first, rows, c0, lds);
+        else moe_shared_product<GATED, kSharedTiles, 2>(a, expert, first, rows, c0, lds);
     } else {
         if (rows <= 16) moe_row_product<GATED, 1>(a, expert, first, rows, c0, lds);
         else moe_row_product<GATED, 2>(a, expert, first, rows, c0, lds);
+    }
+}
+
+// A workgroup: four or eight tiles of W past up to 128 rows of one expert at a time, which the four wavefronts share (SharedStream), for as many rows as a
+// decode batch or a few short prompts bring.  The weights bound such a product, each of which should pass once: tiles of 32 rows read them again for
+// every 32 rows, and blocks and tiles of 128 and 256 rows compute what there is not.  A workgroup has what begins with its tile and ends before the next
+// multiple of kSpan rows, or of a tile if that has more; the tiles in between have nothing to do.
+//
+// A step's experts, us, before / this: 14 of 4096 x 3072, three choices, 100 rows 199 / 192, 130 242 / 197, 160 278 / 201, 300 284 / 227, 500 305 / 247; 14 of
+// 1024 x 3072, 200 rows 106 / 72; 128 of 2048 x 768, eight choices, 400 rows 305 / 246; 8 of 4096 x 14336, two, 104 rows 667 / 445, 400 703 / 566; 8 of
+// 2048 x 8192, 200 rows 276 / 173.  Fewer or more choices per expert: 14 of 4096 x 3072, 64 rows (14 each) 184 / 189, 700 (150) 306 / 438, since most of them
+// then have more than 128.
+constexpr int kSpan = 128;
+template <bool GATED, int RT>
+__global__ void __launch_bounds__(64 * kRowWaves) moe_span_kernel(GemmArgs<__bf16> a, int tile_rows) {
+    constexpr int k2 = SharedStream<RT, 2>::kRing, k4 = SharedStream<RT, 4>::kRing, k8 = SharedStream<RT, 8>::kRing, k24 = k2 > k4 ? k2 : k4;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[k24 > k8 ? k24 : k8];
+    clear_counts(a);
+    const int tile = blockIdx.x / a.col_blocks, cb = blockIdx.x % a.col_blocks;
+    const int expert = a.tiles[2 * tile], row0 = a.tiles[2 * tile + 1], span = tile_rows > kSpan ? tile_rows : kSpan;
+    if (expert < 0 || expert >= a.experts || row0 % span) return;
+    const int first = a.offsets[expert] + row0, end = a.offsets[expert + 1];
+    const int rows = end - first < span ? end - first : span, c0 = cb * (GATED ? 8 : 16) * RT;
+    for (int at = 0; at < rows; at += kSpan) {
+        if (at > 0) __syncthreads();                   // everybody has read what lies in LDS
+        const int here = rows - at < kSpan ? rows - at : kSpan;
+        if (here <= 32) moe_shared_product<GATED, RT, 2>(a, expert, first + at, here, c0, lds);
+        else if (here <= 64) moe_shared_product<GATED, RT, 4>(a, expert, first + at, here, c0, lds);
+        else moe_shared_product<GATED, RT, 8>(a, expert, first + at, here, c0, lds);
     }
 }
 
@@ -725,6 +765,25 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t choices, int64_t max
     const dim3 block(kThreads);
     int64_t grid;
     if constexpr (sizeof(T) == 2) {
+        if (tile_rows >= kSmallRows && a.k % kStreamK == 0 && choices >= 18 * a.experts && choices <= 112 * a.experts) {
+            // eight tiles of W, unless four have the compute units through earlier: a tile takes about three times what the rows beside it do (8 experts of
+            // 1536 x 4096, 100 rows 79 / 68 us; 14 of 4096 x 3072, 130 rows 197 / 205)
+            auto takes = [&](int64_t t) {
+                const int64_t groups = a.experts * ((a.out_cols * (gated ? 2 : 1) + 16 * t - 1) / (16 * t));
+                return (groups + 255) / 256 * (3 * t + 4);
+            };
+            const int tiles = takes(4) < takes(8) ? 4 : 8, per = (gated ? 8 : 16) * tiles;
+            a.col_blocks = (a.out_cols + per - 1) / per;
+            grid = (int64_t)a.max_tiles * a.col_blocks;
+            if (grid > 0x7fffffff) return INFER_KV_EINVAL;
+#define GO(GATED, RT) hipLaunchKernelGGL((moe_span_kernel<GATED, RT>), dim3((unsigned)grid), block, 0, st, a, tile_rows)
+            if (gated && tiles == 8) GO(true, 8);
+            else if (gated) GO(true, 4);
+            else if (tiles == 8) GO(false, 8);
+            else GO(false, 4);
+#undef GO
+            return (int)hipGetLastError();
+        }
         if (tile_rows == kBlockRows) {
             a.col_blocks = (a.out_cols + (gated ? 127 : 255)) / (gated ? 128 : 256);
             grid = ((int64_t)a.max_tiles * a.col_blocks + 7) / 8 * 8;

@@ -653,6 +653,14 @@ def test_moe_rows_of_a_long_k(gpu, width, ff, n):
     test_moe_rows_around_the_tiles_that_weights_stream_past(gpu, width, ff, n)
 
 
+@pytest.mark.parametrize("width,ff", [(64, 128), (256, 72), (520, 192), (2304, 136)])
+@pytest.mark.parametrize("n", [71, 72, 97, 128, 129, 161, 257, 300, 448, 449])
+def test_moe_rows_that_weights_pass_once(gpu, width, ff, n):
+    """The same with so many rows per expert that the weights pass up to 128 of them at once: all at one expert, in tiles of 32, 128 and 256, the last ones
+    of 1 to 128 rows; just outside the range; one product of it alone, where the other's k is no multiple of a step."""
+    test_moe_rows_around_the_tiles_that_weights_stream_past(gpu, width, ff, n)
+
+
 def test_bad_arguments_are_refused(gpu):
     z = torch.zeros(8, 64, device=gpu)
     counts = torch.zeros(4, dtype=torch.int32, device=gpu)
