@@ -222,3 +222,17 @@ def test_steps_that_wavefronts_share(gpu, m, n, k):
     rc = ops._lib.load().infer_skinny_gate_silu_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), fused.data_ptr(), n // 2, m, n // 2, k,
                                                      torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and torch.equal(fused, both)
+
+
+@pytest.mark.parametrize("m", [65, 96, 113, 128])
+@pytest.mark.parametrize("n,k", [(8, 128), (136, 256), (1024, 1536), (4104, 2176), (8184, 2304), (24584, 256)])
+def test_more_than_64_of_the_batch(gpu, m, n, k):
+    """Exact sums for four and eight tiles of weight rows, cut over k and whole, around the last rows of both."""
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = torch.randint(-1, 2, (m, k + 8), generator=g, device=gpu).to(torch.bfloat16)[:, 8:]
+    w = torch.randint(-1, 2, (n, k), generator=g, device=gpu).to(torch.bfloat16)
+    want = reference(x, w)
+    assert want.abs().max() <= 256                      # representable in bf16 without rounding
+    assert torch.equal(ops.skinny_linear(x, w).float(), want)
+    deferred = ops.skinny_linear_deferred(x, w)
+    assert torch.equal((deferred.materialize() if isinstance(deferred, ops.SplitKSum) else deferred).float(), want)
