@@ -753,18 +753,20 @@ __global__ void __launch_bounds__(kThreads) decay_step_kernel(DecayArgs<T> a, De
 }
 
 // ------------------------------------------------------------------ norm and gate
-// One norm over the whole row.  NCH: chunks of VEC columns per thread, kept in registers.
+// One norm over the whole row.  NCH: chunks of VEC columns per thread, kept in registers.  Bound by memory (13,800 rows of 4096: 340 MB): the gate's
+// values are requested with the others instead of behind the sum, all with the streaming hint (a call 264.7 -> 261.5 us; the order alone 263).
 template <class T, int VEC, int NCH>
 __global__ void __launch_bounds__(kThreads) decay_out_row_kernel(DecayOutArgs<T> a) {
     __shared__ float part[4];
     const int64_t row = blockIdx.x;
     const int n = a.heads * a.vdim;
-    float x[NCH][VEC], ss = 0.f;
+    float x[NCH][VEC], g[NCH][VEC], ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
         const int c = (threadIdx.x + j * kThreads) * VEC;
         if (c < n) {
-            load_elems<VEC>(a.o + row * a.o_stride + c, x[j]);
+            load_once<VEC>(a.o + row * a.o_stride + c, x[j]);
+            load_once<VEC>(a.gate + row * a.gate_stride + c, g[j]);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) ss += x[j][e] * x[j][e];
         }
@@ -774,11 +776,10 @@ __global__ void __launch_bounds__(kThreads) decay_out_row_kernel(DecayOutArgs<T>
     for (int j = 0; j < NCH; ++j) {
         const int c = (threadIdx.x + j * kThreads) * VEC;
         if (c < n) {
-            float g[VEC], w[VEC];
-            load_elems<VEC>(a.gate + row * a.gate_stride + c, g);
+            float w[VEC];
             if (a.norm) load_elems<VEC>(a.norm + c, w);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) x[j][e] *= rs * (a.norm ? w[e] : 1.f) * gate_of(a, g[e]);
+            for (int e = 0; e < VEC; ++e) x[j][e] *= rs * (a.norm ? w[e] : 1.f) * gate_of(a, g[j][e]);
             store_elems<VEC>(a.out + row * a.out_stride + c, x[j]);
         }
     }

@@ -42,6 +42,23 @@ __device__ __forceinline__ void load_elems(const __bf16* p, float (&x)[N]) {
         for (int i = 0; i < N; ++i) x[i] = (float)p[i];
     }
 }
+// load_elems of what nobody reads again, with the streaming hint: it leaves the caches to what somebody does.  p: aligned to the N elements, at most 16 bytes.
+template <int N, class T>
+__device__ __forceinline__ void load_once(const T* p, float (&x)[N]) {
+    constexpr int kBytes = N * sizeof(T) < 16 ? N * sizeof(T) : 16, kPer = kBytes / sizeof(T);
+    if constexpr (kBytes % 8 == 0 && N % kPer == 0) {
+        typedef uint32_t Words __attribute__((ext_vector_type(kBytes / 4)));
+        struct Elems { T e[kPer]; };
+#pragma unroll
+        for (int i = 0; i < N / kPer; ++i) {
+            const Elems v = __builtin_bit_cast(Elems, __builtin_nontemporal_load(reinterpret_cast<const Words*>(p) + i));
+#pragma unroll
+            for (int e = 0; e < kPer; ++e) x[kPer * i + e] = (float)v.e[e];
+        }
+    } else {
+        load_elems<N>(p, x);
+    }
+}
 template <int N>
 __device__ __forceinline__ void store_elems(float* p, const float (&x)[N]) {
     if constexpr (N % 4 == 0) {
