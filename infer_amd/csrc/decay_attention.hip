@@ -393,8 +393,9 @@ __global__ void __launch_bounds__(64 * WAVES, PARTS == 2 ? 4 : 2) decay_chunk_ke
     u32x2_t gate[VT][2];                                         // of results, requested a chunk before they are there
     bf16x8_t vf[VT];                                             // values of tokens 8 g .. + 7, column n
     // what the chunk's own tokens add to its results, and their squares
-    // two workgroups of eight wavefronts share a compute unit if a lane has 128 registers: no address stays in one from chunk to chunk
-    auto place = [](int x) { return PARTS == 2 ? renewed(x) : x; };
+    // two workgroups of eight wavefronts share a compute unit if a lane has 128 registers, and behind a rotation 256 do not hold everything: no address stays in
+    // one from chunk to chunk (16 portions of 300 to 800 tokens of 16 heads, rotated, 136.5 us with addresses that stay and seven registers spilt, 130.8 without)
+    auto place = [](int x) { return PARTS == 2 || PC == 3 ? renewed(x) : x; };
     auto own_tokens = [&](int c) {
         const int lane = place(tid & 63), g = lane >> 4, n = lane & 15;
         const unsigned char* pr = pbufs + c % kBufs * 2 * kPMat;
