@@ -317,6 +317,12 @@ __global__ void __launch_bounds__(64 * kWaves, 2) dense_prefill_kernel(DensePref
 // 407 / 288, chunks of 2048 with a bias 570 / 404; one sequence of 1800 in chunks of 512 with a bias, 16 heads 50 / 49.
 constexpr int kGroupB = 1024 + 32, kTileB = 2 * (kStep / 4) * kGroupB, kRing = 3;      // bytes: four rows, keys and values of a step
 
+// A value that the compiler takes for a new one: what is computed from it is not kept in registers over the whole loop.
+__device__ __forceinline__ int renewed(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 template <int MAPS, bool BIASED>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(3, 3))) dense_prefill_ring_kernel(DensePrefillArgs a) {
     constexpr int KS = 4 / MAPS, VT = 8;
@@ -408,8 +414,9 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int t = 0; t < VT; ++t) acc[u][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    const int k_addr = (n >> 2) * kGroupB + (n & 3) * 64 + g * 16;
-    const int v_addr = (kStep / 4) * kGroupB + g * kGroupB + (n >> 2) * 64 + ((n & 3) >> 1) * 16 + (n & 1) * 8;
+    // With a bias 168 registers do not hold everything: addresses in LDS are made anew in every step.  Five spilt ones, whose reads wait for the requests of
+    // later steps as well: 6 sequences of 1100 to 3000, 32 heads, chunks of 2048, 282 us, this 275.
+    auto place = [](int x) { return BIASED ? renewed(x) : x; };
     if (nsteps > first_step) fetch(first_step, 0);               // otherwise no query of the workgroup sees a key
     if (nsteps > first_step + 1) fetch(first_step + 1, kTileB);
     landed_all();                                                // the query, too: the compiler knows nothing of the requests
@@ -423,6 +430,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
         if (kInner || (s >= my_first && s < my_steps)) {
             const unsigned char* buf = lds + ring;
             const int tok0 = s * kStep;
+            const int lane_k = place(lane), k_addr = (lane_k >> 2 & 3) * kGroupB + (lane_k & 3) * 64 + (lane_k >> 4) * 16;
+            const int g = lane_k >> 4, n = lane_k & 15;
             f32x4_t sc[2][2];
             float by = slope;
             if (BIASED) asm volatile("" : "+v"(by));             // its multiples are not kept from step to step
@@ -498,6 +507,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
                 for (int i = 0; i < 8; ++i) pb[u][i] = (__bf16)__builtin_amdgcn_exp2f(x[i]);
                 lacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[u], lacc[u], 0, 0, 0);
             }
+            const int lane_v = place(lane), v_addr = (kStep / 4) * kGroupB + (lane_v >> 4) * kGroupB + (lane_v >> 2 & 3) * 64 + (lane_v >> 1 & 1) * 16 + (lane_v & 1) * 8;
 #pragma unroll
             for (int t = 0; t < VT; ++t) {
                 const unsigned char* src = buf + v_addr + (t >> 1) * 256 + (t & 1) * 32;
