@@ -368,7 +368,9 @@ __global__ void __launch_bounds__(256) skinny_gemm_reduce_kernel(ReduceArgs a) {
 // Three tiles of rows are none of its shapes: 12288 x 4096 with 64 of the batch 21.2 / 22.6.  Few weight rows and a long k: 16 rows give every compute unit
 // a workgroup that reads the batch once per 16 rows; 64 rows, cut over k, read it a quarter as often.  Unreduced sums, 16 / 64 rows (split k): n = 4096,
 // k = 12288 9 of the batch 18.5 / 17.1, 16 20.2 / 17.3, 32 25.9 / 19.0 (now 17.3); with a shorter k the launch that adds the sums up for those who want
-// them costs more than that (n = 4096, k = 4096, 16: 8.4 / 10.4 reduced).
+// them costs more than that (n = 4096, k = 4096, 16: 8.4 / 10.4 reduced).  More than 4096 weight rows and a very long k: tiles of 64 rows leave
+// 160 workgroups that read the batch for half of k each; 128 rows, cut twice as often, read it half as often: 5120 x 25600, 64 of the batch 68 / 49 us (with 4096
+// weight rows the further sums take what that gives: 4096 x 12288 20.7 / 20.2, a step that adds them up 776 / 783).
 constexpr int64_t kMany = 40960, kLongK = 8192, kUnits = 256;
 // 16-row tiles of a workgroup of skinny_shared_kernel: those with which the compute units are through first, counting what a tile takes as three and what every
 // 16 of the batch take beside them as one (151936 x 4096, us per round of 2 / 4 / 8 / 12 / 16 / 20 tiles: 64 of the batch 15 / 24 / 43 / 58 / 74 / 101, 16
@@ -387,7 +389,7 @@ int shared_tiles(int64_t m, int64_t n) {
 }
 int rows_per_workgroup(int64_t m, int64_t n, int64_t k) {
     if (m > 64) return kBN;
-    if (n <= 5120) return m > 32 || (m > 8 && k >= kLongK) ? 64 : 16;
+    if (n <= 5120) return m > 32 && n > 4096 && k >= 2 * kLongK ? 128 : m > 32 || (m > 8 && k >= kLongK) ? 64 : 16;
     if (m <= 16 && n >= kMany && k <= 2048) return 32;
     if (m <= 8) return 16;
     return m > 16 && n > 8192 && n <= 12288 ? 48 : 16 * shared_tiles(m, n);

@@ -236,3 +236,15 @@ def test_more_than_64_of_the_batch(gpu, m, n, k):
     assert torch.equal(ops.skinny_linear(x, w).float(), want)
     deferred = ops.skinny_linear_deferred(x, w)
     assert torch.equal((deferred.materialize() if isinstance(deferred, ops.SplitKSum) else deferred).float(), want)
+
+
+@pytest.mark.parametrize("m", [32, 33, 64])
+@pytest.mark.parametrize("n,k", [(4096, 16384), (4104, 16384), (5120, 16256), (5120, 16384)])
+def test_a_very_long_k(gpu, m, n, k):
+    """Around the line from which more than 4096 weight rows go 128 to a workgroup; one in eight activations is not zero, so that sums stay below 256."""
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    x = (torch.randint(-1, 2, (m, k), generator=g, device=gpu) * (torch.rand((m, k), generator=g, device=gpu) < 0.125)).to(torch.bfloat16)
+    w = torch.randint(-1, 2, (n, k), generator=g, device=gpu).to(torch.bfloat16)
+    want = reference(x, w)
+    assert want.abs().max() <= 256                      # representable in bf16 without rounding
+    assert torch.equal(ops.skinny_linear(x, w).float(), want)
