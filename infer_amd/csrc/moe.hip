@@ -822,6 +822,8 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t choices, int64_t max
 // rows per tile: 0 where only the any-size kernels serve
 int rows_per_tile(int elem, int64_t n, int64_t width, int64_t ff_pad, int64_t experts, int64_t top) {
     if (elem != INFER_ELEM_BF16 || width % 8 || ff_pad % 8) return 0;
+    // The tiles that moe_row_kernel, moe_tile_kernel and moe_block_kernel work on.  With 18 to 112 choices per expert and k in whole steps moe_span_kernel takes what
+    // begins with every 128 rows, whatever the tiles; the figures are of the others.
     // An expert with more than one tile of 32 rows reads its weights again, and around 32 choices per expert half of them have more.  That costs
     // little where the weights are few, more where there are many of them or many experts; us, tiles of 32 rows / the others: 8 experts of
     // 1536 x 4096, 32 choices each 105 / 136; 8 of 2048 x 8192, 28 234 / 275; 14 of 4096 x 3072, 25 261 / 282, 32 330 / 280; 8 of 4096 x 14336, 26
