@@ -755,8 +755,8 @@ __global__ void __launch_bounds__(kThreads) decay_step_kernel(DecayArgs<T> a, De
 
 // ------------------------------------------------------------------ norm and gate
 // One norm over the whole row.  NCH: chunks of VEC columns per thread, kept in registers.  Bound by memory (13,800 rows of 4096: 340 MB): the gate's
-// values are requested with the others instead of behind the sum, all with the streaming hint (a call 264.7 -> 261.5 us; the order alone 263).
-template <class T, int VEC, int NCH>
+// values are requested with the others instead of behind the sum, ONCE (beyond_caches) with the streaming hint (a call 264.7 -> 261.5 us; the order alone 263).
+template <class T, int VEC, int NCH, bool ONCE>
 __global__ void __launch_bounds__(kThreads) decay_out_row_kernel(DecayOutArgs<T> a) {
     __shared__ float part[4];
     const int64_t row = blockIdx.x;
@@ -766,8 +766,8 @@ __global__ void __launch_bounds__(kThreads) decay_out_row_kernel(DecayOutArgs<T>
     for (int j = 0; j < NCH; ++j) {
         const int c = (threadIdx.x + j * kThreads) * VEC;
         if (c < n) {
-            load_once<VEC>(a.o + row * a.o_stride + c, x[j]);
-            load_once<VEC>(a.gate + row * a.gate_stride + c, g[j]);
+            load_once<VEC, ONCE>(a.o + row * a.o_stride + c, x[j]);
+            load_once<VEC, ONCE>(a.gate + row * a.gate_stride + c, g[j]);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) ss += x[j][e] * x[j][e];
         }
@@ -843,7 +843,11 @@ int launch_out(const DecayOutArgs<T>& a, bool per_head, int64_t rows, hipStream_
         return (int)hipGetLastError();
     }
     const int chunks = ((vec ? n / 4 : n) + kThreads - 1) / kThreads;
-#define GO(V, N) hipLaunchKernelGGL((decay_out_row_kernel<T, V, N>), grid, block, 0, st, a)
+    const bool once = vec && beyond_caches(2 * rows * n * (int64_t)sizeof(T));
+#define GO(V, N) do { \
+        if (V > 1 && once) hipLaunchKernelGGL((decay_out_row_kernel<T, V, N, (V > 1)>), grid, block, 0, st, a); \
+        else hipLaunchKernelGGL((decay_out_row_kernel<T, V, N, false>), grid, block, 0, st, a); \
+    } while (0)
     if (vec) {
         if (chunks <= 1) GO(4, 1);
         else if (chunks <= 2) GO(4, 2);

@@ -561,8 +561,8 @@ struct NormArgs {
     T* out; int64_t out_stride;
 };
 
-// Bound by memory: 13,800 rows of 4096 (two read, one written) 340 MB; loads without the streaming hint 3 us more of a call of 267.
-template <class T, int VEC>
+// Bound by memory: 13,800 rows of 4096 (two read, one written) 340 MB.  ONCE: beyond_caches.
+template <class T, int VEC, bool ONCE>
 __global__ void __launch_bounds__(kThreads) ssm_norm_kernel(NormArgs<T> b) {
     __shared__ float part[kThreads / 64];
     const SsmArgs<T>& a = b.a;
@@ -574,8 +574,8 @@ __global__ void __launch_bounds__(kThreads) ssm_norm_kernel(NormArgs<T> b) {
     float x[kKeep][VEC], ss = 0.f;
     auto gated = [&](int c, float (&v)[VEC]) {
         float w[VEC];
-        load_once<VEC>(y + c, v);
-        load_once<VEC>(z + c, w);
+        load_once<VEC, ONCE>(y + c, v);
+        load_once<VEC, ONCE>(z + c, w);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) v[e] *= silu_f(w[e]);
     };
@@ -763,8 +763,9 @@ extern "C" int infer_state_space(int elem, const void* proj, int64_t proj_stride
         const bool vec = size % 8 == 0 && inner % 8 == 0 && proj_stride % 8 == 0 && z_off % 8 == 0 && out_stride % 8 == 0 &&
                          ptr_aligned(proj, 16) && ptr_aligned(y, 16) && ptr_aligned(out, 16) && ptr_aligned(norm, 16);
         const dim3 grid((unsigned)n, (unsigned)norm_parts), block(kThreads);
-        if (vec) hipLaunchKernelGGL((ssm_norm_kernel<T, 8>), grid, block, 0, st, b);
-        else hipLaunchKernelGGL((ssm_norm_kernel<T, 1>), grid, block, 0, st, b);
+        if (vec && beyond_caches(2 * n * inner * (int64_t)sizeof(T))) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, true>), grid, block, 0, st, b);
+        else if (vec) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, false>), grid, block, 0, st, b);
+        else hipLaunchKernelGGL((ssm_norm_kernel<T, 1, false>), grid, block, 0, st, b);
         return (int)hipGetLastError();
     };
     if (elem == INFER_ELEM_BF16) return go(__bf16(0.f));
