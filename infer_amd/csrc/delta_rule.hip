@@ -25,6 +25,7 @@
 // The last `taps` inputs of the convolution live in a ring per sequence (entry position % taps).  A position below
 // zero counts as zero and a portion that starts at position 0 starts from a zero state, so a slot needs no clearing
 // when another sequence takes it over.
+#include "conv_window.h"
 #include "pieces.h"
 #include "segments.h"
 
@@ -239,15 +240,13 @@ __device__ __forceinline__ void conv4_silu(const DeltaArgs<T>& a, const ChunkDes
     }
 #pragma unroll
     for (int j = 0; j < (INNER ? 0 : 11); ++j) {
-        const int t = t0 + j - 3, p = cd.pos0 + t;
-        // positions before the portion are in the ring; those before the sequence or behind the chunk's tokens are zero
-        const bool in = p >= 0 && t < cd.count;
-        const T* src = p >= cd.first_pos || !in ? a.proj + (int64_t)(cd.row0 + (in ? t : 0)) * a.proj_stride + c
-                                                : a.ring + ((int64_t)cd.slot * 4 + (p & 3)) * a.channels + c;
-        load_elems<4>(src, x[j]);
-        if (!in)
+        const int t = t0 + j - 3;
+        const WindowRow from = window_row(cd.count, cd.pos0, cd.first_pos, t);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x[j][e] = 0.f;
+        for (int e = 0; e < 4; ++e) x[j][e] = 0.f;
+        if (from != WindowRow::kNone)
+            load_elems<4>(from == WindowRow::kBatch ? a.proj + (int64_t)(cd.row0 + t) * a.proj_stride + c
+                                                    : a.ring + ((int64_t)cd.slot * 4 + ((cd.pos0 + t) & 3)) * a.channels + c, x[j]);
     }
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -530,7 +529,7 @@ __global__ void __launch_bounds__(256, 4) delta_prep_square_kernel(DeltaArgs<__b
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.y;
     const int lq = lane >> 4, lm = lane & 15, i = tid >> 4, j = tid & 15;
     const ChunkDesc c = chunks[blockIdx.x];
-    const int row0 = c.count > 0 ? c.row0 : 0;                   // what an empty chunk reads is not used, and row 0 exists
+    const int row0 = c.count > 0 ? c.row0 : 0;                   // the gates of an empty chunk read row 0, which exists, and use nothing of it
     float* rec = records + ((int64_t)blockIdx.x * a.heads + h) * record_floats(D, D);
     const int group = a.heads / a.kv_heads, kvh = h / group;
     const float rate = expf(a.a_log[h]);
@@ -565,12 +564,12 @@ __global__ void __launch_bounds__(256, 4) delta_prep_square_kernel(DeltaArgs<__b
     } else {
 #pragma unroll
         for (int x = 0; x < 11; ++x) {
-            const int t = t0 + x - 3, p = c.pos0 + t;
-            // positions before the portion are in the ring; those before the sequence or behind the chunk's tokens are zero
-            const bool in = p >= 0 && t < c.count;
-            raw[x] = *reinterpret_cast<const u32x2*>(p >= c.first_pos || !in ? a.proj + (int64_t)(row0 + (in ? t : 0)) * a.proj_stride + channel
-                                                                             : a.ring + ((int64_t)c.slot * 4 + (p & 3)) * a.channels + channel);
-            if (!in) raw[x] = u32x2{0u, 0u};
+            const int t = t0 + x - 3;
+            const WindowRow from = window_row(c.count, c.pos0, c.first_pos, t);
+            raw[x] = u32x2{0u, 0u};
+            if (from != WindowRow::kNone)
+                raw[x] = *reinterpret_cast<const u32x2*>(from == WindowRow::kBatch ? a.proj + (int64_t)(row0 + t) * a.proj_stride + channel
+                                                                                   : a.ring + ((int64_t)c.slot * 4 + ((c.pos0 + t) & 3)) * a.channels + channel);
         }
     }
     int strong = 0;

@@ -566,6 +566,26 @@ def test_delta_empty_portions_and_chunks(gpu):
     assert torch.equal(c.state[0], before[0]) and torch.equal(c.state[3], before[3]) and (c.state[2] == 0).all()
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+def test_delta_empty_chunks_of_square_heads(gpu, dim):
+    """In front, between, behind a chunk of a few tokens and at the end, with a first row of zero, as a portion from the start and as one that goes on: a chunk
+    without tokens reads no row in front of the batch and changes nothing."""
+    c = DeltaCase(3, 1, dim, dim, 4, 47, torch.bfloat16, seed=6)
+    outs = []
+    for lo, hi in [(0, 21), (21, 47)]:
+        own = [(r, min(16, hi - lo - r), lo + r, lo, 1, 0) for r in range(0, hi - lo, 16)]
+        empty = [(0, 0, lo + x, lo, 1, 0) for x in (0, 16, hi - lo)]
+        chunks = [empty[0], own[0], empty[1], own[1], empty[2]]
+        a = [dev(x[lo:hi], c.dtype) for x in (c.proj, c.decay, c.gate)]
+        out = torch.full((hi - lo, 3 * dim), float("nan"), dtype=c.dtype, device="cuda")
+        ho.delta_chunks(c.s, a[0], c.beta_off, a[1], a[2], *c.weights, c.ring, c.state, dev([(0, len(chunks), 1, lo)], torch.int32), dev(chunks, torch.int32),
+                        dev([(1, hi - lo - 1 - r) for r in range(hi - lo)], torch.int32), dev(np.arange(lo, hi), torch.int64), 0, out)
+        outs.append(out)
+    want, want_state = c.want()
+    close(torch.cat(outs), want, tol(c.dtype, 3e-5, 1e-2))
+    close(c.state[1], want_state, 3e-5)
+
+
 def test_delta_state_of_operands_of_one_sign_does_not_drift(gpu):
     """3200 tokens without decay whose keys, values and inner results are all positive, beside six short portions, so that one workgroup
     holds all columns of a head.  Roundings to nearest of the 200 chunks' sums partly cancel: sqrt(200) of them are 14 x 2^-24, as many as
