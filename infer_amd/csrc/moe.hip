@@ -658,7 +658,7 @@ __device__ __forceinline__ void moe_row_product(const GemmArgs<__bf16>& a, int e
     f32x4_t acc[1][MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[0][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream_product<1, MT, kRowWaves, MT == 1 ? 3 : 2, 0>(w, x, a.k, wave, lds + wave * kRowRing, acc);
+    stream_product<1, MT, kRowWaves, MT == 1 ? 3 : 2, false>(w, x, a.k, 0, wave, lds + wave * kRowRing, acc);
     stream_reduce<1, MT, kRowWaves>(acc, wave, lds, [&](int, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0, sum); });
 }
 // The same, RT tiles of W and up to 16 MT rows, steps shared; k: a multiple of 64
@@ -668,7 +668,7 @@ __device__ __forceinline__ void moe_shared_product(const GemmArgs<__bf16>& a, in
     constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR;
     static_assert(WK == 1 || 4096 * TW * MT <= Stream::kRing, "the sums fit the ring");
     const int n = threadIdx.x & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave % WR;
-    Stream stream(a.k, wave, lds, [&](int i) { return moe_weight_row<GATED>(a, expert, c0, i); }, [&](int i) { return moe_input_row(a, first, rows, i); });
+    Stream stream(a.k, (int)blockIdx.x >> 3, wave, lds, [&](int i) { return moe_weight_row<GATED>(a, expert, c0, i); }, [&](int i) { return moe_input_row(a, first, rows, i); });
     f32x4_t acc[TW][MT];
 #pragma unroll
     for (int r = 0; r < TW; ++r)

@@ -39,15 +39,34 @@ struct GemmArgs {
     float* partial;              // [SK][M][N] when SK > 1
     int m, n, k;
     int chunks;                  // K chunks per split
+    int each;                    // workgroups of either half of the weight rows where the halves are dealt out apart (Share), otherwise 0
+};
+
+// The weight rows n0 .. end - 1 of which a workgroup takes its ROWS (GATED: ROWS / 2 gate rows, and the up rows of the same places), and where it begins its
+// walk over k (stream_start): 2^TURN workgroups at one place, 0 everybody at the front.  Gate rows and up rows are halves of one matrix, and a product of both
+// has to add up as the two by themselves do.  So without a gate a workgroup that is not cut over k lies in one half, and there 2^HALF_TURN of them begin at the
+// place of the twice as many that have the same rows with a gate.  Us, two workgroups of other halves side by side / the halves one behind the other: 6144 x
+// 4096, 48 of the batch 17.0 / 16.8, 151936 x 4096, 4 183.8 / 179.9.
+template <bool GATED, int ROWS, int TURN, int HALF_TURN = TURN>
+struct Share {
+    int n0, end, turn;
+    __device__ __forceinline__ explicit Share(const GemmArgs& a) {
+        const int b = blockIdx.x, half = a.n / 2;
+        const bool apart = !GATED && TURN > 0 && a.each > 0, second = apart && b >= a.each;
+        const int at = second ? b - a.each : b;
+        n0 = at * (GATED ? ROWS / 2 : ROWS) + (second ? half : 0);
+        end = GATED || (apart && !second) ? half : a.n;
+        turn = TURN == 0 ? 0 : GATED ? b >> (HALF_TURN + 1) : apart ? at >> HALF_TURN : b >> TURN;
+    }
 };
 
 __device__ __forceinline__ u32x4 load16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
 __device__ __forceinline__ float round_bf16(float x) { return (float)(__bf16)x; }
 
-// Four sums of row `row` at the places 16 r + 4 g of a workgroup whose weights begin at row n0 (GATED: as described below)
+// Four sums of row `row` at the places 16 r + 4 g of a workgroup whose weights begin at row n0 and end in front of row `end` (GATED: as described below)
 template <bool GATED>
-__device__ __forceinline__ void finish_tile(const GemmArgs& a, int half, int split, int n0, int r, int row, int g, f32x4_t sum) {
+__device__ __forceinline__ void finish_tile(const GemmArgs& a, int end, int split, int n0, int r, int row, int g, f32x4_t sum) {
     if constexpr (GATED) {                         // lanes g = 0, 1 hold gates 4 g + e, lanes g + 2 the up columns of the same place
         bf16x4_t v;
 #pragma unroll
@@ -56,10 +75,10 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& a, int half, int spl
             v[e] = (__bf16)(round_bf16(gate / (1.0f + expf(-gate))) * up);
         }
         const int col = n0 + 8 * r + 4 * g;
-        if (g < 2 && col < half && row < a.m) *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
+        if (g < 2 && col < end && row < a.m) *reinterpret_cast<bf16x4_t*>(a.y + (int64_t)row * a.y_stride0 + col) = v;
     } else {
         const int col = n0 + 16 * r + 4 * g;
-        if (col >= a.n || row >= a.m) return;          // N is a multiple of 8: a quad is in or out as a whole
+        if (col >= end || row >= a.m) return;          // a multiple of 8: a quad is in or out as a whole
         if (a.partial) {
             *reinterpret_cast<f32x4_t*>(a.partial + ((int64_t)split * a.m + row) * a.n + col) = sum;
         } else {
@@ -79,15 +98,15 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
     constexpr int kRing = D * stream_stage_bytes(RT, MT), kLds = NW * (kRing > 1024 * RT * MT ? kRing : 1024 * RT * MT);
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int half = a.n / 2, n0 = blockIdx.x * (GATED ? 8 : 16) * RT, split = blockIdx.y;
+    const int half = a.n / 2, split = blockIdx.y;
+    const Share<GATED, 16 * RT, TURN> share(a);
     const int64_t k_lo = (int64_t)split * a.chunks * kKC;
     const __bf16* w[2 * RT];
     const __bf16* x[2 * MT];
 #pragma unroll
     for (int i = 0; i < 2 * RT; ++i) {
-        int row = n0 + stream_row() + 8 * (GATED ? i / 2 : i);
-        const int rows = GATED ? half : a.n;
-        row = (row < rows ? row : rows - 1) + (GATED && (i & 1) ? half : 0);
+        int row = share.n0 + stream_row() + 8 * (GATED ? i / 2 : i);
+        row = (row < share.end ? row : share.end - 1) + (GATED && (i & 1) ? half : 0);
         w[i] = (const __bf16*)a.w + (int64_t)row * a.k + k_lo;
     }
 #pragma unroll
@@ -100,8 +119,8 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream_product<RT, MT, NW, D, TURN>(w, x, a.chunks * kKC, wave, lds + wave * kRing, acc);
-    stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, half, split, n0, r, 16 * t + n, g, sum); });
+    stream_product<RT, MT, NW, D, (TURN > 0)>(w, x, a.chunks * kKC, share.turn, wave, lds + wave * kRing, acc);
+    stream_reduce<RT, MT, NW>(acc, wave, lds, [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, share.end, split, share.n0, r, 16 * t + n, g, sum); });
 }
 
 // The same, the steps of k shared by the wavefronts (SharedStream)
@@ -112,13 +131,13 @@ __global__ void __launch_bounds__(256) skinny_shared_kernel(GemmArgs a) {
     static_assert(WK == 1 || 4096 * TW * MT <= Stream::kRing, "the sums fit the ring");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[Stream::kRing];
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int half = a.n / 2, n0 = blockIdx.x * (GATED ? 8 : 16) * RT, split = blockIdx.y, wr = wave % WR;
+    const int half = a.n / 2, split = blockIdx.y, wr = wave % WR;
+    const Share<GATED, 16 * RT, 3, 2> share(a);
     const int64_t k_lo = (int64_t)split * a.chunks * kKC;
-    Stream stream(a.chunks * kKC, wave, lds,
+    Stream stream(a.chunks * kKC, share.turn, wave, lds,
         [&](int i) {
-            int row = n0 + stream_row() + 8 * (GATED ? i / 2 : i);
-            const int rows = GATED ? half : a.n;
-            row = (row < rows ? row : rows - 1) + (GATED && (i & 1) ? half : 0);
+            int row = share.n0 + stream_row() + 8 * (GATED ? i / 2 : i);
+            row = (row < share.end ? row : share.end - 1) + (GATED && (i & 1) ? half : 0);
             return (const __bf16*)a.w + (int64_t)row * a.k + k_lo;
         },
         [&](int i) {
@@ -131,7 +150,7 @@ __global__ void __launch_bounds__(256) skinny_shared_kernel(GemmArgs a) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     stream.product(wave, lds, acc);
-    auto finish = [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, half, split, n0, wr * TW + r, 16 * t + n, g, sum); };
+    auto finish = [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, share.end, split, share.n0, wr * TW + r, 16 * t + n, g, sum); };
     if constexpr (WK == 1) {
 #pragma unroll
         for (int r = 0; r < TW; ++r)
@@ -169,16 +188,16 @@ __global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSourc
     static_assert(NW * kRing >= NW * RT * 1024, "sums of the wavefronts");
     extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];      // rings, then rows of x, then sums of squares
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n0 = blockIdx.x * (GATED ? 8 : 16) * RT, half = a.n / 2;
+    const int half = a.n / 2;
+    const Share<GATED, 16 * RT, TURN> share(a);
     const int row_bytes = 2 * a.k + kFewPad;
     unsigned char* xs = few_lds + NW * kRing;
     float* squares = reinterpret_cast<float*>(xs + a.m * row_bytes);               // [kFewRows][8]
     const __bf16* w[2 * RT];
 #pragma unroll
     for (int i = 0; i < 2 * RT; ++i) {
-        int row = n0 + stream_row() + 8 * (GATED ? i / 2 : i);
-        const int rows = GATED ? half : a.n;
-        row = (row < rows ? row : rows - 1) + (GATED && (i & 1) ? half : 0);
+        int row = share.n0 + stream_row() + 8 * (GATED ? i / 2 : i);
+        row = (row < share.end ? row : share.end - 1) + (GATED && (i & 1) ? half : 0);
         w[i] = (const __bf16*)a.w + (int64_t)row * a.k;
     }
     const int groups = (a.k + kNormGroup - 1) / kNormGroup, pieces = a.m * groups;
@@ -263,8 +282,8 @@ __global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSourc
     f32x4_t acc[RT][1];
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream_product_held<RT, NW, D, TURN>(w, xs + (n < a.m ? n : a.m - 1) * row_bytes + 16 * g, a.k, wave, few_lds + wave * kRing, norm, acc);
-    stream_reduce<RT, 1, NW>(acc, wave, few_lds, [&](int r, int, f32x4_t sum) { finish_tile<GATED>(a, half, 0, n0, r, n, g, sum); });
+    stream_product_held<RT, NW, D, (TURN > 0)>(w, xs + (n < a.m ? n : a.m - 1) * row_bytes + 16 * g, a.k, share.turn, wave, few_lds + wave * kRing, norm, acc);
+    stream_reduce<RT, 1, NW>(acc, wave, few_lds, [&](int r, int, f32x4_t sum) { finish_tile<GATED>(a, share.end, 0, share.n0, r, n, g, sum); });
 }
 
 // A product, split over k, of one sequence's attention that still lies in pieces (decode_few.h): a workgroup has up to kPieceHeads heads of k, whose pieces
@@ -330,8 +349,8 @@ __global__ void __launch_bounds__(256) piece_product_kernel(GemmArgs a, FewDecod
         __syncthreads();
     };
     f32x4_t acc[1][1] = {{f32x4_t{0.f, 0.f, 0.f, 0.f}}};
-    stream_product_held<1, NW, D, 0>(w, reinterpret_cast<const unsigned char*>(xs) + 16 * g, a.chunks * kKC, wave, lds + wave * kRing, add, acc);
-    stream_reduce<1, 1, NW>(acc, wave, lds, [&](int r, int, f32x4_t sum) { finish_tile<false>(a, 0, split, n0, r, n, g, sum); });
+    stream_product_held<1, NW, D, false>(w, reinterpret_cast<const unsigned char*>(xs) + 16 * g, a.chunks * kKC, 0, wave, lds + wave * kRing, add, acc);
+    stream_reduce<1, 1, NW>(acc, wave, lds, [&](int r, int, f32x4_t sum) { finish_tile<false>(a, a.n, split, n0, r, n, g, sum); });
 }
 
 struct ReduceArgs {
@@ -418,22 +437,30 @@ int choose_splits(int64_t m, int64_t n, int64_t k) {
 }
 
 // Whether wavefronts that split k begin at different places of it (stream_start).  With few workgroups or a short k, finding out where costs what it gives (a
-// step of 28 layers of a 0.6B model 729 / 733 us).  Products that norm their input have the bits of those that do not: the rule is one for both.
+// step of 28 layers of a 0.6B model 729 / 733 us).  Products that norm their input have the bits of those that do not: the rule is one for both.  What the order of
+// a gate's sums in products without one costs (Share), steps of four layers of an 8B model, 1, 2, 4, 8, 16, 64 sequences, without / with it: 493 / 499, 508 /
+// 510, 516 / 519, 528 / 531, 577 / 575, 700 / 696.
 bool begins_anywhere(int64_t n, int64_t k) { return k > 2048 && n > 8 * kUnits; }
+// The grid of a product whose workgroups have so many weight rows.  turned: their walks begin at different places; then the halves of the rows are dealt out
+// apart, where they can be gate and up (twice half the workgroups are no round of the compute units more).
+dim3 share_out(GemmArgs& a, bool gated, bool turned, int rows, int splits) {
+    a.each = turned && !gated && splits == 1 && a.n % 16 == 0 ? (a.n / 2 + rows - 1) / rows : 0;
+    return dim3((unsigned)(a.each ? 2 * a.each : (a.n + rows - 1) / rows), (unsigned)splits);
+}
 
 template <bool GATED, int MT>
-void launch_shared(const GemmArgs& a, int tiles, int splits, hipStream_t st) {
-    const dim3 grid((unsigned)((a.n + 16 * tiles - 1) / (16 * tiles)), (unsigned)splits);
+void launch_shared(GemmArgs a, int tiles, int splits, hipStream_t st) {
+    const dim3 grid = share_out(a, GATED, SharedStream<2, MT>::turned(a.chunks * kKC), 16 * tiles, splits);
 #define GO(RT) case RT: hipLaunchKernelGGL((skinny_shared_kernel<RT, MT, GATED>), grid, dim3(256), 0, st, a); return
     switch (tiles) { GO(2); GO(4); GO(6); GO(8); GO(10); GO(12); GO(14); GO(16); GO(20); }
 #undef GO
 }
 
 template <bool GATED>
-void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
+void launch_stream(GemmArgs a, int splits, hipStream_t st) {
     const int rows = rows_per_workgroup(a.m, a.n, a.k);
-    const dim3 grid((unsigned)((a.n + rows - 1) / rows), (unsigned)splits);
     const bool turned = begins_anywhere(a.n, a.chunks * kKC);
+    const dim3 grid = share_out(a, GATED, turned && a.m <= 64, rows, splits);
 #define TURNED(RT, MT, NW, D, TURN) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED, TURN>), grid, dim3(64 * NW), 0, st, a)
 #define GO(RT, MT, NW, D) do { if (turned) TURNED(RT, MT, NW, D, 3); else TURNED(RT, MT, NW, D, 0); } while (0)
     if (turned && a.m <= kFewRows && rows == 16 && a.n >= kFewMany && a.n < kMany) TURNED(1, 1, 4, 4, 4);      // in twos, as 32 rows with a norm in front
@@ -444,7 +471,7 @@ void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
     else if (a.m <= 64 && rows == 48) GO(3, 4, 4, 2);
     else if (a.m <= 64) {
         // half as many rows where 64 leave every second compute unit idle: 64 of the batch 4096 x 1024 5.5 / 4.6 us, 1024 x 3072 5.6 / 4.6
-        const int tiles = a.n <= 5120 && grid.x * grid.y <= kUnits / 2 ? 2 : rows / 16;
+        const int tiles = a.n <= 5120 && (a.n + rows - 1) / rows * splits <= kUnits / 2 ? 2 : rows / 16;
         if (a.m <= 16) launch_shared<GATED, 1>(a, tiles, splits, st);
         else if (a.m <= 32) launch_shared<GATED, 2>(a, tiles, splits, st);
         else launch_shared<GATED, 4>(a, tiles, splits, st);
@@ -563,11 +590,11 @@ extern "C" int infer_skinny_gate_silu_bf16(const void* x, int64_t x_stride0, con
 
 namespace {
 template <bool GATED>
-int launch_norm_product(const GemmArgs& a, const NormSource& f, hipStream_t st) {
+int launch_norm_product(GemmArgs a, const NormSource& f, hipStream_t st) {
     const int pieces = a.m * ((a.k + kNormGroup - 1) / kNormGroup), rows = a.n >= kFewMany ? 32 : 16;
     const size_t lds = 4 * 4 * stream_stage_bytes(rows / 16, 0) + (size_t)a.m * (2 * a.k + kFewPad) + kFewRows * 8 * sizeof(float);
-    const dim3 grid((unsigned)((a.n + rows - 1) / rows));
     const bool turned = begins_anywhere(a.n, a.k);
+    const dim3 grid = share_out(a, GATED, turned, rows, 1);
 #define GO(RT, NP, TURN) do { \
         if (lds > 60 * 1024) { \
             const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&norm_product_kernel<RT, NP, GATED, TURN>), \

@@ -20,15 +20,16 @@ __device__ __forceinline__ int stream_col() { return 8 * ((threadIdx.x & 7) ^ ((
 
 // Where a workgroup begins its walk over k, of `steps`; behind the end it goes on at the front.  Rows of weights lie a power of two or a small multiple of
 // one apart, so workgroups that all begin at the front read the same few channels of memory at any one time, and the same lines of the activations.
-// Every eighth workgroup goes to the same die, whose 32 compute units begin evenly spread: `turn` counts eights of workgroups.  Everybody at the front / this, 64 of the
-// batch, us: gate and up of 24576 x 4096 42.8 / 37.2, 65536 x 4096 108 / 90, 8192 x 4096 20.8 / 16.6; four: 16384 x 2048 14.9 / 12.6.
+// Every eighth workgroup goes to the same die, whose 32 compute units begin evenly spread: `turn` counts eights of workgroups or so.  Everybody at the front / this,
+// 64 of the batch, us: gate and up of 24576 x 4096 42.8 / 37.2, 65536 x 4096 108 / 90, 8192 x 4096 20.8 / 16.6; four: 16384 x 2048 14.9 / 12.6.  One turn behind the
+// other: with the 32 places in the order of their bits in reverse 24576 x 4096, steps shared (below), 33.6 / 37.0, four of the batch 32.2 / 38.1.
 __device__ __forceinline__ int stream_start(int turn, int steps) { return (int)((turn & 31) * (unsigned)steps >> 5); }
 
 // w[i], x[i]: this lane's row stream_row() + 8 i of the weights and of the activations, at the first element of k (16-byte aligned);
-// TURN: 0, or 2^TURN workgroups begin at one place (stream_start); k: elements, a multiple of eight; ring: D * stream_stage_bytes(RT, MT) bytes of the wavefront's own.  Adds to acc[r][t] (lane (g, n):
+// TURNED: the walk begins at stream_start(turn), otherwise at the front; k: elements, a multiple of eight; ring: D * stream_stage_bytes(RT, MT) bytes of the wavefront's own.  Adds to acc[r][t] (lane (g, n):
 // row n of tile t of x, rows 4 g + e of tile r of w) what the steps `wave`, `wave` + NW, ... contribute.
-template <int RT, int MT, int NW, int D, int TURN>
-__device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT], const __bf16* const (&x)[2 * MT], int k, int wave,
+template <int RT, int MT, int NW, int D, bool TURNED>
+__device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT], const __bf16* const (&x)[2 * MT], int k, int turn, int wave,
                                                unsigned char* ring, f32x4_t (&acc)[RT][MT]) {
     constexpr int kRequests = 2 * (RT + MT), kStage = stream_stage_bytes(RT, MT);
     static_assert(D >= 2 && D <= 4 && (D - 1) * kRequests <= 63, "requests in flight are counted in six bits");
@@ -36,10 +37,10 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
     const int all = (k + kStreamK - 1) / kStreamK, steps = all > wave ? (all - wave + NW - 1) / NW : 0;
     const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ring);
     // Inline assembly, since the compiler would put a wait for all requests in front of every read of LDS.  Nothing else here uses M0.
-    int ahead = TURN ? stream_start((int)blockIdx.x >> TURN, steps) : 0, now = ahead;      // the steps to be requested and to be multiplied next
+    int ahead = TURNED ? stream_start(turn, steps) : 0, now = ahead;      // the steps to be requested and to be multiplied next
     auto request = [&](int stage) {
         const int at = (ahead * NW + wave) * kStreamK + col, from = at < k ? at : 0;   // behind the end: something, which meets zeros
-        ahead = TURN && ahead + 1 == steps ? 0 : ahead + 1;
+        ahead = TURNED && ahead + 1 == steps ? 0 : ahead + 1;
 #pragma unroll
         for (int i = 0; i < kRequests; ++i) {
             const uint32_t to = base + stage * kStage + 1024 * i;
@@ -73,7 +74,7 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
         __builtin_amdgcn_sched_barrier(0);
         if (s + D < steps) request(stage);
         const int first = (now * NW + wave) * kStreamK;
-        now = TURN && now + 1 == steps ? 0 : now + 1;
+        now = TURNED && now + 1 == steps ? 0 : now + 1;
         if (first + kStreamK > k)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
@@ -93,18 +94,18 @@ __device__ __forceinline__ void stream_product(const __bf16* const (&w)[2 * RT],
 // The same past activations that lie in LDS as a whole: only the weights are requested, and `before` runs behind the first requests, while
 // they are on their way; it puts the activations where x points (this lane's row, at element 8 g of the first step) and ends with a barrier.
 // k: a multiple of kStreamK; ring: D * stream_stage_bytes(RT, 0) bytes.
-template <int RT, int NW, int D, int TURN, class Before>
-__device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 * RT], const unsigned char* x, int k, int wave, unsigned char* ring,
+template <int RT, int NW, int D, bool TURNED, class Before>
+__device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 * RT], const unsigned char* x, int k, int turn, int wave, unsigned char* ring,
                                                     Before before, f32x4_t (&acc)[RT][1]) {
     constexpr int kRequests = 2 * RT, kStage = stream_stage_bytes(RT, 0);
     static_assert(D >= 2 && D <= 4, "the waits below");
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, col = stream_col();
     const int all = k / kStreamK, steps = all > wave ? (all - wave + NW - 1) / NW : 0;
     const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ring);
-    int ahead = TURN ? stream_start((int)blockIdx.x >> TURN, steps) : 0, now = ahead;
+    int ahead = TURNED ? stream_start(turn, steps) : 0, now = ahead;
     auto request = [&](int stage) {
         const int from = (ahead * NW + wave) * kStreamK + col;
-        ahead = TURN && ahead + 1 == steps ? 0 : ahead + 1;
+        ahead = TURNED && ahead + 1 == steps ? 0 : ahead + 1;
 #pragma unroll
         for (int i = 0; i < kRequests; ++i)
             __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" :: "v"(w[i] + from), "s"(base + stage * kStage + 1024 * i) : "memory", "m0");
@@ -125,7 +126,7 @@ __device__ __forceinline__ void stream_product_held(const __bf16* const (&w)[2 *
         bf16x8_t a[RT][2], b[2];
         const unsigned char* p = ring + stage * kStage;
         const unsigned char* from = x + 2 * kStreamK * (now * NW + wave);
-        now = TURN && now + 1 == steps ? 0 : now + 1;
+        now = TURNED && now + 1 == steps ? 0 : now + 1;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
@@ -183,9 +184,11 @@ struct SharedStream {
     uint32_t to[kRequests];
     int ahead, steps;
 
+    // Whether a walk over k begins at stream_start(turn): a short one would find out where for nothing
+    static __host__ __device__ __forceinline__ bool turned(int k) { return k >= 2048; }
     // weights(i), batch(i): this lane's row stream_row() + 8 i of either, at the first element of k (a multiple of kStreamK)
     template <class Weights, class Batch>
-    __device__ __forceinline__ SharedStream(int k, int wave, const unsigned char* ring, Weights weights, Batch batch) {
+    __device__ __forceinline__ SharedStream(int k, int turn, int wave, const unsigned char* ring, Weights weights, Batch batch) {
         const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)ring;
 #pragma unroll
         for (int j = 0; j < kRequests; ++j) {
@@ -194,7 +197,7 @@ struct SharedStream {
             to[j] = __builtin_amdgcn_readfirstlane(base + 1024 * (j < kOfWeights ? i : 2 * RT + of_batch));
         }
         steps = k / kStreamK;
-        ahead = k < 2048 ? 0 : stream_start((int)blockIdx.x >> 3, steps);
+        ahead = turned(k) ? stream_start(turn, steps) : 0;
     }
     __device__ __forceinline__ void request(int stage) {
 #pragma unroll

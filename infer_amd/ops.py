@@ -743,8 +743,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, defer: bool = False):
 
 def gate_up_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``silu_and_mul`` of ``linear(x, weight)``: ``weight`` ``[2 ff, K]`` holds gate rows, then up rows.  One launch where the streaming
-    kernel takes the product whole (few rows, no split over K), with the roundings of the two; above 2048 elements of K it may add them up in another
-    order."""
+    kernel takes the product whole (few rows, no split over K), with the bits of the two."""
     ff = weight.shape[0] // 2
     if _streamable(x, weight) and x.shape[0] <= STREAM_MAX_BATCH and weight.shape[0] == 2 * ff and ff % 8 == 0 and _linear_mode() == "static":
         m, k = x.shape

@@ -248,3 +248,18 @@ def test_a_very_long_k(gpu, m, n, k):
     want = reference(x, w)
     assert want.abs().max() <= 256                      # representable in bf16 without rounding
     assert torch.equal(ops.skinny_linear(x, w).float(), want)
+
+
+@pytest.mark.parametrize("m", [1, 3, 9, 17, 33, 64])
+@pytest.mark.parametrize("ff", [2632, 4104, 6152, 8200, 9728, 12288, 12296, 20496])
+@pytest.mark.parametrize("k", [2048, 2176, 4096])
+def test_gate_and_up_in_one_launch_have_the_bits_of_two(gpu, m, ff, k):
+    """Walks over k begin at different places of it, so every sum has an order of its own: the same one in both, for 16 to 256 weight rows per workgroup, halves that
+    are whole workgroups and halves that are not."""
+    g = torch.Generator(device=gpu).manual_seed(m + ff + k)
+    x = torch.randn((m, k), generator=g, device=gpu).to(torch.bfloat16)
+    w = (0.05 * torch.randn((2 * ff, k), generator=g, device=gpu)).to(torch.bfloat16)
+    want, got = (torch.empty(m, ff, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    ops.silu_and_mul(want, ops.skinny_linear(x, w))
+    rc = ops._lib.load().infer_skinny_gate_silu_bf16(x.data_ptr(), k, w.data_ptr(), got.data_ptr(), ff, m, ff, k, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(got, want)
