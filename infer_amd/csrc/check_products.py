@@ -2,7 +2,8 @@
 
     check_products.py FILE.s KERNEL
 
-The compiler keeps the distances that matrix instructions need only between those that it knows.  For every instance of KERNEL in FILE.s
+The compiler keeps the distances that matrix instructions need only between those that it knows, which are the products outside of inline assembly (where a
+kernel has none marked, every product counts as written there).  For every instance of KERNEL in FILE.s
 this reports, over all ways through the branches: a register copy or other vector instruction that writes an operand of a product less than
 VALU_WAITS wait states in front of it; anything but the product itself that touches a product's result less than RESULT_WAITS behind it
 (eight passes need 11, sixteen 19); and the use of scratch memory, where spilled accumulators would go.  Exit code 1 if there is any of it,
@@ -37,21 +38,25 @@ def kernels(assembly, name):
 
 
 def parse(lines):
-    """Instructions, and for each the ones that may come in front of it."""
-    code, labels = [], {}
+    """Instructions, for each the ones that may come in front of it, and the places of those in inline assembly."""
+    code, labels, inline, inside = [], {}, set(), False
     for line in lines:
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            inside = "#ASMSTART" in line
         line = line.split(";")[0].strip()
         m = re.match(r"^(\.L\w+):", line)
         if m:
             labels[m[1]] = len(code)
         elif line and not line.startswith(".") and not line.endswith(":"):
+            if inside:
+                inline.add(len(code))
             code.append(line)
     before = [[i - 1] if i and not code[i - 1].startswith(("s_branch", "s_endpgm", "s_setpc")) else [] for i in range(len(code))]
     for i, line in enumerate(code):
         m = re.match(r"s_c?branch\w*\s+(\.L\w+)", line)
         if m and labels.get(m[1], len(code)) < len(code):
             before[labels[m[1]]].append(i)
-    return code, before
+    return code, before, inline
 
 
 def within(code, before, at, waits):
@@ -75,11 +80,12 @@ def product(line):
 
 
 def faults(lines):
-    code, before = parse(lines)
-    found = []
+    code, before, inline = parse(lines)
+    found, products = [], {i for i, line in enumerate(code) if product(line)}
+    written = products & inline or products                      # those between which the compiler keeps no distance
     for i, line in enumerate(code):
         used = operands(line)
-        if product(line):
+        if i in written:
             read = set().union(*used[1:])
             for p in within(code, before, i, VALU_WAITS):
                 if code[p].startswith("v_") and not product(code[p]) and operands(code[p]) and operands(code[p])[0] & read:
@@ -87,9 +93,9 @@ def faults(lines):
         touched = set().union(*used) if used else set()
         if touched and not line.startswith("s_"):
             for p in within(code, before, i, RESULT_WAITS):
-                if product(code[p]) and operands(code[p])[0] & touched:
+                if p in products and (p in written or i in written) and operands(code[p])[0] & touched:
                     found.append(f"touches a product's result too early: {code[p]} | {line}")
-    return found, sum(map(product, code))
+    return found, len(written)
 
 
 def scratch(assembly, symbol):

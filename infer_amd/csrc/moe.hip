@@ -6,6 +6,7 @@
 //   moe_block_kernel      products of many rows per expert: 256 rows x 256 columns per workgroup, straight from memory to LDS
 //   moe_tile_kernel       products of large row tiles: 128 rows x 128 columns per workgroup, through registers to LDS
 //   moe_span_kernel       products of up to 128 rows at a time: the weights pass the rows once
+//   moe_uneven_kernel     the same, and blocks for the experts that have more
 //   moe_row_kernel        products of up to 32 rows (decode): the weights stream past the rows; wavefronts split k or share its steps
 //   moe_any_kernel        any size and element type
 //
@@ -449,30 +450,80 @@ __global__ void __launch_bounds__(kThreads, 2) moe_tile_kernel(GemmArgs<__bf16> 
 constexpr int kBlockRows = 256, kBlockThreads = 256;
 // Tiles of an expert that are worked on side by side: a die's compute units then share that many blocks of rows and 32 / kSideTiles of W.
 constexpr int kSideTiles = 8;
-template <bool GATED>
-__global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) moe_block_kernel(GemmArgs<__bf16> a) {
-    constexpr int kMat = kBlockRows * 128;                       // bytes
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[5 * kMat];   // three buffers of W, two of rows
-    if (a.zero && blockIdx.x == 0)
-        for (int i = threadIdx.x; i < a.num_zero; i += kBlockThreads) a.zero[i] = 0;
-    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Workgroups go to the eight dies round-robin, and each die gets a contiguous run of (expert, group of tiles, columns, tile): those that
-    // run at the same time share rows and weights of one expert.  Behind the tiles there are, their number stands (scatter kernel).
-    const int none = a.tiles[2 * a.max_tiles - 2] < 0, total = none ? a.tiles[2 * a.max_tiles - 1] : a.max_tiles;
-    const unsigned columns = (unsigned)a.col_blocks, units = (unsigned)total * columns, die = blockIdx.x & 7u, extra = units & 7u;
-    if ((blockIdx.x >> 3) >= units / 8 + (die < extra ? 1 : 0)) return;
-    const unsigned unit = die * (units / 8) + (die < extra ? die : extra) + (blockIdx.x >> 3);
-    const int some = (int)(unit / columns);                      // a tile of the unit's expert
-    const int expert = a.tiles[2 * some];
-    if (expert < 0 || expert >= a.experts) return;
-    const int row0 = a.offsets[expert], end = a.offsets[expert + 1], tile0 = some - a.tiles[2 * some + 1] / kBlockRows;
+// Which tiles a launch has: all of them, or (MANY) those of experts with more than kSpan rows.
+constexpr int kSpan = 128;
+template <bool MANY>
+struct BlockTiles {
+    const GemmArgs<__bf16>& a;
+    // Of the tiles t .. t + 64 kSets - 1, one a lane and set, those that count; all requests of a kind at once.  Behind the last tile there are no experts.
+    static constexpr int kSets = 3;
+    __device__ __forceinline__ void counted(int t, uint64_t (&set)[kSets]) const {
+        int expert[kSets], rows[kSets];
+#pragma unroll
+        for (int i = 0; i < kSets; ++i) {
+            const int at = t + 64 * i + (int)(threadIdx.x & 63);
+            expert[i] = at < a.max_tiles ? a.tiles[2 * at] : -1;
+        }
+#pragma unroll
+        for (int i = 0; i < kSets; ++i) rows[i] = expert[i] >= 0 && expert[i] < a.experts ? a.offsets[expert[i] + 1] - a.offsets[expert[i]] : 0;
+#pragma unroll
+        for (int i = 0; i < kSets; ++i) set[i] = __ballot(rows[i] > kSpan);
+    }
+    __device__ __forceinline__ int total() const {
+        if constexpr (!MANY) return a.tiles[2 * a.max_tiles - 2] < 0 ? a.tiles[2 * a.max_tiles - 1] : a.max_tiles;      // behind the last their number stands
+        int n = 0;
+        for (int t = 0; t < a.max_tiles; t += 64 * kSets) {
+            uint64_t set[kSets];
+            counted(t, set);
+#pragma unroll
+            for (int i = 0; i < kSets; ++i) n += __popcll(set[i]);
+        }
+        return n;
+    }
+    // tile number `n` of them
+    __device__ __forceinline__ int at(int n) const {
+        if constexpr (!MANY) return n;
+        const int lane = threadIdx.x & 63;
+        for (int t = 0; t < a.max_tiles; t += 64 * kSets) {
+            uint64_t set[kSets];
+            counted(t, set);
+#pragma unroll
+            for (int i = 0; i < kSets; ++i) {
+                const int here = __popcll(set[i]);
+                if (n >= 0 && n < here) return t + 64 * i + __builtin_ctzll(__ballot((set[i] >> lane & 1) && __popcll(set[i] & ((1ull << lane) - 1)) == n));
+                n -= here;
+            }
+        }
+        return 0;
+    }
+};
+// The unit of workgroup number `block`: false if there is none, otherwise its expert, rows first .. first + rows - 1 and columns c0 and on.  Workgroups go to the eight
+// dies round-robin, and each die gets a contiguous run of (expert, group of tiles, columns, tile): those that run at the same time share rows and weights of one
+// expert.
+struct BlockUnit { int expert, first, rows, c0; };
+template <bool GATED, bool MANY>
+__device__ __forceinline__ bool block_unit(const GemmArgs<__bf16>& a, const BlockTiles<MANY>& list, int total, unsigned columns, unsigned block, BlockUnit& u) {
+    const unsigned units = (unsigned)total * columns, die = block & 7u, extra = units & 7u;
+    if ((block >> 3) >= units / 8 + (die < extra ? 1 : 0)) return false;
+    const unsigned unit = die * (units / 8) + (die < extra ? die : extra) + (block >> 3);
+    const int some = (int)(unit / columns), listed = list.at(some);         // a tile of the unit's expert
+    u.expert = a.tiles[2 * listed];
+    if (u.expert < 0 || u.expert >= a.experts) return false;
+    const int row0 = a.offsets[u.expert], end = a.offsets[u.expert + 1], tile0 = some - a.tiles[2 * listed + 1] / kBlockRows;
     const unsigned tiles = (unsigned)(end - row0 + kBlockRows - 1) / kBlockRows, groups = (tiles + kSideTiles - 1) / kSideTiles;
     const unsigned side = (tiles + groups - 1) / groups, of_expert = unit - (unsigned)tile0 * columns, group = of_expert / (side * columns);
     const unsigned here = tiles - group * side < side ? tiles - group * side : side, rest = of_expert - group * side * columns;
-    const int cb = (int)(rest / here), first = row0 + kBlockRows * (int)(group * side + rest % here);
-    const int rows = end - first < kBlockRows ? end - first : kBlockRows;
-    const int c0 = cb * (GATED ? 128 : 256);
+    u.first = row0 + kBlockRows * (int)(group * side + rest % here);
+    u.rows = end - u.first < kBlockRows ? end - u.first : kBlockRows;
+    u.c0 = (int)(rest / here) * (GATED ? 128 : 256);
+    return true;
+}
+constexpr int kBlockLds = 5 * kBlockRows * 128;                  // bytes: three buffers of W, two of rows
+template <bool GATED>
+__device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, const BlockUnit& u, unsigned char* lds) {
+    constexpr int kMat = kBlockRows * 128;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int first = u.first, rows = u.rows, c0 = u.c0;
     // load i of a wavefront fills rows 8 (8 wave + i) .. + 7: lane l place l % 8 of row l / 8
     uint32_t x_off[8], w_off[8];                                 // bytes (checked on the host to fit)
     const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(8192 * wave));
@@ -486,7 +537,7 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
         w_off[i] = 2u * ((uint32_t)(GATED && (r & 32) ? a.up_row + col : col) * (uint32_t)a.w_stride + 8u * unit);
     }
     const __bf16* xs = a.x;
-    const __bf16* ws = a.w + (int64_t)expert * a.w_expert;
+    const __bf16* ws = a.w + (int64_t)u.expert * a.w_expert;
     // Inline assembly, since the compiler would put a wait for all requests in front of every read of LDS.  Nothing else here uses M0.
     auto request = [&](uint32_t off, const __bf16* from, uint32_t at) {
         __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(from), "s"(at) : "memory", "m0");
@@ -605,6 +656,15 @@ __global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per
     }
 }
 
+template <bool GATED>
+__global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) moe_block_kernel(GemmArgs<__bf16> a) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kBlockLds];
+    clear_counts(a);
+    const BlockTiles<false> list{a};
+    BlockUnit u;
+    if (block_unit<GATED>(a, list, list.total(), (unsigned)a.col_blocks, blockIdx.x, u)) moe_block_product<GATED>(a, u, lds);
+}
+
 // A workgroup: up to 32 rows of one expert x some rows of W (a tile: 16, GATED: 8 gate and 8 up), which stream past them; the second half of the rows
 // costs only where there are that many.  64 rows, three of 16 experts of 3072 x 4096: 258 us with 32 rows of W past 16 rows through
 // operand registers, 181 us with one tile and wavefronts that split k (5.9 TB/s of weights).  Two tiles and wavefronts that share the steps of k read the
@@ -704,33 +764,64 @@ __global__ void __launch_bounds__(64 * kRowWaves) moe_row_kernel(GemmArgs<__bf16
     }
 }
 
-// A workgroup: four or eight tiles of W past up to 128 rows of one expert at a time, which the four wavefronts share (SharedStream), for as many rows as a
-// decode batch or a few short prompts bring.  The weights bound such a product, each of which should pass once: tiles of 32 rows read them again for
-// every 32 rows, and blocks and tiles of 128 and 256 rows compute what there is not.  A workgroup has what begins with its tile and ends before the next
-// multiple of kSpan rows, or of a tile if that has more; the tiles in between have nothing to do.
+// A workgroup: four or eight tiles of W past up to kSpan rows of one expert at a time, which the four wavefronts share (SharedStream), for as many rows as a
+// decode batch or a few short prompts bring.  The weights bound such a product, each of which should pass once: tiles of 32 rows read them again for every 32
+// rows, and blocks and tiles of 128 and 256 rows compute what there is not.  A workgroup has what begins with its tile and ends before the next multiple of kSpan
+// rows, or of a tile if that has more; the tiles in between have nothing to do.
 //
 // A step's experts, us, before / this: 14 of 4096 x 3072, three choices, 100 rows 199 / 192, 130 242 / 197, 160 278 / 201, 300 284 / 227, 500 305 / 247; 14 of
 // 1024 x 3072, 200 rows 106 / 72; 128 of 2048 x 768, eight choices, 400 rows 305 / 246; 8 of 4096 x 14336, two, 104 rows 667 / 445, 400 703 / 566; 8 of
 // 2048 x 8192, 200 rows 276 / 173.  Fewer or more choices per expert: 14 of 4096 x 3072, 64 rows (14 each) 184 / 189, 700 (150) 306 / 438, since most of them
 // then have more than 128.
-constexpr int kSpan = 128;
+template <bool GATED, int RT>
+__device__ __forceinline__ void moe_span_rows(const GemmArgs<__bf16>& a, int expert, int first, int rows, int cb, unsigned char* lds) {
+    const int c0 = cb * (GATED ? 8 : 16) * RT;
+    if (rows <= 32) moe_shared_product<GATED, RT, 2>(a, expert, first, rows, c0, lds);
+    else if (rows <= 64) moe_shared_product<GATED, RT, 4>(a, expert, first, rows, c0, lds);
+    else moe_shared_product<GATED, RT, 8>(a, expert, first, rows, c0, lds);
+}
+template <int RT>
+constexpr int span_lds() {
+    constexpr int k2 = SharedStream<RT, 2>::kRing, k4 = SharedStream<RT, 4>::kRing, k8 = SharedStream<RT, 8>::kRing, k24 = k2 > k4 ? k2 : k4;
+    return k24 > k8 ? k24 : k8;
+}
 template <bool GATED, int RT>
 __global__ void __launch_bounds__(64 * kRowWaves) moe_span_kernel(GemmArgs<__bf16> a, int tile_rows) {
-    constexpr int k2 = SharedStream<RT, 2>::kRing, k4 = SharedStream<RT, 4>::kRing, k8 = SharedStream<RT, 8>::kRing, k24 = k2 > k4 ? k2 : k4;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[k24 > k8 ? k24 : k8];
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[span_lds<RT>()];
     clear_counts(a);
     const int tile = blockIdx.x / a.col_blocks, cb = blockIdx.x % a.col_blocks;
     const int expert = a.tiles[2 * tile], row0 = a.tiles[2 * tile + 1], span = tile_rows > kSpan ? tile_rows : kSpan;
     if (expert < 0 || expert >= a.experts || row0 % span) return;
-    const int first = a.offsets[expert] + row0, end = a.offsets[expert + 1];
-    const int rows = end - first < span ? end - first : span, c0 = cb * (GATED ? 8 : 16) * RT;
+    const int first = a.offsets[expert] + row0, end = a.offsets[expert + 1], rows = end - first < span ? end - first : span;
     for (int at = 0; at < rows; at += kSpan) {
         if (at > 0) __syncthreads();                   // everybody has read what lies in LDS
-        const int here = rows - at < kSpan ? rows - at : kSpan;
-        if (here <= 32) moe_shared_product<GATED, RT, 2>(a, expert, first + at, here, c0, lds);
-        else if (here <= 64) moe_shared_product<GATED, RT, 4>(a, expert, first + at, here, c0, lds);
-        else moe_shared_product<GATED, RT, 8>(a, expert, first + at, here, c0, lds);
+        moe_span_rows<GATED, RT>(a, expert, first + at, rows - at < kSpan ? rows - at : kSpan, cb, lds);
     }
+}
+// The same with tiles of 256 rows, but experts with more than kSpan rows go in blocks, which come first.  How many there are is known here alone: the host deals
+// out workgroups for all that there can be, and those behind the last have nothing to do.  All experts in blocks / all in spans / this, us: 14 of 4096 x 3072, 500
+// rows, at most 128 of an expert 303 / 251 / 252, 236 302 / 322 / 249, 402 301 / 333 / 263, all at three 161 / 274 / 162; 8 of 4096 x 14336, 400 rows, 120 705 / 588 /
+// 585, 155 704 / 757 / 684, all at two 437 / 690 / 442; 128 of 2048 x 768, 1200 rows, 101 339 / 312 / 317, 356 377 / 363 / 328, all at half of them 231 / 294 / 240.
+// (As two launches, each of which ends by itself: 255, 352, 337, 168 for the first four.)
+template <bool GATED>
+__global__ void __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) moe_uneven_kernel(GemmArgs<__bf16> a, unsigned block_columns) {
+    constexpr int RT = 8, kSpanLds = span_lds<RT>();
+    static_assert(kBlockThreads == 64 * kRowWaves, "both have four wavefronts");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kBlockLds > kSpanLds ? kBlockLds : kSpanLds];
+    clear_counts(a);
+    const BlockTiles<true> list{a};
+    const int total = list.total();
+    const unsigned blocks = ((unsigned)total * block_columns + 7) / 8 * 8;
+    if (blockIdx.x < blocks) {
+        BlockUnit u;
+        if (block_unit<GATED>(a, list, total, block_columns, blockIdx.x, u)) moe_block_product<GATED>(a, u, lds);
+        return;
+    }
+    const unsigned at = blockIdx.x - blocks, tile = at / (unsigned)a.col_blocks;
+    const int expert = tile < (unsigned)a.max_tiles ? a.tiles[2 * tile] : -1;
+    if (expert < 0 || expert >= a.experts) return;
+    const int first = a.offsets[expert], rows = a.offsets[expert + 1] - first;
+    if (rows <= kSpan) moe_span_rows<GATED, RT>(a, expert, first, rows, (int)(at % (unsigned)a.col_blocks), lds);       // its only tile
 }
 
 // one wavefront per (place, four columns)
@@ -761,10 +852,11 @@ __global__ void __launch_bounds__(kThreads) moe_any_kernel(GemmArgs<T> a) {
 bool size_in(int64_t v, int64_t lo, int64_t hi) { return v >= lo && v <= hi; }
 
 template <class T>
-int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t choices, int64_t max_places, hipStream_t st) {
+int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t tokens, int64_t choices, int64_t max_places, hipStream_t st) {
     const dim3 block(kThreads);
     int64_t grid;
     if constexpr (sizeof(T) == 2) {
+        const int64_t block_columns = (a.out_cols + (gated ? 127 : 255)) / (gated ? 128 : 256);
         if (tile_rows >= kSmallRows && a.k % kStreamK == 0 && choices >= 18 * a.experts && choices <= 112 * a.experts) {
             // eight tiles of W, unless four have the compute units through earlier: a tile takes about three times what the rows beside it do (8 experts of
             // 1536 x 4096, 100 rows 79 / 68 us; 14 of 4096 x 3072, 130 rows 197 / 205)
@@ -775,18 +867,26 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t choices, int64_t max
             const int tiles = takes(4) < takes(8) ? 4 : 8, per = (gated ? 8 : 16) * tiles;
             a.col_blocks = (a.out_cols + per - 1) / per;
             grid = (int64_t)a.max_tiles * a.col_blocks;
+            // An expert with more rows than kSpan reads its weights again for every kSpan of them, and what it computes is bound by LDS.  Where blocks would serve if
+            // all had that many, they serve those that have, next to the others.  With four tiles of W two workgroups share a compute unit, which one with a
+            // block's LDS would not: 8 of 1536 x 4096, 300 rows, at most 151 of an expert 131 us with blocks for both products, 109 with blocks for the first alone.
+            const bool uneven = tile_rows == kBlockRows && tokens > kSpan && tiles == 8;
+            if (uneven) {
+                const int64_t large = choices / (kSpan + 1) < a.experts ? choices / (kSpan + 1) : a.experts;     // so many have more than kSpan at most
+                grid += ((choices / kBlockRows + large) * block_columns + 7) / 8 * 8;
+            }
             if (grid > 0x7fffffff) return INFER_KV_EINVAL;
-#define GO(GATED, RT) hipLaunchKernelGGL((moe_span_kernel<GATED, RT>), dim3((unsigned)grid), block, 0, st, a, tile_rows)
-            if (gated && tiles == 8) GO(true, 8);
-            else if (gated) GO(true, 4);
-            else if (tiles == 8) GO(false, 8);
-            else GO(false, 4);
-#undef GO
+            if (uneven && gated) hipLaunchKernelGGL((moe_uneven_kernel<true>), dim3((unsigned)grid), block, 0, st, a, (unsigned)block_columns);
+            else if (uneven) hipLaunchKernelGGL((moe_uneven_kernel<false>), dim3((unsigned)grid), block, 0, st, a, (unsigned)block_columns);
+            else if (gated && tiles == 8) hipLaunchKernelGGL((moe_span_kernel<true, 8>), dim3((unsigned)grid), block, 0, st, a, tile_rows);
+            else if (gated) hipLaunchKernelGGL((moe_span_kernel<true, 4>), dim3((unsigned)grid), block, 0, st, a, tile_rows);
+            else if (tiles == 8) hipLaunchKernelGGL((moe_span_kernel<false, 8>), dim3((unsigned)grid), block, 0, st, a, tile_rows);
+            else hipLaunchKernelGGL((moe_span_kernel<false, 4>), dim3((unsigned)grid), block, 0, st, a, tile_rows);
             return (int)hipGetLastError();
         }
         if (tile_rows == kBlockRows) {
-            a.col_blocks = (a.out_cols + (gated ? 127 : 255)) / (gated ? 128 : 256);
-            grid = ((int64_t)a.max_tiles * a.col_blocks + 7) / 8 * 8;
+            a.col_blocks = (int)block_columns;
+            grid = (a.max_tiles * block_columns + 7) / 8 * 8;
             if (grid > 0x7fffffff) return INFER_KV_EINVAL;
             if (gated) hipLaunchKernelGGL((moe_block_kernel<true>), dim3((unsigned)grid), dim3(kBlockThreads), 0, st, a);
             else hipLaunchKernelGGL((moe_block_kernel<false>), dim3((unsigned)grid), dim3(kBlockThreads), 0, st, a);
@@ -822,8 +922,8 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t choices, int64_t max
 // rows per tile: 0 where only the any-size kernels serve
 int rows_per_tile(int elem, int64_t n, int64_t width, int64_t ff_pad, int64_t experts, int64_t top) {
     if (elem != INFER_ELEM_BF16 || width % 8 || ff_pad % 8) return 0;
-    // The tiles that moe_row_kernel, moe_tile_kernel and moe_block_kernel work on.  With 18 to 112 choices per expert and k in whole steps moe_span_kernel takes what
-    // begins with every 128 rows, whatever the tiles; the figures are of the others.
+    // The tiles that moe_row_kernel, moe_tile_kernel and moe_block_kernel work on; the figures are of these.  With 18 to 112 choices per expert and k in whole steps
+    // moe_span_kernel takes what begins with every 128 rows, whatever the tiles, but for experts with more where tiles are blocks.
     // An expert with more than one tile of 32 rows reads its weights again, and around 32 choices per expert half of them have more.  That costs
     // little where the weights are few, more where there are many of them or many experts; us, tiles of 32 rows / the others: 8 experts of
     // 1536 x 4096, 32 choices each 105 / 136; 8 of 2048 x 8192, 28 234 / 275; 14 of 4096 x 3072, 25 261 / 282, 32 330 / 280; 8 of 4096 x 14336, 26
@@ -895,11 +995,11 @@ extern "C" int infer_moe(int elem, const void* h, int64_t h_stride, const void* 
         hipLaunchKernelGGL(moe_scatter_kernel, dim3((unsigned)((choices + kThreads - 1) / kThreads)), dim3(kThreads), 0, st, s);
         GemmArgs<T> up{(const T*)h, h_stride, row_token, row_expert, offsets, tiles, (const T*)gate_up, 2 * ff * width, width, (int)width, (int)ff,
                        (int)ff, (T*)act, ff_pad, (int)ff_pad, counts, (int)experts, (int)experts, (int)max_tiles, 0};
-        int rc = gemm(up, true, tile_rows, choices, max_places, st);
+        int rc = gemm(up, true, tile_rows, n, choices, max_places, st);
         if (rc) return rc;
         GemmArgs<T> dn{(const T*)act, ff_pad, nullptr, row_expert, offsets, tiles, (const T*)down, width * ff_pad, ff_pad, (int)ff_pad, (int)width,
                        0, (T*)out, width, (int)width, nullptr, 0, (int)experts, (int)max_tiles, 0};
-        return gemm(dn, false, tile_rows, choices, max_places, st);
+        return gemm(dn, false, tile_rows, n, choices, max_places, st);
     };
     if (elem == INFER_ELEM_BF16) return go(__bf16(0.f));
     if (elem == INFER_ELEM_F32) return go(0.f);

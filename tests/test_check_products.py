@@ -34,6 +34,12 @@ BAD = {
     "a result read behind a branch": [PRODUCT, "s_cbranch_scc1 .LBB0_2", "s_nop 15", "s_nop 15", ".LBB0_2:", "v_accvgpr_read_b32 v8, a3"],
     "a result that enters the next product": [PRODUCT, PRODUCT],
 }
+INLINE = [";;#ASMSTART", PRODUCT, ";;#ASMEND"]
+GOOD["products of the compiler's, which keeps their distances"] = [*INLINE, *OTHERS, OTHERS[0], "v_accvgpr_read_b32 v8, a4"]
+BAD["a product in assembly beside others, its result read at once"] = [*OTHERS, *INLINE, "v_accvgpr_read_b32 v8, a0"]
+BAD["a result that enters a product of the compiler's"] = [*INLINE, PRODUCT]
+BAD["a result of a product of the compiler's"] = [PRODUCT, *INLINE]
+BAD["a copy in front of assembly"] = ["v_mov_b32_e32 v5, v12", *INLINE]
 
 
 @pytest.mark.parametrize("body", GOOD.values(), ids=GOOD)

@@ -1,5 +1,7 @@
 """The kernels of masked attention, of the state space, of the mixture of experts and of the pre-norm residual stream, each alone,
 against ``oracle/dogetar_ref.py`` (float64) on random inputs made so that a wrong key, token, state or expert shows."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -605,9 +607,10 @@ def test_moe_when_all_tokens_want_the_same_expert(gpu):
     close(x, y * (p[:, 4] / p.sum(-1))[:, None], 2e-2)
 
 
-@pytest.mark.parametrize("width,ff,experts,n", [(256, 64, 5, 2600), (64, 5120, 8, 300), (448, 384, 1, 4700)])
+@pytest.mark.parametrize("width,ff,experts,n", [(256, 64, 5, 2600), (64, 5120, 8, 300), (64, 5120, 2, 800), (448, 384, 1, 4700)])
 def test_moe_blocks_of_uneven_experts(gpu, width, ff, experts, n):
-    """Blocks of 256 rows: nearly all rows at one expert, in one and more groups of its tiles; few rows and many columns; one to seven steps.
+    """Blocks of 256 rows: nearly all rows at one expert, in one and more groups of its tiles; few rows and many columns; one to seven steps.  300 rows of eight
+    experts go through 128 at a time.
     Inner results are rounded to bf16, sums of up to 5120 products of theirs to bf16 once more: 2e-2 as for the other kernels."""
     rng, bf = np.random.default_rng(ff), torch.bfloat16
     s = ho.MoeShape(width, ff, experts, 1, 0, 1, 1, 1.0)
@@ -656,9 +659,36 @@ def test_moe_rows_of_a_long_k(gpu, width, ff, n):
 @pytest.mark.parametrize("width,ff", [(64, 128), (256, 72), (520, 192), (2304, 136)])
 @pytest.mark.parametrize("n", [71, 72, 97, 128, 129, 161, 257, 300, 448, 449])
 def test_moe_rows_that_weights_pass_once(gpu, width, ff, n):
-    """The same with so many rows per expert that the weights pass up to 128 of them at once: all at one expert, in tiles of 32, 128 and 256, the last ones
+    """The same with so many rows per expert that the weights pass up to 128 of them at once: all at one expert, in tiles of 32 and 128, the last ones
     of 1 to 128 rows; just outside the range; one product of it alone, where the other's k is no multiple of a step."""
     test_moe_rows_around_the_tiles_that_weights_stream_past(gpu, width, ff, n)
+
+
+@pytest.mark.parametrize("counts", [(128, 129, 0, 1, 256, 100), (129, 129, 1, 129, 129, 129), (0, 0, 0, 600, 0, 0), (128, 128, 128, 128, 128, 0), (257, 33, 65, 0, 8, 64),
+                                    (0, 1, 512, 2, 0, 128)])
+def test_moe_experts_of_128_rows_and_more(gpu, counts):
+    """Rows that would go in blocks if all experts had that many: those of up to 128 go past the weights at once, the others, one and more tiles of an expert and
+    several experts of them or none, in blocks.  Roundings as in the blocks' test."""
+    rng, bf, width, ff, experts, n = np.random.default_rng(sum(counts)), torch.bfloat16, 64, 5120, 6, sum(counts)
+    layout = (ctypes.c_int64 * 3)()
+    assert ho._lib.load().infer_moe_layout(ho.ELEM[bf], n, width, ff, experts, 1, ctypes.addressof(layout)) == 0
+    assert layout[2] == 256 and 18 * experts <= n <= 112 * experts
+    chosen = rng.permutation(np.repeat(np.arange(experts), counts))
+    h = rounded(rng.standard_normal((n, width)), bf)
+    h[:, :experts] = 4.0 * (chosen[:, None] == np.arange(experts))
+    router = np.eye(experts, width)
+    w = [rounded(rng.standard_normal(shape) * shape[-1] ** -0.5, bf) for shape in ((experts, 2 * ff, width), (experts, width, ff))]
+    zero = torch.zeros(experts, dtype=torch.int32, device=gpu)
+    r = ho.moe(ho.MoeShape(width, ff, experts, 1, 0, 1, 1, 1.0), dev(h, bf), dev(router, bf), None, dev(w[0], bf), dev(w[1], bf), zero)
+    x = torch.zeros((n, width), device=gpu)
+    ho.pre_norm(x, torch.ones(width, device=gpu), 1e-6, y=r)
+    want, weight = np.zeros((n, width)), np.exp(4.0) / (np.exp(4.0) + experts - 1)
+    for e in range(experts):
+        at = chosen == e
+        inner = silu(h[at] @ w[0][e][:ff].T) * (h[at] @ w[0][e][ff:].T)
+        want[at] = inner @ w[1][e].T * weight
+    close(x, want, 2e-2)
+    assert (zero == 0).all()
 
 
 def test_bad_arguments_are_refused(gpu):
