@@ -843,7 +843,7 @@ int launch_out(const DecayOutArgs<T>& a, bool per_head, int64_t rows, hipStream_
         return (int)hipGetLastError();
     }
     const int chunks = ((vec ? n / 4 : n) + kThreads - 1) / kThreads;
-    const bool once = vec && beyond_caches(2 * rows * n * (int64_t)sizeof(T));
+    const bool once = vec && beyond_caches(2 * rows * n * (int64_t)sizeof(T), 32);
 #define GO(V, N) do { \
         if (V > 1 && once) hipLaunchKernelGGL((decay_out_row_kernel<T, V, N, (V > 1)>), grid, block, 0, st, a); \
         else hipLaunchKernelGGL((decay_out_row_kernel<T, V, N, false>), grid, block, 0, st, a); \

@@ -42,9 +42,11 @@ __device__ __forceinline__ void load_elems(const __bf16* p, float (&x)[N]) {
         for (int i = 0; i < N; ++i) x[i] = (float)p[i];
     }
 }
-// Whether inputs of so many bytes, just written, have left the second-level caches, so that the streaming hint costs nothing: norms behind the recurrences, a call
-// without / with the hint, us: 12 MB 55.3 / 57, 16 MB 44.2 / 44.6, 38 MB 74 / 71, 90 MB 150.4 / 149.9, 226 MB 271 / 268.
-inline bool beyond_caches(int64_t bytes) { return bytes > (32ll << 20); }
+// Whether inputs of a norm behind a recurrence have left the caches by the time it reads them, so that the streaming hint costs nothing: from `line` MB on, which
+// depends on what else the kernels in front of it write.  A call without / with the hint, us: constant decay of 32 heads, 16 MB 44.0 / 44.6, 30 60.9 / 60.8, 34 66.5 /
+// 65.9, 40 74.5 / 73.1, 200 266 / 262; state space of 32 heads, one portion, 16 MB 58.1 / 59.1, 34 83.5 / 86.1, 38 91.1 / 91.3, 40 95.3 / 93.2; of 64, eight of
+// them, 34 56.7 / 56.7, 40 63.5 / 61.0, 260 304 / 299.
+inline bool beyond_caches(int64_t bytes, int line) { return bytes > ((int64_t)line << 20); }
 
 // load_elems, ONCE: with the streaming hint, of what nobody reads again.  p: then aligned to the N elements, at most 16 bytes.
 template <int N, bool ONCE, class T>

@@ -561,7 +561,8 @@ struct NormArgs {
     T* out; int64_t out_stride;
 };
 
-// Bound by memory: 13,800 rows of 4096 (two read, one written) 340 MB.  ONCE: beyond_caches.
+// Bound by memory: 13,800 rows of 4096 (two read, one written) 340 MB.  ONCE: rows that are kept, with the streaming hint.
+constexpr int kKeep = 4;                   // chunks kept between the sum and the result; more are computed twice
 template <class T, int VEC, bool ONCE>
 __global__ void __launch_bounds__(kThreads) ssm_norm_kernel(NormArgs<T> b) {
     __shared__ float part[kThreads / 64];
@@ -570,7 +571,6 @@ __global__ void __launch_bounds__(kThreads) ssm_norm_kernel(NormArgs<T> b) {
     const int size = a.heads * a.vdim / b.parts, c0 = blockIdx.y * size, tid = threadIdx.x;
     const T* y = a.y + row * a.y_stride + c0;
     const T* z = a.proj + row * a.proj_stride + a.z_off + c0;
-    constexpr int kKeep = 4;               // chunks kept between the sum and the result; more are computed twice
     float x[kKeep][VEC], ss = 0.f;
     auto gated = [&](int c, float (&v)[VEC]) {
         float w[VEC];
@@ -763,7 +763,7 @@ extern "C" int infer_state_space(int elem, const void* proj, int64_t proj_stride
         const bool vec = size % 8 == 0 && inner % 8 == 0 && proj_stride % 8 == 0 && z_off % 8 == 0 && out_stride % 8 == 0 &&
                          ptr_aligned(proj, 16) && ptr_aligned(y, 16) && ptr_aligned(out, 16) && ptr_aligned(norm, 16);
         const dim3 grid((unsigned)n, (unsigned)norm_parts), block(kThreads);
-        if (vec && beyond_caches(2 * n * inner * (int64_t)sizeof(T))) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, true>), grid, block, 0, st, b);
+        if (vec && size <= 8 * kKeep * kThreads && beyond_caches(2 * n * inner * (int64_t)sizeof(T), 39)) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, true>), grid, block, 0, st, b);
         else if (vec) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, false>), grid, block, 0, st, b);
         else hipLaunchKernelGGL((ssm_norm_kernel<T, 1, false>), grid, block, 0, st, b);
         return (int)hipGetLastError();

@@ -408,6 +408,19 @@ def test_state_space_of_unequal_sequences_in_one_step(gpu, dtype):
             close(torch.tensor(y), want[i][lo:lo + c], tol(dtype, 1e-5, 2e-2))
 
 
+@pytest.mark.parametrize("parts", [1, 2, 4])
+def test_state_space_norm_of_more_rows_than_caches_hold(gpu, parts):
+    """Rows are normed alike whether they are read with the streaming hint or without it; parts of one row that stay in registers, just so, and that do not."""
+    m = Ssm(np.random.default_rng(parts), (128, 128, 2, 1, 4, parts), torch.bfloat16)
+    x = m.inputs(4)
+    rows = [(i, 0, x[i:i + 1]) for i in range(4)]
+    few, many = m.run(rows), m.run(rows + [(-1, 0, x[:1])] * 636)
+    assert 2 * 640 * m.s.inner * 2 > 39 << 20
+    for i in range(4):
+        close(torch.tensor(few[i]), m.want(x[i:i + 1])[0], 2e-2)
+        assert (few[i] == many[i]).all()
+
+
 @pytest.mark.parametrize("shape", [SSM[2], SSM[3]])
 def test_state_space_segments_of_a_long_portion(gpu, shape):
     """Few heads and one sequence: the portion is cut into segments whose states are joined."""

@@ -440,6 +440,19 @@ def test_decay_portions_that_take_turns(gpu, kind, heads, lens):
         d.check_state(state, slot, end, state_tol(d, bf))
 
 
+def test_decay_norm_of_more_rows_than_caches_hold(gpu):
+    """Rows are normed alike whether they are read with the streaming hint or without it."""
+    d = Decay("lightning", tuple(1.0 - 2.0 ** -(2 + i % 9) for i in range(32)), 16, 128, 0, torch.bfloat16)
+    x = rounded(d.inputs(4), torch.bfloat16)
+    outs = []
+    for n in (4, 2100):
+        slots = dev([i if i < 4 else -1 for i in range(n)], torch.int32)
+        outs.append(d.run(x[np.arange(n) % 4], d.state(4), slots, torch.zeros(n, dtype=torch.int64, device=gpu), n, []))
+    assert 2 * 2100 * 32 * 128 * 2 > 32 << 20 and torch.equal(outs[0], outs[1][:4])
+    for i in range(4):
+        close(outs[0][i:i + 1], d.want(x[i:i + 1], 0, np.zeros((32, 16, 128)))[0], tol(torch.bfloat16, 1e-5))
+
+
 @BYKIND
 def test_decay_state_does_not_drift_over_many_steps(gpu, kind):
     """4000 decoded tokens of zeros: what is left of the state is decay^4000 of it to float precision."""
