@@ -151,7 +151,7 @@ def test_streamed_weights_of_a_long_k(gpu, m, n, k):
 @pytest.mark.parametrize("m", [33, 48, 64])
 @pytest.mark.parametrize("n,k", [(1536, 9728), (1000, 9728), (4616, 6656), (4608, 3072), (5120, 3200)])
 def test_streamed_weights_cut_into_more_workgroups_than_compute_units_and_fewer(gpu, m, n, k):
-    """As above: more than 256 workgroups of two wavefronts each, and factors that leave 146 and 216 of four."""
+    """As above: more workgroups than compute units, and factors that leave 146 and 216 of them."""
     test_streamed_weights_of_a_long_k(gpu, m, n, k)
 
 
@@ -253,7 +253,7 @@ def test_a_very_long_k(gpu, m, n, k):
 @pytest.mark.parametrize("m", [1, 3, 9, 17, 33, 64])
 @pytest.mark.parametrize("ff", [2632, 4104, 6152, 8200, 9728, 12288, 12296, 20496])
 @pytest.mark.parametrize("k", [2048, 2176, 4096])
-def test_gate_and_up_in_one_launch_have_the_bits_of_two(gpu, m, ff, k):
+def test_gate_and_up_of_a_long_k_have_the_bits_of_two(gpu, m, ff, k):
     """Walks over k begin at different places of it, so every sum has an order of its own: the same one in both, for 16 to 256 weight rows per workgroup, halves that
     are whole workgroups and halves that are not."""
     g = torch.Generator(device=gpu).manual_seed(m + ff + k)
