@@ -518,10 +518,8 @@ def test_delta_slabs_of_few_portions(gpu, heads, dim, vdim):
         assert (rest[:, dim:] == 0).all() and (rest[:, :, vdim:] == 0).all()
 
 
-@pytest.mark.parametrize("heads,dim,vdim", [(90, 64, 64), (90, 24, 20), (260, 32, 80)])
-def test_delta_portions_that_take_turns(gpu, heads, dim, vdim):
-    """More workgroups than compute units: the longest portions go first, equal and empty ones in their order, several to the first round or not even one."""
-    lens = (37, 97, 37, 0, 40)
+def check_turns(heads, dim, vdim, lens):
+    """Portions that take turns, each from the start, one of no tokens among them."""
     c = DeltaCase(heads, heads, dim, vdim, 4, sum(lens), torch.float32, slots=len(lens))
     c.dt -= 2.0
     chunks, portions, ring, pos, row = [], [], [], [], 0
@@ -531,7 +529,7 @@ def test_delta_portions_that_take_turns(gpu, heads, dim, vdim):
         ring += [(slot, k - 1 - r) for r in range(k)]
         pos += range(k)
         row += k
-    assert len(lens) * heads > 256 and row >= 8 * len(lens) ** 2
+    assert row >= 8 * len(lens) ** 2
     out = torch.full((row, heads * vdim), float("nan"), device="cuda")
     ho.delta_chunks(c.s, dev(c.proj), c.beta_off, dev(c.decay), dev(c.gate), *c.weights, c.ring, c.state, dev(portions, torch.int32),
                     dev(chunks, torch.int32), dev(ring, torch.int32), dev(pos, torch.int64), 0, out)
@@ -545,6 +543,27 @@ def test_delta_portions_that_take_turns(gpu, heads, dim, vdim):
         else:
             assert (c.state[slot] == 0).all()
         row += k
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(90, 64, 64), (90, 24, 20), (260, 32, 80)])
+def test_delta_portions_that_take_turns(gpu, heads, dim, vdim):
+    """More workgroups than compute units, one for a head and its columns: the longest portions go first, equal and empty ones in their order, several to the first
+    round or not even one."""
+    assert 5 * heads > 256
+    check_turns(heads, dim, vdim, (37, 97, 37, 0, 40))
+
+
+@pytest.mark.parametrize("heads,dim,vdim,lens", [
+    (110, 12, 32, (17, 60, 17)), (110, 32, 32, (33, 0, 50)), (40, 20, 140, (17, 60, 17)), (100, 48, 44, (17, 60, 17)), (30, 60, 130, (20, 1, 55)), (30, 96, 144, (17, 60, 17)),
+    (22, 128, 256, (17, 60, 17)), (24, 100, 196, (16, 48, 33)), (30, 192, 144, (17, 60, 17)), (30, 250, 140, (40, 16, 32))])
+def test_delta_scan_of_many_heads(gpu, heads, dim, vdim, lens):
+    """Sizes of every number of row tiles that neither one workgroup for a head and its outputs nor one for a few of its columns takes, in turns: heads of more than
+    128 columns, small ones and those of 16, 48, 192 and 256 rows."""
+    rows, tiles, pairs = next(r for r in (16, 32, 48, 64, 96, 128, 192, 256) if r >= dim), -(-vdim // 16), 3 * heads
+    assert (pairs * -(-tiles // 4) if rows == 128 else pairs * tiles / 2.5) > 256                       # otherwise a few columns each
+    assert rows in (16, 48, 192, 256) or tiles > 8 or (rows * tiles * 16 <= 2048 and vdim in (32, 64))    # otherwise a head and its outputs
+    assert pairs * -(-tiles // 4) > 256                                                                 # turns
+    check_turns(heads, dim, vdim, lens)
 
 
 def test_delta_empty_portions_and_chunks(gpu):
@@ -586,23 +605,24 @@ def test_delta_empty_chunks_of_square_heads(gpu, dim):
     close(c.state[1], want_state, 3e-5)
 
 
-def test_delta_state_of_operands_of_one_sign_does_not_drift(gpu):
+@pytest.mark.parametrize("heads,dim,others", [(33, 32, 6), (3, 32, 0), (2, 128, 0), (20, 128, 1), (33, 128, 1)])
+def test_delta_state_of_operands_of_one_sign_does_not_drift(gpu, heads, dim, others):
     """3200 tokens without decay whose keys, values and inner results are all positive, beside six short portions, so that one workgroup
-    holds all columns of a head.  Roundings to nearest of the 200 chunks' sums partly cancel: sqrt(200) of them are 14 x 2^-24, as many as
-    six of the operands' come on top, and ten of beta = sigmoid(-9), whose exponent is rounded at 9 log2(e) = 13 and so is off by 2^-21, with
+    holds all columns of a head, or beside one or none, so that it holds 64, 32 or 16 of them.  Roundings to nearest of the 200 chunks' sums partly
+    cancel: sqrt(200) of them are 14 x 2^-24, as many as six of the operands' come on top, and ten of beta = sigmoid(-9), whose exponent is rounded at 9 log2(e) = 13 and so is off by 2^-21, with
     the constant in it: 30 x 2^-24 = 1.8e-6 of the state's norm.  A rounding towards one side, or terms left out of one sign, in each of a
     chunk's products adds up instead."""
-    heads, n = 33, 3200
-    c = DeltaCase(heads, 1, 32, 32, 4, n + 6 * 16, torch.float32, slots=7, decay=-20.0)
+    n = 3200
+    c = DeltaCase(heads, 1, dim, dim, 4, n + others * 16, torch.float32, slots=7, decay=-20.0)
     rng, f32 = np.random.default_rng(5), lambda x: rounded(x, torch.float32)
     c.proj, c.conv, c.a_log = f32(0.5 + rng.random(c.proj.shape)), f32(0.2 + 0.2 * rng.random(c.conv.shape)), np.zeros(heads)
     c.proj[:, c.beta_off:] = f32(-9 + 0.1 * rng.standard_normal(c.proj[:, c.beta_off:].shape))
-    chunks = [(r, 16, r, 0, 0, 0) for r in range(0, n, 16)] + [(n + 16 * i, 16, 0, 0, i + 1, 0) for i in range(6)]
-    portions = [(0, n // 16, 0, 0)] + [(n // 16 + i, 1, i + 1, 0) for i in range(6)]
-    ring = [(0, n - 1 - r) for r in range(n)] + [(i + 1, 15 - r) for i in range(6) for r in range(16)]
-    out = torch.empty((c.n, heads * 32), device="cuda")
+    chunks = [(r, 16, r, 0, 0, 0) for r in range(0, n, 16)] + [(n + 16 * i, 16, 0, 0, i + 1, 0) for i in range(others)]
+    portions = [(0, n // 16, 0, 0)] + [(n // 16 + i, 1, i + 1, 0) for i in range(others)]
+    ring = [(0, n - 1 - r) for r in range(n)] + [(i + 1, 15 - r) for i in range(others) for r in range(16)]
+    out = torch.empty((c.n, heads * dim), device="cuda")
     ho.delta_chunks(c.s, dev(c.proj), c.beta_off, dev(c.decay), dev(c.gate), *c.weights, c.ring, c.state, dev(portions, torch.int32),
-                    dev(chunks, torch.int32), dev(ring, torch.int32), dev(list(range(n)) + 6 * list(range(16)), torch.int64), 0, out)
+                    dev(chunks, torch.int32), dev(ring, torch.int32), dev(list(range(n)) + others * list(range(16)), torch.int64), 0, out)
     state = host(c.state[0])
     c.n = n
     c.proj, c.decay, c.gate = c.proj[:n], c.decay[:n], c.gate[:n]
