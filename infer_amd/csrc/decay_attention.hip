@@ -170,11 +170,6 @@ __device__ __forceinline__ u32x2_t silu8(u32x2_t x) {            // of half as m
     for (int i = 0; i < 4; ++i) r[i] = (__bf16)silu_f((float)r[i]);
     return __builtin_bit_cast(u32x2_t, r);
 }
-// A value that the compiler takes for a new one: what is computed from it is not kept in registers over the whole loop.
-__device__ __forceinline__ int renewed(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
 
 // A workgroup of four or eight wavefronts serves one head and 16 VT columns of its state per wavefront over the chunks of one segment.
 // Wavefront w owns the columns 16 VT w .. and their part of the state, DT tiles of 32 rows, as accumulators: lane (g, n)

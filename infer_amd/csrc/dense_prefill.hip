@@ -317,12 +317,6 @@ __global__ void __launch_bounds__(64 * kWaves, 2) dense_prefill_kernel(DensePref
 // 407 / 288, chunks of 2048 with a bias 570 / 404; one sequence of 1800 in chunks of 512 with a bias, 16 heads 50 / 49.
 constexpr int kGroupB = 1024 + 32, kTileB = 2 * (kStep / 4) * kGroupB, kRing = 3;      // bytes: four rows, keys and values of a step
 
-// A value that the compiler takes for a new one: what is computed from it is not kept in registers over the whole loop.
-__device__ __forceinline__ int renewed(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
-
 template <int MAPS, bool BIASED>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(3, 3))) dense_prefill_ring_kernel(DensePrefillArgs a) {
     constexpr int KS = 4 / MAPS, VT = 8;

@@ -42,6 +42,12 @@ __device__ __forceinline__ void load_elems(const __bf16* p, float (&x)[N]) {
         for (int i = 0; i < N; ++i) x[i] = (float)p[i];
     }
 }
+// A value that the compiler takes for a new one: what is computed from it is not kept in registers over a whole loop.
+__device__ __forceinline__ int renewed(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 // Whether inputs of a norm behind a recurrence have left the caches by the time it reads them, so that the streaming hint costs nothing: from `line` MB on, which
 // depends on what else the kernels in front of it write.  A call without / with the hint, us: constant decay of 32 heads, 16 MB 44.0 / 44.6, 30 60.9 / 60.8, 34 66.5 /
 // 65.9, 40 74.5 / 73.1, 200 266 / 262; state space of 32 heads, one portion, 16 MB 58.1 / 59.1, 34 83.5 / 86.1, 38 91.1 / 91.3, 40 95.3 / 93.2; of 64, eight of

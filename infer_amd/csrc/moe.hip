@@ -724,26 +724,10 @@ __device__ __forceinline__ void moe_row_product(const GemmArgs<__bf16>& a, int e
 // The same, RT tiles of W and up to 16 MT rows, steps shared; k: a multiple of 64
 template <bool GATED, int RT, int MT>
 __device__ __forceinline__ void moe_shared_product(const GemmArgs<__bf16>& a, int expert, int first, int rows, int c0, unsigned char* lds) {
-    using Stream = SharedStream<RT, MT>;
-    constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR;
-    static_assert(WK == 1 || 4096 * TW * MT <= Stream::kRing, "the sums fit the ring");
-    const int n = threadIdx.x & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave % WR;
-    Stream stream(a.k, (int)blockIdx.x >> 3, wave, lds, [&](int i) { return moe_weight_row<GATED>(a, expert, c0, i); }, [&](int i) { return moe_input_row(a, first, rows, i); });
-    f32x4_t acc[TW][MT];
-#pragma unroll
-    for (int r = 0; r < TW; ++r)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream.product(wave, lds, acc);
-    auto finish = [&](int r, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0 + (GATED ? 8 : 16) * (wr * TW + r), sum); };
-    if constexpr (WK == 1) {
-#pragma unroll
-        for (int r = 0; r < TW; ++r)
-#pragma unroll
-            for (int t = 0; t < MT; ++t) finish(r, t, acc[r][t]);
-    } else {
-        stream_reduce<TW, MT, WK>(acc, wave / WR, lds + wr * (1024 * WK * TW * MT), finish);
-    }
+    const int n = threadIdx.x & 15;
+    shared_product<RT, MT>(a.k, (int)blockIdx.x >> 3, lds, [&](int i) { return moe_weight_row<GATED>(a, expert, c0, i); },
+                           [&](int i) { return moe_input_row(a, first, rows, i); },
+                           [&](int r, int t, f32x4_t sum) { moe_finish<GATED>(a, first, rows, 16 * t + n, c0 + (GATED ? 8 : 16) * r, sum); });
 }
 template <bool GATED, bool SHARED>
 __global__ void __launch_bounds__(64 * kRowWaves) moe_row_kernel(GemmArgs<__bf16> a) {

@@ -8,15 +8,14 @@
 // 256 compute units streaming; this kernel cuts K as well, so that every unit reads its share of
 // the weights exactly once, and pays for it with float32 partial sums that a second kernel adds.
 //
-// * The weights stream through LDS (weight_stream.h): skinny_stream_kernel, whose wavefronts split K among themselves, for the smallest batches, and
+// * The weights stream through LDS (weight_stream.h): skinny_stream_kernel, whose wavefronts split K among themselves, past up to 8 rows of the batch, up to 32
+//   with at most 5120 weight rows and K < 8192, and 17 to 64 with 8193 to 12288 weight rows (16 also past many with a short K); otherwise
 //   skinny_shared_kernel, whose wavefronts share every step of K and with it the batch.  Up to 64 rows K is cut over workgroups only where there are few of
 //   them.
 // * SK == 1: the accumulators are rounded to bf16 and stored.  SK > 1: float32 partial sums
 //   [SK][M][N] go to the workspace and `skinny_gemm_reduce_kernel` adds them and rounds once.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-
-#include <type_traits>
 
 #include "../../include/infer_kv.h"
 #include "decode_few.h"
@@ -25,7 +24,6 @@
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -126,15 +124,11 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
 // The same, the steps of k shared by the wavefronts (SharedStream)
 template <int RT, int MT, bool GATED>
 __global__ void __launch_bounds__(256) skinny_shared_kernel(GemmArgs a) {
-    using Stream = SharedStream<RT, MT>;
-    constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR;
-    static_assert(WK == 1 || 4096 * TW * MT <= Stream::kRing, "the sums fit the ring");
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[Stream::kRing];
-    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int half = a.n / 2, split = blockIdx.y, wr = wave % WR;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[SharedStream<RT, MT>::kRing];
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, half = a.n / 2, split = blockIdx.y;
     const Share<GATED, 16 * RT, 3, 2> share(a);
     const int64_t k_lo = (int64_t)split * a.chunks * kKC;
-    Stream stream(a.chunks * kKC, share.turn, wave, lds,
+    shared_product<RT, MT>(a.chunks * kKC, share.turn, lds,
         [&](int i) {
             int row = share.n0 + stream_row() + 8 * (GATED ? i / 2 : i);
             row = (row < share.end ? row : share.end - 1) + (GATED && (i & 1) ? half : 0);
@@ -143,22 +137,8 @@ __global__ void __launch_bounds__(256) skinny_shared_kernel(GemmArgs a) {
         [&](int i) {
             const int row = stream_row() + 8 * i;
             return (const __bf16*)a.x + (int64_t)(row < a.m ? row : a.m - 1) * a.x_stride0 + k_lo;
-        });
-    f32x4_t acc[TW][MT];
-#pragma unroll
-    for (int r = 0; r < TW; ++r)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    stream.product(wave, lds, acc);
-    auto finish = [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, share.end, split, share.n0, wr * TW + r, 16 * t + n, g, sum); };
-    if constexpr (WK == 1) {
-#pragma unroll
-        for (int r = 0; r < TW; ++r)
-#pragma unroll
-            for (int t = 0; t < MT; ++t) finish(r, t, acc[r][t]);
-    } else {
-        stream_reduce<TW, MT, WK>(acc, wave / WR, lds + wr * (1024 * WK * TW * MT), finish);
-    }
+        },
+        [&](int r, int t, f32x4_t sum) { finish_tile<GATED>(a, share.end, split, share.n0, r, 16 * t + n, g, sum); });
 }
 
 // What stands in front of a product of few rows: y = norm(x + residual) w^T, where x may still be the pieces of a split product.
@@ -377,14 +357,15 @@ __global__ void __launch_bounds__(256) skinny_gemm_reduce_kernel(ReduceArgs a) {
     *reinterpret_cast<u32x4*>(a.y + (int64_t)row * a.y_stride0 + 8 * c) = r.u;
 }
 
-// Weight rows of a workgroup.  At most 8 of the batch, and up to 16 past few rows: 16, wavefronts that split k (skinny_stream_kernel), which are as good
+// Weight rows of a workgroup.  At most 8 of the batch, and up to 32 past few rows: 16, wavefronts that split k (skinny_stream_kernel), which are as good
 // as any (32 past many with a short k: n = 151936 48 us with k = 1024, 54 with 16 rows).  More of the batch: the activations, which every workgroup reads
 // whole, want many rows, and the chip wants a workgroup for every compute unit: wavefronts that share the steps of k (skinny_shared_kernel), 16 times
 // shared_tiles rows.  Us, wavefronts that split k (before they began in different places) / this:
 //   64 of the batch   24576 x 4096 gate and up 42.8 / 33.7   151936 x 4096 240 / 202   151936 x 1024 66 / 59   32000 x 4096 56 / 41   49152 x 2048 50 / 33
 //   32                24576 x 4096 34 / 31   151936 x 4096 213 / 192   16384 x 2048 17 / 12   8192 x 4096 16.1 / 12.8
 //   16                24576 x 4096 34 / 31   151936 x 4096 209 / 184   16384 x 2048 17 / 11.5   4: 30.8 / 30.7, 187 / 181 (these now 175), 14.9 / 11.9 (12.6)
-// Three tiles of rows are none of its shapes: 12288 x 4096 with 64 of the batch 21.2 / 22.6.  Few weight rows and a long k: 16 rows give every compute unit
+// Three tiles of rows are none of its shapes, and 48 rows fill the chip from 8193 to 12288 of them: there 17 to 64 split k (12288 x 4096 with 64 of the batch
+// 21.2 / 22.6).  Few weight rows and a long k: 16 rows give every compute unit
 // a workgroup that reads the batch once per 16 rows; 64 rows, cut over k, read it a quarter as often.  Unreduced sums, 16 / 64 rows (split k): n = 4096,
 // k = 12288 9 of the batch 18.5 / 17.1, 16 20.2 / 17.3, 32 25.9 / 19.0 (now 17.3); with a shorter k the launch that adds the sums up for those who want
 // them costs more than that (n = 4096, k = 4096, 16: 8.4 / 10.4 reduced).  More than 4096 weight rows and a very long k: tiles of 64 rows leave
@@ -465,7 +446,7 @@ void launch_stream(GemmArgs a, int splits, hipStream_t st) {
 #define GO(RT, MT, NW, D) do { if (turned) TURNED(RT, MT, NW, D, 3); else TURNED(RT, MT, NW, D, 0); } while (0)
     if (turned && a.m <= kFewRows && rows == 16 && a.n >= kFewMany && a.n < kMany) TURNED(1, 1, 4, 4, 4);      // in twos, as 32 rows with a norm in front
     else if (a.m <= 16 && rows == 16) GO(1, 1, 4, 4);
-    else if (a.m <= 16 && a.n >= kMany && a.k <= 2048) GO(2, 1, 4, 3);
+    else if (a.m <= 16 && a.n >= kMany && a.k <= 2048) TURNED(2, 1, 4, 3, 0);
     else if (a.m <= 32 && rows == 16) GO(1, 2, 4, 3);
     else if (a.m <= 32 && rows == 48) GO(3, 2, 4, 2);
     else if (a.m <= 64 && rows == 48) GO(3, 4, 4, 2);

@@ -220,12 +220,6 @@ __device__ __forceinline__ bool swapped(int q) { return q & 8; }
 template <int HP>
 __device__ __forceinline__ int mixed_place(int q, int slot, int g) { return (q * HP + (slot ^ (q & (HP - 1)))) * 64 + 16 * (g ^ ((q >> 2) & 3)); }
 
-// A value that the compiler takes for a new one: what is computed from it is not kept in registers over the whole loop.
-__device__ __forceinline__ int renewed(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
-
 // SHARE: the heads of a wavefront have one key/value head.
 template <int KS, int VT, int UH, int QT, bool SHARE>
 __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) talk_mix_kernel(TalkPrefillArgs a) {

@@ -255,3 +255,29 @@ struct SharedStream {
         }
     }
 };
+
+// The product of RT tiles of weight rows and up to 16 MT rows of the batch by a workgroup: f(r, t, sum) gets tile r of the weights, t of the batch in the layout of
+// stream_product, by some wavefront.  lds: SharedStream<RT, MT>::kRing bytes
+template <int RT, int MT, class Weights, class Batch, class F>
+__device__ __forceinline__ void shared_product(int k, int turn, unsigned char* lds, Weights weights, Batch batch, F f) {
+    using Stream = SharedStream<RT, MT>;
+    constexpr int TW = Stream::kTiles, WR = Stream::WR, WK = 4 / WR;
+    static_assert(WK == 1 || 4096 * TW * MT <= Stream::kRing, "the sums fit the ring");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave % WR;
+    Stream stream(k, turn, wave, lds, weights, batch);
+    f32x4_t acc[TW][MT];
+#pragma unroll
+    for (int r = 0; r < TW; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[r][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    stream.product(wave, lds, acc);
+    auto finish = [&](int r, int t, f32x4_t sum) { f(wr * TW + r, t, sum); };
+    if constexpr (WK == 1) {
+#pragma unroll
+        for (int r = 0; r < TW; ++r)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) finish(r, t, acc[r][t]);
+    } else {
+        stream_reduce<TW, MT, WK>(acc, wave / WR, lds + wr * (1024 * WK * TW * MT), finish);
+    }
+}
