@@ -37,24 +37,30 @@ struct GemmArgs {
     float* partial;              // [SK][M][N] when SK > 1
     int m, n, k;
     int chunks;                  // K chunks per split
-    int each;                    // workgroups of either half of the weight rows where the halves are dealt out apart (Share), otherwise 0
 };
+static_assert(sizeof(GemmArgs) == 64, "a line: arguments in another one cost 0.2 us of 5");
 
 // The weight rows n0 .. end - 1 of which a workgroup takes its ROWS (GATED: ROWS / 2 gate rows, and the up rows of the same places), and where it begins its
 // walk over k (stream_start): 2^TURN workgroups at one place, 0 everybody at the front.  Gate rows and up rows are halves of one matrix, and a product of both
-// has to add up as the two by themselves do.  So without a gate a workgroup that is not cut over k lies in one half, and there 2^HALF_TURN of them begin at the
-// place of the twice as many that have the same rows with a gate.  Us, two workgroups of other halves side by side / the halves one behind the other: 6144 x
-// 4096, 48 of the batch 17.0 / 16.8, 151936 x 4096, 4 183.8 / 179.9.
-template <bool GATED, int ROWS, int TURN, int HALF_TURN = TURN>
+// has to add up as the two by themselves do.  So without a gate a workgroup that is not cut over k lies in one half (APART), and there 2^HALF_TURN of them begin
+// at the place of the twice as many that have the same rows with a gate.  Us, two workgroups of other halves side by side / the halves one behind the other:
+// 6144 x 4096, 48 of the batch 17.0 / 16.8, 151936 x 4096, 4 183.8 / 179.9.  APART is no argument: working it out in kernels of 5 us costs 0.1.
+template <bool GATED, int ROWS, int TURN, bool APART, int HALF_TURN = TURN>
 struct Share {
+    static_assert(!(GATED && APART) && (TURN > 0 || !APART), "halves of which somebody else has the other, and walks that begin somewhere");
     int n0, end, turn;
     __device__ __forceinline__ explicit Share(const GemmArgs& a) {
         const int b = blockIdx.x, half = a.n / 2;
-        const bool apart = !GATED && TURN > 0 && a.each > 0, second = apart && b >= a.each;
-        const int at = second ? b - a.each : b;
-        n0 = at * (GATED ? ROWS / 2 : ROWS) + (second ? half : 0);
-        end = GATED || (apart && !second) ? half : a.n;
-        turn = TURN == 0 ? 0 : GATED ? b >> (HALF_TURN + 1) : apart ? at >> HALF_TURN : b >> TURN;
+        if constexpr (APART) {
+            const int each = (half + ROWS - 1) / ROWS, at = b >= each ? b - each : b;
+            n0 = at * ROWS + (b >= each ? half : 0);
+            end = b >= each ? a.n : half;
+            turn = at >> HALF_TURN;
+        } else {
+            n0 = b * (GATED ? ROWS / 2 : ROWS);
+            end = GATED ? half : a.n;
+            turn = TURN == 0 ? 0 : b >> (GATED ? HALF_TURN + 1 : TURN);
+        }
     }
 };
 
@@ -91,13 +97,13 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& a, int end, int spli
 // 16 RT rows of weights past up to 16 MT rows of the batch, NW wavefronts with D steps each in LDS.  GATED: the weights are gate rows and as
 // many up rows, a.n / 2 each; a tile is eight gate rows and the eight up rows of the same places, and y = silu(gate) * up with the
 // roundings of storing both and reading them again.
-template <int RT, int MT, int NW, int D, bool GATED, int TURN>
+template <int RT, int MT, int NW, int D, bool GATED, int TURN, bool APART>
 __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
     constexpr int kRing = D * stream_stage_bytes(RT, MT), kLds = NW * (kRing > 1024 * RT * MT ? kRing : 1024 * RT * MT);
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int half = a.n / 2, split = blockIdx.y;
-    const Share<GATED, 16 * RT, TURN> share(a);
+    const Share<GATED, 16 * RT, TURN, APART> share(a);
     const int64_t k_lo = (int64_t)split * a.chunks * kKC;
     const __bf16* w[2 * RT];
     const __bf16* x[2 * MT];
@@ -122,11 +128,11 @@ __global__ void __launch_bounds__(64 * NW) skinny_stream_kernel(GemmArgs a) {
 }
 
 // The same, the steps of k shared by the wavefronts (SharedStream)
-template <int RT, int MT, bool GATED>
+template <int RT, int MT, bool GATED, bool APART>
 __global__ void __launch_bounds__(256) skinny_shared_kernel(GemmArgs a) {
     __shared__ __attribute__((aligned(1024))) unsigned char lds[SharedStream<RT, MT>::kRing];
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, half = a.n / 2, split = blockIdx.y;
-    const Share<GATED, 16 * RT, 3, 2> share(a);
+    const Share<GATED, 16 * RT, 3, APART, 2> share(a);
     const int64_t k_lo = (int64_t)split * a.chunks * kKC;
     shared_product<RT, MT>(a.chunks * kKC, share.turn, lds,
         [&](int i) {
@@ -162,14 +168,14 @@ constexpr int kFewPad = 64;                                         // bytes beh
 // What bounds it is what all workgroups read in front, rows times their bytes.  Norm and product, us, two launches / one, for 1, 2, 4 rows:
 // 4096 x 1024 behind four pieces 6.2 / 4.2, 6.4 / 4.3, 6.4 / 6.8; 6144 x 1024 gated 7.6 / 5.7, 7.6 / 6.0, 7.7 / 8.0; 6144 x 4096 14.1 / 12.6,
 // 13.5 / 13.3, 13.7 / 22.4; 24576 x 4096 gated 35.5 / 33.7, 33.8 / 42.4.  So one row up to 4096 elements, two of half as many.
-template <int RT, int NP, bool GATED, int TURN>
+template <int RT, int NP, bool GATED, int TURN, bool APART>
 __global__ void __launch_bounds__(256) norm_product_kernel(GemmArgs a, NormSource f) {
     constexpr int NW = 4, D = 4, kRing = D * stream_stage_bytes(RT, 0);
     static_assert(NW * kRing >= NW * RT * 1024, "sums of the wavefronts");
     extern __shared__ __attribute__((aligned(1024))) unsigned char few_lds[];      // rings, then rows of x, then sums of squares
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int half = a.n / 2;
-    const Share<GATED, 16 * RT, TURN> share(a);
+    const Share<GATED, 16 * RT, TURN, APART> share(a);
     const int row_bytes = 2 * a.k + kFewPad;
     unsigned char* xs = few_lds + NW * kRing;
     float* squares = reinterpret_cast<float*>(xs + a.m * row_bytes);               // [kFewRows][8]
@@ -419,30 +425,35 @@ int choose_splits(int64_t m, int64_t n, int64_t k) {
 
 // Whether wavefronts that split k begin at different places of it (stream_start).  With few workgroups or a short k, finding out where costs what it gives (a
 // step of 28 layers of a 0.6B model 729 / 733 us).  Products that norm their input have the bits of those that do not: the rule is one for both.  What the order of
-// a gate's sums in products without one costs (Share), steps of four layers of an 8B model, 1, 2, 4, 8, 16, 64 sequences, without / with it: 493 / 499, 508 /
-// 510, 516 / 519, 528 / 531, 577 / 575, 700 / 696.
+// a gate's sums in products without one costs (Share), steps of three layers of an 8B model, 1, 4, 24, 48, 64 sequences, without / with it: 417 / 422, 437 / 439,
+// 500 / 500, 548 / 546, 579 / 577; by themselves 121 products of other sizes took 1.004 times as long, the most 40832 x 4736 with 25 of the batch 58.2 / 61.4.
 bool begins_anywhere(int64_t n, int64_t k) { return k > 2048 && n > 8 * kUnits; }
-// The grid of a product whose workgroups have so many weight rows.  turned: their walks begin at different places; then the halves of the rows are dealt out
-// apart, where they can be gate and up (twice half the workgroups are no round of the compute units more).
-dim3 share_out(GemmArgs& a, bool gated, bool turned, int rows, int splits) {
-    a.each = turned && !gated && splits == 1 && a.n % 16 == 0 ? (a.n / 2 + rows - 1) / rows : 0;
-    return dim3((unsigned)(a.each ? 2 * a.each : (a.n + rows - 1) / rows), (unsigned)splits);
-}
+// Whether the halves of the weight rows are dealt out apart (Share): where walks begin at different places and the halves can be gate and up
+bool dealt_apart(const GemmArgs& a, bool turned, int splits) { return turned && splits == 1 && a.n % 16 == 0; }
+// Workgroups for so many weight rows each; twice those of a half are no round of the compute units more
+unsigned workgroups(const GemmArgs& a, bool apart, int rows) { return (unsigned)(apart ? 2 * ((a.n / 2 + rows - 1) / rows) : (a.n + rows - 1) / rows); }
 
 template <bool GATED, int MT>
-void launch_shared(GemmArgs a, int tiles, int splits, hipStream_t st) {
-    const dim3 grid = share_out(a, GATED, SharedStream<2, MT>::turned(a.chunks * kKC), 16 * tiles, splits);
-#define GO(RT) case RT: hipLaunchKernelGGL((skinny_shared_kernel<RT, MT, GATED>), grid, dim3(256), 0, st, a); return
+void launch_shared(const GemmArgs& a, int tiles, int splits, hipStream_t st) {
+    const bool apart = !GATED && dealt_apart(a, SharedStream<2, MT>::turned(a.chunks * kKC), splits);
+    const dim3 grid(workgroups(a, apart, 16 * tiles), (unsigned)splits);
+#define GO(RT) case RT: \
+        if (apart) hipLaunchKernelGGL((skinny_shared_kernel<RT, MT, GATED, !GATED>), grid, dim3(256), 0, st, a); \
+        else hipLaunchKernelGGL((skinny_shared_kernel<RT, MT, GATED, false>), grid, dim3(256), 0, st, a); \
+        return
     switch (tiles) { GO(2); GO(4); GO(6); GO(8); GO(10); GO(12); GO(14); GO(16); GO(20); }
 #undef GO
 }
 
 template <bool GATED>
-void launch_stream(GemmArgs a, int splits, hipStream_t st) {
+void launch_stream(const GemmArgs& a, int splits, hipStream_t st) {
     const int rows = rows_per_workgroup(a.m, a.n, a.k);
-    const bool turned = begins_anywhere(a.n, a.chunks * kKC);
-    const dim3 grid = share_out(a, GATED, turned && a.m <= 64, rows, splits);
-#define TURNED(RT, MT, NW, D, TURN) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED, TURN>), grid, dim3(64 * NW), 0, st, a)
+    const bool turned = begins_anywhere(a.n, a.chunks * kKC), apart = !GATED && a.m <= 64 && dealt_apart(a, turned, splits);
+    const dim3 grid(workgroups(a, apart, rows), (unsigned)splits);
+#define TURNED(RT, MT, NW, D, TURN) do { \
+        if (apart) hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED, TURN, !GATED && (TURN > 0)>), grid, dim3(64 * NW), 0, st, a); \
+        else hipLaunchKernelGGL((skinny_stream_kernel<RT, MT, NW, D, GATED, TURN, false>), grid, dim3(64 * NW), 0, st, a); \
+    } while (0)
 #define GO(RT, MT, NW, D) do { if (turned) TURNED(RT, MT, NW, D, 3); else TURNED(RT, MT, NW, D, 0); } while (0)
     if (turned && a.m <= kFewRows && rows == 16 && a.n >= kFewMany && a.n < kMany) TURNED(1, 1, 4, 4, 4);      // in twos, as 32 rows with a norm in front
     else if (a.m <= 16 && rows == 16) GO(1, 1, 4, 4);
@@ -461,8 +472,8 @@ void launch_stream(GemmArgs a, int splits, hipStream_t st) {
         // Rows of the batch in operand registers while weights came straight from memory into theirs / these, 128 of the batch, unreduced, us: 4096 x 12288
         // 29.7 / 25.3, 5120 x 25600 89 / 78, 4096 x 4096 15.1 / 13.2, 1024 x 3072 10.5 / 7.8 (with eight tiles 10.0); 72: 4096 x 4096 13.0 / 11.1
         if (grid.x * grid.y <= kUnits / 2)
-            hipLaunchKernelGGL((skinny_shared_kernel<4, 8, false>), dim3((unsigned)((a.n + 63) / 64), (unsigned)splits), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((skinny_shared_kernel<8, 8, false>), grid, dim3(256), 0, st, a);
+            hipLaunchKernelGGL((skinny_shared_kernel<4, 8, false, false>), dim3((unsigned)((a.n + 63) / 64), (unsigned)splits), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((skinny_shared_kernel<8, 8, false, false>), grid, dim3(256), 0, st, a);
     }
 #undef TURNED
 #undef GO
@@ -571,19 +582,20 @@ extern "C" int infer_skinny_gate_silu_bf16(const void* x, int64_t x_stride0, con
 
 namespace {
 template <bool GATED>
-int launch_norm_product(GemmArgs a, const NormSource& f, hipStream_t st) {
+int launch_norm_product(const GemmArgs& a, const NormSource& f, hipStream_t st) {
     const int pieces = a.m * ((a.k + kNormGroup - 1) / kNormGroup), rows = a.n >= kFewMany ? 32 : 16;
     const size_t lds = 4 * 4 * stream_stage_bytes(rows / 16, 0) + (size_t)a.m * (2 * a.k + kFewPad) + kFewRows * 8 * sizeof(float);
-    const bool turned = begins_anywhere(a.n, a.k);
-    const dim3 grid = share_out(a, GATED, turned, rows, 1);
-#define GO(RT, NP, TURN) do { \
-        if (lds > 60 * 1024) { \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&norm_product_kernel<RT, NP, GATED, TURN>), \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-            if (e != hipSuccess) return (int)e; \
-        } \
-        hipLaunchKernelGGL((norm_product_kernel<RT, NP, GATED, TURN>), grid, dim3(256), lds, st, a, f); \
-    } while (0)
+    const bool turned = begins_anywhere(a.n, a.k), apart = !GATED && dealt_apart(a, turned, 1);
+    const dim3 grid(workgroups(a, apart, rows));
+    auto launch = [&](auto kernel) -> int {
+        if (lds > 60 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return (int)e;
+        }
+        hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, a, f);
+        return (int)hipGetLastError();
+    };
+#define GO(RT, NP, TURN) return apart ? launch(&norm_product_kernel<RT, NP, GATED, TURN, !GATED && (TURN > 0)>) : launch(&norm_product_kernel<RT, NP, GATED, TURN, false>)
     // four pieces: one row of at most 2048, or two of 1024
     if (rows == 16) {
         if (pieces <= 4) GO(1, 1, 0);
@@ -596,7 +608,6 @@ int launch_norm_product(GemmArgs a, const NormSource& f, hipStream_t st) {
         else GO(2, 2, 0);
     }
 #undef GO
-    return (int)hipGetLastError();
 }
 }  // namespace
 
