@@ -182,7 +182,7 @@ __device__ __forceinline__ u32x2_t silu8(u32x2_t x) {            // of half as m
 // each, and with two chunks in LDS one barrier a chunk instead of three.
 // PARTS = 2: 64 columns, and a wavefront has half of the state rows of its 16.  The second half adds up and writes the results.  That is twice as many
 // workgroups, two to a compute unit, so that lengths even out, and shorter chunks (1.9 us by itself, 2.4 with all rows), though q and k are brought
-// twice: 3 portions of 3292 tokens of 32 heads 295 -> 243 us, 6 of 900 to 3700 313 -> 269.  128 registers are all there are: with addresses kept over the loop
+// twice: 3 portions of 3292 tokens of 32 heads 295 -> 243 us, 6 of 900 to 3700 313 -> 264.  128 registers are all there are: with addresses kept over the loop
 // it spilt eight, whose reads wait for the next chunk's requests as well (325).
 __host__ __device__ constexpr int chunk_bufs(int waves) { return waves == 8 ? 2 : 1; }      // chunks in LDS
 
@@ -1012,7 +1012,7 @@ extern "C" int64_t infer_decay_workspace_floats(int elem, int64_t heads, int64_t
                                                 int64_t max_span) {
     int64_t pad[2];
     if (infer_decay_layout(dim, vdim, pad) || heads < 1 || num_spans < 1 || max_span < 1 || !chunks_fit(elem, dim, vdim, rot_dims)) return 0;
-    int64_t n = 1;                                             // for both ways to walk: how many tokens there are is not known here
+    int64_t n = 1;                                             // for all ways to walk: how many tokens there are is not known here
     for (const Walk walk : {kFour, kEight, kHalves}) {
         const int64_t len = segment_len(walk, heads, pad[0], pad[1], num_spans, max_span);
         n = std::max(n, (max_span + len - 1) / len);
