@@ -50,8 +50,8 @@ __device__ __forceinline__ int renewed(int x) {
 
 // Whether inputs of a norm behind a recurrence have left the caches by the time it reads them, so that the streaming hint costs nothing: from `line` MB on, which
 // depends on what else the kernels in front of it write.  A call without / with the hint, us: constant decay of 32 heads, 16 MB 44.0 / 44.6, 30 60.9 / 60.8, 34 66.5 /
-// 65.9, 40 74.5 / 73.1, 200 266 / 262; state space of 32 heads, one portion, 16 MB 58.1 / 59.1, 34 83.5 / 86.1, 38 91.1 / 91.3, 40 95.3 / 93.2; of 64, eight of
-// them, 34 56.7 / 56.7, 40 63.5 / 61.0, 260 304 / 299.
+// 65.9, 40 74.5 / 73.1, 200 266 / 262; state space of 32 heads, one portion, 16 MB 58.1 / 59.1, 34 83.5 / 86.1, 38 91.1 / 91.3, 40 95.3 / 93.2; of 64,
+// one portion, 34 80.1 / 81.6, 38 83.9 / 85.3, 40 87.5 / 86.7, eight of them 34 56.0 / 57.0, 36 58.1 / 57.4, 260 304 / 299, nineteen 36 73.3 / 71.6.
 inline bool beyond_caches(int64_t bytes, int line) { return bytes > ((int64_t)line << 20); }
 
 // load_elems, ONCE: with the streaming hint, of what nobody reads again.  p: then aligned to the N elements, at most 16 bytes.

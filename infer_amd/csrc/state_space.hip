@@ -763,7 +763,7 @@ extern "C" int infer_state_space(int elem, const void* proj, int64_t proj_stride
         const bool vec = size % 8 == 0 && inner % 8 == 0 && proj_stride % 8 == 0 && z_off % 8 == 0 && out_stride % 8 == 0 &&
                          ptr_aligned(proj, 16) && ptr_aligned(y, 16) && ptr_aligned(out, 16) && ptr_aligned(norm, 16);
         const dim3 grid((unsigned)n, (unsigned)norm_parts), block(kThreads);
-        if (vec && size <= 8 * kKeep * kThreads && beyond_caches(2 * n * inner * (int64_t)sizeof(T), 39)) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, true>), grid, block, 0, st, b);
+        if (vec && size <= 8 * kKeep * kThreads && beyond_caches(2 * n * inner * (int64_t)sizeof(T), inner > 2048 ? 35 : 38)) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, true>), grid, block, 0, st, b);
         else if (vec) hipLaunchKernelGGL((ssm_norm_kernel<T, 8, false>), grid, block, 0, st, b);
         else hipLaunchKernelGGL((ssm_norm_kernel<T, 1, false>), grid, block, 0, st, b);
         return (int)hipGetLastError();

@@ -415,7 +415,7 @@ def test_state_space_norm_of_more_rows_than_caches_hold(gpu, parts):
     x = m.inputs(4)
     rows = [(i, 0, x[i:i + 1]) for i in range(4)]
     few, many = m.run(rows), m.run(rows + [(-1, 0, x[:1])] * 636)
-    assert 2 * 640 * m.s.inner * 2 > 39 << 20
+    assert 2 * 640 * m.s.inner * 2 > 38 << 20
     for i in range(4):
         close(torch.tensor(few[i]), m.want(x[i:i + 1])[0], 2e-2)
         assert (few[i] == many[i]).all()
