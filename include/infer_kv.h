@@ -664,7 +664,8 @@ int infer_decay_attention(int elem, const void* proj, int64_t proj_stride, int64
  *
  * infer_delta_step: one token per row; rows with a negative slot are padding (zeros come out).
  * infer_delta_chunks: prompt portions, rows row0 .. row0 + rows - 1.  portions[.][4] = first chunk, chunks, slot,
- * first position; chunks[.][6] = first row, tokens, first position, first position of the portion, slot, 0;
+ * first position; chunks[.][6] = first row, tokens, first position, first position of the portion, slot, 0 (a chunk without
+ * tokens reads no row and changes nothing);
  * ring_slot[row][2] (indexed by batch row) = the slot, and how many rows of the portion follow.
  * records: num_chunks * heads * [2] floats; o: (row0 + rows) * heads * [1] floats. */
 int infer_delta_layout(int64_t dim, int64_t vdim, int64_t* out4);
