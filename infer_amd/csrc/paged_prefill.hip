@@ -185,16 +185,18 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         return;
     }
     const int shift = sk - sq;
-    int my_q[kNQ], my_limit[kNQ];
+    // This lane's query of a tile, and the last key it sees: made anew where they are used, from a lane number that the compiler takes for
+    // another one, since registers for them would be spilled.
+    auto lane_now = [&] {
+        int x = lane;
+        __asm__ volatile("" : "+v"(x));
+        return x;
+    };
+    auto my_q = [&](int u) { return q0 + 16 * u + (lane_now() & 15); };
+    auto limit_of = [&](int q) { return a.causal ? (q + shift < sk - 1 ? q + shift : sk - 1) : sk - 1; };
+    int lim_lo[kNQ];                                       // of a tile's earliest query
 #pragma unroll
-    for (int u = 0; u < kNQ; ++u) {
-        my_q[u] = q0 + 16 * u + n;
-        my_limit[u] = a.causal ? (my_q[u] + shift < sk - 1 ? my_q[u] + shift : sk - 1) : sk - 1;
-    }
-    // lane 0 holds the earliest query of a tile, hence the smallest limit
-    int lim_lo[kNQ];
-#pragma unroll
-    for (int u = 0; u < kNQ; ++u) lim_lo[u] = __builtin_amdgcn_readfirstlane(my_limit[u]);
+    for (int u = 0; u < kNQ; ++u) lim_lo[u] = limit_of(q0 + 16 * u);
     // keys the workgroup walks (its last query block sees the most) and keys this wavefront needs
     auto key_end_of = [&](int first_q, int count) {
         const int last = first_q + count - 1 < sq - 1 ? first_q + count - 1 : sq - 1;
@@ -228,7 +230,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
     for (int u = 0; u < kNQ; ++u) {
         // lanes behind the last query of the sequence load its first query instead: straight-line loads,
         // finite values, and their columns of the result are never stored
-        const uint16_t* qp = a.q + (int64_t)(q_beg + (my_q[u] < sq ? my_q[u] : 0)) * a.q_stride0 + (int64_t)head * kD + 8 * g;
+        const uint16_t* qp = a.q + (int64_t)(q_beg + (my_q(u) < sq ? my_q(u) : 0)) * a.q_stride0 + (int64_t)head * kD + 8 * g;
 #pragma unroll
         for (int j = 0; j < 4; ++j) qreg[u][j] = as_bf16x8(load16(qp + 32 * j));
     }
@@ -367,75 +369,111 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         const int tok0 = s * kStep;
 
         if (QB == 1 || s < my_steps) {   // wavefronts whose queries end earlier skip the keys they cannot see
-        // ---- S^T = K Q^T for both query tiles
+        // ---- S^T = K Q^T for both query tiles.  The order of this step is written out: left alone, the compiler asks for each operand right in front of its
+        // product, and puts all products behind all exponents.  Keys are asked for two k-steps ahead and values before the maxima, one branch asks for
+        // both query tiles whether sums have to be rescaled, and the second tile's exponents run between the first one's products.  The call, us:
+        // 16 sequences of 64 .. 2048 tokens, 32 heads 271 -> 261; one of 4000, 16 heads 106 -> 94; one of 8000, 32 heads 468 -> 439.
+        // (Scores of the next step between the exponents of this one, which takes 210 registers, so two wavefronts a vector unit: 286.)
+        u32x4 kf[4][2];
+        auto keys = [&](int j) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) kf[j][t] = *reinterpret_cast<const u32x4*>(kb + k_addr + 4 * t * kGroupB + j * 256);
+        };
         f32x4 sc[kNQ][2];
 #pragma unroll
         for (int u = 0; u < kNQ; ++u)
 #pragma unroll
             for (int t = 0; t < 2; ++t) sc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        keys(0);
+        keys(1);
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const u32x4 kf = *reinterpret_cast<const u32x4*>(kb + k_addr + 4 * t * kGroupB + j * 256);
-#pragma unroll
-                for (int u = 0; u < kNQ; ++u)
-                    sc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf), qreg[u][j], sc[u][t], 0, 0, 0);
-            }
-
-        // ---- online softmax per query tile.  The running maximum is refreshed only when a row's
-        // maximum grows by more than kLazy (log2 units): until then the probabilities are taken
-        // relative to the stale maximum (at most 2^kLazy, harmless in float32 and bf16) and the
-        // accumulators need no rescaling; the final division by the row sum makes both forms equal.
-        bf16x8 pb[kNQ];
-#pragma unroll
-        for (int u = 0; u < kNQ; ++u) {
-            float sv[8];
+        for (int j = 0; j < 4; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) sv[4 * t + e] = sc[u][t][e];
+                for (int u = 0; u < kNQ; ++u) sc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[j][t]), qreg[u][j], sc[u][t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (j + 2 < 4) keys(j + 2);
+        }
+        bf16x8 vt[8];
+        auto values = [&](int t) {
+            const unsigned char* src = kb + v_addr + (t >> 1) * 256 + (t & 1) * 32;
+            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
+            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 4 * kGroupB));
+            vt[t] = __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        constexpr int kAhead = 3;                          // operands of V under way: registers
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t) values(t);
+        __builtin_amdgcn_sched_barrier(0);
+        float top[kNQ];
+#pragma unroll
+        for (int u = 0; u < kNQ; ++u) {
             if (!kInner && tok0 + kStep - 1 > lim_lo[u]) {      // wave-uniform: off the diagonal no lane masks anything
                 // key tok0 + 8 g + i is masked iff i > rel; written so that nothing but this one
                 // subtraction could be computed ahead of the branch
-                const int rel = my_limit[u] - tok0 - 8 * g;
+                const int rel = limit_of(my_q(u)) - tok0 - 8 * (lane_now() >> 4);
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    if (i > rel) sv[i] = -INFINITY;
+                    if (i > rel) sc[u][i >> 2][i & 3] = -INFINITY;
             }
-            float mx = sv[0];
+            top[u] = sc[u][0][0];
 #pragma unroll
-            for (int i = 1; i < 8; ++i) mx = fmaxf(mx, sv[i]);
-            mx = max_xor32(max_xor16(mx));
-            mx *= a.scale_log2;                                  // scale > 0: the maximum commutes with it
-            // m_neg is minus the running maximum, +inf before the first step: key 0 is visible to every
-            // query, so step 0 always "grows" (inf > kLazy) and sets it.  (A query without any visible key,
-            // sq > sk, keeps +inf; its row is written as zeros at the end.)
-            const bool grow = mx + m_neg[u] > kLazy;
-            if (__any(grow)) {
+            for (int i = 1; i < 8; ++i) top[u] = fmaxf(top[u], sc[u][i >> 2][i & 3]);
+        }
+
+        // ---- online softmax.  The running maximum is refreshed only when a row's
+        // maximum grows by more than kLazy (log2 units): until then the probabilities are taken
+        // relative to the stale maximum (at most 2^kLazy, harmless in float32 and bf16) and the
+        // accumulators need no rescaling; the final division by the row sum makes both forms equal.
+        // Whether some row's does is seen from the lanes' own maxima, without bringing a row's together.
+        // m_neg is minus the running maximum, +inf before the first step: key 0 is visible to every
+        // query, so step 0 always "grows" (inf > kLazy) and sets it.  (A query without any visible key,
+        // sq > sk, keeps +inf; its row is written as zeros at the end.)
+        bool grows = false;
+#pragma unroll
+        for (int u = 0; u < kNQ; ++u) grows |= __builtin_fmaf(top[u], a.scale_log2, m_neg[u]) > kLazy;
+        if (__any(grows)) {
+#pragma unroll
+            for (int u = 0; u < kNQ; ++u) {
+                const float mx = max_xor32(max_xor16(top[u])) * a.scale_log2;     // scale > 0: the maximum commutes with it
+                const bool grow = mx + m_neg[u] > kLazy;
                 const float alpha = grow ? __builtin_amdgcn_exp2f(-m_neg[u] - mx) : 1.f;
                 m_neg[u] = grow ? -mx : m_neg[u];
                 lacc[u] *= alpha;
 #pragma unroll
                 for (int t = 0; t < 8; ++t) acc[u][t] *= alpha;
             }
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                pb[u][i] = (__bf16)__builtin_amdgcn_exp2f(__builtin_fmaf(sv[i], a.scale_log2, m_neg[u]));
-            lacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[u], lacc[u], 0, 0, 0);
         }
-
-        // ---- O^T += V^T P^T, every V fragment used for both query tiles
+        // ---- O^T += V^T P^T, every V fragment used for both query tiles, of which the first one's products run under the exponents of the second
+        bf16x8 pb[kNQ];
+        auto powers = [&](int u) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pb[u][i] = (__bf16)__builtin_amdgcn_exp2f(__builtin_fmaf(sc[u][i >> 2][i & 3], a.scale_log2, m_neg[u]));
+        };
+        auto product = [&](int u, int t) { acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[t], pb[u], acc[u][t], 0, 0, 0); };
+        powers(0);
+        __builtin_amdgcn_sched_barrier(0);
+        lacc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[0], lacc[0], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t) product(0, t);
+        powers(1);
+#pragma unroll
+        for (int i = 0; i <= kAhead; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
-            const unsigned char* src = kb + v_addr + (t >> 1) * 256 + (t & 1) * 32;
-            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src));
-            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 4 * kGroupB));
-            const bf16x8 vt = __builtin_bit_cast(bf16x8, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-            for (int u = 0; u < kNQ; ++u)
-                acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, pb[u], acc[u][t], 0, 0, 0);
+            if (t >= kAhead) product(0, t);
+            product(1, t);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t + kAhead < 8) values(t + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        lacc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[1], lacc[1], 0, 0, 0);
         }
 
         // tile s + 1 must be in LDS for everybody: own loads first, then the barrier
@@ -479,10 +517,11 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int u = 0; u < kNQ; ++u) {
         const float l = lacc[u][0];
-        if (my_q[u] < sq) {
-            const bool none = my_limit[u] < 0;          // no key visible to this query (sq > sk): zeros, whatever the sums hold
+        const int qi = my_q(u);
+        if (qi < sq) {
+            const bool none = limit_of(qi) < 0;          // no key visible to this query (sq > sk): zeros, whatever the sums hold
             const float inv = l > 0.f ? 1.f / l : 0.f;
-            uint16_t* op = a.out + (int64_t)(q_beg + my_q[u]) * a.out_stride0 + (int64_t)head * kD + 4 * g;
+            uint16_t* op = a.out + (int64_t)(q_beg + qi) * a.out_stride0 + (int64_t)head * kD + 4 * g;
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
                 union { __bf16 hv[4]; u32x2 w; } r;
