@@ -16,6 +16,8 @@
 //                     sums talk_sum_kernel adds up.  Between the barriers that enclose the mixture a wavefront computes the scores
 //                     of the next step and the sums of this one, the two wavefronts of a vector unit in opposite order.
 // A lane's eight results of the first two products are those of eight consecutive keys (tile_row_token).
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "elem.h"
@@ -33,20 +35,101 @@ constexpr float kLow = -1e30f;            // a maximum before any key was seen; 
 constexpr float kLazy = 8.f;              // log2 units by which a sum's terms may exceed one before it is rescaled
 constexpr float kBound = 100.f;           // log2 units: powers of scores below it add up in a float as they are
 
+// The order in which workgroups take blocks of queries.  A block sees as many keys as its place in its sequence says, so some take a hundred times as long as
+// others, and a launch is done when its last workgroup is.  Sorted: units of `run` neighbouring blocks in falling order of the steps of their last one, over all
+// sequences, dealt to the dies in turn, so that a unit's blocks share what the L2 of their die holds.  Walks of more than `most` steps are cut into parts of one
+// length (at most `splits`), which are turns of their own.  Otherwise blocks by their place in their sequences.  The call, us, before (blocks by their place in
+// their sequences, walks whole, or all cut alike where blocks are few) / now: 8 sequences of 700 .. 2300 tokens 321 / 301, 6 of 1214 .. 2313 303 / 277, one of 6000 506 / 432,
+// one of 600 49 / 37, 32 of 100 .. 600 161 / 127, 4 of 500 .. 1500 behind 1500 cached 330 / 275, 64 of 61 .. 179 65 / 65.  Runs of 1, 2, 4, 8 blocks: 8 of 700 .. 2300 263, 261,
+// 265, 272 (the same inputs again and again).
+constexpr int kLanes = 64;
+constexpr int kMostKeys = 1 << 30;      // of a sequence, so that numbers of steps can be doubled
+struct Turns { int queries, run, most, splits; bool sorted; int units; };      // queries of a block; run, queries: powers of two; units of the longest sequence
+struct Turn { int seq, q_beg, sq, shift, block, part, parts; };        // shift: keys in front of the sequence's first query
+__device__ __forceinline__ int steps_of(int last_q, int shift) { return last_q + shift < 0 ? 1 : (last_q + shift) / kStep + 1; }
+__device__ __forceinline__ int parts_of(const Turns& t, int steps) {
+    const int n = (steps + t.most - 1) / t.most;
+    return n < t.splits ? n : t.splits;
+}
+// parts of the walks of block `block` of a sequence
+__device__ __forceinline__ int parts_of_block(const Turns& t, int sq, int shift, int block) {
+    if (t.splits == 1) return 1;
+    const int blocks = (sq + t.queries - 1) >> __builtin_ctz(t.queries), in_front = (blocks - 1 - block) & ~(t.run - 1), end = (blocks - in_front) * t.queries;
+    return parts_of(t, steps_of((end < sq ? end : sq) - 1, shift));
+}
+__device__ __forceinline__ int wave_sum(int x) {
+    auto ror = [](int v, auto C) { return __builtin_amdgcn_update_dpp(0, v, decltype(C)::value, 0xf, 0xf, false); };
+    x += ror(x, std::integral_constant<int, 0x128>{});
+    x += ror(x, std::integral_constant<int, 0x124>{});
+    x += ror(x, std::integral_constant<int, 0x122>{});
+    x += ror(x, std::integral_constant<int, 0x121>{});
+    return __builtin_amdgcn_readlane(x, 0) + __builtin_amdgcn_readlane(x, 16) + __builtin_amdgcn_readlane(x, 32) + __builtin_amdgcn_readlane(x, 48);
+}
+// Without an order: turn `rest` of sequence s
+__device__ __forceinline__ Turn plain_turn(const Turns& t, int s, int rest, const int32_t* cu_q, const int32_t* cu_k) {
+    const int part = t.splits == 1 ? 0 : rest / t.units, unit = rest - part * t.units;
+    const int q_beg = cu_q[s], sq = cu_q[s + 1] - q_beg, shift = cu_k[s + 1] - cu_k[s] - sq, block = ((sq + t.queries - 1) >> __builtin_ctz(t.queries)) - 1 - unit;
+    const int parts = block < 0 ? 1 : parts_of_block(t, sq, shift, block);
+    return {s, q_beg, sq, shift, part < parts ? block : -1, part, parts};
+}
+// Block `inside` of the unit whose turn is number `turn`; block < 0: there is none.  Up to 64 sequences, a lane for each.
+__device__ __forceinline__ Turn turn_of(const Turns& t, int turn, int inside, int nseq, const int32_t* cu_q, const int32_t* cu_k) {
+    const int lane = threadIdx.x & 63;
+    int q_beg = 0, sq = 0, shift = 0;
+    if (lane < nseq) {
+        q_beg = cu_q[lane];
+        sq = cu_q[lane + 1] - q_beg;
+        shift = cu_k[lane + 1] - cu_k[lane] - sq;
+        if (sq > kMostKeys || sq + shift > kMostKeys) sq = 0;
+    }
+    const int q_bits = __builtin_ctz(t.queries), run_bits = __builtin_ctz(t.run), blocks = (sq + t.queries - 1) >> q_bits;
+    // units of this lane's sequence with more than x steps
+    auto longer = [&](int x) {
+        const int need = x > 0 ? x * kStep + 1 - shift : 0, from = need > t.queries ? (need + t.queries - 1) >> q_bits : 1;      // blocks that end behind that
+        if (sq <= 0 || (x > 0 && sq - 1 + shift < x * kStep)) return 0;
+        return 1 + (blocks > from ? (blocks - from) >> run_bits : 0);
+    };
+    auto turns_before = [&](int x) {                             // of units with more than x steps, a turn for every part
+        int n = 0;
+        for (int m = 0; m < t.splits; ++m) n += longer(x > m * t.most ? x : m * t.most);
+        return wave_sum(n);
+    };
+    int lo = 0, hi = 16;                                         // the unit has more than lo steps, and at most hi
+    if (turns_before(0) <= turn) return {0, 0, 0, 0, -1, 0, 1};
+    while (turns_before(hi) > turn) {                            // it ends: nobody has more than kMostKeys / kStep
+        lo = hi;
+        hi = 4 * hi < kMostKeys / kStep + 1 ? 4 * hi : kMostKeys / kStep + 1;
+    }
+    while (hi - lo > 1) {
+        const int x = (lo + hi) / 2;
+        if (turns_before(x) > turn) lo = x;
+        else hi = x;
+    }
+    const int parts = parts_of(t, hi), rest = turn - turns_before(hi), mine = longer(hi), with = longer(lo) - mine;
+    const int at = rest / parts;                                 // among the units of hi steps, of which a sequence has three at most
+    const uint64_t one = __ballot(with & 1), two = __ballot(with & 2), below = (1ull << lane) - 1;
+    const int in_front = __popcll(one & below) + 2 * __popcll(two & below);
+    const int s = __builtin_ctzll(__ballot(in_front <= at && at < in_front + with));
+    const int unit = __builtin_amdgcn_readlane(mine + at - in_front, s);
+    auto of = [&](int x) { return __builtin_amdgcn_readlane(x, s); };
+    return {s, of(q_beg), of(sq), of(shift), of(blocks) - 1 - unit * t.run - inside, rest - at * parts, parts};
+}
+
 struct TalkPrefillArgs {
     const __bf16* q; int64_t q_stride;    // [token][head * dim]
     const __bf16* keys; const __bf16* values;                 // tile_pages.h
     int key_pad, vdim_pad;
     const int32_t* bt; int64_t bt_stride; int table_cols, block_size, num_blocks;
     const int32_t* seqs; const int32_t* cu_q; const int32_t* cu_k;
-    int heads, kv_heads, dim, vdim, nseq, qblocks, run;
+    int heads, kv_heads, dim, vdim, nseq;
     float scale_log2;
     const __bf16* talk;                   // [heads][heads]
     float out_scale;
     __bf16* out; int64_t out_stride;      // [token][head * vdim]
-    float* lse; int64_t tokens;           // [heads][tokens]
-    int splits, split_steps;              // steps per split
-    float* part;                          // [splits][tokens][heads * vdim], if splits > 1
+    float* lse; int64_t tokens;           // [heads][tokens], or [sums.splits][heads][tokens] sums of powers of the BOUNDED form
+    Turns turns, sums;                    // of the mixture and of the sums of exponentials
+    bool bounded;
+    float* part;                          // [turns.splits][tokens][heads * vdim], if turns.splits > 1
 };
 
 // The tiles of 32 keys of a sequence, one behind the other; a tile lies in one block, whose id is looked up one block ahead.
@@ -79,33 +162,15 @@ struct PageWalk {
     }
 };
 
-// How query blocks of pairs, late ones, which see the most keys, first, go to the dies; workgroups go to them round-robin.
-constexpr int kShares = 0;       // a die works on its own share of the pairs
-constexpr int kSpread = -1;      // all pairs of a row of blocks one behind the other
-// run > 0: `run` neighbouring blocks of a pair go to one die, the runs of all pairs in turn; the pairs turn from row to row.
-// False: no such block.
-__device__ __forceinline__ bool place_of_block(unsigned id, int pairs, int qblocks, int run, int& pair, int& qblk) {
-    const unsigned die = id & 7u, i = id >> 3, all = (unsigned)pairs;
-    if (run == kSpread) {
-        pair = (int)(id % all);
-        qblk = qblocks - 1 - (int)(id / all);
-    } else if (run == kShares) {
-        const unsigned per_die = (all + 7u) / 8u;
-        pair = (int)(die * per_die + i % per_die);
-        qblk = qblocks - 1 - (int)(i / per_die);
-    } else {
-        const unsigned unit = i / (unsigned)run * 8u + die, row = unit / all;
-        pair = (int)((unit + row) % all);
-        qblk = qblocks - 1 - (int)(row * (unsigned)run + i % (unsigned)run);
-    }
-    pair = __builtin_amdgcn_readfirstlane(pair);
-    qblk = __builtin_amdgcn_readfirstlane(qblk);
-    return pair < pairs && qblk >= 0;
-}
-
 // An operand at an address that all lanes share plus a byte offset of each
 __device__ __forceinline__ bf16x8_t load_operand(const __bf16* base, unsigned lane_bytes) {
     return *reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const char*>(base) + lane_bytes);
+}
+
+// Entries at .. at + 7 of a row of `size` (a multiple of eight), zero behind it; without a branch, behind which the compiler waits for the load
+__device__ __forceinline__ bf16x8_t query_operand(const __bf16* row, int at, int size) {
+    const u32x4_t x = *reinterpret_cast<const u32x4_t*>(row + (at < size ? at : 0)), zero = {0, 0, 0, 0};
+    return __builtin_bit_cast(bf16x8_t, at < size ? x : zero);
 }
 
 // BOUNDED: all scores are below kBound, so that their powers need no maximum.
@@ -113,13 +178,27 @@ template <int KS, int U, bool BOUNDED>
 __global__ void __launch_bounds__(64 * kLseWaves, 2) talk_lse_kernel(TalkPrefillArgs a) {
     constexpr int kLseQ = 16 * U;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, n = lane & 15;
-    int pair, qblk;
-    if (!place_of_block(blockIdx.x, a.nseq * a.heads, a.qblocks, a.run, pair, qblk)) return;
-    const int b = pair / a.heads, h = pair - b * a.heads;
-    const int q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, sk = a.cu_k[b + 1] - a.cu_k[b], shift = sk - sq;
+    int h = blockIdx.x % a.heads;
+    Turn turn;
+    if (a.sums.sorted) turn = turn_of(a.sums, blockIdx.x / a.heads, 0, a.nseq, a.cu_q, a.cu_k);
+    else {                                            // a share of the heads of all sequences for every die
+        const int pairs = a.nseq * a.heads, share = (pairs + 7) / 8, i = blockIdx.x >> 3, rest = i / share, pair = (int)(blockIdx.x & 7u) * share + i - rest * share;
+        if (pair >= pairs) return;
+        h = pair % a.heads;
+        turn = plain_turn(a.sums, pair / a.heads, rest, a.cu_q, a.cu_k);
+    }
+    const auto [b, q_beg, sq, shift, qblk, part, parts] = turn;
+    if (qblk < 0) return;
     const int q0 = (qblk * kLseWaves + wave) * kLseQ;
     if (q0 >= sq) return;
-    const int last_q = q0 + kLseQ < sq ? q0 + kLseQ - 1 : sq - 1, steps = (last_q + shift) / kStep + 1;
+    // sums of powers add up, whoever takes them; a maximum is of the whole walk (parts is 1)
+    const int last_q = q0 + kLseQ < sq ? q0 + kLseQ - 1 : sq - 1, all_steps = steps_of(last_q, shift), each = (all_steps + parts - 1) / parts;
+    const int s0 = part * each, steps = s0 + each < all_steps ? s0 + each : all_steps;
+    float* const lse = a.lse + ((int64_t)part * a.heads + h) * a.tokens + q_beg + q0;
+    if (s0 >= steps) {
+        for (int i = lane; i <= last_q - q0; i += 64) lse[i] = 0.f;
+        return;
+    }
     bf16x8_t q[U][KS];
     float m[U], l[U];
     int limit[U];
@@ -129,19 +208,16 @@ __global__ void __launch_bounds__(64 * kLseWaves, 2) talk_lse_kernel(TalkPrefill
         limit[u] = qi + shift;
         m[u] = BOUNDED ? 0.f : kLow;
         l[u] = 0.f;
-        const __bf16* qp = a.q + (int64_t)(q_beg + qi) * a.q_stride + (int64_t)h * a.dim + 8 * g;
+        const __bf16* qp = a.q + (int64_t)(q_beg + qi) * a.q_stride + (int64_t)h * a.dim;
 #pragma unroll
-        for (int j = 0; j < KS; ++j) {
-            q[u][j] = bf16x8_t{};
-            if (32 * j + 8 * g < a.dim) q[u][j] = *reinterpret_cast<const bf16x8_t*>(qp + 32 * j);
-        }
+        for (int j = 0; j < KS; ++j) q[u][j] = query_operand(qp, 32 * j + 8 * g, a.dim);
     }
     int k_step[KS];                                   // k-steps behind the size repeat the first one, which meets zeros
 #pragma unroll
     for (int j = 0; j < KS; ++j) k_step[j] = tile_key_entry(0, 32 * j < a.key_pad ? 32 * j : 0);
     const int64_t head_at = (int64_t)(h / (a.heads / a.kv_heads)) * a.block_size * a.key_pad;
     const unsigned k_lane = 2u * (unsigned)tile_key_entry(tile_row_token(n, 0), 8 * g);
-    PageWalk walk(a, b);
+    PageWalk walk(a, b, s0);
     bf16x8_t kf[2][KS];
     auto fetch = [&]() {
         const __bf16* src = a.keys + walk.next(a) * kStep * a.key_pad + head_at;
@@ -151,7 +227,7 @@ __global__ void __launch_bounds__(64 * kLseWaves, 2) talk_lse_kernel(TalkPrefill
             for (int j = 0; j < KS; ++j) kf[x][j] = load_operand(src + k_step[j] + tile_key_entry(tile_row_token(0, x), 0), k_lane);
     };
     fetch();
-    for (int s = 0; s < steps; ++s) {
+    for (int s = s0; s < steps; ++s) {
         f32x4_t sc[U][2];
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -196,6 +272,12 @@ __global__ void __launch_bounds__(64 * kLseWaves, 2) talk_lse_kernel(TalkPrefill
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+        if constexpr (BOUNDED) {
+#pragma unroll
+            for (int x = 16; x <= 32; x *= 2) l[u] += __shfl_xor(l[u], x, 64);
+            if (g == 0 && q0 + 16 * u + n < sq) lse[16 * u + n] = l[u];
+            continue;
+        }
 #pragma unroll
         for (int x = 16; x <= 32; x *= 2) {
             const float m2 = __shfl_xor(m[u], x, 64), l2 = __shfl_xor(l[u], x, 64), top = fmaxf(m[u], m2);
@@ -204,7 +286,7 @@ __global__ void __launch_bounds__(64 * kLseWaves, 2) talk_lse_kernel(TalkPrefill
         }
         const float top = fmaxf(m[u], 0.f);
         if (g == 0 && q0 + 16 * u + n < sq)
-            a.lse[(int64_t)h * a.tokens + q_beg + q0 + 16 * u + n] = top + log2f(l[u] * exp2f(m[u] - top) + exp2f(-top));
+            lse[16 * u + n] = top + log2f(l[u] * exp2f(m[u] - top) + exp2f(-top));
     }
 }
 
@@ -232,15 +314,21 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
     unsigned char* pbuf = wbuf + Q * kStep * kRec;               // [Q][HP][32 keys] bf16
     bf16x8_t* talk = reinterpret_cast<bf16x8_t*>(pbuf + Q * HP * 2 * kStep);       // [2][KP][RT][64]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, n = lane & 15;
-    int b, qblk;
-    const int split = blockIdx.y;
-    if (!place_of_block(blockIdx.x, a.nseq, a.qblocks, a.run, b, qblk)) return;
-    const int q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, sk = a.cu_k[b + 1] - a.cu_k[b], shift = sk - sq;
+    Turn turn;
+    const int die = blockIdx.x & 7u, dealt = blockIdx.x >> 3;
+    if (a.turns.sorted) turn = turn_of(a.turns, dealt / a.turns.run * 8 + die, dealt % a.turns.run, a.nseq, a.cu_q, a.cu_k);
+    else {                                            // a share of the sequences for every die, if that comes out even
+        const int share = a.nseq % 8 == 0 ? a.nseq / 8 : a.nseq, i = a.nseq % 8 == 0 ? dealt : (int)blockIdx.x, rest = i / share, s = i - rest * share;
+        turn = plain_turn(a.turns, a.nseq % 8 == 0 ? die * share + s : s, rest, a.cu_q, a.cu_k);
+    }
+    const auto [b, q_beg, sq, shift, qblk, split, parts] = turn;
+    if (qblk < 0) return;
+    const int sk = sq + shift;
     const int q0 = qblk * Q;
-    if (q0 >= sq) return;
-    const int last_q = q0 + Q < sq ? q0 + Q - 1 : sq - 1, all_steps = (last_q + shift) / kStep + 1;
-    const int s0 = split * a.split_steps, steps = s0 + a.split_steps < all_steps ? s0 + a.split_steps : all_steps;
+    const int last_q = q0 + Q < sq ? q0 + Q - 1 : sq - 1, all_steps = steps_of(last_q, shift), each = (all_steps + parts - 1) / parts;
+    const int s0 = split * each, steps = s0 + each < all_steps ? s0 + each : all_steps;
     if (s0 >= steps) return;
+    const int sum_parts = a.bounded ? parts_of_block(a.sums, sq, shift, q0 >> __builtin_ctz(a.sums.queries)) : 0;
     const int group = a.heads / a.kv_heads;
 
     bf16x8_t q[UH][QT][KS];
@@ -259,12 +347,13 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
             const int qi = q0 + 16 * t + n < sq ? q0 + 16 * t + n : sq - 1;
             limit[t] = qi + shift;
             lse[u][t] = a.lse[(int64_t)h * a.tokens + q_beg + qi];
-            const __bf16* qp = a.q + (int64_t)(q_beg + qi) * a.q_stride + (int64_t)h * a.dim + 8 * g;
-#pragma unroll
-            for (int j = 0; j < KS; ++j) {
-                q[u][t][j] = bf16x8_t{};
-                if (32 * j + 8 * g < a.dim) q[u][t][j] = *reinterpret_cast<const bf16x8_t*>(qp + 32 * j);
+            if (sum_parts > 0) {
+                for (int i = 1; i < sum_parts; ++i) lse[u][t] += a.lse[((int64_t)i * a.heads + h) * a.tokens + q_beg + qi];
+                lse[u][t] = log2f(1.f + lse[u][t]);
             }
+            const __bf16* qp = a.q + (int64_t)(q_beg + qi) * a.q_stride + (int64_t)h * a.dim;
+#pragma unroll
+            for (int j = 0; j < KS; ++j) q[u][t][j] = query_operand(qp, 32 * j + 8 * g, a.dim);
         }
     }
     // T^T: entry i of lane (g, n) is column (head) 16 s + 4 g + i / 2 of row (head) 16 r + n, once for either piece; behind it the same
@@ -275,7 +364,9 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int from = 16 * s + 4 * (i % 64 / 16) + (i < KP * RT * 64 ? e : e ^ 4) / 2;
-            x[e] = from < HP && from < a.heads && to < a.heads ? a.talk[(int64_t)to * a.heads + from] : (__bf16)0.f;
+            const bool in = from < HP && from < a.heads && to < a.heads;
+            const __bf16 w = a.talk[in ? to * a.heads + from : 0];           // no branch around a load: behind each there would be a wait
+            x[e] = in ? w : (__bf16)0.f;
         }
         talk[i] = x;
     }
@@ -474,7 +565,7 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
 #pragma unroll
             for (int v = 0; v < VT; ++v) {
                 if (16 * v + 4 * g >= a.vdim) continue;
-                if (a.splits > 1) {
+                if (parts > 1) {
                     *reinterpret_cast<f32x4_t*>(part + 16 * v) = acc[u][t][v];
                     continue;
                 }
@@ -487,111 +578,130 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
     }
 }
 
-// Sums of the splits.  Workgroup: 1024 columns of a token.  queries: of a workgroup of talk_mix_kernel.
-__global__ void __launch_bounds__(256) talk_sum_kernel(TalkPrefillArgs a, int queries) {
-    const int64_t c = ((int64_t)blockIdx.y * 256 + threadIdx.x) * 4, cols = (int64_t)a.heads * a.vdim;
-    const int b = blockIdx.z, q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, sk = a.cu_k[b + 1] - a.cu_k[b], qi = blockIdx.x;
-    if (qi >= sq || c >= cols) return;
-    const int last = (qi / queries + 1) * queries, last_q = last < sq ? last - 1 : sq - 1, steps = (last_q + sk - sq) / kStep + 1;
-    const float* p = a.part + (q_beg + qi) * cols + c;
-    f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s * a.split_steps < steps; ++s) sum += *reinterpret_cast<const f32x4_t*>(p + s * a.tokens * cols);
-    bf16x4_t x;
+// Sums of the parts of walks that were cut.  Workgroup: a token.
+__global__ void __launch_bounds__(256) talk_sum_kernel(TalkPrefillArgs a) {
+    const int cols = a.heads * a.vdim, b = blockIdx.y, q_beg = a.cu_q[b], sq = a.cu_q[b + 1] - q_beg, shift = a.cu_k[b + 1] - a.cu_k[b] - sq, qi = blockIdx.x;
+    if (qi >= sq) return;
+    const int block = qi / a.turns.queries, parts = parts_of_block(a.turns, sq, shift, block);
+    if (parts < 2) return;
+    const int end = (block + 1) * a.turns.queries, steps = steps_of((end < sq ? end : sq) - 1, shift), each = (steps + parts - 1) / parts, there = (steps + each - 1) / each;
+    const float* from = a.part + (int64_t)(q_beg + qi) * cols;
+    __bf16* out = a.out + (int64_t)(q_beg + qi) * a.out_stride;
+    for (int i = 4 * threadIdx.x; i < cols; i += 1024) {
+        f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < there; ++s) sum += *reinterpret_cast<const f32x4_t*>(from + s * a.tokens * cols + i);
+        bf16x4_t x;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = (__bf16)(sum[e] * a.out_scale);
-    *reinterpret_cast<bf16x4_t*>(a.out + (int64_t)(q_beg + qi) * a.out_stride + c) = x;
+        for (int e = 0; e < 4; ++e) x[e] = (__bf16)(sum[e] * a.out_scale);
+        *reinterpret_cast<bf16x4_t*>(out + i) = x;
+    }
 }
 
-// workgroups of the mixture that are worth having: two for every compute unit, since some see more keys than others
-constexpr int64_t kWorkgroups = 512;
-// queries of a workgroup, in tiles of 16, and splits of the keys.  A split has at least eight steps.
-void plan(int64_t heads, int64_t num_seqs, int64_t max_seqlen_q, int64_t max_keys, int& tiles, int& splits, int& split_steps) {
-    auto groups = [&](int t) { return (max_seqlen_q + 16 * t - 1) / (16 * t) * num_seqs; };
-    const int most = heads <= 8 ? 4 : heads <= 16 ? 2 : 1, least = heads <= 8 ? 2 : 1;
-    tiles = groups(most) >= kWorkgroups ? most : least;
+constexpr int64_t kUnits = 256;
+// How long the mixture takes, in us as a model has it whose constants were fitted to its choices: `blocks` walks of all_steps steps together, the longest of
+// `longest`, walks longer than `part` steps cut.  As long as its longest part, as all work shared out over the compute units, or, where there are a few parts more than
+// units, as two of the short ones.  A workgroup takes `fixed` beside its steps (loads of the queries, the first step's way through LDS, stores), and more if it
+// leaves a part.  29 batches (1 sequence of 190 .. 6000 tokens, 64 of 61 .. 179, 4 of 500 .. 1500 behind 1500 cached ones ...), 18 cuts of each: what this chooses takes
+// 0.6 % longer than the best of them, 9 % at most.
+double mix_time(double blocks, double longest, double all_steps, int part, double fixed, double step) {
+    const bool cut = part < longest;
+    const float shape = 1.f / std::max((float)(longest * blocks / all_steps) - 1.f, 0.05f);
+    auto above = [&](double x) { return x >= longest ? 0. : 1. - (double)std::pow((float)(x / longest), shape); };     // share of the walks that are longer than x steps
+    const double left = cut ? 5. : 0.;
+    double pieces = blocks;
+    for (double x = part; x < longest; x += part) pieces += blocks * above(x);
+    const double all = (cut ? 1.39 : 1.53) / kUnits * (pieces * fixed + (pieces - blocks * (1. - above(part))) * left + all_steps * step);
+    double t = std::max(fixed + left + part * step, all);
+    if (pieces > kUnits && pieces < 2 * kUnits) {
+        const double low = blocks * (1. - above(0.5 * part)), paired = 2. * (pieces - kUnits);      // walks of up to half a part
+        const double mean = paired <= low ? 0.25 * part * paired / low : (0.25 * part * low + 0.75 * part * (paired - low)) / paired;
+        t = std::max(t, 2. * (fixed + left + mean * step));
+    }
+    return t + 0.09 * std::min(part * step, all) + (cut ? 4.7 : 0.);
+}
+struct Plan { Turns turns, sums; };
+Plan plan(int64_t heads, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q, int64_t max_keys, bool bounded) {
+    Plan p;
     const int64_t steps = (max_keys + kStep - 1) / kStep;
-    int64_t n = kWorkgroups / (groups(tiles) > 0 ? groups(tiles) : 1);
-    if (n > steps / 8) n = steps / 8;
-    if (n > 8) n = 8;
-    if (n < 1) n = 1;
-    split_steps = (int)((steps + n - 1) / n);
-    if (split_steps < 1) split_steps = 1;
-    splits = (int)((steps + split_steps - 1) / split_steps);
-    if (splits < 1) splits = 1;
+    // a token's sequence is about as long as the mean of the mean and the longest one, and it is in its middle
+    const double seen = ((double)(max_keys - max_seqlen_q) + 0.25 * ((double)tokens / num_seqs + (double)max_seqlen_q)) / kStep + 0.5;
+    const int wide = heads <= 8 ? 4 : heads <= 16 ? 2 : 1, narrow = heads <= 8 ? 2 : 1;
+    const bool orders = num_seqs <= kLanes && max_keys <= kMostKeys;
+    double best = 0.;
+    for (int tiles = wide; tiles >= narrow; tiles /= 2)
+        for (const double share : {1., 0.8, 0.65, 0.5, 0.4, 0.33, 0.25, 0.17, 0.125}) {
+            const int64_t most = std::min(std::max<int64_t>({4, (int64_t)(share * (double)steps), (steps + 7) / 8}), steps);
+            if (most < steps && !orders) break;
+            const double blocks = (double)tokens / (16 * tiles) + 0.5 * num_seqs;
+            const double t = mix_time(blocks, (double)steps, blocks * seen, (int)most, tiles == wide ? 18.8 : 6.65, tiles == wide ? 2.06 : 1.68);
+            if (best > 0. && t >= best) continue;
+            best = t;
+            p.turns = Turns{16 * tiles, 2, (int)most, (int)((steps + most - 1) / most), true, 0};
+        }
+    // few queries: more wavefronts with fewer of them each
+    p.sums = Turns{(max_seqlen_q + 63) / 64 * num_seqs * heads < 2048 ? 128 : 256, 1, (int)steps, 1, true, 0};
+    if (bounded && orders) {               // no walk longer than what a place for a wavefront has to do, eight of a unit
+        const int64_t n = std::max<int64_t>({8, (int64_t)((double)tokens / 64 * heads * seen / (8 * kUnits)) + 1, (steps + 7) / 8});
+        if (5 * n <= 4 * steps) {
+            p.sums.most = (int)n;
+            p.sums.splits = (int)((steps + n - 1) / n);
+        }
+    }
+    // Finding a turn takes 1 to 2 us, which is not worth it where walks are short or all run at once: 24 sequences of 151 .. 441 78 us against 74, 23 of 67 .. 80
+    // 28 against 25, but 32 of 100 .. 600 111 against 148.
+    auto arrange = [&](Turns& t, int64_t at_once) {
+        const int64_t blocks = (max_seqlen_q + t.queries - 1) / t.queries;
+        t.sorted = orders && steps > 16 && t.splits * blocks * num_seqs > at_once;
+        if (!t.sorted) t.run = 1;
+        t.units = (int)((blocks + t.run - 1) / t.run);
+    };
+    arrange(p.turns, kUnits);
+    arrange(p.sums, 2 * kUnits);
+    return p;
 }
-
-// Eight sequences, or sixteen: where each belongs to a die its keys are read once, but a die with the longest one works on when the others
-// are done.  Runs of blocks, unless the lengths are nearly equal or all blocks of the mixture run at once (mixture and sums of exponentials, us,
-// shares / runs: 8 sequences of 700 .. 2300 397 / 323, 16 of 100 .. 1500 324 / 227, 8 of 1500 252 / 260, single blocks there 318).  Two sequences
-// of a die even out between them, so that sixteen have to differ more (of 56 .. 922 165 / 122, of 990 .. 1292 272 / 289), and more of them do
-// without runs (24 of 151 .. 441 76 / 91, 48 of 61 .. 179 45 / 65, 64 of 161 .. 245 85 / 108).  Other numbers of sequences spread by themselves
-// (6 of 1214 .. 2313: 360 / 407).
-bool uneven_dies(const TalkPrefillArgs& a, int64_t max_seqlen_q) {
-    const int64_t longest = a.nseq * max_seqlen_q;     // tokens if all were as long
-    return (max_seqlen_q + 31) / 32 * a.nseq > 256 && ((a.nseq == 8 && 10 * a.tokens < 9 * longest) || (a.nseq == 16 && 4 * a.tokens < 3 * longest));
-}
-// a run, so that every die gets eight of them if there are as many
-int64_t run_of(int64_t pairs, int64_t qblocks, int64_t most) {
-    const int64_t run = pairs * qblocks / 64;
-    return run < 1 ? 1 : run < most ? run : most;
-}
-// workgroups, also of blocks that there are not
-int64_t run_grid(int64_t pairs, int64_t qblocks, int64_t run) {
-    if (run == kSpread) return pairs * qblocks;      // no more: with an odd number of them, splits of a block go to several dies
-    if (run == kShares) return (pairs + 7) / 8 * 8 * qblocks;
-    return (pairs * ((qblocks + run - 1) / run) + 7) / 8 * 8 * run;
+// Turns that there are at most
+int64_t most_turns(const Turns& t, int64_t num_seqs, int64_t tokens) {
+    if (!t.sorted) return (int64_t)t.splits * t.units * num_seqs;
+    return t.splits * (tokens / (t.queries * t.run) + num_seqs);
 }
 
 template <int KS, int U>
-int launch_lse_of(TalkPrefillArgs a, int64_t max_seqlen_q, bool bounded, hipStream_t st) {
-    const int64_t per = 16 * U * kLseWaves, qblocks = (max_seqlen_q + per - 1) / per, pairs = (int64_t)a.nseq * a.heads;
-    const int64_t run = uneven_dies(a, max_seqlen_q) ? run_of(pairs, qblocks, 2) : kShares;
-    const int64_t total = run_grid(pairs, qblocks, run);
+int launch_lse_of(const TalkPrefillArgs& a, int64_t turns, hipStream_t st) {
+    const int64_t total = a.sums.sorted ? turns * a.heads : (a.nseq * (int64_t)a.heads + 7) / 8 * 8 * a.sums.units * a.sums.splits;
     if (total > 0x7fffffff) return INFER_KV_EINVAL;
-    a.qblocks = (int)qblocks;
-    a.run = (int)run;
-    if (bounded) hipLaunchKernelGGL((talk_lse_kernel<KS, U, true>), dim3((unsigned)total), dim3(64 * kLseWaves), 0, st, a);
+    if (a.bounded) hipLaunchKernelGGL((talk_lse_kernel<KS, U, true>), dim3((unsigned)total), dim3(64 * kLseWaves), 0, st, a);
     else hipLaunchKernelGGL((talk_lse_kernel<KS, U, false>), dim3((unsigned)total), dim3(64 * kLseWaves), 0, st, a);
     return (int)hipGetLastError();
 }
 template <int KS>
-int launch_lse(const TalkPrefillArgs& a, int64_t max_seqlen_q, bool bounded, hipStream_t st) {
-    // few queries: more wavefronts with fewer of them each
-    if ((max_seqlen_q + 63) / 64 * a.nseq * a.heads < 2048) return launch_lse_of<KS, 2>(a, max_seqlen_q, bounded, st);
-    return launch_lse_of<KS, 4>(a, max_seqlen_q, bounded, st);
+int launch_lse(const TalkPrefillArgs& a, int64_t turns, hipStream_t st) {
+    return a.sums.queries == 32 * kLseWaves ? launch_lse_of<KS, 2>(a, turns, st) : launch_lse_of<KS, 4>(a, turns, st);
 }
 
 template <int KS, int VT, int UH, int QT, bool SHARE>
-int launch_mix(TalkPrefillArgs a, int64_t max_seqlen_q, hipStream_t st) {
-    const int64_t qblocks = (max_seqlen_q + 16 * QT - 1) / (16 * QT);
-    const int64_t run = uneven_dies(a, max_seqlen_q) ? run_of(a.nseq, qblocks, 8) : a.nseq % 8 == 0 ? kShares : kSpread;
-    const int64_t total = run_grid(a.nseq, qblocks, run);
+int launch_mix(const TalkPrefillArgs& a, int64_t turns, int64_t max_seqlen_q, hipStream_t st) {
+    const int64_t total = (turns + 7) / 8 * 8 * a.turns.run;
     if (total > 0x7fffffff) return INFER_KV_EINVAL;
-    a.run = (int)run;
-    a.qblocks = (int)qblocks;
     auto kernel = &talk_mix_kernel<KS, VT, UH, QT, SHARE>;
     constexpr size_t lds = (size_t)16 * QT * kStep * kMixWaves * UH * (4 + 2) + (UH == 4 ? 4 : 1) * 2048;
     static_assert(lds <= 160 * 1024, "LDS of a compute unit");
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)total, (unsigned)a.splits), dim3(64 * kMixWaves), lds, st, a);
-    if (a.splits > 1) {
-        const unsigned columns = (unsigned)(((int64_t)a.heads * a.vdim + 1023) / 1024);
-        hipLaunchKernelGGL(talk_sum_kernel, dim3((unsigned)max_seqlen_q, columns, (unsigned)a.nseq), dim3(256), 0, st, a, 16 * QT);
-    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(64 * kMixWaves), lds, st, a);
+    if (a.turns.splits > 1) hipLaunchKernelGGL(talk_sum_kernel, dim3((unsigned)max_seqlen_q, (unsigned)a.nseq), dim3(256), 0, st, a);
     return (int)hipGetLastError();
 }
 
 template <int KS, int VT>
-int launch(const TalkPrefillArgs& a, int64_t max_seqlen_q, bool bounded, int tiles, hipStream_t st) {
-    const int rc = launch_lse<KS>(a, max_seqlen_q, bounded, st);
+int launch(const TalkPrefillArgs& a, int64_t sum_turns, int64_t turns, int64_t max_seqlen_q, hipStream_t st) {
+    const int rc = launch_lse<KS>(a, sum_turns, st);
     if (rc) return rc;
-    const int group = a.heads / a.kv_heads;
-    if (a.heads <= 8) return tiles == 4 ? launch_mix<KS, VT, 1, 4, true>(a, max_seqlen_q, st) : launch_mix<KS, VT, 1, 2, true>(a, max_seqlen_q, st);
+    const int group = a.heads / a.kv_heads, tiles = a.turns.queries / 16;
+    if (a.heads <= 8) return tiles == 4 ? launch_mix<KS, VT, 1, 4, true>(a, turns, max_seqlen_q, st) : launch_mix<KS, VT, 1, 2, true>(a, turns, max_seqlen_q, st);
     if (a.heads <= 16 && group % 2 == 0)
-        return tiles == 2 ? launch_mix<KS, VT, 2, 2, true>(a, max_seqlen_q, st) : launch_mix<KS, VT, 2, 1, true>(a, max_seqlen_q, st);
-    if (a.heads <= 16) return tiles == 2 ? launch_mix<KS, VT, 2, 2, false>(a, max_seqlen_q, st) : launch_mix<KS, VT, 2, 1, false>(a, max_seqlen_q, st);
-    return group % 4 == 0 ? launch_mix<KS, VT, 4, 1, true>(a, max_seqlen_q, st) : launch_mix<KS, VT, 4, 1, false>(a, max_seqlen_q, st);
+        return tiles == 2 ? launch_mix<KS, VT, 2, 2, true>(a, turns, max_seqlen_q, st) : launch_mix<KS, VT, 2, 1, true>(a, turns, max_seqlen_q, st);
+    if (a.heads <= 16) return tiles == 2 ? launch_mix<KS, VT, 2, 2, false>(a, turns, max_seqlen_q, st) : launch_mix<KS, VT, 2, 1, false>(a, turns, max_seqlen_q, st);
+    return group % 4 == 0 ? launch_mix<KS, VT, 4, 1, true>(a, turns, max_seqlen_q, st) : launch_mix<KS, VT, 4, 1, false>(a, turns, max_seqlen_q, st);
 }
 
 }  // namespace
@@ -604,10 +714,9 @@ extern "C" int infer_talking_prefill_supported(int64_t heads, int64_t dim, int64
 extern "C" int64_t infer_talking_prefill_workspace_floats(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q,
                                                           int64_t max_keys) {
     if (heads < 1 || vdim < 1 || num_seqs < 1 || tokens < 1 || max_seqlen_q < 1 || max_keys < 1) return 0;
-    int tiles, splits, split_steps;
-    plan(heads, num_seqs, max_seqlen_q, max_keys, tiles, splits, split_steps);
-    const int64_t lse = (heads * tokens + 3) / 4 * 4;
-    return lse + (splits > 1 ? splits * tokens * heads * vdim : 0);
+    const Plan p = plan(heads, num_seqs, tokens, max_seqlen_q, max_keys, true);
+    const int64_t lse = (p.sums.splits * heads * tokens + 3) / 4 * 4;
+    return lse + (p.turns.splits > 1 ? p.turns.splits * tokens * heads * vdim : 0);
 }
 
 extern "C" int infer_talking_prefill(const void* q, int64_t q_stride, const void* keys, const void* values, int64_t key_pad,
@@ -632,14 +741,14 @@ extern "C" int infer_talking_prefill(const void* q, int64_t q_stride, const void
     if (!workspace || !ptr_aligned(workspace, 16) ||
         workspace_floats < infer_talking_prefill_workspace_floats(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys))
         return INFER_KV_EWORKSPACE;
-    int tiles, splits, split_steps;
-    plan(heads, num_seqs, max_seqlen_q, max_keys, tiles, splits, split_steps);
+    const bool bounded = max_score * kLog2e <= kBound;
+    const Plan p = plan(heads, num_seqs, tokens, max_seqlen_q, max_keys, bounded);
     const TalkPrefillArgs a{(const __bf16*)q, q_stride, (const __bf16*)keys, (const __bf16*)values, (int)key_pad, (int)vdim_pad, block_table,
                             bt_stride, (int)table_cols, (int)block_size, (int)num_blocks, seqs, cu_q, cu_k, (int)heads, (int)kv_heads, (int)dim,
-                            (int)vdim, (int)num_seqs, 0, 0, scale * kLog2e, (const __bf16*)talk, out_scale, (__bf16*)out, out_stride, workspace, tokens, splits,
-                            split_steps, workspace + (heads * tokens + 3) / 4 * 4};
+                            (int)vdim, (int)num_seqs, scale * kLog2e, (const __bf16*)talk, out_scale, (__bf16*)out, out_stride, workspace, tokens, p.turns,
+                            p.sums, bounded, workspace + (p.sums.splits * heads * tokens + 3) / 4 * 4};
     hipStream_t st = (hipStream_t)stream;
-    const bool bounded = max_score * kLog2e <= kBound;
-    if (dim <= 64) return vdim <= 64 ? launch<2, 4>(a, max_seqlen_q, bounded, tiles, st) : launch<2, 8>(a, max_seqlen_q, bounded, tiles, st);
-    return vdim <= 64 ? launch<4, 4>(a, max_seqlen_q, bounded, tiles, st) : launch<4, 8>(a, max_seqlen_q, bounded, tiles, st);
+    const int64_t sum_turns = most_turns(p.sums, num_seqs, tokens), turns = most_turns(p.turns, num_seqs, tokens);
+    if (dim <= 64) return vdim <= 64 ? launch<2, 4>(a, sum_turns, turns, max_seqlen_q, st) : launch<2, 8>(a, sum_turns, turns, max_seqlen_q, st);
+    return vdim <= 64 ? launch<4, 4>(a, sum_turns, turns, max_seqlen_q, st) : launch<4, 8>(a, sum_turns, turns, max_seqlen_q, st);
 }
