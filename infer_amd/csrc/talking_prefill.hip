@@ -39,8 +39,9 @@ constexpr float kBound = 100.f;           // log2 units: powers of scores below 
 // others, and a launch is done when its last workgroup is.  Sorted: units of `run` neighbouring blocks in falling order of the steps of their last one, over all
 // sequences, dealt to the dies in turn, so that a unit's blocks share what the L2 of their die holds.  Walks of more than `most` steps are cut into parts of one
 // length (at most `splits`), which are turns of their own.  Otherwise blocks by their place in their sequences.  The call, us, before (blocks by their place in
-// their sequences, walks whole, or all cut alike where blocks are few) / now: 8 sequences of 700 .. 2300 tokens 321 / 301, 6 of 1214 .. 2313 303 / 277, one of 6000 506 / 432,
-// one of 600 49 / 37, 32 of 100 .. 600 161 / 127, 4 of 500 .. 1500 behind 1500 cached 330 / 275, 64 of 61 .. 179 65 / 65.  Runs of 1, 2, 4, 8 blocks: 8 of 700 .. 2300 263, 261,
+// their sequences, walks whole, or all cut alike where blocks are few) / now: 8 sequences of 700 .. 2300 tokens 320 / 297, 6 of 1214 .. 2313 307 / 272, one of 6000 534 / 431,
+// one of 600 49 / 35, 16 of 100 .. 1500 226 / 210, 4 of 500 .. 1500 behind 1500 cached 330 / 270, 64 of 61 .. 179 65 / 58 (5 .. 7 of each by the order of loads and
+// the rows at the end of talk_mix_kernel).  Runs of 1, 2, 4, 8 blocks: 8 of 700 .. 2300 263, 261,
 // 265, 272 (the same inputs again and again).
 constexpr int kLanes = 64;
 constexpr int kMostKeys = 1 << 30;      // of a sequence, so that numbers of steps can be doubled
@@ -331,6 +332,8 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
     const int sum_parts = a.bounded ? parts_of_block(a.sums, sq, shift, q0 >> __builtin_ctz(a.sums.queries)) : 0;
     const int group = a.heads / a.kv_heads;
 
+    PageWalk walk(a, b, s0);
+    int64_t tile = walk.next(a), tile1 = s0 + 1 < steps ? walk.next(a) : tile, tile2 = s0 + 2 < steps ? walk.next(a) : tile1;
     bf16x8_t q[UH][QT][KS];
     float lse[UH][QT];
     int limit[QT];
@@ -347,15 +350,33 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
             const int qi = q0 + 16 * t + n < sq ? q0 + 16 * t + n : sq - 1;
             limit[t] = qi + shift;
             lse[u][t] = a.lse[(int64_t)h * a.tokens + q_beg + qi];
-            if (sum_parts > 0) {
-                for (int i = 1; i < sum_parts; ++i) lse[u][t] += a.lse[((int64_t)i * a.heads + h) * a.tokens + q_beg + qi];
-                lse[u][t] = log2f(1.f + lse[u][t]);
-            }
             const __bf16* qp = a.q + (int64_t)(q_beg + qi) * a.q_stride + (int64_t)h * a.dim;
 #pragma unroll
             for (int j = 0; j < KS; ++j) q[u][t][j] = query_operand(qp, 32 * j + 8 * g, a.dim);
         }
     }
+    if (a.bounded) {
+        for (int i = 1; i < sum_parts; ++i)
+#pragma unroll
+            for (int u = 0; u < UH; ++u)
+#pragma unroll
+                for (int t = 0; t < QT; ++t) {
+                    const int h = wave * UH + u < a.heads ? wave * UH + u : a.heads - 1;
+                    lse[u][t] += a.lse[((int64_t)i * a.heads + h) * a.tokens + q_beg + limit[t] - shift];
+                }
+#pragma unroll
+        for (int u = 0; u < UH; ++u)
+#pragma unroll
+            for (int t = 0; t < QT; ++t) lse[u][t] = log2f(1.f + lse[u][t]);
+    }
+    const unsigned k_lane = 2u * (unsigned)tile_key_entry(tile_row_token(n, 0), 8 * g), v_lane = 2u * (unsigned)tile_value_entry(8 * g, n);
+    bf16x8_t kf[KS];
+    // half x of the keys of head uk; k-steps behind the size repeat the first one, which meets zeros in q
+    auto fetch_k = [&](int64_t tile, int uk, int x) __attribute__((always_inline)) {
+        const __bf16* src = a.keys + tile * kStep * a.key_pad + k_head[uk] + tile_key_entry(tile_row_token(0, x), 0);
+#pragma unroll
+        for (int j = 0; j < KS; ++j) kf[j] = load_operand(src + tile_key_entry(0, 32 * j < a.key_pad ? 32 * j : 0), k_lane);
+    };
     // T^T: entry i of lane (g, n) is column (head) 16 s + 4 g + i / 2 of row (head) 16 r + n, once for either piece; behind it the same
     // for records whose halves are swapped
     for (int i = tid; i < 2 * KP * RT * 64; i += 64 * kMixWaves) {
@@ -379,15 +400,6 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
 #pragma unroll
             for (int v = 0; v < VT; ++v) acc[u][t][v] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    PageWalk walk(a, b, s0);
-    const unsigned k_lane = 2u * (unsigned)tile_key_entry(tile_row_token(n, 0), 8 * g), v_lane = 2u * (unsigned)tile_value_entry(8 * g, n);
-    bf16x8_t kf[KS];
-    // half x of the keys of head uk; k-steps behind the size repeat the first one, which meets zeros in q
-    auto fetch_k = [&](int64_t tile, int uk, int x) __attribute__((always_inline)) {
-        const __bf16* src = a.keys + tile * kStep * a.key_pad + k_head[uk] + tile_key_entry(tile_row_token(0, x), 0);
-#pragma unroll
-        for (int j = 0; j < KS; ++j) kf[j] = load_operand(src + tile_key_entry(0, 32 * j < a.key_pad ? 32 * j : 0), k_lane);
-    };
     constexpr int kRing = UH == 2 ? 3 : 4;                                     // value operands under way
     bf16x8_t vf[kRing];
     // operand i of the step: tile i % VT of head i / VT; tiles behind the size repeat the first one and are not stored
@@ -515,8 +527,6 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
 #pragma unroll
         for (int i = 0; i < kRing; ++i) fetch_v(tile, i);
     };
-    // tiles of this step, the next one and the one behind it; behind the last one it is repeated
-    int64_t tile = walk.next(a), tile1 = s0 + 1 < steps ? walk.next(a) : tile, tile2 = s0 + 2 < steps ? walk.next(a) : tile1;
     __syncthreads();                                             // T
     // A wavefront's part of the walk; both forms meet the same barriers.  Loops of their own, since accumulators that several branches
     // change would be copied where these meet.
@@ -552,6 +562,13 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
     };
     if (wave < kMixWaves / 2) run(std::true_type{});
     else run(std::false_type{});
+    // Results as they lie are 8 bytes of every 32 of a token's row; they go through LDS, which nobody needs any more, so that a head's
+    // row is written in one piece.  With the pages looked up before the queries are asked for, so that their latency runs under these
+    // loads, the call takes, us, before / now: 64 sequences of 61 .. 179 tokens 66.1 / 59.7, 23 of 67 .. 80 25.9 / 23.7, 8 of 700 .. 2300 311 / 302,
+    // 6 of 1214 .. 2313 281 / 275, one of 600 36.4 / 36.3.
+    constexpr int kOutRow = 32 * VT + 16, kRowLanes = 4 * VT;    // bytes; lanes that write a row
+    static_assert(kMixWaves * 16 * kOutRow <= Q * kStep * kRec + Q * HP * 2 * kStep, "room in LDS");
+    unsigned char* obuf = lds + wave * 16 * kOutRow;
 #pragma unroll
     for (int u = 0; u < UH; ++u) {
         const int h = wave * UH + u;
@@ -559,20 +576,28 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
 #pragma unroll
         for (int t = 0; t < QT; ++t) {
             const int qi = q0 + 16 * t + n;
-            if (qi >= sq) continue;
-            __bf16* o = a.out + (int64_t)(q_beg + qi) * a.out_stride + (int64_t)h * a.vdim + 4 * g;
-            float* part = a.part + (((int64_t)split * a.tokens + q_beg + qi) * a.heads + h) * a.vdim + 4 * g;
+            if (parts > 1) {
+                if (qi >= sq) continue;
+                float* part = a.part + (((int64_t)split * a.tokens + q_beg + qi) * a.heads + h) * a.vdim + 4 * g;
+#pragma unroll
+                for (int v = 0; v < VT; ++v)
+                    if (16 * v + 4 * g < a.vdim) *reinterpret_cast<f32x4_t*>(part + 16 * v) = acc[u][t][v];
+                continue;
+            }
 #pragma unroll
             for (int v = 0; v < VT; ++v) {
-                if (16 * v + 4 * g >= a.vdim) continue;
-                if (parts > 1) {
-                    *reinterpret_cast<f32x4_t*>(part + 16 * v) = acc[u][t][v];
-                    continue;
-                }
                 bf16x4_t x;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) x[e] = (__bf16)(acc[u][t][v][e] * a.out_scale);
-                *reinterpret_cast<bf16x4_t*>(o + 16 * v) = x;
+                *reinterpret_cast<bf16x4_t*>(obuf + n * kOutRow + 32 * v + 8 * g) = x;
+            }
+            const int row = lane / kRowLanes, col = 4 * (lane % kRowLanes);
+#pragma unroll
+            for (int i = 0; i < 16 * kRowLanes / 64; ++i) {
+                const int r = row + 64 / kRowLanes * i;
+                const bf16x4_t x = *reinterpret_cast<const bf16x4_t*>(obuf + r * kOutRow + 2 * col);
+                if (q0 + 16 * t + r < sq && col < a.vdim)
+                    *reinterpret_cast<bf16x4_t*>(a.out + (int64_t)(q_beg + q0 + 16 * t + r) * a.out_stride + (int64_t)h * a.vdim + col) = x;
             }
         }
     }
