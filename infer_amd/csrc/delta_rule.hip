@@ -1211,97 +1211,111 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
     put(0);
     fetch(1);
     __syncthreads();
-    for (int c = 0; c < p.chunks; ++c) {
-        const WideBuffer buf{lds + (c & 1) * wide_buffer_units(DT), KS};
-        f32x4_t u = v;
-        if (c + 1 < p.chunks) {
-            v = vn;
-            put((c + 1) & 1);
+    // Loops of their own for wavefronts with columns and for others: where they met, the state would be copied.  Of the two wavefronts of a
+    // vector unit the older one is served first, and the other one is alone for the rest of a step, when nothing covers its latencies (4500 and 6900
+    // clocks): so the younger ones go first until U, the older ones behind it.  8 portions of 500 .. 2600 tokens, 32 heads, the call 737 -> 718 us, 16 of
+    // 800 645 -> 637, 16 heads with 11 of 300 .. 1500 378 -> 365.  Half of the wavefronts with the next record behind the products instead: 734; the products
+    // alone or the next record alone ahead: 733, 739.
+    auto walk = [&](auto owner) __attribute__((always_inline)) {
+        constexpr bool LIVE = decltype(owner)::value;
+        for (int c = 0; c < p.chunks; ++c) {
+            const WideBuffer buf{lds + (c & 1) * wide_buffer_units(DT), KS};
+            if (vt >= 4) __builtin_amdgcn_s_setprio(1);
+            f32x4_t u = v;
+            if (c + 1 < p.chunks) {
+                v = vn;
+                put((c + 1) & 1);
+            }
+            if (c > 0) finish((c - 1) & 1);
+            fetch(c + 2);
+            // rows behind a chunk's last repeat it; an empty chunk has none, and row 0 exists
+            gate = *reinterpret_cast<const t4_t*>(gates + (int64_t)(count > 0 ? row + (out_row < count ? out_row : count - 1) : 0) * a.gate_stride);
+            __builtin_amdgcn_sched_barrier(0);             // requests stay here, a step ahead of their use
+            if constexpr (LIVE) {
+                // The vector unit cuts the next part of the state while the matrix pipe works on one.  The pipe rounds its sums towards one
+                // side, so nothing stays in its accumulators from chunk to chunk: the state takes a chunk's sum by the vector unit.  3200
+                // tokens without decay, all of one sign: error of the state 5.7e-7 of its norm, 6.6e-6 with the state in the pipe's
+                // accumulators and pieces cut off instead of rounded, 1.4e-6 in delta_scan_kernel; 794 -> 807 us for the call with the batch above.
+                f32x4_t x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1, x3 = x1, o1 = x1, o2 = x1, o3 = x1;
+                uint32_t pc[KS][3][4];
+                u32x4_t w[KS][3], qv[KS][3];
+                auto part = [&](int kk) {
+                    const float f[8] = {s[2 * kk][0], s[2 * kk][1], s[2 * kk][2], s[2 * kk][3], s[2 * kk + 1][0], s[2 * kk + 1][1], s[2 * kk + 1][2], s[2 * kk + 1][3]};
+    #pragma unroll
+                    for (int i = 0; i < 3; ++i) { w[kk][i] = buf.wq(0, kk, i)[lane]; qv[kk][i] = buf.wq(1, kk, i)[lane]; }
+                    split3<8>(f, pc[kk]);
+                };
+                part(0);
+    #pragma unroll
+                for (int kk = 0; kk < KS; ++kk) {
+                    const bf16x8_t sh = frag(pc[kk][0]), sm = frag(pc[kk][1]), sl = frag(pc[kk][2]);
+                    if (kk + 1 < KS) part(kk + 1);
+                    x1 = mma(w[kk][0], sh, x1);
+                    o1 = mma(qv[kk][0], sh, o1);
+                    x2 = mma(w[kk][1], sh, x2);
+                    o2 = mma(qv[kk][1], sh, o2);
+                    x3 = mma(w[kk][2], sh, x3);
+                    o3 = mma(qv[kk][2], sh, o3);
+                    x2 = mma(w[kk][0], sm, x2);
+                    o2 = mma(qv[kk][0], sm, o2);
+                    x3 = mma(w[kk][1], sm, x3);
+                    o3 = mma(qv[kk][1], sm, o3);
+                    x3 = mma(w[kk][0], sl, x3);
+                    o3 = mma(qv[kk][0], sl, o3);
+                }
+                if (vt >= 4) __builtin_amdgcn_s_setprio(0);
+                else __builtin_amdgcn_s_setprio(1);
+                u = u - (x1 + (x2 + x3));
+                uint32_t uc[3][2];
+                {
+                    const float f[4] = {u[0], u[1], u[2], u[3]};
+                    split3<4>(f, uc);
+                }
+                const bf16x8_t uhh = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[0][0], uc[0][1], uc[0][0], uc[0][1]});
+                const bf16x8_t umm = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[1][0], uc[1][1], uc[1][0], uc[1][1]});
+                const bf16x8_t ulh = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[2][0], uc[2][1], uc[0][0], uc[0][1]});
+                const u32x4_t b0 = buf.b(0)[lane], b1 = buf.b(1)[lane];
+                o3 = mma(b1, ulh, o3);
+                o2 = mma(b0, umm, o2);
+                o1 = mma(b0, uhh, o1);
+                const f32x4_t* e = reinterpret_cast<const f32x4_t*>(buf.e());
+                u32x4_t k0[DT], k1[DT];
+                f32x4_t ds[DT], et[DT];
+    #pragma unroll
+                for (int t = 0; t < DT; ++t) {
+                    k0[t] = buf.k(t, 0)[lane];
+                    k1[t] = buf.k(t, 1)[lane];
+                    et[t] = e[4 * t + q];
+                }
+    #pragma unroll
+                for (int t = 0; t < DT; ++t) ds[t] = mma(k1[t], ulh, f32x4_t{0.f, 0.f, 0.f, 0.f});
+    #pragma unroll
+                for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], umm, ds[t]);
+    #pragma unroll
+                for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], uhh, ds[t]);
+    #pragma unroll
+                for (int t = 0; t < DT; ++t) {
+    #pragma unroll
+                    for (int r = 0; r < 4; ++r) s[t][r] = __builtin_fmaf(s[t][r], et[t][r], ds[t][r]);
+                }
+                const f32x4_t o = o1 + (o2 + o3);
+                float* to = outputs + ((c & 1) * 16 + 4 * q) * kPitch + 16 * vt + m;
+    #pragma unroll
+                for (int r = 0; r < 4; ++r) to[r * kPitch] = o[r];
+            }
+            __builtin_amdgcn_s_setprio(0);
+            done_row = row;
+            done_count = count;
+            row = __builtin_amdgcn_readfirstlane(next_row);
+            count = __builtin_amdgcn_readfirstlane(next_count);
+            const int after = c + 2 < p.chunks ? c + 2 : p.chunks - 1;
+            next_row = descs[after * kDesc];
+            next_count = descs[after * kDesc + 1];
+            __syncthreads();
         }
-        if (c > 0) finish((c - 1) & 1);
-        fetch(c + 2);
-        // rows behind a chunk's last repeat it; an empty chunk has none, and row 0 exists
-        gate = *reinterpret_cast<const t4_t*>(gates + (int64_t)(count > 0 ? row + (out_row < count ? out_row : count - 1) : 0) * a.gate_stride);
-        __builtin_amdgcn_sched_barrier(0);             // requests stay here, a step ahead of their use
-        if (live) {
-            // The vector unit cuts the next part of the state while the matrix pipe works on one.  The pipe rounds its sums towards one
-            // side, so nothing stays in its accumulators from chunk to chunk: the state takes a chunk's sum by the vector unit.  3200
-            // tokens without decay, all of one sign: error of the state 5.7e-7 of its norm, 6.6e-6 with the state in the pipe's
-            // accumulators and pieces cut off instead of rounded, 1.4e-6 in delta_scan_kernel; 794 -> 807 us for the call with the batch above.
-            f32x4_t x1 = {0.f, 0.f, 0.f, 0.f}, x2 = x1, x3 = x1, o1 = x1, o2 = x1, o3 = x1;
-            uint32_t pc[KS][3][4];
-            u32x4_t w[KS][3], qv[KS][3];
-            auto part = [&](int kk) {
-                const float f[8] = {s[2 * kk][0], s[2 * kk][1], s[2 * kk][2], s[2 * kk][3], s[2 * kk + 1][0], s[2 * kk + 1][1], s[2 * kk + 1][2], s[2 * kk + 1][3]};
-#pragma unroll
-                for (int i = 0; i < 3; ++i) { w[kk][i] = buf.wq(0, kk, i)[lane]; qv[kk][i] = buf.wq(1, kk, i)[lane]; }
-                split3<8>(f, pc[kk]);
-            };
-            part(0);
-#pragma unroll
-            for (int kk = 0; kk < KS; ++kk) {
-                const bf16x8_t sh = frag(pc[kk][0]), sm = frag(pc[kk][1]), sl = frag(pc[kk][2]);
-                if (kk + 1 < KS) part(kk + 1);
-                x1 = mma(w[kk][0], sh, x1);
-                o1 = mma(qv[kk][0], sh, o1);
-                x2 = mma(w[kk][1], sh, x2);
-                o2 = mma(qv[kk][1], sh, o2);
-                x3 = mma(w[kk][2], sh, x3);
-                o3 = mma(qv[kk][2], sh, o3);
-                x2 = mma(w[kk][0], sm, x2);
-                o2 = mma(qv[kk][0], sm, o2);
-                x3 = mma(w[kk][1], sm, x3);
-                o3 = mma(qv[kk][1], sm, o3);
-                x3 = mma(w[kk][0], sl, x3);
-                o3 = mma(qv[kk][0], sl, o3);
-            }
-            u = u - (x1 + (x2 + x3));
-            uint32_t uc[3][2];
-            {
-                const float f[4] = {u[0], u[1], u[2], u[3]};
-                split3<4>(f, uc);
-            }
-            const bf16x8_t uhh = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[0][0], uc[0][1], uc[0][0], uc[0][1]});
-            const bf16x8_t umm = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[1][0], uc[1][1], uc[1][0], uc[1][1]});
-            const bf16x8_t ulh = __builtin_bit_cast(bf16x8_t, u32x4_t{uc[2][0], uc[2][1], uc[0][0], uc[0][1]});
-            const u32x4_t b0 = buf.b(0)[lane], b1 = buf.b(1)[lane];
-            o3 = mma(b1, ulh, o3);
-            o2 = mma(b0, umm, o2);
-            o1 = mma(b0, uhh, o1);
-            const f32x4_t* e = reinterpret_cast<const f32x4_t*>(buf.e());
-            u32x4_t k0[DT], k1[DT];
-            f32x4_t ds[DT], et[DT];
-#pragma unroll
-            for (int t = 0; t < DT; ++t) {
-                k0[t] = buf.k(t, 0)[lane];
-                k1[t] = buf.k(t, 1)[lane];
-                et[t] = e[4 * t + q];
-            }
-#pragma unroll
-            for (int t = 0; t < DT; ++t) ds[t] = mma(k1[t], ulh, f32x4_t{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], umm, ds[t]);
-#pragma unroll
-            for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], uhh, ds[t]);
-#pragma unroll
-            for (int t = 0; t < DT; ++t) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) s[t][r] = __builtin_fmaf(s[t][r], et[t][r], ds[t][r]);
-            }
-            const f32x4_t o = o1 + (o2 + o3);
-            float* to = outputs + ((c & 1) * 16 + 4 * q) * kPitch + 16 * vt + m;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) to[r * kPitch] = o[r];
-        }
-        done_row = row;
-        done_count = count;
-        row = __builtin_amdgcn_readfirstlane(next_row);
-        count = __builtin_amdgcn_readfirstlane(next_count);
-        const int after = c + 2 < p.chunks ? c + 2 : p.chunks - 1;
-        next_row = descs[after * kDesc];
-        next_count = descs[after * kDesc + 1];
-        __syncthreads();
-    }
+    };
+    if (live) walk(std::true_type{});
+    else walk(std::false_type{});
     finish((p.chunks - 1) & 1);
     keep_state();
 }
