@@ -23,15 +23,19 @@
 #include "pieces.h"
 #include "segments.h"
 
+#include <type_traits>
+
 namespace {
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;
 constexpr int kC = 32;          // tokens per chunk
 constexpr int kSlab = 64;       // state columns per workgroup of the chunk kernel
+constexpr int kTaps = 4;        // of the convolution inside the chunk kernel
 
 struct Span { int32_t row0, count, slot, pos0; };       // consecutive tokens of one sequence
 
@@ -135,13 +139,15 @@ __global__ void __launch_bounds__(kThreads) ssm_step_kernel(SsmArgs<T> a, const 
 }
 
 // ------------------------------------------------------------------ convolution of portions
-constexpr int kConvTokens = 16;         // per thread
+constexpr int kConvTokens = 16, kFewTokens = 4;         // per thread; where only B and C are convolved, which 16 leave to too few threads (14.5 us, 13,800 tokens)
 
-// VEC channels per thread over 16 consecutive tokens; TAPS > 0: the inputs it looks back on stay in registers
-template <class T, int VEC, int TAPS>
-__global__ void __launch_bounds__(kThreads) ssm_conv_kernel(SsmArgs<T> a, const Span* spans, T* out) {
+// VEC channels per thread over TOKENS consecutive tokens, from channel `first` on, in kFewTokens form `units` threads side by side; TAPS > 0: the inputs it looks
+// back on stay in registers
+template <class T, int VEC, int TAPS, int TOKENS = kConvTokens>
+__global__ void __launch_bounds__(kThreads) ssm_conv_kernel(SsmArgs<T> a, const Span* spans, T* out, int first, int units) {
     const Span span = spans[blockIdx.z];
-    const int c = (blockIdx.x * kThreads + threadIdx.x) * VEC, i0 = blockIdx.y * kConvTokens;
+    const unsigned item = blockIdx.x * kThreads + threadIdx.x, block = TOKENS == kConvTokens ? blockIdx.y : item / (unsigned)units;
+    const int c = first + (int)(TOKENS == kConvTokens ? item : item - block * units) * VEC, i0 = (int)block * TOKENS;
     if (c >= a.channels || i0 >= span.count || span.slot < 0 || span.slot >= a.num_slots) return;
     const T* in = a.proj + (int64_t)span.row0 * a.proj_stride + a.x_off + c;
     const T* ring = a.ring + (int64_t)span.slot * a.taps * a.channels + c;
@@ -157,7 +163,7 @@ __global__ void __launch_bounds__(kThreads) ssm_conv_kernel(SsmArgs<T> a, const 
         }
     };
     T* o = out + (span.row0 - a.xbc_row0 + i0) * a.xbc_stride + c;
-    const int end = i0 + kConvTokens < span.count ? kConvTokens : span.count - i0;
+    const int end = i0 + TOKENS < span.count ? TOKENS : span.count - i0;
     float bias[VEC];
     load_elems<VEC>(a.conv_bias + c, bias);
     if constexpr (TAPS > 0) {
@@ -170,9 +176,9 @@ __global__ void __launch_bounds__(kThreads) ssm_conv_kernel(SsmArgs<T> a, const 
         for (int k = 0; k + 1 < TAPS; ++k) input(i0 + k - (TAPS - 1), x[k]);
         // inputs are requested in batches: the compiler moves no load in front of a store
         struct alignas(sizeof(T) * VEC < 16 ? sizeof(T) * VEC : 16) Raw { T e[VEC]; };
-        constexpr int kBatch = 8;
+        constexpr int kBatch = TOKENS < 8 ? TOKENS : 8;
 #pragma unroll
-        for (int b = 0; b < kConvTokens; b += kBatch) {
+        for (int b = 0; b < TOKENS; b += kBatch) {
             if (b >= end) break;
             Raw raw[kBatch];
 #pragma unroll
@@ -278,12 +284,13 @@ struct ChunkArgs {
 // eight wavefronts half the state rows each: lane (g, n) holds state rows 16 t + 4 g + e of column n.  That is an operand of the product with C
 // as it lies, when the state rows of a k-step of 32 are taken in the order 16 tau + 4 g + e.  The 32 x 32 products C_i B_j are shared
 // out over the wavefronts of the first half, weighted, and exchanged through LDS; those of the second add up and write the results.
-// OUT = false: only the final state, from zero.
+// OUT = false: only the final state, from zero.  RAW: x comes as it entered the convolution, four taps, which is done here, of the next chunk while this one's products run (the
+// pass 175 -> 220 us under a profiler, the launch that it replaces took 54, the one of B and C that is left 7); the portion is one segment.
 // A portion takes as long as its chunks one after the other, and a chunk as long as one wavefront's instructions and reads of LDS (four
 // wavefronts: 445 and 30 reads, 3900 clocks with three barriers).  Eight halve what follows one another, and where two chunks lie in LDS one
 // barrier is left, behind which a chunk's results are finished under the next one's products.  6 portions of 900 to 3700 tokens of 64 heads,
 // the call: 324 us, 310 with the barriers alone, 286 with eight wavefronts.
-template <int NS, int WAVES, bool OUT>
+template <int NS, int WAVES, bool OUT, bool RAW>
 __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm_chunk_kernel(ChunkArgs args) {
     constexpr int kRow = NS * 64 + 16, kXRow = 2 * kSlab + 16, kMRow = 2 * kC + 16;      // bytes
     constexpr int kThr = 64 * WAVES, kParts = WAVES / 4, NT = 2 * NS / kParts;      // tiles of 16 state rows per wavefront
@@ -299,6 +306,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
     auto& weights = *reinterpret_cast<float(*)[2][kAhead][kC]>(behind + 2 * sizeof(sums));
     auto& mbufs = *reinterpret_cast<unsigned char(*)[2][2 * kC * kMRow]>(behind + 3 * sizeof(sums));               // OUT
     auto& ybufs = *reinterpret_cast<f32x4_t(*)[2][4][2][64]>(behind + 3 * sizeof(sums) + sizeof(mbufs));           // OUT
+    auto& taps = *reinterpret_cast<float(*)[kTaps + 1][kSlab]>(behind + 3 * sizeof(sums) + (OUT ? sizeof(mbufs) + (kParts > 1 ? sizeof(ybufs) : 0) : 0));   // RAW; last: the bias
     const SsmArgs<__bf16>& a = args.a;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 2, cw = wave & 3;
@@ -343,25 +351,46 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
         u_tok[i] = u < kC * units ? u / units : -1;
         u_col[i] = 8 * (u % units);
     }
-    const int x_tok = tid >> 3 & (kC - 1), x_col = 8 * (tid & 7);
-    const bool x_in = tid < 8 * kC && slab * kSlab + x_col < a.vdim;
+    constexpr int XV = RAW && kThr == 512 ? 4 : 8, XR = RAW ? kTaps : 1;       // columns of x and rows of the window that a thread brings
+    typedef typename std::conditional<XV == 4, u32x2_t, u32x4_t>::type xvec_t;
+    const int x_tok = tid / (kSlab / XV) % kC, x_col = XV * (tid % (kSlab / XV));
+    const bool x_in = tid < kSlab / XV * kC && slab * kSlab + x_col < a.vdim;
+    const int x_chan = h * a.vdim + (x_in ? slab * kSlab + x_col : 0);
     const __bf16* rows = a.xbc + (row0 - a.xbc_row0) * a.xbc_stride;
     const __bf16* b_src = rows + inner + grp * N;
     const __bf16* c_src = b_src + a.groups * N;
-    const __bf16* x_src = rows + h * a.vdim + (x_in ? slab * kSlab + x_col : 0);
+    const int64_t x_stride = RAW ? a.proj_stride : a.xbc_stride;
+    const __bf16* x_src = RAW ? a.proj + (int64_t)row0 * a.proj_stride + a.x_off + x_chan : rows + x_chan;
     const __bf16* dt_src = a.proj + (int64_t)row0 * a.proj_stride + a.dt_off + h;
-    u32x4_t breg[NU], creg[NU], xreg;
+    u32x4_t breg[NU], creg[NU];
+    xvec_t xreg[XR];
     __bf16 dtreg;
     auto fetch = [&](int c) {                                    // chunk c; tokens behind the last one re-read it
         const int last = count - 1, t0 = c * kC;
-        auto tok = [&](int i) { return t0 + i < last ? t0 + i : last; };
+        auto tok = [&](int i) -> int64_t { return t0 + i < last ? t0 + i : last; };
 #pragma unroll
         for (int i = 0; i < NU; ++i) {
             const int64_t r = tok(u_tok[i] > 0 ? u_tok[i] : 0) * a.xbc_stride;
             breg[i] = *reinterpret_cast<const u32x4_t*>(b_src + r + u_col[i]);
             if constexpr (OUT) creg[i] = *reinterpret_cast<const u32x4_t*>(c_src + r + u_col[i]);
         }
-        xreg = *reinterpret_cast<const u32x4_t*>(x_src + tok(x_tok) * a.xbc_stride);
+    };
+    auto fetch_x = [&](int c) {                                  // behind fetch(c)
+        const int last = count - 1, t = c * kC + x_tok;
+        const __bf16* r = x_src + (int64_t)((t < last ? t : last) - (XR - 1)) * x_stride;
+#pragma unroll
+        for (int k = 0; k < XR; ++k) xreg[k] = *reinterpret_cast<const xvec_t*>(r + k * x_stride);
+    };
+    // the window of a portion's first tokens looks back on the ring, and on zeros in front of the sequence
+    auto fetch_first = [&] {
+        const int last = count - 1, t = x_tok < last ? x_tok : last;
+#pragma unroll
+        for (int k = 0; k < XR; ++k) {
+            const int i = t + k - (XR - 1), pos = span.pos0 + i;
+            xreg[k] = xvec_t{};
+            if (i >= 0) xreg[k] = *reinterpret_cast<const xvec_t*>(x_src + (int64_t)i * x_stride);
+            else if (pos >= 0) xreg[k] = *reinterpret_cast<const xvec_t*>(a.ring + ((int64_t)span.slot * kTaps + pos % kTaps) * a.channels + x_chan);
+        }
     };
     auto fetch_dt = [&](int c) {
         const int t = c * kC + (lane & 31);
@@ -387,6 +416,36 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
         }
         fetch_dt(c + kAhead + wave);
     };
+    // x of the chunk requested last, as it enters LDS: of eight wavefronts among the products, of four behind the stores of B and C
+    constexpr bool kWithin = WAVES == 8;
+    xvec_t xput;
+    auto convolve = [&]() __attribute__((always_inline)) {
+        if constexpr (!RAW) {
+            xput = xreg[0];
+        } else {
+            float y[XV];
+#pragma unroll
+            for (int q = 0; q < XV; q += 4) {
+                f32x4_t v = *reinterpret_cast<const f32x4_t*>(&taps[kTaps][x_col + q]);
+#pragma unroll
+                for (int k = 0; k < kTaps; ++k) {
+                    const f32x4_t w = *reinterpret_cast<const f32x4_t*>(&taps[k][x_col + q]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t bits = xreg[k][(q + e) / 2];
+                        v[e] += w[e] * __builtin_bit_cast(float, e & 1 ? bits & 0xffff0000u : bits << 16);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[q + e] = silu_f(v[e]);
+            }
+            typedef __bf16 xbf_t __attribute__((ext_vector_type(XV)));
+            xbf_t o;
+#pragma unroll
+            for (int e = 0; e < XV; ++e) o[e] = (__bf16)y[e];
+            xput = __builtin_bit_cast(xvec_t, o);
+        }
+    };
     auto put = [&](int c) {
 #pragma unroll
         for (int i = 0; i < NU; ++i)
@@ -394,7 +453,8 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
                 *reinterpret_cast<u32x4_t*>(bbufs[c % kBufs] + u_tok[i] * kRow + 2 * u_col[i]) = breg[i];
                 if constexpr (OUT) *reinterpret_cast<u32x4_t*>(cbufs[c % kBufs] + u_tok[i] * kRow + 2 * u_col[i]) = creg[i];
             }
-        if (x_in) *reinterpret_cast<u32x4_t*>(xbufs[c % kBufs] + x_tok * kXRow + 2 * x_col) = xreg;
+        if constexpr (!kWithin) convolve();
+        if (x_in) *reinterpret_cast<xvec_t*>(xbufs[c % kBufs] + x_tok * kXRow + 2 * x_col) = xput;
     };
     f32x4_t y[2];
     bf16x8_t xf;
@@ -418,11 +478,23 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
         }
     };
     fetch(0);
+    if constexpr (RAW) fetch_first();
+    else fetch_x(0);
     fetch_dt(wave);
+    if constexpr (RAW)
+        for (int i = tid; i < (kTaps + 1) * kSlab; i += kThr) {
+            const int k = i / kSlab, col = i % kSlab, c = h * a.vdim + slab * kSlab + col;
+            const bool in = slab * kSlab + col < a.vdim;
+            taps[k][col] = !in ? 0.f : k == kTaps ? a.conv_bias[c] : a.conv[(int64_t)c * kTaps + k];
+        }
     __syncthreads();                                             // the zero fill
     put_steps(0);
+    if constexpr (kWithin) convolve();
     put(0);
-    if (chunks > 1) fetch(1);
+    if (chunks > 1) {
+        fetch(1);
+        fetch_x(1);
+    }
     // Behind the barrier the chunk lies in LDS, and the products of the last chunk's tokens, whose results are finished while
     // this chunk's products run.  Everything that is written between two barriers was read last in front of the first.
 #pragma unroll 1                                                 // unrolled it spills
@@ -491,6 +563,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
                 if (kParts > 1 && half == 0) ybufs[c & 1][cw][t][lane] = y[t];
             }
         }
+        if constexpr (kWithin) convolve();
         // the state
         float wx[8], xv[8];
         widen(__builtin_bit_cast(u32x4_t, xf), xv);
@@ -514,7 +587,10 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 && NS <= 4 ? 4 : 2) ssm
             if constexpr (kBufs == 1) __syncthreads();
             if ((c + 1) % kAhead == 0) put_steps(c + 1);
             put(c + 1);
-            if (c + 2 < chunks) fetch(c + 2);
+            if (c + 2 < chunks) {
+                fetch(c + 2);
+                fetch_x(c + 2);
+            }
         }
     }
     if constexpr (OUT) {
@@ -645,12 +721,13 @@ Walk walk_of(int64_t heads, int64_t vdim, int64_t state_n, int64_t num_spans, in
     return Walk{wide ? 8 : 4, (int)seg_len, (int)(max_span > 0 ? (max_span + seg_len - 1) / seg_len : 1)};
 }
 
-template <int NS, int WAVES, bool OUT>
+template <int NS, int WAVES, bool OUT, bool RAW>
 int launch_chunk(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
     constexpr size_t bufs = NS > 4 || WAVES == 4 ? 1 : 2;
     constexpr size_t lds = kC * (bufs * ((OUT ? 2 : 1) * (NS * 64 + 16) + 2 * kSlab + 16) + (OUT ? 2 * 2 * (2 * kC + 16) : 0)) +
-                           3 * 2 * WAVES * kC * sizeof(float) + (OUT && WAVES == 8 ? 2 * 4 * 2 * 64 * sizeof(f32x4_t) : 0);
-    auto kernel = &ssm_chunk_kernel<NS, WAVES, OUT>;
+                           3 * 2 * WAVES * kC * sizeof(float) + (OUT && WAVES == 8 ? 2 * 4 * 2 * 64 * sizeof(f32x4_t) : 0) +
+                           (RAW ? (kTaps + 1) * kSlab * sizeof(float) : 0);
+    auto kernel = &ssm_chunk_kernel<NS, WAVES, OUT, RAW>;
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
@@ -659,16 +736,17 @@ int launch_chunk(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-template <int NS, int WAVES>
+template <int NS, int WAVES, bool RAW>
 int launch_chunks(const ChunkArgs& c, int64_t num_spans, hipStream_t st) {
+    if constexpr (RAW) return launch_chunk<NS, WAVES, true, true>(c, num_spans, st);        // one segment
     if (c.max_seg > 1) {
-        const int rc = launch_chunk<NS, WAVES, false>(c, num_spans, st);
+        const int rc = launch_chunk<NS, WAVES, false, false>(c, num_spans, st);
         if (rc) return rc;
         const int64_t state_len = (int64_t)c.a.state_n * c.a.vdim;
         hipLaunchKernelGGL(ssm_join_kernel, dim3((unsigned)((state_len + kThreads - 1) / kThreads), (unsigned)c.a.heads, (unsigned)num_spans),
                            dim3(kThreads), 0, st, c);
     }
-    return launch_chunk<NS, WAVES, true>(c, num_spans, st);
+    return launch_chunk<NS, WAVES, true, false>(c, num_spans, st);
 }
 
 template <class T>
@@ -681,12 +759,16 @@ int portions(SsmArgs<T>& a, const Span* spans, int64_t num_spans, int64_t max_sp
     a.xbc_row0 = row0;
     const bool vec = a.channels % 8 == 0 && a.proj_stride % 8 == 0 && a.x_off % 8 == 0 && ptr_aligned(a.proj, 16) && ptr_aligned(xbc, 16) &&
                      ptr_aligned(a.ring, 16) && ptr_aligned(a.conv_bias, 16);
-    const int64_t units = vec ? a.channels / 8 : a.channels, token_blocks = (max_span + kConvTokens - 1) / kConvTokens;
+    const int64_t token_blocks = (max_span + kConvTokens - 1) / kConvTokens;
     if (token_blocks > 65535) return INFER_KV_EINVAL;
-    const dim3 grid((unsigned)((units + kThreads - 1) / kThreads), (unsigned)token_blocks, (unsigned)num_spans), block(kThreads);
-    if (vec && a.taps == 4) hipLaunchKernelGGL((ssm_conv_kernel<T, 8, 4>), grid, block, 0, st, a, spans, xbc);
-    else if (vec) hipLaunchKernelGGL((ssm_conv_kernel<T, 8, 0>), grid, block, 0, st, a, spans, xbc);
-    else hipLaunchKernelGGL((ssm_conv_kernel<T, 1, 0>), grid, block, 0, st, a, spans, xbc);
+    const dim3 block(kThreads);
+    auto convolve = [&] {
+        const dim3 grid((unsigned)(((vec ? a.channels / 8 : a.channels) + kThreads - 1) / kThreads), (unsigned)token_blocks, (unsigned)num_spans);
+        if (vec && a.taps == 4) hipLaunchKernelGGL((ssm_conv_kernel<T, 8, 4>), grid, block, 0, st, a, spans, xbc, 0, 0);
+        else if (vec) hipLaunchKernelGGL((ssm_conv_kernel<T, 8, 0>), grid, block, 0, st, a, spans, xbc, 0, 0);
+        else hipLaunchKernelGGL((ssm_conv_kernel<T, 1, 0>), grid, block, 0, st, a, spans, xbc, 0, 0);
+        return (int)hipGetLastError();
+    };
     if constexpr (sizeof(T) == 2) {
         if (chunked(INFER_ELEM_BF16, a.vdim, a.state_n) && vec && a.y_stride % 4 == 0 && ptr_aligned(a.y, 8)) {
             const Walk walk = walk_of(a.heads, a.vdim, a.state_n, num_spans, max_span);
@@ -698,11 +780,30 @@ int portions(SsmArgs<T>& a, const Span* spans, int64_t num_spans, int64_t max_sp
                 c.ws = ws;
                 c.ws_decay = ws + records * len;
             }
-            if (a.state_n > 128) return launch_chunks<8, 4>(c, num_spans, st);
-            if (walk.waves == 8) return a.state_n <= 64 ? launch_chunks<2, 8>(c, num_spans, st) : launch_chunks<4, 8>(c, num_spans, st);
-            return a.state_n <= 64 ? launch_chunks<2, 4>(c, num_spans, st) : launch_chunks<4, 4>(c, num_spans, st);
+            // x is convolved where it is used, and only B and C, which all heads of a group share, by a launch of their own, unless portions are cut,
+            // since their x would be convolved twice (1 of 4000 tokens 123 -> 125 us).  The call, us, x by a launch / inside: 64 heads, 6 portions
+            // of 900 to 3700 tokens 266 / 255, 8 of 1000 152 / 140, 10 of 800 to 1800 229 / 219, 32 of 60 to 200 109 / 107; 32 heads, 20 of 200 to 900 135 / 121,
+            // 9 of 500 to 1500 134 / 127.
+            const int64_t items = (int64_t)(a.channels - a.heads * a.vdim) / 8 * ((max_span + kFewTokens - 1) / kFewTokens);
+            const bool raw = a.taps == kTaps && c.max_seg == 1 && items <= 0x7fffffff;
+            if (raw) {
+                hipLaunchKernelGGL((ssm_conv_kernel<T, 8, kTaps, kFewTokens>), dim3((unsigned)((items + kThreads - 1) / kThreads), 1, (unsigned)num_spans), block, 0, st,
+                                   a, spans, xbc, a.heads * a.vdim, (a.channels - a.heads * a.vdim) / 8);
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess) return (int)e;
+            } else if (const int rc = convolve()) {
+                return rc;
+            }
+            auto walked = [&](auto within) {
+                constexpr bool RAW = decltype(within)::value;
+                if (a.state_n > 128) return launch_chunks<8, 4, RAW>(c, num_spans, st);
+                if (walk.waves == 8) return a.state_n <= 64 ? launch_chunks<2, 8, RAW>(c, num_spans, st) : launch_chunks<4, 8, RAW>(c, num_spans, st);
+                return a.state_n <= 64 ? launch_chunks<2, 4, RAW>(c, num_spans, st) : launch_chunks<4, 4, RAW>(c, num_spans, st);
+            };
+            return raw ? walked(std::true_type{}) : walked(std::false_type{});
         }
     }
+    if (const int rc = convolve()) return rc;
     const dim3 sgrid((unsigned)((a.vdim + 15) / 16), (unsigned)a.heads, (unsigned)num_spans);
     if (a.state_n <= 64) hipLaunchKernelGGL((ssm_scan_any_kernel<T, 4>), sgrid, block, 0, st, a, spans);
     else if (a.state_n <= 256) hipLaunchKernelGGL((ssm_scan_any_kernel<T, 16>), sgrid, block, 0, st, a, spans);

@@ -460,6 +460,25 @@ def test_state_space_portions_that_take_turns(gpu, heads, lens):
         close(m.state[len(lens) - 1 - i], states, 1e-2)
 
 
+@pytest.mark.parametrize("shape", [(3, 72, 64, 1, 4, 1), (5, 64, 128, 1, 4, 1), (2, 136, 256, 2, 4, 4), (520, 8, 16, 2, 4, 1)])
+def test_state_space_portions_begin_around_the_window(gpu, shape):
+    """Convolution where x is used: portions that begin at positions 0 to 4, a row or two long and around a chunk, whose windows look back on the ring, on zeros and on the chunk before."""
+    m = Ssm(np.random.default_rng(shape[1]), shape, torch.bfloat16, slots=9)
+    cuts = [(2, 33), (3, 32), (33, 2, 31), (1, 3, 65), (4, 64), (31, 35), (32, 2), (1, 1, 2, 34)]
+    x = [m.inputs(sum(c)) for c in cuts]
+    got = [[] for _ in cuts]
+    for k in range(4):
+        now = [(i, sum(c[:k]), c[k]) for i, c in enumerate(cuts) if k < len(c)]
+        now.sort(key=lambda p: p[2] > 1)                                           # decoded tokens come first
+        if now:
+            for (i, _, _), y in zip(now, m.run([(i, lo, x[i][lo:lo + n]) for i, lo, n in now])):
+                got[i].append(y)
+    for i, a in enumerate(x):
+        want, states = m.want(a)
+        close(torch.tensor(np.concatenate(got[i])), want, 2e-2)
+        close(m.state[i], states, 1e-2)
+
+
 @pytest.mark.parametrize("shape", [SSM[2], (4, 72, 48, 2, 4, 2)])
 def test_state_space_of_many_portions_and_of_a_long_one(gpu, shape):
     """More workgroups than two per compute unit, walked by four wavefronts each instead of eight, and one portion of many segments."""
