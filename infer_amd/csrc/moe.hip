@@ -448,6 +448,10 @@ __global__ void __launch_bounds__(kThreads, 2) moe_tile_kernel(GemmArgs<__bf16> 
 //
 // A row of a buffer is eight units of 16 bytes, unit c at place c ^ (row % 8), so that reads of a column meet all banks.
 constexpr int kBlockRows = 256, kBlockThreads = 256;
+// What an earlier launch wrote and this one only reads, by the scalar path.  i: the same in all lanes
+__device__ __forceinline__ int fixed_at(const int32_t* p, int64_t i) {
+    return reinterpret_cast<const __attribute__((address_space(4))) int32_t*>((uintptr_t)p)[i];
+}
 // Tiles of an expert that are worked on side by side: a die's compute units then share that many blocks of rows and 32 / kSideTiles of W.
 constexpr int kSideTiles = 8;
 // Which tiles a launch has: all of them, or (MANY) those of experts with more than kSpan rows.
@@ -470,7 +474,10 @@ struct BlockTiles {
         for (int i = 0; i < kSets; ++i) set[i] = __ballot(rows[i] > kSpan);
     }
     __device__ __forceinline__ int total() const {
-        if constexpr (!MANY) return a.tiles[2 * a.max_tiles - 2] < 0 ? a.tiles[2 * a.max_tiles - 1] : a.max_tiles;      // behind the last their number stands
+        if constexpr (!MANY) {                                   // behind the last their number stands
+            const int mark = fixed_at(a.tiles, 2 * (int64_t)a.max_tiles - 2), number = fixed_at(a.tiles, 2 * (int64_t)a.max_tiles - 1);
+            return mark < 0 ? number : a.max_tiles;
+        }
         int n = 0;
         for (int t = 0; t < a.max_tiles; t += 64 * kSets) {
             uint64_t set[kSets];
@@ -507,9 +514,10 @@ __device__ __forceinline__ bool block_unit(const GemmArgs<__bf16>& a, const Bloc
     if ((block >> 3) >= units / 8 + (die < extra ? 1 : 0)) return false;
     const unsigned unit = die * (units / 8) + (die < extra ? die : extra) + (block >> 3);
     const int some = (int)(unit / columns), listed = list.at(some);         // a tile of the unit's expert
-    u.expert = a.tiles[2 * listed];
+    const int in_expert = fixed_at(a.tiles, 2 * (int64_t)listed + 1);
+    u.expert = fixed_at(a.tiles, 2 * (int64_t)listed);
     if (u.expert < 0 || u.expert >= a.experts) return false;
-    const int row0 = a.offsets[u.expert], end = a.offsets[u.expert + 1], tile0 = some - a.tiles[2 * listed + 1] / kBlockRows;
+    const int row0 = fixed_at(a.offsets, u.expert), end = fixed_at(a.offsets, u.expert + 1), tile0 = some - in_expert / kBlockRows;
     const unsigned tiles = (unsigned)(end - row0 + kBlockRows - 1) / kBlockRows, groups = (tiles + kSideTiles - 1) / kSideTiles;
     const unsigned side = (tiles + groups - 1) / groups, of_expert = unit - (unsigned)tile0 * columns, group = of_expert / (side * columns);
     const unsigned here = tiles - group * side < side ? tiles - group * side : side, rest = of_expert - group * side * columns;
@@ -531,7 +539,7 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
     for (int i = 0; i < 8; ++i) {
         const int r = 8 * (8 * wave + i) + (lane >> 3), unit = (lane & 7) ^ (lane >> 3);
         const int xr = first + (r < rows ? r : rows - 1);
-        x_off[i] = 2u * ((uint32_t)(a.row_token ? a.row_token[xr] : xr) * (uint32_t)a.x_stride + 8u * unit);
+        x_off[i] = 2u * ((uint32_t)(GATED ? a.row_token[xr] : xr) * (uint32_t)a.x_stride + 8u * unit);        // the second product's rows lie by expert
         int col = GATED ? c0 + 32 * (r >> 6) + (r & 31) : c0 + r;
         col = col < a.cols ? col : a.cols - 1;
         w_off[i] = 2u * ((uint32_t)(GATED && (r & 32) ? a.up_row + col : col) * (uint32_t)a.w_stride + 8u * unit);
@@ -634,16 +642,19 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
     for (; s + 2 < steps; ++s) step(s, std::true_type{});
     for (; s < steps; ++s) step(s, std::false_type{});
     settle();
-    // lane (g, n): row n of a row tile, columns 4 g + e
+    // Lane (g, n) has row n of a row tile, columns 4 g + e: 8 bytes of every 32 of a row.  They go through LDS, a wavefront's rows to a part of its own, so that
+    // rows are written in one piece.  With the unit's place read by the scalar path (block_unit), us, before / now: 14 experts of 4096 x 3072, 8000 rows 1370 / 1346, 5000
+    // 913 / 899, 1500 448 / 446; of 2880 x 2880, 3000 rows 442 / 435 (without the scalar path 1351, 901, 448, 435).
+    constexpr int kCols = GATED ? 64 : 128, kPitch = 2 * kCols + 16, kRowLanes = kCols / 8;
+    static_assert(4 * 128 * kPitch <= kBlockLds, "room in LDS");
+    __syncthreads();                                             // everybody has read the last step's operands
+    unsigned char* own = lds + wave * 128 * kPitch;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int r = 128 * wm + 16 * j + n;
-        if (r >= rows) continue;
-        __bf16* o = a.out + (int64_t)(first + r) * a.out_stride;
+    for (int j = 0; j < 8; ++j)
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             if (GATED && (i & 2)) continue;
-            const int c = c0 + (GATED ? 64 * wn + 32 * (i >> 2) + 16 * (i & 1) : 128 * wn + 16 * i) + 4 * g;
+            const int at = (GATED ? 32 * (i >> 2) + 16 * (i & 1) : 16 * i) + 4 * g, c = c0 + kCols * wn + at;
             bf16x4_t v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -651,8 +662,14 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
                 if constexpr (GATED) x = silu_f(x) * acc[(i + 2) & 7][j][e];
                 v[e] = (__bf16)(c + e < a.cols ? x : 0.f);
             }
-            if (c + 4 <= a.out_cols) *reinterpret_cast<bf16x4_t*>(o + c) = v;       // out_cols is a multiple of eight
+            *reinterpret_cast<bf16x4_t*>(own + (16 * j + n) * kPitch + 2 * at) = v;
         }
+    const int c = c0 + kCols * wn + 8 * (lane % kRowLanes);
+#pragma unroll
+    for (int i = 0; i < 128 * kRowLanes / 64; ++i) {
+        const int in = 64 / kRowLanes * i + lane / kRowLanes, r = 128 * wm + in;
+        const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(own + in * kPitch + 16 * (lane % kRowLanes));
+        if (r < rows && c < a.out_cols) *reinterpret_cast<bf16x8_t*>(a.out + (int64_t)(first + r) * a.out_stride + c) = v;       // out_cols is a multiple of eight
     }
 }
 
