@@ -506,13 +506,23 @@ struct BlockTiles {
 };
 // The unit of workgroup number `block`: false if there is none, otherwise its expert, rows first .. first + rows - 1 and columns c0 and on.  Workgroups go to the eight
 // dies round-robin, and each die gets a contiguous run of (expert, group of tiles, columns, tile): those that run at the same time share rows and weights of one
-// expert.
+// expert.  Units behind a die's last whole round, if they are half a round at most, are two workgroups each, of half the rows: a round of them takes
+// some 0.6 of one of whole units.  Routing, both products and the sum, us, units of 256 rows / of 128 where an expert has no more left / and these:
+// 14 experts of 4096 x 3072, three each, 8000 rows 1380 / 1370 / 1357, 6000 1095 / 1082 / 1054, 4000 759 / 748 / 731, 3000 648 / 626 / 623, 1500 457 / 449 / 424; of
+// 2880 x 2880, 3000 rows 458 / 448 / 433; of 2048 x 1024, 6000 285 / 281 / 263.  In quarters, of half the columns, too, up to a quarter of a round: 1356, 1066, 734, 629, 418, 433, 260.
 struct BlockUnit { int expert, first, rows, c0; };
+constexpr unsigned kDieUnits = 32;                               // compute units of a die, of which each works on one unit
 template <bool GATED, bool MANY>
 __device__ __forceinline__ bool block_unit(const GemmArgs<__bf16>& a, const BlockTiles<MANY>& list, int total, unsigned columns, unsigned block, BlockUnit& u) {
-    const unsigned units = (unsigned)total * columns, die = block & 7u, extra = units & 7u;
-    if ((block >> 3) >= units / 8 + (die < extra ? 1 : 0)) return false;
-    const unsigned unit = die * (units / 8) + (die < extra ? die : extra) + (block >> 3);
+    const unsigned units = (unsigned)total * columns, die = block & 7u, extra = units & 7u, of_die = units / 8 + (die < extra ? 1 : 0), last = of_die % kDieUnits;
+    unsigned turn = block >> 3, part = 0;
+    const bool halves = !MANY && last <= kDieUnits / 2 && turn >= of_die - last;
+    if (halves) {
+        part = (turn - (of_die - last)) & 1;
+        turn = of_die - last + (turn - (of_die - last)) / 2;
+    }
+    if (turn >= of_die) return false;
+    const unsigned unit = die * (units / 8) + (die < extra ? die : extra) + turn;
     const int some = (int)(unit / columns), listed = list.at(some);         // a tile of the unit's expert
     const int in_expert = fixed_at(a.tiles, 2 * (int64_t)listed + 1);
     u.expert = fixed_at(a.tiles, 2 * (int64_t)listed);
@@ -523,26 +533,35 @@ __device__ __forceinline__ bool block_unit(const GemmArgs<__bf16>& a, const Bloc
     const unsigned here = tiles - group * side < side ? tiles - group * side : side, rest = of_expert - group * side * columns;
     u.first = row0 + kBlockRows * (int)(group * side + rest % here);
     u.rows = end - u.first < kBlockRows ? end - u.first : kBlockRows;
+    if (halves) {
+        u.first += (int)part * (kBlockRows / 2);
+        u.rows = part ? u.rows - kBlockRows / 2 : u.rows < kBlockRows / 2 ? u.rows : kBlockRows / 2;
+        if (u.rows <= 0) return false;
+    }
     u.c0 = (int)(rest / here) * (GATED ? 128 : 256);
     return true;
 }
 constexpr int kBlockLds = 5 * kBlockRows * 128;                  // bytes: three buffers of W, two of rows
-template <bool GATED>
-__device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, const BlockUnit& u, unsigned char* lds) {
+template <bool GATED, int RT>
+__device__ __forceinline__ void moe_block_tiles(const GemmArgs<__bf16>& a, const BlockUnit& u, unsigned char* lds) {
     constexpr int kMat = kBlockRows * 128;
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int first = u.first, rows = u.rows, c0 = u.c0;
-    // load i of a wavefront fills rows 8 (8 wave + i) .. + 7: lane l place l % 8 of row l / 8
-    uint32_t x_off[8], w_off[8];                                 // bytes (checked on the host to fit)
-    const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)(8192 * wave));
+    // load i of a wavefront fills rows 8 (8 wave + i) .. + 7 of W and 8 (RT wave + i) .. + 7 of the rows: lane l place l % 8 of row l / 8
+    uint32_t x_off[RT], w_off[8];                                // bytes (checked on the host to fit)
+    const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
+    const uint32_t to_w = to + 8192u * wave, to_x = to + 3 * kMat + 1024u * RT * wave;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int r = 8 * (8 * wave + i) + (lane >> 3), unit = (lane & 7) ^ (lane >> 3);
-        const int xr = first + (r < rows ? r : rows - 1);
-        x_off[i] = 2u * ((uint32_t)(GATED ? a.row_token[xr] : xr) * (uint32_t)a.x_stride + 8u * unit);        // the second product's rows lie by expert
         int col = GATED ? c0 + 32 * (r >> 6) + (r & 31) : c0 + r;
         col = col < a.cols ? col : a.cols - 1;
         w_off[i] = 2u * ((uint32_t)(GATED && (r & 32) ? a.up_row + col : col) * (uint32_t)a.w_stride + 8u * unit);
+    }
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        const int r = 8 * (RT * wave + i) + (lane >> 3), unit = (lane & 7) ^ (lane >> 3), xr = first + (r < rows ? r : rows - 1);
+        x_off[i] = 2u * ((uint32_t)(GATED ? a.row_token[xr] : xr) * (uint32_t)a.x_stride + 8u * unit);        // the second product's rows lie by expert
     }
     const __bf16* xs = a.x;
     const __bf16* ws = a.w + (int64_t)u.expert * a.w_expert;
@@ -550,36 +569,36 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
     auto request = [&](uint32_t off, const __bf16* from, uint32_t at) {
         __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(from), "s"(at) : "memory", "m0");
     };
-    auto fetch_x = [&](int i, int s) { request(x_off[i], xs + 64 * s, to + (uint32_t)(3 + (s & 1)) * kMat + 1024u * i); };
-    auto fetch_w = [&](int i, int s, uint32_t buf) { request(w_off[i], ws + 64 * s, to + buf + 1024u * i); };
+    auto fetch_x = [&](int i, int s) { request(x_off[i], xs + 64 * s, to_x + (uint32_t)(s & 1) * kMat + 1024u * i); };
+    auto fetch_w = [&](int i, int s, uint32_t buf) { request(w_off[i], ws + 64 * s, to_w + buf + 1024u * i); };
     const int wm = wave & 1, wn = wave >> 1;
-    f32x4_t acc[8][8];                                           // [tile of W][tile of rows]
+    f32x4_t acc[8][RT];                                          // [tile of W][tile of rows]
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < RT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const int steps = a.k / 64;
 #pragma unroll
     for (int i = 0; i < 8; ++i) fetch_w(i, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) fetch_x(i, 0);
+    for (int i = 0; i < RT; ++i) fetch_x(i, 0);
     if (steps > 1) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) fetch_w(i, 1, kMat);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) fetch_x(i, 1);
+        for (int i = 0; i < RT; ++i) fetch_x(i, 1);
     }
-    if (steps > 1) __builtin_amdgcn_s_waitcnt(0x4F70);           // step 0 has landed: 16 requests at most are under way
+    if (steps > 1) __builtin_amdgcn_s_waitcnt(RT == 8 ? 0x4F70 : 0x0F7C);        // step 0 has landed: 8 + RT requests at most are under way
     else __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
-    bf16x8_t xf[2][8], wf[2][8];
-    const unsigned char* xl = lds + 3 * kMat + 128 * 128 * wm + n * 128 + 16 * (g ^ (n & 7));
+    bf16x8_t xf[2][RT], wf[2][8];
+    const unsigned char* xl = lds + 3 * kMat + 128 * 16 * RT * wm + n * 128 + 16 * (g ^ (n & 7));
     const unsigned char* wl = lds + 128 * 128 * wn + n * 128 + 16 * (g ^ (n & 7));
     const int flip = 64 - 2 * (16 * (g ^ (n & 7)) & 64);         // from the unit of the first phase to that of the second
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         wf[0][i] = *reinterpret_cast<const bf16x8_t*>(wl + 2048 * i);
-        xf[0][i] = *reinterpret_cast<const bf16x8_t*>(xl + 2048 * i);
+        if (i < RT) xf[0][i] = *reinterpret_cast<const bf16x8_t*>(xl + 2048 * i);
     }
     // In place by assembly: all accumulation registers are taken, and the compiler, which moves results around, has none to move them through.
     // It does not know these for matrix instructions and so keeps no distance between them and others: operands come from LDS reads alone, which
@@ -588,21 +607,21 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
     auto product = [](f32x4_t& c, const bf16x8_t& w, const bf16x8_t& x) {
         __asm__ volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(w), "v"(x));
     };
-    // 64 products, with `aux(i)`, i < 32, behind two each
-    auto phase = [&](const bf16x8_t (&w)[8], const bf16x8_t (&x)[8], auto aux) {
+    // 8 RT products, with `aux(i)`, i < 4 RT, behind two each
+    auto phase = [&](const bf16x8_t (&w)[8], const bf16x8_t (&x)[RT], auto aux) {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int j = 0; j < 8; j += 2) {
+            for (int j = 0; j < RT; j += 2) {
                 product(acc[i][j], w[i], x[j]);
                 product(acc[i][j + 1], w[i], x[j + 1]);
-                aux(4 * i + j / 2);
+                aux(RT / 2 * i + j / 2);
                 __builtin_amdgcn_sched_barrier(0);
             }
     };
-    auto read = [&](bf16x8_t (&w)[8], bf16x8_t (&x)[8], const unsigned char* wb, const unsigned char* xb, int i) {
-        if (i < 8) x[i] = *reinterpret_cast<const bf16x8_t*>(xb + 2048 * i);
-        else if (i < 16) w[i - 8] = *reinterpret_cast<const bf16x8_t*>(wb + 2048 * (i - 8));
+    auto read = [&](bf16x8_t (&w)[8], bf16x8_t (&x)[RT], const unsigned char* wb, const unsigned char* xb, int i) {
+        if (i < RT) x[i] = *reinterpret_cast<const bf16x8_t*>(xb + 2048 * i);
+        else if (i < RT + 8) w[i - RT] = *reinterpret_cast<const bf16x8_t*>(wb + 2048 * (i - RT));
     };
     uint32_t at_w = 0, far_w = 2 * kMat;                         // buffers of W of this step and of the one after the next
     auto step = [&](int s, auto inner_tag) {
@@ -611,7 +630,7 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
         const unsigned char* wb = wl + at_w;
         phase(wf[0], xf[0], [&](int i) {
             if (kInner || s + 2 < steps)
-                if (i % 4 == 3) fetch_w(i / 4, s + 2, far_w);
+                if (i % (RT / 2) == RT / 2 - 1) fetch_w(i / (RT / 2), s + 2, far_w);
             read(wf[1], xf[1], wb + flip, xb + flip, i);
         });
         far_w = at_w;
@@ -632,10 +651,10 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
     };
     auto settle = [&] {                                          // of accumulators: what is in front of this and behind it stays there
 #pragma unroll
-        for (int i = 0; i < 64; ++i) __asm__ volatile("" : "+a"(acc[i >> 3][i & 7]));
+        for (int i = 0; i < 8 * RT; ++i) __asm__ volatile("" : "+a"(acc[i / RT][i % RT]));
         __asm__ volatile("s_nop 15\n\ts_nop 15");
 #pragma unroll
-        for (int i = 0; i < 64; ++i) __asm__ volatile("" : "+a"(acc[i >> 3][i & 7]));
+        for (int i = 0; i < 8 * RT; ++i) __asm__ volatile("" : "+a"(acc[i / RT][i % RT]));
     };
     settle();
     int s = 0;
@@ -648,9 +667,9 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
     constexpr int kCols = GATED ? 64 : 128, kPitch = 2 * kCols + 16, kRowLanes = kCols / 8;
     static_assert(4 * 128 * kPitch <= kBlockLds, "room in LDS");
     __syncthreads();                                             // everybody has read the last step's operands
-    unsigned char* own = lds + wave * 128 * kPitch;
+    unsigned char* own = lds + wave * 16 * RT * kPitch;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < RT; ++j)
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             if (GATED && (i & 2)) continue;
@@ -666,11 +685,18 @@ __device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, con
         }
     const int c = c0 + kCols * wn + 8 * (lane % kRowLanes);
 #pragma unroll
-    for (int i = 0; i < 128 * kRowLanes / 64; ++i) {
-        const int in = 64 / kRowLanes * i + lane / kRowLanes, r = 128 * wm + in;
+    for (int i = 0; i < 16 * RT * kRowLanes / 64; ++i) {
+        const int in = 64 / kRowLanes * i + lane / kRowLanes, r = 16 * RT * wm + in;
         const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(own + in * kPitch + 16 * (lane % kRowLanes));
         if (r < rows && c < a.out_cols) *reinterpret_cast<bf16x8_t*>(a.out + (int64_t)(first + r) * a.out_stride + c) = v;       // out_cols is a multiple of eight
     }
+}
+
+// Whole units, and those of at most half the rows: a step's requests of W are the same, its products half as many
+template <bool GATED>
+__device__ __forceinline__ void moe_block_product(const GemmArgs<__bf16>& a, const BlockUnit& u, unsigned char* lds) {
+    if (u.rows > kBlockRows / 2) moe_block_tiles<GATED, 8>(a, u, lds);
+    else moe_block_tiles<GATED, 4>(a, u, lds);
 }
 
 template <bool GATED>
@@ -887,7 +913,7 @@ int gemm(GemmArgs<T>& a, bool gated, int tile_rows, int64_t tokens, int64_t choi
         }
         if (tile_rows == kBlockRows) {
             a.col_blocks = (int)block_columns;
-            grid = (a.max_tiles * block_columns + 7) / 8 * 8;
+            grid = (a.max_tiles * block_columns + 7) / 8 * 8 + 8 * (kDieUnits / 2);
             if (grid > 0x7fffffff) return INFER_KV_EINVAL;
             if (gated) hipLaunchKernelGGL((moe_block_kernel<true>), dim3((unsigned)grid), dim3(kBlockThreads), 0, st, a);
             else hipLaunchKernelGGL((moe_block_kernel<false>), dim3((unsigned)grid), dim3(kBlockThreads), 0, st, a);

@@ -639,6 +639,23 @@ def test_moe_when_all_tokens_want_the_same_expert(gpu):
     close(x, y * (p[:, 4] / p.sum(-1))[:, None], 2e-2)
 
 
+@pytest.mark.parametrize("width,ff,n", [(64, 7680, 600), (64, 7680, 2000), (64, 7680, 2305), (64, 7680, 2176), (192, 1088, 640), (64, 2624, 1665), (8000, 64, 513), (1088, 192, 897)])
+def test_moe_blocks_of_the_last_round(gpu, width, ff, n):
+    """Blocks of 256 rows, none to 31 a die behind its last whole round, in halves or whole; a last block of a row, half a block and on; columns that end inside a
+    block; one to 125 steps.  Bounds as below."""
+    rng, bf = np.random.default_rng(n), torch.bfloat16
+    s = ho.MoeShape(width, ff, 1, 1, 0, 1, 1, 1.0)
+    router = np.ones((1, width))
+    gate, up = rounded(rng.standard_normal((2, ff, width)) * width ** -0.5, bf)
+    down = rounded(rng.standard_normal((width, ff)) * ff ** -0.5, bf)
+    h = rounded(rng.standard_normal((n, width)), bf)
+    r = ho.moe(s, dev(h, bf), dev(router, bf), torch.zeros(1, device=gpu), dev(np.concatenate([gate, up])[None], bf), dev(down[None], bf),
+               torch.zeros(1, dtype=torch.int32, device=gpu))
+    x = torch.zeros((n, width), device=gpu)
+    ho.pre_norm(x, torch.ones(width, device=gpu), 1e-6, y=r)
+    close(x, (silu(h @ gate.T) * (h @ up.T)) @ down.T, 2e-2)
+
+
 @pytest.mark.parametrize("width,ff,experts,n", [(256, 64, 5, 2600), (64, 5120, 8, 300), (64, 5120, 2, 800), (448, 384, 1, 4700)])
 def test_moe_blocks_of_uneven_experts(gpu, width, ff, experts, n):
     """Blocks of 256 rows: nearly all rows at one expert, in one and more groups of its tiles; few rows and many columns; one to seven steps.  300 rows of eight
