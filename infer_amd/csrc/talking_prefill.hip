@@ -39,8 +39,8 @@ constexpr float kBound = 100.f;           // log2 units: powers of scores below 
 // others, and a launch is done when its last workgroup is.  Sorted: units of `run` neighbouring blocks in falling order of the steps of their last one, over all
 // sequences, dealt to the dies in turn, so that a unit's blocks share what the L2 of their die holds.  Walks of more than `most` steps are cut into parts of one
 // length (at most `splits`), which are turns of their own.  Otherwise blocks by their place in their sequences.  The call, us, before (blocks by their place in
-// their sequences, walks whole, or all cut alike where blocks are few) / now: 8 sequences of 700 .. 2300 tokens 320 / 297, 6 of 1214 .. 2313 307 / 272, one of 6000 534 / 431,
-// one of 600 49 / 35, 16 of 100 .. 1500 226 / 210, 4 of 500 .. 1500 behind 1500 cached 330 / 270, 64 of 61 .. 179 65 / 58 (5 .. 7 of each by the order of loads and
+// their sequences, walks whole, or all cut alike where blocks are few) / now: 8 sequences of 700 .. 2300 tokens 320 / 290, 6 of 1214 .. 2313 307 / 264, one of 6000 534 / 431,
+// one of 600 49 / 35, 16 of 100 .. 1500 226 / 206, 4 of 500 .. 1500 behind 1500 cached 330 / 270, 64 of 61 .. 179 65 / 58 (5 .. 7 of each by the order of loads and
 // the rows at the end of talk_mix_kernel).  Runs of 1, 2, 4, 8 blocks: 8 of 700 .. 2300 263, 261,
 // 265, 272 (the same inputs again and again).
 constexpr int kLanes = 64;
@@ -665,7 +665,10 @@ Plan plan(int64_t heads, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q,
         }
     // few queries: more wavefronts with fewer of them each
     p.sums = Turns{(max_seqlen_q + 63) / 64 * num_seqs * heads < 2048 ? 128 : 256, 1, (int)steps, 1, true, 0};
-    if (bounded && orders) {               // no walk longer than what a place for a wavefront has to do, eight of a unit
+    // Few workgroups: no walk longer than what a place for a wavefront has to do, eight of a unit.  More even out by themselves, and parts cost each what it takes
+    // to begin; the call, us, cut / whole: 400 workgroups (one sequence of 6000) 431 / 468, 240 (2 of 900 .. 1000) 62.5 / 68.7, 660 (6 of 1214 .. 2313) 274 / 265, 820 (8 of
+    // 700 .. 2300) 303 / 294, 930 (16 of 100 .. 1500) 213 / 209, 960 (32 of 100 .. 600) 126 / 123.
+    if (bounded && orders && ((double)tokens / p.sums.queries + 0.5 * num_seqs) * heads <= 2 * kUnits) {
         const int64_t n = std::max<int64_t>({8, (int64_t)((double)tokens / 64 * heads * seen / (8 * kUnits)) + 1, (steps + 7) / 8});
         if (5 * n <= 4 * steps) {
             p.sums.most = (int)n;
