@@ -569,38 +569,45 @@ __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_pe
     constexpr int kOutRow = 32 * VT + 16, kRowLanes = 4 * VT;    // bytes; lanes that write a row
     static_assert(kMixWaves * 16 * kOutRow <= Q * kStep * kRec + Q * HP * 2 * kStep, "room in LDS");
     unsigned char* obuf = lds + wave * 16 * kOutRow;
+    // The lane number is made anew: what is worked out of it is otherwise kept from before the walk, in registers that the walk is short of
+    // (the form for 17 to 32 heads of 128: 81 spilled registers, 12 to 14 of them met in a step, against 18 and 3 or 4; 32 heads, 8 x 2048 1003 / 701 us, 64 sequences
+    // of 61 .. 179 tokens 131 / 95).
+    auto finish = [&](int lane, int g, int n) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < UH; ++u) {
-        const int h = wave * UH + u;
-        if (h >= a.heads) continue;
+        for (int u = 0; u < UH; ++u) {
+            const int h = wave * UH + u;
+            if (h >= a.heads) continue;
 #pragma unroll
-        for (int t = 0; t < QT; ++t) {
-            const int qi = q0 + 16 * t + n;
-            if (parts > 1) {
-                if (qi >= sq) continue;
-                float* part = a.part + (((int64_t)split * a.tokens + q_beg + qi) * a.heads + h) * a.vdim + 4 * g;
+            for (int t = 0; t < QT; ++t) {
+                const int qi = q0 + 16 * t + n;
+                if (parts > 1) {
+                    if (qi >= sq) continue;
+                    float* part = a.part + (((int64_t)split * a.tokens + q_beg + qi) * a.heads + h) * a.vdim + 4 * g;
 #pragma unroll
-                for (int v = 0; v < VT; ++v)
-                    if (16 * v + 4 * g < a.vdim) *reinterpret_cast<f32x4_t*>(part + 16 * v) = acc[u][t][v];
-                continue;
-            }
+                    for (int v = 0; v < VT; ++v)
+                        if (16 * v + 4 * g < a.vdim) *reinterpret_cast<f32x4_t*>(part + 16 * v) = acc[u][t][v];
+                    continue;
+                }
 #pragma unroll
-            for (int v = 0; v < VT; ++v) {
-                bf16x4_t x;
+                for (int v = 0; v < VT; ++v) {
+                    bf16x4_t x;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = (__bf16)(acc[u][t][v][e] * a.out_scale);
-                *reinterpret_cast<bf16x4_t*>(obuf + n * kOutRow + 32 * v + 8 * g) = x;
-            }
-            const int row = lane / kRowLanes, col = 4 * (lane % kRowLanes);
+                    for (int e = 0; e < 4; ++e) x[e] = (__bf16)(acc[u][t][v][e] * a.out_scale);
+                    *reinterpret_cast<bf16x4_t*>(obuf + n * kOutRow + 32 * v + 8 * g) = x;
+                }
+                const int row = lane / kRowLanes, col = 4 * (lane % kRowLanes);
 #pragma unroll
-            for (int i = 0; i < 16 * kRowLanes / 64; ++i) {
-                const int r = row + 64 / kRowLanes * i;
-                const bf16x4_t x = *reinterpret_cast<const bf16x4_t*>(obuf + r * kOutRow + 2 * col);
-                if (q0 + 16 * t + r < sq && col < a.vdim)
-                    *reinterpret_cast<bf16x4_t*>(a.out + (int64_t)(q_beg + q0 + 16 * t + r) * a.out_stride + (int64_t)h * a.vdim + col) = x;
+                for (int i = 0; i < 16 * kRowLanes / 64; ++i) {
+                    const int r = row + 64 / kRowLanes * i;
+                    const bf16x4_t x = *reinterpret_cast<const bf16x4_t*>(obuf + r * kOutRow + 2 * col);
+                    if (q0 + 16 * t + r < sq && col < a.vdim)
+                        *reinterpret_cast<bf16x4_t*>(a.out + (int64_t)(q_beg + q0 + 16 * t + r) * a.out_stride + (int64_t)h * a.vdim + col) = x;
+                }
             }
         }
-    }
+    };
+    const int late = renewed(lane);
+    finish(late, late >> 4, late & 15);
 }
 
 // Sums of the parts of walks that were cut.  Workgroup: a token.
