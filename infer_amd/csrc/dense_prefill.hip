@@ -49,31 +49,47 @@ struct DensePrefillArgs {
 };
 
 // Results of a wavefront's queries: denominators (and the sink's), the difference of two maps and its norm, the gate.  A lane has 8 bytes of every 32 of a query's
-// row: 16 rows at a time go through `own`, the wavefront's part of LDS that nobody reads any more, and are written a row in one piece.
-// Us, before / now: two maps, 6 sequences of 1100 to 3000 tokens 327 / 324.5, 30 of 100 to 400 97 / 94; 8 x 2048 284 / 274, one of 1800 29.0 / 27.8, 20 of 200 to 600 62 / 60.
+// row.  ROWS: 16 rows at a time go through `own`, the wavefront's part of LDS that nobody reads any more, and are written a row in one piece.
+// The ring kernel, us, as they lie / in rows: two maps, 6 sequences of 1100 to 3000 tokens 299 / 294; one map, a window 195 / 184, a bias 255 / 252, keys of 64 104 / 101.
+// dense_prefill_kernel takes rows for one map and values of 65 to 128 (keys of 192 179 / 174, of 256 353 / 346) and results as they lie elsewhere, where the compiler
+// makes less of its loop with rows: two maps of 128 (four registers spilled, eight accesses in a pair of steps) 8 x 2048 426 / 433, 6 of 1100 to 3000 571 / 583, of 96
+// with values of 64 390 / 411, of 64 with 64 226 / 233; one map, values of 64 and keys of 64 166 / 174, of 128 253 / 261.
 constexpr int out_bytes(int vt) { return 16 * (32 * vt + 16); }
-template <int VT, int MAPS>
+template <int VT, int MAPS, bool ROWS>
 __device__ __forceinline__ void finish(const DensePrefillArgs& a, f32x4_t (&acc)[2][VT], const f32x4_t (&lacc)[2], const float (&m_neg)[2], int q_beg, int q0,
-                                       int sq, int h, int lane, unsigned char* own) {
-    constexpr int kPitch = out_bytes(VT) / 16, kLanes = 4 * VT;
-    const int g = lane >> 4, n = lane & 15, row = lane / kLanes, col = 4 * (lane % kLanes);
-    auto store = [&](int first, auto value) {
+                                       int sq, int h, int lane, int g, int n, unsigned char* own) {
+    auto store = [&](int first, auto value) {                    // queries first .. first + 15
+        if constexpr (ROWS) {
+            constexpr int kPitch = out_bytes(VT) / 16, kLanes = 4 * VT;
+            const int row = lane / kLanes, col = 4 * (lane % kLanes);
 #pragma unroll
-        for (int t = 0; t < VT; ++t) {
-            bf16x4_t v;
+            for (int t = 0; t < VT; ++t) {
+                bf16x4_t v;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (__bf16)value(t, e);
-            *reinterpret_cast<bf16x4_t*>(own + n * kPitch + 32 * t + 8 * g) = v;
-        }
-        __bf16* o = a.out + (int64_t)(q_beg + first + row) * a.out_stride + (int64_t)h * a.vdim + col;
+                for (int e = 0; e < 4; ++e) v[e] = (__bf16)value(t, e);
+                *reinterpret_cast<bf16x4_t*>(own + n * kPitch + 32 * t + 8 * g) = v;
+            }
+            __bf16* o = a.out + (int64_t)(q_beg + first + row) * a.out_stride + (int64_t)h * a.vdim + col;
 #pragma unroll
-        for (int i = 0; i < kLanes / 4; ++i) {
-            const int r = 64 / kLanes * i;
-            const bf16x4_t v = *reinterpret_cast<const bf16x4_t*>(own + (r + row) * kPitch + 2 * col);
-            if (first + r + row < sq && col < a.vdim) *reinterpret_cast<bf16x4_t*>(o + (int64_t)r * a.out_stride) = v;
+            for (int i = 0; i < kLanes / 4; ++i) {
+                const int r = 64 / kLanes * i;
+                const bf16x4_t v = *reinterpret_cast<const bf16x4_t*>(own + (r + row) * kPitch + 2 * col);
+                if (first + r + row < sq && col < a.vdim) *reinterpret_cast<bf16x4_t*>(o + (int64_t)r * a.out_stride) = v;
+            }
+        } else {
+            __bf16* o = a.out + (int64_t)(q_beg + first + n) * a.out_stride + (int64_t)h * a.vdim + 4 * g;
+#pragma unroll
+            for (int t = 0; t < VT; ++t)
+                if (16 * t + 4 * g < a.vdim) {
+                    bf16x4_t v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = (__bf16)value(t, e);
+                    *reinterpret_cast<bf16x4_t*>(o + 16 * t) = v;
+                }
         }
     };
-    auto gate_of = [&](int qi) { return a.gate ? sigmoid_f((float)a.gate[(int64_t)(q_beg + (qi < sq ? qi : sq - 1)) * a.gate_stride + h]) : 1.f; };
+    // of a query; rows that are not written take the last one's
+    auto gate_of = [&](int qi) { return a.gate ? sigmoid_f((float)a.gate[(int64_t)(q_beg + (ROWS && qi >= sq ? sq - 1 : qi)) * a.gate_stride + h]) : 1.f; };
     if constexpr (MAPS == 2) {
         const float f0 = lacc[0][0] > 0.f ? 1.f / lacc[0][0] : 0.f, f1 = lacc[1][0] > 0.f ? -a.lambda / lacc[1][0] : 0.f;
         float ss = 0.f;
@@ -86,14 +102,18 @@ __device__ __forceinline__ void finish(const DensePrefillArgs& a, f32x4_t (&acc)
             }
         ss += __shfl_xor(ss, 16, 64);
         ss += __shfl_xor(ss, 32, 64);
-        const float f = rsqrtf(ss / (float)a.vdim + a.eps) * a.out_scale * gate_of(q0 + n);
+        const int qi = q0 + n;
+        if (!ROWS && qi >= sq) return;
+        const float f = rsqrtf(ss / (float)a.vdim + a.eps) * a.out_scale * gate_of(qi);
         store(q0, [&](int t, int e) { return acc[0][t][e] * f; });
     } else {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
+            const int qi = q0 + 16 * u + n;
+            if (!ROWS && qi >= sq) continue;
             float l = lacc[u][0];
             if (a.sink && l > 0.f) l += __builtin_amdgcn_exp2f(a.sink[h] * kLog2e + m_neg[u]);
-            const float f = (l > 0.f ? a.out_scale / l : 0.f) * gate_of(q0 + 16 * u + n);
+            const float f = (l > 0.f ? a.out_scale / l : 0.f) * gate_of(qi);
             store(q0 + 16 * u, [&](int t, int e) { return acc[u][t][e] * f; });
         }
     }
@@ -305,7 +325,13 @@ __global__ void __launch_bounds__(64 * kWaves, 2) dense_prefill_kernel(DensePref
         if (s + 1 < nsteps) step(s + 1, lds + kBuf, lds, st1, st0);
     }
     static_assert(kWaves * out_bytes(VT) <= sizeof(lds), "room in LDS");
-    if (live) finish<VT, MAPS>(a, acc, lacc, m_neg, q_beg, q0, sq, h, renewed(lane), lds + wave * out_bytes(VT));
+    if (!live) return;
+    if constexpr (MAPS == 1 && VT == 8) {
+        const int late = renewed(lane);
+        finish<VT, MAPS, true>(a, acc, lacc, m_neg, q_beg, q0, sq, h, late, late >> 4, late & 15, lds + wave * out_bytes(VT));
+    } else {
+        finish<VT, MAPS, false>(a, acc, lacc, m_neg, q_beg, q0, sq, h, lane, g, n, nullptr);
+    }
 }
 
 // The same for keys of at most 128 entries (two maps: 64 each) without a part that all heads share, and values of 65 to 128: tiles of keys
@@ -552,7 +578,9 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     if (s < nsteps) step(s, B0{}, B2{}, Outer{});
     if (s + 1 < nsteps) step(s + 1, B1{}, B0{}, Outer{});
     static_assert(kWaves * out_bytes(VT) <= sizeof(lds), "room in LDS");
-    if (live) finish<VT, MAPS>(a, acc, lacc, m_neg, q_beg, q0, sq, h, renewed(lane), lds + wave * out_bytes(VT));
+    if (!live) return;
+    const int late = renewed(lane);
+    finish<VT, MAPS, true>(a, acc, lacc, m_neg, q_beg, q0, sq, h, late, late >> 4, late & 15, lds + wave * out_bytes(VT));
 }
 
 // (k-steps, value tiles) the kernel is built for, smallest first

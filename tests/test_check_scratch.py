@@ -29,7 +29,8 @@ def test_a_kernel_that_is_not_there():
     assert check_scratch.check("", {"walk": 100})
 
 
-@pytest.mark.parametrize("source,limits", [("talking_prefill", {"talk_mix_kernelILi4ELi8ELi4E": 20, "talk_mix_kernel": 9, "talk_lse_kernel": 0})])
+@pytest.mark.parametrize("source,limits", [("talking_prefill", {"talk_mix_kernelILi4ELi8ELi4E": 20, "talk_mix_kernel": 9, "talk_lse_kernel": 0}),
+                                           ("dense_prefill", {"dense_prefill_kernelILi8E": 33, "dense_prefill": 0})])
 def test_last_build(source, limits):
     path = os.path.join(CSRC, source + ".resources.txt")
     if not os.path.exists(path):
