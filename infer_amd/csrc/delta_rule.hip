@@ -1213,14 +1213,15 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
     __syncthreads();
     // Loops of their own for wavefronts with columns and for others: where they met, the state would be copied.  Of the two wavefronts of a
     // vector unit the older one is served first, and the other one is alone for the rest of a step, when nothing covers its latencies (4500 and 6900
-    // clocks): so the younger ones go first until U, the older ones behind it.  8 portions of 500 .. 2600 tokens, 32 heads, the call 737 -> 718 us, 16 of
+    // clocks): so the younger ones go first until U, the older ones behind it, if they have columns (heads of 64 x 64, where none of them has: 401 -> 383, of 128 x 64
+    // 661 -> 647).  8 portions of 500 .. 2600 tokens, 32 heads, the call 737 -> 718 us, 16 of
     // 800 645 -> 637, 16 heads with 11 of 300 .. 1500 378 -> 365.  Half of the wavefronts with the next record behind the products instead: 734; the products
     // alone or the next record alone ahead: 733, 739.
     auto walk = [&](auto owner) __attribute__((always_inline)) {
         constexpr bool LIVE = decltype(owner)::value;
         for (int c = 0; c < p.chunks; ++c) {
             const WideBuffer buf{lds + (c & 1) * wide_buffer_units(DT), KS};
-            if (vt >= 4) __builtin_amdgcn_s_setprio(1);
+            if (LIVE && vt >= 4) __builtin_amdgcn_s_setprio(1);
             f32x4_t u = v;
             if (c + 1 < p.chunks) {
                 v = vn;
