@@ -1242,12 +1242,12 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
                 u32x4_t w[KS][3], qv[KS][3];
                 auto part = [&](int kk) {
                     const float f[8] = {s[2 * kk][0], s[2 * kk][1], s[2 * kk][2], s[2 * kk][3], s[2 * kk + 1][0], s[2 * kk + 1][1], s[2 * kk + 1][2], s[2 * kk + 1][3]};
-    #pragma unroll
+#pragma unroll
                     for (int i = 0; i < 3; ++i) { w[kk][i] = buf.wq(0, kk, i)[lane]; qv[kk][i] = buf.wq(1, kk, i)[lane]; }
                     split3<8>(f, pc[kk]);
                 };
                 part(0);
-    #pragma unroll
+#pragma unroll
                 for (int kk = 0; kk < KS; ++kk) {
                     const bf16x8_t sh = frag(pc[kk][0]), sm = frag(pc[kk][1]), sl = frag(pc[kk][2]);
                     if (kk + 1 < KS) part(kk + 1);
@@ -1282,26 +1282,26 @@ __global__ void __launch_bounds__(512, 2) delta_scan_wide_kernel(DeltaArgs<T> a,
                 const f32x4_t* e = reinterpret_cast<const f32x4_t*>(buf.e());
                 u32x4_t k0[DT], k1[DT];
                 f32x4_t ds[DT], et[DT];
-    #pragma unroll
+#pragma unroll
                 for (int t = 0; t < DT; ++t) {
                     k0[t] = buf.k(t, 0)[lane];
                     k1[t] = buf.k(t, 1)[lane];
                     et[t] = e[4 * t + q];
                 }
-    #pragma unroll
+#pragma unroll
                 for (int t = 0; t < DT; ++t) ds[t] = mma(k1[t], ulh, f32x4_t{0.f, 0.f, 0.f, 0.f});
-    #pragma unroll
+#pragma unroll
                 for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], umm, ds[t]);
-    #pragma unroll
+#pragma unroll
                 for (int t = 0; t < DT; ++t) ds[t] = mma(k0[t], uhh, ds[t]);
-    #pragma unroll
+#pragma unroll
                 for (int t = 0; t < DT; ++t) {
-    #pragma unroll
+#pragma unroll
                     for (int r = 0; r < 4; ++r) s[t][r] = __builtin_fmaf(s[t][r], et[t][r], ds[t][r]);
                 }
                 const f32x4_t o = o1 + (o2 + o3);
                 float* to = outputs + ((c & 1) * 16 + 4 * q) * kPitch + 16 * vt + m;
-    #pragma unroll
+#pragma unroll
                 for (int r = 0; r < 4; ++r) to[r * kPitch] = o[r];
             }
             __builtin_amdgcn_s_setprio(0);
