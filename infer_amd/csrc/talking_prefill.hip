@@ -630,46 +630,65 @@ __global__ void __launch_bounds__(256) talk_sum_kernel(TalkPrefillArgs a) {
 }
 
 constexpr int64_t kUnits = 256;
-// How long the mixture takes, in us as a model has it whose constants were fitted to its choices: `blocks` walks of all_steps steps together, the longest of
-// `longest`, walks longer than `part` steps cut.  As long as its longest part, as all work shared out over the compute units, or, where there are a few parts more than
-// units, as two of the short ones.  A workgroup takes `fixed` beside its steps (loads of the queries, the first step's way through LDS, stores), and more if it
-// leaves a part.  29 batches (1 sequence of 190 .. 6000 tokens, 64 of 61 .. 179, 4 of 500 .. 1500 behind 1500 cached ones ...), 18 cuts of each: what this chooses takes
-// 0.6 % longer than the best of them, 9 % at most.
-double mix_time(double blocks, double longest, double all_steps, int part, double fixed, double step) {
-    const bool cut = part < longest;
-    const float shape = 1.f / std::max((float)(longest * blocks / all_steps) - 1.f, 0.05f);
-    auto above = [&](double x) { return x >= longest ? 0. : 1. - (double)std::pow((float)(x / longest), shape); };     // share of the walks that are longer than x steps
-    const double left = cut ? 5. : 0.;
-    double pieces = blocks;
-    for (double x = part; x < longest; x += part) pieces += blocks * above(x);
-    const double all = (cut ? 1.39 : 1.53) / kUnits * (pieces * fixed + (pieces - blocks * (1. - above(part))) * left + all_steps * step);
-    double t = std::max(fixed + left + part * step, all);
-    if (pieces > kUnits && pieces < 2 * kUnits) {
-        const double low = blocks * (1. - above(0.5 * part)), paired = 2. * (pieces - kUnits);      // walks of up to half a part
-        const double mean = paired <= low ? 0.25 * part * paired / low : (0.25 * part * low + 0.75 * part * (paired - low)) / paired;
-        t = std::max(t, 2. * (fixed + left + mean * step));
+// How long the mixture takes, in us as a model has it.  The walks of `blocks` workgroups, the longest of `longest` steps, are taken for eight lengths, `walks`, each of
+// an eighth of them; those of more than `most` steps are cut.  A workgroup takes cost.fixed beside its steps (loads of the queries, the first step's way through LDS,
+// stores), and kLeft more if it leaves a part.  The launch takes as long as its longest workgroup, as all work shared out over the units, and, since of the 256 k + 1
+// longest workgroups some k + 1 are on one unit, k + 1 times the shortest of these; parts are written and read once more, mb of them a workgroup.
+// The constants were fitted to what is chosen by them: 8, 16 and 32 heads of 128 and of 64 with 8 key heads, 16 and 32 ungrouped ones of 128, 40 batches each (1 to
+// 24 sequences of 190 to 6000 tokens, equal and unequal ones, 64 to 100 of up to 600, 4 to 200 with 64 to 1500 new tokens behind 100 to 8000 cached), every cut that
+// plan() looks at timed.  What it takes is 2.1 % longer than the best of them on average (16 heads of 128: 1.9 %), in nine of ten cases 6.6 % at most, 25 % at worst (100 sequences
+// with 64 new tokens behind 100 to 3000).  The call, us, with constants of 16 heads for all forms and nothing for what parts are in memory / now: 8 x 2048 with 8 heads
+// 251 / 225, 16 heads 343 / 327, 32 heads 706 / 643, 16 x 1000 with 8 heads 158 / 127, of 64 115 / 94, 4 x 2048 with 16 of 64 174 / 151, 64 with 64 new tokens behind 4000 and
+// 8, 16, 32 heads 363 / 343, 556 / 452, 863 / 687; 8 of 700 .. 2300 with 16 heads 279 / 280, 6 of 1214 .. 2313 254 / 262.
+constexpr int kShares = 8;
+constexpr double kLeft = 7.1, kBusy = 1.08, kBusyCut = 1.23, kTraffic = 0.56;
+struct Cost { double fixed, step; };
+// values of up to 64 and of more; 64 and 32 queries of up to 8 heads, 32 and 16 of up to 16, 16 of up to 32
+constexpr Cost kCosts[2][5] = {{{26.9, 3.63}, {18.7, 2.37}, {19.7, 4.26}, {5.6, 2.77}, {4.6, 2.31}}, {{25.8, 4.15}, {19.7, 2.89}, {19., 4.73}, {18.4, 3.35}, {12.3, 4.65}}};
+double mix_time(const double (&walks)[kShares], double blocks, int longest, int most, const Cost& cost, double mb) {
+    struct Piece { double time, count; } pieces[kShares];
+    double number = 0., work = 0., left = 0.;
+    for (int i = 0; i < kShares; ++i) {
+        const int parts = std::max(1, (int)std::ceil(walks[i] / most - 1e-9));
+        pieces[i] = {cost.fixed + (parts > 1 ? kLeft : 0.) + walks[i] / parts * cost.step, blocks / kShares * parts};
+        number += pieces[i].count;
+        work += pieces[i].count * pieces[i].time;
+        if (parts > 1) left += pieces[i].count;
     }
-    return t + 0.09 * std::min(part * step, all) + (cut ? 4.7 : 0.);
+    double t = std::max(cost.fixed + (most < longest ? kLeft : 0.) + most * cost.step, (most < longest ? kBusyCut : kBusy) / kUnits * work);
+    if (number > kUnits) {
+        std::sort(pieces, pieces + kShares, [](const Piece& a, const Piece& b) { return a.time > b.time; });
+        double longer = 0.;
+        int rounds = 1;
+        for (const Piece& p : pieces)
+            for (longer += p.count; rounds < 4 && longer > rounds * kUnits; ++rounds) t = std::max(t, (rounds + 1) * p.time);
+    }
+    return t + kTraffic * mb * left;
 }
 struct Plan { Turns turns, sums; };
-Plan plan(int64_t heads, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q, int64_t max_keys, bool bounded) {
+Plan plan(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q, int64_t max_keys, bool bounded) {
     Plan p;
     const int64_t steps = (max_keys + kStep - 1) / kStep;
     // a token's sequence is about as long as the mean of the mean and the longest one, and it is in its middle
     const double seen = ((double)(max_keys - max_seqlen_q) + 0.25 * ((double)tokens / num_seqs + (double)max_seqlen_q)) / kStep + 0.5;
+    double walks[kShares];
+    for (int i = 0; i < kShares; ++i) walks[i] = std::max(1., (double)steps * std::pow((kShares - i - 0.5) / kShares, std::max((double)steps / seen - 1., 0.004)));
     const int wide = heads <= 8 ? 4 : heads <= 16 ? 2 : 1, narrow = heads <= 8 ? 2 : 1;
     const bool orders = num_seqs <= kLanes && max_keys <= kMostKeys;
     double best = 0.;
-    for (int tiles = wide; tiles >= narrow; tiles /= 2)
-        for (const double share : {1., 0.8, 0.65, 0.5, 0.4, 0.33, 0.25, 0.17, 0.125}) {
-            const int64_t most = std::min(std::max<int64_t>({4, (int64_t)(share * (double)steps), (steps + 7) / 8}), steps);
+    for (int tiles = wide; tiles >= narrow; tiles /= 2) {
+        const int queries = 16 * tiles;
+        const double blocks = std::min((double)tokens / queries + 0.5 * num_seqs, (double)((max_seqlen_q + queries - 1) / queries) * num_seqs);
+        const Cost& cost = kCosts[vdim > 64][(heads <= 8 ? 0 : heads <= 16 ? 2 : 4) + (tiles < wide)];
+        for (const double share : {1., 0.8, 0.65, 1. / 2, 0.4, 1. / 3, 1. / 4, 1. / 6, 1. / 8}) {
+            const int64_t most = std::min(std::max<int64_t>(4, (int64_t)std::ceil(share * (double)steps - 1e-9)), steps);
             if (most < steps && !orders) break;
-            const double blocks = (double)tokens / (16 * tiles) + 0.5 * num_seqs;
-            const double t = mix_time(blocks, (double)steps, blocks * seen, (int)most, tiles == wide ? 18.8 : 6.65, tiles == wide ? 2.06 : 1.68);
+            const double t = mix_time(walks, blocks, (int)steps, (int)most, cost, 4e-6 * (double)(queries * heads * vdim));
             if (best > 0. && t >= best) continue;
             best = t;
-            p.turns = Turns{16 * tiles, 2, (int)most, (int)((steps + most - 1) / most), true, 0};
+            p.turns = Turns{queries, 2, (int)most, (int)((steps + most - 1) / most), true, 0};
         }
+    }
     // few queries: more wavefronts with fewer of them each
     p.sums = Turns{(max_seqlen_q + 63) / 64 * num_seqs * heads < 2048 ? 128 : 256, 1, (int)steps, 1, true, 0};
     // Few workgroups: no walk longer than what a place for a wavefront has to do, eight of a unit.  More even out by themselves, and parts cost each what it takes
@@ -749,7 +768,7 @@ extern "C" int infer_talking_prefill_supported(int64_t heads, int64_t dim, int64
 extern "C" int64_t infer_talking_prefill_workspace_floats(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q,
                                                           int64_t max_keys) {
     if (heads < 1 || vdim < 1 || num_seqs < 1 || tokens < 1 || max_seqlen_q < 1 || max_keys < 1) return 0;
-    const Plan p = plan(heads, num_seqs, tokens, max_seqlen_q, max_keys, true);
+    const Plan p = plan(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys, true);
     const int64_t lse = (p.sums.splits * heads * tokens + 3) / 4 * 4;
     return lse + (p.turns.splits > 1 ? p.turns.splits * tokens * heads * vdim : 0);
 }
@@ -777,7 +796,7 @@ extern "C" int infer_talking_prefill(const void* q, int64_t q_stride, const void
         workspace_floats < infer_talking_prefill_workspace_floats(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys))
         return INFER_KV_EWORKSPACE;
     const bool bounded = max_score * kLog2e <= kBound;
-    const Plan p = plan(heads, num_seqs, tokens, max_seqlen_q, max_keys, bounded);
+    const Plan p = plan(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys, bounded);
     const TalkPrefillArgs a{(const __bf16*)q, q_stride, (const __bf16*)keys, (const __bf16*)values, (int)key_pad, (int)vdim_pad, block_table,
                             bt_stride, (int)table_cols, (int)block_size, (int)num_blocks, seqs, cu_q, cu_k, (int)heads, (int)kv_heads, (int)dim,
                             (int)vdim, (int)num_seqs, scale * kLog2e, (const __bf16*)talk, out_scale, (__bf16*)out, out_stride, workspace, tokens, p.turns,

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+from infer_amd import _lib
 from infer_amd.cache import LayeredLayout
 from infer_amd.config import Config, TuluraxConfig, load_model_config
 from infer_amd.layers import XieluMLP
@@ -264,3 +265,23 @@ def test_lanes_meet_all_banks(per_wave):
             for r0 in (0, 8):
                 units = {record_place(rec, q, row_token(r, x), q & 8) % 128 // 16 for r in range(r0, r0 + 8)}
                 assert len(units) == 8
+
+
+# ------------------------------------------------------------------ the prompt kernels' plan
+def workspace(heads, dim, seqs, tokens, longest, prefix=0):
+    """Floats in front of which nothing is cut: one a head and token."""
+    return _lib.load().infer_talking_prefill_workspace_floats(heads, dim, seqs, tokens, longest, longest + prefix)
+
+
+@pytest.mark.parametrize("heads", [8, 16, 32])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_walks_are_cut_where_that_evens_something_out(heads, dim):
+    """Equal sequences: short and long walks even out over the units as they are, and parts would go through memory.  A long sequence of its own and a few leave units idle."""
+    assert workspace(heads, dim, 8, 8 * 2048, 2048) == heads * 8 * 2048
+    assert workspace(heads, dim, 16, 16 * 1000, 1000) == heads * 16 * 1000
+    assert workspace(heads, dim, 1, 2048, 2048) >= 2 * 2048 * heads * dim
+    if heads < 32:
+        assert workspace(heads, dim, 4, 4000, 1500, 1500) >= 2 * 4000 * heads * dim
+        assert workspace(heads, dim, 64, 64 * 64, 64, 4000) >= 2 * 64 * 64 * heads * dim
+    elif dim == 128:                                             # 256 blocks of 16 queries: one for every unit
+        assert workspace(heads, dim, 64, 64 * 64, 64, 4000) == heads * 64 * 64
