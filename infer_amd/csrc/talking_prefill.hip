@@ -639,7 +639,7 @@ constexpr int64_t kUnits = 256;
 // plan() looks at timed.  What it takes is 2.1 % longer than the best of them on average (16 heads of 128: 1.9 %), in nine of ten cases 6.6 % at most, 25 % at worst (100 sequences
 // with 64 new tokens behind 100 to 3000).  The call, us, with constants of 16 heads for all forms and nothing for what parts are in memory / now: 8 x 2048 with 8 heads
 // 251 / 225, 16 heads 343 / 327, 32 heads 706 / 643, 16 x 1000 with 8 heads 158 / 127, of 64 115 / 94, 4 x 2048 with 16 of 64 174 / 151, 64 with 64 new tokens behind 4000 and
-// 8, 16, 32 heads 363 / 343, 556 / 452, 863 / 687; 8 of 700 .. 2300 with 16 heads 279 / 280, 6 of 1214 .. 2313 254 / 262.
+// 8, 16, 32 heads 363 / 343, 556 / 452, 863 / 687, and 65 of them whole / now 533 / 368, 681 / 595, 1340 / 1154; 8 of 700 .. 2300 with 16 heads 279 / 280, 6 of 1214 .. 2313 254 / 262.
 constexpr int kShares = 8;
 constexpr double kLeft = 7.1, kBusy = 1.08, kBusyCut = 1.23, kTraffic = 0.56;
 struct Cost { double fixed, step; };
@@ -674,7 +674,7 @@ Plan plan(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t
     double walks[kShares];
     for (int i = 0; i < kShares; ++i) walks[i] = std::max(1., (double)steps * std::pow((kShares - i - 0.5) / kShares, std::max((double)steps / seen - 1., 0.004)));
     const int wide = heads <= 8 ? 4 : heads <= 16 ? 2 : 1, narrow = heads <= 8 ? 2 : 1;
-    const bool orders = num_seqs <= kLanes && max_keys <= kMostKeys;
+    const bool orders = num_seqs <= kLanes && max_keys <= kMostKeys;       // walks of more sequences are cut as well, and go out as they lie
     double best = 0.;
     for (int tiles = wide; tiles >= narrow; tiles /= 2) {
         const int queries = 16 * tiles;
@@ -682,7 +682,6 @@ Plan plan(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t
         const Cost& cost = kCosts[vdim > 64][(heads <= 8 ? 0 : heads <= 16 ? 2 : 4) + (tiles < wide)];
         for (const double share : {1., 0.8, 0.65, 1. / 2, 0.4, 1. / 3, 1. / 4, 1. / 6, 1. / 8}) {
             const int64_t most = std::min(std::max<int64_t>(4, (int64_t)std::ceil(share * (double)steps - 1e-9)), steps);
-            if (most < steps && !orders) break;
             const double t = mix_time(walks, blocks, (int)steps, (int)most, cost, 4e-6 * (double)(queries * heads * vdim));
             if (best > 0. && t >= best) continue;
             best = t;
@@ -694,7 +693,7 @@ Plan plan(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t
     // Few workgroups: no walk longer than what a place for a wavefront has to do, eight of a unit.  More even out by themselves, and parts cost each what it takes
     // to begin; the call, us, cut / whole: 400 workgroups (one sequence of 6000) 431 / 468, 240 (2 of 900 .. 1000) 62.5 / 68.7, 660 (6 of 1214 .. 2313) 274 / 265, 820 (8 of
     // 700 .. 2300) 303 / 294, 930 (16 of 100 .. 1500) 213 / 209, 960 (32 of 100 .. 600) 126 / 123.
-    if (bounded && orders && ((double)tokens / p.sums.queries + 0.5 * num_seqs) * heads <= 2 * kUnits) {
+    if (bounded && ((double)tokens / p.sums.queries + 0.5 * num_seqs) * heads <= 2 * kUnits) {
         const int64_t n = std::max<int64_t>({8, (int64_t)((double)tokens / 64 * heads * seen / (8 * kUnits)) + 1, (steps + 7) / 8});
         if (5 * n <= 4 * steps) {
             p.sums.most = (int)n;

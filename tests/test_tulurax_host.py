@@ -285,3 +285,9 @@ def test_walks_are_cut_where_that_evens_something_out(heads, dim):
         assert workspace(heads, dim, 64, 64 * 64, 64, 4000) >= 2 * 64 * 64 * heads * dim
     elif dim == 128:                                             # 256 blocks of 16 queries: one for every unit
         assert workspace(heads, dim, 64, 64 * 64, 64, 4000) == heads * 64 * 64
+
+
+@pytest.mark.parametrize("heads,seqs", [(8, 64), (16, 64), (8, 65), (16, 65), (32, 65), (8, 80), (16, 80), (32, 80)])
+def test_walks_are_cut_however_many_sequences_there_are(heads, seqs):
+    """64 new tokens behind 4000: blocks of 16 to 64 queries with 126 steps each, 64 to 320 of them, for 256 compute units."""
+    assert workspace(heads, 128, seqs, 64 * seqs, 64, 4000) >= 64 * seqs * heads * (1 + 2 * 128)

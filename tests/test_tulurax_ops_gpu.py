@@ -372,10 +372,10 @@ def test_prefill_of_uneven_sequences_on_all_dies(gpu, heads, lens):
 @pytest.mark.parametrize("heads,new,cached,bounded", [
     (16, [0, 1300, 33, 1, 900, 700, 16, 17], [0] * 8, True), (16, [40, 700, 0, 260, 5], [1500, 0, 64, 333, 900], True), (16, [40, 700, 0, 260, 5], [1500, 0, 64, 333, 900], False),
     (8, [1, 600], [2000, 31], True), (16, [601], [0], True), (12, [150, 31], [500, 0], False), (32, [300, 0, 290], [800, 0, 17], True), (6, [640, 33] * 20, [0, 65] * 20, True),
-    (4, [30, 1, 0, 65] * 17, [600, 0, 0, 3] * 17, True)])
+    (4, [30, 1, 0, 65] * 17, [600, 0, 0, 3] * 17, True), (8, [64] * 66, [1500] * 66, True), (16, [64, 1, 0, 40] * 17, [1500, 2000, 7, 0] * 17, False)])
 def test_prefill_in_turns(gpu, heads, new, cached, bounded):
     """Blocks of queries in falling order of their walks, and as they lie where there are few, walks are short or sequences more than 64; walks cut into parts and
-    whole, sums of exponentials that were cut too and those that need a maximum; sequences without queries, behind cached keys and of one query."""
+    whole, in either order, sums of exponentials that were cut too and those that need a maximum; sequences without queries, behind cached keys and of one query."""
     rng, bf = np.random.default_rng(11), torch.bfloat16
     s = ho.TalkShape(heads, 2, 64, 64, 0.1, 0.0)
     lens = [a + b for a, b in zip(new, cached)]
