@@ -373,22 +373,30 @@ def test_prefill_of_uneven_sequences_on_all_dies(gpu, heads, lens):
     (16, [0, 1300, 33, 1, 900, 700, 16, 17], [0] * 8, True), (16, [40, 700, 0, 260, 5], [1500, 0, 64, 333, 900], True), (16, [40, 700, 0, 260, 5], [1500, 0, 64, 333, 900], False),
     (8, [1, 600], [2000, 31], True), (16, [601], [0], True), (12, [150, 31], [500, 0], False), (32, [300, 0, 290], [800, 0, 17], True), (6, [640, 33] * 20, [0, 65] * 20, True),
     (4, [30, 1, 0, 65] * 17, [600, 0, 0, 3] * 17, True), (8, [64] * 66, [1500] * 66, True), (16, [64, 1, 0, 40] * 17, [1500, 2000, 7, 0] * 17, False)])
-def test_prefill_in_turns(gpu, heads, new, cached, bounded):
+def test_prefill_in_turns(gpu, heads, new, cached, bounded, kv_heads=2, dim=64):
     """Blocks of queries in falling order of their walks, and as they lie where there are few, walks are short or sequences more than 64; walks cut into parts and
     whole, in either order, sums of exponentials that were cut too and those that need a maximum; sequences without queries, behind cached keys and of one query."""
     rng, bf = np.random.default_rng(11), torch.bfloat16
-    s = ho.TalkShape(heads, 2, 64, 64, 0.1, 0.0)
+    s = ho.TalkShape(heads, kv_heads, dim, dim, 0.1, 0.0)
     lens = [a + b for a, b in zip(new, cached)]
     p = Pages(rng, [max(n, 1) for n in lens], s, 32, bf)
     cu_q, cu_k = np.cumsum([0] + new), np.cumsum([0] + lens)
-    q = dev(rms_norm(rng.standard_normal((cu_q[-1], heads, 64)), 1.0, 0.0), bf)
+    q = dev(rms_norm(rng.standard_normal((cu_q[-1], heads, dim)), 1.0, 0.0), bf)
     talk = dev(mixing(rng, heads, bf), bf)
-    a, b = (torch.full((int(cu_q[-1]), heads * 64), float("nan"), dtype=bf, device=gpu) for _ in range(2))
-    ho.talking_prefill(s, q.view(-1, heads * 64), *p.pages, talk, p.tables, torch.arange(len(lens), dtype=torch.int32, device=gpu), dev(cu_q, torch.int32),
+    a, b = (torch.full((int(cu_q[-1]), heads * dim), float("nan"), dtype=bf, device=gpu) for _ in range(2))
+    ho.talking_prefill(s, q.view(-1, heads * dim), *p.pages, talk, p.tables, torch.arange(len(lens), dtype=torch.int32, device=gpu), dev(cu_q, torch.int32),
                        dev(cu_k, torch.int32), max(new), max(lens), a, max_score=s.max_score(max(lens)) if bounded else None)
     ctx = np.concatenate([np.arange(c + 1, c + n + 1) for n, c in zip(new, cached)])
     ho.talking_attention(s, q, *p.pages, talk, p.tables, dev(ctx, torch.int32), b, row_seq=dev(np.repeat(np.arange(len(lens)), new), torch.int32), max_keys=max(lens))
     close(a, host(b), 1.5e-2)
+
+
+@pytest.mark.parametrize("heads,kv_heads,new,cached", [(8, 8, [1500, 31, 2100], [2000, 0, 1500]), (8, 2, [600, 31, 900], [2000, 0, 1500]), (16, 8, [700, 0, 450], [900, 31, 0]),
+                                                       (16, 16, [700, 0, 450], [900, 31, 0]), (16, 2, [0, 1300, 33, 1, 900, 700, 16, 17], [0] * 8), (32, 8, [1030, 0, 33], [0, 50, 900]),
+                                                       (32, 32, [400, 0, 290], [800, 0, 17]), (20, 2, [700, 31], [500, 900])])
+def test_prefill_in_turns_of_wide_heads(gpu, heads, kv_heads, new, cached):
+    """Heads of 128 in every form of the mixture, whose walks go out in falling order and in parts, so that a wavefront keeps a part or writes rows behind either walk."""
+    test_prefill_in_turns(gpu, heads, new, cached, True, kv_heads, 128)
 
 
 def test_what_the_prompt_kernels_do_not_serve(gpu):
