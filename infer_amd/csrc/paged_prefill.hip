@@ -371,9 +371,11 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
         if (QB == 1 || s < my_steps) {   // wavefronts whose queries end earlier skip the keys they cannot see
         // ---- S^T = K Q^T for both query tiles.  The order of this step is written out: left alone, the compiler asks for each operand right in front of its
         // product, and puts all products behind all exponents.  Keys are asked for two k-steps ahead and values before the maxima, one branch asks for
-        // both query tiles whether sums have to be rescaled, and the second tile's exponents run between the first one's products.  The call, us:
-        // 16 sequences of 64 .. 2048 tokens, 32 heads 271 -> 261; one of 4000, 16 heads 106 -> 94; one of 8000, 32 heads 468 -> 439.
-        // (Scores of the next step between the exponents of this one, which takes 210 registers, so two wavefronts a vector unit: 286.)
+        // both query tiles whether sums have to be rescaled, and the second tile's exponents run between the first one's products.  The call with its
+        // front end, us, left alone / in this order / with results in rows too (below), in turn on one card, the shortest of five times ten: 16 sequences of 64 .. 2048 tokens, 32
+        // heads 294 / 281 / 263; one of 4000, 16 heads 112 / 99 / 97; one of 8000, 32 heads 497 / 470 / 466; 8 of 800 88 / 84 / 78; 30 of 300 .. 600 159 / 156 / 148; 5 of
+        // 70 .. 2900 141 / 134 / 127; 64 of 52 .. 101 51 / 51 / 45.  (Scores of the next step between the exponents of this one, which takes 210 registers, so two wavefronts a
+        // vector unit: 271 -> 286 where this order gave 261.)
         u32x4 kf[4][2];
         auto keys = [&](int j) {
 #pragma unroll
@@ -515,8 +517,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
 
     if (!live) return;
     // A lane has 8 bytes of every 32 of a query's row.  They go through the ring, in which nothing is read or under way any more, a wavefront's rows to a part
-    // of its own, and are written a row in one piece.  The call, us, before / now: 16 sequences of 64 .. 2048 tokens, 32 heads 294 / 290, 8 of 800 90 / 84, 30 of 300 .. 600 101 / 96,
-    // 5 of 70 .. 2900 146 / 141, one of 8000 474 / 471.
+    // of its own, and are written a row in one piece (times: at the scores).
     constexpr int kPitch = 2 * kD + 16;
     static_assert(WAVES * kQBlock * kPitch <= kRing * kTileBytes, "room in the ring");
     unsigned char* own = lds_all + wave * kQBlock * kPitch;

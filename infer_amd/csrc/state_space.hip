@@ -285,7 +285,7 @@ struct ChunkArgs {
 // as it lies, when the state rows of a k-step of 32 are taken in the order 16 tau + 4 g + e.  The 32 x 32 products C_i B_j are shared
 // out over the wavefronts of the first half, weighted, and exchanged through LDS; those of the second add up and write the results.
 // OUT = false: only the final state, from zero.  RAW: x comes as it entered the convolution, four taps, which is done here, of the next chunk while this one's products run (the
-// pass 175 -> 220 us under a profiler, the launch that it replaces took 54, the one of B and C that is left 7); the portion is one segment.
+// pass 175 -> 202 to 212 us under a profiler, the launch that it replaces took 54, the one of B and C that is left 11); the portion is one segment.
 // A portion takes as long as its chunks one after the other, and a chunk as long as one wavefront's instructions and reads of LDS (four
 // wavefronts: 445 and 30 reads, 3900 clocks with three barriers).  Eight halve what follows one another, and where two chunks lie in LDS one
 // barrier is left, behind which a chunk's results are finished under the next one's products.  6 portions of 900 to 3700 tokens of 64 heads,

@@ -38,11 +38,10 @@ constexpr float kBound = 100.f;           // log2 units: powers of scores below 
 // The order in which workgroups take blocks of queries.  A block sees as many keys as its place in its sequence says, so some take a hundred times as long as
 // others, and a launch is done when its last workgroup is.  Sorted: units of `run` neighbouring blocks in falling order of the steps of their last one, over all
 // sequences, dealt to the dies in turn, so that a unit's blocks share what the L2 of their die holds.  Walks of more than `most` steps are cut into parts of one
-// length (at most `splits`), which are turns of their own.  Otherwise blocks by their place in their sequences.  The call, us, before (blocks by their place in
-// their sequences, walks whole, or all cut alike where blocks are few) / now: 8 sequences of 700 .. 2300 tokens 320 / 290, 6 of 1214 .. 2313 307 / 264, one of 6000 534 / 431,
-// one of 600 49 / 35, 16 of 100 .. 1500 226 / 206, 4 of 500 .. 1500 behind 1500 cached 330 / 270, 64 of 61 .. 179 65 / 58 (5 .. 7 of each by the order of loads and
-// the rows at the end of talk_mix_kernel).  Runs of 1, 2, 4, 8 blocks: 8 of 700 .. 2300 263, 261,
-// 265, 272 (the same inputs again and again).
+// length (at most `splits`), which are turns of their own.  Otherwise blocks by their place in their sequences.  The call, us, 16 heads, by place in their sequences
+// with walks whole, or all cut alike where blocks are few / now (5 .. 7 of each by the order of loads and the rows at the end of talk_mix_kernel), in turn on one card, the
+// shortest of five times ten: 8 sequences of 700 .. 2300 tokens 311 / 281, 6 of 1214 .. 2313 285 / 256, one of 6000 503 / 403, one of 600 49 / 36, 16 of 100 .. 1500 218 / 200, 4 of
+// 500 .. 1500 behind 1500 cached 329 / 258, 64 of 61 .. 179 60 / 51.  Runs of 1, 2, 4, 8 blocks: 8 of 700 .. 2300 263, 261, 265, 272 (the same inputs again and again).
 constexpr int kLanes = 64;
 constexpr int kMostKeys = 1 << 30;      // of a sequence, so that numbers of steps can be doubled
 struct Turns { int queries, run, most, splits; bool sorted; int units; };      // queries of a block; run, queries: powers of two; units of the longest sequence
