@@ -638,7 +638,7 @@ constexpr int64_t kUnits = 256;
 // longest workgroups some k + 1 are on one unit, k + 1 times the shortest of these; parts are written and read once more, mb of them a workgroup.
 // The constants were fitted to what is chosen by them: 8, 16 and 32 heads of 128 and of 64 with 8 key heads, 16 and 32 ungrouped ones of 128, 40 batches each (1 to
 // 24 sequences of 190 to 6000 tokens, equal and unequal ones, 64 to 100 of up to 600, 4 to 200 with 64 to 1500 new tokens behind 100 to 8000 cached), every cut that
-// plan() looks at timed.  What it takes is 2.1 % longer than the best of them on average (16 heads of 128: 1.9 %), in nine of ten cases 6.6 % at most, 25 % at worst (100 sequences
+// mix_turns() looks at timed.  What it takes is 2.1 % longer than the best of them on average (16 heads of 128: 1.9 %), in nine of ten cases 6.6 % at most, 25 % at worst (100 sequences
 // with 64 new tokens behind 100 to 3000).  The call, us, with constants of 16 heads for all forms and nothing for what parts are in memory / now: 8 x 2048 with 8 heads
 // 251 / 225, 16 heads 343 / 327, 32 heads 706 / 643, 16 x 1000 with 8 heads 158 / 127, of 64 115 / 94, 4 x 2048 with 16 of 64 174 / 151, 64 with 64 new tokens behind 4000 and
 // 8, 16, 32 heads 363 / 343, 556 / 452, 863 / 687, and 65 of them whole / now 533 / 368, 681 / 595, 1340 / 1154; 8 of 700 .. 2300 with 16 heads 279 / 280, 6 of 1214 .. 2313 254 / 262.
@@ -667,52 +667,66 @@ double mix_time(const double (&walks)[kShares], double blocks, int longest, int 
     }
     return t + kTraffic * mb * left;
 }
-struct Plan { Turns turns, sums; };
-Plan plan(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q, int64_t max_keys, bool bounded) {
-    Plan p;
+// Finding a turn takes 1 to 2 us, which is not worth it where walks are short or all run at once: 24 sequences of 151 .. 441 78 us against 74, 23 of 67 .. 80
+// 28 against 25, but 32 of 100 .. 600 111 against 148.
+Turns arranged(Turns t, int64_t num_seqs, int64_t max_seqlen_q, int64_t max_keys, int64_t at_once) {
+    const int64_t blocks = (max_seqlen_q + t.queries - 1) / t.queries, steps = (max_keys + kStep - 1) / kStep;
+    t.sorted = num_seqs <= kLanes && max_keys <= kMostKeys && steps > 16 && t.splits * blocks * num_seqs > at_once;
+    if (!t.sorted) t.run = 1;
+    t.units = (int)((blocks + t.run - 1) / t.run);
+    return t;
+}
+// Steps of a token's walk: its sequence is about as long as the mean of the mean and the longest one, and it is in its middle
+double steps_seen(int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q, int64_t max_keys) {
+    return ((double)(max_keys - max_seqlen_q) + 0.25 * ((double)tokens / num_seqs + (double)max_seqlen_q)) / kStep + 0.5;
+}
+// Walks of more sequences than can be sorted are cut as well, and go out as they lie.
+Turns mix_turns(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q, int64_t max_keys) {
     const int64_t steps = (max_keys + kStep - 1) / kStep;
-    // a token's sequence is about as long as the mean of the mean and the longest one, and it is in its middle
-    const double seen = ((double)(max_keys - max_seqlen_q) + 0.25 * ((double)tokens / num_seqs + (double)max_seqlen_q)) / kStep + 0.5;
+    const double exponent = std::max((double)steps / steps_seen(num_seqs, tokens, max_seqlen_q, max_keys) - 1., 0.004);
     double walks[kShares];
-    for (int i = 0; i < kShares; ++i) walks[i] = std::max(1., (double)steps * std::pow((kShares - i - 0.5) / kShares, std::max((double)steps / seen - 1., 0.004)));
+    for (int i = 0; i < kShares; ++i) walks[i] = std::max(1., (double)steps * std::pow((kShares - i - 0.5) / kShares, exponent));
     const int wide = heads <= 8 ? 4 : heads <= 16 ? 2 : 1, narrow = heads <= 8 ? 2 : 1;
-    const bool orders = num_seqs <= kLanes && max_keys <= kMostKeys;       // walks of more sequences are cut as well, and go out as they lie
+    Turns turns{};
     double best = 0.;
     for (int tiles = wide; tiles >= narrow; tiles /= 2) {
         const int queries = 16 * tiles;
         const double blocks = std::min((double)tokens / queries + 0.5 * num_seqs, (double)((max_seqlen_q + queries - 1) / queries) * num_seqs);
         const Cost& cost = kCosts[vdim > 64][(heads <= 8 ? 0 : heads <= 16 ? 2 : 4) + (tiles < wide)];
+        int64_t last = 0;
         for (const double share : {1., 0.8, 0.65, 1. / 2, 0.4, 1. / 3, 1. / 4, 1. / 6, 1. / 8}) {
             const int64_t most = std::min(std::max<int64_t>(4, (int64_t)std::ceil(share * (double)steps - 1e-9)), steps);
+            if (most == last) continue;                          // a short walk has few cuts, and its call waits for the host: 32 sequences of 27 to 85 tokens 18.9 -> 17.5 us
+            last = most;
             const double t = mix_time(walks, blocks, (int)steps, (int)most, cost, 4e-6 * (double)(queries * heads * vdim));
             if (best > 0. && t >= best) continue;
             best = t;
-            p.turns = Turns{queries, 2, (int)most, (int)((steps + most - 1) / most), true, 0};
+            turns = Turns{queries, 2, (int)most, (int)((steps + most - 1) / most), true, 0};
         }
     }
+    return arranged(turns, num_seqs, max_seqlen_q, max_keys, kUnits);
+}
+Turns sum_turns(int64_t heads, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q, int64_t max_keys, bool bounded) {
+    const int64_t steps = (max_keys + kStep - 1) / kStep;
     // few queries: more wavefronts with fewer of them each
-    p.sums = Turns{(max_seqlen_q + 63) / 64 * num_seqs * heads < 2048 ? 128 : 256, 1, (int)steps, 1, true, 0};
+    Turns sums{(max_seqlen_q + 63) / 64 * num_seqs * heads < 2048 ? 128 : 256, 1, (int)steps, 1, true, 0};
     // Few workgroups: no walk longer than what a place for a wavefront has to do, eight of a unit.  More even out by themselves, and parts cost each what it takes
     // to begin; the call, us, cut / whole: 400 workgroups (one sequence of 6000) 431 / 468, 240 (2 of 900 .. 1000) 62.5 / 68.7, 660 (6 of 1214 .. 2313) 274 / 265, 820 (8 of
     // 700 .. 2300) 303 / 294, 930 (16 of 100 .. 1500) 213 / 209, 960 (32 of 100 .. 600) 126 / 123.
-    if (bounded && ((double)tokens / p.sums.queries + 0.5 * num_seqs) * heads <= 2 * kUnits) {
+    if (bounded && ((double)tokens / sums.queries + 0.5 * num_seqs) * heads <= 2 * kUnits) {
+        const double seen = steps_seen(num_seqs, tokens, max_seqlen_q, max_keys);
         const int64_t n = std::max<int64_t>({8, (int64_t)((double)tokens / 64 * heads * seen / (8 * kUnits)) + 1, (steps + 7) / 8});
         if (5 * n <= 4 * steps) {
-            p.sums.most = (int)n;
-            p.sums.splits = (int)((steps + n - 1) / n);
+            sums.most = (int)n;
+            sums.splits = (int)((steps + n - 1) / n);
         }
     }
-    // Finding a turn takes 1 to 2 us, which is not worth it where walks are short or all run at once: 24 sequences of 151 .. 441 78 us against 74, 23 of 67 .. 80
-    // 28 against 25, but 32 of 100 .. 600 111 against 148.
-    auto arrange = [&](Turns& t, int64_t at_once) {
-        const int64_t blocks = (max_seqlen_q + t.queries - 1) / t.queries;
-        t.sorted = orders && steps > 16 && t.splits * blocks * num_seqs > at_once;
-        if (!t.sorted) t.run = 1;
-        t.units = (int)((blocks + t.run - 1) / t.run);
-    };
-    arrange(p.turns, kUnits);
-    arrange(p.sums, 2 * kUnits);
-    return p;
+    return arranged(sums, num_seqs, max_seqlen_q, max_keys, 2 * kUnits);
+}
+// Floats of the denominators, or of the sums that they are made of, and of all parts
+int64_t sum_floats(const Turns& sums, int64_t heads, int64_t tokens) { return (sums.splits * heads * tokens + 3) / 4 * 4; }
+int64_t all_floats(const Turns& sums, const Turns& turns, int64_t heads, int64_t vdim, int64_t tokens) {
+    return sum_floats(sums, heads, tokens) + (turns.splits > 1 ? turns.splits * tokens * heads * vdim : 0);
 }
 // Turns that there are at most
 int64_t most_turns(const Turns& t, int64_t num_seqs, int64_t tokens) {
@@ -769,9 +783,7 @@ extern "C" int infer_talking_prefill_supported(int64_t heads, int64_t dim, int64
 extern "C" int64_t infer_talking_prefill_workspace_floats(int64_t heads, int64_t vdim, int64_t num_seqs, int64_t tokens, int64_t max_seqlen_q,
                                                           int64_t max_keys) {
     if (heads < 1 || vdim < 1 || num_seqs < 1 || tokens < 1 || max_seqlen_q < 1 || max_keys < 1) return 0;
-    const Plan p = plan(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys, true);
-    const int64_t lse = (p.sums.splits * heads * tokens + 3) / 4 * 4;
-    return lse + (p.turns.splits > 1 ? p.turns.splits * tokens * heads * vdim : 0);
+    return all_floats(sum_turns(heads, num_seqs, tokens, max_seqlen_q, max_keys, true), mix_turns(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys), heads, vdim, tokens);
 }
 
 extern "C" int infer_talking_prefill(const void* q, int64_t q_stride, const void* keys, const void* values, int64_t key_pad,
@@ -793,17 +805,16 @@ extern "C" int infer_talking_prefill(const void* q, int64_t q_stride, const void
         return INFER_KV_EINVAL;
     if (q_stride % 8 || out_stride % 4 || !ptr_aligned(q, 16) || !ptr_aligned(keys, 16) || !ptr_aligned(values, 16) || !ptr_aligned(out, 8))
         return INFER_KV_EALIGN;
-    if (!workspace || !ptr_aligned(workspace, 16) ||
-        workspace_floats < infer_talking_prefill_workspace_floats(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys))
-        return INFER_KV_EWORKSPACE;
     const bool bounded = max_score * kLog2e <= kBound;
-    const Plan p = plan(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys, bounded);
+    const Turns mix = mix_turns(heads, vdim, num_seqs, tokens, max_seqlen_q, max_keys), cut = sum_turns(heads, num_seqs, tokens, max_seqlen_q, max_keys, true);
+    if (!workspace || !ptr_aligned(workspace, 16) || workspace_floats < all_floats(cut, mix, heads, vdim, tokens)) return INFER_KV_EWORKSPACE;
+    const Turns sums = bounded ? cut : sum_turns(heads, num_seqs, tokens, max_seqlen_q, max_keys, false);
     const TalkPrefillArgs a{(const __bf16*)q, q_stride, (const __bf16*)keys, (const __bf16*)values, (int)key_pad, (int)vdim_pad, block_table,
                             bt_stride, (int)table_cols, (int)block_size, (int)num_blocks, seqs, cu_q, cu_k, (int)heads, (int)kv_heads, (int)dim,
-                            (int)vdim, (int)num_seqs, scale * kLog2e, (const __bf16*)talk, out_scale, (__bf16*)out, out_stride, workspace, tokens, p.turns,
-                            p.sums, bounded, workspace + (p.sums.splits * heads * tokens + 3) / 4 * 4};
+                            (int)vdim, (int)num_seqs, scale * kLog2e, (const __bf16*)talk, out_scale, (__bf16*)out, out_stride, workspace, tokens, mix,
+                            sums, bounded, workspace + sum_floats(sums, heads, tokens)};
     hipStream_t st = (hipStream_t)stream;
-    const int64_t sum_turns = most_turns(p.sums, num_seqs, tokens), turns = most_turns(p.turns, num_seqs, tokens);
-    if (dim <= 64) return vdim <= 64 ? launch<2, 4>(a, sum_turns, turns, max_seqlen_q, st) : launch<2, 8>(a, sum_turns, turns, max_seqlen_q, st);
-    return vdim <= 64 ? launch<4, 4>(a, sum_turns, turns, max_seqlen_q, st) : launch<4, 8>(a, sum_turns, turns, max_seqlen_q, st);
+    const int64_t most_sums = most_turns(sums, num_seqs, tokens), most_mix = most_turns(mix, num_seqs, tokens);
+    if (dim <= 64) return vdim <= 64 ? launch<2, 4>(a, most_sums, most_mix, max_seqlen_q, st) : launch<2, 8>(a, most_sums, most_mix, max_seqlen_q, st);
+    return vdim <= 64 ? launch<4, 4>(a, most_sums, most_mix, max_seqlen_q, st) : launch<4, 8>(a, most_sums, most_mix, max_seqlen_q, st);
 }
